@@ -100,13 +100,12 @@ torch::Tensor dci_query(py::handle capsule, int dim, int num_queries, torch::Ten
     const int64_t per_query = blind ? std::min(max_num_candidates, num_outer_iterations) : num_neighbours;
     TORCH_CHECK(per_query > 0, "nothing to return per query");
     const int64_t cells = (int64_t)num_queries * per_query;
-    auto ids = torch::empty({cells}, query.options().dtype(torch::kInt32));
-    auto dists = torch::empty({cells}, query.options());
-    check(dcih_query(index_of(capsule), dim, num_queries, query.data_ptr<float>(), num_neighbours,
-                     blind ? 1 : 0, num_outer_iterations, max_num_candidates, block_size,
-                     thread_size, ids.data_ptr<int32_t>(), dists.data_ptr<float>(), nullptr,
-                     stream_of(query)));
-    return torch::cat({ids.to(torch::kFloat32), dists}, 0);
+    auto result = torch::empty({2 * cells}, query.options());
+    float* out = result.data_ptr<float>();
+    check(dcih_query_float_ids(index_of(capsule), dim, num_queries, query.data_ptr<float>(), num_neighbours,
+                               blind ? 1 : 0, num_outer_iterations, max_num_candidates, block_size,
+                               thread_size, out, out + cells, nullptr, stream_of(query)));
+    return result;
 }
 
 // src/dci_cuda.cpp:120-134 (py_dci_multi_query).  One GPU per process here, so the

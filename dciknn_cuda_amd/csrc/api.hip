@@ -502,7 +502,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
                       int num_neighbours, int blind, int num_outer_iterations,
                       int max_num_candidates, int block_size, int thread_size,
                       int32_t* d_nn, float* d_dists, uint64_t* d_counters, void* stream,
-                      bool fixed, const char* who) {
+                      bool fixed, bool float_ids, const char* who) {
     const std::string me(who);
     if (!h) return fail(DCIH_EINVAL, me + ": null handle");
     if (dim != h->dim) return fail(DCIH_EINVAL, me + ": dim differs from the index's");
@@ -573,7 +573,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     a.stop_at = (int64_t)num_outer_iterations * h->L;
     a.max_cand = max_num_candidates;
     a.counters = (unsigned long long*)d_counters;
-    a.out_ids = d_nn; a.out_dists = d_dists;
+    a.out_ids = d_nn; a.out_dists = d_dists; a.float_ids = float_ids ? 1 : 0;
 
     if (fixed && num_results > 8192)
         return fail(DCIH_EUNSUPPORTED, me + ": more than 8192 results per query need the row-per-query "
@@ -587,7 +587,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
         QueryArgs probe = a;
         probe.nq = chunk; probe.kcap = 1;
         const size_t qp_bytes = align_up((size_t)I * chunk * sizeof(float));
-        const size_t rank_bytes = align_up(exhaustive_ws_bytes(h->n, chunk));
+        const size_t rank_bytes = align_up(exhaustive_ws_bytes(h->n, chunk, (int)std::min<int64_t>(h->n, 0x7fffffff)));
         const size_t gs_bytes = align_up(query_gscratch_bytes(probe));
         int rc = get_ws(qp_bytes + rank_bytes + gs_bytes);
         if (rc) return rc;
@@ -613,7 +613,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
         // traversal above.)
         const int chunk = exhaustive_chunk(h->n, num_queries);
         const size_t qp_bytes = d_counters ? align_up((size_t)I * num_queries * sizeof(float)) : 0;
-        int rc = get_ws(qp_bytes + exhaustive_ws_bytes(h->n, chunk));
+        int rc = get_ws(qp_bytes + exhaustive_ws_bytes(h->n, chunk, a.k));
         if (rc) return rc;
         if (d_counters) {
             rc = project(h->d_dirs, I, d_query, num_queries, dim, (float*)ws_base, num_queries, s);
@@ -676,7 +676,16 @@ int dcih_query(dcih_index* h, int dim, int num_queries, const float* d_query,
                int32_t* d_nn, float* d_dists, uint64_t* d_counters, void* stream) {
     return query_impl(h, dim, num_queries, d_query, num_neighbours, blind, num_outer_iterations,
                       max_num_candidates, block_size, thread_size, d_nn, d_dists, d_counters, stream,
-                      false, "dcih_query");
+                      false, false, "dcih_query");
+}
+
+int dcih_query_float_ids(dcih_index* h, int dim, int num_queries, const float* d_query,
+                         int num_neighbours, int blind, int num_outer_iterations,
+                         int max_num_candidates, int block_size, int thread_size,
+                         float* d_nn, float* d_dists, uint64_t* d_counters, void* stream) {
+    return query_impl(h, dim, num_queries, d_query, num_neighbours, blind, num_outer_iterations,
+                      max_num_candidates, block_size, thread_size, (int32_t*)d_nn, d_dists, d_counters, stream,
+                      false, true, "dcih_query_float_ids");
 }
 
 int dcih_query_noalloc(dcih_index* h, int dim, int num_queries, const float* d_query,
@@ -685,7 +694,7 @@ int dcih_query_noalloc(dcih_index* h, int dim, int num_queries, const float* d_q
                        int32_t* d_nn, float* d_dists, uint64_t* d_counters, void* stream) {
     return query_impl(h, dim, num_queries, d_query, num_neighbours, blind, num_outer_iterations,
                       max_num_candidates, block_size, thread_size, d_nn, d_dists, d_counters, stream,
-                      true, "dcih_query_noalloc");
+                      true, false, "dcih_query_noalloc");
 }
 
 int64_t dcih_debug_launch_map(int xcds, int block_size, int num_queries, int64_t block,

@@ -90,6 +90,7 @@ struct QueryArgs {
     int xcds;                // accelerator dies of the device (each has an L2 of its own)
     int q_first, q_count;    // batch kernel: the queries one launch covers
     int32_t* out_ids;        // [nq][k]
+    int float_ids;           // 1: ids are stored as float32 values in the same place
     float* out_dists;        // [nq][k]; blind: null, or the promoting steps as floats
     float* dense;            // null, or [nq][N]: the step-by-step kernel stores every candidate's score here instead of keeping a top-k
 };
@@ -156,22 +157,24 @@ int query_dense_items(const QueryArgs& a, hipStream_t s);
 
 // Full ranking (exhaustive.hip) for num_neighbours above the points per partition,
 // where the traversal provably visits everything: queries are processed `chunk` at
-// a time in `ws` (exhaustive_ws_bytes(N, chunk) bytes); a.qproj is needed only when
+// a time in `ws` (exhaustive_ws_bytes(N, chunk, k) bytes); a.qproj is needed only when
 // a.counters is set.
 int exhaustive_chunk(int64_t N, int nq);
-size_t exhaustive_ws_bytes(int64_t N, int chunk);
+size_t exhaustive_ws_bytes(int64_t N, int chunk, int k);
 int query_exhaustive(const QueryArgs& a, void* ws, int chunk, hipStream_t s);
 // The pieces of it that the dense-row traversal (query_dense) shares: rows of N values
 // at rank_rows_input(ws), `rows` <= chunk of them; rank_rows sorts every row by (value,
 // column) and writes the first k columns (id = column, or -1 for +inf when asked).
 float* rank_rows_input(void* ws);
 int fill_rows(float* d_rows, int64_t cells, float value, hipStream_t s);
-int rank_rows(void* ws, int chunk, int rows, int64_t N, int k, bool inf_is_empty,
+int rank_rows(void* ws, int chunk, int rows, int64_t N, int k, bool inf_is_empty, bool float_ids,
               int32_t* out_ids, float* out_vals, hipStream_t s);
+// k best of the B ascending lists of kcap packed words per query at a.part, to a.out_ids / a.out_dists.
+int merge_lists(const QueryArgs& a, hipStream_t s);
 // More results per query than the top-k tables hold, early stops possible: the
 // step-by-step kernel writes every candidate's score into a dense row of its query
 // (+inf = not a candidate), rank_rows does the rest.  Projects the queries itself
-// (d_dirs), chunk by chunk; ws = I*chunk floats + exhaustive_ws_bytes(N, chunk) bytes.
+// (d_dirs), chunk by chunk; ws = I*chunk floats + exhaustive_ws_bytes(N, chunk, N) bytes.
 int query_dense(const QueryArgs& a, const float* d_dirs, void* ws, int chunk, hipStream_t s);
 
 // ev: null, or five events recorded before the traversal, after the batch kernel (if it

@@ -262,10 +262,16 @@ __global__ __launch_bounds__(kWave) void traverse_kernel(QueryArgs a, Layout y) 
 
         __syncthreads();
         if (!y.topk_bytes) __threadfence();
-        for (int j = lane; j < (a.dense ? 0 : a.kcap); j += kWave) {
-            const unsigned long long v = j < tk_count ? top[j] : ~0ull;
-            part_out[j] = v;
+        if (!a.dense && y.topk_bytes) {      // in ascending order, as the merge takes them (no entry occurs twice)
+            for (int j = lane; j < tk_count; j += kWave) {
+                const unsigned long long v = top[j];
+                int rank = 0;
+                for (int o = 0; o < tk_count; o++) rank += top[o] < v ? 1 : 0;
+                part_out[rank] = v;
+            }
         }
+        for (int j = lane + (y.topk_bytes ? tk_count : 0); j < (a.dense ? 0 : a.kcap); j += kWave)
+            part_out[j] = j < tk_count ? top[j] : ~0ull;
         if (a.counters) {
             for (int o = 32; o > 0; o >>= 1) probes += __shfl_xor(probes, o, kWave);
             if (lane == 0) {
@@ -278,34 +284,95 @@ __global__ __launch_bounds__(kWave) void traverse_kernel(QueryArgs a, Layout y) 
     }
 }
 
+// One result of a query: the id (as float32 where the caller takes ids that way) and the distance.
+__device__ inline void store_result(const QueryArgs& a, int qi, int j, unsigned long long v) {
+    const bool empty = v == ~0ull;
+    const int32_t id = empty ? -1 : (int32_t)(uint32_t)v;
+    a.out_ids[(int64_t)qi * a.k + j] = a.float_ids ? __builtin_bit_cast(int32_t, (float)id) : id;
+    if (a.out_dists)
+        a.out_dists[(int64_t)qi * a.k + j] =
+            empty ? __builtin_inff()
+                  : (a.blind ? (float)(uint32_t)(v >> 32) : __builtin_bit_cast(float, (uint32_t)(v >> 32)));
+}
+
 // k best of the B*kcap per-partition results of one query (get_top_candidates,
-// src/dci_cuda_kernel.cu:691-701): repeated LDS bitonic sorts of the running
-// best k plus as many new entries as fit.
-__global__ __launch_bounds__(kMergeThreads) void merge_topk_kernel(QueryArgs a, int cap) {
-    extern __shared__ unsigned long long buf[];
-    const int qi = blockIdx.x;
-    const unsigned long long* src = a.part + (int64_t)qi * a.B * a.kcap;
-    const int64_t total = (int64_t)a.B * a.kcap;
-    const int keep = a.k < cap ? a.k : cap;   // host guarantees k <= cap / 2
-    const int room = cap - keep;
-    for (int j = threadIdx.x; j < keep; j += blockDim.x) buf[j] = ~0ull;
+// src/dci_cuda_kernel.cu:691-701), more than 256 of them: repeated LDS bitonic sorts of the running
+// best k (kept at buf[0, k)) plus as many new entries as fit cap words; k <= cap / 2.
+__device__ inline void merge_by_sorting(unsigned long long* buf, int cap, int k, const unsigned long long* src, int64_t total) {
+    const int room = cap - k;
+    for (int j = threadIdx.x; j < k; j += blockDim.x) buf[j] = ~0ull;
     for (int64_t p = 0; p < total; p += room) {
         const int m = (int)min((int64_t)room, total - p);
         __syncthreads();
         for (int j = threadIdx.x; j < room; j += blockDim.x)
-            buf[keep + j] = j < m ? src[p + j] : ~0ull;
+            buf[k + j] = j < m ? src[p + j] : ~0ull;
         bitonic_sort_u64(buf, cap);
     }
     __syncthreads();
-    for (int j = threadIdx.x; j < a.k; j += blockDim.x) {
-        const unsigned long long v = buf[j];
-        const bool empty = v == ~0ull;
-        a.out_ids[(int64_t)qi * a.k + j] = empty ? -1 : (int32_t)(uint32_t)v;
-        if (a.out_dists)
-            a.out_dists[(int64_t)qi * a.k + j] =
-                empty ? __builtin_inff()
-                      : (a.blind ? (float)(uint32_t)(v >> 32) : __builtin_bit_cast(float, (uint32_t)(v >> 32)));
+}
+
+__global__ __launch_bounds__(kMergeThreads) void merge_topk_kernel(QueryArgs a, int cap) {
+    extern __shared__ unsigned long long buf[];
+    const int qi = blockIdx.x;
+    merge_by_sorting(buf, cap, a.k, a.part + (int64_t)qi * a.B * a.kcap, (int64_t)a.B * a.kcap);
+    for (int j = threadIdx.x; j < a.k; j += blockDim.x) store_result(a, qi, j, buf[j]);
+}
+
+// The same for k <= NT.  The lists ascend, so the k-th smallest of their first few entries is an
+// upper bound of the k-th best, and only the entries up to it -- k and a few more, all near the
+// lists' beginnings -- are read and sorted.  (The bound comes from the `heads` first entries of
+// every list, at least 2 k in all; where those are more than NT, from the smallest of each thread's
+// share of them.)  Bound by its chain of reads, sorts and barriers: one wavefront per query where
+// the heads fit two per lane.  10000 queries of 58 lists of 10: 171 us with the sorts of 1024 words above.
+template <int NT>
+__global__ __launch_bounds__(NT) void merge_heads_kernel(QueryArgs a, int heads) {
+    constexpr int kCap = NT == kWave ? 256 : 2048, kAhead = 4;
+    __shared__ unsigned long long buf[kCap];
+    __shared__ uint32_t s_count;
+    const int tid = threadIdx.x, qi = blockIdx.x;
+    const unsigned long long* src = a.part + (int64_t)qi * a.B * a.kcap;
+    const int nheads = a.B * heads;
+    unsigned long long best = ~0ull;
+    for (int e = tid; e < nheads; e += NT) {
+        const unsigned long long v = src[(int64_t)(e / heads) * a.kcap + e % heads];
+        best = v < best ? v : best;
     }
+    buf[tid] = best;
+    if (tid == 0) s_count = 0;
+    if constexpr (NT == kWave) bitonic_sort_u64(buf, NT); else bitonic_sort_u64_by256(buf, NT);
+    const unsigned long long bound = buf[a.k - 1];       // (nothing at all in some list heads: ~0, every entry passes)
+    __syncthreads();
+    for (int l = tid; l < a.B; l += NT) {
+        const unsigned long long* list = src + (int64_t)l * a.kcap;
+        for (int j0 = 0; j0 < a.kcap; j0 += kAhead) {
+            unsigned long long v[kAhead];
+#pragma unroll
+            for (int u = 0; u < kAhead; u++) v[u] = list[min(j0 + u, a.kcap - 1)];
+            bool more = true;
+#pragma unroll
+            for (int u = 0; u < kAhead; u++) {
+                const bool take = j0 + u < a.kcap && v[u] <= bound && v[u] != ~0ull;
+                if (take) {
+                    const uint32_t slot = atomicAdd(&s_count, 1u);
+                    if (slot < (uint32_t)kCap) buf[slot] = v[u];
+                }
+                more = more && take;
+            }
+            if (!more) break;
+        }
+    }
+    __syncthreads();
+    const int count = (int)s_count;
+    if (count > kCap) {      // a few lists hold nearly all of the best: the lists as a whole
+        merge_by_sorting(buf, kCap, a.k, src, (int64_t)a.B * a.kcap);
+    } else {
+        int n = kWave;
+        while (n < count || n < a.k) n <<= 1;
+        for (int j = count + tid; j < n; j += NT) buf[j] = ~0ull;
+        if (NT == kMergeThreads && n >= kMergeThreads) bitonic_sort_u64_by256(buf, n);
+        else bitonic_sort_u64(buf, n);
+    }
+    for (int j = tid; j < a.k; j += NT) store_result(a, qi, j, buf[j]);
 }
 
 // Clears n 64-bit words at p and also_n 32-bit words at `also` (either may be null / 0).
@@ -364,6 +431,22 @@ size_t query_gscratch_bytes(const QueryArgs& a) {
     const Layout y = make_layout(a);
     if (y.lds_counters) return 0;
     return (size_t)traverse_grid(a, y) * (size_t)y.counter_words * 4;
+}
+
+int merge_lists(const QueryArgs& a, hipStream_t s) {
+    // (the lists of the step-by-step kernel ascend as long as its top-k stays in LDS)
+    const int heads = min(a.kcap, (int)(((int64_t)2 * a.k + a.B - 1) / a.B));
+    if (a.k <= 32 && (int64_t)a.B * heads <= 2 * kWave) {
+        hipLaunchKernelGGL(merge_heads_kernel<kWave>, dim3((unsigned)a.nq), dim3(kWave), 0, s, a, heads);
+    } else if (a.k <= kMergeThreads && (int64_t)a.B * heads < 0x7fffffffLL) {
+        hipLaunchKernelGGL(merge_heads_kernel<kMergeThreads>, dim3((unsigned)a.nq), dim3(kMergeThreads), 0, s, a, heads);
+    } else {
+        const int cap = merge_cap(a.k, (int64_t)a.B * a.kcap);
+        hipLaunchKernelGGL(merge_topk_kernel, dim3((unsigned)a.nq), dim3(kMergeThreads),
+                           (size_t)cap * sizeof(unsigned long long), s, a, cap);
+    }
+    DCIH_HIP(hipGetLastError());
+    return 0;
 }
 
 int query(const QueryArgs& a_in, hipStream_t s, hipEvent_t* ev, bool* ran) {
@@ -456,9 +539,10 @@ int query(const QueryArgs& a_in, hipStream_t s, hipEvent_t* ev, bool* ran) {
     }
     DCIH_HIP(hipGetLastError());
     if (ev) (void)hipEventRecord(ev[3], s);
-    const int cap = merge_cap(a.k, (int64_t)a.B * a.kcap);
-    hipLaunchKernelGGL(merge_topk_kernel, dim3((unsigned)a.nq), dim3(kMergeThreads),
-                       (size_t)cap * sizeof(unsigned long long), s, a, cap);
+    {
+        const int rc = merge_lists(a, s);
+        if (rc) return rc;
+    }
     if (ev) (void)hipEventRecord(ev[4], s);
     DCIH_HIP(hipGetLastError());
     return 0;
@@ -508,7 +592,7 @@ int query_dense(const QueryArgs& a_in, const float* d_dirs, void* ws, int chunk,
             hipLaunchKernelGGL(traverse_kernel<false>, dim3((unsigned)grid), dim3(kWave), y.lds_bytes, s, a, y);
         }
         DCIH_HIP(hipGetLastError());
-        rc = rank_rows(ws_rank, chunk, a.nq, a.N, a_in.k, true, a_in.out_ids + (int64_t)q0 * a_in.k,
+        rc = rank_rows(ws_rank, chunk, a.nq, a.N, a_in.k, true, a_in.float_ids != 0, a_in.out_ids + (int64_t)q0 * a_in.k,
                        a_in.out_dists ? a_in.out_dists + (int64_t)q0 * a_in.k : nullptr, s);
         if (rc) return rc;
     }

@@ -185,6 +185,15 @@ int dcih_query(dcih_index* h, int dim, int num_queries, const float* d_query,
                int32_t* d_nn, float* d_dists, uint64_t* d_counters, void* stream);
 
 /*
+ * dcih_query with the ids stored as float32 values (-1 for an empty slot), the form in which
+ * src/dci_cuda.cpp:97-107 hands them out; exact up to 2^24, the caller refuses larger indexes.
+ */
+int dcih_query_float_ids(dcih_index* h, int dim, int num_queries, const float* d_query,
+                         int num_neighbours, int blind, int num_outer_iterations,
+                         int max_num_candidates, int block_size, int thread_size,
+                         float* d_nn, float* d_dists, uint64_t* d_counters, void* stream);
+
+/*
  * dcih_query for callers that cannot allocate device memory: code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  It has no
  * counterpart in the reference.  Same arguments and same traversal kernels as
