@@ -129,6 +129,15 @@ struct dcih_index {
     uint16_t* d_rpos = nullptr;         // [I][n] the same, in the order of each composite's first simple index (room kept by the
                                         // build, filled by the first query that runs the batch traversal kernel)
     int rpos_ready = 0;
+    // 8-bit codes of the rows (room kept by the build, filled once the dense kernel's calls have asked
+    // for more candidate rows than forming them costs; rows8.hip)
+    unsigned char* d_rows8 = nullptr;
+    uint32_t* d_rows8_bounds = nullptr;
+    double rows8_demand = 0.0;          // candidate rows asked for so far
+    bool rows8_ready = false;
+    hipStream_t rows8_stream = nullptr; // where they were formed, and the event that says when
+    hipEvent_t rows8_event = nullptr;
+    bool rows8_settled = false;         // the event has been seen to be over
     float* d_own = nullptr;             // rows copied in by dcih_append (the index owns these)
     float* d_ukeys = nullptr;           // [I][own_rows] unsorted projections of the rows in d_own
     int64_t own_rows = 0;               // capacity of d_own / d_ukeys in rows
@@ -187,6 +196,10 @@ int release_sorted(dcih_index* h) {
     h->d_inv = nullptr;
     h->d_rpos = nullptr;
     h->rpos_ready = 0;
+    h->d_rows8 = nullptr;
+    h->d_rows8_bounds = nullptr;
+    h->rows8_ready = false;
+    h->rows8_demand = 0.0;
     h->d_stop_hint = nullptr;
     return 0;
 }
@@ -240,10 +253,10 @@ int ensure_arena(dcih_index* h, int which, size_t bytes) {
 
 // Where the arrays of an index of n points lie inside an arena.
 struct ArenaLayout {
-    size_t keys, ids, inv, rpos, hint, total;   // byte offsets, and the size of it all
+    size_t keys, ids, inv, rpos, hint, rows8, bounds8, total;   // byte offsets, and the size of it all
     bool small_parts;                           // partitions of at most 65536 points: 16-bit tables exist
 };
-ArenaLayout arena_layout(int I, int64_t n, int block_size) {
+ArenaLayout arena_layout(int I, int64_t n, int block_size, int dim) {
     ArenaLayout y;
     const size_t cells = (size_t)I * (size_t)n;
     y.small_parts = (n + block_size - 1) / block_size <= 65536;
@@ -257,8 +270,39 @@ ArenaLayout arena_layout(int I, int64_t n, int block_size) {
     y.inv = y.ids + b_ids;
     y.rpos = y.inv + b_inv;
     y.hint = y.rpos + b_inv;
-    y.total = y.hint + b_hint;
+    y.rows8 = y.hint + b_hint;
+    y.bounds8 = y.rows8 + (rows8_supported(dim) ? align_up((size_t)n * rows8_record_bytes(dim)) : 0);
+    y.total = y.bounds8 + (rows8_supported(dim) ? align_up((size_t)3 * block_size * sizeof(uint32_t) + 8) : 0);
     return y;
+}
+
+// Whether a call on stream `s` that goes to the dense kernel may compare rows by their codes; forms
+// the codes when they have become worth it: a candidate read by its code saves three quarters of its row,
+// forming the codes reads every row and writes a quarter of it, so from twice as many candidates as rows on.
+int use_rows8(dcih_index* h, double candidates, bool may_form, hipStream_t s, bool& use) {
+    use = false;
+    if (!h->d_rows8) return 0;
+    h->rows8_demand += candidates;
+    if (!h->rows8_ready) {
+        if (!may_form || h->rows8_demand < 2.0 * (double)h->n || capturing(s)) return 0;
+        if (!h->rows8_event) DCIH_HIP(hipEventCreateWithFlags(&h->rows8_event, hipEventDisableTiming));
+        const int64_t ppb = (h->n + h->block_size - 1) / h->block_size;
+        const int rc = code_rows(h->d_data, h->n, h->dim, ppb, h->block_size, h->d_rows8, h->d_rows8_bounds, s);
+        if (rc) return rc;
+        DCIH_HIP(hipEventRecord(h->rows8_event, s));
+        h->rows8_stream = s;
+        h->rows8_ready = true;
+        h->rows8_settled = false;
+    } else if (!h->rows8_settled && s != h->rows8_stream) {
+        if (capturing(s)) return 0;
+        if (hipEventQuery(h->rows8_event) == hipSuccess) h->rows8_settled = true;
+        else {
+            (void)hipGetLastError();
+            DCIH_HIP(hipStreamWaitEvent(s, h->rows8_event, 0));
+        }
+    }
+    use = true;
+    return 0;
 }
 
 // Records the start (which = 0) or end (1) event of timer t when profiling.
@@ -339,7 +383,7 @@ static int sort_into(dcih_index* h, int which, const float* d_keys, int64_t key_
                      int64_t num_points, const float* d_data, int block_size, void* d_tmp,
                      hipStream_t s, int64_t merge_from = 0) {
     const int I = num_indices(h);
-    const ArenaLayout y = arena_layout(I, num_points, block_size);
+    const ArenaLayout y = arena_layout(I, num_points, block_size, h->dim);
     char* base = (char*)h->arena[which];
     float* skeys = (float*)(base + y.keys);
     int32_t* sids = (int32_t*)(base + y.ids);
@@ -364,6 +408,10 @@ static int sort_into(dcih_index* h, int which, const float* d_keys, int64_t key_
     h->d_skeys = skeys; h->d_sids = sids; h->d_inv = inv; h->d_stop_hint = hint;
     h->d_rpos = y.small_parts ? (uint16_t*)(base + y.rpos) : nullptr;
     h->rpos_ready = 0;
+    h->d_rows8 = rows8_supported(h->dim) ? (unsigned char*)(base + y.rows8) : nullptr;
+    h->d_rows8_bounds = rows8_supported(h->dim) ? (uint32_t*)(base + y.bounds8) : nullptr;
+    h->rows8_ready = false;
+    h->rows8_demand = 0.0;
     h->cur = which;
     h->d_data = d_data;
     h->n = num_points;
@@ -388,7 +436,7 @@ int dcih_add(dcih_index* h, int dim, int64_t num_points, const float* d_data,
     // (the unsorted keys): a rebuild of the same size allocates and frees nothing
     const size_t b_keys = align_up((size_t)I * num_points * sizeof(float));
     const size_t tmp_bytes = segsort_tmp_bytes(I, num_points, block_size);
-    int rc = ensure_arena(h, h->cur, arena_layout(I, num_points, block_size).total);
+    int rc = ensure_arena(h, h->cur, arena_layout(I, num_points, block_size, dim).total);
     if (rc == DCIH_OK) rc = ensure_ws(h, b_keys + align_up(tmp_bytes), s);
     if (rc == DCIH_OK) {
         float* d_keys = (float*)h->ws;
@@ -452,8 +500,8 @@ int dcih_append(dcih_index* h, int dim, int64_t num_points, const float* d_data,
     }
     const size_t tmp_bytes = merge ? segsort_append_tmp_bytes(I, total) : segsort_tmp_bytes(I, total, block_size);
     int rc = ensure_arena(h, h->n > 0 ? spare : h->cur,
-                          std::max(arena_layout(I, total, block_size).total,
-                                   arena_layout(I, cap, block_size).total));
+                          std::max(arena_layout(I, total, block_size, dim).total,
+                                   arena_layout(I, cap, block_size, dim).total));
     if (rc == DCIH_OK && tmp_bytes) rc = ensure_ws(h, align_up(tmp_bytes), s);
     hipError_t e = hipSuccess;
     if (rc == DCIH_OK && h->n > 0 && rows != h->d_data)        // rows (and projections) indexed so far
@@ -551,6 +599,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     a.wide_items = nullptr; a.wide_count = nullptr; a.wide_cap = 0;
     a.block_list = nullptr; a.block_list_count = nullptr; a.full_tables = 0;
     a.dense_min_promos = h->dense_min_promos;
+    a.rows8 = nullptr; a.rows8_rec = 0; a.rows8_bounds = nullptr; a.query8 = nullptr;
     a.phase_ticks = h->d_phase_ticks;
     // the hints describe where traversals of one query shape stop; forget them when it
     // changes (cleared by a kernel: a memset node is not safe in a captured graph)
@@ -626,6 +675,19 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
         return rc;
     }
 
+    size_t q8_bytes = 0;
+    if (!blind && dense_traversal_supported(a, nullptr)) {
+        const bool all_dense = takes_dense_kernel(a);
+        bool use = false;
+        const double per_item = std::min((double)a.ppb, expected_promotions(a));
+        const int rc8 = use_rows8(h, all_dense ? (double)num_queries * block_size * per_item : 0.0, all_dense && !fixed, s, use);
+        if (rc8) return rc8;
+        if (use) {
+            a.rows8 = h->d_rows8; a.rows8_rec = rows8_record_bytes(dim); a.rows8_bounds = h->d_rows8_bounds;
+            if (dense_traversal_supported(a, nullptr)) q8_bytes = align_up((size_t)num_queries * rows8_query_bytes(dim));
+            else a.rows8 = nullptr;      // (no room for the longer list of what is kept)
+        }
+    }
     const size_t qp_bytes = align_up((size_t)I * num_queries * sizeof(float));
     const size_t part_bytes = align_up(query_part_bytes(a));
     const size_t gs_bytes = align_up(query_gscratch_bytes(a));
@@ -638,7 +700,9 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     // (the second pass may have to take every item, up to what one launch of 256-thread workgroups covers)
     a.wide_cap = std::min((int64_t)num_queries * block_size, (int64_t)1 << 23);
     const size_t wide_bytes = align_up((size_t)a.wide_cap * sizeof(int32_t));
-    int rc = get_ws(qp_bytes + part_bytes + gs_bytes + redo_bytes + 256 + dense_bytes + wide_bytes);
+    const size_t ws_bytes = qp_bytes + part_bytes + gs_bytes + redo_bytes + 256 + dense_bytes + wide_bytes;
+    if (fixed && ws_bytes + q8_bytes > kScratchBytes) { a.rows8 = nullptr; q8_bytes = 0; }
+    int rc = get_ws(ws_bytes + q8_bytes);
     if (rc) return rc;
     char* base = ws_base;
     float* d_qproj = (float*)base;
@@ -656,6 +720,12 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     rc = project(h->d_dirs, I, d_query, num_queries, dim, d_qproj, num_queries, s);
     mark(h, DCIH_T_QPROJECT, 1, s);
     if (rc) return rc;
+    if (a.rows8) {
+        unsigned char* q8 = (unsigned char*)(base + qp_bytes + part_bytes + gs_bytes + redo_bytes + 256 + dense_bytes + wide_bytes);
+        rc = code_queries(d_query, num_queries, dim, q8, s);
+        if (rc) return rc;
+        a.query8 = q8;
+    }
     // events in the order query() records them: traversal start, batch kernel end, dense
     // kernel end, traversal end, merge end
     hipEvent_t qev[5] = {h->ev[2 * DCIH_T_TRAVERSE], h->ev[2 * DCIH_T_BATCH + 1], h->ev[2 * DCIH_T_DENSE + 1],
@@ -829,6 +899,7 @@ int dcih_free(dcih_index* h) {
     if (h->ws) (void)hipFree(h->ws);
     if (h->d_dirs) (void)hipFree(h->d_dirs);
     for (auto& e : h->ev) if (e) (void)hipEventDestroy(e);
+    if (h->rows8_event) (void)hipEventDestroy(h->rows8_event);
     delete h;
     return DCIH_OK;
 }

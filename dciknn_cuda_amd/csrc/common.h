@@ -130,6 +130,17 @@ __device__ inline unsigned long long wave_max_u64(unsigned long long v) {
     w = lane_xor<1>(v); v = w > v ? w : v;
     return v;
 }
+// Sums over the lanes up to and including each one's, by DPP row shifts and broadcasts.
+__device__ inline uint32_t wave_scan_u32(uint32_t v) {
+    int x = (int)v;
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);      // row_shr:1
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);      // row_bcast:15 into rows 1 and 3
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);      // row_bcast:31 into rows 2 and 3
+    return (uint32_t)x;
+}
 __device__ inline int lane_id() { return (int)(threadIdx.x & (kWave - 1)); }
 
 // Euclidean distances (compute_dist_device, src/dci_cuda_kernel.cu:36-44) from R
@@ -168,48 +179,6 @@ __device__ inline void wave_row_dists(const float* const (&rows)[R], const float
             for (int r = 0; r < R; r++) {
                 const float d = rows[r][j] - qj;
                 acc[r] = __builtin_fmaf(d, d, acc[r]);
-            }
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < R; r++) dist[r] = sqrtf(wave_sum(acc[r]));
-}
-// The same sums in the same order for 16-byte aligned rows of at least 256
-// elements, with no lane condition around a read: U pieces (256 elements apart) of each of
-// the R rows are read at once by every lane; a lane whose piece would begin past the row's
-// end reads the row's first piece again and adds nothing.  (Rows whose length is no multiple
-// of 256 elements otherwise end in an extra round of reads by a few lanes.)
-template <int R, int U>
-__device__ inline void wave_row_dists_wide(const float* const (&rows)[R], const float* q, int dim,
-                                           float (&dist)[R]) {
-    typedef float v4f __attribute__((ext_vector_type(4)));
-    const int lane = lane_id();
-    float acc[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) acc[r] = 0.f;
-    for (int j0 = 0; j0 < dim; j0 += U * kWave * 4) {
-        v4f x[U][R];
-        int jc[U];
-        bool ok[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int ju = j0 + u * kWave * 4 + lane * 4;
-            ok[u] = ju < dim;
-            jc[u] = ok[u] ? ju : lane * 4;
-#pragma unroll
-            for (int r = 0; r < R; r++) x[u][r] = *reinterpret_cast<const v4f*>(rows[r] + jc[u]);
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const float q0 = q[jc[u]], q1 = q[jc[u] + 1], q2 = q[jc[u] + 2], q3 = q[jc[u] + 3];
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                float s2 = acc[r];
-                float d = x[u][r].x - q0; s2 = __builtin_fmaf(d, d, s2);
-                d = x[u][r].y - q1; s2 = __builtin_fmaf(d, d, s2);
-                d = x[u][r].z - q2; s2 = __builtin_fmaf(d, d, s2);
-                d = x[u][r].w - q3; s2 = __builtin_fmaf(d, d, s2);
-                acc[r] = ok[u] ? s2 : acc[r];
             }
         }
     }
@@ -264,14 +233,13 @@ __device__ inline void bitonic_sort_u64(unsigned long long* s, int n, int tid = 
     __syncthreads();
 }
 
-// The same sort for n = 256 * E words by a workgroup of exactly 256 threads, E a power of
+// The same sort for n = NT * E words by a workgroup of exactly NT threads, E a power of
 // two: every thread keeps E consecutive words in registers, exchanges within a thread and
 // within a wavefront need neither LDS nor a barrier, and only the steps whose partners lie in
-// another wavefront (two or three of them in all) go through `s`.
-template <int E>
-__device__ inline void bitonic_sort_u64_regs(unsigned long long* s) {
-    constexpr int n = 256 * E;
-    const int tid = (int)threadIdx.x;
+// another wavefront (two or three of them in all for 256 threads) go through `s`.
+template <int E, int NT>
+__device__ __forceinline__ void bitonic_sort_u64_regs(unsigned long long* s, int tid) {
+    constexpr int n = NT * E;
     unsigned long long v[E];
     __syncthreads();
 #pragma unroll
@@ -320,13 +288,33 @@ __device__ inline void bitonic_sort_u64_regs(unsigned long long* s) {
     for (int i = 0; i < E; i++) s[tid * E + i] = v[i];
     __syncthreads();
 }
-// n words by 256 threads: the register variant where it applies.
-__device__ inline void bitonic_sort_u64_by256(unsigned long long* s, int n) {
-    if (n == 256) bitonic_sort_u64_regs<1>(s);
-    else if (n == 512) bitonic_sort_u64_regs<2>(s);
-    else if (n == 1024) bitonic_sort_u64_regs<4>(s);
-    else bitonic_sort_u64(s, n);
+// The words of a wavefront's lanes, ascending by lane.
+__device__ __forceinline__ unsigned long long wave_sort_u64(unsigned long long v) {
+    const int lane = lane_id();
+    auto step = [&](unsigned long long w, int size, int stride) {
+        const bool take_min = ((lane & size) == 0) == ((lane & stride) == 0);
+        v = (w < v) == take_min ? w : v;
+    };
+    step(lane_xor<1>(v), 2, 1);
+    step(lane_xor<2>(v), 4, 2); step(lane_xor<1>(v), 4, 1);
+    step(lane_xor<4>(v), 8, 4); step(lane_xor<2>(v), 8, 2); step(lane_xor<1>(v), 8, 1);
+    step(lane_xor<8>(v), 16, 8); step(lane_xor<4>(v), 16, 4); step(lane_xor<2>(v), 16, 2); step(lane_xor<1>(v), 16, 1);
+    step(lane_xor<16>(v), 32, 16); step(lane_xor<8>(v), 32, 8); step(lane_xor<4>(v), 32, 4); step(lane_xor<2>(v), 32, 2);
+    step(lane_xor<1>(v), 32, 1);
+    step(lane_xor<32>(v), 64, 32); step(lane_xor<16>(v), 64, 16); step(lane_xor<8>(v), 64, 8); step(lane_xor<4>(v), 64, 4);
+    step(lane_xor<2>(v), 64, 2); step(lane_xor<1>(v), 64, 1);
+    return v;
 }
+// n words by NT threads: the register variant up to MAXE words per thread (each is a piece of
+// straight-line code of its own, and four words per thread take 15 KB of it).
+template <int NT, int MAXE>
+__device__ __forceinline__ void bitonic_sort_u64_by(unsigned long long* s, int n, int tid) {
+    if (n == NT) { bitonic_sort_u64_regs<1, NT>(s, tid); return; }
+    if constexpr (MAXE >= 2) if (n == 2 * NT) { bitonic_sort_u64_regs<2, NT>(s, tid); return; }
+    if constexpr (MAXE >= 4) if (n == 4 * NT) { bitonic_sort_u64_regs<4, NT>(s, tid); return; }
+    bitonic_sort_u64(s, n, tid);
+}
+__device__ inline void bitonic_sort_u64_by256(unsigned long long* s, int n) { bitonic_sort_u64_by<256, 4>(s, n, (int)threadIdx.x); }
 #endif
 
 }  // namespace dcih

@@ -2,6 +2,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <stdint.h>
 
 namespace dcih {
@@ -87,6 +88,12 @@ struct QueryArgs {
     const int32_t* block_list;        // null = the launch covers queries q_first .. q_first + q_count; else workgroup w takes block_list[w]
     const uint32_t* block_list_count; // ... for w below this number
     int full_tables;         // 1: the batch kernel keeps its per-point flags as bits whatever the shape
+    // dense kernel: the rows' and the queries' 8-bit codes (rows8.hip; null = read whole rows)
+    const unsigned char* rows8;      // [N][rows8_rec]
+    int rows8_rec;                   // bytes per record
+    uint32_t* rows8_bounds;          // [B][2]: largest coding error and largest squared norm of a partition's rows (float
+                                     // bits), then [B]: 1 = codes found useless in this partition
+    const unsigned char* query8;     // [nq][rows8_query_bytes(dim)]
     int xcds;                // accelerator dies of the device (each has an L2 of its own)
     int q_first, q_count;    // batch kernel: the queries one launch covers
     int32_t* out_ids;        // [nq][k]
@@ -94,6 +101,17 @@ struct QueryArgs {
     float* out_dists;        // [nq][k]; blind: null, or the promoting steps as floats
     float* dense;            // null, or [nq][N]: the step-by-step kernel stores every candidate's score here instead of keeping a top-k
 };
+// About how many promotions a partition's traversal takes before it stops: k_stop of them by a window's
+// first lane, which takes about k_stop * T in all.  The step limit can ask for more: a traversal
+// that must consume the fraction f of a composite's windows before it may stop has by then promoted about
+// f^L of the partition (a point needs all L of its windows; nearby windows come first, so this is on
+// the low side), unless max_cand first-lane promotions end it earlier.
+inline double expected_promotions(const QueryArgs& a) {
+    const double windows = (double)a.L * ((double)a.ppb / (double)a.T);
+    const double f = fmin(1.0, (double)a.stop_at / fmax(1.0, windows));
+    const double by_steps = fmin((double)a.ppb * pow(f, (double)a.L), (double)a.max_cand * (double)a.T);
+    return fmax((double)a.k_stop * (double)a.T, by_steps);
+}
 // The query scratch keeps its list lengths in 64 consecutive words that one kernel clears: the
 // step-by-step kernel's redo list, one hand-over list per die (up to 32), and in the last word
 // the batch kernel's second-pass list.
@@ -155,6 +173,14 @@ int query_block(const QueryArgs& a, hipStream_t s);
 bool dense_traversal_supported(const QueryArgs& a, size_t* lds_bytes);
 int query_dense_items(const QueryArgs& a, hipStream_t s);
 
+// 8-bit codes of rows and queries (rows8.hip); bounds: 3 * B words.
+bool rows8_supported(int dim);
+int rows8_record_bytes(int dim);
+int rows8_query_bytes(int dim);
+int code_rows(const float* d_data, int64_t n, int dim, int64_t ppb, int B, unsigned char* d_recs, uint32_t* d_bounds,
+              hipStream_t s);
+int code_queries(const float* d_query, int nq, int dim, unsigned char* d_recs, hipStream_t s);
+
 // Full ranking (exhaustive.hip) for num_neighbours above the points per partition,
 // where the traversal provably visits everything: queries are processed `chunk` at
 // a time in `ws` (exhaustive_ws_bytes(N, chunk, k) bytes); a.qproj is needed only when
@@ -176,6 +202,9 @@ int merge_lists(const QueryArgs& a, hipStream_t s);
 // (+inf = not a candidate), rank_rows does the rest.  Projects the queries itself
 // (d_dirs), chunk by chunk; ws = I*chunk floats + exhaustive_ws_bytes(N, chunk, N) bytes.
 int query_dense(const QueryArgs& a, const float* d_dirs, void* ws, int chunk, hipStream_t s);
+
+// Whether a call goes to the dense kernel as a whole (given that the shape fits it).
+bool takes_dense_kernel(const QueryArgs& a);
 
 // ev: null, or five events recorded before the traversal, after the batch kernel (if it
 // ran: ran[0]), after the dense kernel (if it ran: ran[1]), between traversal and merge,

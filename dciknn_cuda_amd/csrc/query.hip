@@ -433,6 +433,13 @@ size_t query_gscratch_bytes(const QueryArgs& a) {
     return (size_t)traverse_grid(a, y) * (size_t)y.counter_words * 4;
 }
 
+// Left to choose: from the number of promotions at which the dense kernel is the cheaper one, every
+// item goes straight to it (no hints needed: also a first call is routed right).
+bool takes_dense_kernel(const QueryArgs& a) {
+    if (a.mode == 3) return true;
+    return a.mode == 0 && !a.blind && a.dense_min_promos > 0 && expected_promotions(a) >= (double)a.dense_min_promos;
+}
+
 int merge_lists(const QueryArgs& a, hipStream_t s) {
     // (the lists of the step-by-step kernel ascend as long as its top-k stays in LDS)
     const int heads = min(a.kcap, (int)(((int64_t)2 * a.k + a.B - 1) / a.B));
@@ -468,19 +475,7 @@ int query(const QueryArgs& a_in, hipStream_t s, hipEvent_t* ev, bool* ran) {
         return fail(-4, "query: this shape does not fit the batch traversal kernel");
     if (a.mode == 3 && !can_dense)
         return fail(-4, "query: this shape does not fit the dense traversal kernel");
-    // Left to choose: the stop rule needs k promotions by a window's first lane, which takes
-    // about k * T promotions in all; from the number at which the dense kernel is the cheaper
-    // one, every item goes straight to it (no hints needed: also a first call is routed right).
-    // The step limit can ask for more: a traversal that must consume the fraction f of a
-    // composite's windows before it may stop has by then promoted about f^L of the partition
-    // (a point needs all L of its windows; nearby windows come first, so this is on the low
-    // side), unless max_candidates first-lane promotions end it earlier.
-    if (a.mode == 0 && can_dense && !a.blind && a.dense_min_promos > 0) {
-        const double windows = (double)a.L * ((double)a.ppb / (double)a.T);
-        const double f = fmin(1.0, (double)a.stop_at / fmax(1.0, windows));
-        const double by_steps = fmin((double)a.ppb * pow(f, (double)a.L), (double)a.max_cand * (double)a.T);
-        if (fmax((double)a.k_stop * (double)a.T, by_steps) >= (double)a.dense_min_promos) a.mode = 3;
-    }
+    if (can_dense && takes_dense_kernel(a)) a.mode = 3;
     const bool use_block = a.mode != 1 && a.mode != 3 && can_block;
     // the batch kernel hands items that need many promotions to the dense kernel
     if (!(use_block && a.mode == 0 && can_dense && a.dense_items && a.dense_min_promos > 0)) {

@@ -107,13 +107,7 @@ BlockLayout make_block_layout(const QueryArgs& a) {
     // is redone by the step-by-step kernel
     // The tables grow with the promotions a stop needs (about k * T, more when the
     // step limit rather than c0 >= k ends the traversal): fewer, larger epochs.
-    // (the step limit can ask for more than k * T: a traversal that must consume the fraction f of a
-    //  composite's windows before it may stop has by then promoted about f^L of the partition, unless
-    //  max_candidates first-lane promotions end it earlier -- the estimate the kernel choice uses)
-    const double windows = (double)a.L * ((double)a.ppb / (double)a.T);
-    const double f = fmin(1.0, (double)a.stop_at / fmax(1.0, windows));
-    const double by_steps = fmin((double)a.ppb * pow(f, (double)a.L), (double)a.max_cand * (double)a.T);
-    const double expected = fmax((double)a.k_stop * (double)a.T, by_steps);
+    const double expected = expected_promotions(a);
     y.promo_cap = 128;
     while ((double)y.promo_cap < 2.0 * expected && y.promo_cap < 2048) y.promo_cap <<= 1;
     y.promo_max = y.promo_cap * 5 / 8;

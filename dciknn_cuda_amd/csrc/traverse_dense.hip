@@ -25,6 +25,7 @@
 // are left to the other kernels through the same hand-over list.
 #include <type_traits>
 
+#include "bucket_core.h"
 #include "common.h"
 #include "kernels.h"
 #include "radix_core.h"
@@ -34,45 +35,51 @@ namespace dcih {
 
 namespace {
 
-constexpr int kDT = 256;                 // threads per workgroup
-constexpr int kDWaves = kDT / kWave;
 constexpr uint32_t kNever = 0xffffu;     // step field of a point that is never promoted
 
 enum DMisc {   // 32-bit scalars shared by the workgroup
-    dWin = 0, dFail, dArmed, dMaxc, dCand, dProbes, dMore, dOr, dAnd, dMaxW, dWavePend0,
+    dWin = 0, dFail, dArmed, dMaxc, dCand, dProbes, dMore, dOr, dAnd, dMaxW, dMaxBits, dUse8,
     dMiscWords = 16
 };
 
+// Partitions of few points: workgroups of one wavefront, or an item would mostly wait for its own chain of
+// reads and barriers.
+constexpr int64_t kNarrowPoints = 512;
+constexpr size_t kLdsBytes = 160 * 1024;
+
 struct DenseLayout {
-    int ipt;          // windows per thread the sort holds (cap = 256 * ipt per composite)
+    int nt;           // threads per workgroup
+    int ipt;          // windows per thread the sort holds (cap = nt * ipt per composite)
     int off_idx;      // per simple index: p, qp, left start, right start   (4 * I words)
     int off_seg;      // per composite: 2L + 1 segment starts, 2L stream numbers, 2L table places of window 0
     int off_q;        // query row
     int off_time;     // uint16 per point: step << 1 | lane-0 flag
     int off_sort;     // k best + pending candidates, 64-bit words
-    int off_stage;    // radix staging; later the rank table, then the step histogram
+    int off_stage;
     int off_misc, off_wlist;
     int sort_cap, quota;
+    int front8, quota8;   // the same buffer where rows are compared by their codes: words kept, entries per wavefront between two merges
     int tiles;        // 1: rows of at most 128 elements, 16-byte aligned, distances wanted: whole batches of 64 rows
     size_t lds_bytes;
 };
 
-constexpr int kWlist = 2 * kWave;        // candidates a wavefront keeps listed
-
-int dense_ipt_for(int64_t windows) {
-    for (int ipt : {9, 17, 25, 33, 41})
-        if (windows <= (int64_t)kDT * ipt) return ipt;
-    return 0;
+// Buckets of the windows' ranking: about as many as windows, as far as two workgroups still fit a
+// CU's LDS beside ten thousand points.
+constexpr int dense_bucket_bits(int cap) {
+    return cap <= 320 ? 8 : (cap <= 1280 ? 10 : (cap <= 2560 ? 11 : (cap <= 4608 || cap > 6656 ? 12 : 13)));
 }
+constexpr int kWlist = 2 * kWave;        // candidates a wavefront keeps listed
 
 // Upper bound of the windows of one composite index: per simple index at most
 // ceil((p+1)/T) + floor((n+T-3-p)/T) + 1 <= n/T + 3.
 int64_t dense_max_windows(const QueryArgs& a) { return (int64_t)a.L * (a.ppb / a.T + 3); }
 
-DenseLayout make_dense_layout(const QueryArgs& a) {
+DenseLayout dense_layout_for(const QueryArgs& a, int nt, int ipt) {
     DenseLayout y;
     const int I = a.M * a.L;
-    y.ipt = dense_ipt_for(dense_max_windows(a));
+    y.nt = nt;
+    y.ipt = ipt;
+    const int waves = y.nt / kWave;
     int o = dMiscWords * 4 + 64 * 4;      // scalars, then scratch of the block scans
     y.off_misc = 0;
     y.off_idx = o;      o += 4 * I * 4;
@@ -80,19 +87,55 @@ DenseLayout make_dense_layout(const QueryArgs& a) {
     y.off_q = o;        o += ((a.dim + 3) & ~3) * 4;
     y.off_time = o;     o += (int)(((a.ppb + 1) & ~(int64_t)1) * 2);
     o = (o + 15) & ~15;
-    // k best plus room for candidates that beat the current k-th: four wavefronts fill
+    // k best plus room for candidates that beat the current k-th: the wavefronts fill
     // a quota each between two merges
-    // (batches of 64 rows: room for one whole batch beyond what a wavefront may hold already)
     y.tiles = (!a.blind && a.dim <= 128 && (a.dim & 3) == 0 &&
                (reinterpret_cast<uintptr_t>(a.data) & 15) == 0) ? 1 : 0;
+    // (a wavefront's share takes at least one whole batch of 64 candidates, of eight where rows are
+    //  read eight at a time; compared by their codes, at least twice as many as the k best and 64 are kept)
     y.sort_cap = 64;
-    while (y.sort_cap < a.kcap + 4 * (y.tiles ? 96 : 8)) y.sort_cap <<= 1;
-    y.quota = (y.sort_cap - a.kcap) / kDWaves;
+    while (y.sort_cap < max(a.kcap + waves * (y.tiles || a.blind ? 96 : 16), a.rows8 ? 2 * a.kcap + 64 + waves * 64 : 0)) y.sort_cap <<= 1;
+    y.quota = (y.sort_cap - a.kcap) / waves;
+    y.quota8 = max(64, (y.sort_cap - 2 * a.kcap - 64) / waves);
+    y.front8 = y.sort_cap - waves * y.quota8;
+    // staging words (later the step table, then the step histogram), behind them the buckets' counters, and
+    // behind those what the window ranking does not need meanwhile: the radix passes' counters, which are
+    // larger, reach into it
+    y.off_stage = o;    o += (nt * ipt + 4) * 4;
+    const int counters = o;
+    o += ((1 << dense_bucket_bits(nt * ipt)) / 2 + 4) * 4;
+    y.off_wlist = o;    o += waves * kWlist * 2;
     y.off_sort = o;     o += y.sort_cap * 8;
-    y.off_wlist = o;    o += kDWaves * kWlist * 2;
-    y.off_stage = o;    o += (y.ipt + 8) * kDT * 4;      // staging words, then the digit counters
+    o = max(o, counters + 8 * nt * 4);
     y.lds_bytes = (size_t)o;
     return y;
+}
+
+// Threads per workgroup and windows per thread; ipt = 0: too many windows.  With up to nine windows per
+// thread the registers allow 16 wavefronts per CU, and the kernel needs them all to hide its chains of LDS
+// and memory reads: one per workgroup where partitions are small, four where four workgroups' tables fit
+// a CU's LDS, else eight.  More windows per thread need twice the registers -- kept to 128, the ranking's
+// spills cost more than the wavefronts gain (7021 windows per composite, two workgroups per CU: 114 us per
+// item against 43) -- so there eight wavefronts per CU, of two workgroups as far as a thread can hold the windows.
+DenseLayout make_dense_layout(const QueryArgs& a) {
+    const int64_t windows = dense_max_windows(a);
+    if (a.ppb <= kNarrowPoints)
+        for (int i : {5, 9})
+            if (windows <= (int64_t)64 * i) return dense_layout_for(a, 64, i);
+    for (int i : {5, 9})
+        if (windows <= (int64_t)256 * i) {
+            const DenseLayout y = dense_layout_for(a, 256, i);
+            if (4 * y.lds_bytes <= kLdsBytes) return y;
+            break;
+        }
+    for (int i : {5, 9})
+        if (windows <= (int64_t)512 * i) return dense_layout_for(a, 512, i);
+    for (int i : {25, 33})
+        if (windows <= (int64_t)256 * i) return dense_layout_for(a, 256, i);
+    if (windows <= (int64_t)512 * 21) return dense_layout_for(a, 512, 21);
+    DenseLayout none;
+    none.ipt = 0;
+    return none;
 }
 
 // Sums of N rows' lane values over a group of N lanes at once: on entry lane s of the group
@@ -100,50 +143,91 @@ DenseLayout make_dense_layout(const QueryArgs& a) {
 // the lanes s and s ^ H and halves the rows a lane carries, adding exactly the operands the
 // butterfly  v += shfl_xor(v, H)  of wave_sum adds for that row, in the same order of levels,
 // so every total has the bits wave_row_dists gives (N - 1 exchanges for N rows, not N log N).
-template <int N>
-__device__ inline float group_row_sums(float (&v)[N], int s) {
+template <int N, class V>
+__device__ inline V group_row_sums(V (&v)[N], int s) {
     if constexpr (N == 1) {
         return v[0];
     } else {
         constexpr int H = N / 2;
         const bool upper = (s & H) != 0;
-        float nv[H];
+        V nv[H];
 #pragma unroll
         for (int i = 0; i < H; i++) {
-            const float send = upper ? v[i] : v[i + H];
-            const float keep = upper ? v[i + H] : v[i];
+            const V send = upper ? v[i] : v[i + H];
+            const V keep = upper ? v[i + H] : v[i];
             nv[i] = keep + lane_xor<H>(send);
         }
         return group_row_sums<H>(nv, s);
     }
 }
 
+// The first lane's value, in scalar registers.
+__device__ inline float uniform_f32(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+}
+__device__ inline unsigned long long uniform_u64(unsigned long long v) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    return ((unsigned long long)hi << 32) | lo;
+}
+
 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// WPS = wavefronts per SIMD the register allocation leaves room for: three where the tables let
-// three workgroups share a CU's LDS, else two (and 256 registers instead of 168).
-template <int IPT, int WPS>
-__global__ __launch_bounds__(kDT, WPS) void traverse_dense_kernel(QueryArgs a, DenseLayout y) {
+struct DenseArgs { QueryArgs a; DenseLayout y; };
+
+// Where the workgroup's tables lie in LDS.
+struct DenseTables {
+    int* p;                       // per simple index: position of the query, its projection,
+    float* qp;
+    int* tabbase;                 // where its windows start in the step table (there they lie in the order of the
+    int* shift;                   // positions they cover), and the shift that makes (position + shift) / T a window's place among them
+    int* seg;                     // 2L + 1 segment starts (layout order)
+    int* segstream;               // stream (2h + side) of a segment
+    int* segw;                    // table place of a segment's window 0
+    float* q;
+    uint16_t* time;
+    unsigned long long* sortbuf;
+    uint32_t* stage;
+    uint16_t* rank16;
+    uint16_t* wlist;              // per wavefront: kWlist candidates
+    template <class A, class Y>
+    __device__ __forceinline__ DenseTables(unsigned char* smem, const A& a, const Y& y) {
+        const int I = a.M * a.L;
+        p = reinterpret_cast<int*>(smem + y.off_idx);
+        qp = reinterpret_cast<float*>(p + I);
+        tabbase = reinterpret_cast<int*>(qp + I);
+        shift = tabbase + I;
+        seg = reinterpret_cast<int*>(smem + y.off_seg);
+        segstream = seg + 2 * a.L + 1;
+        segw = segstream + 2 * a.L;
+        q = reinterpret_cast<float*>(smem + y.off_q);
+        time = reinterpret_cast<uint16_t*>(smem + y.off_time);
+        sortbuf = reinterpret_cast<unsigned long long*>(smem + y.off_sort);
+        stage = reinterpret_cast<uint32_t*>(smem + y.off_stage);
+        rank16 = reinterpret_cast<uint16_t*>(stage);
+        wlist = reinterpret_cast<uint16_t*>(smem + y.off_wlist);
+    }
+};
+
+template <int NT, int IPT, int WAVES>      // WAVES: wavefronts per SIMD the registers are shared out for
+__global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
+    // The arguments are read where they are used, through a pointer that every phase makes opaque again:
+    // read once, ahead of the loop over the items, they would be carried through it in spilled registers.
+    typedef const DenseArgs __attribute__((address_space(4)))* ArgsPtr;
+    // (Loops that may end for some threads only begin with a pointer of their own.)
+    auto fresh_args = [&]() -> ArgsPtr {
+        ArgsPtr p = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(p));
+        return p;
+    };
+    ArgsPtr args = fresh_args();
     extern __shared__ __align__(16) unsigned char smem[];
+    constexpr int kWaves = NT / kWave;
+    constexpr int kBucketBits = dense_bucket_bits(NT * IPT);
     uint32_t* misc = reinterpret_cast<uint32_t*>(smem);
     uint32_t* scan_tmp = misc + dMiscWords;                           // 64 words
-    int* s_p = reinterpret_cast<int*>(smem + y.off_idx);
-    float* s_qp = reinterpret_cast<float*>(s_p + a.M * a.L);
-    // per simple index: where its windows start in the step table (there they lie in the order
-    // of the positions they cover), and the shift that makes (position + shift) / T a window's
-    // place among them
-    int* s_tabbase = reinterpret_cast<int*>(s_qp + a.M * a.L);
-    int* s_shift = s_tabbase + a.M * a.L;
-    int* s_seg = reinterpret_cast<int*>(smem + y.off_seg);            // 2L + 1 segment starts (layout order)
-    int* s_segstream = s_seg + 2 * a.L + 1;                           // stream (2h + side) of a segment
-    float* s_q = reinterpret_cast<float*>(smem + y.off_q);
-    uint16_t* s_time = reinterpret_cast<uint16_t*>(smem + y.off_time);
-    unsigned long long* sortbuf = reinterpret_cast<unsigned long long*>(smem + y.off_sort);
-    uint32_t* stage = reinterpret_cast<uint32_t*>(smem + y.off_stage);
-    uint16_t* rank16 = reinterpret_cast<uint16_t*>(stage);
-    uint16_t* s_wlist = reinterpret_cast<uint16_t*>(smem + y.off_wlist);   // per wavefront: kWlist candidates
-    int* s_segw = s_segstream + 2 * a.L;                              // table place of a segment's window 0
+    DenseTables tb(smem, args->a, args->y);
 
     // The thread numbers are made opaque again at the start of every phase, and every phase ends
     // in an exit that is never taken but that the compiler cannot rule out (PHASE_END): otherwise
@@ -165,71 +249,79 @@ __global__ __launch_bounds__(kDT, WPS) void traverse_dense_kernel(QueryArgs a, D
         asm volatile("" : "+s"(leave_now));              \
         if (leave_now) return;                           \
         fresh_thread_ids();                              \
+        args = fresh_args();                             \
+        tb = DenseTables(smem, args->a, args->y);        \
     } while (0)
-    const int I = a.M * a.L;
-    const int T = a.T;
-    const int X = a.xcds;
+    const int I = args->a.M * args->a.L;
+    const int T = args->a.T;
+    const int X = args->a.xcds;
     const int xcd = (int)(blockIdx.x % X);
     const int64_t g0 = blockIdx.x / X, G = gridDim.x / X;
-    const bool listed = a.dense_items != nullptr && a.mode != 3;
-    const int64_t my_count = listed ? (int64_t)a.dense_count[xcd]
-                                    : block_items(X, a.B, a.q_count) / X;
+    const bool listed = args->a.dense_items != nullptr && args->a.mode != 3;
+    const int64_t my_count = listed ? (int64_t)args->a.dense_count[xcd]
+                                    : block_items(X, args->a.B, args->a.q_count) / X;
 
     // optional phase profile: thread 0 adds the 100 MHz ticks each phase took
     unsigned long long tick = 0ull;
     auto phase = [&](int which) {
-        if (a.phase_ticks && tid == 0) {
+        if (args->a.phase_ticks && tid == 0) {
             const unsigned long long now = wall_clock64();
-            atomicAdd(&a.phase_ticks[which], now - tick);
+            atomicAdd(&args->a.phase_ticks[which], now - tick);
             tick = now;
         }
     };
 
     for (int64_t slot = g0; slot < my_count; slot += G) {
+        ArgsPtr args = fresh_args();
+        DenseTables tb(smem, args->a, args->y);
         int b, qi;
         if (listed) {
-            const int64_t item = a.dense_items[(int64_t)xcd * a.dense_cap + slot];
-            b = (int)(item % a.B);
-            qi = (int)(item / a.B);
+            const int64_t item = args->a.dense_items[(int64_t)xcd * args->a.dense_cap + slot];
+            b = (int)(item % args->a.B);
+            qi = (int)(item / args->a.B);
         } else {
-            if (!block_item(slot * X + xcd, X, a.B, a.q_count, b, qi)) continue;
-            qi += a.q_first;
+            if (!block_item(slot * X + xcd, X, args->a.B, args->a.q_count, b, qi)) continue;
+            qi += args->a.q_first;
         }
-        const int64_t item = (int64_t)qi * a.B + b;
-        const int64_t off = (int64_t)b * a.ppb;
-        const int n = (int)min(a.N - off, a.ppb);
-        unsigned long long* part_out = a.part + item * a.kcap;
+        b = __builtin_amdgcn_readfirstlane(b);      // (what is the same for all threads stays in scalar registers)
+        qi = __builtin_amdgcn_readfirstlane(qi);
+        const int64_t item = (int64_t)qi * args->a.B + b;
+        const int64_t off = (int64_t)b * args->a.ppb;
+        const int n = (int)min(args->a.N - off, args->a.ppb);
+        unsigned long long* part_out = args->a.part + item * args->a.kcap;
         __syncthreads();                         // the previous item's tables are done with
         if (n <= 0) {
-            for (int j = tid; j < a.kcap; j += kDT) part_out[j] = ~0ull;
+            for (int j = tid; j < args->a.kcap; j += NT) part_out[j] = ~0ull;
             continue;
         }
 
         // ---- set-up: query row, positioning searches (:279-297) -------------------
-        if (a.phase_ticks) tick = wall_clock64();
+        if (args->a.phase_ticks) tick = wall_clock64();
         if (tid < dMiscWords) misc[tid] = 0;
-        for (int j = tid; j < a.dim; j += kDT) s_q[j] = a.query[(int64_t)qi * a.dim + j];
-        for (int pt = tid; pt < n; pt += kDT) s_time[pt] = (uint16_t)((kNever << 1) & 0xffffu);
+        for (int j = tid; j < args->a.dim; j += NT) tb.q[j] = args->a.query[(int64_t)qi * args->a.dim + j];
+        for (int pt = tid; pt < n; pt += NT) tb.time[pt] = (uint16_t)((kNever << 1) & 0xffffu);
         uint32_t probes = 0;
         {
-            const int per_wave = (I + kDWaves - 1) / kDWaves;
+            const int per_wave = (I + kWaves - 1) / kWaves;
             const int lg = min(3, floor_log2(kWave / per_wave > 0 ? kWave / per_wave : 1)), Gq = 1 << lg;
             const int slots = kWave >> lg;
-            for (int i0 = 0; i0 < I; i0 += slots * kDWaves) {
+            for (int i0 = 0; i0 < I; i0 += slots * kWaves) {
                 const int sl = lane >> lg, i = i0 + wave * slots + sl;
                 const bool active = i < I;
-                const float* key = a.skeys + (int64_t)(active ? i : 0) * a.N + off;
-                const float qp = active ? a.qproj[(int64_t)i * a.nq + qi] : 0.f;
+                const float* key = args->a.skeys + (int64_t)(active ? i : 0) * args->a.N + off;
+                const float qp = active ? args->a.qproj[(int64_t)i * args->a.nq + qi] : 0.f;
                 const int lo = group_partition_point(0, n, active, lg, sl * Gq, lane - sl * Gq,
                                                      [&](int j) { return key[j] < qp; }, probes);
-                if (active && lane == sl * Gq) { s_p[i] = lo - 1; s_qp[i] = qp; }
+                if (active && lane == sl * Gq) { tb.p[i] = lo - 1; tb.qp[i] = qp; }
             }
         }
         __syncthreads();
         PHASE_END(0);
 
         unsigned long long maxw = 0;             // most windows any composite has
-        for (int m = 0; m < a.M; m++) {
+        for (int m = 0; m < args->a.M; m++) {
+            ArgsPtr args = fresh_args();
+            DenseTables tb(smem, args->a, args->y);
             // ---- layout of the composite's windows: per simple index its left stream, then
             // its right one; where the query lies above every key the single (ghost) right
             // window comes first, as dci_next_closest_proj orders it (:264-265)
@@ -237,8 +329,8 @@ __global__ __launch_bounds__(kDT, WPS) void traverse_dense_kernel(QueryArgs a, D
             if (wave == 0) {
                 const int h = lane;
                 int nl = 0, nr = 0, p = 0;
-                if (h < a.L) {
-                    p = s_p[m * a.L + h];
+                if (h < args->a.L) {
+                    p = tb.p[m * args->a.L + h];
                     nl = stream_windows(n, T, p, 0);
                     nr = stream_windows(n, T, p, 1);
                 }
@@ -249,52 +341,57 @@ __global__ __launch_bounds__(kDT, WPS) void traverse_dense_kernel(QueryArgs a, D
                     if (lane >= o) incl += t2;
                 }
                 const int at = incl - (nl + nr);
-                if (h < a.L) {
-                    const int i = m * a.L + h;
+                if (h < args->a.L) {
+                    const int i = m * args->a.L + h;
                     const bool corner = p == n - 1 && T >= 2;
                     // In the table the index's windows lie by the positions they cover: left
                     // window j at place nl - 1 - j, right window j at nl + j; a position pos
                     // belongs to the window at place (pos + nl * T - p - 1) / T and is its first
                     // lane where that division leaves no remainder.
-                    s_tabbase[i] = at;
-                    s_shift[i] = nl * T - p - 1;
+                    tb.tabbase[i] = at;
+                    tb.shift[i] = nl * T - p - 1;
                     const int w_left = at + nl - 1, w_right = at + nl;
                     if (corner) {
-                        s_seg[2 * h] = at; s_segstream[2 * h] = 2 * h + 1; s_segw[2 * h] = w_right;
-                        s_seg[2 * h + 1] = at + nr; s_segstream[2 * h + 1] = 2 * h; s_segw[2 * h + 1] = w_left;
+                        tb.seg[2 * h] = at; tb.segstream[2 * h] = 2 * h + 1; tb.segw[2 * h] = w_right;
+                        tb.seg[2 * h + 1] = at + nr; tb.segstream[2 * h + 1] = 2 * h; tb.segw[2 * h + 1] = w_left;
                     } else {
-                        s_seg[2 * h] = at; s_segstream[2 * h] = 2 * h; s_segw[2 * h] = w_left;
-                        s_seg[2 * h + 1] = at + nl; s_segstream[2 * h + 1] = 2 * h + 1; s_segw[2 * h + 1] = w_right;
+                        tb.seg[2 * h] = at; tb.segstream[2 * h] = 2 * h; tb.segw[2 * h] = w_left;
+                        tb.seg[2 * h + 1] = at + nl; tb.segstream[2 * h + 1] = 2 * h + 1; tb.segw[2 * h + 1] = w_right;
                     }
                 }
-                const int total = __shfl(incl, a.L - 1, kWave);
+                const int total = __shfl(incl, args->a.L - 1, kWave);
                 if (lane == 0) {
-                    s_seg[2 * a.L] = total;
+                    misc[dMaxBits] = 0;
+                    tb.seg[2 * args->a.L] = total;
                     misc[dWin] = (uint32_t)total;
-                    if (total > kDT * IPT || total >= 0x7fff) misc[dFail] = 1;
+                    if (total > NT * IPT || total >= 0x7fff) misc[dFail] = 1;
                     misc[dOr] = 0; misc[dAnd] = 0xffffffffu;
                 }
             }
             __syncthreads();
-            if (misc[dFail]) break;
-            const int W = (int)misc[dWin];
+            if (__builtin_amdgcn_readfirstlane((int)misc[dFail])) break;
+            const int W = __builtin_amdgcn_readfirstlane((int)misc[dWin]);
             maxw = max(maxw, (unsigned long long)W);
 
             // ---- priorities of the windows, blocked: thread t holds layout indices t*IPT.. ----
+            // (formed a second time in the rare case that the ranking by buckets gives up)
+            for (bool by_radix = false;; by_radix = true) {
+            ArgsPtr args = fresh_args();
+            DenseTables tb(smem, args->a, args->y);
             uint32_t k[IPT], rp[IPT];
             {
                 int seg = 0;
                 const int first = tid * IPT;
                 {   // the first segment that ends behind `first` (empty segments are skipped)
-                    int lo = 0, hi = 2 * a.L - 1;
+                    int lo = 0, hi = 2 * args->a.L - 1;
                     while (lo < hi) {
                         const int mid = (lo + hi) >> 1;
-                        if (s_seg[mid + 1] <= first) lo = mid + 1; else hi = mid;
+                        if (tb.seg[mid + 1] <= first) lo = mid + 1; else hi = mid;
                     }
                     seg = lo;
                 }
                 // (offsets from the composite's first slice; all reads are issued before any is used)
-                const float* kbase = a.skeys + (int64_t)m * a.L * a.N + off;
+                const float* kbase = args->a.skeys + (int64_t)m * args->a.L * args->a.N + off;
                 uint32_t koff[IPT];
                 float qv[IPT];
                 // Per segment: where its windows' keys lie and which way they run.  Window j of
@@ -305,20 +402,20 @@ __global__ __launch_bounds__(kDT, WPS) void traverse_dense_kernel(QueryArgs a, D
                 uint32_t h_base;
                 float q_seg;
                 auto enter = [&](int idx) {
-                    seg_end = s_seg[seg + 1];
-                    const int sidx = s_segstream[seg], j = idx - s_seg[seg], h = sidx >> 1;
-                    const int p = s_p[m * a.L + h];
-                    q_seg = s_qp[m * a.L + h];
-                    h_base = (uint32_t)h * (uint32_t)a.N;
-                    if (sidx & 1) { pos_step = T; pos_cur = p + 1 + j * T; w_step = 1; w_cur = s_segw[seg] + j; }
-                    else { pos_step = -T; pos_cur = p - T + 1 - j * T; w_step = -1; w_cur = s_segw[seg] - j; }
+                    seg_end = tb.seg[seg + 1];
+                    const int sidx = tb.segstream[seg], j = idx - tb.seg[seg], h = sidx >> 1;
+                    const int p = tb.p[m * args->a.L + h];
+                    q_seg = tb.qp[m * args->a.L + h];
+                    h_base = (uint32_t)h * (uint32_t)args->a.N;
+                    if (sidx & 1) { pos_step = T; pos_cur = p + 1 + j * T; w_step = 1; w_cur = tb.segw[seg] + j; }
+                    else { pos_step = -T; pos_cur = p - T + 1 - j * T; w_step = -1; w_cur = tb.segw[seg] - j; }
                 };
                 enter(first);
 #pragma unroll
                 for (int r = 0; r < IPT; r++) {
                     const int idx = first + r;
-                    if (idx >= seg_end && seg < 2 * a.L - 1) {
-                        do { seg++; } while (seg < 2 * a.L - 1 && s_seg[seg + 1] <= idx);
+                    if (idx >= seg_end && seg < 2 * args->a.L - 1) {
+                        do { seg++; } while (seg < 2 * args->a.L - 1 && tb.seg[seg + 1] <= idx);
                         enter(idx);
                     }
                     koff[r] = h_base + (uint32_t)(idx < W ? min(max(pos_cur, 0), n - 1) : 0);
@@ -330,68 +427,118 @@ __global__ __launch_bounds__(kDT, WPS) void traverse_dense_kernel(QueryArgs a, D
                 float kv[IPT];
 #pragma unroll
                 for (int r = 0; r < IPT; r++) kv[r] = kbase[koff[r]];
-                uint32_t vor = 0, vand = 0xffffffffu;
+                int most = 0;
 #pragma unroll
                 for (int r = 0; r < IPT; r++) {
                     const int idx = first + r;
                     const uint32_t bits = __builtin_bit_cast(uint32_t, fabsf(kv[r] - qv[r]));
                     k[r] = idx < W ? bits : 0xffffffffu;      // pads sort last and stay last
-                    vor |= idx < W ? bits : 0u;
-                    vand &= idx < W ? bits : 0xffffffffu;
+                    most = max(most, idx < W ? (int)bits : 0);
                 }
                 probes += IPT;
-                for (int o = 32; o > 0; o >>= 1) {
-                    vor |= (uint32_t)__shfl_xor((int)vor, o, kWave);
-                    vand &= (uint32_t)__shfl_xor((int)vand, o, kWave);
-                }
-                if (lane == 0) { atomicOr(&misc[dOr], vor); atomicAnd(&misc[dAnd], vand); }
+                most = wave_max_i32(most);
+                if (lane == 0) atomicMax(&misc[dMaxBits], (uint32_t)most);
             }
             __syncthreads();
             PHASE_END(1);
             // the step of every window: its place in the sorted order, stored doubled with bit 0
             // set: a lookup subtracts one where the point is not the window's first lane, which
             // leaves the lane-0 flag beside the step
-            bool sorted_small = false;
-            if constexpr (IPT == 9) {
-                // Up to 1024 windows (short partitions): a bitonic sort held in registers of
-                // (priority, layout index, table place) words — the layout index makes equal
-                // priorities keep their order, as the stable radix passes do — takes a few
-                // microseconds where eight radix passes over 2304 slots take thirty.
-                if (W <= 1024) {
-                    sorted_small = true;
-                    const int np = W <= 256 ? 256 : (W <= 512 ? 512 : 1024);
-                    unsigned long long* s64 = reinterpret_cast<unsigned long long*>(stage);
+            if constexpr (IPT <= 9) if (W <= 2 * NT) {
+                // Few windows: a bitonic sort held in registers of (priority, layout index, table place)
+                // words; the layout index makes equal priorities keep their order.
+                const int np = W <= NT ? NT : 2 * NT;
+                unsigned long long* s64 = reinterpret_cast<unsigned long long*>(tb.stage);
 #pragma unroll
-                    for (int r = 0; r < IPT; r++) {
-                        const int idx = tid * IPT + r;
-                        if (idx < np)
-                            s64[idx] = idx < W ? ((unsigned long long)k[r] << 32) | ((unsigned long long)idx << 16) | (rp[r] & 0xffffu)
-                                               : ~0ull;
-                    }
-                    bitonic_sort_u64_by256(s64, np);
-                    unsigned long long mine[4];
-                    const int per = np / kDT;
+                for (int r = 0; r < IPT; r++) {
+                    const int idx = tid * IPT + r;
+                    if (idx < np)
+                        s64[idx] = idx < W ? ((unsigned long long)k[r] << 32) | ((unsigned long long)idx << 16) | (rp[r] & 0xffffu)
+                                           : ~0ull;
+                }
+                if (np == NT) bitonic_sort_u64_regs<1, NT>(s64, tid); else bitonic_sort_u64_regs<2, NT>(s64, tid);
+                unsigned long long mine[2];
 #pragma unroll
-                    for (int e = 0; e < 4; e++) mine[e] = e < per ? s64[tid * per + e] : ~0ull;
-                    __syncthreads();                    // the table takes the sorted words' room
+                for (int e = 0; e < 2; e++) mine[e] = e * NT < np ? s64[e * NT + tid] : 0ull;
+                __syncthreads();                    // the table takes the sorted words' room
 #pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const int sp = tid * per + e;
-                        if (e < per && sp < W) rank16[(uint32_t)mine[e] & 0xffffu] = (uint16_t)((sp << 1) | 1);
-                    }
+                for (int e = 0; e < 2; e++)
+                    if (e * NT + tid < W) tb.rank16[(uint32_t)mine[e] & 0xffffu] = (uint16_t)(((e * NT + tid) << 1) | 1);
+                break;
+            }
+            const uint32_t max_bits = (uint32_t)__builtin_amdgcn_readfirstlane((int)misc[dMaxBits]);
+            const float scale = 4294966016.0f / __builtin_bit_cast(float, max_bits);
+            bool ranked = false;
+            int fix_rank;
+            uint32_t fix_place;
+            if (!by_radix && max_bits < kInfBits && scale < 4e38f) {      // (else, or if priorities cluster, the radix passes)
+                // two windows of equal list words: windows of one stream keep their order, others are
+                // compared by their priorities, then by their order in the layout
+                auto before = [&](int x, int z) __attribute__((always_inline)) {
+                    auto seg_of = [&](int idx) {
+                        int lo = 0, hi = 2 * args->a.L - 1;
+                        while (lo < hi) {
+                            const int mid = (lo + hi) >> 1;
+                            if (tb.seg[mid + 1] <= idx) lo = mid + 1; else hi = mid;
+                        }
+                        return lo;
+                    };
+                    const int gx = seg_of(x), gz = seg_of(z);
+                    if (gx == gz) return x < z;
+                    auto prio = [&](int idx, int g) {
+                        const int sidx = tb.segstream[g], i = m * args->a.L + (sidx >> 1);
+                        Stream st;
+                        st.key = args->a.skeys + (int64_t)i * args->a.N + off;
+                        st.n = n; st.T = T; st.p = tb.p[i]; st.side = sidx & 1; st.q = tb.qp[i];
+                        return stream_prio_bits(st, idx - tb.seg[g]);
+                    };
+                    const uint32_t bx = prio(x, gx), bz = prio(z, gz);
+                    return bx != bz ? bx < bz : x < z;
+                };
+                ranked = lds_bucket_ranks<NT, IPT, kBucketBits>(
+                    k, rp, W, scale, tb.stage, tb.stage + IPT * NT + 4, scan_tmp, reinterpret_cast<unsigned long long*>(tb.wlist),
+                    kWaves * kWlist * 2 / 8, tid, fix_rank, fix_place, before);
+                if (ranked) {
+                    __syncthreads();                    // the table takes the lists' room
+                    int own = W - tid * IPT;            // (opaque: no lane masks kept for it across the ranking)
+                    asm volatile("" : "+v"(own));
+#pragma unroll
+                    for (int r = 0; r < IPT; r++)
+                        if (r < own) tb.rank16[rp[r] & 0xffffu] = (uint16_t)(((rp[r] >> 16) << 1) | 1);
+                    __syncthreads();
+                    if (fix_rank >= 0) tb.rank16[fix_place] = (uint16_t)((fix_rank << 1) | 1);
                 }
             }
-            if (!sorted_small) {
+            if (ranked) break;
+            if (by_radix) {
+                uint32_t vor = 0, vand = 0xffffffffu;
+                int own = W - tid * IPT;
+                asm volatile("" : "+v"(own));
+#pragma unroll
+                for (int r = 0; r < IPT; r++) {
+                    const bool real = r < own;
+                    vor |= real ? k[r] : 0u;
+                    vand &= real ? k[r] : 0xffffffffu;
+                }
+                for (int o = 32; o > 0; o >>= 1) {
+                    vor |= (uint32_t)__shfl_xor((int)vor, o, kWave);
+                    vand &= (uint32_t)__shfl_xor((int)vand, o, kWave);
+                }
+                if (lane == 0) { atomicOr(&misc[dOr], vor); atomicAnd(&misc[dAnd], vand); }
+                __syncthreads();
                 // (the pads need no pass of their own: they start behind every window, every
                 //  digit of theirs is the largest, and the passes are stable)
                 const uint32_t varying = misc[dOr] ^ misc[dAnd];
-                lds_radix_passes<kDT, IPT>(k, rp, stage, stage + IPT * kDT, scan_tmp, varying);
+                lds_radix_passes<NT, IPT>(k, rp, tb.stage, tb.stage + IPT * NT + 4, scan_tmp, varying);
                 __syncthreads();
 #pragma unroll
                 for (int r = 0; r < IPT; r++) {
                     const int sp = tid * IPT + r;
-                    if (sp < W) rank16[rp[r] & 0xffffu] = (uint16_t)((sp << 1) | 1);      // (the first W sorted items are the windows)
+                    if (sp < W) tb.rank16[rp[r] & 0xffffu] = (uint16_t)((sp << 1) | 1);      // (the first W sorted items are the windows)
                 }
+                break;
+            }
+            __syncthreads();
             }
             __syncthreads();
             PHASE_END(2);
@@ -407,32 +554,32 @@ __global__ __launch_bounds__(kDT, WPS) void traverse_dense_kernel(QueryArgs a, D
             // phase is bound by vector-ALU issue, so the lookups are kept branch-free and short:
             // for a power-of-two T two points at a time in packed 16-bit arithmetic, otherwise
             // with 24-bit multiplies (32-bit ones run at a quarter of the rate).
-            const uint16_t* invm = a.inv + (int64_t)m * a.L * a.N + off;
+            const uint16_t* invm = args->a.inv + (int64_t)m * args->a.L * args->a.N + off;
             auto store_time = [&](int pt, uint32_t b) __attribute__((always_inline)) {
-                const uint32_t old = s_time[pt];      // ties: the earlier composite stays
-                if ((b >> 1) < (old >> 1)) s_time[pt] = (uint16_t)b;
+                const uint32_t old = tb.time[pt];      // ties: the earlier composite stays
+                if ((b >> 1) < (old >> 1)) tb.time[pt] = (uint16_t)b;
             };
             if (n < 8) {
-                for (int pt = tid; pt < n; pt += kDT) {
+                for (int pt = tid; pt < n; pt += NT) {
                     uint32_t best = 0u;
-                    for (int h = 0; h < a.L; h++) {
-                        const int i = m * a.L + h;
-                        const uint32_t x = (uint32_t)invm[(int64_t)h * a.N + pt] + (uint32_t)s_shift[i];
-                        const uint32_t w = T > 1 ? __umulhi(x, a.T_magic) : x;
-                        best = max(best, (uint32_t)rank16[s_tabbase[i] + w] - (x - w * (uint32_t)T != 0u ? 1u : 0u));
+                    for (int h = 0; h < args->a.L; h++) {
+                        const int i = m * args->a.L + h;
+                        const uint32_t x = (uint32_t)invm[(int64_t)h * args->a.N + pt] + (uint32_t)tb.shift[i];
+                        const uint32_t w = T > 1 ? __umulhi(x, args->a.T_magic) : x;
+                        best = max(best, (uint32_t)tb.rank16[tb.tabbase[i] + w] - (x - w * (uint32_t)T != 0u ? 1u : 0u));
                     }
                     store_time(pt, best);
                 }
             } else {
                 auto run = [&](auto path_tag) __attribute__((always_inline)) {
-                    constexpr int kPath = decltype(path_tag)::value;     // 0: T = 2^s, s >= 1; 1: any T >= 2; 2: T = 1
-                    constexpr int kH = 2, kD = 4, kChunk = kDT * 8;
-                    const int ngrp = (a.L + kH - 1) / kH;
+                    constexpr int kPath = decltype(path_tag)::value;     // 0: T = 2^s; 1: any other T
+                    constexpr int kH = 2, kD = 4, kChunk = NT * 8;
+                    const int ngrp = (args->a.L + kH - 1) / kH;
                     const int NG = ((n + kChunk - 1) / kChunk) * ngrp;
-                    const unsigned char* tab0 = reinterpret_cast<const unsigned char*>(rank16);
+                    const unsigned char* tab0 = reinterpret_cast<const unsigned char*>(tb.rank16);
                     // path 0
-                    const uint32_t sm1 = (uint32_t)floor_log2(T > 1 ? T : 2) - 1u;
-                    const u16x2 sm1_pk = {(uint16_t)sm1, (uint16_t)sm1};
+                    const uint16_t sh = (uint16_t)floor_log2(T);
+                    const u16x2 sh_pk = {sh, sh};
                     const u16x2 mask_pk = {(uint16_t)(T - 1), (uint16_t)(T - 1)};
                     const u16x2 one_pk = {1, 1};
                     // path 1: d / T for 0 <= d < 65536 is the upper 32 bits of (d << q_sh) *
@@ -440,14 +587,14 @@ __global__ __launch_bounds__(kDT, WPS) void traverse_dense_kernel(QueryArgs a, D
                     // which never reaches the next integer; q_sh = 8 serves 2 <= T <= 256, q_sh = 0
                     // the wider windows, and both factors stay below 2^24 either way.
                     const uint32_t q_sh = T <= 256 ? 8u : 0u;
-                    const uint32_t q_magic = T > 1 ? (uint32_t)(((1ull << (32 - q_sh)) + (uint32_t)T - 1) / (uint32_t)T) : 0u;
+                    const uint32_t q_magic = (uint32_t)(((1ull << (32 - q_sh)) + (uint32_t)T - 1) / (uint32_t)T);
                     const uint32_t q_T = (uint32_t)T << q_sh;
                     uint32_t best[kPath == 0 ? 4 : 8];     // path 0: two points a word
                     auto chunk_start = [&](int c0) { return min(c0 + 8 * tid, n - 8); };
                     auto issue = [&](int c0, int h0, u32x4 (&pv)[kH]) __attribute__((always_inline)) {
 #pragma unroll
                         for (int hh = 0; hh < kH; hh++) {
-                            const uint16_t* invh = invm + (int64_t)min(h0 + hh, a.L - 1) * a.N;
+                            const uint16_t* invh = invm + (int64_t)min(h0 + hh, args->a.L - 1) * args->a.N;
                             __builtin_memcpy(&pv[hh], invh + (uint32_t)chunk_start(c0), 16);
                         }
                     };
@@ -461,9 +608,9 @@ __global__ __launch_bounds__(kDT, WPS) void traverse_dense_kernel(QueryArgs a, D
                         u16x2 rem[kH][4];
 #pragma unroll
                         for (int hh = 0; hh < kH; hh++) {
-                            const int i = m * a.L + min(h0 + hh, a.L - 1);   // (past L: the last index again)
-                            const uint32_t shift = (uint32_t)s_shift[i];
-                            const unsigned char* tab = tab0 + 2 * s_tabbase[i];
+                            const int i = m * args->a.L + min(h0 + hh, args->a.L - 1);   // (past L: the last index again)
+                            const uint32_t shift = (uint32_t)tb.shift[i];
+                            const unsigned char* tab = tab0 + 2 * tb.tabbase[i];
                             const uint32_t wd[4] = {pv[hh].x, pv[hh].y, pv[hh].z, pv[hh].w};
 #pragma unroll
                             for (int j = 0; j < 4; j++) {
@@ -471,7 +618,7 @@ __global__ __launch_bounds__(kDT, WPS) void traverse_dense_kernel(QueryArgs a, D
                                     const u16x2 shift_pk = {(uint16_t)shift, (uint16_t)shift};
                                     const u16x2 x = __builtin_bit_cast(u16x2, wd[j]) + shift_pk;
                                     // twice the window's place: the byte offset of its table entry
-                                    const uint32_t w2 = __builtin_bit_cast(uint32_t, x >> sm1_pk) & 0xfffefffeu;
+                                    const uint32_t w2 = __builtin_bit_cast(uint32_t, (x >> sh_pk) << one_pk);
                                     // (spelled out: the compiler's own form of min(r, 1) is
                                     //  two compares, two selects and a byte permute)
                                     asm("v_pk_min_u16 %0, %1, %2" : "=v"(rem[hh][j]) : "v"(x & mask_pk), "v"(one_pk));
@@ -481,16 +628,12 @@ __global__ __launch_bounds__(kDT, WPS) void traverse_dense_kernel(QueryArgs a, D
 #pragma unroll
                                     for (int e = 0; e < 2; e++) {
                                         const uint32_t pos = e ? wd[j] >> 16 : wd[j] & 0xffffu;
-                                        if constexpr (kPath == 1) {
-                                            const uint32_t xs = (pos << q_sh) + (shift << q_sh);
-                                            uint32_t w;
-                                            asm("v_mul_hi_u32_u24 %0, %1, %2" : "=v"(w) : "s"(q_magic), "v"(xs));
-                                            tv[hh][2 * j + e] = *reinterpret_cast<const uint16_t*>(tab + 2 * w);
-                                            const uint32_t off_lane = (uint32_t)((uint32_t)__umul24(w, q_T) != xs);
-                                            if (e) rem[hh][j].y = (uint16_t)off_lane; else rem[hh][j].x = (uint16_t)off_lane;
-                                        } else {
-                                            tv[hh][2 * j + e] = *reinterpret_cast<const uint16_t*>(tab + 2 * (pos + shift));
-                                        }
+                                        const uint32_t xs = (pos << q_sh) + (shift << q_sh);
+                                        uint32_t w;
+                                        asm("v_mul_hi_u32_u24 %0, %1, %2" : "=v"(w) : "s"(q_magic), "v"(xs));
+                                        tv[hh][2 * j + e] = *reinterpret_cast<const uint16_t*>(tab + 2 * w);
+                                        const uint32_t off_lane = (uint32_t)((uint32_t)__umul24(w, q_T) != xs);
+                                        if (e) rem[hh][j].y = (uint16_t)off_lane; else rem[hh][j].x = (uint16_t)off_lane;
                                     }
                                 }
                             }
@@ -504,28 +647,25 @@ __global__ __launch_bounds__(kDT, WPS) void traverse_dense_kernel(QueryArgs a, D
                                         __builtin_bit_cast(u16x2, tv[hh][2 * j] | (tv[hh][2 * j + 1] << 16)) - rem[hh][j];
                                     best[j] = __builtin_bit_cast(uint32_t,
                                         __builtin_elementwise_max(__builtin_bit_cast(u16x2, best[j]), val));
-                                } else if constexpr (kPath == 1) {
+                                } else {
                                     best[2 * j] = max(best[2 * j], tv[hh][2 * j] - (uint32_t)rem[hh][j].x);
                                     best[2 * j + 1] = max(best[2 * j + 1], tv[hh][2 * j + 1] - (uint32_t)rem[hh][j].y);
-                                } else {
-                                    best[2 * j] = max(best[2 * j], tv[hh][2 * j]);
-                                    best[2 * j + 1] = max(best[2 * j + 1], tv[hh][2 * j + 1]);
                                 }
                             }
-                        if (h0 + kH >= a.L) {
+                        if (h0 + kH >= args->a.L) {
                             // (read, choose, write back unconditionally: a point that two threads
                             //  hold, at the moved-back end of a slice, gets the same value from both)
                             const int pt0 = chunk_start(c0);
                             uint32_t old[8];
 #pragma unroll
-                            for (int e = 0; e < 8; e++) old[e] = s_time[pt0 + e];
+                            for (int e = 0; e < 8; e++) old[e] = tb.time[pt0 + e];
 #pragma unroll
                             for (int e = 0; e < 8; e++) {
                                 uint32_t b;
                                 if constexpr (kPath == 0) b = (best[e >> 1] >> ((e & 1) * 16)) & 0xffffu;
                                 else b = best[e];
                                 // ties: the earlier composite stays
-                                s_time[pt0 + e] = (uint16_t)((b >> 1) < (old[e] >> 1) ? b : old[e]);
+                                tb.time[pt0 + e] = (uint16_t)((b >> 1) < (old[e] >> 1) ? b : old[e]);
                             }
                         }
                     };
@@ -534,7 +674,7 @@ __global__ __launch_bounds__(kDT, WPS) void traverse_dense_kernel(QueryArgs a, D
                     // under way are only exact in straight-line code): past the last group the reads
                     // repeat the slice's last chunk and the lookups change nothing that is stored.
                     int cc = 0, hc = 0, ci = 0, hi = 0;     // (chunk base, first simple index) of the group to consume / to issue
-                    auto advance = [&](int& c, int& h) { h += kH; if (h >= a.L) { h = 0; c += kChunk; } };
+                    auto advance = [&](int& c, int& h) { h += kH; if (h >= args->a.L) { h = 0; c += kChunk; } };
                     u32x4 pv[kD][kH];
 #pragma unroll
                     for (int d = 0; d < kD; d++) {
@@ -551,36 +691,35 @@ __global__ __launch_bounds__(kDT, WPS) void traverse_dense_kernel(QueryArgs a, D
                         }
                     }
                 };
-                if (T > 1 && (T & (T - 1)) == 0) run(std::integral_constant<int, 0>{});
-                else if (T > 1) run(std::integral_constant<int, 1>{});
-                else run(std::integral_constant<int, 2>{});
+                if ((T & (T - 1)) == 0) run(std::integral_constant<int, 0>{});
+                else run(std::integral_constant<int, 1>{});
             }
             __syncthreads();
             PHASE_END(3);
         }
-        if (misc[dFail]) {      // does not fit the tables: the step-by-step kernel takes the item
+        if (__builtin_amdgcn_readfirstlane((int)misc[dFail])) {      // does not fit the tables: the step-by-step kernel takes the item
             if (tid == 0) {
-                const uint32_t s2 = atomicAdd(a.redo_count, 1u);
-                a.redo_items[s2] = (int32_t)item;
+                const uint32_t s2 = atomicAdd(args->a.redo_count, 1u);
+                args->a.redo_items[s2] = (int32_t)item;
             }
             continue;
         }
 
         // ---- stop step from the histogram of the steps of lane-0 candidates -----------
         const int HW = ((int)maxw + 2) / 2;                 // 32-bit words of the histogram (two steps each)
-        for (int w = tid; w < HW; w += kDT) stage[w] = 0;
+        for (int w = tid; w < HW; w += NT) tb.stage[w] = 0;
         if (tid == 0) { misc[dArmed] = 0xffffffffu; misc[dMaxc] = 0xffffffffu; }
         __syncthreads();
-        for (int pt = tid; pt < n; pt += kDT) {
-            const uint32_t v = s_time[pt];
-            if ((v & 1u) && (v >> 1) != (kNever & 0x7fffu)) atomicAdd(&stage[v >> 2], 1u << (((v >> 1) & 1u) * 16));
+        for (int pt = tid; pt < n; pt += NT) {
+            const uint32_t v = tb.time[pt];
+            if ((v & 1u) && (v >> 1) != (kNever & 0x7fffu)) atomicAdd(&tb.stage[v >> 2], 1u << (((v >> 1) & 1u) * 16));
         }
         __syncthreads();
         {
-            const int per = (HW + kDT - 1) / kDT;           // words per thread, contiguous
+            const int per = (HW + NT - 1) / NT;           // words per thread, contiguous
             const int w0 = tid * per, w1 = min(HW, w0 + per);
             uint32_t sum = 0;
-            for (int w = w0; w < w1; w++) { const uint32_t v = stage[w]; sum += (v & 0xffffu) + (v >> 16); }
+            for (int w = w0; w < w1; w++) { const uint32_t v = tb.stage[w]; sum += (v & 0xffffu) + (v >> 16); }
             uint32_t incl = sum;
 #pragma unroll
             for (int o = 1; o < kWave; o <<= 1) {
@@ -591,10 +730,10 @@ __global__ __launch_bounds__(kDT, WPS) void traverse_dense_kernel(QueryArgs a, D
             __syncthreads();
             uint32_t run = incl - sum;
             for (int w2 = 0; w2 < wave; w2++) run += scan_tmp[w2];
-            const uint32_t need_k = (uint32_t)a.k_stop;
-            const uint32_t need_c = (uint32_t)min((int64_t)0x7fffffff, max((int64_t)1, a.max_cand));
+            const uint32_t need_k = (uint32_t)args->a.k_stop;
+            const uint32_t need_c = (uint32_t)min((int64_t)0x7fffffff, max((int64_t)1, args->a.max_cand));
             for (int w = w0; w < w1; w++) {
-                const uint32_t v = stage[w];
+                const uint32_t v = tb.stage[w];
                 const uint32_t c_lo = run + (v & 0xffffu), c_hi = c_lo + (v >> 16);
                 if (run < need_k && c_lo >= need_k) atomicMin(&misc[dArmed], (uint32_t)(2 * w));
                 else if (c_lo < need_k && c_hi >= need_k) atomicMin(&misc[dArmed], (uint32_t)(2 * w + 1));
@@ -604,11 +743,12 @@ __global__ __launch_bounds__(kDT, WPS) void traverse_dense_kernel(QueryArgs a, D
             }
         }
         __syncthreads();
-        const uint32_t t_armed = misc[dArmed], t_maxc = misc[dMaxc];
+        const uint32_t t_armed = (uint32_t)__builtin_amdgcn_readfirstlane((int)misc[dArmed]);
+        const uint32_t t_maxc = (uint32_t)__builtin_amdgcn_readfirstlane((int)misc[dMaxc]);
         const bool stop = t_armed != 0xffffffffu;
         unsigned long long t_stop = ~0ull;                  // candidates: promoted at a step <= t_stop
         if (stop) {
-            const unsigned long long last_needed = a.stop_at > 0 ? (unsigned long long)(a.stop_at - 1) : 0ull;
+            const unsigned long long last_needed = args->a.stop_at > 0 ? (unsigned long long)(args->a.stop_at - 1) : 0ull;
             const unsigned long long by_count = t_maxc != 0xffffffffu ? (unsigned long long)t_maxc : ~0ull;
             t_stop = max((unsigned long long)t_armed, min(last_needed, by_count));
         }
@@ -617,213 +757,448 @@ __global__ __launch_bounds__(kDT, WPS) void traverse_dense_kernel(QueryArgs a, D
         PHASE_END(4);
 
         // ---- distances of the candidates, k best ---------------------------------------
-        // Every wavefront walks a quarter of the points; a candidate whose packed
-        // (distance, id) does not beat the current k-th best is dropped at once, the others
-        // wait in the wavefront's share of the buffer until the next merge.
-        // Rows of up to 64 (128) elements are read by 16 (32) lanes each, four (two) rows
-        // per load instruction and up to four such loads in flight; the lanes' partial sums
-        // and the order in which they are added are those of wave_row_dists (the lanes a
-        // short row leaves idle there add zeros), so the distances have the same bits.
-        const bool vec4 = rows_vec4(a.data, a.dim);
-        const int chunk = (n + kDWaves - 1) / kDWaves;
-        int at = wave * chunk;                              // next point of this wavefront (wave-uniform)
-        const int at_end = min(n, at + chunk);
-        uint16_t* wl = s_wlist + wave * kWlist;             // this wavefront's candidates, listed 64 points at a time
+        // Every wavefront walks its share of the points and lists its candidates, a batch at a
+        // time; entries that may be among the k best wait in the wavefront's share of the buffer
+        // until the next merge.
+        typedef float v4f __attribute__((ext_vector_type(4)));
+        const bool vec4 = rows_vec4(args->a.data, args->a.dim);
+        const int chunk = (n + kWaves - 1) / kWaves;
+        const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+        const int at_end = min(n, (wave_u + 1) * chunk);
+        int at = wave_u * chunk;                            // next point of this wavefront
+        uint16_t* wl = tb.wlist + wave_u * kWlist;             // this wavefront's candidates
         int list_len = 0, list_pos = 0;
         uint32_t ncand = 0;
         int topn = 0;
-        // end of a round: the wavefronts' pending candidates are merged into the k best;
-        // returns whether any wavefront has points left
-        auto merge_round = [&](int mine, unsigned long long* my_slots) -> bool {
-            for (int j = mine + lane; j < y.quota; j += kWave) my_slots[j] = ~0ull;
-            const bool more = list_pos < list_len || at < at_end;
-            if (lane == 0) {
-                scan_tmp[8 + wave] = (uint32_t)mine;
-                scan_tmp[16 + wave] = more ? 1u : 0u;
-            }
-            // (slots between the k best held so far and the first wavefront's share)
-            for (int j = topn + tid; j < a.kcap; j += kDT) sortbuf[j] = ~0ull;
-            for (int j = a.kcap + kDWaves * y.quota + tid; j < y.sort_cap; j += kDT) sortbuf[j] = ~0ull;
-            __syncthreads();
-            int added = 0, any_more = 0;
-            for (int w2 = 0; w2 < kDWaves; w2++) { added += (int)scan_tmp[8 + w2]; any_more |= (int)scan_tmp[16 + w2]; }
-            if (added > 0) {
-                bitonic_sort_u64_by256(sortbuf, y.sort_cap);
-                topn = min(a.kcap, topn + added);
-            } else {
-                __syncthreads();
-            }
-            return any_more != 0;
-        };
-        auto run_rounds = [&](auto gtag, auto rtag) {
-            constexpr int GL = decltype(gtag)::value;       // lanes per row
-            constexpr int R = decltype(rtag)::value;        // rows per lane group in flight
-            constexpr int NG = kWave / GL;                  // lane groups
-            constexpr int RB = NG * R;                      // rows per batch
-            const int grp = lane / GL, sl = lane & (GL - 1);
-            for (;;) {
-                unsigned long long kth = ~0ull;
-                if (topn >= a.kcap) kth = sortbuf[a.kcap - 1];
-                int mine = 0;                               // entries this wavefront has pending
-                unsigned long long* my_slots = sortbuf + a.kcap + wave * y.quota;
-                for (;;) {
-                    if (list_pos >= list_len) {
-                        if (at >= at_end) break;
-                        const int pt = at + lane;
-                        const uint32_t v = pt < at_end ? (uint32_t)s_time[pt] : 0xffffu;
-                        const bool is_cand = (v >> 1) <= t_lim;
-                        const unsigned long long m = __ballot(is_cand);
-                        if (is_cand) wl[__popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)pt;
-                        list_len = __popcll(m);
-                        list_pos = 0;
-                        at += kWave;
-                        ncand += (uint32_t)list_len;
-                        continue;
-                    }
-                    if (mine + RB > y.quota) break;         // no room for a whole batch: merge first
-                    int pts[R];
-                    bool valid[R];
-                    unsigned long long e[R];
-#pragma unroll
-                    for (int r = 0; r < R; r++) {
-                        const int c = list_pos + r * NG + grp;
-                        valid[r] = c < list_len;
-                        pts[r] = (int)wl[min(c, list_len - 1)];
-                    }
-                    if (a.blind) {      // scored by the promoting step (:498-505), no row is read
-#pragma unroll
-                        for (int r = 0; r < R; r++)
-                            e[r] = ((unsigned long long)(s_time[pts[r]] >> 1) << 32) | (uint32_t)(off + pts[r]);
-                    } else {
-                        const float* rows[R];
-#pragma unroll
-                        for (int r = 0; r < R; r++) rows[r] = a.data + (off + pts[r]) * a.dim;
-                        float d[R];
-                        const float* const (&crows)[R] = rows;
-                        if (R > 2) wave_row_dists_wide<R, 16 / R>(crows, s_q, a.dim, d);  // (only chosen for aligned rows of 512 elements or more)
-                        else wave_row_dists<R>(crows, s_q, a.dim, vec4, d);
-#pragma unroll
-                        for (int r = 0; r < R; r++)
-                            e[r] = ((unsigned long long)__builtin_bit_cast(uint32_t, d[r]) << 32) | (uint32_t)(off + pts[r]);
-                    }
-#pragma unroll
-                    for (int r = 0; r < R; r++) {
-                        const bool keep = valid[r] && sl == 0 && e[r] < kth;
-                        const unsigned long long m = __ballot(keep);
-                        if (keep) my_slots[mine + __popcll(m & ((1ull << lane) - 1ull))] = e[r];
-                        mine += __popcll(m);
-                    }
-                    list_pos += RB;
+        // lists at least `want` candidates, while points are left
+        auto list_more = [&](int want) {
+            while (list_len - list_pos < want && at < at_end) {
+                if (list_pos > 0) {      // what is left moves to the front (one wavefront: its LDS operations keep their order)
+                    const int rest = list_len - list_pos;
+                    const uint16_t v = lane < rest ? wl[list_pos + lane] : (uint16_t)0;
+                    __builtin_amdgcn_wave_barrier();
+                    if (lane < rest) wl[lane] = v;
+                    list_len = rest;
+                    list_pos = 0;
                 }
-                if (!merge_round(mine, my_slots)) break;
+                const int pt = at + lane;
+                const uint32_t v = pt < at_end ? (uint32_t)tb.time[pt] : 0xffffu;
+                const bool is_cand = (v >> 1) <= t_lim;
+                const unsigned long long m = __ballot(is_cand);
+                if (is_cand) wl[list_len + __popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)pt;
+                list_len += __popcll(m);
+                at += kWave;
+                ncand += (uint32_t)__popcll(m);
             }
+            __builtin_amdgcn_wave_barrier();
         };
-        // Rows of at most 4 * GL elements: a batch is 64 candidates, GL lanes read a row (16
-        // bytes each) and every lane group takes GL rows, eight loads in flight per lane; the
-        // GL partial sums a lane ends up with are reduced for all its rows together, which
-        // leaves lane c of the wavefront with the distance of candidate c: one comparison, one
-        // ballot and one store per batch instead of one per row.
-        auto run_tiles = [&](auto gtag) {
-            typedef float v4f __attribute__((ext_vector_type(4)));
+        // Distances of eight rows by one wavefront, all eight reads under way together: the sums and
+        // their order are those of wave_row_dists, level by level; lane l has that of row l >> 3.
+        auto eight_rows = [&](const int (&pts)[8]) -> float {
+            float acc[8];
+            const float* rows[8];                               // (the points are the same for all lanes: addresses in scalar registers)
+            const float* data = args->a.data;
+            const int dim = args->a.dim;
+#pragma unroll
+            for (int r = 0; r < 8; r++) { acc[r] = 0.f; rows[r] = data + (off + __builtin_amdgcn_readfirstlane(pts[r])) * dim; }
+            if (vec4) {
+                for (int j = lane * 4; j < dim; j += kWave * 4) {
+                    v4f x[8];
+#pragma unroll
+                    for (int r = 0; r < 8; r++) x[r] = *reinterpret_cast<const v4f*>(rows[r] + j);
+                    const float q0 = tb.q[j], q1 = tb.q[j + 1], q2 = tb.q[j + 2], q3 = tb.q[j + 3];
+#pragma unroll
+                    for (int r = 0; r < 8; r++) {
+                        float dd = x[r].x - q0; acc[r] = __builtin_fmaf(dd, dd, acc[r]);
+                        dd = x[r].y - q1; acc[r] = __builtin_fmaf(dd, dd, acc[r]);
+                        dd = x[r].z - q2; acc[r] = __builtin_fmaf(dd, dd, acc[r]);
+                        dd = x[r].w - q3; acc[r] = __builtin_fmaf(dd, dd, acc[r]);
+                    }
+                }
+            } else {
+                for (int j = lane; j < dim; j += kWave) {
+                    float x[8];
+#pragma unroll
+                    for (int r = 0; r < 8; r++) x[r] = rows[r][j];
+                    const float qj = tb.q[j];
+#pragma unroll
+                    for (int r = 0; r < 8; r++) { const float dd = x[r] - qj; acc[r] = __builtin_fmaf(dd, dd, acc[r]); }
+                }
+            }
+            float v4[4], v2[2];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const bool up = (lane & 32) != 0;
+                v4[i] = (up ? acc[i + 4] : acc[i]) + lane_xor<32>(up ? acc[i] : acc[i + 4]);
+            }
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const bool up = (lane & 16) != 0;
+                v2[i] = (up ? v4[i + 2] : v4[i]) + lane_xor<16>(up ? v4[i] : v4[i + 2]);
+            }
+            const bool up = (lane & 8) != 0;
+            float v = (up ? v2[1] : v2[0]) + lane_xor<8>(up ? v2[0] : v2[1]);
+            v += lane_xor<4>(v); v += lane_xor<2>(v); v += lane_xor<1>(v);
+            return sqrtf(v);
+        };
+        auto pack = [&](uint32_t score, int pt) { return ((unsigned long long)score << 32) | (uint32_t)(off + pt); };
+
+        // Candidates by their rows' 8-bit codes (rows8.hip).  The distance d~ between coded row and coded
+        // query is off by at most the two coding errors (their sum: err) and by the rounding of its square
+        // (delta), so a candidate more than 2 err + delta's part behind the k-th smallest d~ cannot be
+        // among the k best: the others -- k and some -- are kept, and only their rows are read.
+        // What d~ may be at most, given the k-th smallest:
+        const int rec = args->a.rows8_rec, code_bytes = (args->a.dim + 15) & ~15;
+        const unsigned char* qrec = args->a.query8 + (int64_t)qi * (16 + 2 * code_bytes);
+        enum { kBlind = 1, kRows = 8, kRows16 = 16, kRows32 = 32, kCodes8 = 108, kCodes16 = 116, kCodes64 = 164 };
+        int path = args->a.blind ? kBlind : (!args->y.tiles ? kRows : (args->a.dim <= 64 ? kRows16 : kRows32));
+        float q_scale = 0.f, q_n2 = 0.f, err = 0.f, delta = 0.f;
+        if (args->a.rows8) {
+            if (tid == 0) misc[dUse8] = args->a.rows8_bounds[2 * args->a.B + b] == 0u ? 1u : 0u;     // (others may set it meanwhile: one reads)
+            __syncthreads();
+            const float* qh = reinterpret_cast<const float*>(qrec);
+            q_scale = qh[0]; q_n2 = qh[1];
+            err = __builtin_bit_cast(float, args->a.rows8_bounds[2 * b]) + qh[2];
+            delta = (__builtin_bit_cast(float, args->a.rows8_bounds[2 * b + 1]) + q_n2) * 9.5367431640625e-7f;   // 2^-20
+            q_scale = uniform_f32(q_scale); q_n2 = uniform_f32(q_n2); err = uniform_f32(err); delta = uniform_f32(delta);
+            if (__builtin_amdgcn_readfirstlane((int)misc[dUse8]) != 0 && err < 1e30f && delta < 1e30f)
+                path = code_bytes <= 128 ? kCodes8 : (code_bytes <= 256 ? kCodes16 : kCodes64);
+        }
+        auto limit = [&](float d) {
+            const float part = d * d > 4.0f * delta ? 2.0f * delta / d : 4.0f * sqrtf(delta);
+            return (d + 2.0f * err + part) * 1.0001f;
+        };
+        // One batch of nb candidates (listed at cur) by their codes: G lanes read a record, 16 codes
+        // each; the integer sums are exact.  Lane c has the entry (d~, point) of candidate c.
+        auto batch_codes = [&](auto gtag, const uint16_t* cur, int nb) -> unsigned long long {
+            constexpr int G = decltype(gtag)::value;            // lanes per record
+            constexpr int RB = G < 32 ? G : 32;                 // records per lane group and batch
+            constexpr int CB = kWave / G * RB;                  // candidates per batch
+            constexpr int kInFlight = RB < 8 ? RB : 8;
+            const int grp = lane / G, sl = lane & (G - 1);
+            const bool has = sl * 16 < code_bytes;
+            const int my_off = 16 + (has ? sl * 16 : 0);
+            u32x4 qh = *reinterpret_cast<const u32x4*>(qrec + my_off);
+            u32x4 ql = *reinterpret_cast<const u32x4*>(qrec + code_bytes + my_off);
+            if (!has) qh = ql = u32x4{0, 0, 0, 0};              // (idle lanes add nothing)
+            const unsigned char* base = args->a.rows8 + off * rec;
+            const int mypt = (int)cur[min(lane & (CB - 1), nb - 1)];
+            const float2 head = *reinterpret_cast<const float2*>(base + (uint32_t)mypt * (uint32_t)rec);
+            int acc[RB];
+#pragma unroll
+            for (int r0 = 0; r0 < RB; r0 += kInFlight) {
+                u32x4 x[kInFlight];
+#pragma unroll
+                for (int r = 0; r < kInFlight; r++) {
+                    const int pt = (int)cur[min(grp * RB + r0 + r, nb - 1)];
+                    x[r] = *reinterpret_cast<const u32x4*>(base + ((uint32_t)pt * (uint32_t)rec + (uint32_t)my_off));
+                }
+#pragma unroll
+                for (int r = 0; r < kInFlight; r++) {
+                    int dh = __builtin_amdgcn_sdot4((int)x[r].x, (int)qh.x, 0, false);
+                    dh = __builtin_amdgcn_sdot4((int)x[r].y, (int)qh.y, dh, false);
+                    dh = __builtin_amdgcn_sdot4((int)x[r].z, (int)qh.z, dh, false);
+                    dh = __builtin_amdgcn_sdot4((int)x[r].w, (int)qh.w, dh, false);
+                    int dl = __builtin_amdgcn_sdot4((int)x[r].x, (int)ql.x, dh << 7, false);
+                    dl = __builtin_amdgcn_sdot4((int)x[r].y, (int)ql.y, dl, false);
+                    dl = __builtin_amdgcn_sdot4((int)x[r].z, (int)ql.z, dl, false);
+                    acc[r0 + r] = __builtin_amdgcn_sdot4((int)x[r].w, (int)ql.w, dl, false);
+                }
+            }
+            if constexpr (G > RB) {
+#pragma unroll
+                for (int r = 0; r < RB; r++) acc[r] += lane_xor<32>(acc[r]);
+            }
+            const int dot = group_row_sums<RB>(acc, sl);           // of candidate lane (mod CB)
+            const float d2 = head.y + q_n2 - 2.0f * (head.x * q_scale * (float)dot);
+            const float d = sqrtf(fmaxf(d2, 0.0f));
+            return ((unsigned long long)__builtin_bit_cast(uint32_t, d) << 32) | (uint32_t)mypt;
+        };
+        // The same by whole rows of at most 4 * GL elements: GL lanes read a row (16 bytes each), every
+        // lane group takes GL rows; the partial sums a lane ends up with are reduced for all its rows
+        // together, which leaves lane c of the wavefront with the distance of candidate c.
+        auto batch_rows = [&](auto gtag, const uint16_t* cur, int nb) -> unsigned long long {
             constexpr int GL = decltype(gtag)::value;
-            constexpr int kInFlight = 16;                   // row reads under way per lane
+            constexpr int kInFlight = 8;                        // row reads under way per lane
             const int grp = lane / GL, sl = lane & (GL - 1);
             const int j = sl * 4;
-            const bool has = j < a.dim;
+            const bool has = j < args->a.dim;
             float q0 = 0.f, q1 = 0.f, q2 = 0.f, q3 = 0.f;
-            if (has) { q0 = s_q[j]; q1 = s_q[j + 1]; q2 = s_q[j + 2]; q3 = s_q[j + 3]; }
-            const float* base = a.data + off * a.dim + (has ? j : 0);
-            for (;;) {
-                unsigned long long kth = ~0ull;
-                if (topn >= a.kcap) kth = sortbuf[a.kcap - 1];
-                int mine = 0;
-                unsigned long long* my_slots = sortbuf + a.kcap + wave * y.quota;
-                for (;;) {
-                    // list at least a whole batch, while points are left
-                    while (list_len - list_pos < kWave && at < at_end) {
-                        if (list_pos > 0) {      // what is left moves to the front (one wavefront: its LDS operations keep their order)
-                            const int rest = list_len - list_pos;
-                            const uint16_t v = lane < rest ? wl[list_pos + lane] : (uint16_t)0;
-                            if (lane < rest) wl[lane] = v;
-                            list_len = rest;
-                            list_pos = 0;
-                        }
-                        const int pt = at + lane;
-                        const uint32_t v = pt < at_end ? (uint32_t)s_time[pt] : 0xffffu;
-                        const bool is_cand = (v >> 1) <= t_lim;
-                        const unsigned long long m = __ballot(is_cand);
-                        if (is_cand) wl[list_len + __popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)pt;
-                        list_len += __popcll(m);
-                        at += kWave;
-                        ncand += (uint32_t)__popcll(m);
-                    }
-                    const int nb = min(kWave, list_len - list_pos);
-                    if (nb <= 0) break;
-                    if (mine + kWave > y.quota) break;      // no room for a whole batch: merge first
-                    const uint16_t* cur = wl + list_pos;
-                    float acc[GL];
+            if (has) { q0 = tb.q[j]; q1 = tb.q[j + 1]; q2 = tb.q[j + 2]; q3 = tb.q[j + 3]; }
+            const float* base = args->a.data + off * args->a.dim + (has ? j : 0);
+            float acc[GL];
 #pragma unroll
-                    for (int r0 = 0; r0 < GL; r0 += kInFlight) {
-                        v4f x[kInFlight];
+            for (int r0 = 0; r0 < GL; r0 += kInFlight) {
+                v4f x[kInFlight];
 #pragma unroll
-                        for (int r = 0; r < kInFlight; r++) {
-                            // (lanes beyond the row's end read its head and add nothing: a load
-                            //  under a condition would wait for the loads before it)
-                            const int pt = (int)cur[min(grp * GL + r0 + r, nb - 1)];
-                            x[r] = *reinterpret_cast<const v4f*>(base + pt * a.dim);
-                        }
+                for (int r = 0; r < kInFlight; r++) {
+                    // (lanes beyond the row's end read its head and add nothing: a load
+                    //  under a condition would wait for the loads before it)
+                    const int pt = (int)cur[min(grp * GL + r0 + r, nb - 1)];
+                    x[r] = *reinterpret_cast<const v4f*>(base + pt * args->a.dim);
+                }
 #pragma unroll
-                        for (int r = 0; r < kInFlight; r++) {
-                            float s2 = 0.f;
-                            float dd = x[r].x - q0; s2 = __builtin_fmaf(dd, dd, s2);
-                            dd = x[r].y - q1; s2 = __builtin_fmaf(dd, dd, s2);
-                            dd = x[r].z - q2; s2 = __builtin_fmaf(dd, dd, s2);
-                            dd = x[r].w - q3; s2 = __builtin_fmaf(dd, dd, s2);
-                            acc[r0 + r] = has ? s2 : 0.f;
-                        }
-                    }
-                    const float total = group_row_sums<GL>(acc, sl);      // of candidate grp * GL + sl = lane
-                    const int mypt = (int)cur[min(lane, nb - 1)];
-                    const unsigned long long e =
-                        ((unsigned long long)__builtin_bit_cast(uint32_t, sqrtf(total)) << 32) | (uint32_t)(off + mypt);
-                    const bool keep = lane < nb && e < kth;
+                for (int r = 0; r < kInFlight; r++) {
+                    float s2 = 0.f;
+                    float dd = x[r].x - q0; s2 = __builtin_fmaf(dd, dd, s2);
+                    dd = x[r].y - q1; s2 = __builtin_fmaf(dd, dd, s2);
+                    dd = x[r].z - q2; s2 = __builtin_fmaf(dd, dd, s2);
+                    dd = x[r].w - q3; s2 = __builtin_fmaf(dd, dd, s2);
+                    acc[r0 + r] = has ? s2 : 0.f;
+                }
+            }
+            const float total = group_row_sums<GL>(acc, sl);      // of candidate grp * GL + sl = lane
+            return pack(__builtin_bit_cast(uint32_t, sqrtf(total)), (int)cur[min(lane, nb - 1)]);
+        };
+        // Every wavefront goes through its batches; entries that may still be among the k best go to its share
+        // of the buffer.  What may be is known from a histogram of the scores seen so far (256 bins over
+        // the range of every wavefront's first batch, one for all, without a barrier: a count that is
+        // read late only loosens the cut): the upper edge of the bin that holds the k-th smallest bounds it.  A share that is full
+        // is cleared of what has fallen behind the cut meanwhile; where that makes no room, the round
+        // ends: the shares are sorted in with what is held.  Nearly always there is one such sort, at the end.
+        // Compared by codes, the kept entries get their exact distances before that sort.
+        // Bound by the latency of the records' reads (eight 16-byte reads per lane under way).  12808 candidates
+        // of 128 elements, k = 100, two workgroups per CU: 98 us per item, 207 by whole rows and a sort per
+        // full buffer; 1325 of 512 elements: 69, and 426 by whole rows.
+        constexpr int kBins = 256;
+        uint32_t* hist = tb.stage;
+        unsigned long long cut = ~0ull;                         // entries above it are out
+        unsigned long long pend = ~0ull;                        // lane's entry of a batch that did not fit the share
+        bool have_pend = false, first = true, last = false;
+        float h_lo = 0.f, h_scale = 0.f;                        // (no histogram while the scale is 0)
+        int batches = 0;
+        unsigned long long* res = tb.sortbuf;                      // where the result lies
+        for (;;) {
+            const bool codes = path >= kCodes8;
+            const int front = codes ? args->y.front8 : args->a.kcap, quota = codes ? args->y.quota8 : args->y.quota;
+            const int CB = path == kRows ? 8 : (path == kCodes64 ? 32 : kWave);
+            unsigned long long* my_slots = tb.sortbuf + front + wave_u * quota;
+            auto score = [&](unsigned long long e) {
+                return args->a.blind ? (float)(uint32_t)(e >> 32) : __builtin_bit_cast(float, (uint32_t)(e >> 32));
+            };
+            auto count = [&](bool keep, unsigned long long e) {
+                const int bin = max(0, (int)((score(e) - h_lo) * h_scale));
+                if (keep && bin < kBins) atomicAdd(&hist[bin], 1u);
+            };
+            auto tighten = [&]() {
+                const u32x4 c = reinterpret_cast<const u32x4*>(hist)[lane];
+                const uint32_t c1 = c.x + c.y, c2 = c1 + c.z, upto = wave_scan_u32(c2 + c.w), before = upto - (c2 + c.w);
+                const uint32_t want = (uint32_t)args->a.kcap;
+                const unsigned long long m = __ballot(upto >= want);
+                if (m) {
+                    const int bin = 4 * lane + (before + c.x >= want ? 0 : (before + c1 >= want ? 1 : (before + c2 >= want ? 2 : 3)));
+                    const float edge = (h_lo + (float)(__shfl(bin, __ffsll((long long)m) - 1, kWave) + 1) / h_scale) * 1.00001f;
+                    const uint32_t top = codes ? __builtin_bit_cast(uint32_t, limit(edge))
+                                               : (args->a.blind ? (uint32_t)edge : __builtin_bit_cast(uint32_t, edge));
+                    cut = uniform_u64(min(cut, ((unsigned long long)top << 32) | 0xffffffffull));
+                }
+            };
+            int mine = 0, added = 0;
+            bool any_more = false;
+            // drops what has fallen behind the cut from the wavefront's share
+            auto clear_share = [&]() {
+                int kept = 0;
+                for (int j0 = 0; j0 < mine; j0 += kWave) {
+                    const unsigned long long v = j0 + lane < mine ? my_slots[j0 + lane] : ~0ull;
+                    const bool stay = v != ~0ull && v <= cut;
+                    const unsigned long long m = __ballot(stay);
+                    __builtin_amdgcn_wave_barrier();
+                    if (stay) my_slots[kept + __popcll(m & ((1ull << lane) - 1ull))] = v;
+                    kept += __popcll(m);
+                }
+                __builtin_amdgcn_wave_barrier();
+                mine = kept;
+            };
+            if (!last) {
+                auto push = [&](bool keep, unsigned long long e) -> bool {
                     const unsigned long long m = __ballot(keep);
+                    if (mine + __popcll(m) > quota) return false;
                     if (keep) my_slots[mine + __popcll(m & ((1ull << lane) - 1ull))] = e;
                     mine += __popcll(m);
-                    list_pos += nb;
+                    return true;
+                };
+                if (have_pend) {
+                    if (batches == 1 && h_scale > 0.f) count(pend != ~0ull, pend);      // (the first batch: now there is a histogram)
+                    push(pend != ~0ull && pend <= cut, pend);      // (a share takes a whole batch)
                 }
-                if (!merge_round(mine, my_slots)) break;
+                have_pend = false;
+                for (;;) {
+                    list_more(CB);
+                    const int nb = min(CB, list_len - list_pos);
+                    if (nb <= 0) break;
+                    const uint16_t* cur = wl + list_pos;
+                    using std::integral_constant;
+                    unsigned long long e;
+                    bool valid = lane < nb;
+                    // (opaque, or the compiler makes a copy of the whole loop, sorts included, for every path)
+                    int how = path;
+                    asm volatile("" : "+v"(how));
+                    how = __builtin_amdgcn_readfirstlane(how);
+                    fresh_thread_ids();      // (nor are lane-derived addresses of all paths kept across the batches)
+                    if (how == kCodes8) e = batch_codes(integral_constant<int, 8>{}, cur, nb);
+                    else if (how == kCodes16) e = batch_codes(integral_constant<int, 16>{}, cur, nb);
+                    else if (how == kCodes64) e = batch_codes(integral_constant<int, 64>{}, cur, nb);
+                    else if (how == kRows16) e = batch_rows(integral_constant<int, 16>{}, cur, nb);
+                    else if (how == kRows32) e = batch_rows(integral_constant<int, 32>{}, cur, nb);
+                    else if (how == kRows) {
+                        int pts[8];
+#pragma unroll
+                        for (int r = 0; r < 8; r++) pts[r] = (int)cur[min(r, nb - 1)];
+                        const float d = eight_rows(pts);
+                        e = pack(__builtin_bit_cast(uint32_t, d), (int)cur[min(lane >> 3, nb - 1)]);
+                        valid = (lane & 7) == 0 && (lane >> 3) < nb;
+                    } else {      // blind: scored by the promoting step (:498-505), no row is read
+                        const int pt = (int)cur[min(lane, nb - 1)];
+                        e = pack((uint32_t)tb.time[pt] >> 1, pt);
+                    }
+                    list_pos += nb;
+                    batches++;
+                    bool keep = valid && e <= cut;
+                    if (first) { pend = keep ? e : ~0ull; have_pend = true; break; }
+                    if (h_scale > 0.f) {
+                        count(keep, e);
+                        if (batches <= 4 || (batches & 3) == 0) {
+                            tighten();
+                            keep = keep && e <= cut;
+                        }
+                    }
+                    if (!push(keep, e)) {
+                        clear_share();
+                        if (!push(keep, e)) { pend = keep ? e : ~0ull; have_pend = true; break; }
+                    }
+                }
+                if (first) {      // the range of the histogram, and an empty one
+                    const uint32_t bits = have_pend && pend != ~0ull ? __builtin_bit_cast(uint32_t, score(pend)) : 0x7fffffffu;
+                    const uint32_t least = wave_min_u32(bits);
+                    const int most = wave_max_i32(bits == 0x7fffffffu ? 0 : (int)bits);
+                    if (lane == 0) { scan_tmp[24 + wave] = least; scan_tmp[40 + wave] = (uint32_t)most; }
+                    for (int j = tid; j < kBins; j += NT) hist[j] = 0;
+                    __syncthreads();
+                    uint32_t lo = 0x7fffffffu, hi = 0;
+                    for (int w2 = 0; w2 < kWaves; w2++) { lo = min(lo, scan_tmp[24 + w2]); hi = max(hi, scan_tmp[40 + w2]); }
+                    const float f_lo = __builtin_bit_cast(float, lo), width = __builtin_bit_cast(float, hi) - f_lo;
+                    if (lo < hi && hi < kInfBits && width > 1e-30f && width < 1e30f) { h_lo = uniform_f32(f_lo); h_scale = uniform_f32((float)kBins / width); }
+                    first = false;
+                    continue;
+                }
+                if (lane == 0) {
+                    scan_tmp[8 + wave] = (uint32_t)mine;
+                    scan_tmp[16 + wave] = have_pend || list_pos < list_len || at < at_end ? 1u : 0u;
+                }
+                __syncthreads();
+                for (int w2 = 0; w2 < kWaves; w2++) { added += (int)scan_tmp[8 + w2]; any_more = any_more || scan_tmp[16 + w2] != 0u; }
+                added = __builtin_amdgcn_readfirstlane(added);
+                any_more = __builtin_amdgcn_readfirstlane((int)any_more) != 0;
             }
-        };
-        {
-            using std::integral_constant;
-            if (y.tiles && vec4 && a.dim <= 64 && y.quota >= kWave) run_tiles(integral_constant<int, 16>{});
-            else if (y.tiles && vec4 && a.dim <= 128 && y.quota >= kWave) run_tiles(integral_constant<int, 32>{});
-            // long rows: sixteen 16-byte reads in flight per lane, as whole 1 KiB pieces of as few rows as hold them
-            else if (vec4 && !a.blind && a.dim == 512 && y.quota >= 8) run_rounds(integral_constant<int, 64>{}, integral_constant<int, 8>{});
-            else if (vec4 && !a.blind && a.dim > 512 && y.quota >= 4) run_rounds(integral_constant<int, 64>{}, integral_constant<int, 4>{});
-            else run_rounds(integral_constant<int, 64>{}, integral_constant<int, 2>{});
+            int words = args->y.sort_cap;
+            res = tb.sortbuf;
+            bool whole = false;                                 // one round did: what is left fits the tables' room, side by side
+            int left = topn;                                    // entries to be given their exact distances (codes)
+            if (!last && !any_more && topn == 0) {
+                if (h_scale > 0.f) tighten();
+                clear_share();
+                if (lane == 0) scan_tmp[wave] = (uint32_t)mine;
+                __syncthreads();
+                int base = 0;
+                added = 0;
+                for (int w2 = 0; w2 < kWaves; w2++) { const int c = (int)scan_tmp[w2]; if (w2 < wave_u) base += c; added += c; }
+                added = __builtin_amdgcn_readfirstlane(added);
+                int np = added <= kWave ? kWave : NT;
+                while (np < added) np <<= 1;
+                if (np * 8 <= args->y.off_wlist - args->y.off_stage) {
+                    whole = true;
+                    left = added;
+                    words = np;
+                    res = reinterpret_cast<unsigned long long*>(tb.stage);
+                    for (int j = lane; j < mine; j += kWave) res[base + j] = my_slots[j];
+                    for (int j = added + tid; j < np; j += NT) res[j] = ~0ull;
+                    if (codes) __syncthreads();
+                }
+            }
+            if (!whole && !last) {
+                for (int j = mine + lane; j < quota; j += kWave) my_slots[j] = ~0ull;
+                for (int j = topn + tid; j < front; j += NT) tb.sortbuf[j] = ~0ull;
+                for (int j = front + kWaves * quota + tid; j < args->y.sort_cap; j += NT) tb.sortbuf[j] = ~0ull;
+            } else if (codes) {
+                for (int j0 = wave * 8; j0 < left; j0 += 8 * kWaves) {
+                    int pts[8];
+#pragma unroll
+                    for (int r = 0; r < 8; r++) pts[r] = (int)(uint32_t)res[min(j0 + r, left - 1)];
+                    const float d = eight_rows(pts);
+                    const int j = j0 + (lane >> 3);
+                    int mypt = pts[0];
+#pragma unroll
+                    for (int r = 1; r < 8; r++) mypt = (lane >> 3) == r ? pts[r] : mypt;
+                    if ((lane & 7) == 0 && j < left) res[j] = pack(__builtin_bit_cast(uint32_t, d), mypt);
+                }
+                if (last) for (int j = topn + tid; j < args->y.sort_cap; j += NT) tb.sortbuf[j] = ~0ull;
+            }
+            if (NT > kWave && words == kWave) {
+                __syncthreads();
+                if (wave == 0) res[lane] = wave_sort_u64(res[lane]);
+                __syncthreads();
+            } else {
+                bitonic_sort_u64_by<NT, NT == 64 ? 4 : (IPT > 9 ? 1 : 2)>(res, words, tid);
+            }
+            if (whole) { topn = min(added, args->a.kcap); break; }
+            topn += added;
+            if (last) { topn = min(topn, args->a.kcap); break; }
+            if (topn >= args->a.kcap) {
+                const unsigned long long kth = tb.sortbuf[args->a.kcap - 1];
+                if (codes) {
+                    cut = ((unsigned long long)__builtin_bit_cast(uint32_t, limit(__builtin_bit_cast(float, (uint32_t)(kth >> 32)))) << 32) | 0xffffffffull;
+                    cut = uniform_u64(cut);
+                    int lo = args->a.kcap, hi = topn;                     // words ascend: the first one past the cut
+                    while (lo < hi) {
+                        const int mid = (lo + hi) >> 1;
+                        if (tb.sortbuf[mid] <= cut) lo = mid + 1; else hi = mid;
+                    }
+                    topn = __builtin_amdgcn_readfirstlane(lo);
+                } else {
+                    cut = uniform_u64(kth);
+                    topn = args->a.kcap;
+                }
+            }
+            __syncthreads();
+            if (topn > front) {
+                // more has to be kept than the buffer holds: this partition's rows lie too close together for
+                // their codes; whole rows from now on
+                if (tid == 0) args->a.rows8_bounds[2 * args->a.B + b] = 1u;
+                path = !args->y.tiles ? kRows : (args->a.dim <= 64 ? kRows16 : kRows32);
+                at = wave_u * chunk;
+                list_len = list_pos = topn = batches = 0;
+                ncand = 0;
+                have_pend = false;
+                first = true;
+                h_scale = 0.f;
+                cut = ~0ull;
+                continue;
+            }
+            if (!any_more) {
+                if (!codes) break;
+                last = true;
+            }
         }
         if (lane == 0) atomicAdd(&misc[dCand], ncand);
-        for (int j = tid; j < a.kcap; j += kDT) part_out[j] = j < topn ? sortbuf[j] : ~0ull;
+        for (int j = tid; j < args->a.kcap; j += NT) part_out[j] = j < topn ? res[j] : ~0ull;
         PHASE_END(5);
-        if (a.phase_ticks && tid == 0) atomicAdd(&a.phase_ticks[9], 1ull);
+        if (args->a.phase_ticks && tid == 0) atomicAdd(&args->a.phase_ticks[9], 1ull);
 
         // ---- hints for the batch kernel's routing, counters -----------------------------
         __syncthreads();
-        const unsigned long long bound = (unsigned long long)n * a.L * T;
+        const unsigned long long bound = (unsigned long long)n * args->a.L * T;
         unsigned long long steps = min(bound, maxw + 1);
         if (stop) steps = min(t_stop + 1, steps);
-        if (a.stop_hint && tid == 0 && stop) record_stop(a.stop_hint, a.B, b, qi, (float)(t_stop + 1), (float)misc[dCand]);
-        if (a.counters) {
+        if (args->a.stop_hint && tid == 0 && stop) record_stop(args->a.stop_hint, args->a.B, b, qi, (float)(t_stop + 1), (float)misc[dCand]);
+        if (args->a.counters) {
             probes = wave_sum_u32(probes);
             if (lane == 0) atomicAdd(&misc[dProbes], probes);
             __syncthreads();
             if (tid == 0) {
-                atomicAdd(&a.counters[(int64_t)qi * 4 + 0], (unsigned long long)n * I);
-                atomicAdd(&a.counters[(int64_t)qi * 4 + 1], (unsigned long long)misc[dCand]);
-                atomicAdd(&a.counters[(int64_t)qi * 4 + 2], (unsigned long long)misc[dProbes]);
-                atomicAdd(&a.counters[(int64_t)qi * 4 + 3], steps);
+                atomicAdd(&args->a.counters[(int64_t)qi * 4 + 0], (unsigned long long)n * I);
+                atomicAdd(&args->a.counters[(int64_t)qi * 4 + 1], (unsigned long long)misc[dCand]);
+                atomicAdd(&args->a.counters[(int64_t)qi * 4 + 2], (unsigned long long)misc[dProbes]);
+                atomicAdd(&args->a.counters[(int64_t)qi * 4 + 3], steps);
             }
         }
     }
@@ -836,10 +1211,10 @@ __global__ __launch_bounds__(kDT, WPS) void traverse_dense_kernel(QueryArgs a, D
 bool dense_traversal_supported(const QueryArgs& a, size_t* lds_bytes) {
     if (!a.inv || a.ppb > 32766 || a.T < 1) return false;
     if (a.M > 64 || a.L > 64 || a.kcap > 512 || (int64_t)a.L * a.N >= 0x7fffffffLL) return false;
-    if (dense_ipt_for(dense_max_windows(a)) == 0) return false;
     if (dense_max_windows(a) >= 0x7fff || a.ppb + (int64_t)a.T >= 65536) return false;
     if (a.xcds < 1 || a.xcds > 32 || (int64_t)a.nq * (a.B + a.xcds) >= 0x7fffffffLL) return false;
     const DenseLayout y = make_dense_layout(a);
+    if (y.ipt == 0) return false;
     if (lds_bytes) *lds_bytes = y.lds_bytes;
     return y.lds_bytes <= 160 * 1024 - 512;
 }
@@ -851,29 +1226,37 @@ int query_dense_items(const QueryArgs& a_in, hipStream_t s) {
     a.q_first = 0;
     a.q_count = a.nq;
     // enough resident workgroups to fill the device, each striding over its die's items
-    const int per_cu = (int)max((size_t)1, min((size_t)4, (size_t)(160 * 1024) / y.lds_bytes));
+    const int by_regs = (y.ipt > 9 ? 512 : 1024) / y.nt;
+    const int per_cu = (int)max((size_t)1, min((size_t)by_regs, kLdsBytes / y.lds_bytes));
     int64_t per_xcd = (int64_t)32 * per_cu * 2;
     const int64_t most = a.dense_items && a.mode != 3 ? (int64_t)a.dense_cap
                                                       : block_items(a.xcds, a.B, a.nq) / a.xcds;
     per_xcd = max((int64_t)1, min(per_xcd, most));
     const unsigned grid = (unsigned)(per_xcd * a.xcds);
-#define DCIH_DENSE(IPT, WPS)                                                                        \
+#define DCIH_DENSE(NT, IPT, WAVES)                                                                 \
     do {                                                                                         \
         static DeviceOnce once;                                                                  \
         const int rc_attr = once.run([]() -> int {                                               \
-            DCIH_HIP(hipFuncSetAttribute((const void*)traverse_dense_kernel<IPT, WPS>,             \
+            DCIH_HIP(hipFuncSetAttribute((const void*)traverse_dense_kernel<NT, IPT, WAVES>,      \
                                          hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024)); \
             return 0;                                                                            \
         });                                                                                      \
         if (rc_attr) return rc_attr;                                                             \
-        hipLaunchKernelGGL((traverse_dense_kernel<IPT, WPS>), dim3(grid), dim3(kDT), y.lds_bytes, s, a, y); \
+        hipLaunchKernelGGL((traverse_dense_kernel<NT, IPT, WAVES>), dim3(grid), dim3(NT), y.lds_bytes, s, DenseArgs{a, y}); \
     } while (0)
-    if (y.ipt == 9 && per_cu >= 3) DCIH_DENSE(9, 3);
-    else if (y.ipt == 9) DCIH_DENSE(9, 2);
-    else if (y.ipt == 17) DCIH_DENSE(17, 2);
-    else if (y.ipt == 25) DCIH_DENSE(25, 2);
-    else if (y.ipt == 33) DCIH_DENSE(33, 2);
-    else DCIH_DENSE(41, 2);
+    if (y.nt == 64) {
+        if (y.ipt == 5) DCIH_DENSE(64, 5, 4); else DCIH_DENSE(64, 9, 4);
+    } else if (y.nt == 512) {
+        if (y.ipt == 5) DCIH_DENSE(512, 5, 4); else if (y.ipt == 9) DCIH_DENSE(512, 9, 4); else DCIH_DENSE(512, 21, 2);
+    } else if (y.ipt == 5) {
+        DCIH_DENSE(256, 5, 4);
+    } else if (y.ipt == 9) {
+        DCIH_DENSE(256, 9, 4);
+    } else if (y.ipt == 25) {
+        DCIH_DENSE(256, 25, 2);
+    } else {
+        DCIH_DENSE(256, 33, 2);
+    }
 #undef DCIH_DENSE
     DCIH_HIP(hipGetLastError());
     return 0;
