@@ -151,6 +151,7 @@ struct dcih_index {
     int hint_k = 0, hint_outer = 0, hint_T = 0, hint_maxc = 0;   // query shape the hints belong to
     int traversal = 0;                  // DCIH_OPT_TRAVERSAL value
     int dense_min_promos = 160;         // DCIH_OPT_DENSE_MIN_PROMOTIONS value
+    int dense_by_cost = 1;              // until that option is set
     int append_mode = 0;                // DCIH_OPT_APPEND value
     unsigned long long* d_phase_ticks = nullptr;   // optional profile of the batch kernel
     // grow-only workspace: query scratch, and the unsorted keys during a build
@@ -641,6 +642,8 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     a.wide_items = nullptr; a.wide_count = nullptr; a.wide_cap = 0;
     a.block_list = nullptr; a.block_list_count = nullptr; a.full_tables = 0;
     a.dense_min_promos = h->dense_min_promos;
+    a.dense_by_cost = h->dense_by_cost;
+    a.hand_over_at = 0;
     a.rows8 = nullptr; a.rows8_rec = 0; a.rows8_bounds = nullptr; a.query8 = nullptr;
     a.phase_ticks = h->d_phase_ticks;
     // the hints describe where traversals of one query shape stop; forget them when it
@@ -736,7 +739,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     const size_t redo_bytes = align_up((size_t)num_queries * block_size * sizeof(int32_t));
     // per die one list of the items the batch kernel leaves to the dense kernel
     a.dense_cap = (int64_t)num_queries * (block_size / h->xcds + 1) + 64;
-    const bool dense_lists = h->traversal == 0 && h->dense_min_promos > 0 && !blind &&
+    const bool dense_lists = h->traversal == 0 && h->dense_min_promos > 0 &&
                              dense_traversal_supported(a, nullptr) && block_traversal_supported(a, nullptr);
     const size_t dense_bytes = dense_lists ? align_up((size_t)h->xcds * a.dense_cap * sizeof(int32_t)) : 0;
     // (the second pass may have to take every item, up to what one launch of 256-thread workgroups covers)
@@ -855,6 +858,7 @@ int dcih_set_option(dcih_index* h, int option, int value) {
     }
     if (option == DCIH_OPT_DENSE_MIN_PROMOTIONS && value >= 0) {
         h->dense_min_promos = value;
+        h->dense_by_cost = 0;
         return DCIH_OK;
     }
     if (option == DCIH_OPT_APPEND && value >= 0 && value <= 2) {

@@ -79,6 +79,8 @@ struct QueryArgs {
     int32_t* dense_items;    // null, or [xcds][dense_cap]
     uint32_t* dense_count;   // [xcds]
     int64_t dense_cap;
+    int dense_by_cost;       // 1: the estimates below decide, too, and say when an item is handed over
+    int hand_over_at;        // promotions from which the batch kernel hands an item over
     int dense_min_promos;    // promotions per (query, partition) from which the dense kernel is the cheaper one
     // second pass of the batch kernel: items that outgrow its compact per-item tables are listed and
     // taken up again by the variant with the full tables
@@ -111,6 +113,22 @@ inline double expected_promotions(const QueryArgs& a) {
     const double f = fmin(1.0, (double)a.stop_at / fmax(1.0, windows));
     const double by_steps = fmin((double)a.ppb * pow(f, (double)a.L), (double)a.max_cand * (double)a.T);
     return fmax((double)a.k_stop * (double)a.T, by_steps);
+}
+// What the two kernels take, in us on an MI355X, fitted to 450 shapes of 24 to 4000 points per partition
+// (T 2 to 64, L 7 and 15, 400 and 20000 items, Gaussian rows): a time one item takes from end to end, and
+// a time per item once they fill the device.  The dense kernel's grow with the windows it ranks and the
+// points it looks up, the batch kernel's with the promotions it replays.
+struct TraversalCosts { double dense_item, batch_item, batch_per_promotion, dense, batch; };
+inline TraversalCosts traversal_costs(const QueryArgs& a, double promotions) {
+    TraversalCosts c;
+    const double ppb = (double)a.ppb, windows = (double)a.L * (ppb / (double)a.T + 3.0);
+    const double size = (double)a.M / 2.0, length = (double)a.L / 7.0, items = (double)a.nq * (double)a.B;
+    c.dense_item = (0.0086 + 1.8e-5 * windows + 1.1e-6 * (double)a.L * ppb) * size;
+    c.batch_per_promotion = 1.37e-3 * length * size;
+    c.batch_item = 0.0063 * length * size + c.batch_per_promotion * promotions;
+    c.dense = 45.0 + (0.0115 * windows + 0.005 * ppb) * size + items * c.dense_item;
+    c.batch = 153.0 + 7.0 * promotions * length * sqrt(length) * size + items * c.batch_item;
+    return c;
 }
 // The query scratch keeps its list lengths in 64 consecutive words that one kernel clears: the
 // step-by-step kernel's redo list, one hand-over list per die (up to 32), and in the last word

@@ -433,11 +433,18 @@ size_t query_gscratch_bytes(const QueryArgs& a) {
     return (size_t)traverse_grid(a, y) * (size_t)y.counter_words * 4;
 }
 
-// Left to choose: from the number of promotions at which the dense kernel is the cheaper one, every
-// item goes straight to it (no hints needed: also a first call is routed right).
+// Left to choose: from the number of promotions at which the dense kernel is the cheaper one for sure,
+// and where it is estimated to be, every item goes straight to it (no hints needed: also a first call is
+// routed right).  The estimates mostly decide for small partitions (69 points, L = 7, 390 items: 26 us
+// against the batch kernel's 156) and for calls of few items, which wait for the batch kernel's chain of epochs.
 bool takes_dense_kernel(const QueryArgs& a) {
     if (a.mode == 3) return true;
-    return a.mode == 0 && !a.blind && a.dense_min_promos > 0 && expected_promotions(a) >= (double)a.dense_min_promos;
+    if (a.mode != 0 || a.dense_min_promos <= 0) return false;
+    const double promotions = fmin(expected_promotions(a), (double)a.ppb);
+    if (promotions >= (double)a.dense_min_promos) return true;
+    if (!a.dense_by_cost) return false;
+    const TraversalCosts c = traversal_costs(a, promotions);
+    return c.dense < c.batch;
 }
 
 int merge_lists(const QueryArgs& a, hipStream_t s) {
@@ -476,6 +483,16 @@ int query(const QueryArgs& a_in, hipStream_t s, hipEvent_t* ev, bool* ran) {
     if (a.mode == 3 && !can_dense)
         return fail(-4, "query: this shape does not fit the dense traversal kernel");
     if (can_dense && takes_dense_kernel(a)) a.mode = 3;
+    // An item that is already under way in the batch kernel is worth moving only from twice the number of
+    // promotions at which a whole call is routed to the dense kernel: below that, finishing it there is
+    // cheaper than starting over here.  By cost: from one and a half times the promotions that take as long as the
+    // dense kernel takes for all (1000 points, T = 2, L = 15, k = 1, 20000 items: 1.8 ms, 13.5 ms at a fixed 320;
+    // at one half of them calls whose traversals mostly stop soon after take up to twice as long).
+    a.hand_over_at = 2 * a.dense_min_promos;
+    if (a.dense_by_cost) {
+        const TraversalCosts c = traversal_costs(a, 0.0);
+        a.hand_over_at = (int)fmin((double)a.hand_over_at, fmax(16.0, 1.5 * c.dense_item / c.batch_per_promotion));
+    }
     const bool use_block = a.mode != 1 && a.mode != 3 && can_block;
     // the batch kernel hands items that need many promotions to the dense kernel
     if (!(use_block && a.mode == 0 && can_dense && a.dense_items && a.dense_min_promos > 0)) {
@@ -485,7 +502,8 @@ int query(const QueryArgs& a_in, hipStream_t s, hipEvent_t* ev, bool* ran) {
         const int rc = allow_full_lds();
         if (rc) return rc;
     }
-    {   // zero the counters and the list lengths with a kernel (safe under graph capture);
+    const bool lists = a.mode != 3;         // the dense kernel alone leaves no item to another
+    if (lists || a.counters) {   // zero the counters and the list lengths with a kernel (safe under graph capture);
         // the dense lists' lengths follow the hand-over list's
         const int64_t cells = a.counters ? (int64_t)a.nq * 4 : 0;
         hipLaunchKernelGGL(zero_u64_kernel, dim3((unsigned)max((int64_t)1, min((int64_t)1024, (cells + 255) / 256))),
@@ -512,7 +530,9 @@ int query(const QueryArgs& a_in, hipStream_t s, hipEvent_t* ev, bool* ran) {
             if (ev) (void)hipEventRecord(ev[2], s);
             if (ran) ran[1] = true;
         }
-        // whatever those kernels handed back goes through the step-by-step kernel
+    }
+    if (use_block) {
+        // whatever the batch kernel handed back goes through the step-by-step kernel
         a.item_list = a.redo_items;
         a.item_count = a.redo_count;
         if (y.lds_counters) {
@@ -523,7 +543,7 @@ int query(const QueryArgs& a_in, hipStream_t s, hipEvent_t* ev, bool* ran) {
             const int64_t grid = min(traverse_grid(a, y), (int64_t)1024);
             hipLaunchKernelGGL(traverse_kernel<false>, dim3((unsigned)grid), dim3(kWave), y.lds_bytes, s, a, y);
         }
-    } else {
+    } else if (a.mode != 3) {
         const int64_t grid = traverse_grid(a, y);
         if (y.lds_counters) {
             hipLaunchKernelGGL(traverse_kernel<true>, dim3((unsigned)grid), dim3(kWave), y.lds_bytes, s, a, y);

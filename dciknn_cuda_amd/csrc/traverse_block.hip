@@ -248,10 +248,7 @@ __device__ __forceinline__ void traverse_block_item(const QueryArgs& a, const Bl
     // traversal itself has gone that far.  Which kernel finishes an item never shows in
     // the results.
     const bool may_hand_over = a.dense_items != nullptr && a.dense_min_promos > 0;
-    // An item that is already under way here is worth moving only from twice the number of
-    // promotions at which a whole call is routed to the dense kernel: below that, finishing
-    // it here is cheaper than starting over there.
-    const int64_t hand_over_at = 2 * (int64_t)a.dense_min_promos;
+    const int64_t hand_over_at = a.hand_over_at;
     auto hand_to_dense = [&]() {
         if (threadIdx.x == 0) {
             const int x = (int)(blockIdx.x % a.xcds);

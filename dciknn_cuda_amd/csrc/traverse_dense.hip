@@ -38,7 +38,7 @@ namespace {
 constexpr uint32_t kNever = 0xffffu;     // step field of a point that is never promoted
 
 enum DMisc {   // 32-bit scalars shared by the workgroup
-    dWin = 0, dFail, dArmed, dMaxc, dCand, dProbes, dMore, dOr, dAnd, dMaxW, dMaxBits, dUse8,
+    dWin = 0, dArmed, dMaxc, dCand, dProbes, dMore, dOr, dAnd, dMaxW, dMaxBits, dUse8,
     dMiscWords = 16
 };
 
@@ -71,7 +71,7 @@ constexpr int dense_bucket_bits(int cap) {
 constexpr int kWlist = 2 * kWave;        // candidates a wavefront keeps listed
 
 // Upper bound of the windows of one composite index: per simple index at most
-// ceil((p+1)/T) + floor((n+T-3-p)/T) + 1 <= n/T + 3.
+// ceil((p+1)/T) + floor((n+T-3-p)/T) + 1 <= n/T + 3.  (A layout holds that many, so every item fits it.)
 int64_t dense_max_windows(const QueryArgs& a) { return (int64_t)a.L * (a.ppb / a.T + 3); }
 
 DenseLayout dense_layout_for(const QueryArgs& a, int nt, int ipt) {
@@ -364,12 +364,10 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
                     misc[dMaxBits] = 0;
                     tb.seg[2 * args->a.L] = total;
                     misc[dWin] = (uint32_t)total;
-                    if (total > NT * IPT || total >= 0x7fff) misc[dFail] = 1;
                     misc[dOr] = 0; misc[dAnd] = 0xffffffffu;
                 }
             }
             __syncthreads();
-            if (__builtin_amdgcn_readfirstlane((int)misc[dFail])) break;
             const int W = __builtin_amdgcn_readfirstlane((int)misc[dWin]);
             maxw = max(maxw, (unsigned long long)W);
 
@@ -697,14 +695,6 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
             __syncthreads();
             PHASE_END(3);
         }
-        if (__builtin_amdgcn_readfirstlane((int)misc[dFail])) {      // does not fit the tables: the step-by-step kernel takes the item
-            if (tid == 0) {
-                const uint32_t s2 = atomicAdd(args->a.redo_count, 1u);
-                args->a.redo_items[s2] = (int32_t)item;
-            }
-            continue;
-        }
-
         // ---- stop step from the histogram of the steps of lane-0 candidates -----------
         const int HW = ((int)maxw + 2) / 2;                 // 32-bit words of the histogram (two steps each)
         for (int w = tid; w < HW; w += NT) tb.stage[w] = 0;
