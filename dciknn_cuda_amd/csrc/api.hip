@@ -148,6 +148,7 @@ struct dcih_index {
     bool used_any = false, used_many = false;
     bool cleared_behind = false;        // dcih_clear did not wait for work under way on used_stream
     float* d_stop_hint = nullptr;       // [3][block_size] epoch-size hints learnt from earlier queries
+    bool hints_clear = false;           // as the build leaves them: no query has run
     int hint_k = 0, hint_outer = 0, hint_T = 0, hint_maxc = 0;   // query shape the hints belong to
     int traversal = 0;                  // DCIH_OPT_TRAVERSAL value
     int dense_min_promos = 160;         // DCIH_OPT_DENSE_MIN_PROMOTIONS value
@@ -452,6 +453,7 @@ static int sort_into(dcih_index* h, int which, const float* d_keys, int64_t key_
     h->n = num_points;
     h->block_size = block_size;
     h->hint_k = h->hint_outer = h->hint_T = h->hint_maxc = 0;
+    h->hints_clear = true;
     return DCIH_OK;
 }
 
@@ -640,22 +642,26 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     a.xcds = h->xcds; a.q_first = 0; a.q_count = num_queries;
     a.dense_items = nullptr; a.dense_count = nullptr; a.dense_cap = 0;
     a.wide_items = nullptr; a.wide_count = nullptr; a.wide_cap = 0;
-    a.block_list = nullptr; a.block_list_count = nullptr; a.full_tables = 0;
+    a.block_list = nullptr; a.block_list_count = nullptr; a.full_tables = a.few_items = 0;
     a.dense_min_promos = h->dense_min_promos;
     a.dense_by_cost = h->dense_by_cost;
     a.hand_over_at = 0;
+    a.expect_steps = a.expect_promotions = 0.0f;
     a.rows8 = nullptr; a.rows8_rec = 0; a.rows8_bounds = nullptr; a.query8 = nullptr;
     a.phase_ticks = h->d_phase_ticks;
     // the hints describe where traversals of one query shape stop; forget them when it
     // changes (cleared by a kernel: a memset node is not safe in a captured graph)
     if (h->hint_k != num_neighbours || h->hint_outer != num_outer_iterations ||
         h->hint_T != thread_size || h->hint_maxc != max_num_candidates) {
-        const int rc = zero_words64(h->d_stop_hint, (int64_t)(((size_t)3 * block_size * sizeof(float) + 7) / 8), s);
-        if (rc) return rc;
+        if (!h->hints_clear) {
+            const int rc = zero_words64(h->d_stop_hint, (int64_t)(((size_t)3 * block_size * sizeof(float) + 7) / 8), s);
+            if (rc) return rc;
+        }
         h->hint_k = num_neighbours; h->hint_outer = num_outer_iterations;
         h->hint_T = thread_size; h->hint_maxc = max_num_candidates;
         a.hints_cold = 1;
     }
+    h->hints_clear = false;
     a.stop_hint = h->d_stop_hint;
     a.N = h->n;
     a.ppb = (h->n + block_size - 1) / block_size;

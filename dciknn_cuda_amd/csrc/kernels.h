@@ -89,6 +89,8 @@ struct QueryArgs {
     int64_t wide_cap;
     const int32_t* block_list;        // null = the launch covers queries q_first .. q_first + q_count; else workgroup w takes block_list[w]
     const uint32_t* block_list_count; // ... for w below this number
+    float expect_steps, expect_promotions;      // the batch kernel's first guess at where a full partition's traversal stops
+    int few_items;           // 1: the batch kernel gives every item four wavefronts
     int full_tables;         // 1: the batch kernel keeps its per-point flags as bits whatever the shape
     // dense kernel: the rows' and the queries' 8-bit codes (rows8.hip; null = read whole rows)
     const unsigned char* rows8;      // [N][rows8_rec]
@@ -113,6 +115,14 @@ inline double expected_promotions(const QueryArgs& a) {
     const double f = fmin(1.0, (double)a.stop_at / fmax(1.0, windows));
     const double by_steps = fmin((double)a.ppb * pow(f, (double)a.L), (double)a.max_cand * (double)a.T);
     return fmax((double)a.k_stop * (double)a.T, by_steps);
+}
+// About the step at which a partition's traversal stops, by the same reasoning (0.55 to 1.0 of this in
+// Gaussian rows, unit vectors, manifolds and mixtures of 0.4 to 1 million rows, mostly above 0.9).
+inline double expected_stop(const QueryArgs& a) {
+    const double windows = (double)a.L * ((double)a.ppb / (double)a.T);
+    auto fraction = [&](double promotions) { return fmin(1.0, pow(promotions * (double)a.T / (double)a.ppb, 1.0 / (double)a.L)); };
+    const double by_steps = fmin((double)a.stop_at / fmax(1.0, windows), fraction((double)a.max_cand));
+    return windows * fmin(1.0, fmax(fraction((double)a.k_stop), by_steps));
 }
 // What the two kernels take, in us on an MI355X, fitted to 450 shapes of 24 to 4000 points per partition
 // (T 2 to 64, L 7 and 15, 400 and 20000 items, Gaussian rows): a time one item takes from end to end, and

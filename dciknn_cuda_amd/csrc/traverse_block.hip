@@ -264,6 +264,8 @@ __device__ __forceinline__ void traverse_block_item(const QueryArgs& a, const Bl
     if (threadIdx.x == 0 && a.stop_hint) {
         float steps, promotions;
         usual_stop(a.stop_hint, a.B, b, steps, promotions);
+        // nothing on record yet: the estimate from the shape, on the short side (a jump too far is undone)
+        if (steps <= 0.0f) steps = a.expect_steps * ((float)n / (float)a.ppb);
         misc[kHintSteps] = __builtin_bit_cast(uint32_t, steps);
         misc[kHintPromos] = __builtin_bit_cast(uint32_t, promotions);
     }
@@ -349,7 +351,7 @@ __device__ __forceinline__ void traverse_block_item(const QueryArgs& a, const Bl
     const float kPromoAim = 0.6f * (float)y.promo_max;
     const float inv_L = 1.0f / (float)a.L;
     const float kHintFirst = fminf(1.12f,
-        fast_pow(kPromoAim / fmaxf(1.0f, hint_promos > 0.0f ? hint_promos : (float)a.k_stop * (float)T), inv_L));
+        fast_pow(kPromoAim / fmaxf(1.0f, hint_promos > 0.0f ? hint_promos : a.expect_promotions), inv_L));
     {
         int first = 4;           // (every wavefront reduces the S <= 128 stream lengths on its own)
         for (int s = lane; s < S; s += kWave) first = max(first, s_ns[s] / 128);
@@ -1150,6 +1152,7 @@ __global__ __launch_bounds__(NT, MINW) void traverse_block_list_kernel(QueryArgs
 constexpr int kBlockThreads = 256;
 constexpr int kNarrowThreads = 128;     // workgroups of two wavefronts: more (query, partition) items per CU
 constexpr int kLeadQueries = 32;
+constexpr size_t kMostLds = 160 * 1024 - 512;
 
 #undef PHASE_END
 #undef PHASE_FENCE
@@ -1167,8 +1170,11 @@ bool block_traversal_supported(const QueryArgs& a, size_t* lds_bytes) {
     if ((int64_t)a.L * (a.ppb + 2 * (int64_t)a.T) >= 0x7fffffffLL) return false;   // steps fit 32 bits
     if ((int64_t)a.ppb + 2 * (int64_t)a.T >= 0x7fffffffLL) return false;
     if (a.xcds < 1 || block_queries_per_launch(a.xcds, a.B, a.nq) < 1) return false;
-    return y.lds_bytes <= 160 * 1024 - 512;
+    return y.lds_bytes <= kMostLds;
 }
+
+// Workgroups of four wavefronts a CU holds.
+static int wide_fit(const BlockLayout& y) { return std::max(1, std::min(7, (int)(160 * 1024 / y.lds_bytes))); }
 
 // One launch of the kernel variant that suits the layout: `items` workgroups.
 static int launch_block(const QueryArgs& a, const BlockLayout& y, int64_t items, hipStream_t s) {
@@ -1210,8 +1216,9 @@ static int launch_block(const QueryArgs& a, const BlockLayout& y, int64_t items,
         DCIH_HIP(hipGetLastError());
         return 0;
     }
-    const bool narrow = 4 * a.M * a.L <= kNarrowThreads && fit >= 10;
+    const bool narrow = !a.few_items && 4 * a.M * a.L <= kNarrowThreads && fit >= 10;
     int minw = narrow ? (fit * (kNarrowThreads / 64) + 3) / 4 : fit;      // wavefronts per SIMD
+    if (a.few_items) minw = std::min(minw, (int)((items + a.xcds * 32 - 1) / (a.xcds * 32)));
     minw = minw >= 7 ? 7 : (minw < 3 ? 3 : minw);
     if (narrow) {
         if (minw >= 7) DCIH_LAUNCH(kNarrowThreads, 7); else if (minw == 6) DCIH_LAUNCH(kNarrowThreads, 6);
@@ -1229,7 +1236,23 @@ static int launch_block(const QueryArgs& a, const BlockLayout& y, int64_t items,
     return 0;
 }
 
-int query_block(const QueryArgs& a_in, hipStream_t s) {
+int query_block(const QueryArgs& a_query, hipStream_t s) {
+    QueryArgs a_in = a_query;
+    a_in.expect_promotions = (float)((double)a_in.k_stop * (double)a_in.T);
+    // Where nothing is on record the first epoch aims at the step the shape lets expect, instead of
+    // doubling its way forward from 1/128 of a stream.  A call of so few items that the device holds them
+    // all at once waits for its slowest item: four wavefronts per item then, with the tables that need no
+    // second pass.  (17242-point partitions, thread_size 2: rebuild and 16 queries 2.7 -> 0.75 ms, one query
+    // 437 -> 166 us.)
+    // (Asked for by name, the kernel keeps the variant for many items and feels its way forward at first.)
+    if (a_in.mode == 0) {
+        a_in.expect_steps = (float)(0.9 * expected_stop(a_in));
+        a_in.expect_promotions = (float)expected_promotions(a_in);
+        QueryArgs wide = a_in;
+        wide.full_tables = 1;
+        const BlockLayout y4 = make_block_layout(wide);
+        if (y4.lds_bytes <= kMostLds && (int64_t)a_in.nq * a_in.B <= (int64_t)a_in.xcds * 32 * wide_fit(y4)) a_in.full_tables = a_in.few_items = 1;
+    }
     const BlockLayout y = make_block_layout(a_in);
     // as many queries per launch as the launch limit allows (nearly always all of them)
     const int per_launch = block_queries_per_launch(a_in.xcds, a_in.B, a_in.nq);
@@ -1245,7 +1268,7 @@ int query_block(const QueryArgs& a_in, hipStream_t s) {
     second.q_count = a_in.nq;
     const BlockLayout y2 = make_block_layout(second);
     const bool two_passes = y.set_slots != 0 && a_in.wide_items != nullptr && a_in.wide_cap > 0 &&
-                            y2.lds_bytes <= 160 * 1024 - 512;
+                            y2.lds_bytes <= kMostLds;
     // With nothing known yet about where traversals stop, a few queries go ahead in a launch of
     // their own: their stops are on record when the others start, which then size their first
     // epoch from them instead of feeling their way forward (the first resident round of every
