@@ -148,8 +148,7 @@ struct dcih_index {
     bool used_any = false, used_many = false;
     bool cleared_behind = false;        // dcih_clear did not wait for work under way on used_stream
     float* d_stop_hint = nullptr;       // [3][block_size] epoch-size hints learnt from earlier queries
-    bool hints_clear = false;           // as the build leaves them: no query has run
-    int hint_k = 0, hint_outer = 0, hint_T = 0, hint_maxc = 0;   // query shape the hints belong to
+    int hint_k = 0, hint_outer = 0, hint_T = 0, hint_maxc = 0;   // query shape the hints belong to (zeros: none, as after a build)
     int traversal = 0;                  // DCIH_OPT_TRAVERSAL value
     int dense_min_promos = 160;         // DCIH_OPT_DENSE_MIN_PROMOTIONS value
     int dense_by_cost = 1;              // until that option is set
@@ -425,17 +424,14 @@ static int sort_into(dcih_index* h, int which, const float* d_keys, int64_t key_
     int32_t* sids = (int32_t*)(base + y.ids);
     uint16_t* inv = y.small_parts ? (uint16_t*)(base + y.inv) : nullptr;
     float* hint = (float*)(base + y.hint);
-    // (the table's room is a multiple of 256 bytes, so whole 64-bit words may be cleared)
-    int rc = zero_words64(hint, (int64_t)(((size_t)3 * block_size * sizeof(float) + 7) / 8), s);
-    if (rc == DCIH_OK) {
-        mark(h, DCIH_T_SEGSORT, 0, s);
-        if (merge_from > 0)
-            rc = segsort_append(h->d_skeys, h->d_sids, merge_from, d_keys, key_stride, I, num_points, block_size,
-                                skeys, sids, inv, nullptr, d_tmp, s);
-        else
-            rc = segsort(d_keys, key_stride, I, num_points, block_size, skeys, sids, inv, nullptr, d_tmp, s);
-        mark(h, DCIH_T_SEGSORT, 1, s);
-    }
+    int rc;
+    mark(h, DCIH_T_SEGSORT, 0, s);
+    if (merge_from > 0)
+        rc = segsort_append(h->d_skeys, h->d_sids, merge_from, d_keys, key_stride, I, num_points, block_size,
+                            skeys, sids, inv, nullptr, d_tmp, s);
+    else
+        rc = segsort(d_keys, key_stride, I, num_points, block_size, skeys, sids, inv, nullptr, d_tmp, s);
+    mark(h, DCIH_T_SEGSORT, 1, s);
     // like the reference's dci_add, the call returns when the index is complete
     const hipError_t se = hipStreamSynchronize(s);
     if (rc == DCIH_OK && se != hipSuccess)
@@ -453,7 +449,6 @@ static int sort_into(dcih_index* h, int which, const float* d_keys, int64_t key_
     h->n = num_points;
     h->block_size = block_size;
     h->hint_k = h->hint_outer = h->hint_T = h->hint_maxc = 0;
-    h->hints_clear = true;
     return DCIH_OK;
 }
 
@@ -649,20 +644,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     a.expect_steps = a.expect_promotions = 0.0f;
     a.rows8 = nullptr; a.rows8_rec = 0; a.rows8_bounds = nullptr; a.query8 = nullptr;
     a.phase_ticks = h->d_phase_ticks;
-    // the hints describe where traversals of one query shape stop; forget them when it
-    // changes (cleared by a kernel: a memset node is not safe in a captured graph)
-    if (h->hint_k != num_neighbours || h->hint_outer != num_outer_iterations ||
-        h->hint_T != thread_size || h->hint_maxc != max_num_candidates) {
-        if (!h->hints_clear) {
-            const int rc = zero_words64(h->d_stop_hint, (int64_t)(((size_t)3 * block_size * sizeof(float) + 7) / 8), s);
-            if (rc) return rc;
-        }
-        h->hint_k = num_neighbours; h->hint_outer = num_outer_iterations;
-        h->hint_T = thread_size; h->hint_maxc = max_num_candidates;
-        a.hints_cold = 1;
-    }
-    h->hints_clear = false;
-    a.stop_hint = h->d_stop_hint;
+    a.stop_hint = nullptr;
     a.N = h->n;
     a.ppb = (h->n + block_size - 1) / block_size;
     a.dim = dim; a.M = h->M; a.L = h->L; a.B = block_size; a.T = thread_size;
@@ -738,6 +720,20 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
             if (dense_traversal_supported(a, nullptr)) q8_bytes = align_up((size_t)num_queries * rows8_query_bytes(dim));
             else a.rows8 = nullptr;      // (no room for the longer list of what is kept)
         }
+    }
+    // The hints, which only the batch kernel reads, describe where traversals of one query shape stop;
+    // forget them when it changes (cleared by a kernel: a memset node is not safe in a captured graph; the
+    // table's room is a multiple of 256 bytes, so whole 64-bit words may be cleared)
+    if (!(dense_traversal_supported(a, nullptr) && takes_dense_kernel(a))) {
+        if (h->hint_k != num_neighbours || h->hint_outer != num_outer_iterations ||
+            h->hint_T != thread_size || h->hint_maxc != max_num_candidates) {
+            const int rc = zero_words64(h->d_stop_hint, (int64_t)(((size_t)3 * block_size * sizeof(float) + 7) / 8), s);
+            if (rc) return rc;
+            h->hint_k = num_neighbours; h->hint_outer = num_outer_iterations;
+            h->hint_T = thread_size; h->hint_maxc = max_num_candidates;
+            a.hints_cold = 1;
+        }
+        a.stop_hint = h->d_stop_hint;
     }
     const size_t qp_bytes = align_up((size_t)I * num_queries * sizeof(float));
     const size_t part_bytes = align_up(query_part_bytes(a));
