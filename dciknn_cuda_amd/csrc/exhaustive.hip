@@ -27,6 +27,7 @@ constexpr int kExCols = 32;       // columns staged per LDS tile
 constexpr int kExPitch = 36;      // row pitch in LDS: conflict-free 16-byte reads
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef v4f v4f_any __attribute__((aligned(4)));      // a 16-byte read that may start at any float
+typedef const __attribute__((address_space(4))) v4f_any cv4f;
 
 // out[q][row] = || data[row] - query[q] ||, the squares summed one after the
 // other in index order like compute_dist_device (src/dci_cuda_kernel.cu:36-44);
@@ -37,7 +38,8 @@ typedef v4f v4f_any __attribute__((aligned(4)));      // a 16-byte read that may
 // meanwhile, and every lane keeps its row's QN sums; the queries' values are the
 // same for all lanes and come through the scalar cache.  Bound by vector issue, three
 // instructions per element and query, once enough wavefronts run, hence fewer queries per
-// wavefront where rows and queries are few.  (500 queries, 3000 rows of 100: 86 us before.)
+// wavefront where rows and queries are few.  (500 queries, 3000 rows of 100:
+// 86 us before, 22 now; 4000 queries, 9582 rows: 440 us with the queries read where they are used, 364 ahead.)
 template <int QN>
 __global__ __launch_bounds__(kExRows) void exact_dists_kernel(
     const float* __restrict__ data, int64_t N, int dim, const float* __restrict__ query, int nq,
@@ -88,17 +90,45 @@ __global__ __launch_bounds__(kExRows) void exact_dists_kernel(
         __syncthreads();
         const float* x = &tile[lane * kExPitch];
         int kk = 0;
-#pragma unroll 2
-        for (; kk + 4 <= kc; kk += 4) {
-            const v4f v = *reinterpret_cast<const v4f*>(x + kk);
+        // The queries' next four elements are read while the present four are worked on.  (Scalar reads
+        // return in any order, so a wait is for all of them: the present ones are made to arrive first.)
+        auto fetch = [&](int at, v4f (&q)[QN]) __attribute__((always_inline)) {
+            const int c = min(at, max(dim - 4, 0));
+#pragma unroll
+            for (int j = 0; j < QN; j++) q[j] = *(cv4f*)(qv[j] + c);
+        };
+        auto arrived = [&](v4f (&q)[QN]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < QN; j++) asm volatile("" :: "s"(q[j]));
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto add = [&](const v4f& v, const v4f (&q)[QN]) __attribute__((always_inline)) {
 #pragma unroll
             for (int j = 0; j < QN; j++) {
-                const cfloat* q = qv[j] + k0 + kk;
-                float d = v.x - q[0]; acc[j] = acc[j] + d * d;
-                d = v.y - q[1]; acc[j] = acc[j] + d * d;
-                d = v.z - q[2]; acc[j] = acc[j] + d * d;
-                d = v.w - q[3]; acc[j] = acc[j] + d * d;
+                float d = v.x - q[j].x; acc[j] = acc[j] + d * d;
+                d = v.y - q[j].y; acc[j] = acc[j] + d * d;
+                d = v.z - q[j].z; acc[j] = acc[j] + d * d;
+                d = v.w - q[j].w; acc[j] = acc[j] + d * d;
             }
+        };
+        if (kc >= 4) {
+            v4f qa[QN], qb[QN];
+            fetch(k0, qa);
+            v4f va = *reinterpret_cast<const v4f*>(x), vb;
+#pragma unroll 1
+            for (; kk + 8 <= kc; kk += 8) {
+                arrived(qa);
+                fetch(k0 + kk + 4, qb);
+                vb = *reinterpret_cast<const v4f*>(x + kk + 4);
+                __builtin_amdgcn_sched_barrier(0);
+                add(va, qa);
+                arrived(qb);
+                fetch(k0 + kk + 8, qa);
+                va = *reinterpret_cast<const v4f*>(x + min(kk + 8, kExCols - 4));
+                __builtin_amdgcn_sched_barrier(0);
+                add(vb, qb);
+            }
+            if (kk + 4 <= kc) { add(va, qa); kk += 4; }
         }
 #pragma unroll 1
         for (; kk < kc; kk++) {
@@ -347,11 +377,11 @@ int query_exhaustive(const QueryArgs& a, void* ws, int chunk, hipStream_t s) {
     const ExSelect sel = exhaustive_select(a.N, a.k);
     for (int q0 = 0; q0 < a.nq; q0 += chunk) {
         const int nqc = min(chunk, a.nq - q0);
-        // as many queries per wavefront as leave two wavefronts to every SIMD (a row is read once for all of them)
+        // as many queries per wavefront as leave a wavefront to every SIMD (a row is read once for all of them)
         const auto waves = [&](int qn) { return row_groups * ((nqc + qn - 1) / qn); };
-        if (waves(8) >= 2048) launch_dists<8>(a, q0, nqc, d_dist, s);
-        else if (waves(4) >= 2048) launch_dists<4>(a, q0, nqc, d_dist, s);
-        else if (waves(2) >= 2048) launch_dists<2>(a, q0, nqc, d_dist, s);
+        if (waves(8) >= 1024) launch_dists<8>(a, q0, nqc, d_dist, s);
+        else if (waves(4) >= 1024) launch_dists<4>(a, q0, nqc, d_dist, s);
+        else if (waves(2) >= 1024) launch_dists<2>(a, q0, nqc, d_dist, s);
         else launch_dists<1>(a, q0, nqc, d_dist, s);
         DCIH_HIP(hipGetLastError());
         int32_t* out_ids = a.out_ids + (int64_t)q0 * a.k;
