@@ -258,7 +258,7 @@ __device__ __forceinline__ void bitonic_sort_u64_regs(unsigned long long* s, int
                     const int e = tid * E + i;
                     const unsigned long long o = s[e ^ stride];
                     const bool keep_min = ((e & stride) == 0) == ((e & size) == 0);
-                    v[i] = keep_min ? (v[i] < o ? v[i] : o) : (v[i] > o ? v[i] : o);
+                    v[i] = (o < v[i]) == keep_min ? o : v[i];
                 }
             } else if (stride >= E) {
 #pragma unroll
@@ -266,7 +266,7 @@ __device__ __forceinline__ void bitonic_sort_u64_regs(unsigned long long* s, int
                     const int e = tid * E + i;
                     const unsigned long long o = lane_xor_any(v[i], stride / E);
                     const bool keep_min = ((e & stride) == 0) == ((e & size) == 0);
-                    v[i] = keep_min ? (v[i] < o ? v[i] : o) : (v[i] > o ? v[i] : o);
+                    v[i] = (o < v[i]) == keep_min ? o : v[i];
                 }
             } else {
 #pragma unroll
@@ -288,22 +288,30 @@ __device__ __forceinline__ void bitonic_sort_u64_regs(unsigned long long* s, int
     for (int i = 0; i < E; i++) s[tid * E + i] = v[i];
     __syncthreads();
 }
-// The words of a wavefront's lanes, ascending by lane.
-__device__ __forceinline__ unsigned long long wave_sort_u64(unsigned long long v) {
-    const int lane = lane_id();
-    auto step = [&](unsigned long long w, int size, int stride) {
-        const bool take_min = ((lane & size) == 0) == ((lane & stride) == 0);
-        v = (w < v) == take_min ? w : v;
-    };
-    step(lane_xor<1>(v), 2, 1);
-    step(lane_xor<2>(v), 4, 2); step(lane_xor<1>(v), 4, 1);
-    step(lane_xor<4>(v), 8, 4); step(lane_xor<2>(v), 8, 2); step(lane_xor<1>(v), 8, 1);
-    step(lane_xor<8>(v), 16, 8); step(lane_xor<4>(v), 16, 4); step(lane_xor<2>(v), 16, 2); step(lane_xor<1>(v), 16, 1);
-    step(lane_xor<16>(v), 32, 16); step(lane_xor<8>(v), 32, 8); step(lane_xor<4>(v), 32, 4); step(lane_xor<2>(v), 32, 2);
-    step(lane_xor<1>(v), 32, 1);
-    step(lane_xor<32>(v), 64, 32); step(lane_xor<16>(v), 64, 16); step(lane_xor<8>(v), 64, 8); step(lane_xor<4>(v), 64, 4);
-    step(lane_xor<2>(v), 64, 2); step(lane_xor<1>(v), 64, 1);
-    return v;
+// The same for the 64 * E words of one wavefront, lane l holding words l * E .. l * E + E - 1.
+template <int E>
+__device__ __forceinline__ void wave_sort_u64(unsigned long long (&v)[E], int lane) {
+#pragma unroll
+    for (int size = 2; size <= kWave * E; size <<= 1) {
+#pragma unroll
+        for (int stride = size >> 1; stride > 0; stride >>= 1) {
+#pragma unroll
+            for (int i = 0; i < E; i++) {
+                const int e = lane * E + i;
+                const bool up = (e & size) == 0;
+                if (stride >= E) {
+                    const unsigned long long o = lane_xor_any(v[i], stride / E);
+                    const bool keep_min = ((e & stride) == 0) == up;
+                    v[i] = (o < v[i]) == keep_min ? o : v[i];
+                } else if ((i & stride) == 0) {
+                    const unsigned long long x = v[i], y = v[i | stride];
+                    const bool swap = (x > y) == up;
+                    v[i] = swap ? y : x;
+                    v[i | stride] = swap ? x : y;
+                }
+            }
+        }
+    }
 }
 // n words by NT threads: the register variant up to MAXE words per thread (each is a piece of
 // straight-line code of its own, and four words per thread take 15 KB of it).

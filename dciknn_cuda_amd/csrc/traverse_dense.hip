@@ -371,9 +371,75 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
             const int W = __builtin_amdgcn_readfirstlane((int)misc[dWin]);
             maxw = max(maxw, (unsigned long long)W);
 
+            // The step of every window is its place in the order of priorities, stored doubled with bit 0
+            // set: a lookup subtracts one where the point is not the window's first lane, which
+            // leaves the lane-0 flag beside the step.
+            bool few_windows = false;
+            if constexpr (IPT <= 9) if (W <= 2 * NT) {
+                // ---- few windows: one or two per thread, as (priority, layout index, table place) words; the
+                // layout index makes equal priorities keep their order.  Sorted in registers, up to 256 words
+                // by one wavefront: bound by vector issue, and the exchanges inside a lane are done once, not
+                // by both sides.
+                few_windows = true;
+                const int np = W <= 4 * kWave ? (W <= kWave ? kWave : (W <= 2 * kWave ? 2 * kWave : 4 * kWave)) : (W <= NT ? NT : 2 * NT);
+                unsigned long long* s64 = reinterpret_cast<unsigned long long*>(tb.stage);
+#pragma unroll
+                for (int e = 0; e < 2; e++) {
+                    const int idx = e * NT + tid;
+                    unsigned long long word = ~0ull;
+                    if (idx < W) {
+                        int lo = 0, hi = 2 * args->a.L - 1;      // the first segment that ends behind idx
+                        while (lo < hi) {
+                            const int mid = (lo + hi) >> 1;
+                            if (tb.seg[mid + 1] <= idx) lo = mid + 1; else hi = mid;
+                        }
+                        const int sidx = tb.segstream[lo], j = idx - tb.seg[lo], h = sidx >> 1;
+                        const int p = tb.p[m * args->a.L + h];
+                        const int pos = sidx & 1 ? p + 1 + j * T : p - T + 1 - j * T;
+                        const int place = sidx & 1 ? tb.segw[lo] + j : tb.segw[lo] - j;
+                        const float key = args->a.skeys[(int64_t)(m * args->a.L + h) * args->a.N + off + min(max(pos, 0), n - 1)];
+                        const float prio = fabsf(key - tb.qp[m * args->a.L + h]);
+                        word = ((unsigned long long)__builtin_bit_cast(uint32_t, prio) << 32) | ((uint32_t)idx << 16) | (uint32_t)place;
+                        probes++;
+                    }
+                    if (idx < np) s64[idx] = word;
+                }
+                __syncthreads();
+                PHASE_END(1);
+                auto by_one_wave = [&](auto etag) __attribute__((always_inline)) {
+                    constexpr int E = decltype(etag)::value;
+                    if (wave == 0) {
+                        unsigned long long v[E];
+#pragma unroll
+                        for (int i = 0; i < E; i++) v[i] = s64[lane * E + i];
+                        wave_sort_u64(v, lane);
+                        __builtin_amdgcn_wave_barrier();                // the table takes the words' room
+#pragma unroll
+                        for (int i = 0; i < E; i++)
+                            if (v[i] != ~0ull) tb.rank16[(uint32_t)v[i] & 0xffffu] = (uint16_t)(((lane * E + i) << 1) | 1);
+                    }
+                };
+                if (np == kWave) by_one_wave(std::integral_constant<int, 1>{});
+                else if (np == 2 * kWave) by_one_wave(std::integral_constant<int, 2>{});
+                else if constexpr (NT > kWave) {
+                    if (np == 4 * kWave) {
+                        by_one_wave(std::integral_constant<int, 4>{});
+                    } else {
+                        if constexpr (NT > 4 * kWave) if (np == NT) bitonic_sort_u64_regs<1, NT>(s64, tid);
+                        if (np == 2 * NT) bitonic_sort_u64_regs<2, NT>(s64, tid);
+                        unsigned long long mine[2];
+#pragma unroll
+                        for (int e = 0; e < 2; e++) mine[e] = e * NT < np ? s64[e * NT + tid] : 0ull;
+                        __syncthreads();                    // the table takes the sorted words' room
+#pragma unroll
+                        for (int e = 0; e < 2; e++)
+                            if (e * NT + tid < W) tb.rank16[(uint32_t)mine[e] & 0xffffu] = (uint16_t)(((e * NT + tid) << 1) | 1);
+                    }
+                }
+            }
             // ---- priorities of the windows, blocked: thread t holds layout indices t*IPT.. ----
             // (formed a second time in the rare case that the ranking by buckets gives up)
-            for (bool by_radix = false;; by_radix = true) {
+            for (bool by_radix = false; !few_windows; by_radix = true) {
             ArgsPtr args = fresh_args();
             DenseTables tb(smem, args->a, args->y);
             uint32_t k[IPT], rp[IPT];
@@ -439,31 +505,6 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
             }
             __syncthreads();
             PHASE_END(1);
-            // the step of every window: its place in the sorted order, stored doubled with bit 0
-            // set: a lookup subtracts one where the point is not the window's first lane, which
-            // leaves the lane-0 flag beside the step
-            if constexpr (IPT <= 9) if (W <= 2 * NT) {
-                // Few windows: a bitonic sort held in registers of (priority, layout index, table place)
-                // words; the layout index makes equal priorities keep their order.
-                const int np = W <= NT ? NT : 2 * NT;
-                unsigned long long* s64 = reinterpret_cast<unsigned long long*>(tb.stage);
-#pragma unroll
-                for (int r = 0; r < IPT; r++) {
-                    const int idx = tid * IPT + r;
-                    if (idx < np)
-                        s64[idx] = idx < W ? ((unsigned long long)k[r] << 32) | ((unsigned long long)idx << 16) | (rp[r] & 0xffffu)
-                                           : ~0ull;
-                }
-                if (np == NT) bitonic_sort_u64_regs<1, NT>(s64, tid); else bitonic_sort_u64_regs<2, NT>(s64, tid);
-                unsigned long long mine[2];
-#pragma unroll
-                for (int e = 0; e < 2; e++) mine[e] = e * NT < np ? s64[e * NT + tid] : 0ull;
-                __syncthreads();                    // the table takes the sorted words' room
-#pragma unroll
-                for (int e = 0; e < 2; e++)
-                    if (e * NT + tid < W) tb.rank16[(uint32_t)mine[e] & 0xffffu] = (uint16_t)(((e * NT + tid) << 1) | 1);
-                break;
-            }
             const uint32_t max_bits = (uint32_t)__builtin_amdgcn_readfirstlane((int)misc[dMaxBits]);
             const float scale = 4294966016.0f / __builtin_bit_cast(float, max_bits);
             bool ranked = false;
@@ -573,7 +614,9 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
                     constexpr int kPath = decltype(path_tag)::value;     // 0: T = 2^s; 1: any other T
                     constexpr int kH = 2, kD = 4, kChunk = NT * 8;
                     const int ngrp = (args->a.L + kH - 1) / kH;
-                    const int NG = ((n + kChunk - 1) / kChunk) * ngrp;
+                    // (a wavefront whose points of a chunk all lie past the slice's end has no part in that chunk)
+                    const int own_chunks = max(0, (n - 8 * kWave * __builtin_amdgcn_readfirstlane(wave) + kChunk - 1) / kChunk);
+                    const int NG = own_chunks * ngrp;
                     const unsigned char* tab0 = reinterpret_cast<const unsigned char*>(tb.rank16);
                     // path 0
                     const uint16_t sh = (uint16_t)floor_log2(T);
@@ -674,6 +717,7 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
                     int cc = 0, hc = 0, ci = 0, hi = 0;     // (chunk base, first simple index) of the group to consume / to issue
                     auto advance = [&](int& c, int& h) { h += kH; if (h >= args->a.L) { h = 0; c += kChunk; } };
                     u32x4 pv[kD][kH];
+                    if (NG == 0) return;
 #pragma unroll
                     for (int d = 0; d < kD; d++) {
                         issue(ci, hi, pv[d]);
@@ -1125,7 +1169,11 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
             }
             if (NT > kWave && words == kWave) {
                 __syncthreads();
-                if (wave == 0) res[lane] = wave_sort_u64(res[lane]);
+                if (wave == 0) {
+                    unsigned long long v[1] = {res[lane]};
+                    wave_sort_u64(v, lane);
+                    res[lane] = v[0];
+                }
                 __syncthreads();
             } else {
                 bitonic_sort_u64_by<NT, NT == 64 ? 4 : (IPT > 9 ? 1 : 2)>(res, words, tid);
