@@ -340,6 +340,13 @@ def main():
     hbm_bytes = 8.0 * I * N + nq * (4.0 * dim + 4.0 * dim * C + 8.0 * min(k, ppb) * cfg["bs"])
     hbm_model = ("index slices once (8 B per entry) + per query its row, %.0f candidate rows of %d B and "
                  "its per-partition result lists" % (C, 4 * dim))
+    if kernel == "traverse_dense_kernel" and 96 <= dim <= 1024:
+        # rows of these lengths are compared by their 8-bit codes; at least the k best of every
+        # partition are read whole as well
+        rec = max(128, 16 + (dim + 15) // 16 * 16)
+        hbm_bytes = 8.0 * I * N + nq * (4.0 * dim + rec * C + (4.0 * dim + 8.0) * min(k, ppb) * cfg["bs"])
+        hbm_model = ("index slices once (8 B per entry) + per query its row, %.0f candidates' codes of %d B, %d rows of "
+                     "%d B per partition and its per-partition result lists" % (C, rec, min(k, ppb), 4 * dim))
     if kernel.startswith("exact_dists"):
         # direct ranking: the rows once, per (query, point) a distance written, sorted and read back
         hbm_bytes = 4.0 * N * dim + nq * (4.0 * dim + 12.0 * N + 8.0 * k)
