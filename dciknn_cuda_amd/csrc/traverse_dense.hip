@@ -172,6 +172,7 @@ __device__ inline unsigned long long uniform_u64(unsigned long long v) {
 }
 
 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) uint16_t lds_u16;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct DenseArgs { QueryArgs a; DenseLayout y; };
@@ -617,7 +618,7 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
                     // (a wavefront whose points of a chunk all lie past the slice's end has no part in that chunk)
                     const int own_chunks = max(0, (n - 8 * kWave * __builtin_amdgcn_readfirstlane(wave) + kChunk - 1) / kChunk);
                     const int NG = own_chunks * ngrp;
-                    const unsigned char* tab0 = reinterpret_cast<const unsigned char*>(tb.rank16);
+                    const uint32_t tab0 = (uint32_t)(uintptr_t)(lds_u16*)tb.rank16;      // LDS address
                     // path 0
                     const uint16_t sh = (uint16_t)floor_log2(T);
                     const u16x2 sh_pk = {sh, sh};
@@ -651,20 +652,24 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
                         for (int hh = 0; hh < kH; hh++) {
                             const int i = m * args->a.L + min(h0 + hh, args->a.L - 1);   // (past L: the last index again)
                             const uint32_t shift = (uint32_t)tb.shift[i];
-                            const unsigned char* tab = tab0 + 2 * tb.tabbase[i];
+                            const uint32_t tab = tab0 + 2 * (uint32_t)tb.tabbase[i];
                             const uint32_t wd[4] = {pv[hh].x, pv[hh].y, pv[hh].z, pv[hh].w};
 #pragma unroll
                             for (int j = 0; j < 4; j++) {
                                 if constexpr (kPath == 0) {
                                     const u16x2 shift_pk = {(uint16_t)shift, (uint16_t)shift};
                                     const u16x2 x = __builtin_bit_cast(u16x2, wd[j]) + shift_pk;
-                                    // twice the window's place: the byte offset of its table entry
-                                    const uint32_t w2 = __builtin_bit_cast(uint32_t, (x >> sh_pk) << one_pk);
+                                    const u16x2 w = x >> sh_pk;
                                     // (spelled out: the compiler's own form of min(r, 1) is
                                     //  two compares, two selects and a byte permute)
                                     asm("v_pk_min_u16 %0, %1, %2" : "=v"(rem[hh][j]) : "v"(x & mask_pk), "v"(one_pk));
-                                    tv[hh][2 * j] = *reinterpret_cast<const uint16_t*>(tab + (w2 & 0xffffu));
-                                    tv[hh][2 * j + 1] = *reinterpret_cast<const uint16_t*>(tab + (w2 >> 16));
+                                    // (one instruction takes a window's place out of its half, doubles it and
+                                    //  adds the table's address)
+                                    uint32_t a0, a1;
+                                    asm("v_mad_u32_u16 %0, %1, 2, %2" : "=v"(a0) : "v"(w), "v"(tab));
+                                    asm("v_mad_u32_u16 %0, %1, 2, %2 op_sel:[1,0,0,0]" : "=v"(a1) : "v"(w), "v"(tab));
+                                    tv[hh][2 * j] = *(const lds_u16*)a0;
+                                    tv[hh][2 * j + 1] = *(const lds_u16*)a1;
                                 } else {
 #pragma unroll
                                     for (int e = 0; e < 2; e++) {
@@ -672,7 +677,7 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
                                         const uint32_t xs = (pos << q_sh) + (shift << q_sh);
                                         uint32_t w;
                                         asm("v_mul_hi_u32_u24 %0, %1, %2" : "=v"(w) : "s"(q_magic), "v"(xs));
-                                        tv[hh][2 * j + e] = *reinterpret_cast<const uint16_t*>(tab + 2 * w);
+                                        tv[hh][2 * j + e] = *(const lds_u16*)(tab + 2 * w);
                                         const uint32_t off_lane = (uint32_t)((uint32_t)__umul24(w, q_T) != xs);
                                         if (e) rem[hh][j].y = (uint16_t)off_lane; else rem[hh][j].x = (uint16_t)off_lane;
                                     }
