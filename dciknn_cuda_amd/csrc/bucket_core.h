@@ -9,8 +9,8 @@ namespace {
 
 constexpr int kBucketMost = 48;          // items one bucket may hold before the radix passes are the cheaper way
 
-// Thread t holds the items t*IPT .. t*IPT+IPT-1 of W (the rest are pads): k[r] the bits of a
-// non-negative finite float, rp[r] a payload of 14 bits.  On return the item's place in the ascending
+// Thread t holds the items t*IPT .. t*IPT+IPT-1 (STRIDED: t, t+NT, t+2*NT ...) of W (the rest are pads): k[r] the bits of a
+// non-negative finite float, rp[r] a payload of 16 bits.  On return the item's place in the ascending
 // order of (k, item number) is in rp[r]'s high half, the payload still in its low half; k is used up.
 //
 // x * scale (scale maps the largest x below 2^32) grows with x; its upper NBITS bits name a bucket,
@@ -31,17 +31,18 @@ constexpr int kBucketMost = 48;          // items one bucket may hold before the
 // LDS: `list` IPT * NT + 4 words, `cnt32` (1 << NBITS) / 2 + 1 words, `misc` 32 words, `work` work_cap <= NT
 // 64-bit words.  All threads call this; it ends with reads of `list` under way (callers need a
 // barrier before they reuse it).
-template <int NT, int IPT, int NBITS, class Before>
+template <int NT, int IPT, int NBITS, bool STRIDED = false, class Before>
 __device__ inline bool lds_bucket_ranks(uint32_t (&k)[IPT], uint32_t (&rp)[IPT], int W, float scale,
                                         uint32_t* list, uint32_t* cnt32, uint32_t* misc, unsigned long long* work,
                                         int work_cap, int tid, int& fix_rank, uint32_t& fix_payload, Before before) {
-    static_assert(NT * IPT <= (1 << 14), "item numbers of 14 bits");
+    static_assert(NT * IPT <= (1 << 15), "places of 16 bits");
     constexpr int kWords = (1 << NBITS) / 2, kPer = kWords / NT, kGroup = 4;
     const int lane = tid & 63, wave = tid >> 6;
     const uint16_t* cnt = reinterpret_cast<const uint16_t*>(cnt32);
     // items of this thread that are no pads; made opaque again for every pass, or the compiler keeps the
     // IPT comparisons with it as lane masks across all of them
-    int own = min(max(W - tid * IPT, 0), IPT);
+    int own = STRIDED ? (W > tid ? (W - tid + NT - 1) / NT : 0) : min(max(W - tid * IPT, 0), IPT);
+    auto number = [&](int r) { return STRIDED ? r * NT + tid : tid * IPT + r; };
     auto fresh = [&]() { asm volatile("" : "+v"(own)); };
 #pragma unroll
     for (int w = 0; w < kPer; w++) cnt32[tid + w * NT] = 0;
@@ -93,7 +94,7 @@ __device__ inline bool lds_bucket_ranks(uint32_t (&k)[IPT], uint32_t (&rp)[IPT],
         // (a pad's word goes to its own place behind the items)
         const bool real = r < own;
         const uint32_t at = (uint32_t)cnt[k[r] >> (32 - NBITS)] + (rp[r] >> 16);
-        list[real ? at : (uint32_t)(tid * IPT + r)] = real ? k[r] : 0xffffffffu;
+        list[real ? at : (uint32_t)number(r)] = real ? k[r] : 0xffffffffu;
         if ((r & 7) == 7) __builtin_amdgcn_sched_barrier(0);
     }
     __syncthreads();
@@ -145,7 +146,7 @@ __device__ inline bool lds_bucket_ranks(uint32_t (&k)[IPT], uint32_t (&rp)[IPT],
                 if (upto[g] > 1u && r0 + g < own) {
                     const uint32_t slot = atomicAdd(&misc[17], 1u);
                     if (slot < (uint32_t)work_cap)
-                        work[slot] = ((unsigned long long)rp[r0 + g] << 32) | (uint32_t)(tid * IPT + r0 + g);
+                        work[slot] = ((unsigned long long)rp[r0 + g] << 32) | (uint32_t)number(r0 + g);
                 }
             }
         }

@@ -13,8 +13,11 @@
 // columns copied out.  The traversal counters have closed forms too: every
 // index entry is visited once, every point is a candidate, and the outer steps
 // follow from the window counts on either side of the positioning search.
+#include "bucket_core.h"
 #include "common.h"
 #include "kernels.h"
+#include "radix_core.h"
+#include "traverse_common.h"
 
 namespace dcih {
 
@@ -233,6 +236,130 @@ __global__ __launch_bounds__(kSelThreads) void select_rows_kernel(const float* _
     }
 }
 
+// One row of distances per workgroup, ranked in LDS by buckets (bucket_core.h; by radix passes where the distances
+// cluster) and written out in order, the first k of them.  Such calls are few rows, so what counts is one
+// row's time: sixteen wavefronts on it, the whole LDS for it, no kernel to cut and convert the result after
+// it.  (20 rows of 9582: 22 us; the segmented sort and that kernel 39 + 4.)  Beyond 16 items per thread 128
+// registers do not hold them and eight wavefronts take as long as the segmented sort (20000: 63 and 62 us).
+constexpr int rank_bits(int items) { return items <= 2048 ? 11 : (items <= 4096 ? 12 : (items <= 8192 ? 13 : 14)); }
+constexpr int rank_counter_words(int nt, int ipt) {
+    return (1 << rank_bits(nt * ipt)) / 2 + 4 > 8 * nt ? (1 << rank_bits(nt * ipt)) / 2 + 4 : 8 * nt;
+}
+constexpr size_t rank_lds(int nt, int ipt) {
+    return (size_t)(64 + nt * ipt + 4 + rank_counter_words(nt, ipt)) * 4 + (size_t)nt * 8;
+}
+template <int NT, int IPT>
+__global__ __launch_bounds__(NT, NT / 256) void rank_row_kernel(const float* __restrict__ dists, int n, int k, int float_ids,
+                                                                   int32_t* __restrict__ out_ids, float* __restrict__ out_vals) {
+    extern __shared__ __align__(16) unsigned char rank_smem[];
+    uint32_t* misc = reinterpret_cast<uint32_t*>(rank_smem);             // 32 words for the ranking, then the extremes
+    unsigned long long* work = reinterpret_cast<unsigned long long*>(misc + 64);
+    uint32_t* list = reinterpret_cast<uint32_t*>(work + NT);
+    uint32_t* cnt = list + NT * IPT + 4;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const float* row = dists + (int64_t)blockIdx.x * n;
+    out_ids += (int64_t)blockIdx.x * k;
+    out_vals += (int64_t)blockIdx.x * k;
+    if (tid == 0) { misc[32] = 0xffffffffu; misc[33] = 0; misc[34] = 0; misc[35] = 0xffffffffu; }
+    __syncthreads();
+    uint32_t key[IPT], rp[IPT];
+    {
+        uint32_t least = 0xffffffffu, most = 0;
+#pragma unroll
+        for (int r = 0; r < IPT; r++) {
+            const int j = r * NT + tid;
+            key[r] = __builtin_bit_cast(uint32_t, row[min(j, n - 1)]);
+            rp[r] = (uint32_t)j;
+            least = min(least, key[r]);
+            most = max(most, key[r]);
+        }
+        least = wave_min_u32(least);
+        most = ~wave_min_u32(~most);
+        if (lane == 0) { atomicMin(&misc[32], least); atomicMax(&misc[33], most); }
+    }
+    __syncthreads();
+    const uint32_t lo_bits = misc[32], hi_bits = misc[33];
+    const float lo = __builtin_bit_cast(float, lo_bits), width = __builtin_bit_cast(float, hi_bits) - lo;
+    const float scale = 4294966016.0f / width;
+    int fix_rank = -1;
+    uint32_t fix_item = 0;
+    bool ranked = false;
+    if (hi_bits < kInfBits && scale < 4e38f) {
+        auto before = [&](int x, int z) __attribute__((always_inline)) {
+            const uint32_t bx = __builtin_bit_cast(uint32_t, row[x]), bz = __builtin_bit_cast(uint32_t, row[z]);
+            return bx != bz ? bx < bz : x < z;
+        };
+#pragma unroll
+        for (int r = 0; r < IPT; r++) key[r] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(float, key[r]) - lo);
+        ranked = lds_bucket_ranks<NT, IPT, rank_bits(NT * IPT), true>(key, rp, n, scale, list, cnt, misc, work, NT, tid, fix_rank,
+                                                                 fix_item, before);
+    }
+    auto store = [&](int at, uint32_t bits, uint32_t item) {
+        if (at >= k) return;
+        out_vals[at] = __builtin_bit_cast(float, bits);
+        out_ids[at] = float_ids ? __builtin_bit_cast(int32_t, (float)(int)item) : (int)item;
+    };
+    __syncthreads();
+    if (ranked) {
+        // through LDS, so that the results leave in order: the row's numbers first, from which the values follow
+        uint16_t* order = reinterpret_cast<uint16_t*>(list);
+        int own = n > tid ? (n - tid + NT - 1) / NT : 0;
+        asm volatile("" : "+v"(own));
+#pragma unroll
+        for (int r = 0; r < IPT; r++)
+            if (r < own) order[rp[r] >> 16] = (uint16_t)(r * NT + tid);
+        __syncthreads();
+        if (fix_rank >= 0) order[fix_rank] = (uint16_t)fix_item;
+        __syncthreads();
+        const int end = min(n, k);
+        for (int j = tid; j < end; j += NT) {
+            const uint32_t item = order[j];
+            store(j, __builtin_bit_cast(uint32_t, row[item]), item);
+        }
+        return;
+    }
+    uint32_t vor = 0, vand = 0xffffffffu;
+#pragma unroll
+    for (int r = 0; r < IPT; r++) {
+        const int j = tid * IPT + r;
+        key[r] = j < n ? __builtin_bit_cast(uint32_t, row[j]) : 0xffffffffu;      // (pads stay behind everything: the passes are stable)
+        rp[r] = (uint32_t)j;
+        vor |= j < n ? key[r] : 0u;
+        vand &= j < n ? key[r] : 0xffffffffu;
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        vor |= (uint32_t)__shfl_xor((int)vor, o, kWave);
+        vand &= (uint32_t)__shfl_xor((int)vand, o, kWave);
+    }
+    if (lane == 0) { atomicOr(&misc[34], vor); atomicAnd(&misc[35], vand); }
+    __syncthreads();
+    lds_radix_passes<NT, IPT>(key, rp, list, cnt, misc, misc[34] ^ misc[35]);
+#pragma unroll
+    for (int r = 0; r < IPT; r++)
+        if (tid * IPT + r < n) store(tid * IPT + r, key[r], rp[r] & 0xffffu);
+}
+static bool rank_fits(int64_t n) { return n <= 1024 * 16; }
+static int rank_rows_in_lds(const float* d_dist, int rows, int n, int k, int float_ids, int32_t* out_ids, float* out_vals,
+                            hipStream_t s) {
+#define DCIH_RANK(NT, IPT)                                                                              \
+    do {                                                                                            \
+        static DeviceOnce once;                                                                     \
+        const int rc_attr = once.run([]() -> int {                                                  \
+            DCIH_HIP(hipFuncSetAttribute((const void*)rank_row_kernel<NT, IPT>,                         \
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));  \
+            return 0;                                                                               \
+        });                                                                                         \
+        if (rc_attr) return rc_attr;                                                                \
+        hipLaunchKernelGGL((rank_row_kernel<NT, IPT>), dim3((unsigned)rows), dim3(NT), rank_lds(NT, IPT), s, d_dist, n, k, \
+                           float_ids, out_ids, out_vals);                                           \
+    } while (0)
+    if (n <= 1024 * 2) DCIH_RANK(1024, 2); else if (n <= 1024 * 4) DCIH_RANK(1024, 4); else if (n <= 1024 * 8) DCIH_RANK(1024, 8);
+    else if (n <= 1024 * 12) DCIH_RANK(1024, 12); else DCIH_RANK(1024, 16);
+#undef DCIH_RANK
+    DCIH_HIP(hipGetLastError());
+    return 0;
+}
+
 // The first k columns of every sorted row.  Columns past the end of a row and, when
 // asked, entries whose value is +inf (points that never became candidates) read as
 // "no result": id -1, +inf.
@@ -400,7 +527,9 @@ int query_exhaustive(const QueryArgs& a, void* ws, int chunk, hipStream_t s) {
             if (rc) return rc;
             continue;
         }
-        const int rc = rank_rows(ws, chunk, nqc, a.N, a.k, false, a.float_ids != 0, out_ids, out_dists, s);
+        const int rc = rank_fits(a.N)
+            ? rank_rows_in_lds(d_dist, nqc, (int)a.N, a.k, a.float_ids, out_ids, out_dists, s)
+            : rank_rows(ws, chunk, nqc, a.N, a.k, false, a.float_ids != 0, out_ids, out_dists, s);
         if (rc) return rc;
     }
     if (a.counters) {
