@@ -24,7 +24,7 @@ size_t segsort_tmp_bytes(int num_indices, int64_t n, int block_size);
 // index does not keep them).
 int segsort(const float* d_keys, int64_t key_stride, int num_indices, int64_t n, int block_size,
             float* d_skeys, int32_t* d_sids, uint16_t* d_inv, uint16_t* d_lids, void* d_tmp,
-            hipStream_t s);
+            hipStream_t s, bool float_ids = false);
 
 // Appending: the index over n1 points from the sorted arrays of the index over their first
 // n0 points (same block_size) and the unsorted keys of the others (index i's key of point id

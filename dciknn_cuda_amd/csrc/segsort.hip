@@ -35,7 +35,11 @@ struct SegGeom {
     // sorted, one run per partition from partition b_first on; -1 = everything
     int64_t tail_from;
     int b_first;
+    int float_ids;    // 1: ids are stored as float32 values in the same place
 };
+__device__ inline int32_t stored_id(int float_ids, uint32_t id) {
+    return float_ids ? __builtin_bit_cast(int32_t, (float)(int)id) : (int32_t)id;
+}
 
 __device__ inline unsigned long long pack_key(float key, uint32_t pos) {
     // key + 0.0f folds -0.0 into +0.0 so equal floats always tie on the id
@@ -70,7 +74,7 @@ __global__ void segsort_tile_kernel(const float* __restrict__ keys, SegGeom g,
         const unsigned long long w = s[j];
         if (FINAL) {
             skeys[base + j] = ord2f((uint32_t)(w >> 32));
-            sids[base + j] = (int32_t)(off + (uint32_t)w);
+            sids[base + j] = stored_id(g.float_ids, off + (uint32_t)w);
             if (lids) lids[base + j] = (uint16_t)(uint32_t)w;
         } else {
             packed[base + j] = w;
@@ -223,7 +227,7 @@ __global__ __launch_bounds__(kRadixThreads, (kRadixThreads == 256 && IPT > 45) ?
     __syncthreads();
     for (int j = tid; j < n; j += kRadixThreads) {
         const uint32_t id = stage16[j];
-        sids[base + j] = (int32_t)(off + id);
+        sids[base + j] = stored_id(g.float_ids, off + id);
         if (lids) lids[base + j] = (uint16_t)id;
         if (inv) inv[base + j] = pos_of[j];
     }
@@ -412,7 +416,7 @@ __global__ __launch_bounds__(NT, WPS) void segsort_radix1w_kernel(
     __syncthreads();
     for (int j = tid; j < n; j += NT) {
         const uint32_t id = stage16[j];
-        sids[base + j] = (int32_t)(off + id);
+        sids[base + j] = stored_id(g.float_ids, off + id);
         if (lids) lids[base + j] = (uint16_t)id;
         if (inv) inv[base + j] = pos_of[j];
     }
@@ -476,7 +480,7 @@ __device__ inline void merge_piece(MergeScratch& ms, const unsigned long long* _
                                    const unsigned long long* __restrict__ Bv, int64_t lb, int64_t d0, int64_t d1,
                                    unsigned long long* __restrict__ dst, int64_t out0, int64_t base, int64_t off,
                                    float* __restrict__ skeys, int32_t* __restrict__ sids,
-                                   uint16_t* __restrict__ inv, uint16_t* __restrict__ lids) {
+                                   uint16_t* __restrict__ inv, uint16_t* __restrict__ lids, int float_ids = 0) {
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
     const int cnt = (int)(d1 - d0);
     if (wave < 2) {
@@ -519,7 +523,7 @@ __device__ inline void merge_piece(MergeScratch& ms, const unsigned long long* _
             const unsigned long long w = ms.out[j];
             const int64_t e = base + out0 + j;
             skeys[e] = ord2f((uint32_t)(w >> 32));
-            sids[e] = (int32_t)(off + (uint32_t)w);
+            sids[e] = stored_id(float_ids, off + (uint32_t)w);
             if (inv) inv[base + (uint32_t)w] = (uint16_t)(out0 + j);
             if (lids) lids[e] = (uint16_t)(uint32_t)w;
         }
@@ -552,7 +556,7 @@ __global__ __launch_bounds__(kMergeThreads) void segsort_merge_kernel(
     const int64_t d0 = o0 - ps;                               // first output of this workgroup
     const int64_t d1 = min(d0 + kMergeChunk, la + lb);
     merge_piece(ms, src + base + a0, la, src + base + b0, lb, d0, d1, dst, ps + d0, base, off,
-                skeys, sids, inv, lids);
+                skeys, sids, inv, lids, g.float_ids);
 }
 
 // ---------------------------------------------------------------------------
@@ -689,7 +693,7 @@ static int next_pow2(int v) {
 
 int segsort(const float* d_keys, int64_t key_stride, int num_indices, int64_t n, int block_size,
             float* d_skeys, int32_t* d_sids, uint16_t* d_inv, uint16_t* d_lids, void* d_tmp,
-            hipStream_t s) {
+            hipStream_t s, bool float_ids) {
     if (n <= 0) return 0;
     if (key_stride < n) return fail(-1, "segsort: key rows overlap");
     SegGeom g;
@@ -701,6 +705,7 @@ int segsort(const float* d_keys, int64_t key_stride, int num_indices, int64_t n,
     g.tile_size = kTileCap;
     g.tail_from = -1;
     g.b_first = 0;
+    g.float_ids = float_ids ? 1 : 0;
     const int np2 = next_pow2((int)min((int64_t)kTileCap, g.ppb));
     // at most kTileCap / 1024 elements per thread (the inverse-permutation pass relies on it)
     const int threads = max(64, min(1024, np2 / 2));
@@ -857,6 +862,7 @@ int segsort_append(const float* d_old_skeys, const int32_t* d_old_sids, int64_t 
         g.kstride = key_stride; g.n = n1; g.B = block_size; g.ppb = ag.p1;
         g.tiles = 1; g.tile_size = 0;
         g.tail_from = n0;
+        g.float_ids = 0;
         g.b_first = (int)(n0 / ag.p1);
         int64_t longest = 0;                               // longest run of new points in one partition
         for (int b = g.b_first; b < block_size; b++)
