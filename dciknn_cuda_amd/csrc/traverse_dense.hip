@@ -63,10 +63,10 @@ struct DenseLayout {
     size_t lds_bytes;
 };
 
-// Buckets of the windows' ranking: about as many as windows, as far as two workgroups still fit a
-// CU's LDS beside ten thousand points.
+// Buckets of the windows' ranking: about as many as windows, 4096 at most: twice as many rank 7021 windows no
+// faster, and their 8 KB can be what keeps a second workgroup out of a CU (14000 points: 7.0 and 10.2 ms).
 constexpr int dense_bucket_bits(int cap) {
-    return cap <= 320 ? 8 : (cap <= 1280 ? 10 : (cap <= 2560 ? 11 : (cap <= 4608 || cap > 6656 ? 12 : 13)));
+    return cap <= 320 ? 8 : (cap <= 1280 ? 10 : (cap <= 2560 ? 11 : 12));
 }
 constexpr int kWlist = 2 * kWave;        // candidates a wavefront keeps listed
 
@@ -111,12 +111,12 @@ DenseLayout dense_layout_for(const QueryArgs& a, int nt, int ipt) {
     return y;
 }
 
-// Threads per workgroup and windows per thread; ipt = 0: too many windows.  With up to nine windows per
-// thread the registers allow 16 wavefronts per CU, and the kernel needs them all to hide its chains of LDS
-// and memory reads: one per workgroup where partitions are small, four where four workgroups' tables fit
-// a CU's LDS, else eight.  More windows per thread need twice the registers -- kept to 128, the ranking's
-// spills cost more than the wavefronts gain (7021 windows per composite, two workgroups per CU: 114 us per
-// item against 43) -- so there eight wavefronts per CU, of two workgroups as far as a thread can hold the windows.
+// Threads per workgroup and windows per thread; ipt = 0: too many windows.  With up to fifteen windows per
+// thread 128 registers do, which allow 16 wavefronts per CU, and the kernel needs them all to hide its chains
+// of LDS and memory reads: one per workgroup where partitions are small, four where four workgroups' tables
+// fit a CU's LDS, else eight (7021 windows per composite: 22.2 ms; four wavefronts per workgroup and eight per
+// CU 25.8).  With more, 128 registers spill in the ranking (17: 46 ms), so there eight wavefronts per CU, of
+// two workgroups as far as a thread can hold the windows.
 DenseLayout make_dense_layout(const QueryArgs& a) {
     const int64_t windows = dense_max_windows(a);
     if (a.ppb <= kNarrowPoints)
@@ -128,10 +128,9 @@ DenseLayout make_dense_layout(const QueryArgs& a) {
             if (4 * y.lds_bytes <= kLdsBytes) return y;
             break;
         }
-    for (int i : {5, 9})
+    for (int i : {5, 9, 13, 15})
         if (windows <= (int64_t)512 * i) return dense_layout_for(a, 512, i);
-    for (int i : {25, 33})
-        if (windows <= (int64_t)256 * i) return dense_layout_for(a, 256, i);
+    if (windows <= (int64_t)256 * 33) return dense_layout_for(a, 256, 33);
     if (windows <= (int64_t)512 * 21) return dense_layout_for(a, 512, 21);
     DenseLayout none;
     none.ipt = 0;
@@ -1269,7 +1268,7 @@ int query_dense_items(const QueryArgs& a_in, hipStream_t s) {
     a.q_first = 0;
     a.q_count = a.nq;
     // enough resident workgroups to fill the device, each striding over its die's items
-    const int by_regs = (y.ipt > 9 ? 512 : 1024) / y.nt;
+    const int by_regs = (y.ipt > 15 ? 512 : 1024) / y.nt;
     const int per_cu = (int)max((size_t)1, min((size_t)by_regs, kLdsBytes / y.lds_bytes));
     int64_t per_xcd = (int64_t)32 * per_cu * 2;
     const int64_t most = a.dense_items && a.mode != 3 ? (int64_t)a.dense_cap
@@ -1289,16 +1288,14 @@ int query_dense_items(const QueryArgs& a_in, hipStream_t s) {
     } while (0)
     if (y.nt == 64) {
         if (y.ipt == 5) DCIH_DENSE(64, 5, 4); else DCIH_DENSE(64, 9, 4);
-    } else if (y.nt == 512) {
-        if (y.ipt == 5) DCIH_DENSE(512, 5, 4); else if (y.ipt == 9) DCIH_DENSE(512, 9, 4); else DCIH_DENSE(512, 21, 2);
-    } else if (y.ipt == 5) {
-        DCIH_DENSE(256, 5, 4);
-    } else if (y.ipt == 9) {
-        DCIH_DENSE(256, 9, 4);
-    } else if (y.ipt == 25) {
-        DCIH_DENSE(256, 25, 2);
+    } else if (y.nt == 256) {
+        if (y.ipt == 5) DCIH_DENSE(256, 5, 4); else if (y.ipt == 9) DCIH_DENSE(256, 9, 4); else DCIH_DENSE(256, 33, 2);
+    } else if (y.ipt <= 9) {
+        if (y.ipt == 5) DCIH_DENSE(512, 5, 4); else DCIH_DENSE(512, 9, 4);
+    } else if (y.ipt <= 15) {
+        if (y.ipt == 13) DCIH_DENSE(512, 13, 4); else DCIH_DENSE(512, 15, 4);
     } else {
-        DCIH_DENSE(256, 33, 2);
+        DCIH_DENSE(512, 21, 2);
     }
 #undef DCIH_DENSE
     DCIH_HIP(hipGetLastError());
