@@ -38,7 +38,7 @@ namespace {
 constexpr uint32_t kNever = 0xffffu;     // step field of a point that is never promoted
 
 enum DMisc {   // 32-bit scalars shared by the workgroup
-    dWin = 0, dArmed, dMaxc, dCand, dProbes, dMore, dOr, dAnd, dMaxW, dMaxBits, dUse8,
+    dWin = 0, dArmed, dMaxc, dCand, dProbes, dMore, dOr, dAnd, dMaxW, dMaxBits, dUse8, dNoStep,
     dMiscWords = 16
 };
 
@@ -1014,9 +1014,11 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
             auto score = [&](unsigned long long e) {
                 return args->a.blind ? (float)(uint32_t)(e >> 32) : __builtin_bit_cast(float, (uint32_t)(e >> 32));
             };
+            // (compared as a number before it becomes a bin: a NaN, which sorts behind everything, must not
+            //  be counted among the nearest, where the conversion would put it)
             auto count = [&](bool keep, unsigned long long e) {
-                const int bin = max(0, (int)((score(e) - h_lo) * h_scale));
-                if (keep && bin < kBins) atomicAdd(&hist[bin], 1u);
+                const float at_bin = (score(e) - h_lo) * h_scale;
+                if (keep && at_bin < (float)kBins) atomicAdd(&hist[max(0, (int)at_bin)], 1u);
             };
             auto tighten = [&]() {
                 const u32x4 c = reinterpret_cast<const u32x4*>(hist)[lane];
