@@ -613,7 +613,6 @@ __device__ __forceinline__ void traverse_block_item(const QueryArgs& a, const Bl
             const uint32_t rho = s_rho[m];
             const Stream st = load_stream(active ? sidx : 0);
             bool more = active && c < ns && rho < kInfBits;
-            const bool searched = more;
             int lo = c, hi = c;
             int64_t span = 2 * (int64_t)(active ? s_stride[sidx] : 1);
             while (__any(more)) {
@@ -625,11 +624,16 @@ __device__ __forceinline__ void traverse_block_item(const QueryArgs& a, const Bl
                     else { lo = r; more = false; }
                 }
             }
-            // (NaN priorities: take the rest so the epoch loop ends)
-            const int cn = searched ? lo : (active && c < ns ? ns : c);
             if (active && g == 0) {
-                s_c[sidx] = cn;
-                atomicAdd(&s_K[m], (uint32_t)cn);
+                if (c < ns && rho >= kInfBits) {
+                    // Every stream of the composite is close to windows of no finite priority (rows that hold
+                    // infinities or NaN).  They are a stream's last and are never reached, because the loop takes
+                    // the first minimum below infinity (:466-478): the stream ends before them.
+                    lo = count_below(st, kInfBits, true, c, ns, probes);
+                    s_ns[sidx] = lo;
+                }
+                s_c[sidx] = lo;
+                atomicAdd(&s_K[m], (uint32_t)lo);
             }
         }
         __syncthreads();

@@ -318,7 +318,7 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
         __syncthreads();
         PHASE_END(0);
 
-        unsigned long long maxw = 0;             // most windows any composite has
+        unsigned long long maxw = 0;             // most windows any composite has a step for
         for (int m = 0; m < args->a.M; m++) {
             ArgsPtr args = fresh_args();
             DenseTables tb(smem, args->a, args->y);
@@ -362,6 +362,7 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
                 const int total = __shfl(incl, args->a.L - 1, kWave);
                 if (lane == 0) {
                     misc[dMaxBits] = 0;
+                    misc[dNoStep] = 0;
                     tb.seg[2 * args->a.L] = total;
                     misc[dWin] = (uint32_t)total;
                     misc[dOr] = 0; misc[dAnd] = 0xffffffffu;
@@ -369,11 +370,12 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
             }
             __syncthreads();
             const int W = __builtin_amdgcn_readfirstlane((int)misc[dWin]);
-            maxw = max(maxw, (unsigned long long)W);
 
             // The step of every window is its place in the order of priorities, stored doubled with bit 0
             // set: a lookup subtracts one where the point is not the window's first lane, which
-            // leaves the lane-0 flag beside the step.
+            // leaves the lane-0 flag beside the step.  A window whose priority is not finite (rows that hold
+            // infinities or NaN) is never reached: the loop takes the first minimum below infinity (:466-478).
+            // Such windows come last in the order and get kNever; their number is misc[dNoStep].
             bool few_windows = false;
             if constexpr (IPT <= 9) if (W <= 2 * NT) {
                 // ---- few windows: one or two per thread, as (priority, layout index, table place) words; the
@@ -400,12 +402,16 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
                         const float key = args->a.skeys[(int64_t)(m * args->a.L + h) * args->a.N + off + min(max(pos, 0), n - 1)];
                         const float prio = fabsf(key - tb.qp[m * args->a.L + h]);
                         word = ((unsigned long long)__builtin_bit_cast(uint32_t, prio) << 32) | ((uint32_t)idx << 16) | (uint32_t)place;
+                        if (__builtin_bit_cast(uint32_t, prio) >= kInfBits) atomicAdd(&misc[dNoStep], 1u);
                         probes++;
                     }
                     if (idx < np) s64[idx] = word;
                 }
                 __syncthreads();
                 PHASE_END(1);
+                auto step_of = [&](unsigned long long word, int at) {
+                    return (uint32_t)(word >> 32) < kInfBits ? (uint16_t)((at << 1) | 1) : (uint16_t)kNever;
+                };
                 auto by_one_wave = [&](auto etag) __attribute__((always_inline)) {
                     constexpr int E = decltype(etag)::value;
                     if (wave == 0) {
@@ -416,7 +422,7 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
                         __builtin_amdgcn_wave_barrier();                // the table takes the words' room
 #pragma unroll
                         for (int i = 0; i < E; i++)
-                            if (v[i] != ~0ull) tb.rank16[(uint32_t)v[i] & 0xffffu] = (uint16_t)(((lane * E + i) << 1) | 1);
+                            if (v[i] != ~0ull) tb.rank16[(uint32_t)v[i] & 0xffffu] = step_of(v[i], lane * E + i);
                     }
                 };
                 if (np == kWave) by_one_wave(std::integral_constant<int, 1>{});
@@ -433,7 +439,7 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
                         __syncthreads();                    // the table takes the sorted words' room
 #pragma unroll
                         for (int e = 0; e < 2; e++)
-                            if (e * NT + tid < W) tb.rank16[(uint32_t)mine[e] & 0xffffu] = (uint16_t)(((e * NT + tid) << 1) | 1);
+                            if (e * NT + tid < W) tb.rank16[(uint32_t)mine[e] & 0xffffu] = step_of(mine[e], e * NT + tid);
                     }
                 }
             }
@@ -570,16 +576,21 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
                 const uint32_t varying = misc[dOr] ^ misc[dAnd];
                 lds_radix_passes<NT, IPT>(k, rp, tb.stage, tb.stage + IPT * NT + 4, scan_tmp, varying);
                 __syncthreads();
+                uint32_t no_step = 0;
 #pragma unroll
                 for (int r = 0; r < IPT; r++) {
                     const int sp = tid * IPT + r;
-                    if (sp < W) tb.rank16[rp[r] & 0xffffu] = (uint16_t)((sp << 1) | 1);      // (the first W sorted items are the windows)
+                    const bool never = k[r] >= kInfBits;
+                    if (sp < W) tb.rank16[rp[r] & 0xffffu] = never ? (uint16_t)kNever : (uint16_t)((sp << 1) | 1);      // (the first W sorted items are the windows)
+                    no_step += sp < W && never ? 1u : 0u;
                 }
+                if (no_step) atomicAdd(&misc[dNoStep], no_step);
                 break;
             }
             __syncthreads();
             }
             __syncthreads();
+            maxw = max(maxw, (unsigned long long)(misc[dWin] - misc[dNoStep]));
             PHASE_END(2);
 
             // ---- every point: the latest of the steps of its L windows ------------------
