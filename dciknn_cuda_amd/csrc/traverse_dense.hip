@@ -57,6 +57,7 @@ struct DenseLayout {
     int off_sort;     // k best + pending candidates, 64-bit words
     int off_stage;
     int off_misc, off_wlist;
+    int whole_bytes;  // room from off_stage on for the results of one round
     int sort_cap, quota;
     int front8, quota8;   // the same buffer where rows are compared by their codes: words kept, entries per wavefront between two merges
     int tiles;        // 1: rows of at most 128 elements, 16-byte aligned, distances wanted: whole batches of 64 rows
@@ -69,6 +70,7 @@ constexpr int dense_bucket_bits(int cap) {
     return cap <= 320 ? 8 : (cap <= 1280 ? 10 : (cap <= 2560 ? 11 : 12));
 }
 constexpr int kWlist = 2 * kWave;        // candidates a wavefront keeps listed
+constexpr int kBins = 256;               // of the histogram of scores, which lies at the start of the staging words
 
 // Upper bound of the windows of one composite index: per simple index at most
 // ceil((p+1)/T) + floor((n+T-3-p)/T) + 1 <= n/T + 3.  (A layout holds that many, so every item fits it.)
@@ -104,8 +106,15 @@ DenseLayout dense_layout_for(const QueryArgs& a, int nt, int ipt) {
     y.off_stage = o;    o += (nt * ipt + 4) * 4;
     const int counters = o;
     o += ((1 << dense_bucket_bits(nt * ipt)) / 2 + 4) * 4;
+    // The ranking is over when the first candidate is kept: where its room holds the buffer of kept ones twice,
+    // the buffer lies in its upper half and the results of one round in its lower one.  (22223 points, 2640
+    // windows, k = 50: 74576 bytes, two workgroups per CU, 1.60 ms for 4096 items; with the buffer
+    // behind everything 82768 bytes, one, and 2.25.)
+    const bool inside = o - y.off_stage >= y.sort_cap * 8 + max(y.sort_cap * 8, kBins * 4);
+    y.off_sort = inside ? o - y.sort_cap * 8 : o + waves * kWlist * 2;
+    y.whole_bytes = (inside ? y.off_sort : o) - y.off_stage;
     y.off_wlist = o;    o += waves * kWlist * 2;
-    y.off_sort = o;     o += y.sort_cap * 8;
+    if (!inside) o += y.sort_cap * 8;
     o = max(o, counters + 8 * nt * 4);
     y.lds_bytes = (size_t)o;
     return y;
@@ -1009,7 +1018,6 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
         // Bound by the latency of the records' reads (eight 16-byte reads per lane under way).  12808 candidates
         // of 128 elements, k = 100, two workgroups per CU: 98 us per item, 207 by whole rows and a sort per
         // full buffer; 1325 of 512 elements: 69, and 426 by whole rows.
-        constexpr int kBins = 256;
         uint32_t* hist = tb.stage;
         unsigned long long cut = ~0ull;                         // entries above it are out
         unsigned long long pend = ~0ull;                        // lane's entry of a batch that did not fit the share
@@ -1156,7 +1164,7 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
                 added = __builtin_amdgcn_readfirstlane(added);
                 int np = added <= kWave ? kWave : NT;
                 while (np < added) np <<= 1;
-                if (np * 8 <= args->y.off_wlist - args->y.off_stage) {
+                if (np * 8 <= args->y.whole_bytes) {
                     whole = true;
                     left = added;
                     words = np;

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 # workgroup of 64, 256 or 512 threads holds at 5, 9, 13, 15, 33 and 21 windows per thread
 TABLES = [(1, 3, 2, 1), (7, 2, 2, 3), (314, 2, 2, 2), (316, 2, 2, 2), (378, 1, 3, 2), (512, 1, 3, 1), (513, 1, 3, 1),
           (1225, 2, 10, 10), (2031, 2, 9, 8), (2045, 1, 5, 4), (4072, 1, 9, 8), (4080, 1, 9, 8), (5103, 1, 10, 8), (5300, 1, 10, 8), (5565, 2, 11, 8),
-          (6127, 1, 11, 8), (6140, 2, 11, 8), (9000, 1, 3, 300)]
+          (6127, 1, 11, 8), (6140, 2, 11, 8), (9000, 1, 3, 300), (22223, 1, 15, 128)]
 
 
 @pytest.mark.parametrize("ppb,B,L,T", TABLES)
