@@ -183,7 +183,7 @@ typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) uint16_t lds_u16;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-struct DenseArgs { QueryArgs a; DenseLayout y; };
+struct DenseArgs { QueryArgs a; DenseLayout y; int run; };      // run: neighbouring items a workgroup takes; 0: it strides over all
 
 // Where the workgroup's tables lie in LDS.
 struct DenseTables {
@@ -265,10 +265,13 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
     const int T = args->a.T;
     const int X = args->a.xcds;
     const int xcd = (int)(blockIdx.x % X);
-    const int64_t g0 = blockIdx.x / X, G = gridDim.x / X;
+    const int64_t g0 = blockIdx.x / X;
     const bool listed = args->a.dense_items != nullptr && args->a.mode != 3;
     const int64_t my_count = listed ? (int64_t)args->a.dense_count[xcd]
                                     : block_items(X, args->a.B, args->a.q_count) / X;
+    const int items = args->run;
+    const int64_t slot_end = items > 0 ? min(my_count, (g0 + 1) * items) : my_count;
+    const int64_t slot_step = items > 0 ? 1 : (int64_t)(gridDim.x / X);
 
     // optional phase profile: thread 0 adds the 100 MHz ticks each phase took
     unsigned long long tick = 0ull;
@@ -280,7 +283,7 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
         }
     };
 
-    for (int64_t slot = g0; slot < my_count; slot += G) {
+    for (int64_t slot = items > 0 ? g0 * items : g0; slot < slot_end; slot += slot_step) {
         ArgsPtr args = fresh_args();
         DenseTables tb(smem, args->a, args->y);
         int b, qi;
@@ -1288,13 +1291,25 @@ int query_dense_items(const QueryArgs& a_in, hipStream_t s) {
     if (y.ipt == 0) return fail(-4, "query: this shape does not fit the dense traversal kernel");
     a.q_first = 0;
     a.q_count = a.nq;
-    // enough resident workgroups to fill the device, each striding over its die's items
+    // Items whose number only the device knows (a list), and few items, are shared out by strides among enough
+    // workgroups to fill the device.  Else one workgroup takes one item, or as short a run of neighbouring ones
+    // as a launch of 2^32 - 1 threads covers: workgroups start in order, so a die's resident ones work on
+    // neighbouring queries of one partition and its slices stay in the L2, where resident workgroups that stride
+    // over everything drift apart into several partitions (20M points, 900 partitions, 2000 queries: 984 ms by
+    // strides, 608 in order).  From eight times as many items as the die holds at a time in order is 0 to 13 %
+    // faster; below, starting more workgroups can cost up to 5 % (2000 points, 3200 items: 211 and 222 us), and
+    // so it can where registers leave one workgroup to a CU, which nothing covers while the next one
+    // starts (10000 points, 10030 windows: 390 and 397 ms).
     const int by_regs = (y.ipt > 15 ? 512 : 1024) / y.nt;
     const int per_cu = (int)max((size_t)1, min((size_t)by_regs, kLdsBytes / y.lds_bytes));
-    int64_t per_xcd = (int64_t)32 * per_cu * 2;
-    const int64_t most = a.dense_items && a.mode != 3 ? (int64_t)a.dense_cap
-                                                      : block_items(a.xcds, a.B, a.nq) / a.xcds;
-    per_xcd = max((int64_t)1, min(per_xcd, most));
+    const bool listed = a.dense_items && a.mode != 3;
+    const int64_t most = listed ? (int64_t)a.dense_cap : block_items(a.xcds, a.B, a.nq) / a.xcds;
+    int64_t per_xcd = max((int64_t)1, min((int64_t)32 * per_cu * 2, most));
+    int run = 0;
+    if (!listed && y.ipt <= 15 && most >= (int64_t)32 * per_cu * 8) {
+        run = (int)((most * a.xcds * y.nt + 0xfffffffeLL) / 0xffffffffLL);
+        per_xcd = (most + run - 1) / run;
+    }
     const unsigned grid = (unsigned)(per_xcd * a.xcds);
 #define DCIH_DENSE(NT, IPT, WAVES)                                                                 \
     do {                                                                                         \
@@ -1305,7 +1320,7 @@ int query_dense_items(const QueryArgs& a_in, hipStream_t s) {
             return 0;                                                                            \
         });                                                                                      \
         if (rc_attr) return rc_attr;                                                             \
-        hipLaunchKernelGGL((traverse_dense_kernel<NT, IPT, WAVES>), dim3(grid), dim3(NT), y.lds_bytes, s, DenseArgs{a, y}); \
+        hipLaunchKernelGGL((traverse_dense_kernel<NT, IPT, WAVES>), dim3(grid), dim3(NT), y.lds_bytes, s, DenseArgs{a, y, run}); \
     } while (0)
     if (y.nt == 64) {
         if (y.ipt == 5) DCIH_DENSE(64, 5, 4); else DCIH_DENSE(64, 9, 4);

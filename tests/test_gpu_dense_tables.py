@@ -54,3 +54,21 @@ def test_dense_tables(gpu, oracle, ppb, B, L, T, kind, dim):
     for (si, sd, sc), (di, dd, dc) in zip(got["step"], got["dense"]):
         assert torch.equal(si, di) and torch.equal(sd, dd)
         assert torch.equal(sc[:, 1], dc[:, 1])
+
+
+# items from eight times what the device holds on: one workgroup each, in order (narrow workgroups, wide ones)
+@pytest.mark.parametrize("ppb,B,nq", [(20, 37, 1100), (600, 13, 800), (3, 1, 40_000)])
+def test_many_items(gpu, ppb, B, nq):
+    rng = np.random.default_rng(ppb)
+    dim, M, L, T, k, outer = 8, 2, 3, 4, 10, 60
+    X = rng.standard_normal((ppb * B - 1, dim)).astype(np.float32)      # the last partition is one short
+    Q = torch.from_numpy(rng.standard_normal((nq, dim)).astype(np.float32)).cuda()
+    got = {}
+    for traversal in ("step", "dense"):
+        dci = gpu.DCI(dim, M, L, B, T, seed=3, traversal=traversal)
+        dci.add(torch.from_numpy(X).cuda())
+        got[traversal] = dci.query(Q, min(k, len(X)), outer, return_int=True, return_counters=True)
+        dci.free()
+    for j in (0, 1):
+        assert torch.equal(got["step"][j], got["dense"][j])
+    assert torch.equal(got["step"][2][:, [1, 3]], got["dense"][2][:, [1, 3]])
