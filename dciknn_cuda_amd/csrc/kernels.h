@@ -96,7 +96,7 @@ struct QueryArgs {
     const unsigned char* rows8;      // [N][rows8_rec]
     int rows8_rec;                   // bytes per record
     uint32_t* rows8_bounds;          // [B][2]: largest coding error and largest squared norm of a partition's rows (float
-                                     // bits), then [B]: 1 = codes found useless in this partition
+                                     // bits), then [B]: how many items the codes did not do for lately (traverse_dense.hip)
     const unsigned char* query8;     // [nq][rows8_query_bytes(dim)]
     int xcds;                // accelerator dies of the device (each has an L2 of its own)
     int q_first, q_count;    // batch kernel: the queries one launch covers

@@ -14,13 +14,15 @@ extern "C" {
 #endif
 
 /*
- * Phase profile of the batch traversal kernel (no counterpart in the
+ * Phase profile of the batch and dense traversal kernels (no counterpart in the
  * reference).  d_ticks is NULL (off) or a zeroed device array of 16 uint64 that
  * later dcih_query calls add to: [0..7] = 100 MHz ticks one thread of every
  * workgroup spent in set-up, bound selection, range search, streaming, undo,
  * promotion ranking, replay, distances/top-k; [8] = epochs, [9] = items finished by
  * the batch kernel (either pass), [10] = items it handed back (to its second pass with
- * the full tables, or to the step-by-step kernel), [11..14] = those by reason.
+ * the full tables, or to the step-by-step kernel), [11..14] = those by reason.  The dense
+ * kernel adds to [0..5] set-up, priorities, ranking, lookups, stop step, distances/top-k, to
+ * [9] its items and to [15] those of them it compared by their rows' 8-bit codes.
  */
 int dcih_phase_profile(dcih_index* h, uint64_t* d_ticks);
 
