@@ -142,11 +142,6 @@ struct dcih_index {
     float* d_ukeys = nullptr;           // [I][own_rows] unsorted projections of the rows in d_own
     int64_t own_rows = 0;               // capacity of d_own / d_ukeys in rows
     int64_t ukeys_rows = 0;             // leading rows of d_own whose projections d_ukeys holds
-    // the stream every call since the last wait for the device has used; `many`: there were several, or a call
-    // was recorded into a graph (which may be replayed on any)
-    hipStream_t used_stream = nullptr;
-    bool used_any = false, used_many = false;
-    bool cleared_behind = false;        // dcih_clear did not wait for work under way on used_stream
     float* d_stop_hint = nullptr;       // [3][block_size] epoch-size hints learnt from earlier queries
     int hint_k = 0, hint_outer = 0, hint_T = 0, hint_maxc = 0;   // query shape the hints belong to (zeros: none, as after a build)
     int traversal = 0;                  // DCIH_OPT_TRAVERSAL value
@@ -237,26 +232,6 @@ int release_index(dcih_index* h) {
 bool capturing(hipStream_t s) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
-}
-
-void note_stream(dcih_index* h, hipStream_t s) {
-    if ((h->used_any && h->used_stream != s) || capturing(s)) h->used_many = true;
-    h->used_stream = s;
-    h->used_any = true;
-}
-
-int wait_for_device(dcih_index* h) {
-    DCIH_HIP(hipDeviceSynchronize());
-    h->used_any = h->used_many = h->cleared_behind = false;
-    return 0;
-}
-
-// Before work on stream `s` that overwrites what the calls before dcih_clear may still be reading.
-int settle_clear(dcih_index* h, hipStream_t s) {
-    if (!h->cleared_behind) return 0;
-    if (s != h->used_stream) return wait_for_device(h);
-    h->cleared_behind = false;
-    return 0;
 }
 
 int ensure_ws(dcih_index* h, size_t bytes, hipStream_t s) {
@@ -399,10 +374,6 @@ int dcih_set_directions(dcih_index* h, const float* h_dirs) {
     if (!h || !h_dirs) return fail(DCIH_EINVAL, "dcih_set_directions: null argument");
     if (h->n > 0) return fail(DCIH_ESTATE, "dcih_set_directions: index is not empty");
     DeviceGuard guard(h->device);
-    if (h->cleared_behind) {
-        const int rc = wait_for_device(h);
-        if (rc) return rc;
-    }
     std::memcpy(h->h_dirs.data(), h_dirs, h->h_dirs.size() * sizeof(float));
     DCIH_HIP(hipMemcpy(h->d_dirs, h_dirs, h->h_dirs.size() * sizeof(float), hipMemcpyHostToDevice));
     return DCIH_OK;
@@ -468,11 +439,8 @@ int dcih_add(dcih_index* h, int dim, int64_t num_points, const float* d_data,
     // (the unsorted keys): a rebuild of the same size allocates and frees nothing
     const size_t b_keys = align_up((size_t)I * num_points * sizeof(float));
     const size_t tmp_bytes = segsort_tmp_bytes(I, num_points, block_size);
-    int rc = settle_clear(h, s);
-    if (rc) return rc;
-    note_stream(h, s);
     release_rows(h);                // (rows of appends before a clear: this index borrows its rows)
-    rc = ensure_arena(h, h->cur, arena_layout(I, num_points, block_size, dim).total);
+    int rc = ensure_arena(h, h->cur, arena_layout(I, num_points, block_size, dim).total);
     if (rc == DCIH_OK) rc = ensure_ws(h, b_keys + align_up(tmp_bytes), s);
     if (rc == DCIH_OK) {
         float* d_keys = (float*)h->ws;
@@ -521,9 +489,6 @@ int dcih_append(dcih_index* h, int dim, int64_t num_points, const float* d_data,
                        segsort_append_supported(h->n, total, block_size);
     if (h->append_mode == 2 && h->n > 0 && !merge)
         return fail(DCIH_EUNSUPPORTED, "dcih_append: this shape cannot be appended by merging (partitions too long)");
-    int rc = settle_clear(h, s);
-    if (rc) return rc;
-    note_stream(h, s);
     float* fresh_rows = nullptr;
     float* fresh_keys = nullptr;
     if (!rows || cap < total) {
@@ -538,7 +503,7 @@ int dcih_append(dcih_index* h, int dim, int64_t num_points, const float* d_data,
         ukeys = fresh_keys;
     }
     const size_t tmp_bytes = merge ? segsort_append_tmp_bytes(I, total) : segsort_tmp_bytes(I, total, block_size);
-    rc = ensure_arena(h, h->n > 0 ? spare : h->cur,
+    int rc = ensure_arena(h, h->n > 0 ? spare : h->cur,
                           std::max(arena_layout(I, total, block_size, dim).total,
                                    arena_layout(I, cap, block_size, dim).total));
     if (rc == DCIH_OK && tmp_bytes) rc = ensure_ws(h, align_up(tmp_bytes), s);
@@ -609,7 +574,6 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     if (num_queries == 0) return DCIH_OK;
     DeviceGuard guard(h->device);
     hipStream_t s = (hipStream_t)stream;
-    note_stream(h, s);
     const int I = num_indices(h);
     // the scratch of this call: the handle's workspace, grown as needed, or the static array
     char* ws_base = nullptr;
@@ -927,15 +891,9 @@ int64_t dcih_num_points(const dcih_index* h) { return h ? h->n : 0; }
 int dcih_clear(dcih_index* h) {
     if (!h) return fail(DCIH_EINVAL, "dcih_clear: null handle");
     DeviceGuard guard(h->device);
-    // Borrowed rows are the caller's again when this returns, so nothing may be reading them.  Rows
-    // the index owns stay with it: where all work under way is on one stream, what comes next on it
-    // comes after that work anyway (a call on another stream, or with new directions, waits first).
-    if (h->used_many || h->d_data != h->d_own) {
-        const int rc = wait_for_device(h);
-        if (rc) return rc;
-    } else if (h->used_any) {
-        h->cleared_behind = true;
-    }
+    // Borrowed rows are the caller's again when this returns, and rows the index owns are what the next append
+    // writes, on whatever stream: nothing may be reading them.
+    DCIH_HIP(hipDeviceSynchronize());
     return release_index(h);
 }
 
@@ -943,7 +901,6 @@ int dcih_reset(dcih_index* h) {
     const int rc = dcih_clear(h);
     if (rc) return rc;
     DeviceGuard guard(h->device);
-    DCIH_HIP(hipDeviceSynchronize());
     return draw_directions(h);
 }
 

@@ -1,0 +1,97 @@
+"""What a handle keeps from one call to the next, over streams: clear while queries are under way and
+what comes after it on the same stream, another one, with new directions or by `add`."""
+import threading
+
+import numpy as np
+import pytest
+import torch
+
+from util import engine_index
+
+pytestmark = pytest.mark.gpu
+
+DIM, M, L, B, T, K, OUTER = 64, 2, 7, 40, 10, 10, 2000
+PER_THREAD = 2          # hipStreamPerThread
+
+
+def _rows(seed, n):
+    return torch.randn(n, DIM, generator=torch.Generator().manual_seed(seed)).cuda()
+
+
+def _query(dci, Q, stream, nn, dists):
+    from dciknn_cuda_amd import _capi
+    _capi.check(dci._lib.dcih_query(dci._dci_inst, DIM, Q.shape[0], Q.data_ptr(), K, 0, OUTER, 10 * K, B, T,
+                                    nn.data_ptr(), dists.data_ptr(), None, stream))
+
+
+def _append(dci, X, stream):
+    from dciknn_cuda_amd import _capi
+    _capi.check(dci._lib.dcih_append(dci._dci_inst, DIM, X.shape[0], X.data_ptr(), B, T, stream))
+    dci.num_points += X.shape[0]
+
+
+def _out(Q):
+    return (torch.full((Q.shape[0], K), -7, dtype=torch.int32, device="cuda"),
+            torch.full((Q.shape[0], K), -7.0, device="cuda"))
+
+
+def _same(a, b):
+    return all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("then", ["same stream", "other stream", "per-thread stream", "new directions", "add"])
+def test_clear_while_a_query_is_under_way(gpu, then):
+    X1, X2, Q = _rows(1, 200_000), _rows(2, 200_000), _rows(3, 2000)
+    one, two = gpu.DCI(DIM, M, L, B, T, seed=7), gpu.DCI(DIM, M, L, B, T, seed=7)
+    other_dirs = gpu.DCI(DIM, M, L, B, T, seed=8).directions
+    one.add(X1)
+    if then == "new directions":
+        two.directions = other_dirs
+    two.add(X2)
+    want1, want2 = _out(Q), _out(Q)
+    _query(one, Q, 0, *want1)
+    _query(two, Q, 0, *want2)
+    torch.cuda.synchronize()
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    first = PER_THREAD if then == "per-thread stream" else a.cuda_stream
+    second = {"other stream": b.cuda_stream, "per-thread stream": PER_THREAD}.get(then, a.cuda_stream)
+    dci = gpu.DCI(DIM, M, L, B, T, seed=7)
+    _append(dci, X1, first)
+    _query(dci, Q, first, *_out(Q))           # (the workspace has its size now)
+    got1, got2 = _out(Q), _out(Q)
+    torch.cuda.synchronize()
+
+    begun, over = threading.Event(), threading.Event()
+
+    def begin():
+        for _ in range(8):                    # (milliseconds of work)
+            _query(dci, Q, first, *got1)
+        begun.set()
+        over.wait(60)                         # (a thread's own stream lives as long as the thread)
+
+    def go_on():
+        dci.clear()
+        if then == "new directions":
+            dci.directions = other_dirs
+        if then == "add":
+            with torch.cuda.stream(a):
+                dci.add(X2)
+        else:
+            _append(dci, X2, second)
+        _query(dci, Q, second, *got2)
+
+    t = threading.Thread(target=begin)        # (another thread: so is its per-thread stream)
+    t.start()
+    assert begun.wait(60)
+    go_on()
+    torch.cuda.synchronize()
+    over.set()
+    t.join()
+    assert _same(got1, want1)
+    assert _same(got2, want2)
+    keys, ids = engine_index(dci)
+    keys2, ids2 = engine_index(two)
+    np.testing.assert_array_equal(keys, keys2)
+    np.testing.assert_array_equal(ids, ids2)
+    for d in (one, two, dci):
+        d.free()
