@@ -75,6 +75,9 @@ constexpr int kWlist = 2 * kWave;        // candidates a wavefront keeps listed
 // kRest items, then one item tries them again: a partition whose rows lie too close together for their codes
 // costs one wasted attempt in kRest + 1, and a query far outside the data costs its own items only.
 constexpr int kGiveUp = 16, kRest = 64;
+// How an item takes the codes (misc[dUse8]): not at all, with no doubt about them, with some, as the one that tries again.
+// kCodesFailed is added when they did not do.
+enum { kCodesOff = 0, kCodesOn, kCodesDoubted, kCodesTried, kCodesFailed };
 constexpr int kBins = 256;               // of the histogram of scores, which lies at the start of the staging words
 
 // Upper bound of the windows of one composite index: per simple index at most
@@ -331,6 +334,20 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
                                                      [&](int j) { return key[j] < qp; }, probes);
                 if (active && lane == sl * Gq) { tb.p[i] = lo - 1; tb.qp[i] = qp; }
             }
+        }
+        if (args->a.rows8 && tid == 0) {          // (other items change the word meanwhile: one thread decides)
+            int* doubt = reinterpret_cast<int*>(args->a.rows8_bounds) + 2 * args->a.B + b;
+            int have = __hip_atomic_load(doubt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            uint32_t use = have <= 0 ? kCodesOn : (have < kGiveUp ? kCodesDoubted : kCodesOff);
+            for (int tries = 0; tries < 8 && use == kCodesOff && have > kGiveUp; tries++) {      // counts the rest down
+                const int was = atomicCAS(doubt, have, have - 1);
+                if (was == have) {
+                    if (have == kGiveUp + 1) use = kCodesTried;
+                    break;
+                }
+                have = was;
+            }
+            misc[dUse8] = use;
         }
         __syncthreads();
         PHASE_END(0);
@@ -919,32 +936,15 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
         enum { kBlind = 1, kRows = 8, kRows16 = 16, kRows32 = 32, kCodes8 = 108, kCodes16 = 116, kCodes64 = 164 };
         int path = args->a.blind ? kBlind : (!args->y.tiles ? kRows : (args->a.dim <= 64 ? kRows16 : kRows32));
         float q_scale = 0.f, q_n2 = 0.f, err = 0.f, delta = 0.f;
-        // How this item takes the codes: 0 not at all, 1 no item gave up lately, 2 some did, 3 as the one that tries again.
-        enum { kCodesOff = 0, kCodesOn, kCodesDoubted, kCodesTried };
         if (args->a.rows8) {
             const float* qh = reinterpret_cast<const float*>(qrec);
             q_scale = qh[0]; q_n2 = qh[1];
             err = __builtin_bit_cast(float, args->a.rows8_bounds[2 * b]) + qh[2];
             delta = (__builtin_bit_cast(float, args->a.rows8_bounds[2 * b + 1]) + q_n2) * 9.5367431640625e-7f;   // 2^-20
             q_scale = uniform_f32(q_scale); q_n2 = uniform_f32(q_n2); err = uniform_f32(err); delta = uniform_f32(delta);
-            if (err < 1e30f && delta < 1e30f) {
-                if (tid == 0) {          // (other items change the word meanwhile: one thread decides)
-                    int* doubt = reinterpret_cast<int*>(args->a.rows8_bounds) + 2 * args->a.B + b;
-                    int have = __hip_atomic_load(doubt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    uint32_t use = have <= 0 ? kCodesOn : (have < kGiveUp ? kCodesDoubted : kCodesOff);
-                    for (int tries = 0; tries < 8 && use == kCodesOff && have > kGiveUp; tries++) {      // counts the rest down
-                        const int was = atomicCAS(doubt, have, have - 1);
-                        if (was == have) {
-                            if (have == kGiveUp + 1) use = kCodesTried;
-                            break;
-                        }
-                        have = was;
-                    }
-                    misc[dUse8] = use;
-                }
-                __syncthreads();
-                if (__builtin_amdgcn_readfirstlane((int)misc[dUse8]) != kCodesOff)
-                    path = code_bytes <= 128 ? kCodes8 : (code_bytes <= 256 ? kCodes16 : kCodes64);
+            if (__builtin_amdgcn_readfirstlane((int)misc[dUse8]) != kCodesOff) {
+                if (err < 1e30f && delta < 1e30f) path = code_bytes <= 128 ? kCodes8 : (code_bytes <= 256 ? kCodes16 : kCodes64);
+                else if (tid == 0) misc[dUse8] |= kCodesFailed;      // (no useful codes of these rows, or of this query)
             }
         }
         auto limit = [&](float d) {
@@ -1251,12 +1251,7 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
             if (topn > front) {
                 // more has to be kept than the buffer holds: these rows lie too close together, as seen from this
                 // query, for their codes; whole rows for this item
-                if (tid == 0) {
-                    int* doubt = reinterpret_cast<int*>(args->a.rows8_bounds) + 2 * args->a.B + b;
-                    const int have = __hip_atomic_load(doubt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    if (misc[dUse8] == kCodesTried) atomicExch(doubt, kGiveUp + kRest);
-                    else if (have < kGiveUp && atomicAdd(doubt, 1) >= kGiveUp - 1) atomicMax(doubt, kGiveUp + kRest);
-                }
+                if (tid == 0) misc[dUse8] |= kCodesFailed;
                 path = !args->y.tiles ? kRows : (args->a.dim <= 64 ? kRows16 : kRows32);
                 at = wave_u * chunk;
                 list_len = list_pos = topn = batches = 0;
@@ -1272,19 +1267,22 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
                 last = true;
             }
         }
-        if (path >= kCodes8 && tid == 0) {
-            if (misc[dUse8] >= kCodesDoubted) {          // (the codes did)
-                int* doubt = reinterpret_cast<int*>(args->a.rows8_bounds) + 2 * args->a.B + b;
-                const int have = __hip_atomic_load(doubt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (misc[dUse8] == kCodesTried) atomicExch(doubt, 0);
-                else if (have > 0 && have < kGiveUp && atomicSub(doubt, 1) <= 0) atomicAdd(doubt, 1);
-            }
-            if (args->a.phase_ticks) atomicAdd(&args->a.phase_ticks[15], 1ull);
-        }
         if (lane == 0) atomicAdd(&misc[dCand], ncand);
         for (int j = tid; j < args->a.kcap; j += NT) part_out[j] = j < topn ? res[j] : ~0ull;
         PHASE_END(5);
         if (args->a.phase_ticks && tid == 0) atomicAdd(&args->a.phase_ticks[9], 1ull);
+        if (tid == 0 && misc[dUse8] != kCodesOff) {
+            const uint32_t use = misc[dUse8];
+            if (use != kCodesOn) {
+                int* doubt = reinterpret_cast<int*>(args->a.rows8_bounds) + 2 * args->a.B + b;
+                const int have = __hip_atomic_load(doubt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (use == kCodesTried) atomicExch(doubt, 0);
+                else if (use == kCodesTried + kCodesFailed) atomicExch(doubt, kGiveUp + kRest);
+                else if (use > kCodesFailed) { if (have < kGiveUp && atomicAdd(doubt, 1) >= kGiveUp - 1) atomicMax(doubt, kGiveUp + kRest); }
+                else if (have > 0 && have < kGiveUp && atomicSub(doubt, 1) <= 0) atomicAdd(doubt, 1);
+            }
+            if (args->a.phase_ticks && use < kCodesFailed) atomicAdd(&args->a.phase_ticks[15], 1ull);
+        }
 
         // ---- hints for the batch kernel's routing, counters -----------------------------
         __syncthreads();
