@@ -129,15 +129,13 @@ struct dcih_index {
     uint16_t* d_rpos = nullptr;         // [I][n] the same, in the order of each composite's first simple index (room kept by the
                                         // build, filled by the first query that runs the batch traversal kernel)
     int rpos_ready = 0;
-    // 8-bit codes of the rows (room kept by the build, filled once the dense kernel's calls have asked
-    // for more candidate rows than forming them costs; rows8.hip)
+    // 8-bit codes of the rows and the partitions' bounds behind them (rows8.hip): room taken and codes formed
+    // once the dense kernel's calls have asked for more candidate rows than forming them costs
     unsigned char* d_rows8 = nullptr;
-    uint32_t* d_rows8_bounds = nullptr;
+    size_t rows8_bytes = 0;
     double rows8_demand = 0.0;          // candidate rows asked for so far
     bool rows8_ready = false;
-    hipStream_t rows8_stream = nullptr; // where they were formed, and the event that says when
-    hipEvent_t rows8_event = nullptr;
-    bool rows8_settled = false;         // the event has been seen to be over
+    bool rows8_no_room = false;         // there was no memory for them: not asked for again until the next build
     float* d_own = nullptr;             // rows copied in by dcih_append (the index owns these)
     float* d_ukeys = nullptr;           // [I][own_rows] unsorted projections of the rows in d_own
     int64_t own_rows = 0;               // capacity of d_own / d_ukeys in rows
@@ -190,6 +188,17 @@ int draw_directions(dcih_index* h) {
     return 0;
 }
 
+// The rows change: their codes are formed anew, in the same room if it holds them.
+void forget_rows8(dcih_index* h) {
+    h->rows8_ready = h->rows8_no_room = false;
+    h->rows8_demand = 0.0;
+}
+
+void release_rows8(dcih_index* h) {
+    forget_rows8(h);
+    if (h->d_rows8) { (void)hipFree(h->d_rows8); h->d_rows8 = nullptr; h->rows8_bytes = 0; }
+}
+
 // Drops the sorted arrays (their arena stays allocated for the next build) but keeps the rows.
 int release_sorted(dcih_index* h) {
     h->d_skeys = nullptr;
@@ -197,10 +206,7 @@ int release_sorted(dcih_index* h) {
     h->d_inv = nullptr;
     h->d_rpos = nullptr;
     h->rpos_ready = 0;
-    h->d_rows8 = nullptr;
-    h->d_rows8_bounds = nullptr;
-    h->rows8_ready = false;
-    h->rows8_demand = 0.0;
+    forget_rows8(h);
     h->d_stop_hint = nullptr;
     return 0;
 }
@@ -259,10 +265,10 @@ int ensure_arena(dcih_index* h, int which, size_t bytes) {
 
 // Where the arrays of an index of n points lie inside an arena.
 struct ArenaLayout {
-    size_t keys, ids, inv, rpos, hint, rows8, bounds8, total;   // byte offsets, and the size of it all
+    size_t keys, ids, inv, rpos, hint, total;   // byte offsets, and the size of it all
     bool small_parts;                           // partitions of at most 65536 points: 16-bit tables exist
 };
-ArenaLayout arena_layout(int I, int64_t n, int block_size, int dim) {
+ArenaLayout arena_layout(int I, int64_t n, int block_size) {
     ArenaLayout y;
     const size_t cells = (size_t)I * (size_t)n;
     y.small_parts = (n + block_size - 1) / block_size <= 65536;
@@ -276,36 +282,42 @@ ArenaLayout arena_layout(int I, int64_t n, int block_size, int dim) {
     y.inv = y.ids + b_ids;
     y.rpos = y.inv + b_inv;
     y.hint = y.rpos + b_inv;
-    y.rows8 = y.hint + b_hint;
-    y.bounds8 = y.rows8 + (rows8_supported(dim) ? align_up((size_t)n * rows8_record_bytes(dim)) : 0);
-    y.total = y.bounds8 + (rows8_supported(dim) ? align_up((size_t)3 * block_size * sizeof(uint32_t) + 8) : 0);
+    y.total = y.hint + b_hint;
     return y;
+}
+
+size_t rows8_records(const dcih_index* h, int64_t n) { return align_up((size_t)n * rows8_record_bytes(h->dim)); }
+size_t rows8_room(const dcih_index* h, int64_t n, int block_size) {
+    return rows8_records(h, n) + align_up((size_t)3 * block_size * sizeof(uint32_t) + 8);
 }
 
 // Whether a call on stream `s` that goes to the dense kernel may compare rows by their codes; forms
 // the codes when they have become worth it: a candidate read by its code saves three quarters of its row,
 // forming the codes reads every row and writes a quarter of it, so from twice as many candidates as rows on.
+// The call that forms them waits for them, so that later ones may come on any stream.
 int use_rows8(dcih_index* h, double candidates, bool may_form, hipStream_t s, bool& use) {
     use = false;
-    if (!h->d_rows8) return 0;
+    if (!rows8_supported(h->dim) || h->rows8_no_room) return 0;
     h->rows8_demand += candidates;
     if (!h->rows8_ready) {
         if (!may_form || h->rows8_demand < 2.0 * (double)h->n || capturing(s)) return 0;
-        if (!h->rows8_event) DCIH_HIP(hipEventCreateWithFlags(&h->rows8_event, hipEventDisableTiming));
-        const int64_t ppb = (h->n + h->block_size - 1) / h->block_size;
-        const int rc = code_rows(h->d_data, h->n, h->dim, ppb, h->block_size, h->d_rows8, h->d_rows8_bounds, s);
-        if (rc) return rc;
-        DCIH_HIP(hipEventRecord(h->rows8_event, s));
-        h->rows8_stream = s;
-        h->rows8_ready = true;
-        h->rows8_settled = false;
-    } else if (!h->rows8_settled && s != h->rows8_stream) {
-        if (capturing(s)) return 0;
-        if (hipEventQuery(h->rows8_event) == hipSuccess) h->rows8_settled = true;
-        else {
-            (void)hipGetLastError();
-            DCIH_HIP(hipStreamWaitEvent(s, h->rows8_event, 0));
+        const size_t need = rows8_room(h, h->n, h->block_size);
+        if (need > h->rows8_bytes) {
+            if (h->d_rows8) { DCIH_HIP(hipFree(h->d_rows8)); h->d_rows8 = nullptr; h->rows8_bytes = 0; }
+            if (hipMalloc((void**)&h->d_rows8, need) != hipSuccess) {      // whole rows do as well
+                (void)hipGetLastError();
+                h->d_rows8 = nullptr;
+                h->rows8_no_room = true;
+                return 0;
+            }
+            h->rows8_bytes = need;
         }
+        const int64_t ppb = (h->n + h->block_size - 1) / h->block_size;
+        const int rc = code_rows(h->d_data, h->n, h->dim, ppb, h->block_size, h->d_rows8,
+                                 (uint32_t*)(h->d_rows8 + rows8_records(h, h->n)), s);
+        if (rc) return rc;
+        DCIH_HIP(hipStreamSynchronize(s));
+        h->rows8_ready = true;
     }
     use = true;
     return 0;
@@ -389,7 +401,7 @@ static int sort_into(dcih_index* h, int which, const float* d_keys, int64_t key_
                      int64_t num_points, const float* d_data, int block_size, void* d_tmp,
                      hipStream_t s, int64_t merge_from = 0) {
     const int I = num_indices(h);
-    const ArenaLayout y = arena_layout(I, num_points, block_size, h->dim);
+    const ArenaLayout y = arena_layout(I, num_points, block_size);
     char* base = (char*)h->arena[which];
     float* skeys = (float*)(base + y.keys);
     int32_t* sids = (int32_t*)(base + y.ids);
@@ -411,10 +423,7 @@ static int sort_into(dcih_index* h, int which, const float* d_keys, int64_t key_
     h->d_skeys = skeys; h->d_sids = sids; h->d_inv = inv; h->d_stop_hint = hint;
     h->d_rpos = y.small_parts ? (uint16_t*)(base + y.rpos) : nullptr;
     h->rpos_ready = 0;
-    h->d_rows8 = rows8_supported(h->dim) ? (unsigned char*)(base + y.rows8) : nullptr;
-    h->d_rows8_bounds = rows8_supported(h->dim) ? (uint32_t*)(base + y.bounds8) : nullptr;
-    h->rows8_ready = false;
-    h->rows8_demand = 0.0;
+    forget_rows8(h);
     h->cur = which;
     h->d_data = d_data;
     h->n = num_points;
@@ -440,7 +449,8 @@ int dcih_add(dcih_index* h, int dim, int64_t num_points, const float* d_data,
     const size_t b_keys = align_up((size_t)I * num_points * sizeof(float));
     const size_t tmp_bytes = segsort_tmp_bytes(I, num_points, block_size);
     release_rows(h);                // (rows of appends before a clear: this index borrows its rows)
-    int rc = ensure_arena(h, h->cur, arena_layout(I, num_points, block_size, dim).total);
+    if (h->rows8_bytes < rows8_room(h, num_points, block_size)) release_rows8(h);
+    int rc = ensure_arena(h, h->cur, arena_layout(I, num_points, block_size).total);
     if (rc == DCIH_OK) rc = ensure_ws(h, b_keys + align_up(tmp_bytes), s);
     if (rc == DCIH_OK) {
         float* d_keys = (float*)h->ws;
@@ -489,6 +499,8 @@ int dcih_append(dcih_index* h, int dim, int64_t num_points, const float* d_data,
                        segsort_append_supported(h->n, total, block_size);
     if (h->append_mode == 2 && h->n > 0 && !merge)
         return fail(DCIH_EUNSUPPORTED, "dcih_append: this shape cannot be appended by merging (partitions too long)");
+    // (codes of the rows so far are not the next index's; their room goes where it will not hold its codes)
+    if (h->rows8_bytes < rows8_room(h, total, block_size)) release_rows8(h);
     float* fresh_rows = nullptr;
     float* fresh_keys = nullptr;
     if (!rows || cap < total) {
@@ -504,8 +516,8 @@ int dcih_append(dcih_index* h, int dim, int64_t num_points, const float* d_data,
     }
     const size_t tmp_bytes = merge ? segsort_append_tmp_bytes(I, total) : segsort_tmp_bytes(I, total, block_size);
     int rc = ensure_arena(h, h->n > 0 ? spare : h->cur,
-                          std::max(arena_layout(I, total, block_size, dim).total,
-                                   arena_layout(I, cap, block_size, dim).total));
+                          std::max(arena_layout(I, total, block_size).total,
+                                   arena_layout(I, cap, block_size).total));
     if (rc == DCIH_OK && tmp_bytes) rc = ensure_ws(h, align_up(tmp_bytes), s);
     hipError_t e = hipSuccess;
     if (rc == DCIH_OK && h->n > 0 && rows != h->d_data)        // rows (and projections) indexed so far
@@ -680,7 +692,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
         const int rc8 = use_rows8(h, all_dense ? (double)num_queries * block_size * per_item : 0.0, all_dense && !fixed, s, use);
         if (rc8) return rc8;
         if (use) {
-            a.rows8 = h->d_rows8; a.rows8_rec = rows8_record_bytes(dim); a.rows8_bounds = h->d_rows8_bounds;
+            a.rows8 = h->d_rows8; a.rows8_rec = rows8_record_bytes(dim); a.rows8_bounds = (uint32_t*)(h->d_rows8 + rows8_records(h, h->n));
             if (dense_traversal_supported(a, nullptr)) q8_bytes = align_up((size_t)num_queries * rows8_query_bytes(dim));
             else a.rows8 = nullptr;      // (no room for the longer list of what is kept)
         }
@@ -910,11 +922,11 @@ int dcih_free(dcih_index* h) {
     (void)hipDeviceSynchronize();
     (void)release_index(h);
     release_rows(h);
+    release_rows8(h);
     (void)release_arena(h);
     if (h->ws) (void)hipFree(h->ws);
     if (h->d_dirs) (void)hipFree(h->d_dirs);
     for (auto& e : h->ev) if (e) (void)hipEventDestroy(e);
-    if (h->rows8_event) (void)hipEventDestroy(h->rows8_event);
     delete h;
     return DCIH_OK;
 }

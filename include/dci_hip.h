@@ -168,6 +168,14 @@ int dcih_append(dcih_index* h, int dim, int64_t num_points, const float* d_data,
  * in a row of num_points cells per query and the rows are sorted; both paths work
  * through the queries in chunks and use up to 2 GB of workspace.
  *
+ * The call may allocate: its workspace grows to the largest call's, and where the dense
+ * kernel's calls have asked for twice as many candidates as there are rows of 96 to 1024
+ * elements, the call that gets there forms 8-bit codes of the rows, about a quarter of
+ * their size, and waits for them (without memory for them whole rows are compared).
+ * Later calls compare rows by their codes first; results do not depend on it.  Under
+ * stream capture nothing is allocated and no codes are formed; what calls before the
+ * capture have allocated and formed is used.
+ *
  * blind != 0 (query_config.blind, :498-505, :754-773, :859-864): the same
  * traversal under the same stop rule, but no distance is computed.  d_nn is
  * [num_queries][R] with R = min(max_num_candidates, num_outer_iterations), the
@@ -218,7 +226,9 @@ int dcih_query_float_ids(dcih_index* h, int dim, int num_queries, const float* d
  * than 8192 results per query return DCIH_EUNSUPPORTED.  All calls on one GPU
  * share that GPU's array: calls that overlap in time on the same GPU (different
  * streams or threads) race and must be serialised by the caller; a call that
- * follows another on the same stream is safe, it overwrites what it uses.
+ * follows another on the same stream is safe, it overwrites what it uses.  It uses
+ * 8-bit codes of the rows that calls of dcih_query have formed (see there) and forms none:
+ * a program that serves long rows through it lets dcih_query answer its first batches.
  */
 #define DCIH_NOALLOC_SCRATCH_BYTES (32u << 20)
 int dcih_query_noalloc(dcih_index* h, int dim, int num_queries, const float* d_query,

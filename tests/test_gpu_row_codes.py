@@ -73,3 +73,77 @@ def test_rows_too_close_for_their_codes(gpu):
     for _ in range(4):
         assert p.ask(Q) == 0
     p.free()
+
+
+def _device_bytes():
+    torch.cuda.synchronize()
+    free, total = torch.cuda.mem_get_info()
+    return total - free
+
+
+def test_room_for_the_codes_is_taken_when_they_are_formed(gpu):
+    n = 400_000                               # codes: 109 MB; index arrays: 5 MB per simple index
+    X, Q = torch.randn(n, DIM, device="cuda"), torch.randn(400, DIM, device="cuda")
+    codes = n * (16 + DIM)
+    dci = gpu.DCI(DIM, 1, 2, 64, T, seed=3, traversal="dense")
+    before = _device_bytes()
+    dci.add(X)
+    assert _device_bytes() - before < codes // 2
+    for _ in range(3):
+        first = dci.query(Q, K, OUTER, return_int=True)
+    held = _device_bytes()
+    assert held - before > codes
+    dci.clear()                               # the same size again: the same room
+    dci.add(X)
+    for _ in range(3):
+        again = dci.query(Q, K, OUTER, return_int=True)
+    assert torch.equal(first[0], again[0]) and torch.equal(first[1], again[1])
+    assert abs(_device_bytes() - held) < codes // 4
+    dci.free()
+    assert _device_bytes() - before < codes // 2
+
+
+def test_codes_on_two_streams_and_in_a_graph(gpu):
+    from dciknn_cuda_amd import _capi
+    rng = np.random.default_rng(4)
+    Q = torch.from_numpy(_rows(rng, 300)).cuda()
+    X = torch.from_numpy(_rows(rng, N)).cuda()
+    step = gpu.DCI(DIM, M, L, B, T, seed=3, traversal="step")
+    step.add(X)
+    want = step.query(Q, K, OUTER, return_int=True)
+    dci = gpu.DCI(DIM, M, L, B, T, seed=3, traversal="dense")
+    dci.add(X)
+    ticks = torch.zeros(16, dtype=torch.int64, device="cuda")
+    _capi.check(dci._lib.dcih_phase_profile(dci._dci_inst, ticks.data_ptr()))
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    outs = [(torch.full((300, K), -7, dtype=torch.int32, device="cuda"), torch.full((300, K), -7.0, device="cuda"))
+            for _ in range(3)]
+
+    def call(stream, out):
+        _capi.check(dci._lib.dcih_query(dci._dci_inst, DIM, 300, Q.data_ptr(), K, 0, OUTER, 10 * K, B, T,
+                                        out[0].data_ptr(), out[1].data_ptr(), None, stream))
+
+    torch.cuda.synchronize()
+    call(a.cuda_stream, outs[0])              # forms the codes
+    b.wait_stream(a)                          # (the workspace is the handle's: its calls are kept in order)
+    call(b.cuda_stream, outs[1])
+    torch.cuda.synchronize()
+    assert int(ticks[15]) == int(ticks[9]) == 2 * 300 * B
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=a):
+        call(torch.cuda.current_stream().cuda_stream, outs[2])
+    for _ in range(3):
+        for out in outs[2]:
+            out.fill_(-5)
+        ticks.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert int(ticks[15]) == 300 * B
+        call(b.cuda_stream, outs[1])          # eager work between the replays
+        torch.cuda.synchronize()
+        for ids, dists in outs:
+            assert torch.equal(ids, want[0]) and torch.equal(dists, want[1])
+    _capi.check(dci._lib.dcih_phase_profile(dci._dci_inst, None))
+    del g
+    dci.free()
+    step.free()
