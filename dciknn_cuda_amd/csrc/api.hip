@@ -486,9 +486,6 @@ int dcih_append(dcih_index* h, int dim, int64_t num_points, const float* d_data,
     // Everything that can fail for lack of memory happens before the index is touched:
     // room for the rows and their projections (both owned by the index, capacity doubles
     // so that copies amortise), for the next index in the spare arena, and for the sort.
-    float* rows = h->d_own;
-    float* ukeys = h->d_ukeys;
-    int64_t cap = h->own_rows;
     int64_t have_keys = (h->n > 0 && h->d_data == h->d_own) ? std::min(h->ukeys_rows, h->n) : 0;
     const int spare = 1 - h->cur;
     // Merging the old slices with the sorted new points instead of sorting everything again.
@@ -499,6 +496,11 @@ int dcih_append(dcih_index* h, int dim, int64_t num_points, const float* d_data,
                        segsort_append_supported(h->n, total, block_size);
     if (h->append_mode == 2 && h->n > 0 && !merge)
         return fail(DCIH_EUNSUPPORTED, "dcih_append: this shape cannot be appended by merging (partitions too long)");
+    // An empty index has no rows to keep: room of earlier ones that does not hold the new ones goes first.
+    if (h->n == 0 && h->own_rows < total) release_rows(h);
+    float* rows = h->d_own;
+    float* ukeys = h->d_ukeys;
+    int64_t cap = h->own_rows;
     // (codes of the rows so far are not the next index's; their room goes where it will not hold its codes)
     if (h->rows8_bytes < rows8_room(h, total, block_size)) release_rows8(h);
     float* fresh_rows = nullptr;

@@ -90,3 +90,23 @@ def test_merge_refuses_long_partitions(gpu):
     d.append(x)                                        # left to choose, it sorts
     assert d.num_points == 40000
     d.free()
+
+
+def test_append_after_clear_takes_no_more_than_a_fresh_handle(gpu):
+    x = torch.randn(600_000, 64, device="cuda")
+
+    def used_by(first):
+        torch.cuda.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        d = gpu.DCI(64, 1, 2, 50, 4, seed=1)
+        if first:
+            d.append(x[:first])
+            d.clear()
+        d.append(x)                                    # 154 MB of rows, 5 of projections
+        torch.cuda.synchronize()
+        used = before - torch.cuda.mem_get_info()[0]
+        d.free()
+        return used
+
+    fresh = used_by(0)
+    assert used_by(500_000) < fresh + (40 << 20)       # room for twice the first rows would be 106 MB more
