@@ -588,6 +588,8 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     if (num_queries == 0) return DCIH_OK;
     DeviceGuard guard(h->device);
     hipStream_t s = (hipStream_t)stream;
+    // Under capture nothing runs: what this call's kernels fill or clear for later calls has not been when it returns.
+    const bool recorded = capturing(s);
     const int I = num_indices(h);
     // the scratch of this call: the handle's workspace, grown as needed, or the static array
     char* ws_base = nullptr;
@@ -609,7 +611,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     h->ev_valid[DCIH_T_BATCH] = h->ev_valid[DCIH_T_DENSE] = false;
     QueryArgs a;
     a.skeys = h->d_skeys; a.sids = h->d_sids; a.inv = h->d_inv; a.data = h->d_data; a.query = d_query;
-    a.rpos = h->d_rpos; a.rpos_ready = &h->rpos_ready;
+    a.rpos = h->d_rpos; a.rpos_ready = &h->rpos_ready; a.recorded = recorded ? 1 : 0;
     a.hints_cold = 0;
     a.mode = h->traversal; a.item_list = nullptr; a.item_count = nullptr; a.dense = nullptr;
     a.xcds = h->xcds; a.q_first = 0; a.q_count = num_queries;
@@ -707,8 +709,10 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
             h->hint_T != thread_size || h->hint_maxc != max_num_candidates) {
             const int rc = zero_words64(h->d_stop_hint, (int64_t)(((size_t)3 * block_size * sizeof(float) + 7) / 8), s);
             if (rc) return rc;
-            h->hint_k = num_neighbours; h->hint_outer = num_outer_iterations;
-            h->hint_T = thread_size; h->hint_maxc = max_num_candidates;
+            if (!recorded) {
+                h->hint_k = num_neighbours; h->hint_outer = num_outer_iterations;
+                h->hint_T = thread_size; h->hint_maxc = max_num_candidates;
+            }
             a.hints_cold = 1;
         }
         a.stop_hint = h->d_stop_hint;

@@ -51,6 +51,7 @@ struct QueryArgs {
                              // slice is the position, in this simple index, of the point that stands at place s of the
                              // first one's slice (null if ppb > 65536; filled on the first use, see fill_positions_by_first)
     int* rpos_ready;         // host flag of the index: rpos has been filled
+    int recorded;            // 1: the call is recorded into a graph, its kernels do not run now
     const float* data;       // [N][dim]
     const float* query;      // [nq][dim]
     const float* qproj;      // [I][nq]

@@ -1,5 +1,6 @@
-"""What a handle keeps from one call to the next, over streams: clear while queries are under way and
-what comes after it on the same stream, another one, with new directions or by `add`."""
+"""What a handle keeps from one call to the next, over streams and graphs: clear while queries are
+under way and what comes after it on the same stream, another one, with new directions or by `add`;
+a first query that is recorded and not run."""
 import threading
 
 import numpy as np
@@ -95,3 +96,38 @@ def test_clear_while_a_query_is_under_way(gpu, then):
     np.testing.assert_array_equal(ids, ids2)
     for d in (one, two, dci):
         d.free()
+
+
+def test_first_batch_traversal_recorded(gpu):
+    """The table of positions that the batch kernel reads is filled by the first call that uses it: a call
+    that is only recorded fills it when its graph runs, so an eager call before that fills it as well."""
+    X, Q = _rows(5, 100_000), _rows(6, 64)
+    step = gpu.DCI(DIM, M, L, B, T, seed=7, traversal="step")
+    step.add(X)
+    dci = gpu.DCI(DIM, M, L, B, T, seed=7, traversal="step")
+    dci.add(X)
+    want = _out(Q)
+    _query(step, Q, 0, *want)
+    _query(dci, Q, 0, *_out(Q))               # (the workspace has its size now)
+    torch.cuda.synchronize()
+    dci.set_traversal("batch")
+    s, recorded, eager = torch.cuda.Stream(), _out(Q), _out(Q)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        _query(dci, Q, torch.cuda.current_stream().cuda_stream, *recorded)
+    _query(dci, Q, 0, *eager)
+    torch.cuda.synchronize()
+    assert _same(eager, want)
+    for _ in range(3):
+        for out in recorded:
+            out.fill_(-5)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert _same(recorded, want)
+        _query(dci, Q, 0, *eager)
+        torch.cuda.synchronize()
+        assert _same(eager, want)
+    del g
+    dci.free()
+    step.free()
