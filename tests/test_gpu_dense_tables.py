@@ -13,15 +13,13 @@ pytestmark = pytest.mark.gpu
 # workgroup of 64, 256 or 512 threads holds at 5, 9, 13, 15, 33 and 21 windows per thread
 TABLES = [(1, 3, 2, 1), (7, 2, 2, 3), (314, 2, 2, 2), (316, 2, 2, 2), (378, 1, 3, 2), (512, 1, 3, 1), (513, 1, 3, 1),
           (1225, 2, 10, 10), (2031, 2, 9, 8), (2045, 1, 5, 4), (4072, 1, 9, 8), (4080, 1, 9, 8), (5103, 1, 10, 8), (5300, 1, 10, 8), (5565, 2, 11, 8),
-          (6127, 1, 11, 8), (6140, 2, 11, 8), (9000, 1, 3, 300), (22223, 1, 15, 128)]
+          (6127, 1, 11, 8), (6140, 2, 11, 8), (6127, 1, 14, 8), (9000, 1, 3, 300), (22223, 1, 15, 128)]
 
 
 @pytest.mark.parametrize("ppb,B,L,T", TABLES)
 @pytest.mark.parametrize("kind,dim", [("normal", 12), ("ties", 12), ("outlier", 12), ("normal", 100), ("close", 100),
                                       ("normal", 201), ("normal", 300), ("outlier", 520)])
 def test_dense_tables(gpu, oracle, ppb, B, L, T, kind, dim):
-    if dim > 200 and ppb > 3000:
-        pytest.skip("the row's length changes nothing of the tables")
     rng = np.random.default_rng(ppb + 7 * L + dim)
     n, M, nq, outer = ppb * B, 2, 24, 10_000
     X = rng.standard_normal((n, dim)).astype(np.float32)
@@ -72,3 +70,13 @@ def test_many_items(gpu, ppb, B, nq):
     for j in (0, 1):
         assert torch.equal(got["step"][j], got["dense"][j])
     assert torch.equal(got["step"][2][:, [1, 3]], got["dense"][2][:, [1, 3]])
+
+
+def test_one_window_too_many_is_refused(gpu):
+    from dciknn_cuda_amd import _capi
+    dci = gpu.DCI(8, 1, 14, 1, 8, seed=3, traversal="dense")
+    X = torch.randn(6128, 8, device="cuda")            # 14 * (6128 / 8 + 3) = 10766 windows, 10752 fit
+    dci.add(X)
+    with pytest.raises(_capi.DCIError, match="dense"):
+        dci.query(X[:4].contiguous(), 5, 50, return_int=True)
+    dci.free()

@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 import torch
 
-from util import engine_index, engine_project, engine_segsort, set_agreement
+from util import dense_fits, engine_index, engine_project, engine_segsort, set_agreement
 
 pytestmark = pytest.mark.gpu
 
@@ -229,19 +229,13 @@ CASES = [
 ]
 
 
-def _dense_fits(n, M, L, B, T, k):
-    ppb = -(-n // B)
-    return (M <= 64 and L <= 64 and ppb <= 32766 and min(k, ppb) <= 512 and
-            L * (ppb // T + 3) <= 41 * 256)
-
-
 @pytest.mark.parametrize("traversal", ["step", "batch", "dense", "auto"])
 @pytest.mark.parametrize("case", CASES, ids=[str(c[:9]) for c in CASES])
 def test_traversal_parity(gpu, oracle, case, traversal):
     n, nq, dim, M, L, B, T, k, outer, kind = case
     if traversal == "batch" and (2 * M * L > 256 or M > 64 or min(k, -(-n // B)) > 512):
         pytest.skip("shape outside the batch kernel's tables (it refuses; auto mode falls back)")
-    if traversal == "dense" and not _dense_fits(n, M, L, B, T, k):
+    if traversal == "dense" and not dense_fits(n, M, L, B, T, k):
         pytest.skip("shape outside the dense kernel's tables (it refuses; auto mode does not route there)")
     X, Q = _data(n * 7 + T, n, nq, dim, kind)
     ids, dists, ctr, ref = _run_l1(gpu, oracle, X, Q, M, L, B, T, k, outer, traversal=traversal)
