@@ -116,8 +116,9 @@ def parse():
     return p.parse_args()
 
 
-def load_traffic(config, cfg, traversal, n, nq):
-    """HBM bytes per launch of the dominant kernel from the committed counter summary."""
+def load_traffic(config, cfg, traversal, n, nq, kernel, launch_ms):
+    """HBM bytes per launch of the dominant kernel from the committed counter summary; None where
+    that describes another kernel, or one whose launches took another time (more than a tenth off)."""
     path = os.path.join(ROOT, "profiles", "hbm_traffic.json")
     try:
         with open(path) as f:
@@ -127,7 +128,9 @@ def load_traffic(config, cfg, traversal, n, nq):
     for row in table.get("runs", []):
         if (row.get("config") == config and row.get("bs") == cfg["bs"] and row.get("ts") == cfg["ts"]
                 and row.get("outer") == cfg["outer"] and row.get("traversal", "auto") == traversal
-                and row.get("points") == n and row.get("queries") == nq):
+                and row.get("points") == n and row.get("queries") == nq
+                and row.get("kernel", "").split("<")[0] == kernel
+                and abs(row.get("kernel_ms_in_counter_run", 0.0) - launch_ms) <= 0.1 * launch_ms):
             return row
     return None
 
@@ -135,8 +138,7 @@ def load_traffic(config, cfg, traversal, n, nq):
 def main():
     a = parse()
     if a.gpus != 1:
-        print("bench.py: this build runs on ONE GPU; --gpus %d is not supported "
-              "(every box in this pipeline has one GPU)" % a.gpus, file=sys.stderr)
+        print("bench.py: this engine runs on ONE GPU; --gpus %d is not supported" % a.gpus, file=sys.stderr)
         sys.exit(2)
     import numpy as np
     import torch
@@ -333,7 +335,7 @@ def main():
     elif batch_ms > 0:
         kernel, launch_ms = "traverse_block_kernel", batch_ms
     else:   # neither traversal kernel ran: the traversal provably runs dry and the ranking is computed directly
-        kernel, launch_ms = "exact_dists_kernel + segmented sort", trav_ms
+        kernel, launch_ms = "exact_dists_kernel + " + ("select_rows_kernel" if k <= 256 else "full sort"), trav_ms
     # bytes the launch has to bring from HBM in this layout: the index slices once (keys,
     # 16-bit ids, 16-bit inverse positions), per query its row, the rows of its candidates and
     # its per-partition result lists
@@ -348,9 +350,12 @@ def main():
         hbm_model = ("index slices once (8 B per entry) + per query its row, %.0f candidates' codes of %d B, %d rows of "
                      "%d B per partition and its per-partition result lists" % (C, rec, min(k, ppb), 4 * dim))
     if kernel.startswith("exact_dists"):
-        # direct ranking: the rows once, per (query, point) a distance written, sorted and read back
-        hbm_bytes = 4.0 * N * dim + nq * (4.0 * dim + 12.0 * N + 8.0 * k)
-        hbm_model = "rows once + per (query, point) a 4-byte distance out and 8 bytes through the sort"
+        # direct ranking: the rows once, per (query, point) a distance written and read back, with a
+        # full ranking its number as well
+        per_pair = 8.0 if k <= 256 else 12.0
+        hbm_bytes = 4.0 * N * dim + nq * (4.0 * dim + per_pair * N + 8.0 * k)
+        hbm_model = "rows once + %d bytes per (query, point): a distance out and back%s" % (
+            per_pair, "" if k <= 256 else ", its number out")
     hbm_gbs = hbm_bytes / (launch_ms * 1e-3) / 1e9
     valu_ops = MIN_INSTR_PER_ENTRY * float(own[0]) * nq
     valu_gops = valu_ops / (launch_ms * 1e-3) / 1e9
@@ -378,7 +383,7 @@ def main():
                     contract_bytes_gbs=contract_bytes * nq / (launch_ms * 1e-3) / 1e9,
                     contract_note="contract_bytes_* prices every visit at the reference's 8 bytes per "
                                   "(key, id) entry; it is not a bound for this layout and may exceed the HBM peak")
-    prof = load_traffic(config, cfg, a.traversal, N, nq)
+    prof = load_traffic(config, cfg, a.traversal, N, nq, kernel, launch_ms)
     roofline["traffic"] = prof["fetch_bytes"] + prof["write_bytes"] if prof else None
     if prof:
         roofline["traffic_source"] = {key: prof[key] for key in prof if key not in ("fetch_bytes", "write_bytes")}
