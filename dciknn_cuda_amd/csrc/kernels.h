@@ -125,10 +125,14 @@ inline double expected_stop(const QueryArgs& a) {
     const double by_steps = fmin((double)a.stop_at / fmax(1.0, windows), fraction((double)a.max_cand));
     return windows * fmin(1.0, fmax(fraction((double)a.k_stop), by_steps));
 }
-// What the two kernels take, in us on an MI355X, fitted to 450 shapes of 24 to 4000 points per partition
-// (T 2 to 64, L 7 and 15, 400 and 20000 items, Gaussian rows): a time one item takes from end to end, and
-// a time per item once they fill the device.  The dense kernel's grow with the windows it ranks and the
-// points it looks up, the batch kernel's with the promotions it replays.
+// What the two kernels take, in us on an MI355X: a time one item takes from end to end, and a time per item
+// once they fill the device.  The dense kernel's grow with the windows it ranks and the points it looks up,
+// the batch kernel's with the promotions it replays.  Fitted to Gaussian rows (24 to 4000 points per partition,
+// T 2 to 64, L 7 and 15); today's kernels are faster than this by about a tenth (dense) and a quarter (batch),
+// which leaves the choice where it was: over 692 shapes of 24 to 20000 points, T 1 to 64, L 3 to 15, M 1 to 3
+// (profiles/kernel_choice.txt) a call left to choose takes 1.3 % longer than the best of batch, dense and the
+// two together in the geometric mean, and more than a tenth longer in 27, mostly at M = 1; factors of their
+// own for each M would make that 0.9 % and 19.
 struct TraversalCosts { double dense_item, batch_item, batch_per_promotion, dense, batch; };
 inline TraversalCosts traversal_costs(const QueryArgs& a, double promotions) {
     TraversalCosts c;

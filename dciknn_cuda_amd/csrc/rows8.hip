@@ -180,8 +180,8 @@ __global__ __launch_bounds__(kThreads) void code_queries_kernel(const float* __r
 }  // namespace
 
 // Rows of fewer than 96 elements span at most three 128-byte lines: reading them whole costs less than
-// their record, a longer list and the rows of what is kept (64 elements, 1111 candidates each: 24 us of
-// distances per item against 48 by codes; 512 elements: 210 against 31).
+// their record, a longer list and the rows of what is kept (1111 candidates each, k = 50; 64 elements: 24 us of
+// distances per item by whole rows, 48 by codes; 512 elements: 102 and 70).
 bool rows8_supported(int dim) { return dim >= 96 && dim <= 1024; }
 // (a record that fits one 128-byte line gets one to itself)
 int rows8_record_bytes(int dim) { const int b = 16 + ((dim + 15) & ~15); return b <= 128 ? 128 : b; }

@@ -131,8 +131,8 @@ DenseLayout dense_layout_for(const QueryArgs& a, int nt, int ipt) {
 // Threads per workgroup and windows per thread; ipt = 0: too many windows.  With up to fifteen windows per
 // thread 128 registers do, which allow 16 wavefronts per CU, and the kernel needs them all to hide its chains
 // of LDS and memory reads: one per workgroup where partitions are small, four where four workgroups' tables
-// fit a CU's LDS, else eight (7021 windows per composite: 22.2 ms; four wavefronts per workgroup and eight per
-// CU 25.8).  With more, 128 registers spill in the ranking (17: 46 ms), so there eight wavefronts per CU, of
+// fit a CU's LDS, else eight (7021 windows per composite, items taken up by strides: 22.2 ms; four wavefronts per
+// workgroup and eight per CU 25.8).  With more, 128 registers spill in the ranking (17: 46 ms), so there eight wavefronts per CU, of
 // two workgroups as far as a thread can hold the windows.
 DenseLayout make_dense_layout(const QueryArgs& a) {
     const int64_t windows = dense_max_windows(a);
@@ -1040,9 +1040,9 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
         // is cleared of what has fallen behind the cut meanwhile; where that makes no room, the round
         // ends: the shares are sorted in with what is held.  Nearly always there is one such sort, at the end.
         // Compared by codes, the kept entries get their exact distances before that sort.
-        // Bound by the latency of the records' reads (eight 16-byte reads per lane under way).  12808 candidates
-        // of 128 elements, k = 100, two workgroups per CU: 98 us per item, 207 by whole rows and a sort per
-        // full buffer; 1325 of 512 elements: 69, and 426 by whole rows.
+        // Bound by the latency of the records' reads (eight 16-byte reads per lane under way).  12801 candidates
+        // of 96 elements, k = 100, two workgroups per CU: 75 us per item, 140 by whole rows; 1285 of 960
+        // elements, k = 10: 55, and 198 by whole rows.
         uint32_t* hist = tb.stage;
         unsigned long long cut = ~0ull;                         // entries above it are out
         unsigned long long pend = ~0ull;                        // lane's entry of a batch that did not fit the share
