@@ -15,8 +15,9 @@ def _rows(rng, n, spread=1.0):
 class _Pair:
     """The same rows behind the dense kernel and behind the step-by-step kernel."""
 
-    def __init__(self, gpu, X):
-        self.dense, self.step = (gpu.DCI(DIM, M, L, B, T, seed=3, traversal=t) for t in ("dense", "step"))
+    def __init__(self, gpu, X, parts=B):
+        self.parts = parts
+        self.dense, self.step = (gpu.DCI(DIM, M, L, parts, T, seed=3, traversal=t) for t in ("dense", "step"))
         xd = torch.from_numpy(X).cuda()
         self.dense.add(xd)
         self.step.add(xd)
@@ -33,7 +34,7 @@ class _Pair:
         _capi.check(lib.dcih_phase_profile(h, None))
         want = self.step.query(q, K, OUTER, return_int=True)
         assert torch.equal(ids, want[0]) and torch.equal(dists, want[1])
-        assert int(self.ticks[9]) == len(Q) * B
+        assert int(self.ticks[9]) == len(Q) * self.parts
         return int(self.ticks[15])
 
     def free(self):
@@ -54,15 +55,20 @@ def test_an_outlying_query_costs_only_itself(gpu):
     p.free()
 
 
-def test_many_outlying_queries_rest_the_codes_for_a_while(gpu):
+# (few long partitions, many short ones: different numbers of items are under way together)
+@pytest.mark.parametrize("parts,every", [(4, 1), (4, 2), (24, 1), (24, 2), (24, 3)])
+def test_many_outlying_queries_rest_the_codes_for_a_while(gpu, parts, every):
     rng = np.random.default_rng(2)
-    p = _Pair(gpu, _rows(rng, N))
-    Q = _rows(rng, 300)
+    p = _Pair(gpu, _rows(rng, N), parts)
+    Q = _rows(rng, 600)
     p.ask(Q)
-    assert p.ask(1e5 * Q) == 0
-    for _ in range(3):                        # rests are counted in items: an ordinary batch ends them
+    far = Q.copy()
+    far[::every] *= 1e5
+    for _ in range(3):
+        assert p.ask(far) <= (600 - len(far[::every])) * parts
+    for _ in range(3):                        # rests are counted in items: ordinary batches end them
         took = p.ask(Q)
-    assert took == 300 * B
+    assert took == 600 * parts
     p.free()
 
 
