@@ -1343,7 +1343,8 @@ int query_dense_items(const QueryArgs& a_in, hipStream_t s) {
     int64_t per_xcd = max((int64_t)1, min((int64_t)32 * per_cu * 2, most));
     int run = 0;
     if (!listed && y.ipt <= 15 && most >= (int64_t)32 * per_cu * 8) {
-        run = (int)((most * a.xcds * y.nt + 0xfffffffeLL) / 0xffffffffLL);
+        const int64_t fit = 0xffffffffLL / ((int64_t)a.xcds * y.nt);
+        run = (int)((most + fit - 1) / fit);
         per_xcd = (most + run - 1) / run;
     }
     const unsigned grid = (unsigned)(per_xcd * a.xcds);
