@@ -21,7 +21,9 @@ steps run on the final index.  Prints ONE JSON line:
                  it: `frac` is always achieved / peak of that limit (<= 1).  For the
                  batch traversal kernel the limit is vector-ALU issue (lane
                  instructions; its L2-side figure is given beside it), for the dense
-                 traversal kernel HBM bytes (candidate rows + index slices); the figure by the reference's 8-byte index
+                 traversal kernel the bytes each query reads for itself (candidate rows or codes + index
+                 slices) against HBM, of which the L2s answer what queries of one partition
+                 share (the counted traffic is beside it); the figure by the reference's 8-byte index
                  entries is kept as contract_bytes_* and is not a bound.  `traffic`
                  = HBM bytes per launch from profiles/hbm_traffic.json (rocprofv3
                  counter runs of this file), null when that file has no entry for
