@@ -140,6 +140,11 @@ struct dcih_index {
     float* d_ukeys = nullptr;           // [I][own_rows] unsorted projections of the rows in d_own
     int64_t own_rows = 0;               // capacity of d_own / d_ukeys in rows
     int64_t ukeys_rows = 0;             // leading rows of d_own whose projections d_ukeys holds
+    // the end of the last call that reads rows the index owns, on its stream, and through it of all before it:
+    // what comes after dcih_clear, on whatever stream, is put behind it
+    hipEvent_t busy = nullptr;
+    bool busy_set = false;
+    bool recorded = false;              // such a call was recorded into a graph: when it runs is not known
     float* d_stop_hint = nullptr;       // [3][block_size] epoch-size hints learnt from earlier queries
     int hint_k = 0, hint_outer = 0, hint_T = 0, hint_maxc = 0;   // query shape the hints belong to (zeros: none, as after a build)
     int traversal = 0;                  // DCIH_OPT_TRAVERSAL value
@@ -238,6 +243,24 @@ int release_index(dcih_index* h) {
 bool capturing(hipStream_t s) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
+
+// Puts what follows on stream `s` behind the calls so far that read owned rows.
+int after_readers(dcih_index* h, hipStream_t s) {
+    if (h->busy_set && !capturing(s)) DCIH_HIP(hipStreamWaitEvent(s, h->busy, 0));
+    return 0;
+}
+// Marks the end of such a call; where that cannot be done, waits for it.
+void mark_reader(dcih_index* h, hipStream_t s) {
+    if (capturing(s)) { h->recorded = true; return; }
+    h->busy_set = h->busy && hipEventRecord(h->busy, s) == hipSuccess;
+    if (!h->busy_set) { (void)hipGetLastError(); (void)hipDeviceSynchronize(); }
+}
+// The host waits for them.
+int wait_for_readers(dcih_index* h) {
+    if (h->busy_set) DCIH_HIP(hipEventSynchronize(h->busy));
+    h->busy_set = false;
+    return 0;
 }
 
 int ensure_ws(dcih_index* h, size_t bytes, hipStream_t s) {
@@ -386,6 +409,8 @@ int dcih_set_directions(dcih_index* h, const float* h_dirs) {
     if (!h || !h_dirs) return fail(DCIH_EINVAL, "dcih_set_directions: null argument");
     if (h->n > 0) return fail(DCIH_ESTATE, "dcih_set_directions: index is not empty");
     DeviceGuard guard(h->device);
+    const int rc = wait_for_readers(h);
+    if (rc) return rc;
     std::memcpy(h->h_dirs.data(), h_dirs, h->h_dirs.size() * sizeof(float));
     DCIH_HIP(hipMemcpy(h->d_dirs, h_dirs, h->h_dirs.size() * sizeof(float), hipMemcpyHostToDevice));
     return DCIH_OK;
@@ -448,9 +473,11 @@ int dcih_add(dcih_index* h, int dim, int64_t num_points, const float* d_data,
     // (the unsorted keys): a rebuild of the same size allocates and frees nothing
     const size_t b_keys = align_up((size_t)I * num_points * sizeof(float));
     const size_t tmp_bytes = segsort_tmp_bytes(I, num_points, block_size);
+    int rc = wait_for_readers(h);
+    if (rc) return rc;
     release_rows(h);                // (rows of appends before a clear: this index borrows its rows)
     if (h->rows8_bytes < rows8_room(h, num_points, block_size)) release_rows8(h);
-    int rc = ensure_arena(h, h->cur, arena_layout(I, num_points, block_size).total);
+    rc = ensure_arena(h, h->cur, arena_layout(I, num_points, block_size).total);
     if (rc == DCIH_OK) rc = ensure_ws(h, b_keys + align_up(tmp_bytes), s);
     if (rc == DCIH_OK) {
         float* d_keys = (float*)h->ws;
@@ -496,6 +523,11 @@ int dcih_append(dcih_index* h, int dim, int64_t num_points, const float* d_data,
                        segsort_append_supported(h->n, total, block_size);
     if (h->append_mode == 2 && h->n > 0 && !merge)
         return fail(DCIH_EUNSUPPORTED, "dcih_append: this shape cannot be appended by merging (partitions too long)");
+    if (!h->busy) DCIH_HIP(hipEventCreateWithFlags(&h->busy, hipEventDisableTiming));
+    // (calls that read borrowed rows are not marked)
+    if (h->n > 0 && h->d_data != h->d_own) DCIH_HIP(hipDeviceSynchronize());
+    int rc = after_readers(h, s);
+    if (rc) return rc;
     // An empty index has no rows to keep: room of earlier ones that does not hold the new ones goes first.
     if (h->n == 0 && h->own_rows < total) release_rows(h);
     float* rows = h->d_own;
@@ -517,7 +549,7 @@ int dcih_append(dcih_index* h, int dim, int64_t num_points, const float* d_data,
         ukeys = fresh_keys;
     }
     const size_t tmp_bytes = merge ? segsort_append_tmp_bytes(I, total) : segsort_tmp_bytes(I, total, block_size);
-    int rc = ensure_arena(h, h->n > 0 ? spare : h->cur,
+    rc = ensure_arena(h, h->n > 0 ? spare : h->cur,
                           std::max(arena_layout(I, total, block_size).total,
                                    arena_layout(I, cap, block_size).total));
     if (rc == DCIH_OK && tmp_bytes) rc = ensure_ws(h, align_up(tmp_bytes), s);
@@ -545,6 +577,7 @@ int dcih_append(dcih_index* h, int dim, int64_t num_points, const float* d_data,
                        tmp_bytes ? h->ws : nullptr, s, merge ? h->n : 0);
     else
         (void)hipStreamSynchronize(s);
+    h->busy_set = false;            // (the stream was waited for, and was behind them)
     if (rc) {       // the index stays as it was
         if (fresh_rows) (void)hipFree(fresh_rows);
         if (fresh_keys) (void)hipFree(fresh_keys);
@@ -590,6 +623,15 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     hipStream_t s = (hipStream_t)stream;
     // Under capture nothing runs: what this call's kernels fill or clear for later calls has not been when it returns.
     const bool recorded = capturing(s);
+    struct Reader {                 // (whatever way the call ends)
+        dcih_index* h;
+        hipStream_t s;
+        ~Reader() { if (h) mark_reader(h, s); }
+    } reader{h->d_data == h->d_own ? h : nullptr, s};
+    if (reader.h) {
+        const int rc = after_readers(h, s);
+        if (rc) return rc;
+    }
     const int I = num_indices(h);
     // the scratch of this call: the handle's workspace, grown as needed, or the static array
     char* ws_base = nullptr;
@@ -909,17 +951,21 @@ int64_t dcih_num_points(const dcih_index* h) { return h ? h->n : 0; }
 int dcih_clear(dcih_index* h) {
     if (!h) return fail(DCIH_EINVAL, "dcih_clear: null handle");
     DeviceGuard guard(h->device);
-    // Borrowed rows are the caller's again when this returns, and rows the index owns are what the next append
-    // writes, on whatever stream: nothing may be reading them.
-    DCIH_HIP(hipDeviceSynchronize());
+    // Borrowed rows are the caller's again when this returns, so nothing may be reading them.  Rows the index
+    // owns stay with it: what comes next is put behind the calls that read them, unless they are in a graph.
+    if (h->recorded || h->d_data != h->d_own) {
+        DCIH_HIP(hipDeviceSynchronize());
+        h->busy_set = h->recorded = false;
+    }
     return release_index(h);
 }
 
 int dcih_reset(dcih_index* h) {
-    const int rc = dcih_clear(h);
+    int rc = dcih_clear(h);
     if (rc) return rc;
     DeviceGuard guard(h->device);
-    return draw_directions(h);
+    rc = wait_for_readers(h);
+    return rc ? rc : draw_directions(h);
 }
 
 int dcih_free(dcih_index* h) {
@@ -933,6 +979,7 @@ int dcih_free(dcih_index* h) {
     if (h->ws) (void)hipFree(h->ws);
     if (h->d_dirs) (void)hipFree(h->d_dirs);
     for (auto& e : h->ev) if (e) (void)hipEventDestroy(e);
+    if (h->busy) (void)hipEventDestroy(h->busy);
     delete h;
     return DCIH_OK;
 }

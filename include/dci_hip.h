@@ -261,9 +261,11 @@ int dcih_last_timings(dcih_index* h, float* h_ms);
 int64_t dcih_num_points(const dcih_index* h);
 
 /*
- * Replaces dci_clear (include/dci.h:77, src/dci_cuda_kernel.cu:878-885).  Waits
- * for the device; the index is empty then, and borrowed rows are the caller's
- * again.  The device memory its arrays occupied stays with the handle, so that the
+ * Replaces dci_clear (include/dci.h:77, src/dci_cuda_kernel.cu:878-885).  The index
+ * is empty then, and borrowed rows are the caller's again: it waits for the device.
+ * Rows that dcih_append copied in are the index's own: there it does not wait (unless
+ * a query was recorded into a graph), and calls that follow, on whatever stream, are
+ * ordered behind the queries before it.  The device memory its arrays occupied stays with the handle, so that the
  * next dcih_add allocates nothing, and so does the room of rows and projections
  * that dcih_append copied in, for the next appends.  The next dcih_add gives that
  * room back, dcih_free all of it.

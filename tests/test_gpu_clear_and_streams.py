@@ -40,7 +40,7 @@ def _same(a, b):
     return all(torch.equal(x, y) for x, y in zip(a, b))
 
 
-@pytest.mark.parametrize("then", ["same stream", "other stream", "per-thread stream", "new directions", "add"])
+@pytest.mark.parametrize("then", ["same stream", "other stream", "per-thread stream", "new directions", "add", "reset", "after a graph"])
 def test_clear_while_a_query_is_under_way(gpu, then):
     X1, X2, Q = _rows(1, 200_000), _rows(2, 200_000), _rows(3, 2000)
     one, two = gpu.DCI(DIM, M, L, B, T, seed=7), gpu.DCI(DIM, M, L, B, T, seed=7)
@@ -48,10 +48,8 @@ def test_clear_while_a_query_is_under_way(gpu, then):
     one.add(X1)
     if then == "new directions":
         two.directions = other_dirs
-    two.add(X2)
     want1, want2 = _out(Q), _out(Q)
     _query(one, Q, 0, *want1)
-    _query(two, Q, 0, *want2)
     torch.cuda.synchronize()
     a, b = torch.cuda.Stream(), torch.cuda.Stream()
     first = PER_THREAD if then == "per-thread stream" else a.cuda_stream
@@ -63,15 +61,27 @@ def test_clear_while_a_query_is_under_way(gpu, then):
     torch.cuda.synchronize()
 
     begun, over = threading.Event(), threading.Event()
+    graph = torch.cuda.CUDAGraph() if then == "after a graph" else None
+    if graph is not None:
+        with torch.cuda.graph(graph, stream=a):
+            _query(dci, Q, torch.cuda.current_stream().cuda_stream, *got1)
 
     def begin():
         for _ in range(8):                    # (milliseconds of work)
-            _query(dci, Q, first, *got1)
+            if graph is not None:
+                with torch.cuda.stream(a):
+                    graph.replay()
+            else:
+                _query(dci, Q, first, *got1)
         begun.set()
         over.wait(60)                         # (a thread's own stream lives as long as the thread)
 
     def go_on():
-        dci.clear()
+        if then == "reset":
+            dci.reset()
+            two.directions = dci.directions
+        else:
+            dci.clear()
         if then == "new directions":
             dci.directions = other_dirs
         if then == "add":
@@ -88,6 +98,10 @@ def test_clear_while_a_query_is_under_way(gpu, then):
     torch.cuda.synchronize()
     over.set()
     t.join()
+    two.add(X2)
+    _query(two, Q, 0, *want2)
+    torch.cuda.synchronize()
+    del graph
     assert _same(got1, want1)
     assert _same(got2, want2)
     keys, ids = engine_index(dci)
