@@ -194,7 +194,8 @@ typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) uint16_t lds_u16;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-struct DenseArgs { QueryArgs a; DenseLayout y; int run; };      // run: neighbouring items a workgroup takes; 0: it strides over all
+// Workgroup g of its die takes the items from g * first on, every step-th one, below g * first + len.
+struct DenseArgs { QueryArgs a; DenseLayout y; int first, step; int64_t len; };
 
 // Where the workgroup's tables lie in LDS.
 struct DenseTables {
@@ -280,9 +281,7 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
     const bool listed = args->a.dense_items != nullptr && args->a.mode != 3;
     const int64_t my_count = listed ? (int64_t)args->a.dense_count[xcd]
                                     : block_items(X, args->a.B, args->a.q_count) / X;
-    const int items = args->run;
-    const int64_t slot_end = items > 0 ? min(my_count, (g0 + 1) * items) : my_count;
-    const int64_t slot_step = items > 0 ? 1 : (int64_t)(gridDim.x / X);
+    const int slot_first = (int)g0 * args->first, slot_end = (int)min(my_count, (int64_t)slot_first + args->len);
 
     // optional phase profile: thread 0 adds the 100 MHz ticks each phase took
     unsigned long long tick = 0ull;
@@ -294,7 +293,9 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
         }
     };
 
-    for (int64_t slot = items > 0 ? g0 * items : g0; slot < slot_end; slot += slot_step) {
+    // (a die's items number below 2^28; the step is read where it is used: one more scalar carried through the loop
+    //  costs 1 % where a call is a few rounds of items)
+    for (int slot = slot_first; slot < slot_end; slot += fresh_args()->step) {
         ArgsPtr args = fresh_args();
         DenseTables tb(smem, args->a, args->y);
         int b, qi;
@@ -303,7 +304,7 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
             b = (int)(item % args->a.B);
             qi = (int)(item / args->a.B);
         } else {
-            if (!block_item(slot * X + xcd, X, args->a.B, args->a.q_count, b, qi)) continue;
+            if (!block_item((int64_t)slot * X + xcd, X, args->a.B, args->a.q_count, b, qi)) continue;
             qi += args->a.q_first;
         }
         b = __builtin_amdgcn_readfirstlane(b);      // (what is the same for all threads stays in scalar registers)
@@ -1341,11 +1342,13 @@ int query_dense_items(const QueryArgs& a_in, hipStream_t s) {
     const bool listed = a.dense_items && a.mode != 3;
     const int64_t most = listed ? (int64_t)a.dense_cap : block_items(a.xcds, a.B, a.nq) / a.xcds;
     int64_t per_xcd = max((int64_t)1, min((int64_t)32 * per_cu * 2, most));
-    int run = 0;
+    DenseArgs args{a, y, 1, (int)per_xcd, most};
     if (!listed && y.ipt <= 15 && most >= (int64_t)32 * per_cu * 8) {
         const int64_t fit = 0xffffffffLL / ((int64_t)a.xcds * y.nt);
-        run = (int)((most + fit - 1) / fit);
-        per_xcd = (most + run - 1) / run;
+        args.first = (int)((most + fit - 1) / fit);
+        args.len = args.first;
+        args.step = 1;
+        per_xcd = (most + args.first - 1) / args.first;
     }
     const unsigned grid = (unsigned)(per_xcd * a.xcds);
 #define DCIH_DENSE(NT, IPT, WAVES)                                                                 \
@@ -1357,7 +1360,7 @@ int query_dense_items(const QueryArgs& a_in, hipStream_t s) {
             return 0;                                                                            \
         });                                                                                      \
         if (rc_attr) return rc_attr;                                                             \
-        hipLaunchKernelGGL((traverse_dense_kernel<NT, IPT, WAVES>), dim3(grid), dim3(NT), y.lds_bytes, s, DenseArgs{a, y, run}); \
+        hipLaunchKernelGGL((traverse_dense_kernel<NT, IPT, WAVES>), dim3(grid), dim3(NT), y.lds_bytes, s, args); \
     } while (0)
     if (y.nt == 64) {
         if (y.ipt == 5) DCIH_DENSE(64, 5, 4); else DCIH_DENSE(64, 9, 4);
