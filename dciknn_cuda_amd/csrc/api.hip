@@ -134,7 +134,9 @@ struct dcih_index {
     unsigned char* d_rows8 = nullptr;
     size_t rows8_bytes = 0;
     double rows8_demand = 0.0;          // candidate rows asked for so far
-    bool rows8_ready = false;
+    bool rows8_ready = false;           // formed, or under way on some stream:
+    hipEvent_t rows8_event = nullptr;   // ... until this is over,
+    bool rows8_settled = false;         // ... as has been seen
     bool rows8_no_room = false;         // there was no memory for them: not asked for again until the next build
     float* d_own = nullptr;             // rows copied in by dcih_append (the index owns these)
     float* d_ukeys = nullptr;           // [I][own_rows] unsorted projections of the rows in d_own
@@ -247,12 +249,12 @@ bool capturing(hipStream_t s) {
 
 // Puts what follows on stream `s` behind the calls so far that read owned rows.
 int after_readers(dcih_index* h, hipStream_t s) {
-    if (h->busy_set && !capturing(s)) DCIH_HIP(hipStreamWaitEvent(s, h->busy, 0));
+    if (h->busy_set) DCIH_HIP(hipStreamWaitEvent(s, h->busy, 0));
     return 0;
 }
 // Marks the end of such a call; where that cannot be done, waits for it.
-void mark_reader(dcih_index* h, hipStream_t s) {
-    if (capturing(s)) { h->recorded = true; return; }
+void mark_reader(dcih_index* h, hipStream_t s, bool recording) {
+    if (recording) { h->recorded = true; return; }
     h->busy_set = h->busy && hipEventRecord(h->busy, s) == hipSuccess;
     if (!h->busy_set) { (void)hipGetLastError(); (void)hipDeviceSynchronize(); }
 }
@@ -317,13 +319,24 @@ size_t rows8_room(const dcih_index* h, int64_t n, int block_size) {
 // Whether a call on stream `s` that goes to the dense kernel may compare rows by their codes; forms
 // the codes when they have become worth it: a candidate read by its code saves three quarters of its row,
 // forming the codes reads every row and writes a quarter of it, so from twice as many candidates as rows on.
-// The call that forms them waits for them, so that later ones may come on any stream.
+// Until they have been seen to be there, calls are put behind their event, whatever the stream.
+bool rows8_there(dcih_index* h, hipStream_t s) {
+    if (h->rows8_settled) return true;
+    // (the event is no part of a capture under way: asking after it is all right there)
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool recording = capturing(s) && hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    h->rows8_settled = hipEventQuery(h->rows8_event) == hipSuccess;
+    if (!h->rows8_settled) (void)hipGetLastError();
+    if (recording) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return h->rows8_settled;
+}
 int use_rows8(dcih_index* h, double candidates, bool may_form, hipStream_t s, bool& use) {
     use = false;
     if (!rows8_supported(h->dim) || h->rows8_no_room) return 0;
     h->rows8_demand += candidates;
     if (!h->rows8_ready) {
         if (!may_form || h->rows8_demand < 2.0 * (double)h->n || capturing(s)) return 0;
+        if (!h->rows8_event) DCIH_HIP(hipEventCreateWithFlags(&h->rows8_event, hipEventDisableTiming));
         const size_t need = rows8_room(h, h->n, h->block_size);
         if (need > h->rows8_bytes) {
             if (h->d_rows8) { DCIH_HIP(hipFree(h->d_rows8)); h->d_rows8 = nullptr; h->rows8_bytes = 0; }
@@ -339,8 +352,12 @@ int use_rows8(dcih_index* h, double candidates, bool may_form, hipStream_t s, bo
         const int rc = code_rows(h->d_data, h->n, h->dim, ppb, h->block_size, h->d_rows8,
                                  (uint32_t*)(h->d_rows8 + rows8_records(h, h->n)), s);
         if (rc) return rc;
-        DCIH_HIP(hipStreamSynchronize(s));
+        DCIH_HIP(hipEventRecord(h->rows8_event, s));
         h->rows8_ready = true;
+        h->rows8_settled = false;
+    } else if (!rows8_there(h, s)) {
+        if (capturing(s)) return 0;
+        DCIH_HIP(hipStreamWaitEvent(s, h->rows8_event, 0));
     }
     use = true;
     return 0;
@@ -523,7 +540,8 @@ int dcih_append(dcih_index* h, int dim, int64_t num_points, const float* d_data,
                        segsort_append_supported(h->n, total, block_size);
     if (h->append_mode == 2 && h->n > 0 && !merge)
         return fail(DCIH_EUNSUPPORTED, "dcih_append: this shape cannot be appended by merging (partitions too long)");
-    if (!h->busy) DCIH_HIP(hipEventCreateWithFlags(&h->busy, hipEventDisableTiming));
+    // (a release to the device is all its waiters need: they overwrite what was read)
+    if (!h->busy) DCIH_HIP(hipEventCreateWithFlags(&h->busy, hipEventDisableTiming | hipEventReleaseToDevice));
     // (calls that read borrowed rows are not marked)
     if (h->n > 0 && h->d_data != h->d_own) DCIH_HIP(hipDeviceSynchronize());
     int rc = after_readers(h, s);
@@ -626,9 +644,10 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     struct Reader {                 // (whatever way the call ends)
         dcih_index* h;
         hipStream_t s;
-        ~Reader() { if (h) mark_reader(h, s); }
-    } reader{h->d_data == h->d_own ? h : nullptr, s};
-    if (reader.h) {
+        bool recording;
+        ~Reader() { if (h) mark_reader(h, s, recording); }
+    } reader{h->d_data == h->d_own ? h : nullptr, s, recorded};
+    if (reader.h && !recorded) {
         const int rc = after_readers(h, s);
         if (rc) return rc;
     }
@@ -980,6 +999,7 @@ int dcih_free(dcih_index* h) {
     if (h->d_dirs) (void)hipFree(h->d_dirs);
     for (auto& e : h->ev) if (e) (void)hipEventDestroy(e);
     if (h->busy) (void)hipEventDestroy(h->busy);
+    if (h->rows8_event) (void)hipEventDestroy(h->rows8_event);
     delete h;
     return DCIH_OK;
 }

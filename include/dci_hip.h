@@ -171,7 +171,7 @@ int dcih_append(dcih_index* h, int dim, int64_t num_points, const float* d_data,
  * The call may allocate: its workspace grows to the largest call's, and where the dense
  * kernel's calls have asked for twice as many candidates as there are rows of 96 to 1024
  * elements, the call that gets there forms 8-bit codes of the rows, about a quarter of
- * their size, and waits for them (without memory for them whole rows are compared).
+ * their size (without memory for them whole rows are compared).
  * Later calls compare rows by their codes first; results do not depend on it.  Under
  * stream capture nothing is allocated and no codes are formed; what calls before the
  * capture have allocated and formed is used.

@@ -109,7 +109,8 @@ def test_room_for_the_codes_is_taken_when_they_are_formed(gpu):
     assert _device_bytes() - before < codes // 2
 
 
-def test_codes_on_two_streams_and_in_a_graph(gpu):
+@pytest.mark.parametrize("then", ["on another stream", "in a graph"])
+def test_codes_just_formed(gpu, then):
     from dciknn_cuda_amd import _capi
     rng = np.random.default_rng(4)
     Q = torch.from_numpy(_rows(rng, 300)).cuda()
@@ -131,23 +132,27 @@ def test_codes_on_two_streams_and_in_a_graph(gpu):
 
     torch.cuda.synchronize()
     call(a.cuda_stream, outs[0])              # forms the codes
+    g = None
+    if then == "in a graph":                  # (the very next call is recorded, on another stream)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=b):
+            call(torch.cuda.current_stream().cuda_stream, outs[2])
     b.wait_stream(a)                          # (the workspace is the handle's: its calls are kept in order)
     call(b.cuda_stream, outs[1])
     torch.cuda.synchronize()
     assert int(ticks[15]) == int(ticks[9]) == 2 * 300 * B
-    g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g, stream=a):
-        call(torch.cuda.current_stream().cuda_stream, outs[2])
     for _ in range(3):
-        for out in outs[2]:
-            out.fill_(-5)
-        ticks.zero_()
-        g.replay()
-        torch.cuda.synchronize()
-        assert int(ticks[15]) == 300 * B
+        if g is not None:
+            for out in outs[2]:
+                out.fill_(-5)
+            ticks.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert int(ticks[15]) == 300 * B
         call(b.cuda_stream, outs[1])          # eager work between the replays
         torch.cuda.synchronize()
-        for ids, dists in outs:
+        for ids, dists in outs if g is not None else outs[:2]:
             assert torch.equal(ids, want[0]) and torch.equal(dists, want[1])
     _capi.check(dci._lib.dcih_phase_profile(dci._dci_inst, None))
     del g
