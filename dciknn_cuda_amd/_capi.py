@@ -15,6 +15,7 @@ OPT_TRAVERSAL = 0
 OPT_DENSE_MIN_PROMOTIONS = 1
 OPT_FORGET_HINTS = 2
 OPT_APPEND = 3
+OPT_ROUNDS = 4
 APPEND_AUTO, APPEND_SORT, APPEND_MERGE = 0, 1, 2
 TRAVERSAL_AUTO, TRAVERSAL_STEP, TRAVERSAL_BATCH, TRAVERSAL_DENSE = 0, 1, 2, 3
 NOALLOC_SCRATCH_BYTES = 32 << 20

@@ -153,6 +153,7 @@ struct dcih_index {
     int dense_min_promos = 160;         // DCIH_OPT_DENSE_MIN_PROMOTIONS value
     int dense_by_cost = 1;              // until that option is set
     int append_mode = 0;                // DCIH_OPT_APPEND value
+    int rounds = 0;                     // DCIH_OPT_ROUNDS value
     unsigned long long* d_phase_ticks = nullptr;   // optional profile of the batch kernel
     // grow-only workspace: query scratch, and the unsorted keys during a build
     void* ws = nullptr;
@@ -684,6 +685,8 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     a.hand_over_at = 0;
     a.expect_steps = a.expect_promotions = 0.0f;
     a.rows8 = nullptr; a.rows8_rec = 0; a.rows8_bounds = nullptr; a.query8 = nullptr;
+    a.picked = nullptr; a.picked_count = nullptr; a.picked_expect = a.picked_cover = 0; a.only = nullptr; a.only_round = 0;
+    a.share = 1.0; a.pick_first = 0.0; a.pick_rounds = a.pick_rank = 0; a.pick_rule = fixed ? 1 : h->rounds;
     a.phase_ticks = h->d_phase_ticks;
     a.stop_hint = nullptr;
     a.N = h->n;
@@ -749,12 +752,13 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
         return rc;
     }
 
+    (void)plan_rounds(a);
     size_t q8_bytes = 0;
     if (!blind && dense_traversal_supported(a, nullptr)) {
         const bool all_dense = takes_dense_kernel(a);
         bool use = false;
         const double per_item = std::min((double)a.ppb, expected_promotions(a));
-        const int rc8 = use_rows8(h, all_dense ? (double)num_queries * block_size * per_item : 0.0, all_dense && !fixed, s, use);
+        const int rc8 = use_rows8(h, all_dense ? (double)num_queries * block_size * per_item * a.share : 0.0, all_dense && !fixed, s, use);
         if (rc8) return rc8;
         if (use) {
             a.rows8 = h->d_rows8; a.rows8_rec = rows8_record_bytes(dim); a.rows8_bounds = (uint32_t*)(h->d_rows8 + rows8_records(h, h->n));
@@ -792,7 +796,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     const size_t wide_bytes = align_up((size_t)a.wide_cap * sizeof(int32_t));
     const size_t ws_bytes = qp_bytes + part_bytes + gs_bytes + redo_bytes + 256 + dense_bytes + wide_bytes;
     if (fixed && ws_bytes + q8_bytes > kScratchBytes) { a.rows8 = nullptr; q8_bytes = 0; }
-    int rc = get_ws(ws_bytes + q8_bytes);
+    int rc = get_ws(ws_bytes + q8_bytes + (a.pick_rounds ? bounds_bytes(a) : 0));
     if (rc) return rc;
     char* base = ws_base;
     float* d_qproj = (float*)base;
@@ -821,7 +825,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     hipEvent_t qev[5] = {h->ev[2 * DCIH_T_TRAVERSE], h->ev[2 * DCIH_T_BATCH + 1], h->ev[2 * DCIH_T_DENSE + 1],
                          h->ev[2 * DCIH_T_TRAVERSE + 1], h->ev[2 * DCIH_T_MERGE + 1]};
     bool ran[2] = {false, false};
-    rc = query(a, s, h->profiling ? qev : nullptr, ran);
+    rc = query(a, base + ws_bytes + q8_bytes, s, h->profiling ? qev : nullptr, ran);
     if (rc == DCIH_OK && h->profiling) {
         h->ev_valid[DCIH_T_TRAVERSE] = h->ev_valid[DCIH_T_MERGE] = true;
         h->ev_valid[DCIH_T_BATCH] = ran[0];
@@ -908,6 +912,10 @@ int dcih_set_option(dcih_index* h, int option, int value) {
     }
     if (option == DCIH_OPT_APPEND && value >= 0 && value <= 2) {
         h->append_mode = value;
+        return DCIH_OK;
+    }
+    if (option == DCIH_OPT_ROUNDS && value >= 0 && value <= 2) {
+        h->rounds = value;
         return DCIH_OK;
     }
     if (option == DCIH_OPT_FORGET_HINTS) {

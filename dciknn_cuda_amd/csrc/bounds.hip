@@ -1,0 +1,614 @@
+// Which partitions of a query have to be traversed at all.
+//
+// A query's answer is the k best of all partitions' candidates (get_top_candidates,
+// src/dci_cuda_kernel.cu:691-701), and a partition none of whose rows lies nearer than the k-th of
+// them adds nothing to it, whatever its traversal would promote.  So a call of many items first
+// bounds, for every (query, partition), the distance of the partition's nearest row from below --
+// a matrix product on the matrix cores whose epilogue keeps a minimum -- and then traverses
+//   round 1: the partitions whose bound is within what the query's k nearest rows are bounded by,
+//   round 2: of the others about as many again, as far as their bound does not exceed the k-th distance found,
+//   round 3: all others whose bound does not exceed the k-th distance found by then.
+// What is left out lies further than that, so the results are those of traversing everything; where
+// traversals miss near rows (low recall), or a bound is poor, the later rounds are larger, up to everything.
+// (Calls of about a millisecond go without round 2: its launches would cost more than the items it saves.)
+// The k nearest rows are told apart by bounds of parts of a partition: among S of them, k nearest rows that fall into
+// the same part are k^2 / 2 S, which is what round 1's limit is too large by.
+//
+// The bound.  Rows and queries are rounded to 16-bit floats x', q' (scaled by powers of two, so that nothing
+// overflows; what does, or is not finite, has an unbounded error).  |x - q| >= |x' - q'| - |x - x'| - |q - q'|,
+// the two errors being summed where the rounding is done, and |x' - q'|^2 = |x'|^2 + |q'|^2 - 2 x'.q' comes
+// from 16-bit products added up in float32, lowered by what those additions can be off.  The distance
+// the traversal kernels compute is a float32 sum itself; the bound is lowered by its relative error too.
+#include "common.h"
+#include "kernels.h"
+
+namespace dcih {
+
+namespace {
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef v4f v4f_any __attribute__((aligned(4)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+constexpr int kPackThreads = 256;
+constexpr int kTile = 32;                 // rows and queries of one matrix instruction
+constexpr int kStep = 16;                 // elements of one
+constexpr int kChunk = 256;               // columns staged at a time where a row tile does not fit LDS as a whole
+constexpr int kSample = 16;               // rows and queries the scales are taken from
+constexpr int kMostParts = 2048;           // bounds kept per query
+constexpr int kListQueries = 1024;        // queries of a partition listed by one workgroup
+constexpr float kHalfMax = 65504.0f, kHalfMin = 6.103515625e-05f;       // largest, and smallest normal, 16-bit float
+constexpr uint32_t kInf = 0x7f800000u;
+
+struct Header { float row_scale, query_scale; };
+
+// 2^e with the sample's largest value at 64 .. 128: outliers of five hundred times that still fit, and what is
+// flushed to zero is 2^-20 of it.  The exponent is limited so that no sum below can overflow.
+__device__ inline float scale_for(float most) {
+    if (!(most > 0.0f)) return 1.0f;
+    const int e = (int)(__builtin_bit_cast(uint32_t, most) >> 23) - 127;
+    const int up = min(40, max(-40, 6 - e));
+    return __builtin_bit_cast(float, (uint32_t)(up + 127) << 23);
+}
+
+__device__ inline float sample_most(const float* base, int64_t rows, int dim, float* tmp) {
+    const int take = (int)min((int64_t)kSample, rows);
+    float most = 0.0f;
+#pragma unroll 4
+    for (int e = threadIdx.x; e < take * dim; e += kPackThreads) {
+        const int r = e / dim;
+        const float v = fabsf(base[(rows * r / take) * dim + (e - r * dim)]);
+        most = v < 3e38f ? fmaxf(most, v) : most;
+    }
+    tmp[threadIdx.x] = most;
+    __syncthreads();
+    for (int o = kPackThreads / 2; o > 0; o >>= 1) {
+        if ((int)threadIdx.x < o) tmp[threadIdx.x] = fmaxf(tmp[threadIdx.x], tmp[threadIdx.x + o]);
+        __syncthreads();
+    }
+    most = tmp[0];
+    __syncthreads();
+    return most;
+}
+
+// Eight consecutive elements of a row, j a multiple of eight, zeros past its end; dim >= 8.  Rows of
+// whole octets are read as such; else the last octet is read from the row's end and moved down.
+template <bool OCTETS>
+__device__ inline void load_octet(const float* row, int dim, int j, float (&x)[8]) {
+    const int from = OCTETS ? min(j, dim - 8) : max(0, min(j, dim - 8));
+    const v4f lo = *reinterpret_cast<const v4f_any*>(row + from), hi = *reinterpret_cast<const v4f_any*>(row + from + 4);
+    x[0] = lo.x; x[1] = lo.y; x[2] = lo.z; x[3] = lo.w;
+    x[4] = hi.x; x[5] = hi.y; x[6] = hi.z; x[7] = hi.w;
+}
+template <bool OCTETS>
+__device__ inline void place_octet(int dim, int j, float (&x)[8]) {
+    const int shift = j - max(0, min(j, dim - 8));
+    if constexpr (!OCTETS) {
+        const bool s4 = (shift & 4) != 0, s2 = (shift & 2) != 0, s1 = (shift & 1) != 0;
+#pragma unroll
+        for (int i = 0; i < 8; i++) x[i] = s4 ? (i + 4 < 8 ? x[i + 4] : 0.0f) : x[i];
+#pragma unroll
+        for (int i = 0; i < 8; i++) x[i] = s2 ? (i + 2 < 8 ? x[i + 2] : 0.0f) : x[i];
+#pragma unroll
+        for (int i = 0; i < 8; i++) x[i] = s1 ? (i + 1 < 8 ? x[i + 1] : 0.0f) : x[i];
+    }
+    if (shift >= 8)
+#pragma unroll
+        for (int i = 0; i < 8; i++) x[i] = 0.0f;
+}
+// Rounds to 16 bits and sums the squares of the rounded values and of what was rounded off.
+// (Values too small for a normal 16-bit float become zero here: what the matrix cores make of them does not matter.)
+__device__ inline v8h round_octet(const float (&x)[8], float scale, float most, float& sq, float& err) {
+    v8h out;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        float v = x[i] * scale;
+        const bool finite = fabsf(v) < 3e38f;
+        if (!finite) { v = 0.0f; err = __builtin_inff(); }
+        float c = fminf(most, fmaxf(-most, v));
+        c = fabsf(c) < kHalfMin ? 0.0f : c;
+        out[i] = (_Float16)c;
+        const float back = (float)out[i], off = v - back;
+        sq = __builtin_fmaf(back, back, sq);
+        err = __builtin_fmaf(off, off, err);
+    }
+    return out;
+}
+
+// The first workgroups round 32 queries each, into the order the matrix instructions take them
+// ([32 queries][16 elements]: 64 lanes of 8), times -2; all of them clear what the later launches
+// take as cleared: the bounds (infinite), the partitions' lists (empty) and the lists' lengths.
+struct PackArgs {
+    const float* query; const float* data;
+    int64_t n;
+    int nq, dim, steps, tiles;            // steps: of 16 elements; tiles: of 32 queries
+    Header* header; uint32_t* counts;
+    float2* qinfo;                        // [tiles * 32]: |q'|^2 and an upper bound of |q - q'|
+    _Float16* frags;
+    uint32_t* bounds; int64_t num_bounds;
+    unsigned long long* part; int64_t num_part;
+};
+template <bool OCTETS>
+__global__ __launch_bounds__(kPackThreads) void pack_queries_kernel(PackArgs a) {
+    __shared__ float tmp[kPackThreads];
+    const int tid = threadIdx.x;
+    const int64_t at = (int64_t)blockIdx.x * kPackThreads + tid, all = (int64_t)gridDim.x * kPackThreads;
+    for (int64_t e = at; e < a.num_bounds; e += all) a.bounds[e] = kInf;
+    for (int64_t e = at; e < a.num_part; e += all) a.part[e] = ~0ull;
+    if ((int)blockIdx.x >= a.tiles) return;
+    const float scale = scale_for(sample_most(a.query, a.nq, a.dim, tmp));
+    if (blockIdx.x == 0) {
+        const float rows = scale_for(sample_most(a.data, a.n, a.dim, tmp));
+        if (tid == 0) { a.header->row_scale = rows; a.header->query_scale = scale; }
+    }
+    const int qt = tid >> 3, q = (int)blockIdx.x * kTile + qt;
+    const float* row = a.query + (int64_t)min(q, a.nq - 1) * a.dim;
+    float sq = 0.0f, err = 0.0f;
+    for (int o = tid & 7; o < 2 * a.steps; o += 8) {
+        float x[8];
+        load_octet<OCTETS>(row, a.dim, o * 8, x);
+        place_octet<OCTETS>(a.dim, o * 8, x);
+        v8h h = round_octet(x, scale, 0.5f * kHalfMax, sq, err);
+#pragma unroll
+        for (int i = 0; i < 8; i++) h[i] = (_Float16)((float)h[i] * -2.0f);      // (exact)
+        *reinterpret_cast<v8h*>(a.frags + (((int64_t)blockIdx.x * a.steps + (o >> 1)) * 64 + (o & 1) * 32 + qt) * 8) = h;
+    }
+    sq += lane_xor<4>(sq); sq += lane_xor<2>(sq); sq += lane_xor<1>(sq);
+    err += lane_xor<4>(err); err += lane_xor<2>(err); err += lane_xor<1>(err);
+    if ((tid & 7) == 0) {
+        const float inv = 1.0f / scale;
+        a.qinfo[q] = make_float2(sq * inv * inv, sqrtf(err) * 1.001f * inv);
+    }
+}
+
+struct BoundArgs {
+    const float* data;
+    int64_t n, ppb;
+    int dim, steps, nq, tiles, chunk_steps;
+    int row_tiles, parts;                 // row tiles (workgroups) per partition, and the parts bounds are kept for
+    const Header* header; const float2* qinfo; const _Float16* frags;
+    uint32_t* bounds;                     // [B * parts][nq] float bits
+};
+
+// A workgroup takes R = 32 RT WR rows of one partition, rounds them into LDS and multiplies them with all
+// queries: WR wavefronts along the rows, WC along the queries, each with RT x CT accumulators of 32 x 32.  A row's
+// squared length is where its accumulators start, so what is left to do with a sum is to keep the
+// smallest, in the lane that holds the query's column.  WHOLE: the rows fit LDS over their whole length and stay there;
+// else they are staged kChunk columns at a time, anew for every pass over 32 CT WC queries.
+// 10000 queries on 1M rows of 128 (58 partitions, 10 results): 2.9 ms, 0.88 PFLOP/s, where traversing all 580000 pairs took 24.0 ms
+// and traversing the 112400 that are left takes 6.4; 512 on 10M rows of 96 (100 results): 2.3 ms, bound by staging its rows,
+// 72.5 -> 21 ms; 1000 on 1M rows of 128 with the defaults: 0.43 ms, 19.0 -> 2.3 ms.
+template <int RT, int CT, int WR, int WC, int WAVES, bool WHOLE, bool OCTETS>
+__global__ __launch_bounds__(64 * WR * WC, WAVES) void partition_bounds_kernel(BoundArgs a) {
+    constexpr int kWaves = WR * WC, R = kTile * RT * WR, kGroups = R / 8 / kWaves;
+    static_assert(kGroups >= 1, "eight rows per wavefront at least");
+    extern __shared__ __align__(16) unsigned char smem[];
+    float* s_n = reinterpret_cast<float*>(smem);                    // [R] squared lengths, scaled
+    float* s_red = s_n + R;                                         // [2 * kWaves]
+    v8h* s_rows = reinterpret_cast<v8h*>(smem + R * 4 + 2 * kWaves * 4);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int b = blockIdx.x / a.row_tiles, rt = blockIdx.x % a.row_tiles;
+    const int64_t off = (int64_t)b * a.ppb;
+    const int in_part = (int)min(a.n - off, a.ppb);
+    const int first = rt * R, rows = min(R, in_part - first);
+    if (rows <= 0) return;
+    const float* base = a.data + (off + first) * a.dim;
+    const float row_scale = a.header->row_scale, query_scale = a.header->query_scale;
+    float sq[kGroups], err[kGroups];
+#pragma unroll
+    for (int g = 0; g < kGroups; g++) sq[g] = err[g] = 0.0f;
+
+    // Rounds columns [16 s0, 16 (s0 + ns)) of the tile into LDS, in the order the matrix instructions take them.
+    // A lane group of eight takes eight rows, so that its stores hit different banks; eight such groups read 256 bytes of a row.
+    auto stage = [&](int s0, int ns, bool sums) {
+        const int octets = 2 * ns;
+#pragma unroll
+        for (int g = 0; g < kGroups; g++) {
+            const int r = (g * kWaves + wave) * 8 + (lane & 7);
+            const float* row = base + (int64_t)min(r, rows - 1) * a.dim;
+            for (int o0 = 0; o0 < octets; o0 += 16) {
+                float x[2][8];
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    const int o = min(o0 + 8 * u + (lane >> 3), octets - 1);
+                    load_octet<OCTETS>(row, a.dim, s0 * kStep + o * 8, x[u]);
+                }
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    const int o = o0 + 8 * u + (lane >> 3);
+                    if (o < octets) {
+                        place_octet<OCTETS>(a.dim, s0 * kStep + o * 8, x[u]);
+                        float s2 = 0.0f, e2 = 0.0f;
+                        const v8h h = round_octet(x[u], row_scale, kHalfMax, s2, e2);
+                        if (sums) { sq[g] += s2; err[g] += e2; }
+                        s_rows[((r >> 5) * a.chunk_steps + (o >> 1)) * 64 + (o & 1) * 32 + (r & 31)] = h;
+                    }
+                }
+            }
+        }
+    };
+    float most_n = 0.0f, most_e = 0.0f;      // of the tile's rows, not scaled
+    auto finish_sums = [&]() {
+        const float to_sum = query_scale / row_scale, inv = 1.0f / row_scale;
+        float mn = 0.0f, me = 0.0f;
+#pragma unroll
+        for (int g = 0; g < kGroups; g++) {
+            const int r = (g * kWaves + wave) * 8 + (lane & 7);
+            float s2 = sq[g], e2 = err[g];
+            s2 += lane_xor<32>(s2); s2 += lane_xor<16>(s2); s2 += lane_xor<8>(s2);
+            e2 += lane_xor<32>(e2); e2 += lane_xor<16>(e2); e2 += lane_xor<8>(e2);
+            if (r < rows) { mn = fmaxf(mn, s2); me = fmaxf(me, e2); }
+            if (lane < 8) s_n[r] = r < rows ? s2 * to_sum : __builtin_inff();
+        }
+        mn = fmaxf(mn, lane_xor<4>(mn)); mn = fmaxf(mn, lane_xor<2>(mn)); mn = fmaxf(mn, lane_xor<1>(mn));
+        me = fmaxf(me, lane_xor<4>(me)); me = fmaxf(me, lane_xor<2>(me)); me = fmaxf(me, lane_xor<1>(me));
+        if (lane == 0) { s_red[wave] = mn; s_red[kWaves + wave] = me; }
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < kWaves; w++) { most_n = fmaxf(most_n, s_red[w]); most_e = fmaxf(most_e, s_red[kWaves + w]); }
+        most_n *= inv * inv;
+        most_e = sqrtf(most_e) * 1.001f * inv;
+    };
+    const int wr = wave / WC, wc = wave % WC;
+    auto lengths = [&](int r) -> v16f {      // the accumulators' start: squared lengths of row tile r of this wavefront
+        v16f v;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const v4f t = *reinterpret_cast<const v4f*>(s_n + (wr * RT + r) * kTile + 8 * i + 4 * (lane >> 5));
+            v[4 * i] = t.x; v[4 * i + 1] = t.y; v[4 * i + 2] = t.z; v[4 * i + 3] = t.w;
+        }
+        return v;
+    };
+    const float unscale = 1.0f / (row_scale * query_scale);
+    const float sum_error = (float)(a.steps * kStep + 64) * 0x1.8p-22f, dist_error = 1.0f - (float)(a.dim + 32) * 0x1p-23f;
+    uint32_t* out = a.bounds + ((int64_t)b * a.parts + rt * a.parts / a.row_tiles) * a.nq;
+    // The smallest sum of each of 32 CT queries over the wavefront's rows -> their partition's bounds.
+    auto finish = [&](const v16f (&acc)[RT][CT], int q, bool mine, float2 info, uint32_t have) {
+        float best[CT];
+#pragma unroll
+        for (int c = 0; c < CT; c++) {
+            best[c] = acc[0][c][0];
+#pragma unroll
+            for (int r = 0; r < RT; r++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) best[c] = fminf(best[c], acc[r][c][i]);
+            best[c] = fminf(best[c], lane_xor<32>(best[c]));
+        }
+        const float v = CT == 2 && lane >= 32 ? best[CT - 1] : best[0];
+        const float d2 = v * unscale + info.x - sum_error * (most_n + info.x);
+        float d = sqrtf(fmaxf(d2, 0.0f)) - most_e - info.y;
+        d = fmaxf(d, 0.0f) * dist_error;
+        if (!(d > 1e-14f)) d = 0.0f;                          // (squares below the smallest float count as nothing in the distances)
+        const uint32_t bits = __builtin_bit_cast(uint32_t, d);
+        if (mine && bits < have) atomicMin(&out[q], bits);
+    };
+    const v8h* frags = reinterpret_cast<const v8h*>(a.frags);
+    constexpr int kPass = CT * WC;                            // query tiles of one pass
+    if constexpr (WHOLE) {
+        stage(0, a.steps, true);
+        finish_sums();
+        __syncthreads();
+        v16f start[RT];
+#pragma unroll
+        for (int r = 0; r < RT; r++) start[r] = lengths(r);
+        const v8h* rows_at = s_rows + (wr * RT) * a.chunk_steps * 64 + lane;
+        for (int t = wc * CT; t < a.tiles; t += kPass) {
+            const v8h* at[CT];
+#pragma unroll
+            for (int c = 0; c < CT; c++) at[c] = frags + (int64_t)min(t + c, a.tiles - 1) * a.steps * 64 + lane;
+            const int q = (t + (lane >> 5)) * kTile + (lane & 31);
+            const bool mine = q < a.nq && (CT == 2 || lane < 32);
+            const float2 info = a.qinfo[min(q, a.nq - 1)];
+            const uint32_t have = out[min(q, a.nq - 1)];
+            v16f acc[RT][CT];
+            v8h next[CT];
+#pragma unroll
+            for (int c = 0; c < CT; c++) next[c] = at[c][0];
+#pragma unroll
+            for (int r = 0; r < RT; r++)
+#pragma unroll
+                for (int c = 0; c < CT; c++) acc[r][c] = start[r];
+            for (int s = 0; s < a.steps; s++) {
+                v8h q8[CT];
+#pragma unroll
+                for (int c = 0; c < CT; c++) { q8[c] = next[c]; next[c] = at[c][min(s + 1, a.steps - 1) * 64]; }
+#pragma unroll
+                for (int r = 0; r < RT; r++) {
+                    const v8h x8 = rows_at[(r * a.chunk_steps + s) * 64];
+#pragma unroll
+                    for (int c = 0; c < CT; c++) acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x8, q8[c], acc[r][c], 0, 0, 0);
+                }
+            }
+            finish(acc, q, mine, info, have);
+        }
+    } else {
+        for (int t0 = 0; t0 < a.tiles; t0 += kPass) {
+            const int t = t0 + wc * CT;
+            const bool busy = t < a.tiles;
+            const int q = (t + (lane >> 5)) * kTile + (lane & 31);
+            const bool mine = busy && q < a.nq && (CT == 2 || lane < 32);
+            const float2 info = a.qinfo[min(q, a.nq - 1)];
+            const uint32_t have = out[min(q, a.nq - 1)];
+            v16f acc[RT][CT];
+#pragma unroll
+            for (int r = 0; r < RT; r++)
+#pragma unroll
+                for (int c = 0; c < CT; c++)
+#pragma unroll
+                    for (int i = 0; i < 16; i++) acc[r][c][i] = 0.0f;
+            for (int s0 = 0; s0 < a.steps; s0 += a.chunk_steps) {
+                const int ns = min(a.chunk_steps, a.steps - s0);
+                __syncthreads();                              // the columns before are done with
+                stage(s0, ns, t0 == 0);
+                __syncthreads();
+                if (!busy) continue;
+                const v8h* at[CT];
+#pragma unroll
+                for (int c = 0; c < CT; c++) at[c] = frags + ((int64_t)min(t + c, a.tiles - 1) * a.steps + s0) * 64 + lane;
+                const v8h* rows_at = s_rows + (wr * RT) * a.chunk_steps * 64 + lane;
+                v8h next[CT];
+#pragma unroll
+                for (int c = 0; c < CT; c++) next[c] = at[c][0];
+                for (int s = 0; s < ns; s++) {
+                    v8h q8[CT];
+#pragma unroll
+                    for (int c = 0; c < CT; c++) { q8[c] = next[c]; next[c] = at[c][min(s + 1, ns - 1) * 64]; }
+#pragma unroll
+                    for (int r = 0; r < RT; r++) {
+                        const v8h x8 = rows_at[(r * a.chunk_steps + s) * 64];
+#pragma unroll
+                        for (int c = 0; c < CT; c++) acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x8, q8[c], acc[r][c], 0, 0, 0);
+                    }
+                }
+            }
+            if (t0 == 0) {
+                __syncthreads();
+                finish_sums();
+                __syncthreads();
+            }
+#pragma unroll
+            for (int r = 0; r < RT; r++) {
+                const v16f n2 = lengths(r);
+#pragma unroll
+                for (int c = 0; c < CT; c++)
+#pragma unroll
+                    for (int i = 0; i < 16; i++) acc[r][c][i] += n2[i];
+            }
+            if (busy) finish(acc, q, mine, info, have);
+        }
+    }
+}
+
+// Of each query's S bounds the j1-th and the j2-th smallest, rounded up to 16 bits of their mantissa: one wavefront per
+// query, bit by bit the largest prefix that fewer than j bounds lie below.  A workgroup reads the bounds of `per`
+// neighbouring queries into LDS first.
+template <int V>
+__global__ __launch_bounds__(256) void pick_limits_kernel(const uint32_t* __restrict__ bounds, int S, int nq, int per, int j1, int j2,
+                                                          uint32_t* __restrict__ limits, uint32_t* __restrict__ last_round) {
+    extern __shared__ uint32_t s_b[];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q0 = (int)blockIdx.x * per, pitch = per + 1;
+#pragma unroll 4
+    for (int e = threadIdx.x; e < S * per; e += 256) {
+        const int i = e / per, q = e - i * per;
+        s_b[i * pitch + q] = bounds[(int64_t)i * nq + min(q0 + q, nq - 1)];
+    }
+    __syncthreads();
+    for (int q = wave; q < per && q0 + q < nq; q += 4) {
+        uint32_t v[V];
+#pragma unroll
+        for (int i = 0; i < V; i++) v[i] = i * 64 + lane < S ? s_b[(i * 64 + lane) * pitch + q] >> 8 : 0xffffffu;
+        uint32_t at1 = 0, at2 = 0;
+#pragma unroll 1
+        for (int bit = 22; bit >= 0; bit--) {
+            const uint32_t t1 = at1 | (1u << bit), t2 = at2 | (1u << bit);
+            int below1 = 0, below2 = 0;
+#pragma unroll
+            for (int i = 0; i < V; i++) { below1 += __popcll(__ballot(v[i] < t1)); below2 += __popcll(__ballot(v[i] < t2)); }
+            if (below1 < j1) at1 = t1;
+            if (below2 < j2) at2 = t2;
+        }
+        // (all ones where there are fewer than j)
+        if (lane == 0) { limits[q0 + q] = (at1 << 8) | 0xffu; limits[nq + q0 + q] = (at2 << 8) | 0xffu; last_round[q0 + q] = 0; }
+    }
+}
+
+// Lists the (query, partition) pairs of a round by partition, then query: each die takes one run of the list, so that its
+// resident workgroups work on one partition and its slices stay in the die's L2, whatever partitions the pairs are of.  (In the order in
+// which workgroups came to reserve their places, a die's 832 items of 17242 points were of five partitions, and took twice as long.)
+// One workgroup per kListQueries queries of a partition; the first launch counts, the second adds up the counts before its own.
+struct ListArgs {
+    const uint32_t* bounds; const uint32_t* limits;
+    const float* worst; int64_t worst_stride;      // the k-th distance each query has so far
+    uint32_t* last_round;                          // the round that last took a partition of the query
+    int B, parts, nq, groups, round, rounds;
+    int32_t* items; uint32_t* count; uint32_t* part_counts;
+};
+__device__ inline bool takes_item(const ListArgs& a, int b, int q) {
+    uint32_t v = a.bounds[(int64_t)b * a.parts * a.nq + q];
+    for (int p = 1; p < a.parts; p++) v = min(v, a.bounds[((int64_t)b * a.parts + p) * a.nq + q]);
+    const uint32_t l1 = a.limits[q], l2 = a.rounds > 2 ? a.limits[a.nq + q] : l1;
+    if (a.round == 0) return v <= l1;
+    // (what is infinite or NaN so far is bounded by nothing)
+    return v > l1 && (a.round + 1 < a.rounds ? v <= l2 : (a.rounds == 2 || v > l2)) &&
+           !(__builtin_bit_cast(float, v) > a.worst[(int64_t)q * a.worst_stride]);
+}
+template <bool COUNT>
+__global__ __launch_bounds__(256) void list_items_kernel(ListArgs a) {
+    __shared__ uint32_t s_wave[4], s_before[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int b = blockIdx.x / a.groups, q0 = (int)(blockIdx.x % a.groups) * kListQueries, q1 = min(a.nq, q0 + kListQueries);
+    unsigned long long m[kListQueries / 256];
+    uint32_t mine = 0;
+#pragma unroll
+    for (int i = 0; i < kListQueries / 256; i++) {      // (a wavefront's queries are consecutive)
+        const int q = q0 + wave * (kListQueries / 4) + i * 64 + lane;
+        m[i] = __ballot(q < q1 && takes_item(a, b, min(q, a.nq - 1)));
+        mine += (uint32_t)__popcll(m[i]);
+    }
+    uint32_t before = 0;
+    if (!COUNT) {
+        for (int e = tid; e < (int)blockIdx.x; e += 256) before += a.part_counts[e];
+        before = wave_sum_u32(before);
+    }
+    if (lane == 0) { s_wave[wave] = mine; s_before[wave] = before; }
+    __syncthreads();
+    if (COUNT) {
+        if (tid == 0) a.part_counts[blockIdx.x] = s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
+        return;
+    }
+    uint32_t at = s_before[0] + s_before[1] + s_before[2] + s_before[3];
+    if (blockIdx.x + 1 == gridDim.x && tid == 0) *a.count = at + s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
+    for (int w = 0; w < wave; w++) at += s_wave[w];
+#pragma unroll
+    for (int i = 0; i < kListQueries / 256; i++) {
+        const int q = q0 + wave * (kListQueries / 4) + i * 64 + lane;
+        if ((m[i] >> lane) & 1ull) {
+            a.items[at + (uint32_t)__popcll(m[i] & ((1ull << lane) - 1ull))] = (int32_t)((int64_t)q * a.B + b);
+            if (a.round > 0) a.last_round[q] = (uint32_t)a.round;
+        }
+        at += (uint32_t)__popcll(m[i]);
+    }
+}
+
+size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
+
+struct Room { size_t header, counts, qinfo, frags, bounds, limits, last, items, part_counts, total; int steps, tiles, parts; };
+Room room_of(const QueryArgs& a) {
+    Room r;
+    r.steps = (a.dim + kStep - 1) / kStep;
+    r.tiles = (a.nq + kTile - 1) / kTile;
+    // parts of a partition: 24 k in all, as far as that leaves them a row tile each and a query 2048 of them
+    const int64_t row_tiles = max((int64_t)1, a.ppb / 128);
+    r.parts = 1;
+    while (2 * r.parts <= row_tiles && (int64_t)a.B * r.parts < 24 * (int64_t)a.k && (int64_t)a.B * r.parts * 2 <= kMostParts) r.parts *= 2;
+    size_t o = 0;
+    r.header = o; o += 256;
+    r.counts = o; o += align256(kPickCountWords * 4);
+    r.qinfo = o;  o += align256((size_t)r.tiles * kTile * sizeof(float2));
+    r.frags = o;  o += align256((size_t)r.tiles * r.steps * 64 * 16);
+    r.bounds = o; o += align256((size_t)a.B * r.parts * a.nq * 4);
+    r.limits = o; o += align256((size_t)2 * a.nq * 4);
+    r.last = o;   o += align256((size_t)a.nq * 4);
+    r.items = o;  o += align256((size_t)a.nq * a.B * 4);
+    r.part_counts = o; o += align256((size_t)a.B * ((a.nq + kListQueries - 1) / kListQueries) * 4);
+    r.total = o;
+    return r;
+}
+
+// How the product is cut: wavefronts along rows and queries, row tiles each, and whether rows stay in LDS whole.
+struct Shape { int rt, ct, wr, wc; bool whole; };
+Shape shape_of(const QueryArgs& a) {
+    const int dim = (a.dim + kStep - 1) / kStep * kStep;
+    if (a.nq <= 32) return {1, 1, 4, 1, dim <= kChunk};
+    if (a.nq <= 64) return {1, 2, 4, 1, dim <= kChunk};
+    if (a.nq <= 128) return {2, 2, 2, 2, dim <= kChunk};
+    if (dim <= kChunk) return {4, 2, 1, 4, true};
+    return {2, 2, 1, 8, false};
+}
+
+}  // namespace
+
+bool bounds_supported(const QueryArgs& a) {
+    return !a.blind && !a.counters && a.dim >= 8 && a.dim <= 4096 && a.nq >= 1 && a.B >= 2 && a.B <= kMostParts &&
+           (int64_t)a.nq * a.B < 0x7fffffffLL && (a.ppb + kTile - 1) / kTile * (int64_t)a.B < 0x7fffffffLL;
+}
+
+size_t bounds_bytes(const QueryArgs& a) { return room_of(a).total; }
+
+double bounds_cost(const QueryArgs& a) {
+    const Shape y = shape_of(a);
+    const int R = kTile * y.rt * y.wr;
+    const double dim = (double)((a.dim + kStep - 1) / kStep * kStep);
+    const double rows = (double)((a.ppb + R - 1) / R * R) * (double)a.B;
+    const double passes = y.whole ? 1.0 : ceil((double)a.nq / (double)(kTile * y.ct * y.wc));
+    const double queries = ceil((double)a.nq / (kTile * y.ct)) * (kTile * y.ct);
+    return 12.0 + fmax(2.0 * rows * queries * dim / 500e6, passes * rows * (double)a.dim * 4.0 / 3e6);
+}
+
+static int pack(const QueryArgs& a, const Room& r, char* ws, hipStream_t s) {
+    PackArgs p{a.query, a.data, a.N, a.nq, a.dim, r.steps, r.tiles, (Header*)(ws + r.header), (uint32_t*)(ws + r.counts),
+               (float2*)(ws + r.qinfo), (_Float16*)(ws + r.frags), (uint32_t*)(ws + r.bounds), (int64_t)a.B * r.parts * a.nq,
+               a.part, (int64_t)a.nq * a.B * a.kcap};
+    const int64_t clear = (p.num_part + p.num_bounds + kPackThreads * 16 - 1) / (kPackThreads * 16);
+    const unsigned blocks = (unsigned)max((int64_t)r.tiles, min((int64_t)2048, clear));
+    if (a.dim % 8 == 0) hipLaunchKernelGGL(pack_queries_kernel<true>, dim3(blocks), dim3(kPackThreads), 0, s, p);
+    else hipLaunchKernelGGL(pack_queries_kernel<false>, dim3(blocks), dim3(kPackThreads), 0, s, p);
+    DCIH_HIP(hipGetLastError());
+    return 0;
+}
+
+template <int RT, int CT, int WR, int WC, int WAVES, bool WHOLE>
+static int launch_bounds(const BoundArgs& p, int B, hipStream_t s) {
+    constexpr int R = kTile * RT * WR, NT = 64 * WR * WC;
+    const size_t lds = (size_t)R * 4 + 2 * WR * WC * 4 + (size_t)R * p.chunk_steps * kStep * 2;
+    static DeviceOnce once;
+    const int rc = once.run([]() -> int {
+        DCIH_HIP(hipFuncSetAttribute((const void*)partition_bounds_kernel<RT, CT, WR, WC, WAVES, WHOLE, true>,
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        DCIH_HIP(hipFuncSetAttribute((const void*)partition_bounds_kernel<RT, CT, WR, WC, WAVES, WHOLE, false>,
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        return 0;
+    });
+    if (rc) return rc;
+    BoundArgs a = p;
+    a.row_tiles = (int)((p.ppb + R - 1) / R);
+    const dim3 grid((unsigned)((int64_t)a.row_tiles * B));
+    if (a.dim % 8 == 0)
+        hipLaunchKernelGGL((partition_bounds_kernel<RT, CT, WR, WC, WAVES, WHOLE, true>), grid, dim3(NT), lds, s, a);
+    else
+        hipLaunchKernelGGL((partition_bounds_kernel<RT, CT, WR, WC, WAVES, WHOLE, false>), grid, dim3(NT), lds, s, a);
+    DCIH_HIP(hipGetLastError());
+    return 0;
+}
+
+int partition_bounds(const QueryArgs& a, void* ws_, hipStream_t s) {
+    char* ws = (char*)ws_;
+    const Room r = room_of(a);
+    const int rc = pack(a, r, ws, s);
+    if (rc) return rc;
+    const Shape y = shape_of(a);
+    BoundArgs p{a.data, a.N, a.ppb, a.dim, r.steps, a.nq, r.tiles, y.whole ? r.steps : kChunk / kStep, 0, r.parts,
+                (const Header*)(ws + r.header), (const float2*)(ws + r.qinfo), (const _Float16*)(ws + r.frags),
+                (uint32_t*)(ws + r.bounds)};
+    if (y.wr == 4 && y.ct == 1) return y.whole ? launch_bounds<1, 1, 4, 1, 4, true>(p, a.B, s) : launch_bounds<1, 1, 4, 1, 4, false>(p, a.B, s);
+    if (y.wr == 4) return y.whole ? launch_bounds<1, 2, 4, 1, 4, true>(p, a.B, s) : launch_bounds<1, 2, 4, 1, 4, false>(p, a.B, s);
+    if (y.wr == 2) return y.whole ? launch_bounds<2, 2, 2, 2, 2, true>(p, a.B, s) : launch_bounds<2, 2, 2, 2, 2, false>(p, a.B, s);
+    if (y.whole) return launch_bounds<4, 2, 1, 4, 2, true>(p, a.B, s);
+    return launch_bounds<2, 2, 1, 8, 3, false>(p, a.B, s);
+}
+
+int pick_items(const QueryArgs& a, void* ws_, int round, int rounds, hipStream_t s) {
+    char* ws = (char*)ws_;
+    const Room r = room_of(a);
+    uint32_t* bounds = (uint32_t*)(ws + r.bounds);
+    uint32_t* limits = (uint32_t*)(ws + r.limits);
+    uint32_t* last = (uint32_t*)(ws + r.last);
+    if (round == 0) {
+        const int S = a.B * r.parts, per = a.nq >= 8192 && S <= 512 ? 16 : 4;
+        const dim3 grid((unsigned)((a.nq + per - 1) / per));
+#define DCIH_LIMITS(V)                                                                                              \
+    hipLaunchKernelGGL(pick_limits_kernel<V>, grid, dim3(256), (size_t)S * (per + 1) * 4, s, bounds, S, a.nq, per, \
+                       a.pick_rank, 2 * a.pick_rank, limits, last)
+        if (S <= 64) DCIH_LIMITS(1); else if (S <= 128) DCIH_LIMITS(2); else if (S <= 256) DCIH_LIMITS(4);
+        else if (S <= 512) DCIH_LIMITS(8); else if (S <= 1024) DCIH_LIMITS(16); else DCIH_LIMITS(32);
+#undef DCIH_LIMITS
+        DCIH_HIP(hipGetLastError());
+    }
+    const int groups = (a.nq + kListQueries - 1) / kListQueries;
+    ListArgs p{bounds, limits, a.out_dists + (a.k - 1), a.k, last, a.B, r.parts, a.nq, groups, round, rounds,
+               (int32_t*)(ws + r.items), (uint32_t*)(ws + r.counts) + round, (uint32_t*)(ws + r.part_counts)};
+    const dim3 grid((unsigned)((int64_t)a.B * groups));
+    hipLaunchKernelGGL(list_items_kernel<true>, grid, dim3(256), 0, s, p);
+    hipLaunchKernelGGL(list_items_kernel<false>, grid, dim3(256), 0, s, p);
+    DCIH_HIP(hipGetLastError());
+    return 0;
+}
+
+Picked picked_items(const QueryArgs& a, void* ws_, int round) {
+    char* ws = (char*)ws_;
+    const Room r = room_of(a);
+    return Picked{(const int32_t*)(ws + r.items), (const uint32_t*)(ws + r.counts) + round, (const uint32_t*)(ws + r.last)};
+}
+
+}  // namespace dcih

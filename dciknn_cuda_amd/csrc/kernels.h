@@ -104,6 +104,18 @@ struct QueryArgs {
     int32_t* out_ids;        // [nq][k]
     int float_ids;           // 1: ids are stored as float32 values in the same place
     float* out_dists;        // [nq][k]; blind: null, or the promoting steps as floats
+    // a call in rounds (bounds.hip)
+    const int32_t* picked;   // null = all nq * B items, else the round's, of which every die takes one run
+    const uint32_t* picked_count;
+    int64_t picked_expect;   // about how many there are
+    int64_t picked_cover;    // ... and how many there seldom are more of: what a launch of one workgroup per item covers
+    const uint32_t* only;    // merge: null, or only the queries whose word here is only_round
+    uint32_t only_round;
+    int pick_rounds;         // 0: everything is traversed at once
+    int pick_rank;           // the first round takes the partitions of so many nearest rows
+    int pick_rule;           // DCIH_OPT_ROUNDS value
+    double pick_first;       // partitions per query the first round is expected to take
+    double share;            // share of all items that are expected to be traversed (1 but for such calls)
     float* dense;            // null, or [nq][N]: the step-by-step kernel stores every candidate's score here instead of keeping a top-k
 };
 // About how many promotions a partition's traversal takes before it stops: k_stop of them by a window's
@@ -137,7 +149,7 @@ struct TraversalCosts { double dense_item, batch_item, batch_per_promotion, dens
 inline TraversalCosts traversal_costs(const QueryArgs& a, double promotions) {
     TraversalCosts c;
     const double ppb = (double)a.ppb, windows = (double)a.L * (ppb / (double)a.T + 3.0);
-    const double size = (double)a.M / 2.0, length = (double)a.L / 7.0, items = (double)a.nq * (double)a.B;
+    const double size = (double)a.M / 2.0, length = (double)a.L / 7.0, items = (double)a.nq * (double)a.B * a.share;
     c.dense_item = (0.0086 + 1.8e-5 * windows + 1.1e-6 * (double)a.L * ppb) * size;
     c.batch_per_promotion = 1.37e-3 * length * size;
     c.batch_item = 0.0063 * length * size + c.batch_per_promotion * promotions;
@@ -199,6 +211,7 @@ size_t query_gscratch_bytes(const QueryArgs& a);
 // Batch traversal (traverse_block.hip): whether the shape fits its fixed LDS
 // tables, and the launch itself.
 bool block_traversal_supported(const QueryArgs& a, size_t* lds_bytes);
+bool block_takes_lists(const QueryArgs& a);
 int query_block(const QueryArgs& a, hipStream_t s);
 // Dense traversal (traverse_dense.hip): every point's promoting step at once.  Works
 // through the lists the batch kernel filled (a.dense_items) or, with a.mode == 3,
@@ -213,6 +226,26 @@ int rows8_query_bytes(int dim);
 int code_rows(const float* d_data, int64_t n, int dim, int64_t ppb, int B, unsigned char* d_recs, uint32_t* d_bounds,
               hipStream_t s);
 int code_queries(const float* d_query, int nq, int dim, unsigned char* d_recs, hipStream_t s);
+
+// The run of a list of `count` items that die x of X takes: its first item and their number.
+__device__ inline int64_t picked_run(const uint32_t* d_count, int x, int X, int64_t& first) {
+    const int64_t count = *d_count, each = (count + X - 1) / X;
+    first = each * x;
+    return min(each, max((int64_t)0, count - first));
+}
+// Calls in rounds (bounds.hip): lower bounds of every (query, partition)'s nearest distance, and the items each
+// round takes.  Scratch of bounds_bytes(); bounds_cost: about how long the bounds take, us.  partition_bounds also
+// clears a.part.
+constexpr int kPickCountWords = 64;
+struct Picked { const int32_t* items; const uint32_t* count; const uint32_t* last_round; };
+bool bounds_supported(const QueryArgs& a);
+size_t bounds_bytes(const QueryArgs& a);
+double bounds_cost(const QueryArgs& a);
+int partition_bounds(const QueryArgs& a, void* ws, hipStream_t s);
+int pick_items(const QueryArgs& a, void* ws, int round, int rounds, hipStream_t s);
+Picked picked_items(const QueryArgs& a, void* ws, int round);
+// Whether a call is worth its rounds; sets a.pick_rounds, a.pick_first and a.share.
+bool plan_rounds(QueryArgs& a);
 
 // Full ranking (exhaustive.hip) for num_neighbours above the points per partition,
 // where the traversal provably visits everything: queries are processed `chunk` at
@@ -239,9 +272,10 @@ int query_dense(const QueryArgs& a, const float* d_dirs, void* ws, int chunk, hi
 // Whether a call goes to the dense kernel as a whole (given that the shape fits it).
 bool takes_dense_kernel(const QueryArgs& a);
 
+// bounds_ws: bounds_bytes(a) of scratch where a.pick_rounds is set.
 // ev: null, or five events recorded before the traversal, after the batch kernel (if it
 // ran: ran[0]), after the dense kernel (if it ran: ran[1]), between traversal and merge,
 // and after the merge.
-int query(const QueryArgs& a, hipStream_t s, hipEvent_t* ev, bool* ran);
+int query(const QueryArgs& a, void* bounds_ws, hipStream_t s, hipEvent_t* ev, bool* ran);
 
 }  // namespace dcih

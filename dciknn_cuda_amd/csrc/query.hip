@@ -314,6 +314,7 @@ __device__ inline void merge_by_sorting(unsigned long long* buf, int cap, int k,
 __global__ __launch_bounds__(kMergeThreads) void merge_topk_kernel(QueryArgs a, int cap) {
     extern __shared__ unsigned long long buf[];
     const int qi = blockIdx.x;
+    if (a.only && a.only[qi] != a.only_round) return;
     merge_by_sorting(buf, cap, a.k, a.part + (int64_t)qi * a.B * a.kcap, (int64_t)a.B * a.kcap);
     for (int j = threadIdx.x; j < a.k; j += blockDim.x) store_result(a, qi, j, buf[j]);
 }
@@ -330,6 +331,7 @@ __global__ __launch_bounds__(NT) void merge_heads_kernel(QueryArgs a, int heads)
     __shared__ unsigned long long buf[kCap];
     __shared__ uint32_t s_count;
     const int tid = threadIdx.x, qi = blockIdx.x;
+    if (a.only && a.only[qi] != a.only_round) return;
     const unsigned long long* src = a.part + (int64_t)qi * a.B * a.kcap;
     const int nheads = a.B * heads;
     unsigned long long best = ~0ull;
@@ -447,9 +449,44 @@ bool takes_dense_kernel(const QueryArgs& a) {
     return c.dense < c.batch;
 }
 
+bool plan_rounds(QueryArgs& a) {
+    a.pick_rounds = 0;
+    a.share = 1.0;
+    if (a.mode != 0 || a.pick_rule == 1 || !bounds_supported(a)) return false;
+    // The r nearest rows of a query lie in about B (1 - e^(-r/B)) partitions (rows in no particular order).  Round 1
+    // takes those of the k nearest, and where traversals find most of them the later rounds add a tenth.  A call of so few items
+    // that twice as many partitions are one more item for some workgroups takes those of the 2 k nearest instead: a second
+    // round is then mostly empty, and waiting for one more item would take longer.
+    const double B = (double)a.B;
+    auto parts_of = [&](double r) { return fmin(B, B * (1.0 - exp(-r / B)) + 0.5); };
+    const bool few = (double)a.nq * parts_of(2.0 * (double)a.k) <= 1024.0;
+    const double first = parts_of(few ? 2.0 * (double)a.k : (double)a.k);
+    const double share = fmin(1.0, (few ? first : 1.1 * first + 0.2) / B);
+    const bool can_dense = dense_traversal_supported(a, nullptr), can_block = block_traversal_supported(a, nullptr);
+    bool fits = true;
+    auto time = [&](double part) {
+        QueryArgs p = a;
+        p.share = part;
+        const TraversalCosts c = traversal_costs(p, fmin(expected_promotions(a), (double)a.ppb));
+        const bool dense = can_dense && takes_dense_kernel(p);
+        fits = fits && (dense || (can_block && block_takes_lists(a)));      // (the step-by-step kernel takes no round's items)
+        return dense ? c.dense : c.batch;
+    };
+    const double whole = time(1.0), rounds = time(first / B) + (few ? 15.0 : time(share - first / B)) + bounds_cost(a) + 30.0;
+    (void)time(share);
+    if (!fits || (a.pick_rule == 0 && rounds > 0.85 * whole)) return false;
+    a.pick_rounds = few ? 2 : (whole > 1500.0 || a.pick_rule == 2 ? 3 : 2);
+    a.pick_rank = few ? 2 * a.k : a.k;
+    a.pick_first = first;
+    a.share = share;
+    return true;
+}
+
 int merge_lists(const QueryArgs& a, hipStream_t s) {
     // (the lists of the step-by-step kernel ascend as long as its top-k stays in LDS)
-    const int heads = min(a.kcap, (int)(((int64_t)2 * a.k + a.B - 1) / a.B));
+    // (after a round only the lists of the partitions taken so far, about pick_first of them, hold anything)
+    const double lists = a.pick_rounds ? fmax(1.0, a.pick_first) : (double)a.B;
+    const int heads = min(a.kcap, (int)ceil((a.pick_rounds ? 3.0 : 2.0) * (double)a.k / lists));
     if (a.k <= 32 && (int64_t)a.B * heads <= 2 * kWave) {
         hipLaunchKernelGGL(merge_heads_kernel<kWave>, dim3((unsigned)a.nq), dim3(kWave), 0, s, a, heads);
     } else if (a.k <= kMergeThreads && (int64_t)a.B * heads < 0x7fffffffLL) {
@@ -463,7 +500,7 @@ int merge_lists(const QueryArgs& a, hipStream_t s) {
     return 0;
 }
 
-int query(const QueryArgs& a_in, hipStream_t s, hipEvent_t* ev, bool* ran) {
+int query(const QueryArgs& a_in, void* bounds_ws, hipStream_t s, hipEvent_t* ev, bool* ran) {
     QueryArgs a = a_in;
     if (a.nq <= 0) return 0;
     if (a.k > 8192)
@@ -502,55 +539,81 @@ int query(const QueryArgs& a_in, hipStream_t s, hipEvent_t* ev, bool* ran) {
         const int rc = allow_full_lds();
         if (rc) return rc;
     }
-    const bool lists = a.mode != 3;         // the dense kernel alone leaves no item to another
-    if (lists || a.counters) {   // zero the counters and the list lengths with a kernel (safe under graph capture);
-        // the dense lists' lengths follow the hand-over list's
-        const int64_t cells = a.counters ? (int64_t)a.nq * 4 : 0;
-        hipLaunchKernelGGL(zero_u64_kernel, dim3((unsigned)max((int64_t)1, min((int64_t)1024, (cells + 255) / 256))),
-                           dim3(256), 0, s, a.counters, cells, a.redo_count, kListCountWords);
-    }
-    if (ev) (void)hipEventRecord(ev[0], s);
-    a.item_list = nullptr;
-    a.item_count = nullptr;
-    if (use_block || a.mode == 3) {
-        if (use_block) {
-            if (a.rpos_ready && !*a.rpos_ready) {      // the first batch traversal over this index
-                const int rc = fill_positions_by_first(a.sids, a.inv, const_cast<uint16_t*>(a.rpos), a.N, a.M, a.L, s);
+    auto traverse = [&](QueryArgs a) -> int {
+        const bool lists = a.mode != 3;         // the dense kernel alone leaves no item to another
+        if (lists || a.counters) {   // zero the counters and the list lengths with a kernel (safe under graph capture);
+            // the dense lists' lengths follow the hand-over list's
+            const int64_t cells = a.counters ? (int64_t)a.nq * 4 : 0;
+            hipLaunchKernelGGL(zero_u64_kernel, dim3((unsigned)max((int64_t)1, min((int64_t)1024, (cells + 255) / 256))),
+                               dim3(256), 0, s, a.counters, cells, a.redo_count, kListCountWords);
+        }
+        a.item_list = nullptr;
+        a.item_count = nullptr;
+        if (use_block || a.mode == 3) {
+            if (use_block) {
+                if (a.rpos_ready && !*a.rpos_ready) {      // the first batch traversal over this index
+                    const int rc = fill_positions_by_first(a.sids, a.inv, const_cast<uint16_t*>(a.rpos), a.N, a.M, a.L, s);
+                    if (rc) return rc;
+                    if (!a.recorded) *a.rpos_ready = 1;
+                }
+                const int rc = query_block(a, s);
                 if (rc) return rc;
-                if (!a.recorded) *a.rpos_ready = 1;
+                if (ev) (void)hipEventRecord(ev[1], s);
+                if (ran) ran[0] = true;
             }
-            const int rc = query_block(a, s);
-            if (rc) return rc;
-            if (ev) (void)hipEventRecord(ev[1], s);
-            if (ran) ran[0] = true;
+            if (a.mode == 3 || a.dense_items) {
+                QueryArgs d = a;
+                if (use_block) d.picked = nullptr;      // what the batch kernel handed over
+                const int rc = query_dense_items(d, s);
+                if (rc) return rc;
+                if (ev) (void)hipEventRecord(ev[2], s);
+                if (ran) ran[1] = true;
+            }
         }
-        if (a.mode == 3 || a.dense_items) {
-            const int rc = query_dense_items(a, s);
-            if (rc) return rc;
-            if (ev) (void)hipEventRecord(ev[2], s);
-            if (ran) ran[1] = true;
+        if (use_block) {
+            // whatever the batch kernel handed back goes through the step-by-step kernel
+            a.item_list = a.redo_items;
+            a.item_count = a.redo_count;
+            if (y.lds_counters) {
+                const int64_t grid = min((int64_t)a.nq * a.B, (int64_t)1024);
+                hipLaunchKernelGGL(traverse_kernel<true>, dim3((unsigned)grid), dim3(kWave), y.lds_bytes, s, a, y);
+            } else {      // partitions whose visit counters do not fit LDS: a slice of global scratch per workgroup
+                if (!a.gscratch) return fail(-1, "query: counter scratch missing");
+                const int64_t grid = min(traverse_grid(a, y), (int64_t)1024);
+                hipLaunchKernelGGL(traverse_kernel<false>, dim3((unsigned)grid), dim3(kWave), y.lds_bytes, s, a, y);
+            }
+        } else if (a.mode != 3) {
+            const int64_t grid = traverse_grid(a, y);
+            if (y.lds_counters) {
+                hipLaunchKernelGGL(traverse_kernel<true>, dim3((unsigned)grid), dim3(kWave), y.lds_bytes, s, a, y);
+            } else {
+                if (!a.gscratch) return fail(-1, "query: counter scratch missing");
+                hipLaunchKernelGGL(traverse_kernel<false>, dim3((unsigned)grid), dim3(kWave), y.lds_bytes, s, a, y);
+            }
         }
-    }
-    if (use_block) {
-        // whatever the batch kernel handed back goes through the step-by-step kernel
-        a.item_list = a.redo_items;
-        a.item_count = a.redo_count;
-        if (y.lds_counters) {
-            const int64_t grid = min((int64_t)a.nq * a.B, (int64_t)1024);
-            hipLaunchKernelGGL(traverse_kernel<true>, dim3((unsigned)grid), dim3(kWave), y.lds_bytes, s, a, y);
-        } else {      // partitions whose visit counters do not fit LDS: a slice of global scratch per workgroup
-            if (!a.gscratch) return fail(-1, "query: counter scratch missing");
-            const int64_t grid = min(traverse_grid(a, y), (int64_t)1024);
-            hipLaunchKernelGGL(traverse_kernel<false>, dim3((unsigned)grid), dim3(kWave), y.lds_bytes, s, a, y);
+        DCIH_HIP(hipGetLastError());
+        return 0;
+    };
+    if (ev) (void)hipEventRecord(ev[0], s);
+    if (!a.pick_rounds) {
+        const int rc = traverse(a);
+        if (rc) return rc;
+    } else {      // rounds (bounds.hip): the results of one bound what the next has to take
+        int rc = partition_bounds(a, bounds_ws, s);
+        const double all = (double)a.nq * (double)a.B * a.share, first = (double)a.nq * a.pick_first;
+        for (int round = 0; round < a.pick_rounds && !rc; round++) {
+            if (round > 0) rc = merge_lists(a, s);
+            if (!rc) rc = pick_items(a, bounds_ws, round, a.pick_rounds, s);
+            const Picked p = picked_items(a, bounds_ws, round);
+            a.picked = p.items;
+            a.picked_count = p.count;
+            a.picked_expect = (int64_t)fmax(round ? all - first : first, 1.0);
+            a.picked_cover = (int64_t)(round ? 0.6 * first : 1.25 * first) + 64;
+            if (!rc) rc = traverse(a);
+            a.only = round > 0 ? p.last_round : nullptr;
+            a.only_round = (uint32_t)round;
         }
-    } else if (a.mode != 3) {
-        const int64_t grid = traverse_grid(a, y);
-        if (y.lds_counters) {
-            hipLaunchKernelGGL(traverse_kernel<true>, dim3((unsigned)grid), dim3(kWave), y.lds_bytes, s, a, y);
-        } else {
-            if (!a.gscratch) return fail(-1, "query: counter scratch missing");
-            hipLaunchKernelGGL(traverse_kernel<false>, dim3((unsigned)grid), dim3(kWave), y.lds_bytes, s, a, y);
-        }
+        if (rc) return rc;
     }
     DCIH_HIP(hipGetLastError());
     if (ev) (void)hipEventRecord(ev[3], s);

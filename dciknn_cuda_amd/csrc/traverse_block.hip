@@ -1140,6 +1140,30 @@ __global__ __launch_bounds__(NT, MINW) void traverse_block_kernel(QueryArgs a, B
     if (!block_item((int64_t)blockIdx.x, a.xcds, a.B, a.q_count, b, qi)) return;
     traverse_block_item<NT, MINW, COMPACT>(a, y, b, qi + a.q_first);
 }
+// The items a round of a call picked (bounds.hip): a list per die, in the same order, one workgroup each.  (With a loop
+// around the item the registers no longer do: 32 bytes of scratch per lane where there are none.)
+template <int NT, int MINW, bool COMPACT>
+__global__ __launch_bounds__(NT, MINW) void traverse_block_picked_kernel(QueryArgs a, BlockLayout y) {
+    const uint32_t X = (uint32_t)a.xcds, die = blockIdx.x % X, w = blockIdx.x / X;
+    const uint32_t count = *a.picked_count, each = (count + X - 1) / X, at = die * each + w;
+    if (w >= each || at >= count) return;
+    const int32_t item = a.picked[at];
+    const int b = __builtin_amdgcn_readfirstlane(item % a.B), qi = __builtin_amdgcn_readfirstlane(item / a.B);
+    // (nothing waits here: without it this compiler keeps an operand of the item's code in the wrong class of registers)
+    asm volatile("" ::: "memory");
+    __syncthreads();
+    traverse_block_item<NT, MINW, COMPACT>(a, y, b, qi);
+}
+// What more than the launch above covers (more partitions of a query at the same bound than one expects): strides over the rest.
+__global__ __launch_bounds__(256, 3) void traverse_block_rest_kernel(QueryArgs a, BlockLayout y, int64_t covered) {
+    int64_t first;
+    const int64_t count = picked_run(a.picked_count, (int)(blockIdx.x % (unsigned)a.xcds), a.xcds, first);
+    for (int64_t w = covered + blockIdx.x / (unsigned)a.xcds; w < count; w += gridDim.x / (unsigned)a.xcds) {
+        const int32_t item = __builtin_amdgcn_readfirstlane(a.picked[first + w]);
+        traverse_block_item<256, 3, false>(a, y, item % a.B, item / a.B);
+        __syncthreads();          // the next item reuses the tables
+    }
+}
 // Second pass: the workgroups stride over the list of items the compact variants handed back
 // (its length is only known on the device, so the grid is a fixed number of resident workgroups).
 template <int NT, int MINW>
@@ -1177,6 +1201,13 @@ bool block_traversal_supported(const QueryArgs& a, size_t* lds_bytes) {
     return y.lds_bytes <= kMostLds;
 }
 
+// Whether the items of a call's rounds can go to this kernel (what a launch does not cover takes the full tables).
+bool block_takes_lists(const QueryArgs& a) {
+    QueryArgs full = a;
+    full.full_tables = 1;
+    return make_block_layout(full).lds_bytes <= kMostLds;
+}
+
 // Workgroups of four wavefronts a CU holds.
 static int wide_fit(const BlockLayout& y) { return std::max(1, std::min(7, (int)(160 * 1024 / y.lds_bytes))); }
 
@@ -1194,12 +1225,17 @@ static int launch_block(const QueryArgs& a, const BlockLayout& y, int64_t items,
         if (rc_attr) return rc_attr;                                                               \
         hipLaunchKernelGGL(KERNEL, dim3((unsigned)(GRID)), dim3(NT), y.lds_bytes, s, a, y);        \
     } while (0)
-#define DCIH_LAUNCH_COMPACT(MW) DCIH_LAUNCH_KERNEL((traverse_block_kernel<kWave, MW, true>), kWave, items)
+#define DCIH_LAUNCH_COMPACT(MW)                                                                    \
+    do {                                                                                           \
+        if (a.picked) DCIH_LAUNCH_KERNEL((traverse_block_picked_kernel<kWave, MW, true>), kWave, items); \
+        else DCIH_LAUNCH_KERNEL((traverse_block_kernel<kWave, MW, true>), kWave, items);           \
+    } while (0)
     // (the second pass: as many workgroups as the device holds at a time, striding over the list)
     const int64_t resident = std::min(items, (int64_t)a.xcds * 32 * std::max(1, fit));
 #define DCIH_LAUNCH(NT, MW)                                                                        \
     do {                                                                                           \
         if (a.block_list) DCIH_LAUNCH_KERNEL((traverse_block_list_kernel<NT, MW>), NT, resident);  \
+        else if (a.picked) DCIH_LAUNCH_KERNEL((traverse_block_picked_kernel<NT, MW, false>), NT, items); \
         else DCIH_LAUNCH_KERNEL((traverse_block_kernel<NT, MW, false>), NT, items);                \
     } while (0)
     // The kernel's time is chains of dependent reads, so what counts is how many items a CU holds: as
@@ -1255,7 +1291,7 @@ int query_block(const QueryArgs& a_query, hipStream_t s) {
         QueryArgs wide = a_in;
         wide.full_tables = 1;
         const BlockLayout y4 = make_block_layout(wide);
-        if (y4.lds_bytes <= kMostLds && (int64_t)a_in.nq * a_in.B <= (int64_t)a_in.xcds * 32 * wide_fit(y4)) a_in.full_tables = a_in.few_items = 1;
+        if (y4.lds_bytes <= kMostLds && (a_in.picked ? a_in.picked_expect : (int64_t)a_in.nq * a_in.B) <= (int64_t)a_in.xcds * 32 * wide_fit(y4)) a_in.full_tables = a_in.few_items = 1;
     }
     const BlockLayout y = make_block_layout(a_in);
     // as many queries per launch as the launch limit allows (nearly always all of them)
@@ -1268,6 +1304,7 @@ int query_block(const QueryArgs& a_query, hipStream_t s) {
     second.block_list = a_in.wide_items;
     second.block_list_count = a_in.wide_count;
     second.wide_items = nullptr;
+    second.picked = nullptr;
     second.q_first = 0;
     second.q_count = a_in.nq;
     const BlockLayout y2 = make_block_layout(second);
@@ -1277,8 +1314,34 @@ int query_block(const QueryArgs& a_query, hipStream_t s) {
     // their own: their stops are on record when the others start, which then size their first
     // epoch from them instead of feeling their way forward (the first resident round of every
     // partition would otherwise do that in the middle of the large launch).  Results do not depend on it.
-    const int lead = a_in.hints_cold && a_in.stop_hint && a_in.nq >= 8 * kLeadQueries ? kLeadQueries : 0;
-    for (int q0 = 0; q0 < a_in.nq; q0 += (q0 < lead ? lead : per_launch)) {
+    const int lead = !a_in.picked && a_in.hints_cold && a_in.stop_hint && a_in.nq >= 8 * kLeadQueries ? kLeadQueries : 0;
+    if (a_in.picked) {
+        QueryArgs a = a_in;
+        if (!two_passes) a.wide_items = nullptr;
+        a.q_first = 0;
+        a.q_count = a.nq;
+        // a workgroup per item, as far as their number can be told; those without one cost 0.2 ns each
+        const int64_t X = a.xcds;
+        const int64_t each = std::min<int64_t>(std::min((a.picked_cover + X - 1) / X, ((int64_t)a.nq * a.B + X - 1) / X),
+                                               0xffffffffLL / 256 / X);
+        int rc = launch_block(a, y, each * X, s);
+        if (rc) return rc;
+        if (each * X < (int64_t)a.nq * a.B) {
+            static DeviceOnce once;
+            rc = once.run([]() -> int {
+                DCIH_HIP(hipFuncSetAttribute((const void*)traverse_block_rest_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+                return 0;
+            });
+            if (rc) return rc;
+            QueryArgs rest = a;
+            rest.full_tables = 1;
+            rest.wide_items = nullptr;
+            const BlockLayout y4 = make_block_layout(rest);
+            hipLaunchKernelGGL(traverse_block_rest_kernel, dim3((unsigned)(X * 32 * wide_fit(y4))), dim3(256), y4.lds_bytes, s, rest, y4, each);
+            DCIH_HIP(hipGetLastError());
+        }
+    }
+    for (int q0 = a_in.picked ? a_in.nq : 0; q0 < a_in.nq; q0 += (q0 < lead ? lead : per_launch)) {
         QueryArgs a = a_in;
         if (!two_passes) a.wide_items = nullptr;
         a.q_first = q0;

@@ -278,9 +278,18 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
     const int X = args->a.xcds;
     const int xcd = (int)(blockIdx.x % X);
     const int64_t g0 = blockIdx.x / X;
-    const bool listed = args->a.dense_items != nullptr && args->a.mode != 3;
-    const int64_t my_count = listed ? (int64_t)args->a.dense_count[xcd]
-                                    : block_items(X, args->a.B, args->a.q_count) / X;
+    int64_t my_count;
+    const int32_t* my_items = nullptr;
+    if (args->a.picked) {
+        int64_t first;
+        my_count = picked_run(args->a.picked_count, xcd, X, first);
+        my_items = args->a.picked + first;
+    } else if (args->a.dense_items != nullptr && args->a.mode != 3) {
+        my_count = (int64_t)args->a.dense_count[xcd];
+        my_items = args->a.dense_items + (int64_t)xcd * args->a.dense_cap;
+    } else {
+        my_count = block_items(X, args->a.B, args->a.q_count) / X;
+    }
     const int slot_first = (int)g0 * args->first, slot_end = (int)min(my_count, (int64_t)slot_first + args->len);
 
     // optional phase profile: thread 0 adds the 100 MHz ticks each phase took
@@ -299,8 +308,8 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
         ArgsPtr args = fresh_args();
         DenseTables tb(smem, args->a, args->y);
         int b, qi;
-        if (listed) {
-            const int64_t item = args->a.dense_items[(int64_t)xcd * args->a.dense_cap + slot];
+        if (my_items) {
+            const int64_t item = my_items[slot];
             b = (int)(item % args->a.B);
             qi = (int)(item / args->a.B);
         } else {
@@ -1339,8 +1348,8 @@ int query_dense_items(const QueryArgs& a_in, hipStream_t s) {
     // starts (10000 points, 10030 windows: 390 and 397 ms).
     const int by_regs = (y.ipt > 15 ? 512 : 1024) / y.nt;
     const int per_cu = (int)max((size_t)1, min((size_t)by_regs, kLdsBytes / y.lds_bytes));
-    const bool listed = a.dense_items && a.mode != 3;
-    const int64_t most = listed ? (int64_t)a.dense_cap : block_items(a.xcds, a.B, a.nq) / a.xcds;
+    const bool listed = a.picked || (a.dense_items && a.mode != 3);
+    const int64_t most = a.picked || !listed ? block_items(a.xcds, a.B, a.nq) / a.xcds : (int64_t)a.dense_cap;
     int64_t per_xcd = max((int64_t)1, min((int64_t)32 * per_cu * 2, most));
     DenseArgs args{a, y, 1, (int)per_xcd, most};
     if (!listed && y.ipt <= 15 && most >= (int64_t)32 * per_cu * 8) {
@@ -1349,6 +1358,12 @@ int query_dense_items(const QueryArgs& a_in, hipStream_t s) {
         args.len = args.first;
         args.step = 1;
         per_xcd = (most + args.first - 1) / args.first;
+    }
+    // (what a round picked is about so many items: enough workgroups that nearly every one takes one item, in order)
+    if (a.picked && y.ipt <= 15 && a.picked_expect / a.xcds >= (int64_t)32 * per_cu * 8) {
+        const int64_t fit = 0xffffffffLL / ((int64_t)a.xcds * y.nt);
+        per_xcd = min(min(fit, most), a.picked_cover / a.xcds);
+        args.step = (int)per_xcd;
     }
     const unsigned grid = (unsigned)(per_xcd * a.xcds);
 #define DCIH_DENSE(NT, IPT, WAVES)                                                                 \

@@ -80,7 +80,8 @@ enum {
  * runs of the new ones, the new points sorted, the runs merged (error where the shape
  * does not allow it: partitions of more than 32256 points).  All give the same index.
  */
-enum { DCIH_OPT_TRAVERSAL = 0, DCIH_OPT_DENSE_MIN_PROMOTIONS = 1, DCIH_OPT_FORGET_HINTS = 2, DCIH_OPT_APPEND = 3 };
+enum { DCIH_OPT_TRAVERSAL = 0, DCIH_OPT_DENSE_MIN_PROMOTIONS = 1, DCIH_OPT_FORGET_HINTS = 2, DCIH_OPT_APPEND = 3,
+       DCIH_OPT_ROUNDS = 4 };
 
 /* Message for the last failing call on this thread ("" if none). */
 const char* dcih_last_error(void);

@@ -1,0 +1,165 @@
+"""Queries that first bound the partitions' nearest distances and then traverse, in rounds, only the partitions
+that can hold a result (DCIH_OPT_ROUNDS), against the same queries traversed as a whole: ids and distances
+must be equal to the bit, whatever the rows are, because a partition is left out only where none of its rows can
+be as near as the k-th result.  Every traversal kernel that can run a round is covered."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+NEVER, ALWAYS = 1, 2
+
+
+def _ask(dci, lib, rounds, Q, k, outer, **kw):
+    from dciknn_cuda_amd import _capi
+    _capi.check(lib.dcih_set_option(dci._dci_inst, _capi.OPT_ROUNDS, rounds))
+    ids, dists = dci.query(Q, k, outer, return_int=True, **kw)
+    torch.cuda.synchronize()
+    return ids.clone(), dists.clone()
+
+
+def _same(gpu, X, Q, M, L, B, T, k, outer, tag=""):
+    dci = gpu.DCI(X.shape[1], M, L, B, T, seed=3)
+    dci.add(X)
+    want = _ask(dci, dci._lib, NEVER, Q, k, outer)
+    got = _ask(dci, dci._lib, ALWAYS, Q, k, outer)
+    dci.free()
+    assert torch.equal(got[0], want[0]), tag
+    assert torch.equal(got[1].view(torch.int32), want[1].view(torch.int32)), tag
+    return want
+
+
+def _rows(kind, n, nq, dim, seed):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    def randn(*s):
+        return torch.randn(*s, generator=g, device="cuda")
+    x = randn(n + nq, dim)
+    if kind == "clusters":
+        x = 30.0 * randn(20, dim)[torch.randint(0, 20, (n + nq,), generator=g, device="cuda")] + x
+    elif kind == "sorted":          # a query's neighbours all lie in one or two partitions
+        x = x[torch.argsort(x[:, 0])]
+        x = x[torch.cat([torch.arange(0, n, device="cuda"), torch.randint(0, n, (nq,), generator=g, device="cuda")])]
+        x[n:] += 0.01 * randn(nq, dim)
+    elif kind == "dup":             # equal distances, by the id alone
+        x = x[torch.randint(0, max(1, n // 8), (n + nq,), generator=g, device="cuda")]
+    elif kind == "grid":
+        x = torch.randint(0, 3, (n + nq, dim), generator=g, device="cuda").float()
+    elif kind == "offset":          # squared lengths a million times the distances'
+        x = x + 3000.0
+    elif kind == "scales":          # rows from 1e-6 to 1e6: most of them outside what 16-bit floats of one scale hold
+        x = x * 10.0 ** (12.0 * torch.rand(n + nq, 1, generator=g, device="cuda") - 6.0)
+    elif kind == "tiny":            # squares below the smallest float: all distances are computed as zero
+        x = x * 1e-25
+    elif kind == "huge":            # squares that overflow
+        x = x * 1e25
+    elif kind == "broken":          # some rows and queries are not finite
+        x[::97] = float("nan")
+        x[5::101, 0] = float("inf")
+        x[7::103, 0] = -float("inf")
+    elif kind == "zero":
+        x[: (n + nq) // 2] = 0.0
+    return x[:n].contiguous(), x[n:].contiguous()
+
+
+# one shape per kernel form: queries 1..32, 33..64, 65..128 and more, rows whole in LDS and staged by columns
+# (past 256 elements), with and without whole octets, one element and one tile past each edge
+@pytest.mark.parametrize("nq", [1, 32, 33, 65, 129, 300])
+@pytest.mark.parametrize("dim", [8, 9, 16, 67, 256, 257, 520])
+def test_forms_of_the_product(gpu, nq, dim):
+    X, Q = _rows("clusters", 5000 + dim, nq, dim, nq * 1000 + dim)
+    _same(gpu, X, Q, 2, 5, 11, 8, 5, 40, "dim %d nq %d" % (dim, nq))
+
+
+@pytest.mark.parametrize("kind", ["normal", "clusters", "sorted", "dup", "grid", "offset", "scales", "tiny", "huge", "broken", "zero"])
+@pytest.mark.parametrize("shape", [(2, 7, 20, 10, 10, 5000), (2, 10, 13, 2, 4, 100), (3, 5, 40, 64, 30, 20), (1, 3, 7, 130, 1, 5)],
+                         ids=["defaults", "narrow", "wide", "one"])
+@pytest.mark.parametrize("dim", [24, 33, 300])
+def test_rows_of_every_kind(gpu, kind, shape, dim):
+    M, L, B, T, k, outer = shape
+    X, Q = _rows(kind, 9001, 150, dim, 17 + dim)
+    ids, _ = _same(gpu, X, Q, M, L, B, T, k, outer, kind)
+    assert ids.shape == (150, k)
+
+
+@pytest.mark.parametrize("n,B", [(130, 2), (257, 128), (1000, 999), (4096, 32), (4097, 32), (31 * 129, 31)])
+def test_partitions_at_the_edges_of_tiles(gpu, n, B):
+    """Partitions of 1, 2, 3, 65, 128, 129 rows, some of them empty, more results asked for than a partition holds."""
+    for k in (1, 3, 40):
+        X, Q = _rows("normal", n, 70, 40, n + k)
+        _same(gpu, X, Q, 2, 4, B, 2, k, 3, "n %d B %d k %d" % (n, B, k))
+
+
+def test_rows_off_their_boundaries(gpu):
+    """Rows and queries that start four bytes past a 16-byte boundary."""
+    X, Q = _rows("clusters", 6001, 90, 64, 5)
+    pool_x = torch.empty(X.numel() + 1, device="cuda")
+    pool_q = torch.empty(Q.numel() + 1, device="cuda")
+    x, q = pool_x[1:].view(X.shape), pool_q[1:].view(Q.shape)
+    x.copy_(X)
+    q.copy_(Q)
+    assert x.data_ptr() % 16 == 4 and q.data_ptr() % 16 == 4
+    _same(gpu, x, q, 2, 7, 20, 10, 10, 500)
+
+
+@pytest.mark.parametrize("k,T,outer", [(3, 2, 100), (10, 10, 5000)], ids=["batch", "dense"])
+def test_more_partitions_at_one_bound_than_expected(gpu, k, T, outer):
+    """Queries that are not finite bound nothing: all their partitions come in round 1, far more items than its
+    launch was sized for."""
+    X, Q = _rows("normal", 60000, 700, 20, 8)
+    Q[::2] = float("nan")
+    _same(gpu, X, Q, 2, 8, 60, T, k, outer)
+
+
+@pytest.mark.parametrize("k,T,outer", [(3, 2, 100), (10, 10, 5000)], ids=["batch", "dense"])
+def test_rounds_in_a_graph(gpu, k, T, outer):
+    from dciknn_cuda_amd import _capi
+    n, dim, nq, B = 30000, 48, 96, 16
+    X, Q = _rows("clusters", n, nq, dim, 21)
+    dci = gpu.DCI(dim, 2, 7, B, T, seed=9)
+    dci.add(X)
+    want = _ask(dci, dci._lib, NEVER, Q, k, outer)
+    _capi.check(dci._lib.dcih_set_option(dci._dci_inst, _capi.OPT_ROUNDS, ALWAYS))
+    ids = torch.empty((nq, k), dtype=torch.int32, device="cuda")
+    dists = torch.empty((nq, k), dtype=torch.float32, device="cuda")
+
+    def call(stream):
+        _capi.check(dci._lib.dcih_query(dci._dci_inst, dim, nq, Q.data_ptr(), k, 0, outer, 10 * k, B, T,
+                                        ids.data_ptr(), dists.data_ptr(), None, stream))
+    s = torch.cuda.Stream()
+    call(s.cuda_stream)
+    call(s.cuda_stream)
+    s.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        call(torch.cuda.current_stream().cuda_stream)
+    for _ in range(4):
+        ids.fill_(-5)
+        dists.fill_(-5.0)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(ids, want[0]) and torch.equal(dists, want[1])
+        call(0)                                # eager work between the replays
+        torch.cuda.synchronize()
+    del g
+    dci.free()
+
+
+def test_what_asks_for_everything_gets_everything(gpu):
+    """Counters and blind queries are of whole traversals, also where rounds are asked for."""
+    from dciknn_cuda_amd import _capi
+    X, Q = _rows("normal", 20000, 40, 32, 4)
+    dci = gpu.DCI(32, 2, 7, 25, 10, seed=3)
+    dci.add(X)
+    res = []
+    for rounds in (NEVER, ALWAYS):
+        _capi.check(dci._lib.dcih_set_option(dci._dci_inst, _capi.OPT_ROUNDS, rounds))
+        counted = dci.query(Q, 10, 500, return_int=True, return_counters=True)
+        blind = dci.query(Q, 10, 500, blind=True, return_int=True)
+        torch.cuda.synchronize()
+        res.append([t.clone() for t in counted] + [t.clone() for t in (blind if isinstance(blind, tuple) else (blind,))])
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
+    dci.free()
