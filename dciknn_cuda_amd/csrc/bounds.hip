@@ -28,13 +28,14 @@ namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef v4f v4f_any __attribute__((aligned(4)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
 constexpr int kPackThreads = 256;
 constexpr int kTile = 32;                 // rows and queries of one matrix instruction
 constexpr int kStep = 16;                 // elements of one
-constexpr int kChunk = 256;               // columns staged at a time where a row tile does not fit LDS as a whole
+constexpr int kWholeDim = 256;            // rows up to here can be kept in LDS whole
 constexpr int kSample = 16;               // rows and queries the scales are taken from
 constexpr int kMostParts = 2048;           // bounds kept per query
 constexpr int kListQueries = 1024;        // queries of a partition listed by one workgroup
@@ -97,24 +98,40 @@ __device__ inline void place_octet(int dim, int j, float (&x)[8]) {
 #pragma unroll
         for (int i = 0; i < 8; i++) x[i] = 0.0f;
 }
-// Rounds to 16 bits and sums the squares of the rounded values and of what was rounded off.
-// (Values too small for a normal 16-bit float become zero here: what the matrix cores make of them does not matter.)
+// Rounds to 16 bits (towards zero: one instruction for two) and sums the squares of the rounded values and of what was
+// rounded off.  What does not fit, or is not finite, makes the first sum so: it is cut to `most` and to zero, the second sum infinite
+// for the latter.  (16-bit floats below 2^-14, which the matrix cores may take as zeros, are allowed for in rounding_floor.)
 __device__ inline v8h round_octet(const float (&x)[8], float scale, float most, float& sq, float& err) {
     v8h out;
+    float s2 = 0.0f, e2 = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        float v = x[i] * scale;
-        const bool finite = fabsf(v) < 3e38f;
-        if (!finite) { v = 0.0f; err = __builtin_inff(); }
-        float c = fminf(most, fmaxf(-most, v));
-        c = fabsf(c) < kHalfMin ? 0.0f : c;
-        out[i] = (_Float16)c;
-        const float back = (float)out[i], off = v - back;
-        sq = __builtin_fmaf(back, back, sq);
-        err = __builtin_fmaf(off, off, err);
+    for (int i = 0; i < 8; i += 2) {
+        const float a = x[i] * scale, b = x[i + 1] * scale;
+        const v2h h = __builtin_bit_cast(v2h, __builtin_amdgcn_cvt_pkrtz(a, b));
+        out[i] = h[0]; out[i + 1] = h[1];
+        s2 = __builtin_amdgcn_fdot2(h, h, s2, false);
+        const float oa = __builtin_fmaf((float)h[0], -1.0f, a), ob = __builtin_fmaf((float)h[1], -1.0f, b);
+        e2 = __builtin_fmaf(oa, oa, e2);
+        e2 = __builtin_fmaf(ob, ob, e2);
     }
+    if (!(s2 < 8.0f * most * most && e2 < 1e30f)) {
+        s2 = e2 = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            float v = x[i] * scale;
+            if (!(fabsf(v) < 3e38f)) { v = 0.0f; e2 = __builtin_inff(); }
+            out[i] = (_Float16)fminf(most, fmaxf(-most, v));
+            const float back = (float)out[i], off = v - back;
+            s2 = __builtin_fmaf(back, back, s2);
+            e2 = __builtin_fmaf(off, off, e2);
+        }
+    }
+    sq += s2;
+    err += e2;
     return out;
 }
+// The largest length of what the values below 2^-14 make up, scaled.
+__device__ inline float rounding_floor(int elements) { return sqrtf((float)elements) * kHalfMin; }
 
 // The first workgroups round 32 queries each, into the order the matrix instructions take them
 // ([32 queries][16 elements]: 64 lanes of 8), times -2; all of them clear what the later launches
@@ -158,79 +175,80 @@ __global__ __launch_bounds__(kPackThreads) void pack_queries_kernel(PackArgs a) 
     err += lane_xor<4>(err); err += lane_xor<2>(err); err += lane_xor<1>(err);
     if ((tid & 7) == 0) {
         const float inv = 1.0f / scale;
-        a.qinfo[q] = make_float2(sq * inv * inv, sqrtf(err) * 1.001f * inv);
+        a.qinfo[q] = make_float2(sq * inv * inv, (sqrtf(err) * 1.001f + rounding_floor(a.steps * kStep)) * inv);
     }
 }
 
 struct BoundArgs {
     const float* data;
     int64_t n, ppb;
-    int dim, steps, nq, tiles, chunk_steps;
-    int row_tiles, parts;                 // row tiles (workgroups) per partition, and the parts bounds are kept for
+    int dim, steps, nq, tiles;
+    int column_steps;                     // staged at a time (even)
+    int next_part, next_tile;             // from a workgroup's row tile to its next one
+    int num_parts, row_tiles, parts;      // partitions, row tiles of each, and the parts of each that bounds are kept for
     const Header* header; const float2* qinfo; const _Float16* frags;
     uint32_t* bounds;                     // [B * parts][nq] float bits
 };
 
-// A workgroup takes R = 32 RT WR rows of one partition, rounds them into LDS and multiplies them with all
-// queries: WR wavefronts along the rows, WC along the queries, each with RT x CT accumulators of 32 x 32.  A row's
-// squared length is where its accumulators start, so what is left to do with a sum is to keep the
-// smallest, in the lane that holds the query's column.  WHOLE: the rows fit LDS over their whole length and stay there;
-// else they are staged kChunk columns at a time, anew for every pass over 32 CT WC queries.
-// 10000 queries on 1M rows of 128 (58 partitions, 10 results): 2.9 ms, 0.88 PFLOP/s, where traversing all 580000 pairs took 24.0 ms
-// and traversing the 112400 that are left takes 6.4; 512 on 10M rows of 96 (100 results): 2.3 ms, bound by staging its rows,
-// 72.5 -> 21 ms; 1000 on 1M rows of 128 with the defaults: 0.43 ms, 19.0 -> 2.3 ms.
-template <int RT, int CT, int WR, int WC, int WAVES, bool WHOLE, bool OCTETS>
-__global__ __launch_bounds__(64 * WR * WC, WAVES) void partition_bounds_kernel(BoundArgs a) {
-    constexpr int kWaves = WR * WC, R = kTile * RT * WR, kGroups = R / 8 / kWaves;
-    static_assert(kGroups >= 1, "eight rows per wavefront at least");
-    extern __shared__ __align__(16) unsigned char smem[];
-    float* s_n = reinterpret_cast<float*>(smem);                    // [R] squared lengths, scaled
-    float* s_red = s_n + R;                                         // [2 * kWaves]
-    v8h* s_rows = reinterpret_cast<v8h*>(smem + R * 4 + 2 * kWaves * 4);
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int b = blockIdx.x / a.row_tiles, rt = blockIdx.x % a.row_tiles;
-    const int64_t off = (int64_t)b * a.ppb;
-    const int in_part = (int)min(a.n - off, a.ppb);
-    const int first = rt * R, rows = min(R, in_part - first);
-    if (rows <= 0) return;
-    const float* base = a.data + (off + first) * a.dim;
-    const float row_scale = a.header->row_scale, query_scale = a.header->query_scale;
-    float sq[kGroups], err[kGroups];
-#pragma unroll
-    for (int g = 0; g < kGroups; g++) sq[g] = err[g] = 0.0f;
+// What the kernels below share.  A workgroup of WR wavefronts along the rows and WC along the queries takes tiles of R = 32 RT WR
+// rows of a partition, each wavefront RT x CT accumulators of 32 x 32.  A row's squared length is where its
+// accumulators start (or is added at their end), so what is left to do with a sum is to keep the smallest, in the lane that holds the
+// query's column.
+template <int RT, int CT, int WR, int WC, int COLUMNS, bool OCTETS>
+struct BoundTile {
+    static constexpr int kWaves = WR * WC, R = kTile * RT * WR, kGroups = R / 8 / kWaves, kOctets = COLUMNS / 64;
+    static_assert(kGroups >= 1 && kOctets >= 1, "eight rows per wavefront at least");
+    typedef float Octets[kGroups][kOctets][8];
+    const BoundArgs& a;
+    const int lane;
+    const bool reads;                     // (streamed rows: the first kWaves wavefronts read, the others multiply)
+    const int wave, wr, wc;
+    const float row_scale, query_scale;
+    const float* base;                    // of the tile: its first row, number of rows, and its bounds
+    int rows;
+    uint32_t* out;
 
-    // Rounds columns [16 s0, 16 (s0 + ns)) of the tile into LDS, in the order the matrix instructions take them.
-    // A lane group of eight takes eight rows, so that its stores hit different banks; eight such groups read 256 bytes of a row.
-    auto stage = [&](int s0, int ns, bool sums) {
-        const int octets = 2 * ns;
+    __device__ __forceinline__ BoundTile(const BoundArgs& args)
+        : a(args), lane((int)(threadIdx.x & 63)), reads(__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) < kWaves),
+          wave(__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) % kWaves), wr(wave / WC), wc(wave % WC),
+          row_scale(args.header->row_scale), query_scale(args.header->query_scale), base(nullptr), rows(0), out(nullptr) {}
+
+    // Row tile rt of partition b.
+    __device__ __forceinline__ void take(int b, int rt) {
+        const int64_t off = (int64_t)b * a.ppb, first = off + (int64_t)rt * R;
+        rows = (int)min((int64_t)R, min(a.n, off + a.ppb) - first);
+        base = a.data + first * a.dim;
+        out = a.bounds + ((int64_t)b * a.parts + rt * a.parts / a.row_tiles) * a.nq;
+    }
+    // Columns [16 s0 + 8 o0, ..) of the tile's rows, kOctets octets per lane of each of its kGroups rows: read, then rounded into LDS in
+    // the order the matrix instructions take them.  A lane group of eight takes eight rows, so that its stores hit different banks; eight
+    // such groups read 256 bytes of a row.  All of a wavefront's reads are under way before the first is used.
+    __device__ __forceinline__ void read(Octets& x, int s0, int o0, int octets) const {
 #pragma unroll
         for (int g = 0; g < kGroups; g++) {
             const int r = (g * kWaves + wave) * 8 + (lane & 7);
             const float* row = base + (int64_t)min(r, rows - 1) * a.dim;
-            for (int o0 = 0; o0 < octets; o0 += 16) {
-                float x[2][8];
 #pragma unroll
-                for (int u = 0; u < 2; u++) {
-                    const int o = min(o0 + 8 * u + (lane >> 3), octets - 1);
-                    load_octet<OCTETS>(row, a.dim, s0 * kStep + o * 8, x[u]);
-                }
+            for (int u = 0; u < kOctets; u++) load_octet<OCTETS>(row, a.dim, s0 * kStep + min(o0 + 8 * u + (lane >> 3), octets - 1) * 8, x[g][u]);
+        }
+    }
+    __device__ __forceinline__ void place(Octets& x, v8h* to, int pitch, int s0, int o0, int octets, float (&sq)[kGroups], float (&err)[kGroups]) const {
 #pragma unroll
-                for (int u = 0; u < 2; u++) {
-                    const int o = o0 + 8 * u + (lane >> 3);
-                    if (o < octets) {
-                        place_octet<OCTETS>(a.dim, s0 * kStep + o * 8, x[u]);
-                        float s2 = 0.0f, e2 = 0.0f;
-                        const v8h h = round_octet(x[u], row_scale, kHalfMax, s2, e2);
-                        if (sums) { sq[g] += s2; err[g] += e2; }
-                        s_rows[((r >> 5) * a.chunk_steps + (o >> 1)) * 64 + (o & 1) * 32 + (r & 31)] = h;
-                    }
+        for (int g = 0; g < kGroups; g++) {
+            const int r = (g * kWaves + wave) * 8 + (lane & 7);
+#pragma unroll
+            for (int u = 0; u < kOctets; u++) {
+                const int o = o0 + 8 * u + (lane >> 3);
+                if (o < octets) {
+                    place_octet<OCTETS>(a.dim, s0 * kStep + o * 8, x[g][u]);
+                    to[((r >> 5) * pitch + (o >> 1)) * 64 + (o & 1) * 32 + (r & 31)] = round_octet(x[g][u], row_scale, kHalfMax, sq[g], err[g]);
                 }
             }
         }
-    };
-    float most_n = 0.0f, most_e = 0.0f;      // of the tile's rows, not scaled
-    auto finish_sums = [&]() {
-        const float to_sum = query_scale / row_scale, inv = 1.0f / row_scale;
+    }
+    // Squared lengths, scaled as the products are (infinite past the last row), and the wavefront's largest length and error.
+    __device__ __forceinline__ void put_sums(const float (&sq)[kGroups], const float (&err)[kGroups], float* s_n, float* s_red) const {
+        const float to_sum = query_scale / row_scale;
         float mn = 0.0f, me = 0.0f;
 #pragma unroll
         for (int g = 0; g < kGroups; g++) {
@@ -244,14 +262,16 @@ __global__ __launch_bounds__(64 * WR * WC, WAVES) void partition_bounds_kernel(B
         mn = fmaxf(mn, lane_xor<4>(mn)); mn = fmaxf(mn, lane_xor<2>(mn)); mn = fmaxf(mn, lane_xor<1>(mn));
         me = fmaxf(me, lane_xor<4>(me)); me = fmaxf(me, lane_xor<2>(me)); me = fmaxf(me, lane_xor<1>(me));
         if (lane == 0) { s_red[wave] = mn; s_red[kWaves + wave] = me; }
-        __syncthreads();
+    }
+    // Largest squared length and largest error of the tile's rows.
+    __device__ __forceinline__ float2 most(const float* s_red) const {
+        float n = 0.0f, e = 0.0f;
 #pragma unroll
-        for (int w = 0; w < kWaves; w++) { most_n = fmaxf(most_n, s_red[w]); most_e = fmaxf(most_e, s_red[kWaves + w]); }
-        most_n *= inv * inv;
-        most_e = sqrtf(most_e) * 1.001f * inv;
-    };
-    const int wr = wave / WC, wc = wave % WC;
-    auto lengths = [&](int r) -> v16f {      // the accumulators' start: squared lengths of row tile r of this wavefront
+        for (int w = 0; w < kWaves; w++) { n = fmaxf(n, s_red[w]); e = fmaxf(e, s_red[kWaves + w]); }
+        const float inv = 1.0f / row_scale;
+        return make_float2(n * inv * inv, (sqrtf(e) * 1.001f + rounding_floor(a.steps * kStep)) * inv);
+    }
+    __device__ __forceinline__ v16f lengths(const float* s_n, int r) const {      // of row tile r of this wavefront
         v16f v;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -259,124 +279,259 @@ __global__ __launch_bounds__(64 * WR * WC, WAVES) void partition_bounds_kernel(B
             v[4 * i] = t.x; v[4 * i + 1] = t.y; v[4 * i + 2] = t.z; v[4 * i + 3] = t.w;
         }
         return v;
+    }
+    // The queries' steps in the order a wavefront multiplies them: all of tiles first .. first + CT - 1, then of those kPass
+    // further on, and from the beginning again.  q8 holds the next two; a step's registers take the step after the next one once it has
+    // been multiplied, no sooner, or the compiler copies them, which waits for what is under way.
+    struct Queries {
+        v8h q8[2][CT];
+        uint32_t at, group, left;         // bytes from a.frags on: the step read next and its tiles' first one; steps left of those
+        uint32_t first, end, stride;      // the first tiles; past the last; from tiles to the next tiles
+        uint32_t mine[CT];                // the lane's place in a step
     };
-    const float unscale = 1.0f / (row_scale * query_scale);
-    const float sum_error = (float)(a.steps * kStep + 64) * 0x1.8p-22f, dist_error = 1.0f - (float)(a.dim + 32) * 0x1p-23f;
-    uint32_t* out = a.bounds + ((int64_t)b * a.parts + rt * a.parts / a.row_tiles) * a.nq;
-    // The smallest sum of each of 32 CT queries over the wavefront's rows -> their partition's bounds.
-    auto finish = [&](const v16f (&acc)[RT][CT], int q, bool mine, float2 info, uint32_t have) {
+    __device__ __forceinline__ void read_queries(Queries& y, v8h (&q)[CT]) const {
+#pragma unroll
+        for (int c = 0; c < CT; c++) q[c] = *reinterpret_cast<const v8h*>(reinterpret_cast<const char*>(a.frags) + (y.at + y.mine[c]));
+    }
+    __device__ __forceinline__ void next_step(Queries& y) const {
+        y.left--;
+        const uint32_t on = y.group + y.stride, group = on < y.end ? on : y.first;
+        const bool over = y.left == 0;
+        y.at = over ? group : y.at + 1024;
+        y.group = over ? group : y.group;
+        y.left = over ? (uint32_t)a.steps : y.left;
+    }
+    __device__ __forceinline__ void start_queries(Queries& y, int tile) const {
+        constexpr int kPass = CT * WC;
+        const uint32_t bytes = (uint32_t)a.steps * 1024u;
+        y.first = (uint32_t)tile * bytes;
+        y.end = (uint32_t)a.tiles * bytes;
+        y.stride = kPass * bytes;
+        y.at = y.group = y.first;
+        y.left = (uint32_t)a.steps;
+#pragma unroll
+        for (int c = 0; c < CT; c++) y.mine[c] = c * bytes + lane * 16;
+        read_queries(y, y.q8[0]);
+        next_step(y);
+        read_queries(y, y.q8[1]);
+        next_step(y);
+    }
+    // The next ns (an even number of) steps.
+    __device__ __forceinline__ void multiply_steps(v16f (&acc)[RT][CT], const v8h* rows_at, int pitch, Queries& y, int ns) const {
+        v8h x8[2][RT];
+#pragma unroll
+        for (int r = 0; r < RT; r++) x8[0][r] = rows_at[r * pitch * 64];
+        auto one = [&](const v8h* next_rows, v8h (&x)[RT], v8h (&x_next)[RT], v8h (&q)[CT]) {
+#pragma unroll
+            for (int r = 0; r < RT; r++) x_next[r] = next_rows[r * pitch * 64];
+            Queries then = y;
+            next_step(then);
+#pragma unroll
+            for (int r = 0; r < RT; r++)
+#pragma unroll
+                for (int c = 0; c < CT; c++) acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[r], q[c], acc[r][c], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            read_queries(y, q);
+            __builtin_amdgcn_sched_barrier(0);
+            y.at = then.at; y.group = then.group; y.left = then.left;
+        };
+        for (int s = 0; s < ns; s += 2) {
+            one(rows_at + (s + 1) * 64, x8[0], x8[1], y.q8[0]);
+            one(rows_at + min(s + 2, ns - 1) * 64, x8[1], x8[0], y.q8[1]);
+        }
+    }
+    // The smallest sum of each of 32 CT queries over the wavefront's rows -> their bounds; q: the lane's query of the first 64.
+    __device__ __forceinline__ void finish(const v16f (&acc)[RT][CT], int q, bool mine, const float2 (&info)[(CT + 1) / 2],
+                                           const uint32_t (&have)[(CT + 1) / 2], float2 most) const {
+        const float unscale = 1.0f / (row_scale * query_scale);
+        const float sum_error = (float)(a.steps * kStep + 64) * 0x1.8p-22f, dist_error = 1.0f - (float)(a.dim + 32) * 0x1p-23f;
         float best[CT];
 #pragma unroll
-        for (int c = 0; c < CT; c++) {
-            best[c] = acc[0][c][0];
+        for (int c = 0; c < CT; c++) {      // (four chains each: a single one would wait for every result)
+            float part[4];
 #pragma unroll
-            for (int r = 0; r < RT; r++)
+            for (int i = 0; i < 4; i++) part[i] = fminf(fminf(acc[0][c][i], acc[0][c][i + 4]), acc[0][c][i + 8]);
 #pragma unroll
-                for (int i = 0; i < 16; i++) best[c] = fminf(best[c], acc[r][c][i]);
-            best[c] = fminf(best[c], lane_xor<32>(best[c]));
+            for (int i = 0; i < 4; i++) {
+                part[i] = fminf(part[i], acc[0][c][i + 12]);
+#pragma unroll
+                for (int r = 1; r < RT; r++) {
+                    part[i] = fminf(fminf(part[i], acc[r][c][i]), acc[r][c][i + 4]);
+                    part[i] = fminf(fminf(part[i], acc[r][c][i + 8]), acc[r][c][i + 12]);
+                }
+            }
+            best[c] = fminf(fminf(part[0], part[1]), fminf(part[2], part[3]));
         }
-        const float v = CT == 2 && lane >= 32 ? best[CT - 1] : best[0];
-        const float d2 = v * unscale + info.x - sum_error * (most_n + info.x);
-        float d = sqrtf(fmaxf(d2, 0.0f)) - most_e - info.y;
-        d = fmaxf(d, 0.0f) * dist_error;
-        if (!(d > 1e-14f)) d = 0.0f;                          // (squares below the smallest float count as nothing in the distances)
-        const uint32_t bits = __builtin_bit_cast(uint32_t, d);
-        if (mine && bits < have) atomicMin(&out[q], bits);
-    };
-    const v8h* frags = reinterpret_cast<const v8h*>(a.frags);
+#pragma unroll
+        for (int c = 0; c < CT; c++) best[c] = fminf(best[c], lane_xor<32>(best[c]));
+#pragma unroll
+        for (int c = 0; c < (CT + 1) / 2; c++) {
+            const float v = CT >= 2 && lane >= 32 ? best[min(2 * c + 1, CT - 1)] : best[2 * c];
+            const float d2 = v * unscale + info[c].x - sum_error * (most.x + info[c].x);
+            float d = sqrtf(fmaxf(d2, 0.0f)) - most.y - info[c].y;
+            d = fmaxf(d, 0.0f) * dist_error;
+            if (!(d > 1e-14f)) d = 0.0f;                      // (squares below the smallest float count as nothing in the distances)
+            const uint32_t bits = __builtin_bit_cast(uint32_t, d);
+            if (mine && q + 64 * c < a.nq && bits < have[c]) atomicMin(&out[q + 64 * c], bits);
+        }
+    }
+};
+
+// Many queries, rows of at most kWholeDim elements: a workgroup keeps one row tile in LDS and takes all queries past it.  Bound by
+// the matrix cores and the reads of the queries from L2 (32 bytes per CU and clock at the full rate).
+template <int RT, int CT, int WC, int WAVES, bool OCTETS>
+__global__ __launch_bounds__(64 * WC, WAVES) void bounds_resident_kernel(BoundArgs a) {
+    typedef BoundTile<RT, CT, 1, WC, 128, OCTETS> Tile;
+    extern __shared__ __align__(16) unsigned char smem[];
+    float* s_n = reinterpret_cast<float*>(smem);
+    float* s_red = s_n + Tile::R;
+    v8h* s_rows = reinterpret_cast<v8h*>(s_red + 2 * Tile::kWaves);
+    Tile y(a);
+    y.take((int)(blockIdx.x / (unsigned)a.row_tiles), (int)(blockIdx.x % (unsigned)a.row_tiles));
+    if (y.rows <= 0) return;
+    const int lane = y.lane;
+    {
+        float sq[Tile::kGroups] = {}, err[Tile::kGroups] = {};
+        for (int o0 = 0; o0 < 2 * a.steps; o0 += 8 * Tile::kOctets) {
+            typename Tile::Octets x;
+            y.read(x, 0, o0, 2 * a.steps);
+            y.place(x, s_rows, a.steps, 0, o0, 2 * a.steps, sq, err);
+        }
+        y.put_sums(sq, err, s_n, s_red);
+    }
+    __syncthreads();
+    const float2 most = y.most(s_red);
     constexpr int kPass = CT * WC;                            // query tiles of one pass
-    if constexpr (WHOLE) {
-        stage(0, a.steps, true);
-        finish_sums();
-        __syncthreads();
-        v16f start[RT];
+    const int first = y.wc * CT;
+    if (first >= a.tiles) return;
+    typename Tile::Queries queries;
+    y.start_queries(queries, first);
+    for (int t = first; t < a.tiles; t += kPass) {
+        const int q = (t + (lane >> 5)) * kTile + (lane & 31);
+        const bool mine = q < a.nq && (CT == 2 || lane < 32);
+        const float2 info[1] = {a.qinfo[min(q, a.nq - 1)]};
+        const uint32_t have[1] = {y.out[min(q, a.nq - 1)]};
+        v16f acc[RT][CT];
 #pragma unroll
-        for (int r = 0; r < RT; r++) start[r] = lengths(r);
-        const v8h* rows_at = s_rows + (wr * RT) * a.chunk_steps * 64 + lane;
-        for (int t = wc * CT; t < a.tiles; t += kPass) {
-            const v8h* at[CT];
+        for (int r = 0; r < RT; r++) {
+            const v16f start = y.lengths(s_n, r);
 #pragma unroll
-            for (int c = 0; c < CT; c++) at[c] = frags + (int64_t)min(t + c, a.tiles - 1) * a.steps * 64 + lane;
-            const int q = (t + (lane >> 5)) * kTile + (lane & 31);
-            const bool mine = q < a.nq && (CT == 2 || lane < 32);
-            const float2 info = a.qinfo[min(q, a.nq - 1)];
-            const uint32_t have = out[min(q, a.nq - 1)];
-            v16f acc[RT][CT];
-            v8h next[CT];
-#pragma unroll
-            for (int c = 0; c < CT; c++) next[c] = at[c][0];
-#pragma unroll
-            for (int r = 0; r < RT; r++)
-#pragma unroll
-                for (int c = 0; c < CT; c++) acc[r][c] = start[r];
-            for (int s = 0; s < a.steps; s++) {
-                v8h q8[CT];
-#pragma unroll
-                for (int c = 0; c < CT; c++) { q8[c] = next[c]; next[c] = at[c][min(s + 1, a.steps - 1) * 64]; }
-#pragma unroll
-                for (int r = 0; r < RT; r++) {
-                    const v8h x8 = rows_at[(r * a.chunk_steps + s) * 64];
-#pragma unroll
-                    for (int c = 0; c < CT; c++) acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x8, q8[c], acc[r][c], 0, 0, 0);
-                }
-            }
-            finish(acc, q, mine, info, have);
+            for (int c = 0; c < CT; c++) acc[r][c] = start;
         }
-    } else {
+        y.multiply_steps(acc, s_rows + lane, a.steps, queries, a.steps);
+        y.finish(acc, q, mine, info, have, most);
+    }
+}
+
+// A barrier that waits for the wavefront's LDS accesses only: __syncthreads() would wait for the reads from memory under way as well,
+// which are to arrive in registers during what follows.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// Fewer queries, or longer rows: the rows are streamed through two halves of LDS, COLUMNS columns of a tile at a time, by four wavefronts
+// that read and round, while four others multiply what the first have placed before; a workgroup goes on from tile to tile.
+// (One set of wavefronts for both cannot: their reads of the queries would wait for the reads of rows issued before them,
+// 592 us for 512 queries on 2M rows of 96.)  ONE: a row is no longer than COLUMNS, and all queries are taken past it while it lies there;
+// else its columns come once for every pass over 32 CT WC queries.
+template <int RT, int CT, int WR, int WC, int COLUMNS, int WAVES, bool ONE, bool OCTETS>
+__global__ __launch_bounds__(128 * WR * WC, WAVES) void bounds_stream_kernel(BoundArgs a) {
+    typedef BoundTile<RT, CT, WR, WC, COLUMNS, OCTETS> Tile;
+    constexpr int kPass = CT * WC;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int pitch = a.column_steps, half = Tile::R * pitch * 2;      // 16-byte words
+    float* s_n = reinterpret_cast<float*>(smem);              // [2][R], by turns of tiles
+    float* s_red = s_n + 2 * Tile::R;                         // [2][2 * kWaves]
+    v8h* s_rows = reinterpret_cast<v8h*>(s_red + 4 * Tile::kWaves);
+    Tile y(a);
+    int b = (int)(blockIdx.x / (unsigned)a.row_tiles), rt = (int)(blockIdx.x % (unsigned)a.row_tiles);
+    auto go_on = [&]() {                                      // the workgroup's next tile that has rows
+        do {
+            b += a.next_part;
+            rt += a.next_tile;
+            if (rt >= a.row_tiles) { rt -= a.row_tiles; b++; }
+            if (b < a.num_parts) y.take(b, rt);
+        } while (b < a.num_parts && y.rows <= 0);
+    };
+    y.take(b, rt);
+    if (y.rows <= 0) go_on();
+    if (b >= a.num_parts) return;
+    int side = 0, turn = 0;
+    if (y.reads) {
+        // ---- reads and rounds: what comes next is under way while the others multiply what lies in LDS.  (One place that reads, and
+        // under no condition: registers that come together from two are copied, which waits for them.)
+        const int passes = ONE ? 1 : (a.tiles + kPass - 1) / kPass;
+        typename Tile::Octets next;
+        float sq[Tile::kGroups], err[Tile::kGroups];
+        int s0 = 0, pass = 0;
+        y.read(next, 0, 0, 2 * pitch);
+        for (;;) {
+            if (s0 == 0)
+#pragma unroll
+                for (int g = 0; g < Tile::kGroups; g++) sq[g] = err[g] = 0.0f;
+            y.place(next, s_rows + side * half, pitch, s0, 0, 2 * min(pitch, a.steps - s0), sq, err);
+            s0 += pitch;
+            if (s0 >= a.steps) {
+                s0 = 0;
+                if (pass == 0) y.put_sums(sq, err, s_n + turn * Tile::R, s_red + turn * 2 * Tile::kWaves);
+                if (++pass == passes) { pass = 0; turn ^= 1; go_on(); }
+            }
+            y.read(next, s0, 0, 2 * min(pitch, a.steps - s0));      // (past the last tile: its columns again)
+            side ^= 1;
+            lds_barrier();
+            if (b >= a.num_parts) return;
+        }
+    }
+    // ---- multiplies
+    const int lane = y.lane, first = y.wc * CT;
+    typename Tile::Queries queries;
+    y.start_queries(queries, min(first, a.tiles - CT));
+    for (; b < a.num_parts; go_on(), turn ^= 1) {
+        const float* n_here = s_n + turn * Tile::R;
+        const float* red_here = s_red + turn * 2 * Tile::kWaves;
+        float2 most;
+        if constexpr (ONE) {
+            lds_barrier();
+            most = y.most(red_here);
+        }
         for (int t0 = 0; t0 < a.tiles; t0 += kPass) {
-            const int t = t0 + wc * CT;
+            const int t = t0 + first;
             const bool busy = t < a.tiles;
+            if (ONE && !busy) break;
             const int q = (t + (lane >> 5)) * kTile + (lane & 31);
-            const bool mine = busy && q < a.nq && (CT == 2 || lane < 32);
-            const float2 info = a.qinfo[min(q, a.nq - 1)];
-            const uint32_t have = out[min(q, a.nq - 1)];
+            const bool mine = busy && q < a.nq && (CT >= 2 || lane < 32);
+            float2 info[(CT + 1) / 2];
+            uint32_t have[(CT + 1) / 2];
+#pragma unroll
+            for (int c = 0; c < (CT + 1) / 2; c++) { const int qc = min(q + 64 * c, a.nq - 1); info[c] = a.qinfo[qc]; have[c] = y.out[qc]; }
             v16f acc[RT][CT];
-#pragma unroll
-            for (int r = 0; r < RT; r++)
-#pragma unroll
-                for (int c = 0; c < CT; c++)
-#pragma unroll
-                    for (int i = 0; i < 16; i++) acc[r][c][i] = 0.0f;
-            for (int s0 = 0; s0 < a.steps; s0 += a.chunk_steps) {
-                const int ns = min(a.chunk_steps, a.steps - s0);
-                __syncthreads();                              // the columns before are done with
-                stage(s0, ns, t0 == 0);
-                __syncthreads();
-                if (!busy) continue;
-                const v8h* at[CT];
-#pragma unroll
-                for (int c = 0; c < CT; c++) at[c] = frags + ((int64_t)min(t + c, a.tiles - 1) * a.steps + s0) * 64 + lane;
-                const v8h* rows_at = s_rows + (wr * RT) * a.chunk_steps * 64 + lane;
-                v8h next[CT];
-#pragma unroll
-                for (int c = 0; c < CT; c++) next[c] = at[c][0];
-                for (int s = 0; s < ns; s++) {
-                    v8h q8[CT];
-#pragma unroll
-                    for (int c = 0; c < CT; c++) { q8[c] = next[c]; next[c] = at[c][min(s + 1, ns - 1) * 64]; }
-#pragma unroll
-                    for (int r = 0; r < RT; r++) {
-                        const v8h x8 = rows_at[(r * a.chunk_steps + s) * 64];
-#pragma unroll
-                        for (int c = 0; c < CT; c++) acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x8, q8[c], acc[r][c], 0, 0, 0);
-                    }
-                }
-            }
-            if (t0 == 0) {
-                __syncthreads();
-                finish_sums();
-                __syncthreads();
-            }
 #pragma unroll
             for (int r = 0; r < RT; r++) {
-                const v16f n2 = lengths(r);
+                v16f start = {};
+                if constexpr (ONE) start = y.lengths(n_here, r);
 #pragma unroll
-                for (int c = 0; c < CT; c++)
-#pragma unroll
-                    for (int i = 0; i < 16; i++) acc[r][c][i] += n2[i];
+                for (int c = 0; c < CT; c++) acc[r][c] = start;
             }
-            if (busy) finish(acc, q, mine, info, have);
+            if constexpr (ONE) {
+                y.multiply_steps(acc, s_rows + side * half + y.wr * RT * pitch * 64 + lane, pitch, queries, a.steps);
+            } else {
+                for (int s0 = 0; s0 < a.steps; s0 += pitch) {
+                    lds_barrier();
+                    if (busy)
+                        y.multiply_steps(acc, s_rows + side * half + y.wr * RT * pitch * 64 + lane, pitch, queries, min(pitch, a.steps - s0));
+                    side ^= 1;
+                }
+                most = y.most(red_here);
+#pragma unroll
+                for (int r = 0; r < RT; r++) {
+                    const v16f n2 = y.lengths(n_here, r);
+#pragma unroll
+                    for (int c = 0; c < CT; c++)
+#pragma unroll
+                        for (int i = 0; i < 16; i++) acc[r][c][i] += n2[i];
+                }
+            }
+            y.finish(acc, q, mine, info, have, most);
         }
+        if constexpr (ONE) side ^= 1;
     }
 }
 
@@ -471,13 +626,27 @@ __global__ __launch_bounds__(256) void list_items_kernel(ListArgs a) {
     }
 }
 
+// How the product is cut: row tiles and query tiles per wavefront, wavefronts along rows and queries; rows streamed or a tile of them
+// resident, and read once or once for every pass over the queries.
+struct Shape { int rt, ct, wr, wc; bool stream, one; };
+Shape shape_of(const QueryArgs& a) {
+    if (a.nq <= 32) return {1, 1, 4, 1, true, a.dim <= 128};
+    if (a.nq <= 64) return {1, 2, 4, 1, true, a.dim <= 128};
+    if (a.nq <= 128) return {2, 2, 2, 2, true, a.dim <= 128};
+    if (a.dim > kWholeDim) return {2, 4, 1, 4, true, false};
+    if (a.nq <= 1024) return {4, 2, 1, 4, true, true};
+    return {4, 2, 1, 4, false, true};
+}
+
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 struct Room { size_t header, counts, qinfo, frags, bounds, limits, last, items, part_counts, total; int steps, tiles, parts; };
 Room room_of(const QueryArgs& a) {
     Room r;
-    r.steps = (a.dim + kStep - 1) / kStep;
-    r.tiles = (a.nq + kTile - 1) / kTile;
+    r.steps = (a.dim + 2 * kStep - 1) / (2 * kStep) * 2;       // an even number of them
+    // (whole groups of the query tiles a wavefront takes at a time)
+    const int group = shape_of(a).ct;
+    r.tiles = (a.nq + kTile * group - 1) / (kTile * group) * group;
     // parts of a partition: 24 k in all, as far as that leaves them a row tile each and a query 2048 of them
     const int64_t row_tiles = max((int64_t)1, a.ppb / 128);
     r.parts = 1;
@@ -496,21 +665,11 @@ Room room_of(const QueryArgs& a) {
     return r;
 }
 
-// How the product is cut: wavefronts along rows and queries, row tiles each, and whether rows stay in LDS whole.
-struct Shape { int rt, ct, wr, wc; bool whole; };
-Shape shape_of(const QueryArgs& a) {
-    const int dim = (a.dim + kStep - 1) / kStep * kStep;
-    if (a.nq <= 32) return {1, 1, 4, 1, dim <= kChunk};
-    if (a.nq <= 64) return {1, 2, 4, 1, dim <= kChunk};
-    if (a.nq <= 128) return {2, 2, 2, 2, dim <= kChunk};
-    if (dim <= kChunk) return {4, 2, 1, 4, true};
-    return {2, 2, 1, 8, false};
-}
-
 }  // namespace
 
 bool bounds_supported(const QueryArgs& a) {
     return !a.blind && !a.counters && a.dim >= 8 && a.dim <= 4096 && a.nq >= 1 && a.B >= 2 && a.B <= kMostParts &&
+           ((int64_t)a.nq + 128) * (a.dim + 32) < (1LL << 30) &&      // (the rounded queries are addressed by 32 bits)
            (int64_t)a.nq * a.B < 0x7fffffffLL && (a.ppb + kTile - 1) / kTile * (int64_t)a.B < 0x7fffffffLL;
 }
 
@@ -519,9 +678,9 @@ size_t bounds_bytes(const QueryArgs& a) { return room_of(a).total; }
 double bounds_cost(const QueryArgs& a) {
     const Shape y = shape_of(a);
     const int R = kTile * y.rt * y.wr;
-    const double dim = (double)((a.dim + kStep - 1) / kStep * kStep);
+    const double dim = (double)((a.dim + 2 * kStep - 1) / (2 * kStep) * 2 * kStep);
     const double rows = (double)((a.ppb + R - 1) / R * R) * (double)a.B;
-    const double passes = y.whole ? 1.0 : ceil((double)a.nq / (double)(kTile * y.ct * y.wc));
+    const double passes = y.one ? 1.0 : ceil((double)a.nq / (double)(kTile * y.ct * y.wc));
     const double queries = ceil((double)a.nq / (kTile * y.ct)) * (kTile * y.ct);
     return 12.0 + fmax(2.0 * rows * queries * dim / 500e6, passes * rows * (double)a.dim * 4.0 / 3e6);
 }
@@ -538,44 +697,74 @@ static int pack(const QueryArgs& a, const Room& r, char* ws, hipStream_t s) {
     return 0;
 }
 
-template <int RT, int CT, int WR, int WC, int WAVES, bool WHOLE>
-static int launch_bounds(const BoundArgs& p, int B, hipStream_t s) {
-    constexpr int R = kTile * RT * WR, NT = 64 * WR * WC;
-    const size_t lds = (size_t)R * 4 + 2 * WR * WC * 4 + (size_t)R * p.chunk_steps * kStep * 2;
+template <int RT, int CT, int WR, int WC, int COLUMNS, int WAVES, bool ONE>
+static int launch_stream(const BoundArgs& p, int xcds, hipStream_t s) {
+    constexpr int R = kTile * RT * WR, NT = 128 * WR * WC, kColumnSteps = COLUMNS / kStep;
+    BoundArgs a = p;
+    // stretches of columns of about the same length
+    const int stretches = ONE ? 1 : (p.steps + kColumnSteps - 1) / kColumnSteps;
+    a.column_steps = (p.steps + 2 * stretches - 1) / (2 * stretches) * 2;
+    const size_t lds = (size_t)2 * R * 4 + 4 * WR * WC * 4 + (size_t)2 * R * a.column_steps * kStep * 2;
+    a.row_tiles = (int)((p.ppb + R - 1) / R);
+    // as many workgroups as the device holds at a time
+    const int per_cu = max(1, min((int)(160 * 1024 / lds), WAVES * 4 / (NT / 64)));
+    const int64_t grid = min((int64_t)a.row_tiles * a.num_parts, (int64_t)xcds * 32 * per_cu);
+    a.next_part = (int)(grid / a.row_tiles);
+    a.next_tile = (int)(grid % a.row_tiles);
     static DeviceOnce once;
     const int rc = once.run([]() -> int {
-        DCIH_HIP(hipFuncSetAttribute((const void*)partition_bounds_kernel<RT, CT, WR, WC, WAVES, WHOLE, true>,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-        DCIH_HIP(hipFuncSetAttribute((const void*)partition_bounds_kernel<RT, CT, WR, WC, WAVES, WHOLE, false>,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        DCIH_HIP(hipFuncSetAttribute((const void*)bounds_stream_kernel<RT, CT, WR, WC, COLUMNS, WAVES, ONE, true>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        DCIH_HIP(hipFuncSetAttribute((const void*)bounds_stream_kernel<RT, CT, WR, WC, COLUMNS, WAVES, ONE, false>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         return 0;
     });
     if (rc) return rc;
-    BoundArgs a = p;
-    a.row_tiles = (int)((p.ppb + R - 1) / R);
-    const dim3 grid((unsigned)((int64_t)a.row_tiles * B));
-    if (a.dim % 8 == 0)
-        hipLaunchKernelGGL((partition_bounds_kernel<RT, CT, WR, WC, WAVES, WHOLE, true>), grid, dim3(NT), lds, s, a);
-    else
-        hipLaunchKernelGGL((partition_bounds_kernel<RT, CT, WR, WC, WAVES, WHOLE, false>), grid, dim3(NT), lds, s, a);
+    if (p.dim % 8 == 0) hipLaunchKernelGGL((bounds_stream_kernel<RT, CT, WR, WC, COLUMNS, WAVES, ONE, true>), dim3((unsigned)grid), dim3(NT), lds, s, a);
+    else hipLaunchKernelGGL((bounds_stream_kernel<RT, CT, WR, WC, COLUMNS, WAVES, ONE, false>), dim3((unsigned)grid), dim3(NT), lds, s, a);
     DCIH_HIP(hipGetLastError());
     return 0;
 }
 
-int partition_bounds(const QueryArgs& a, void* ws_, hipStream_t s) {
-    char* ws = (char*)ws_;
-    const Room r = room_of(a);
-    const int rc = pack(a, r, ws, s);
-    if (rc) return rc;
-    const Shape y = shape_of(a);
-    BoundArgs p{a.data, a.N, a.ppb, a.dim, r.steps, a.nq, r.tiles, y.whole ? r.steps : kChunk / kStep, 0, r.parts,
+static int products(const QueryArgs& a, const Room& r, char* ws, hipStream_t s) {
+    BoundArgs p{a.data, a.N, a.ppb, a.dim, r.steps, a.nq, r.tiles, 0, 0, 0, a.B, 0, r.parts,
                 (const Header*)(ws + r.header), (const float2*)(ws + r.qinfo), (const _Float16*)(ws + r.frags),
                 (uint32_t*)(ws + r.bounds)};
-    if (y.wr == 4 && y.ct == 1) return y.whole ? launch_bounds<1, 1, 4, 1, 4, true>(p, a.B, s) : launch_bounds<1, 1, 4, 1, 4, false>(p, a.B, s);
-    if (y.wr == 4) return y.whole ? launch_bounds<1, 2, 4, 1, 4, true>(p, a.B, s) : launch_bounds<1, 2, 4, 1, 4, false>(p, a.B, s);
-    if (y.wr == 2) return y.whole ? launch_bounds<2, 2, 2, 2, 2, true>(p, a.B, s) : launch_bounds<2, 2, 2, 2, 2, false>(p, a.B, s);
-    if (y.whole) return launch_bounds<4, 2, 1, 4, 2, true>(p, a.B, s);
-    return launch_bounds<2, 2, 1, 8, 3, false>(p, a.B, s);
+    const Shape y = shape_of(a);
+    if (!y.stream) {
+        constexpr int R = 128;
+        p.row_tiles = (int)((p.ppb + R - 1) / R);
+        const dim3 grid((unsigned)((int64_t)p.row_tiles * a.B));
+        const size_t lds = (size_t)R * 4 + 2 * 4 * 4 + (size_t)R * p.steps * kStep * 2;
+        static DeviceOnce once;
+        const int rc_attr = once.run([]() -> int {
+            DCIH_HIP(hipFuncSetAttribute((const void*)bounds_resident_kernel<4, 2, 4, 2, true>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+            DCIH_HIP(hipFuncSetAttribute((const void*)bounds_resident_kernel<4, 2, 4, 2, false>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+            return 0;
+        });
+        if (rc_attr) return rc_attr;
+        if (a.dim % 8 == 0) hipLaunchKernelGGL((bounds_resident_kernel<4, 2, 4, 2, true>), grid, dim3(256), lds, s, p);
+        else hipLaunchKernelGGL((bounds_resident_kernel<4, 2, 4, 2, false>), grid, dim3(256), lds, s, p);
+        DCIH_HIP(hipGetLastError());
+        return 0;
+    }
+    // (COLUMNS is what the registers hold that are read ahead into; longer rows come in stretches)
+    const int columns = r.steps * kStep;
+    if (y.ct == 1) {
+        if (columns <= 64) return launch_stream<1, 1, 4, 1, 64, 4, true>(p, a.xcds, s);
+        return columns <= 128 ? launch_stream<1, 1, 4, 1, 128, 4, true>(p, a.xcds, s) : launch_stream<1, 1, 4, 1, 64, 4, false>(p, a.xcds, s);
+    }
+    if (y.wr == 4) {
+        if (columns <= 64) return launch_stream<1, 2, 4, 1, 64, 4, true>(p, a.xcds, s);
+        return columns <= 128 ? launch_stream<1, 2, 4, 1, 128, 4, true>(p, a.xcds, s) : launch_stream<1, 2, 4, 1, 64, 4, false>(p, a.xcds, s);
+    }
+    if (y.wr == 2) return columns <= 128 ? launch_stream<2, 2, 2, 2, 128, 3, true>(p, a.xcds, s) : launch_stream<2, 2, 2, 2, 64, 4, false>(p, a.xcds, s);
+    if (y.ct == 4) return launch_stream<2, 4, 1, 4, 256, 2, false>(p, a.xcds, s);
+    return columns <= 128 ? launch_stream<4, 2, 1, 4, 128, 2, true>(p, a.xcds, s) : launch_stream<4, 2, 1, 4, 256, 2, true>(p, a.xcds, s);
+}
+
+int partition_bounds(const QueryArgs& a, void* ws, hipStream_t s) {
+    const Room r = room_of(a);
+    const int rc = pack(a, r, (char*)ws, s);
+    return rc ? rc : products(a, r, (char*)ws, s);
 }
 
 int pick_items(const QueryArgs& a, void* ws_, int round, int rounds, hipStream_t s) {
