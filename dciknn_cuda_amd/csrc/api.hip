@@ -686,7 +686,8 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     a.expect_steps = a.expect_promotions = 0.0f;
     a.rows8 = nullptr; a.rows8_rec = 0; a.rows8_bounds = nullptr; a.query8 = nullptr;
     a.picked = nullptr; a.picked_count = nullptr; a.picked_expect = a.picked_cover = 0; a.only = nullptr; a.only_round = 0;
-    a.share = 1.0; a.pick_first = 0.0; a.pick_rounds = a.pick_rank = 0; a.pick_rule = fixed ? 1 : h->rounds;
+    a.share = 1.0; a.pick_first = 0.0; a.pick_rounds = a.pick_rank = a.pick_near = 0;
+    a.near_bounds = nullptr; a.near_limit = nullptr; a.near_stride = 0; a.near_shift = a.near_tiles = 0; a.pick_rule = fixed ? 1 : h->rounds;
     a.phase_ticks = h->d_phase_ticks;
     a.stop_hint = nullptr;
     a.N = h->n;
@@ -754,7 +755,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
 
     (void)plan_rounds(a);
     size_t q8_bytes = 0;
-    if (!blind && dense_traversal_supported(a, nullptr)) {
+    if (!blind && !a.pick_near && dense_traversal_supported(a, nullptr)) {      // (near rows only: few enough to be read whole)
         const bool all_dense = takes_dense_kernel(a);
         bool use = false;
         const double per_item = std::min((double)a.ppb, expected_promotions(a));

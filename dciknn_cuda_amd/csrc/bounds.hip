@@ -5,19 +5,26 @@
 // them adds nothing to it, whatever its traversal would promote.  So a call of many items first
 // bounds, for every (query, partition), the distance of the partition's nearest row from below --
 // a matrix product on the matrix cores whose epilogue keeps a minimum -- and then traverses
-//   round 1: the partitions whose bound is within what the query's k nearest rows are bounded by,
-//   round 2: of the others about as many again, as far as their bound does not exceed the k-th distance found,
-//   round 3: all others whose bound does not exceed the k-th distance found by then.
+//   first the partitions whose bound is within what the query's k nearest rows are bounded by,
+//   then, as far as their bound does not exceed the k-th distance found so far, those within the bounds of the 2 k and of the 4 k nearest,
+//   last all others whose bound does not exceed it.
 // What is left out lies further than that, so the results are those of traversing everything; where
 // traversals miss near rows (low recall), or a bound is poor, the later rounds are larger, up to everything.
-// (Calls of about a millisecond go without round 2: its launches would cost more than the items it saves.)
+// (123457 normal rows of 67 elements, 37 partitions, 7 results, half of the pairs needed: 27 pairs a query in three rounds, 22 in
+// four.  Calls of about a millisecond take the first and the last round only: a round's launches would cost more than the pairs it saves.)
 // The k nearest rows are told apart by bounds of parts of a partition: among S of them, k nearest rows that fall into
-// the same part are k^2 / 2 S, which is what round 1's limit is too large by.
+// the same part are k^2 / 2 S, which is what the first limit is too large by.
 //
-// The bound.  Rows and queries are rounded to 16-bit floats x', q' (scaled by powers of two, so that nothing
-// overflows; what does, or is not finite, has an unbounded error).  |x - q| >= |x' - q'| - |x - x'| - |q - q'|,
+// For the dense kernel the bounds of all tiles of 64 or 128 rows are kept, and it forms the distances of those candidates only whose
+// tile can hold one that matters: in the first round one within the bounds of the 32 k nearest rows (a query whose k-th result turns out
+// further away has those partitions taken again), later one within the k-th distance found.  512 queries on 10M unit vectors of 96: 21.4 -> 15.3 ms,
+// 500 on 1M rows of 960 3.2 -> 2.6.
+//
+// The bound.  Rows and queries, less a common centre, are rounded to 16-bit floats x', q' (scaled by powers of two, so that
+// nothing overflows; what does, or is not finite, has an unbounded error).  |x - q| >= |x' - q'| - |x - x'| - |q - q'|,
 // the two errors being summed where the rounding is done, and |x' - q'|^2 = |x'|^2 + |q'|^2 - 2 x'.q' comes
-// from 16-bit products added up in float32, lowered by what those additions can be off.  The distance
+// from 16-bit products added up in float32, lowered by what those additions can be off (the less, the nearer the data
+// lies to the centre: on 1M rows of 128 elements of 0 to 300 a bound of 0.25 % below the distance takes 12 % more pairs).  The distance
 // the traversal kernels compute is a float32 sum itself; the bound is lowered by its relative error too.
 #include "common.h"
 #include "kernels.h"
@@ -38,11 +45,13 @@ constexpr int kStep = 16;                 // elements of one
 constexpr int kWholeDim = 256;            // rows up to here can be kept in LDS whole
 constexpr int kSample = 16;               // rows and queries the scales are taken from
 constexpr int kMostParts = 2048;           // bounds kept per query
+constexpr int kLimits = kMostRounds;       // per query: of the rounds but the last, and round 1's limit of what is near
 constexpr int kListQueries = 1024;        // queries of a partition listed by one workgroup
 constexpr float kHalfMax = 65504.0f, kHalfMin = 6.103515625e-05f;       // largest, and smallest normal, 16-bit float
 constexpr uint32_t kInf = 0x7f800000u;
 
-struct Header { float row_scale, query_scale; };
+struct Header { float row_scale, query_scale; };      // the centre follows, kCentre floats in
+constexpr int kCentre = 16;
 
 // 2^e with the sample's largest value at 64 .. 128: outliers of five hundred times that still fit, and what is
 // flushed to zero is 2^-20 of it.  The exponent is limited so that no sum below can overflow.
@@ -53,24 +62,51 @@ __device__ inline float scale_for(float most) {
     return __builtin_bit_cast(float, (uint32_t)(up + 127) << 23);
 }
 
-__device__ inline float sample_most(const float* base, int64_t rows, int dim, float* tmp) {
+__device__ inline float block_max(float v, float* tmp) {
+    v = __builtin_bit_cast(float, wave_max_i32(__builtin_bit_cast(int, v)));      // (not negative)
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) tmp[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return fmaxf(fmaxf(tmp[0], tmp[1]), fmaxf(tmp[2], tmp[3]));
+}
+// Of some rows, a column per thread and all of them under way together: sum, smallest and largest value of each column that are finite.
+template <class F>
+__device__ inline void sample_columns(const float* base, int64_t rows, int dim, F use) {
     const int take = (int)min((int64_t)kSample, rows);
+    for (int j = threadIdx.x; j < dim; j += kPackThreads) {
+        float x[kSample], sum = 0.0f, lo = 3e38f, hi = -3e38f;
+#pragma unroll
+        for (int r = 0; r < kSample; r++) x[r] = base[(rows * min(r, take - 1) / take) * dim + j];
+#pragma unroll
+        for (int r = 0; r < kSample; r++) {
+            const bool in = r < take && fabsf(x[r]) < 3e38f;
+            sum += in ? x[r] : 0.0f;
+            lo = in ? fminf(lo, x[r]) : lo;
+            hi = in ? fmaxf(hi, x[r]) : hi;
+        }
+        use(j, sum / (float)take, lo, hi);
+    }
+}
+// The common centre: the mean of some rows, in steps of 2^-7 of the power of two at their largest magnitude, so that whole numbers stay
+// whole.  Returns those rows' largest magnitude less the centre.  s_centre: 3 * width floats, of which the first `width` are the centre.
+__device__ inline float sample_centre(const float* base, int64_t rows, int dim, int width, float* s_centre, float* tmp) {
+    float* s_lo = s_centre + width;
+    float* s_hi = s_lo + width;
     float most = 0.0f;
-#pragma unroll 4
-    for (int e = threadIdx.x; e < take * dim; e += kPackThreads) {
-        const int r = e / dim;
-        const float v = fabsf(base[(rows * r / take) * dim + (e - r * dim)]);
-        most = v < 3e38f ? fmaxf(most, v) : most;
+    sample_columns(base, rows, dim, [&](int j, float mean, float lo, float hi) {
+        s_centre[j] = mean; s_lo[j] = lo; s_hi[j] = hi;
+        most = fmaxf(most, lo <= hi ? fmaxf(fabsf(lo), fabsf(hi)) : 0.0f);
+    });
+    most = block_max(most, tmp);
+    const float step = __builtin_bit_cast(float, (uint32_t)max(1, (int)(__builtin_bit_cast(uint32_t, most) >> 23) - 7) << 23);
+    float away = 0.0f;
+    for (int j = threadIdx.x; j < width; j += kPackThreads) {      // (the thread's own columns)
+        const float mean = j < dim ? rintf(s_centre[j] / step) * step : 0.0f;
+        const float centre = fabsf(mean) <= most ? mean : 0.0f;
+        if (j < dim && s_lo[j] <= s_hi[j]) away = fmaxf(away, fmaxf(fabsf(s_lo[j] - centre), fabsf(s_hi[j] - centre)));
+        s_centre[j] = centre;
     }
-    tmp[threadIdx.x] = most;
-    __syncthreads();
-    for (int o = kPackThreads / 2; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) tmp[threadIdx.x] = fmaxf(tmp[threadIdx.x], tmp[threadIdx.x + o]);
-        __syncthreads();
-    }
-    most = tmp[0];
-    __syncthreads();
-    return most;
+    return block_max(away, tmp);
 }
 
 // Eight consecutive elements of a row, j a multiple of eight, zeros past its end; dim >= 8.  Rows of
@@ -98,16 +134,18 @@ __device__ inline void place_octet(int dim, int j, float (&x)[8]) {
 #pragma unroll
         for (int i = 0; i < 8; i++) x[i] = 0.0f;
 }
-// Rounds to 16 bits (towards zero: one instruction for two) and sums the squares of the rounded values and of what was
-// rounded off.  What does not fit, or is not finite, makes the first sum so: it is cut to `most` and to zero, the second sum infinite
-// for the latter.  (16-bit floats below 2^-14, which the matrix cores may take as zeros, are allowed for in rounding_floor.)
-__device__ inline v8h round_octet(const float (&x)[8], float scale, float most, float& sq, float& err) {
+// Rounds x - centre to 16 bits and sums the squares of the rounded values and of what was rounded off (the subtraction's
+// own rounding is allowed for where the sums are used).  What does not fit, or is not finite, makes the first sum so: it is cut to
+// `most` and to zero, the second sum infinite for the latter.  (16-bit floats below 2^-14, which the matrix cores may
+// take as zeros, are allowed for in rounding_floor.)
+__device__ inline v8h round_octet(const float (&x)[8], const float (&centre)[8], float scale, float most, float& sq, float& err) {
     v8h out;
     float s2 = 0.0f, e2 = 0.0f;
 #pragma unroll
     for (int i = 0; i < 8; i += 2) {
-        const float a = x[i] * scale, b = x[i + 1] * scale;
-        const v2h h = __builtin_bit_cast(v2h, __builtin_amdgcn_cvt_pkrtz(a, b));
+        const float a = (x[i] - centre[i]) * scale, b = (x[i + 1] - centre[i + 1]) * scale;
+        v2h h;
+        h[0] = (_Float16)a; h[1] = (_Float16)b;
         out[i] = h[0]; out[i + 1] = h[1];
         s2 = __builtin_amdgcn_fdot2(h, h, s2, false);
         const float oa = __builtin_fmaf((float)h[0], -1.0f, a), ob = __builtin_fmaf((float)h[1], -1.0f, b);
@@ -118,7 +156,7 @@ __device__ inline v8h round_octet(const float (&x)[8], float scale, float most, 
         s2 = e2 = 0.0f;
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            float v = x[i] * scale;
+            float v = (x[i] - centre[i]) * scale;
             if (!(fabsf(v) < 3e38f)) { v = 0.0f; e2 = __builtin_inff(); }
             out[i] = (_Float16)fminf(most, fmaxf(-most, v));
             const float back = (float)out[i], off = v - back;
@@ -132,6 +170,11 @@ __device__ inline v8h round_octet(const float (&x)[8], float scale, float most, 
 }
 // The largest length of what the values below 2^-14 make up, scaled.
 __device__ inline float rounding_floor(int elements) { return sqrtf((float)elements) * kHalfMin; }
+// An upper bound of |x - x'|, scaled, from the two sums: of what was rounded off (a float32 sum), of the values below 2^-14, and of the
+// subtraction of the centre, a float32 ulp or less of what it gave.
+__device__ inline float rounding_error(float sq, float err, int elements) {
+    return sqrtf(err) * 1.001f + rounding_floor(elements) + sqrtf(sq + err) * 0x1p-22f;
+}
 
 // The first workgroups round 32 queries each, into the order the matrix instructions take them
 // ([32 queries][16 elements]: 64 lanes of 8), times -2; all of them clear what the later launches
@@ -144,20 +187,29 @@ struct PackArgs {
     float2* qinfo;                        // [tiles * 32]: |q'|^2 and an upper bound of |q - q'|
     _Float16* frags;
     uint32_t* bounds; int64_t num_bounds;
+    uint32_t* near; int64_t num_near;     // (only where they are formed by atomics)
     unsigned long long* part; int64_t num_part;
 };
 template <bool OCTETS>
 __global__ __launch_bounds__(kPackThreads) void pack_queries_kernel(PackArgs a) {
-    __shared__ float tmp[kPackThreads];
+    __shared__ float tmp[4];
+    extern __shared__ float s_centre[];                       // [3][steps * 16]
     const int tid = threadIdx.x;
     const int64_t at = (int64_t)blockIdx.x * kPackThreads + tid, all = (int64_t)gridDim.x * kPackThreads;
     for (int64_t e = at; e < a.num_bounds; e += all) a.bounds[e] = kInf;
+    for (int64_t e = at; e < a.num_near; e += all) a.near[e] = kInf;
     for (int64_t e = at; e < a.num_part; e += all) a.part[e] = ~0ull;
     if ((int)blockIdx.x >= a.tiles) return;
-    const float scale = scale_for(sample_most(a.query, a.nq, a.dim, tmp));
+    const int width = a.steps * kStep;
+    const float row_scale = scale_for(sample_centre(a.data, a.n, a.dim, width, s_centre, tmp));
+    float most = 0.0f;
+    sample_columns(a.query, a.nq, a.dim, [&](int j, float, float lo, float hi) {
+        if (lo <= hi) most = fmaxf(most, fmaxf(fabsf(lo - s_centre[j]), fabsf(hi - s_centre[j])));
+    });
+    const float scale = scale_for(block_max(most, tmp));
     if (blockIdx.x == 0) {
-        const float rows = scale_for(sample_most(a.data, a.n, a.dim, tmp));
-        if (tid == 0) { a.header->row_scale = rows; a.header->query_scale = scale; }
+        if (tid == 0) { a.header->row_scale = row_scale; a.header->query_scale = scale; }
+        for (int j = tid; j < width; j += kPackThreads) reinterpret_cast<float*>(a.header)[kCentre + j] = s_centre[j];
     }
     const int qt = tid >> 3, q = (int)blockIdx.x * kTile + qt;
     const float* row = a.query + (int64_t)min(q, a.nq - 1) * a.dim;
@@ -166,7 +218,10 @@ __global__ __launch_bounds__(kPackThreads) void pack_queries_kernel(PackArgs a) 
         float x[8];
         load_octet<OCTETS>(row, a.dim, o * 8, x);
         place_octet<OCTETS>(a.dim, o * 8, x);
-        v8h h = round_octet(x, scale, 0.5f * kHalfMax, sq, err);
+        float centre[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) centre[i] = s_centre[o * 8 + i];
+        v8h h = round_octet(x, centre, scale, 0.5f * kHalfMax, sq, err);
 #pragma unroll
         for (int i = 0; i < 8; i++) h[i] = (_Float16)((float)h[i] * -2.0f);      // (exact)
         *reinterpret_cast<v8h*>(a.frags + (((int64_t)blockIdx.x * a.steps + (o >> 1)) * 64 + (o & 1) * 32 + qt) * 8) = h;
@@ -175,7 +230,7 @@ __global__ __launch_bounds__(kPackThreads) void pack_queries_kernel(PackArgs a) 
     err += lane_xor<4>(err); err += lane_xor<2>(err); err += lane_xor<1>(err);
     if ((tid & 7) == 0) {
         const float inv = 1.0f / scale;
-        a.qinfo[q] = make_float2(sq * inv * inv, (sqrtf(err) * 1.001f + rounding_floor(a.steps * kStep)) * inv);
+        a.qinfo[q] = make_float2(sq * inv * inv, rounding_error(sq, err, a.steps * kStep) * inv);
     }
 }
 
@@ -188,7 +243,11 @@ struct BoundArgs {
     int num_parts, row_tiles, parts;      // partitions, row tiles of each, and the parts of each that bounds are kept for
     const Header* header; const float2* qinfo; const _Float16* frags;
     uint32_t* bounds;                     // [B * parts][nq] float bits
+    uint32_t* tile_bounds;                // null, or the same of every near_rows(RT) rows
 };
+
+// The rows a near tile holds: one wavefront's, 64 at least.
+__host__ __device__ constexpr int near_rows(int rt) { return kTile * (rt < 2 ? 2 : rt); }
 
 // What the kernels below share.  A workgroup of WR wavefronts along the rows and WC along the queries takes tiles of R = 32 RT WR
 // rows of a partition, each wavefront RT x CT accumulators of 32 x 32.  A row's squared length is where its
@@ -207,11 +266,12 @@ struct BoundTile {
     const float* base;                    // of the tile: its first row, number of rows, and its bounds
     int rows;
     uint32_t* out;
+    int64_t tile_out;                     // (where the tile's own ones begin)
 
     __device__ __forceinline__ BoundTile(const BoundArgs& args)
         : a(args), lane((int)(threadIdx.x & 63)), reads(__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) < kWaves),
           wave(__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) % kWaves), wr(wave / WC), wc(wave % WC),
-          row_scale(args.header->row_scale), query_scale(args.header->query_scale), base(nullptr), rows(0), out(nullptr) {}
+          row_scale(args.header->row_scale), query_scale(args.header->query_scale), base(nullptr), rows(0), out(nullptr), tile_out(0) {}
 
     // Row tile rt of partition b.
     __device__ __forceinline__ void take(int b, int rt) {
@@ -219,6 +279,7 @@ struct BoundTile {
         rows = (int)min((int64_t)R, min(a.n, off + a.ppb) - first);
         base = a.data + first * a.dim;
         out = a.bounds + ((int64_t)b * a.parts + rt * a.parts / a.row_tiles) * a.nq;
+        tile_out = (((int64_t)b * a.row_tiles + rt) * (R / near_rows(RT)) + wr * RT * kTile / near_rows(RT)) * a.nq;
     }
     // Columns [16 s0 + 8 o0, ..) of the tile's rows, kOctets octets per lane of each of its kGroups rows: read, then rounded into LDS in
     // the order the matrix instructions take them.  A lane group of eight takes eight rows, so that its stores hit different banks; eight
@@ -232,19 +293,29 @@ struct BoundTile {
             for (int u = 0; u < kOctets; u++) load_octet<OCTETS>(row, a.dim, s0 * kStep + min(o0 + 8 * u + (lane >> 3), octets - 1) * 8, x[g][u]);
         }
     }
-    __device__ __forceinline__ void place(Octets& x, v8h* to, int pitch, int s0, int o0, int octets, float (&sq)[kGroups], float (&err)[kGroups]) const {
+    __device__ __forceinline__ void place(Octets& x, v8h* to, const float* s_centre, int pitch, int s0, int o0, int octets,
+                                          float (&sq)[kGroups], float (&err)[kGroups]) const {
 #pragma unroll
-        for (int g = 0; g < kGroups; g++) {
-            const int r = (g * kWaves + wave) * 8 + (lane & 7);
+        for (int u = 0; u < kOctets; u++) {
+            const int o = o0 + 8 * u + (lane >> 3);
+            if (o < octets) {
+                float centre[8];
+                const v4f lo = *reinterpret_cast<const v4f*>(s_centre + s0 * kStep + o * 8), hi = *reinterpret_cast<const v4f*>(s_centre + s0 * kStep + o * 8 + 4);
+                centre[0] = lo.x; centre[1] = lo.y; centre[2] = lo.z; centre[3] = lo.w;
+                centre[4] = hi.x; centre[5] = hi.y; centre[6] = hi.z; centre[7] = hi.w;
 #pragma unroll
-            for (int u = 0; u < kOctets; u++) {
-                const int o = o0 + 8 * u + (lane >> 3);
-                if (o < octets) {
+                for (int g = 0; g < kGroups; g++) {
+                    const int r = (g * kWaves + wave) * 8 + (lane & 7);
                     place_octet<OCTETS>(a.dim, s0 * kStep + o * 8, x[g][u]);
-                    to[((r >> 5) * pitch + (o >> 1)) * 64 + (o & 1) * 32 + (r & 31)] = round_octet(x[g][u], row_scale, kHalfMax, sq[g], err[g]);
+                    to[((r >> 5) * pitch + (o >> 1)) * 64 + (o & 1) * 32 + (r & 31)] = round_octet(x[g][u], centre, row_scale, kHalfMax, sq[g], err[g]);
                 }
             }
         }
+    }
+    // The centre into LDS, by the whole workgroup.
+    __device__ __forceinline__ void copy_centre(float* s_centre) const {
+        for (int j = threadIdx.x; j < a.steps * kStep; j += blockDim.x) s_centre[j] = reinterpret_cast<const float*>(a.header)[kCentre + j];
+        __syncthreads();
     }
     // Squared lengths, scaled as the products are (infinite past the last row), and the wavefront's largest length and error.
     __device__ __forceinline__ void put_sums(const float (&sq)[kGroups], const float (&err)[kGroups], float* s_n, float* s_red) const {
@@ -269,7 +340,7 @@ struct BoundTile {
 #pragma unroll
         for (int w = 0; w < kWaves; w++) { n = fmaxf(n, s_red[w]); e = fmaxf(e, s_red[kWaves + w]); }
         const float inv = 1.0f / row_scale;
-        return make_float2(n * inv * inv, (sqrtf(e) * 1.001f + rounding_floor(a.steps * kStep)) * inv);
+        return make_float2(n * inv * inv, rounding_error(n, e, a.steps * kStep) * inv);
     }
     __device__ __forceinline__ v16f lengths(const float* s_n, int r) const {      // of row tile r of this wavefront
         v16f v;
@@ -344,7 +415,9 @@ struct BoundTile {
     __device__ __forceinline__ void finish(const v16f (&acc)[RT][CT], int q, bool mine, const float2 (&info)[(CT + 1) / 2],
                                            const uint32_t (&have)[(CT + 1) / 2], float2 most) const {
         const float unscale = 1.0f / (row_scale * query_scale);
-        const float sum_error = (float)(a.steps * kStep + 64) * 0x1.8p-22f, dist_error = 1.0f - (float)(a.dim + 32) * 0x1p-23f;
+        // (every addition off by 2^-23 of the largest magnitude a partial sum can have, twice what rounding to nearest allows;
+        //  the squared lengths by half of that)
+        const float sum_error = (float)(a.steps * kStep + 32) * 0x1p-23f, dist_error = 1.0f - (float)(a.dim + 32) * 0x1p-23f;
         float best[CT];
 #pragma unroll
         for (int c = 0; c < CT; c++) {      // (four chains each: a single one would wait for every result)
@@ -367,12 +440,18 @@ struct BoundTile {
 #pragma unroll
         for (int c = 0; c < (CT + 1) / 2; c++) {
             const float v = CT >= 2 && lane >= 32 ? best[min(2 * c + 1, CT - 1)] : best[2 * c];
-            const float d2 = v * unscale + info[c].x - sum_error * (most.x + info[c].x);
+            const float d2 = v * unscale + info[c].x - sum_error * (1.5f * most.x + 2.0f * sqrtf(most.x * info[c].x) + 0.5f * info[c].x);
             float d = sqrtf(fmaxf(d2, 0.0f)) - most.y - info[c].y;
             d = fmaxf(d, 0.0f) * dist_error;
             if (!(d > 1e-14f)) d = 0.0f;                      // (squares below the smallest float count as nothing in the distances)
             const uint32_t bits = __builtin_bit_cast(uint32_t, d);
-            if (mine && q + 64 * c < a.nq && bits < have[c]) atomicMin(&out[q + 64 * c], bits);
+            if (mine && q + 64 * c < a.nq) {
+                if (a.tile_bounds) {
+                    if constexpr (RT * kTile < near_rows(RT)) atomicMin(&a.tile_bounds[tile_out + q + 64 * c], bits);
+                    else a.tile_bounds[tile_out + q + 64 * c] = bits;
+                }
+                if (bits < have[c]) atomicMin(&out[q + 64 * c], bits);
+            }
         }
     }
 };
@@ -385,17 +464,19 @@ __global__ __launch_bounds__(64 * WC, WAVES) void bounds_resident_kernel(BoundAr
     extern __shared__ __align__(16) unsigned char smem[];
     float* s_n = reinterpret_cast<float*>(smem);
     float* s_red = s_n + Tile::R;
-    v8h* s_rows = reinterpret_cast<v8h*>(s_red + 2 * Tile::kWaves);
+    float* s_centre = s_red + 2 * Tile::kWaves;
+    v8h* s_rows = reinterpret_cast<v8h*>(s_centre + a.steps * kStep);
     Tile y(a);
     y.take((int)(blockIdx.x / (unsigned)a.row_tiles), (int)(blockIdx.x % (unsigned)a.row_tiles));
     if (y.rows <= 0) return;
     const int lane = y.lane;
+    y.copy_centre(s_centre);
     {
         float sq[Tile::kGroups] = {}, err[Tile::kGroups] = {};
         for (int o0 = 0; o0 < 2 * a.steps; o0 += 8 * Tile::kOctets) {
             typename Tile::Octets x;
             y.read(x, 0, o0, 2 * a.steps);
-            y.place(x, s_rows, a.steps, 0, o0, 2 * a.steps, sq, err);
+            y.place(x, s_rows, s_centre, a.steps, 0, o0, 2 * a.steps, sq, err);
         }
         y.put_sums(sq, err, s_n, s_red);
     }
@@ -440,8 +521,10 @@ __global__ __launch_bounds__(128 * WR * WC, WAVES) void bounds_stream_kernel(Bou
     const int pitch = a.column_steps, half = Tile::R * pitch * 2;      // 16-byte words
     float* s_n = reinterpret_cast<float*>(smem);              // [2][R], by turns of tiles
     float* s_red = s_n + 2 * Tile::R;                         // [2][2 * kWaves]
-    v8h* s_rows = reinterpret_cast<v8h*>(s_red + 4 * Tile::kWaves);
+    float* s_centre = s_red + 4 * Tile::kWaves;
+    v8h* s_rows = reinterpret_cast<v8h*>(s_centre + a.steps * kStep);
     Tile y(a);
+    y.copy_centre(s_centre);
     int b = (int)(blockIdx.x / (unsigned)a.row_tiles), rt = (int)(blockIdx.x % (unsigned)a.row_tiles);
     auto go_on = [&]() {                                      // the workgroup's next tile that has rows
         do {
@@ -467,7 +550,7 @@ __global__ __launch_bounds__(128 * WR * WC, WAVES) void bounds_stream_kernel(Bou
             if (s0 == 0)
 #pragma unroll
                 for (int g = 0; g < Tile::kGroups; g++) sq[g] = err[g] = 0.0f;
-            y.place(next, s_rows + side * half, pitch, s0, 0, 2 * min(pitch, a.steps - s0), sq, err);
+            y.place(next, s_rows + side * half, s_centre, pitch, s0, 0, 2 * min(pitch, a.steps - s0), sq, err);
             s0 += pitch;
             if (s0 >= a.steps) {
                 s0 = 0;
@@ -535,12 +618,14 @@ __global__ __launch_bounds__(128 * WR * WC, WAVES) void bounds_stream_kernel(Bou
     }
 }
 
-// Of each query's S bounds the j1-th and the j2-th smallest, rounded up to 16 bits of their mantissa: one wavefront per
-// query, bit by bit the largest prefix that fewer than j bounds lie below.  A workgroup reads the bounds of `per`
-// neighbouring queries into LDS first.
+// Of each query's S bounds about the j-th, the 2 j-th, the 4 j-th and the near_rank-th smallest, one wavefront per query: the
+// largest in the histogram's bins up to the one that holds it, 1024 bins over the range of those that are finite.  A workgroup reads the
+// bounds of `per` neighbouring queries into LDS first.  (Bit by bit, with a ballot per bit, limit and 64 bounds: 3 times as long.)
 template <int V>
-__global__ __launch_bounds__(256) void pick_limits_kernel(const uint32_t* __restrict__ bounds, int S, int nq, int per, int j1, int j2,
+__global__ __launch_bounds__(256) void pick_limits_kernel(const uint32_t* __restrict__ bounds, int S, int nq, int per, int j, int near_rank,
                                                           uint32_t* __restrict__ limits, uint32_t* __restrict__ last_round) {
+    constexpr int kBins = 1024, kMine = kBins / 64;
+    __shared__ uint32_t s_hist[4][kBins];
     extern __shared__ uint32_t s_b[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q0 = (int)blockIdx.x * per, pitch = per + 1;
 #pragma unroll 4
@@ -549,22 +634,50 @@ __global__ __launch_bounds__(256) void pick_limits_kernel(const uint32_t* __rest
         s_b[i * pitch + q] = bounds[(int64_t)i * nq + min(q0 + q, nq - 1)];
     }
     __syncthreads();
-    for (int q = wave; q < per && q0 + q < nq; q += 4) {
-        uint32_t v[V];
+    uint32_t* hist = s_hist[wave];
+    for (int q = wave; q < per; q += 4) {      // (each wavefront its own histogram; no barrier below)
+        uint32_t v[V], lo = kInf;
+        int hi = 0;
 #pragma unroll
-        for (int i = 0; i < V; i++) v[i] = i * 64 + lane < S ? s_b[(i * 64 + lane) * pitch + q] >> 8 : 0xffffffu;
-        uint32_t at1 = 0, at2 = 0;
-#pragma unroll 1
-        for (int bit = 22; bit >= 0; bit--) {
-            const uint32_t t1 = at1 | (1u << bit), t2 = at2 | (1u << bit);
-            int below1 = 0, below2 = 0;
-#pragma unroll
-            for (int i = 0; i < V; i++) { below1 += __popcll(__ballot(v[i] < t1)); below2 += __popcll(__ballot(v[i] < t2)); }
-            if (below1 < j1) at1 = t1;
-            if (below2 < j2) at2 = t2;
+        for (int i = 0; i < V; i++) {
+            v[i] = i * 64 + lane < S ? s_b[(i * 64 + lane) * pitch + q] : kInf;
+            lo = min(lo, v[i]);
+            hi = max(hi, v[i] < kInf ? (int)v[i] : 0);
         }
-        // (all ones where there are fewer than j)
-        if (lane == 0) { limits[q0 + q] = (at1 << 8) | 0xffu; limits[nq + q0 + q] = (at2 << 8) | 0xffu; last_round[q0 + q] = 0; }
+        const float f_lo = __builtin_bit_cast(float, wave_min_u32(lo));
+        const float range = __builtin_bit_cast(float, wave_max_i32(hi)) - f_lo;
+        const float scale = range > 1e-30f ? (float)kBins / range : 0.0f;
+        auto bin = [&](uint32_t x) { return x < kInf ? min(kBins - 1, (int)((__builtin_bit_cast(float, x) - f_lo) * scale)) : kBins; };
+#pragma unroll
+        for (int i = 0; i < kMine; i++) hist[i * 64 + lane] = 0;
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < V; i++) if (v[i] < kInf) atomicAdd(&hist[bin(v[i])], 1u);
+        __builtin_amdgcn_wave_barrier();
+        uint32_t mine[kMine], sum = 0;
+#pragma unroll
+        for (int i = 0; i < kMine; i++) { mine[i] = hist[lane * kMine + i]; sum += mine[i]; }
+        const uint32_t upto = wave_scan_u32(sum);
+        uint32_t limit[kLimits];
+#pragma unroll
+        for (int w = 0; w < kLimits; w++) {
+            const uint32_t rank = (uint32_t)(w == kMostRounds - 1 ? near_rank : j << w);
+            uint32_t run = upto - sum;
+            int at = kBins - 1;
+#pragma unroll
+            for (int i = 0; i < kMine; i++) { run += mine[i]; at = run >= rank ? min(at, lane * kMine + i) : at; }
+            at = (int)wave_min_u32((uint32_t)at);
+            int most = 0;
+#pragma unroll
+            for (int i = 0; i < V; i++) most = max(most, bin(v[i]) <= at ? (int)v[i] : 0);
+            most = wave_max_i32(most);
+            limit[w] = __ballot(upto >= rank) ? (uint32_t)most : kInf;          // (infinite where there are fewer)
+        }
+        if (q0 + q < nq) {
+            if (lane < kLimits) limits[(int64_t)lane * nq + q0 + q] = lane == 0 ? limit[0] : (lane == 1 ? limit[1] : (lane == 2 ? limit[2] : limit[3]));
+            if (lane == 0) last_round[q0 + q] = 0;
+        }
+        __builtin_amdgcn_wave_barrier();
     }
 }
 
@@ -576,17 +689,21 @@ struct ListArgs {
     const uint32_t* bounds; const uint32_t* limits;
     const float* worst; int64_t worst_stride;      // the k-th distance each query has so far
     uint32_t* last_round;                          // the round that last took a partition of the query
-    int B, parts, nq, groups, round, rounds;
+    int B, parts, nq, groups, round, rounds, near;
     int32_t* items; uint32_t* count; uint32_t* part_counts;
 };
 __device__ inline bool takes_item(const ListArgs& a, int b, int q) {
     uint32_t v = a.bounds[(int64_t)b * a.parts * a.nq + q];
     for (int p = 1; p < a.parts; p++) v = min(v, a.bounds[((int64_t)b * a.parts + p) * a.nq + q]);
-    const uint32_t l1 = a.limits[q], l2 = a.rounds > 2 ? a.limits[a.nq + q] : l1;
-    if (a.round == 0) return v <= l1;
+    // a round takes what lies between two limits, the last one everything above the last limit
+    if (a.round + 1 < a.rounds && v > a.limits[(int64_t)a.round * a.nq + q]) return false;
+    if (a.round == 0) return true;
     // (what is infinite or NaN so far is bounded by nothing)
-    return v > l1 && (a.round + 1 < a.rounds ? v <= l2 : (a.rounds == 2 || v > l2)) &&
-           !(__builtin_bit_cast(float, v) > a.worst[(int64_t)q * a.worst_stride]);
+    const float worst = a.worst[(int64_t)q * a.worst_stride];
+    if (__builtin_bit_cast(float, v) > worst) return false;
+    if (v > a.limits[(int64_t)(a.round - 1) * a.nq + q]) return true;
+    // round 1 took no candidates further away than its limit: where its k-th is, its partitions are taken again
+    return a.near && a.round == 1 && !(worst <= __builtin_bit_cast(float, a.limits[(int64_t)(kLimits - 1) * a.nq + q]));
 }
 template <bool COUNT>
 __global__ __launch_bounds__(256) void list_items_kernel(ListArgs a) {
@@ -640,27 +757,28 @@ Shape shape_of(const QueryArgs& a) {
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
-struct Room { size_t header, counts, qinfo, frags, bounds, limits, last, items, part_counts, total; int steps, tiles, parts; };
+struct Room { size_t header, counts, qinfo, frags, bounds, limits, last, items, part_counts, near, total; int steps, tiles, parts; };
 Room room_of(const QueryArgs& a) {
     Room r;
     r.steps = (a.dim + 2 * kStep - 1) / (2 * kStep) * 2;       // an even number of them
     // (whole groups of the query tiles a wavefront takes at a time)
     const int group = shape_of(a).ct;
     r.tiles = (a.nq + kTile * group - 1) / (kTile * group) * group;
-    // parts of a partition: 24 k in all, as far as that leaves them a row tile each and a query 2048 of them
+    // parts of a partition: 64 k in all, as far as that leaves them a row tile each and a query 2048 of them
     const int64_t row_tiles = max((int64_t)1, a.ppb / 128);
     r.parts = 1;
-    while (2 * r.parts <= row_tiles && (int64_t)a.B * r.parts < 24 * (int64_t)a.k && (int64_t)a.B * r.parts * 2 <= kMostParts) r.parts *= 2;
+    while (2 * r.parts <= row_tiles && (int64_t)a.B * r.parts < 64 * (int64_t)a.k && (int64_t)a.B * r.parts * 2 <= kMostParts) r.parts *= 2;
     size_t o = 0;
-    r.header = o; o += 256;
+    r.header = o; o += align256((size_t)(kCentre + r.steps * kStep) * 4);
     r.counts = o; o += align256(kPickCountWords * 4);
     r.qinfo = o;  o += align256((size_t)r.tiles * kTile * sizeof(float2));
     r.frags = o;  o += align256((size_t)r.tiles * r.steps * 64 * 16);
     r.bounds = o; o += align256((size_t)a.B * r.parts * a.nq * 4);
-    r.limits = o; o += align256((size_t)2 * a.nq * 4);
+    r.limits = o; o += align256((size_t)kLimits * a.nq * 4);
     r.last = o;   o += align256((size_t)a.nq * 4);
     r.items = o;  o += align256((size_t)a.nq * a.B * 4);
     r.part_counts = o; o += align256((size_t)a.B * ((a.nq + kListQueries - 1) / kListQueries) * 4);
+    r.near = o;   o += a.pick_near ? align256(near_bytes(a)) : 0;
     r.total = o;
     return r;
 }
@@ -673,7 +791,18 @@ bool bounds_supported(const QueryArgs& a) {
            (int64_t)a.nq * a.B < 0x7fffffffLL && (a.ppb + kTile - 1) / kTile * (int64_t)a.B < 0x7fffffffLL;
 }
 
+// Of a partition, those of its last row tile that hold no rows among them.
+static int64_t near_tiles_of(const QueryArgs& a) {
+    const Shape y = shape_of(a);
+    const int R = kTile * y.rt * y.wr;
+    return (a.ppb + R - 1) / R * (R / near_rows(y.rt));
+}
+
 size_t bounds_bytes(const QueryArgs& a) { return room_of(a).total; }
+
+size_t near_bytes(const QueryArgs& a) {
+    return (size_t)near_tiles_of(a) * a.B * a.nq * 4;
+}
 
 double bounds_cost(const QueryArgs& a) {
     const Shape y = shape_of(a);
@@ -687,12 +816,14 @@ double bounds_cost(const QueryArgs& a) {
 
 static int pack(const QueryArgs& a, const Room& r, char* ws, hipStream_t s) {
     PackArgs p{a.query, a.data, a.N, a.nq, a.dim, r.steps, r.tiles, (Header*)(ws + r.header), (uint32_t*)(ws + r.counts),
-               (float2*)(ws + r.qinfo), (_Float16*)(ws + r.frags), (uint32_t*)(ws + r.bounds), (int64_t)a.B * r.parts * a.nq,
+               (float2*)(ws + r.qinfo), (_Float16*)(ws + r.frags), (uint32_t*)(ws + r.bounds), (int64_t)a.B * r.parts * a.nq, (uint32_t*)(ws + r.near),
+               a.pick_near && shape_of(a).rt * kTile < near_rows(shape_of(a).rt) ? (int64_t)near_bytes(a) / 4 : 0,
                a.part, (int64_t)a.nq * a.B * a.kcap};
-    const int64_t clear = (p.num_part + p.num_bounds + kPackThreads * 16 - 1) / (kPackThreads * 16);
+    const int64_t clear = (p.num_part + p.num_bounds + p.num_near + kPackThreads * 16 - 1) / (kPackThreads * 16);
     const unsigned blocks = (unsigned)max((int64_t)r.tiles, min((int64_t)2048, clear));
-    if (a.dim % 8 == 0) hipLaunchKernelGGL(pack_queries_kernel<true>, dim3(blocks), dim3(kPackThreads), 0, s, p);
-    else hipLaunchKernelGGL(pack_queries_kernel<false>, dim3(blocks), dim3(kPackThreads), 0, s, p);
+    const size_t lds = (size_t)3 * r.steps * kStep * 4;
+    if (a.dim % 8 == 0) hipLaunchKernelGGL(pack_queries_kernel<true>, dim3(blocks), dim3(kPackThreads), lds, s, p);
+    else hipLaunchKernelGGL(pack_queries_kernel<false>, dim3(blocks), dim3(kPackThreads), lds, s, p);
     DCIH_HIP(hipGetLastError());
     return 0;
 }
@@ -704,7 +835,7 @@ static int launch_stream(const BoundArgs& p, int xcds, hipStream_t s) {
     // stretches of columns of about the same length
     const int stretches = ONE ? 1 : (p.steps + kColumnSteps - 1) / kColumnSteps;
     a.column_steps = (p.steps + 2 * stretches - 1) / (2 * stretches) * 2;
-    const size_t lds = (size_t)2 * R * 4 + 4 * WR * WC * 4 + (size_t)2 * R * a.column_steps * kStep * 2;
+    const size_t lds = (size_t)2 * R * 4 + 4 * WR * WC * 4 + (size_t)p.steps * kStep * 4 + (size_t)2 * R * a.column_steps * kStep * 2;
     a.row_tiles = (int)((p.ppb + R - 1) / R);
     // as many workgroups as the device holds at a time
     const int per_cu = max(1, min((int)(160 * 1024 / lds), WAVES * 4 / (NT / 64)));
@@ -727,13 +858,13 @@ static int launch_stream(const BoundArgs& p, int xcds, hipStream_t s) {
 static int products(const QueryArgs& a, const Room& r, char* ws, hipStream_t s) {
     BoundArgs p{a.data, a.N, a.ppb, a.dim, r.steps, a.nq, r.tiles, 0, 0, 0, a.B, 0, r.parts,
                 (const Header*)(ws + r.header), (const float2*)(ws + r.qinfo), (const _Float16*)(ws + r.frags),
-                (uint32_t*)(ws + r.bounds)};
+                (uint32_t*)(ws + r.bounds), a.pick_near ? (uint32_t*)(ws + r.near) : nullptr};
     const Shape y = shape_of(a);
     if (!y.stream) {
         constexpr int R = 128;
         p.row_tiles = (int)((p.ppb + R - 1) / R);
         const dim3 grid((unsigned)((int64_t)p.row_tiles * a.B));
-        const size_t lds = (size_t)R * 4 + 2 * 4 * 4 + (size_t)R * p.steps * kStep * 2;
+        const size_t lds = (size_t)R * 4 + 2 * 4 * 4 + (size_t)p.steps * kStep * 4 + (size_t)R * p.steps * kStep * 2;
         static DeviceOnce once;
         const int rc_attr = once.run([]() -> int {
             DCIH_HIP(hipFuncSetAttribute((const void*)bounds_resident_kernel<4, 2, 4, 2, true>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
@@ -778,14 +909,14 @@ int pick_items(const QueryArgs& a, void* ws_, int round, int rounds, hipStream_t
         const dim3 grid((unsigned)((a.nq + per - 1) / per));
 #define DCIH_LIMITS(V)                                                                                              \
     hipLaunchKernelGGL(pick_limits_kernel<V>, grid, dim3(256), (size_t)S * (per + 1) * 4, s, bounds, S, a.nq, per, \
-                       a.pick_rank, 2 * a.pick_rank, limits, last)
+                       a.pick_rank, min(32 * a.pick_rank, max(4 * a.pick_rank, S / 2)), limits, last)
         if (S <= 64) DCIH_LIMITS(1); else if (S <= 128) DCIH_LIMITS(2); else if (S <= 256) DCIH_LIMITS(4);
         else if (S <= 512) DCIH_LIMITS(8); else if (S <= 1024) DCIH_LIMITS(16); else DCIH_LIMITS(32);
 #undef DCIH_LIMITS
         DCIH_HIP(hipGetLastError());
     }
     const int groups = (a.nq + kListQueries - 1) / kListQueries;
-    ListArgs p{bounds, limits, a.out_dists + (a.k - 1), a.k, last, a.B, r.parts, a.nq, groups, round, rounds,
+    ListArgs p{bounds, limits, a.out_dists + (a.k - 1), a.k, last, a.B, r.parts, a.nq, groups, round, rounds, a.pick_near,
                (int32_t*)(ws + r.items), (uint32_t*)(ws + r.counts) + round, (uint32_t*)(ws + r.part_counts)};
     const dim3 grid((unsigned)((int64_t)a.B * groups));
     hipLaunchKernelGGL(list_items_kernel<true>, grid, dim3(256), 0, s, p);
@@ -797,7 +928,16 @@ int pick_items(const QueryArgs& a, void* ws_, int round, int rounds, hipStream_t
 Picked picked_items(const QueryArgs& a, void* ws_, int round) {
     char* ws = (char*)ws_;
     const Room r = room_of(a);
-    return Picked{(const int32_t*)(ws + r.items), (const uint32_t*)(ws + r.counts) + round, (const uint32_t*)(ws + r.last)};
+    Picked p{(const int32_t*)(ws + r.items), (const uint32_t*)(ws + r.counts) + round, (const uint32_t*)(ws + r.last), nullptr, nullptr, 0, 0, 0};
+    if (a.pick_near) {
+        p.near_bounds = (const uint32_t*)(ws + r.near);
+        // (later rounds: the k-th distance found so far)
+        p.near_limit = round ? a.out_dists + (a.k - 1) : (const float*)(ws + r.limits) + (int64_t)(kLimits - 1) * a.nq;
+        p.near_stride = round ? a.k : 1;
+        p.near_shift = near_rows(shape_of(a).rt) == 64 ? 6 : 7;
+        p.near_tiles = (int)near_tiles_of(a);
+    }
+    return p;
 }
 
 }  // namespace dcih

@@ -111,6 +111,13 @@ struct QueryArgs {
     int64_t picked_cover;    // ... and how many there seldom are more of: what a launch of one workgroup per item covers
     const uint32_t* only;    // merge: null, or only the queries whose word here is only_round
     uint32_t only_round;
+    // dense kernel, in rounds: lower bounds per tile of 2^near_shift rows ([B * near_tiles][nq]) and the distance of each query from
+    // which on a candidate does not matter to the round; null = all candidates' distances are wanted
+    const uint32_t* near_bounds;
+    const float* near_limit;
+    int64_t near_stride;
+    int near_shift, near_tiles;
+    int pick_near;           // 1: a call in rounds goes to the dense kernel and keeps those bounds
     int pick_rounds;         // 0: everything is traversed at once
     int pick_rank;           // the first round takes the partitions of so many nearest rows
     int pick_rule;           // DCIH_OPT_ROUNDS value
@@ -236,10 +243,14 @@ __device__ inline int64_t picked_run(const uint32_t* d_count, int x, int X, int6
 // Calls in rounds (bounds.hip): lower bounds of every (query, partition)'s nearest distance, and the items each
 // round takes.  Scratch of bounds_bytes(); bounds_cost: about how long the bounds take, us.  partition_bounds also
 // clears a.part.
-constexpr int kPickCountWords = 64;
-struct Picked { const int32_t* items; const uint32_t* count; const uint32_t* last_round; };
+constexpr int kPickCountWords = 64, kMostRounds = 4;
+struct Picked {
+    const int32_t* items; const uint32_t* count; const uint32_t* last_round;
+    const uint32_t* near_bounds; const float* near_limit; int64_t near_stride; int near_shift, near_tiles;
+};
 bool bounds_supported(const QueryArgs& a);
 size_t bounds_bytes(const QueryArgs& a);
+size_t near_bytes(const QueryArgs& a);      // the part of it that pick_near adds
 double bounds_cost(const QueryArgs& a);
 int partition_bounds(const QueryArgs& a, void* ws, hipStream_t s);
 int pick_items(const QueryArgs& a, void* ws, int round, int rounds, hipStream_t s);

@@ -450,7 +450,7 @@ bool takes_dense_kernel(const QueryArgs& a) {
 }
 
 bool plan_rounds(QueryArgs& a) {
-    a.pick_rounds = 0;
+    a.pick_rounds = a.pick_near = 0;
     a.share = 1.0;
     if (a.mode != 0 || a.pick_rule == 1 || !bounds_supported(a)) return false;
     // The r nearest rows of a query lie in about B (1 - e^(-r/B)) partitions (rows in no particular order).  Round 1
@@ -460,7 +460,8 @@ bool plan_rounds(QueryArgs& a) {
     const double B = (double)a.B;
     auto parts_of = [&](double r) { return fmin(B, B * (1.0 - exp(-r / B)) + 0.5); };
     const bool few = (double)a.nq * parts_of(2.0 * (double)a.k) <= 1024.0;
-    const double first = parts_of(few ? 2.0 * (double)a.k : (double)a.k);
+    const int rank = few ? 2 * a.k : a.k + a.k / 16;      // (a few are missed: 10M unit vectors, k = 100: 111 pairs a query at 100, 102 at 110)
+    const double first = parts_of((double)rank);
     const double share = fmin(1.0, (few ? first : 1.1 * first + 0.2) / B);
     const bool can_dense = dense_traversal_supported(a, nullptr), can_block = block_traversal_supported(a, nullptr);
     bool fits = true;
@@ -475,10 +476,11 @@ bool plan_rounds(QueryArgs& a) {
     const double whole = time(1.0), rounds = time(first / B) + (few ? 15.0 : time(share - first / B)) + bounds_cost(a) + 30.0;
     (void)time(share);
     if (!fits || (a.pick_rule == 0 && rounds > 0.85 * whole)) return false;
-    a.pick_rounds = few ? 2 : (whole > 1500.0 || a.pick_rule == 2 ? 3 : 2);
-    a.pick_rank = few ? 2 * a.k : a.k;
+    a.pick_rounds = few ? 2 : (whole > 1500.0 || a.pick_rule == 2 ? kMostRounds : 2);
+    a.pick_rank = rank;
     a.pick_first = first;
     a.share = share;
+    a.pick_near = can_dense && takes_dense_kernel(a) && near_bytes(a) <= ((size_t)1 << 30) ? 1 : 0;
     return true;
 }
 
@@ -563,7 +565,7 @@ int query(const QueryArgs& a_in, void* bounds_ws, hipStream_t s, hipEvent_t* ev,
             }
             if (a.mode == 3 || a.dense_items) {
                 QueryArgs d = a;
-                if (use_block) d.picked = nullptr;      // what the batch kernel handed over
+                if (use_block) { d.picked = nullptr; d.near_bounds = nullptr; }      // what the batch kernel handed over
                 const int rc = query_dense_items(d, s);
                 if (rc) return rc;
                 if (ev) (void)hipEventRecord(ev[2], s);
@@ -607,6 +609,8 @@ int query(const QueryArgs& a_in, void* bounds_ws, hipStream_t s, hipEvent_t* ev,
             const Picked p = picked_items(a, bounds_ws, round);
             a.picked = p.items;
             a.picked_count = p.count;
+            a.near_bounds = p.near_bounds; a.near_limit = p.near_limit; a.near_stride = p.near_stride;
+            a.near_shift = p.near_shift; a.near_tiles = p.near_tiles;
             a.picked_expect = (int64_t)fmax(round ? all - first : first, 1.0);
             a.picked_cover = (int64_t)(round ? 0.6 * first : 1.25 * first) + 64;
             if (!rc) rc = traverse(a);

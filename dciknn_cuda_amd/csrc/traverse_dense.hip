@@ -866,9 +866,31 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
         int list_len = 0, list_pos = 0;
         uint32_t ncand = 0;
         int topn = 0;
+        // In a call's rounds only the tiles of rows that can hold one of the round's wanted distances are gone through (one bit
+        // each, in words of the scan's scratch that this phase does not use): 13000 candidates of 96 elements, k = 100, of 25000
+        // rows in 196 tiles, a handful of them near: 76 -> 12 us per item.
+        uint32_t* near_bits = scan_tmp + 48;
+        const bool near = args->a.near_bounds != nullptr;
+        const int near_shift = args->a.near_shift;
+        if (near) {
+            if (tid < 16) near_bits[tid] = 0;
+            __syncthreads();
+            const float most = args->a.near_limit[(int64_t)qi * args->a.near_stride];
+            const uint32_t* bounds = args->a.near_bounds + (int64_t)b * args->a.near_tiles * args->a.nq + qi;
+            const int tiles = (n + (1 << near_shift) - 1) >> near_shift;
+            for (int t = tid; t < tiles; t += NT)
+                if (!(__builtin_bit_cast(float, bounds[(int64_t)t * args->a.nq]) > most)) atomicOr(&near_bits[t >> 5], 1u << (t & 31));
+            __syncthreads();
+        }
         // lists at least `want` candidates, while points are left
         auto list_more = [&](int want) {
             while (list_len - list_pos < want && at < at_end) {
+                int end = at_end;
+                if (near) {
+                    const int t = at >> near_shift;
+                    end = min(at_end, (t + 1) << near_shift);
+                    if (!((uint32_t)__builtin_amdgcn_readfirstlane((int)near_bits[t >> 5]) >> (t & 31) & 1u)) { at = end; continue; }
+                }
                 if (list_pos > 0) {      // what is left moves to the front (one wavefront: its LDS operations keep their order)
                     const int rest = list_len - list_pos;
                     const uint16_t v = lane < rest ? wl[list_pos + lane] : (uint16_t)0;
@@ -878,12 +900,12 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
                     list_pos = 0;
                 }
                 const int pt = at + lane;
-                const uint32_t v = pt < at_end ? (uint32_t)tb.time[pt] : 0xffffu;
+                const uint32_t v = pt < end ? (uint32_t)tb.time[pt] : 0xffffu;
                 const bool is_cand = (v >> 1) <= t_lim;
                 const unsigned long long m = __ballot(is_cand);
                 if (is_cand) wl[list_len + __popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)pt;
                 list_len += __popcll(m);
-                at += kWave;
+                at = near ? min(at + kWave, end) : at + kWave;
                 ncand += (uint32_t)__popcll(m);
             }
             __builtin_amdgcn_wave_barrier();
