@@ -456,7 +456,7 @@ size_t exhaustive_ws_bytes(int64_t N, int chunk, int k) {
     const size_t cells = (size_t)chunk * (size_t)N;
     if (exhaustive_selects(k)) {
         const ExSelect e = exhaustive_select(N, k);
-        return align256(cells * 4) + align256((size_t)chunk * e.pieces * e.kc * sizeof(unsigned long long));
+        return align256(cells * 4) + align256(max((size_t)chunk * e.pieces * e.kc * sizeof(unsigned long long), nearest_least_bytes(N, chunk)));
     }
     return 3 * align256(cells * 4) + align256(segsort_tmp_bytes(chunk, N, 1));
 }
@@ -506,6 +506,11 @@ int query_exhaustive(const QueryArgs& a, void* ws, int chunk, hipStream_t s) {
     const ExSelect sel = exhaustive_select(a.N, a.k);
     for (int q0 = 0; q0 < a.nq; q0 += chunk) {
         const int nqc = min(chunk, a.nq - q0);
+        if (a.pick_rule != 1 && nearest_supported(a.N, a.dim, a.k) && (a.pick_rule == 2 || nearest_pays(a.N, a.dim, nqc))) {
+            const int rc = query_nearest(a, q0, nqc, d_dist, (float*)((char*)ws + align256((size_t)chunk * (size_t)a.N * 4)), s);
+            if (rc) return rc;
+            continue;
+        }
         // as many queries per wavefront as leave a wavefront to every SIMD (a row is read once for all of them)
         const auto waves = [&](int qn) { return row_groups * ((nqc + qn - 1) / qn); };
         if (waves(8) >= 1024) launch_dists<8>(a, q0, nqc, d_dist, s);

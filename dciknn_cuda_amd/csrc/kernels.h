@@ -265,6 +265,12 @@ bool plan_rounds(QueryArgs& a);
 int exhaustive_chunk(int64_t N, int nq);
 size_t exhaustive_ws_bytes(int64_t N, int chunk, int k);
 int query_exhaustive(const QueryArgs& a, void* ws, int chunk, hipStream_t s);
+// The same for few results (nearest.hip): distances only of the rows whose lower bound says that they can be among them.
+// d_bounds: [nq][N] floats; d_least: nearest_least_bytes.
+bool nearest_supported(int64_t N, int dim, int k);
+bool nearest_pays(int64_t N, int dim, int nq);
+size_t nearest_least_bytes(int64_t N, int nq);
+int query_nearest(const QueryArgs& a, int q0, int nq, float* d_bounds, float* d_least, hipStream_t s);
 // The pieces of it that the dense-row traversal (query_dense) shares: rows of N values
 // at rank_rows_input(ws), `rows` <= chunk of them; rank_rows sorts every row by (value,
 // column) and writes the first k columns (id = column, or -1 for +inf when asked).

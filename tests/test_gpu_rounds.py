@@ -163,3 +163,31 @@ def test_what_asks_for_everything_gets_everything(gpu):
     for a, b in zip(*res):
         assert torch.equal(a, b)
     dci.free()
+
+
+# Where no partition stops early the k nearest of all rows are selected by bounds of their distances: columns in one part and in
+# several, whole octets and quads or not, the most columns there can be, the fewest rows, k either side of 32 and the largest.
+@pytest.mark.parametrize("kind", ["normal", "clusters", "dup", "grid", "offset", "scales", "tiny", "huge", "broken", "zero"])
+@pytest.mark.parametrize("n,dim,nq,k", [(1500, 150, 300, 10), (3000, 67, 301, 4), (6001, 41, 250, 33), (6500, 640, 65, 100),
+                                         (1024, 8, 1, 16), (1100, 4096, 3, 7), (8200, 9, 70, 128)])
+def test_nearest_of_all_rows(gpu, kind, n, dim, nq, k):
+    X, Q = _rows(kind, n, nq, dim, n + dim)
+    dci = gpu.DCI(dim, 2, 7, n // 20, 10, seed=3)
+    dci.add(X)
+    want = _ask(dci, dci._lib, NEVER, Q, k, 5000)
+    got = _ask(dci, dci._lib, ALWAYS, Q, k, 5000)
+    dci.free()
+    assert torch.equal(got[0], want[0])
+    assert torch.equal(got[1].view(torch.int32), want[1].view(torch.int32))
+
+
+def test_nearest_of_many_rows(gpu):      # more than 512 workgroups of the product
+    X, Q = _rows("clusters", 40000, 500, 72, 12)
+    Q[7] = float("nan")
+    dci = gpu.DCI(72, 2, 7, 1000, 64, seed=3)
+    dci.add(X)
+    want = _ask(dci, dci._lib, NEVER, Q, 64, 100)
+    got = _ask(dci, dci._lib, 0, Q, 64, 100)
+    dci.free()
+    assert torch.equal(got[0], want[0])
+    assert torch.equal(got[1].view(torch.int32), want[1].view(torch.int32))
