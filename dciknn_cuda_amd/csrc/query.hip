@@ -325,13 +325,13 @@ __global__ __launch_bounds__(kMergeThreads) void merge_topk_kernel(QueryArgs a, 
 // every list, at least 2 k in all; where those are more than NT, from the smallest of each thread's
 // share of them.)  Bound by its chain of reads, sorts and barriers: one wavefront per query where
 // the heads fit two per lane.  10000 queries of 58 lists of 10: 171 us with the sorts of 1024 words above.
-template <int NT>
+template <int NT, bool ROUNDS>      // ROUNDS: some queries' results stay as they are
 __global__ __launch_bounds__(NT) void merge_heads_kernel(QueryArgs a, int heads) {
     constexpr int kCap = NT == kWave ? 256 : 2048, kAhead = 4;
     __shared__ unsigned long long buf[kCap];
     __shared__ uint32_t s_count;
     const int tid = threadIdx.x, qi = blockIdx.x;
-    if (a.only && a.only[qi] != a.only_round) return;
+    if (ROUNDS && a.only[qi] != a.only_round) return;
     const unsigned long long* src = a.part + (int64_t)qi * a.B * a.kcap;
     const int nheads = a.B * heads;
     unsigned long long best = ~0ull;
@@ -490,9 +490,10 @@ int merge_lists(const QueryArgs& a, hipStream_t s) {
     const double lists = a.pick_rounds ? fmax(1.0, a.pick_first) : (double)a.B;
     const int heads = min(a.kcap, (int)ceil((a.pick_rounds ? 3.0 : 2.0) * (double)a.k / lists));
     if (a.k <= 32 && (int64_t)a.B * heads <= 2 * kWave) {
-        hipLaunchKernelGGL(merge_heads_kernel<kWave>, dim3((unsigned)a.nq), dim3(kWave), 0, s, a, heads);
+        hipLaunchKernelGGL((a.only ? merge_heads_kernel<kWave, true> : merge_heads_kernel<kWave, false>), dim3((unsigned)a.nq), dim3(kWave), 0, s, a, heads);
     } else if (a.k <= kMergeThreads && (int64_t)a.B * heads < 0x7fffffffLL) {
-        hipLaunchKernelGGL(merge_heads_kernel<kMergeThreads>, dim3((unsigned)a.nq), dim3(kMergeThreads), 0, s, a, heads);
+        hipLaunchKernelGGL((a.only ? merge_heads_kernel<kMergeThreads, true> : merge_heads_kernel<kMergeThreads, false>), dim3((unsigned)a.nq),
+                           dim3(kMergeThreads), 0, s, a, heads);
     } else {
         const int cap = merge_cap(a.k, (int64_t)a.B * a.kcap);
         hipLaunchKernelGGL(merge_topk_kernel, dim3((unsigned)a.nq), dim3(kMergeThreads),

@@ -231,7 +231,9 @@ struct DenseTables {
     }
 };
 
-template <int NT, int IPT, int WAVES>      // WAVES: wavefronts per SIMD the registers are shared out for
+// WAVES: wavefronts per SIMD the registers are shared out for.  PICKED: the items are those of a call's round.  (Both in one
+// kernel cost whole calls 3 %: 5000 items of 1350 rows, 418 and 429 us.)
+template <int NT, int IPT, int WAVES, bool PICKED>
 __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
     // The arguments are read where they are used, through a pointer that every phase makes opaque again:
     // read once, ahead of the loop over the items, they would be carried through it in spilled registers.
@@ -280,7 +282,7 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
     const int64_t g0 = blockIdx.x / X;
     int64_t my_count;
     const int32_t* my_items = nullptr;
-    if (args->a.picked) {
+    if constexpr (PICKED) {
         int64_t first;
         my_count = picked_run(args->a.picked_count, xcd, X, first);
         my_items = args->a.picked + first;
@@ -308,7 +310,7 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
         ArgsPtr args = fresh_args();
         DenseTables tb(smem, args->a, args->y);
         int b, qi;
-        if (my_items) {
+        if (PICKED || my_items) {
             const int64_t item = my_items[slot];
             b = (int)(item % args->a.B);
             qi = (int)(item / args->a.B);
@@ -870,7 +872,7 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
         // each, in words of the scan's scratch that this phase does not use): 13000 candidates of 96 elements, k = 100, of 25000
         // rows in 196 tiles, a handful of them near: 76 -> 12 us per item.
         uint32_t* near_bits = scan_tmp + 48;
-        const bool near = args->a.near_bounds != nullptr;
+        const bool near = PICKED && args->a.near_bounds != nullptr;
         const int near_shift = args->a.near_shift;
         if (near) {
             if (tid < 16) near_bits[tid] = 0;
@@ -1340,6 +1342,19 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
 
 #undef PHASE_END
 
+template <int NT, int IPT, int WAVES, bool PICKED>
+int launch_dense(const DenseArgs& args, unsigned grid, hipStream_t s) {
+    static DeviceOnce once;
+    const int rc = once.run([]() -> int {
+        DCIH_HIP(hipFuncSetAttribute((const void*)traverse_dense_kernel<NT, IPT, WAVES, PICKED>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        return 0;
+    });
+    if (rc) return rc;
+    hipLaunchKernelGGL((traverse_dense_kernel<NT, IPT, WAVES, PICKED>), dim3(grid), dim3(NT), args.y.lds_bytes, s, args);
+    DCIH_HIP(hipGetLastError());
+    return 0;
+}
+
 }  // namespace
 
 bool dense_traversal_supported(const QueryArgs& a, size_t* lds_bytes) {
@@ -1388,17 +1403,8 @@ int query_dense_items(const QueryArgs& a_in, hipStream_t s) {
         args.step = (int)per_xcd;
     }
     const unsigned grid = (unsigned)(per_xcd * a.xcds);
-#define DCIH_DENSE(NT, IPT, WAVES)                                                                 \
-    do {                                                                                         \
-        static DeviceOnce once;                                                                  \
-        const int rc_attr = once.run([]() -> int {                                               \
-            DCIH_HIP(hipFuncSetAttribute((const void*)traverse_dense_kernel<NT, IPT, WAVES>,      \
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024)); \
-            return 0;                                                                            \
-        });                                                                                      \
-        if (rc_attr) return rc_attr;                                                             \
-        hipLaunchKernelGGL((traverse_dense_kernel<NT, IPT, WAVES>), dim3(grid), dim3(NT), y.lds_bytes, s, args); \
-    } while (0)
+#define DCIH_DENSE(NT, IPT, WAVES) rc = a.picked ? launch_dense<NT, IPT, WAVES, true>(args, grid, s) : launch_dense<NT, IPT, WAVES, false>(args, grid, s)
+    int rc;
     if (y.nt == 64) {
         if (y.ipt == 5) DCIH_DENSE(64, 5, 4); else DCIH_DENSE(64, 9, 4);
     } else if (y.nt == 256) {
@@ -1411,8 +1417,7 @@ int query_dense_items(const QueryArgs& a_in, hipStream_t s) {
         DCIH_DENSE(512, 21, 2);
     }
 #undef DCIH_DENSE
-    DCIH_HIP(hipGetLastError());
-    return 0;
+    return rc;
 }
 
 }  // namespace dcih
