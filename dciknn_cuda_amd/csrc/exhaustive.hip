@@ -338,7 +338,224 @@ __global__ __launch_bounds__(NT, NT / 256) void rank_row_kernel(const float* __r
     for (int r = 0; r < IPT; r++)
         if (tid * IPT + r < n) store(tid * IPT + r, key[r], rp[r] & 0xffffu);
 }
-static bool rank_fits(int64_t n) { return n <= 1024 * 16; }
+// Longer rows, and rows fewer than CUs: `parts` workgroups to a row, each of which finds the part of the order that is its own,
+// lists that part's items in LDS and ranks them there as above.  The parts are cut at bins of an even division of the row's range:
+// every workgroup counts all of the row, 4096 bins, and cuts where the bins pass p / parts of it.  Where a part does not fit
+// (distances that cluster) or a distance is not finite, its first and last item are found by their digits instead, eight bits of
+// (distance, number) at a time.  Bound by vector issue and LDS operations, of the passes over the row and of the ranking.
+// (Ranks of 64 rows of 20000: 61 us by the segmented sort, 30 in four parts each; read again by each of the four passes: 34.  16 rows of
+// 16000: 30 -> 16 us; of 50000: 74 -> 50.)
+constexpr int kRankMaxN = 1024 * 16;
+constexpr int kPartThreads = 1024, kPartBins = 4096, kPartMaxN = 65536;      // (numbers of 16 bits)
+constexpr size_t part_lds(int ipt) {
+    const size_t items = (size_t)kPartThreads * ipt;
+    return 160 * 4 + (size_t)kPartThreads * 8 + (2 * items + 4 + rank_counter_words(kPartThreads, ipt)) * 4 + items * 2;
+}
+template <int IPT, int ROW>      // ROW: items of the whole row per thread, in registers; 0: read again by every pass
+__global__ __launch_bounds__(kPartThreads, 4) void rank_part_kernel(const float* __restrict__ dists, int n, int k, int float_ids,
+                                                                 int32_t* __restrict__ out_ids, float* __restrict__ out_vals) {
+    constexpr int NT = kPartThreads, kItems = NT * IPT, kWaves = NT / kWave;
+    static_assert(kItems >= kPartBins, "the bins are where the items are listed later");
+    extern __shared__ __align__(16) unsigned char rank_smem[];
+    uint32_t* misc = reinterpret_cast<uint32_t*>(rank_smem);             // 32 words for the ranking
+    uint32_t* extremes = misc + 32;                                      // of the row, of the part; digits that differ
+    uint32_t* wave_sum = misc + 40;                                      // [kWaves]
+    uint32_t* cut = misc + 64;                                           // [parts + 1] bins, parts at most 32,
+    uint32_t* cut_at = misc + 112;                                       // and the items before them
+    unsigned long long* work = reinterpret_cast<unsigned long long*>(misc + 160);
+    uint32_t* list = reinterpret_cast<uint32_t*>(work + NT);             // [kItems + 4]; the bins first
+    uint32_t* cnt = list + kItems + 4;                                   // [rank_counter_words]
+    uint32_t* bits = cnt + rank_counter_words(NT, IPT);                                       // [kItems]: the part's distances, in order of their numbers
+    uint16_t* number = reinterpret_cast<uint16_t*>(bits + kItems);       // [kItems]
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int part = blockIdx.x, parts = gridDim.x;
+    const float* row = dists + (int64_t)blockIdx.y * n;
+    out_ids += (int64_t)blockIdx.y * k;
+    out_vals += (int64_t)blockIdx.y * k;
+    const int share = (n + kWaves - 1) / kWaves, from = min(n, wave * share), to = min(n, from + share);      // this wavefront's items
+    uint32_t w[ROW ? ROW : 1];
+#pragma unroll
+    for (int r = 0; r < ROW; r++) w[r] = __builtin_bit_cast(uint32_t, row[min(from + r * kWave + lane, n - 1)]);
+    auto each = [&](auto use) __attribute__((always_inline)) {           // use(number, bits, whether there is one): all lanes, in order
+#pragma unroll
+        for (int r = 0; r < ROW; r++) {
+            if (from + r * kWave >= to) break;
+            use(from + r * kWave + lane, w[r], from + r * kWave + lane < to);
+        }
+        if constexpr (ROW == 0) {
+#pragma unroll 8
+            for (int j = from + lane; j < to + lane; j += kWave) use(j, __builtin_bit_cast(uint32_t, row[min(j, n - 1)]), j < to);
+        }
+    };
+    // Exclusive sum over the workgroup's threads.
+    auto scan = [&](uint32_t sum) {
+        uint32_t incl = sum;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t t = (uint32_t)__shfl_up((int)incl, o, 64);
+            if (lane >= o) incl += t;
+        }
+        __syncthreads();
+        if (lane == 63) wave_sum[wave] = incl;
+        __syncthreads();
+        for (int w = 0; w < wave; w++) incl += wave_sum[w];
+        return incl - sum;
+    };
+    if (tid < 8) extremes[tid] = (tid & 1) ? 0u : 0xffffffffu;
+    for (int j = tid; j < kPartBins; j += NT) list[j] = 0;
+    __syncthreads();
+    {
+        uint32_t least = 0xffffffffu, most = 0;
+        each([&](int, uint32_t b, bool) { least = min(least, b); most = max(most, b); });      // (the row's last item again does no harm)
+        least = wave_min_u32(least);
+        most = ~wave_min_u32(~most);
+        if (lane == 0) { atomicMin(&extremes[0], least); atomicMax(&extremes[1], most); }
+    }
+    __syncthreads();
+    const uint32_t hi_bits = extremes[1];
+    const float lo = __builtin_bit_cast(float, extremes[0]), scale = 4294966016.0f / (__builtin_bit_cast(float, hi_bits) - lo);
+    bool even = hi_bits < kInfBits && scale < 4e38f;                     // (the same for all of a row's workgroups)
+    auto bin_of = [&](uint32_t b) { return (uint32_t)((__builtin_bit_cast(float, b) - lo) * scale) >> 20; };
+    auto cut_of = [&](int p) { return (uint32_t)((int64_t)n * p / parts); };
+    if (even) {
+        each([&](int, uint32_t b, bool in) { if (in) atomicAdd(&list[bin_of(b)], 1u); });
+        __syncthreads();
+        constexpr int kPer = kPartBins / NT;
+        uint32_t v[kPer], sum = 0;
+#pragma unroll
+        for (int i = 0; i < kPer; i++) { v[i] = list[tid * kPer + i]; sum += v[i]; }
+        uint32_t run = scan(sum);
+#pragma unroll
+        for (int i = 0; i < kPer; i++) { list[tid * kPer + i] = run; run += v[i]; }
+        __syncthreads();
+        if (tid <= parts) {      // the first bin that begins at the part's share or behind it
+            int a = 0, b = kPartBins;
+            while (a < b) {
+                const int mid = (a + b) >> 1;
+                if (list[mid] < cut_of(tid)) a = mid + 1; else b = mid;
+            }
+            cut[tid] = (uint32_t)a;
+            cut_at[tid] = a < kPartBins ? list[a] : (uint32_t)n;
+        }
+        __syncthreads();
+        for (int p = 0; p < parts; p++) even = even && cut_at[p + 1] - cut_at[p] <= (uint32_t)kItems;
+    }
+    unsigned long long item0 = 0, item1 = ~0ull;                         // (distance, number): the part's first, and the first behind it
+    // (by their bits as in rank_row_kernel, in rows too long for it by value as in the segmented sort: NaN of either sign)
+    const uint32_t negative = n > kRankMaxN ? 0xffffffffu : 0u, positive = n > kRankMaxN ? 0x80000000u : 0u;
+    auto order_of = [&](uint32_t b) { return b ^ (b >> 31 ? negative : positive); };
+    auto item_of = [&](uint32_t b, int j) { return ((unsigned long long)order_of(b) << 16) | (uint32_t)j; };
+    uint32_t first = cut_of(part);
+    if (even) {
+        first = cut_at[part];
+    } else {
+#pragma unroll 1
+        for (int end = 0; end < 2; end++) {      // the item with `place` others before it
+            uint32_t place = end ? cut_of(part + 1) : first;
+            if (place == 0 || place == (uint32_t)n) continue;
+            unsigned long long found = 0;
+#pragma unroll 1
+            for (int shift = 40; shift >= 0; shift -= 8) {
+                __syncthreads();
+                if (tid < 256) list[tid] = 0;
+                __syncthreads();
+                each([&](int j, uint32_t b, bool in) {
+                    const unsigned long long e = item_of(b, j);
+                    if (in && (e >> shift >> 8) == found) atomicAdd(&list[(uint32_t)(e >> shift) & 255u], 1u);
+                });
+                __syncthreads();
+                uint32_t digit = 0;
+                for (; digit < 255u && list[digit] <= place; digit++) place -= list[digit];      // (the same for all threads)
+                found = found << 8 | digit;
+            }
+            (end ? item1 : item0) = found;
+        }
+    }
+    if (first >= (uint32_t)k) return;
+    // The part's items, in order of their numbers.
+    const uint32_t bin0 = even ? cut[part] : 0, bin1 = even ? cut[part + 1] : 0;
+    auto mine = [&](int j, uint32_t b) {
+        if (even) { const uint32_t bin = bin_of(b); return bin >= bin0 && bin < bin1; }
+        const unsigned long long e = item_of(b, j);
+        return e >= item0 && e < item1;
+    };
+    uint32_t have = 0;
+    each([&](int j, uint32_t b, bool in) { have += in && mine(j, b) ? 1u : 0u; });
+    uint32_t at = scan(have);      // (lane 0's is the wavefront's)
+    at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+    int count = 0;
+    for (int w = 0; w < kWaves; w++) count += (int)wave_sum[w];
+    {
+        uint32_t least = 0xffffffffu, most = 0, all_or = 0, all_and = 0xffffffffu;
+        each([&](int j, uint32_t b, bool in) {
+            const bool take = in && mine(j, b);
+            const unsigned long long m = __ballot(take);
+            if (take) {
+                const uint32_t to_at = at + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+                bits[to_at] = b;
+                number[to_at] = (uint16_t)j;
+                least = min(least, b); most = max(most, b);
+                all_or |= order_of(b); all_and &= order_of(b);
+            }
+            at += (uint32_t)__popcll(m);
+        });
+        least = wave_min_u32(least);
+        most = ~wave_min_u32(~most);
+        for (int o = 32; o > 0; o >>= 1) {
+            all_or |= (uint32_t)__shfl_xor((int)all_or, o, kWave);
+            all_and &= (uint32_t)__shfl_xor((int)all_and, o, kWave);
+        }
+        if (lane == 0) { atomicMin(&extremes[2], least); atomicMax(&extremes[3], most); atomicAnd(&extremes[4], all_and); atomicOr(&extremes[5], all_or); }
+    }
+    __syncthreads();
+    if (count == 0) return;
+    uint32_t key[IPT], rp[IPT];
+    int fix_rank = -1;
+    uint32_t fix_item = 0;
+    bool ranked = false;
+    const float part_lo = __builtin_bit_cast(float, extremes[2]), part_scale = 4294966016.0f / (__builtin_bit_cast(float, extremes[3]) - part_lo);
+    if (extremes[3] < kInfBits && part_scale < 4e38f) {
+#pragma unroll
+        for (int r = 0; r < IPT; r++) {
+            const int j = r * NT + tid;
+            key[r] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(float, bits[min(j, count - 1)]) - part_lo);
+            rp[r] = (uint32_t)j;
+        }
+        auto before = [&](int x, int z) __attribute__((always_inline)) { return bits[x] != bits[z] ? bits[x] < bits[z] : x < z; };
+        ranked = lds_bucket_ranks<NT, IPT, rank_bits(kItems), true>(key, rp, count, part_scale, list, cnt, misc, work, NT, tid, fix_rank, fix_item,
+                                                                    before);
+    }
+    auto store = [&](uint32_t place, uint32_t b, uint32_t item) {
+        if (place >= (uint32_t)k) return;
+        out_vals[place] = __builtin_bit_cast(float, b);
+        out_ids[place] = float_ids ? __builtin_bit_cast(int32_t, (float)(int)item) : (int)item;
+    };
+    __syncthreads();
+    if (ranked) {      // through LDS, so that the results leave in order
+        uint16_t* order = reinterpret_cast<uint16_t*>(list);
+        int own = count > tid ? (count - tid + NT - 1) / NT : 0;
+        asm volatile("" : "+v"(own));
+#pragma unroll
+        for (int r = 0; r < IPT; r++)
+            if (r < own) order[rp[r] >> 16] = (uint16_t)(r * NT + tid);
+        __syncthreads();
+        if (fix_rank >= 0) order[fix_rank] = (uint16_t)fix_item;
+        __syncthreads();
+        for (int j = tid; j < count; j += NT) store(first + (uint32_t)j, bits[order[j]], number[order[j]]);
+        return;
+    }
+#pragma unroll
+    for (int r = 0; r < IPT; r++) {
+        const int j = tid * IPT + r;
+        key[r] = j < count ? order_of(bits[j]) : 0xffffffffu;      // (pads stay behind everything: the passes are stable)
+        rp[r] = (uint32_t)j;
+    }
+    lds_radix_passes<NT, IPT>(key, rp, list, cnt, misc, extremes[4] ^ extremes[5]);
+#pragma unroll
+    for (int r = 0; r < IPT; r++)
+        if (tid * IPT + r < count) store(first + (uint32_t)(tid * IPT + r), bits[rp[r] & 0xffffu], number[rp[r] & 0xffffu]);
+}
+static bool rank_fits(int64_t n) { return n <= kRankMaxN; }
 static int rank_rows_in_lds(const float* d_dist, int rows, int n, int k, int float_ids, int32_t* out_ids, float* out_vals,
                             hipStream_t s) {
 #define DCIH_RANK(NT, IPT)                                                                              \
@@ -358,6 +575,35 @@ static int rank_rows_in_lds(const float* d_dist, int rows, int n, int k, int flo
 #undef DCIH_RANK
     DCIH_HIP(hipGetLastError());
     return 0;
+}
+
+template <int IPT, int ROW>
+static int launch_parts(const float* d_dist, int parts, int rows, int n, int k, int float_ids, int32_t* out_ids, float* out_vals, hipStream_t s) {
+    static DeviceOnce once;
+    const int rc = once.run([]() -> int {
+        DCIH_HIP(hipFuncSetAttribute((const void*)rank_part_kernel<IPT, ROW>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        return 0;
+    });
+    if (rc) return rc;
+    hipLaunchKernelGGL((rank_part_kernel<IPT, ROW>), dim3((unsigned)parts, (unsigned)rows), dim3(kPartThreads), part_lds(IPT), s, d_dist, n, k,
+                       float_ids, out_ids, out_vals);
+    DCIH_HIP(hipGetLastError());
+    return 0;
+}
+// How many workgroups to a row: as many as leave one to a CU, if they hold it; 1: the kernels for whole rows.  (With rows on the device
+// twice, 64 of 16000, 4 / 6 parts: 33 / 52 us.  Short rows lose by the passes over the whole, 64 of 4000: 16 us whole, 18 in parts; 9582:
+// 28, 26.  More than 16 gain nothing.)
+constexpr int part_items(int64_t n, int parts) { return (int)(n / parts) * 21 / 20 + 64; }      // (bins are a few items)
+static int rank_parts(int64_t n, int rows) {
+    const int parts = (int)min((int64_t)16, (int64_t)256 / rows);
+    return n >= 8192 && n <= kPartMaxN && parts > 1 && part_items(n, parts) <= kPartThreads * 10 ? parts : 1;
+}
+static int rank_rows_in_parts(const float* d_dist, int parts, int rows, int n, int k, int float_ids, int32_t* out_ids, float* out_vals, hipStream_t s) {
+    const int most = part_items(n, parts);
+    const auto launch = n <= 20480 ? (most <= 4096 ? launch_parts<4, 20> : most <= 6144 ? launch_parts<6, 20> : launch_parts<10, 20>)
+                      : n <= 32768 ? (most <= 4096 ? launch_parts<4, 32> : most <= 6144 ? launch_parts<6, 32> : launch_parts<10, 32>)
+                                   : (most <= 4096 ? launch_parts<4, 0> : most <= 6144 ? launch_parts<6, 0> : launch_parts<10, 0>);
+    return launch(d_dist, parts, rows, n, k, float_ids, out_ids, out_vals, s);
 }
 
 // The first k columns of every sorted row.  Columns past the end of a row and, when
@@ -534,7 +780,9 @@ int query_exhaustive(const QueryArgs& a, void* ws, int chunk, hipStream_t s) {
             if (rc) return rc;
             continue;
         }
-        const int rc = rank_fits(a.N)
+        const int parts = rank_parts(a.N, nqc);
+        const int rc = parts > 1 ? rank_rows_in_parts(d_dist, parts, nqc, (int)a.N, a.k, a.float_ids, out_ids, out_dists, s)
+            : rank_fits(a.N)
             ? rank_rows_in_lds(d_dist, nqc, (int)a.N, a.k, a.float_ids, out_ids, out_dists, s)
             : rank_rows(ws, chunk, nqc, a.N, a.k, false, a.float_ids != 0, out_ids, out_dists, s);
         if (rc) return rc;

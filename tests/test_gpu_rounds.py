@@ -191,3 +191,22 @@ def test_nearest_of_many_rows(gpu):      # more than 512 workgroups of the produ
     dci.free()
     assert torch.equal(got[0], want[0])
     assert torch.equal(got[1].view(torch.int32), want[1].view(torch.int32))
+
+
+# Rows ranked by several workgroups (few rows) and by one (many): sizes at the edges of both, of the rows that are kept in registers
+# and of the numbers of 16 bits; distances spread evenly, equal, in clusters too dense for a part, and not finite.
+@pytest.mark.parametrize("kind", ["normal", "grid", "zero", "huge", "broken"])
+@pytest.mark.parametrize("n", [8191, 8192, 10001, 16384, 16385, 20480, 20481, 32768, 32769, 65536, 65537])
+def test_ranking_in_parts(gpu, kind, n):
+    X, Q = _rows(kind, n, 300, 9, n)
+    dci = gpu.DCI(9, 2, 3, 50, 10, seed=3)
+    dci.add(X)
+    want = dci.query(Q, return_int=True)
+    for some in (Q[:1], Q[40:56], Q[40:104]):
+        got = dci.query(some.contiguous(), return_int=True)
+        first = 0 if len(some) == 1 else 40
+        assert torch.equal(got[0], want[0][first:first + len(some)])
+        assert torch.equal(got[1].view(torch.int32), want[1][first:first + len(some)].view(torch.int32))
+    few = dci.query(Q[:3].contiguous(), 8200 if n > 8200 else 300, 5000, return_int=True)
+    dci.free()
+    assert torch.equal(few[0], want[0][:3, :few[0].shape[1]])
