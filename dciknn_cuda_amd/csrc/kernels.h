@@ -91,7 +91,7 @@ struct QueryArgs {
     const int32_t* block_list;        // null = the launch covers queries q_first .. q_first + q_count; else workgroup w takes block_list[w]
     const uint32_t* block_list_count; // ... for w below this number
     float expect_steps, expect_promotions;      // the batch kernel's first guess at where a full partition's traversal stops
-    int few_items;           // 1: the batch kernel gives every item four wavefronts
+    int few_items;           // 1: the batch kernel gives every item four wavefronts or more; 2: and larger tables
     int full_tables;         // 1: the batch kernel keeps its per-point flags as bits whatever the shape
     // dense kernel: the rows' and the queries' 8-bit codes (rows8.hip; null = read whole rows)
     const unsigned char* rows8;      // [N][rows8_rec]

@@ -109,12 +109,15 @@ BlockLayout make_block_layout(const QueryArgs& a) {
     // step limit rather than c0 >= k ends the traversal): fewer, larger epochs.
     const double expected = expected_promotions(a);
     y.promo_cap = 128;
-    while ((double)y.promo_cap < 2.0 * expected && y.promo_cap < 2048) y.promo_cap <<= 1;
+    const double room = a.few_items == 2 ? 8.0 : 2.0;
+    // (an epoch of one window per stream should fit too where that is easily had: what does not goes to the step-by-step kernel)
+    const double least = a.few_items == 2 ? 2.0 * a.M * a.L * a.T : 0.0;
+    while ((double)y.promo_cap < fmax(room * expected, least) && y.promo_cap < 2048) y.promo_cap <<= 1;
     y.promo_max = y.promo_cap * 5 / 8;
     const bool compact = block_layout_compact(a, y.promo_cap);
     y.set_slots = compact ? kSetSlots : 0;
     y.set_limit = kSetSlots * 7 / 16;     // every promotion adds at most two entries: the set stays under 7/8 full
-    y.event_cap = compact ? y.promo_cap : 2 * y.promo_cap;
+    y.event_cap = compact ? y.promo_cap : (a.few_items == 2 ? 4 : 2) * y.promo_cap;
     y.sort_cap = 64;           // top-k plus a batch of at least 48 new candidates
     while (y.sort_cap < a.kcap + 48) y.sort_cap <<= 1;
     // the accepted candidates of a replay share the room of the priority samples and the
@@ -1256,6 +1259,16 @@ static int launch_block(const QueryArgs& a, const BlockLayout& y, int64_t items,
         DCIH_HIP(hipGetLastError());
         return 0;
     }
+    // Items fewer than the device holds of them: each has sixteen wavefronts where that is one to a CU, eight up to four.  (1M x 128,
+    // thread_size 2, one query: 118 us of four wavefronts, 88 of sixteen; 928 items 288 of four, 263 of eight; sixteen at two to a CU: 237, 182 of eight.)
+    const int64_t cus = (int64_t)a.xcds * 32;
+    if (a.few_items && items <= 4 * cus) {
+        if (a.picked) DCIH_LAUNCH_KERNEL((traverse_block_picked_kernel<512, 4, false>), 512, items);
+        else if (items <= cus) DCIH_LAUNCH_KERNEL((traverse_block_kernel<1024, 4, false>), 1024, items);
+        else DCIH_LAUNCH_KERNEL((traverse_block_kernel<512, 4, false>), 512, items);
+        DCIH_HIP(hipGetLastError());
+        return 0;
+    }
     const bool narrow = !a.few_items && 4 * a.M * a.L <= kNarrowThreads && fit >= 10;
     int minw = narrow ? (fit * (kNarrowThreads / 64) + 3) / 4 : fit;      // wavefronts per SIMD
     if (a.few_items) minw = std::min(minw, (int)((items + a.xcds * 32 - 1) / (a.xcds * 32)));
@@ -1283,15 +1296,20 @@ int query_block(const QueryArgs& a_query, hipStream_t s) {
     // doubling its way forward from 1/128 of a stream.  A call of so few items that the device holds them
     // all at once waits for its slowest item: four wavefronts per item then, with the tables that need no
     // second pass.  (17242-point partitions, thread_size 2: rebuild and 16 queries 2.7 -> 0.75 ms, one query
-    // 437 -> 166 us.)
+    // 437 -> 166 us.)  Larger tables if the items fit with them as well: an epoch may then go as far as nearly every stop (one
+    // query: 26 % of the items needed a second epoch, 150 -> 118 us without).
     // (Asked for by name, the kernel keeps the variant for many items and feels its way forward at first.)
     if (a_in.mode == 0) {
         a_in.expect_steps = (float)(0.9 * expected_stop(a_in));
         a_in.expect_promotions = (float)expected_promotions(a_in);
-        QueryArgs wide = a_in;
-        wide.full_tables = 1;
-        const BlockLayout y4 = make_block_layout(wide);
-        if (y4.lds_bytes <= kMostLds && (a_in.picked ? a_in.picked_expect : (int64_t)a_in.nq * a_in.B) <= (int64_t)a_in.xcds * 32 * wide_fit(y4)) a_in.full_tables = a_in.few_items = 1;
+        const int64_t items = a_in.picked ? a_in.picked_expect : (int64_t)a_in.nq * a_in.B;
+        for (int few = 2; few >= 1 && !a_in.few_items; few--) {
+            QueryArgs wide = a_in;
+            wide.full_tables = 1;
+            wide.few_items = few;
+            const BlockLayout y4 = make_block_layout(wide);
+            if (y4.lds_bytes <= kMostLds && items <= (int64_t)a_in.xcds * 32 * wide_fit(y4)) { a_in.full_tables = 1; a_in.few_items = few; }
+        }
     }
     const BlockLayout y = make_block_layout(a_in);
     // as many queries per launch as the launch limit allows (nearly always all of them)

@@ -72,3 +72,22 @@ def test_ranking_where_nothing_stops_early(gpu, oracle, n, dim, k, nq, kind):
     np.testing.assert_array_equal(ids.cpu().numpy(), order)
     np.testing.assert_array_equal(dists.cpu().numpy(), np.take_along_axis(d, order, 1))
     dci.free()
+
+
+# Items fewer than the device holds have workgroups of more wavefronts and larger tables: one item to a CU, up to four, and more.
+@pytest.mark.parametrize("nq", [1, 4, 5, 17, 18, 29])
+@pytest.mark.parametrize("M,L,T,k,outer", [(2, 10, 2, 10, 500), (2, 15, 3, 40, 50), (1, 30, 10, 1, 5000), (4, 16, 1, 5, 300)])
+def test_items_of_more_wavefronts(gpu, nq, M, L, T, k, outer):
+    from dciknn_cuda_amd import _capi
+    gen = torch.Generator().manual_seed(nq)
+    X = torch.randn(400011, 24, generator=gen).cuda()
+    Q = torch.randn(150, 24, generator=gen).cuda()
+    dci = gpu.DCI(24, M, L, 58, T, seed=3)
+    dci.add(X)
+    _capi.check(dci._lib.dcih_set_option(dci._dci_inst, _capi.OPT_ROUNDS, 1))      # every partition is traversed
+    want = [t.clone() for t in dci.query(Q, k, outer, return_int=True)]
+    for start in (0, 60):
+        got = dci.query(Q[start:start + nq].contiguous(), k, outer, return_int=True)
+        assert torch.equal(got[0], want[0][start:start + nq])
+        assert torch.equal(got[1].view(torch.int32), want[1][start:start + nq].view(torch.int32))
+    dci.free()
