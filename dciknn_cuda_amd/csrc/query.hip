@@ -344,9 +344,12 @@ __global__ __launch_bounds__(NT) void merge_heads_kernel(QueryArgs a, int heads)
     if constexpr (NT == kWave) bitonic_sort_u64(buf, NT); else bitonic_sort_u64_by256(buf, NT);
     const unsigned long long bound = buf[a.k - 1];       // (nothing at all in some list heads: ~0, every entry passes)
     __syncthreads();
-    for (int l = tid; l < a.B; l += NT) {
+    // (as many threads to a list as there are, every one with its own entries: two lists of 100, 17 -> 10 us)
+    int lg = 0;
+    while ((2 * a.B << lg) <= NT) lg++;
+    for (int l = tid >> lg; l < a.B; l += NT >> lg) {
         const unsigned long long* list = src + (int64_t)l * a.kcap;
-        for (int j0 = 0; j0 < a.kcap; j0 += kAhead) {
+        for (int j0 = (tid & ((1 << lg) - 1)) * kAhead; j0 < a.kcap; j0 += kAhead << lg) {
             unsigned long long v[kAhead];
 #pragma unroll
             for (int u = 0; u < kAhead; u++) v[u] = list[min(j0 + u, a.kcap - 1)];
