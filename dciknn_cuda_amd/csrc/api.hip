@@ -890,7 +890,7 @@ int dcih_debug_positions(dcih_index* h, uint16_t* d_inv, uint16_t* d_rpos, void*
         if (!h->rpos_ready) {
             // (rows of the first simple indices are never written: clear the table so that they read as zeros)
             DCIH_HIP(hipMemsetAsync(h->d_rpos, 0, cells * sizeof(uint16_t), s));
-            const int rc = fill_positions_by_first(h->d_sids, h->d_inv, h->d_rpos, h->n, h->M, h->L, s);
+            const int rc = fill_positions_by_first(h->d_sids, h->d_inv, h->d_rpos, h->n, h->M, h->L, (h->n + h->block_size - 1) / h->block_size, h->block_size, s);
             if (rc) return rc;
             h->rpos_ready = 1;
         }

@@ -40,7 +40,7 @@ int segsort_append(const float* d_old_skeys, const int32_t* d_old_sids, int64_t 
 
 // rpos (above inv's layout, [I][n] 16-bit values): rpos[i][e] = inv[i][sids[first(i)][e]], first(i) = the first simple
 // index of i's composite; the rows of the first simple indices themselves are left alone (the identity).
-int fill_positions_by_first(const int32_t* d_sids, const uint16_t* d_inv, uint16_t* d_rpos, int64_t n, int M, int L,
+int fill_positions_by_first(const int32_t* d_sids, const uint16_t* d_inv, uint16_t* d_rpos, int64_t n, int M, int L, int64_t ppb, int B,
                             hipStream_t s);
 
 struct QueryArgs {

@@ -558,7 +558,7 @@ int query(const QueryArgs& a_in, void* bounds_ws, hipStream_t s, hipEvent_t* ev,
         if (use_block || a.mode == 3) {
             if (use_block) {
                 if (a.rpos_ready && !*a.rpos_ready) {      // the first batch traversal over this index
-                    const int rc = fill_positions_by_first(a.sids, a.inv, const_cast<uint16_t*>(a.rpos), a.N, a.M, a.L, s);
+                    const int rc = fill_positions_by_first(a.sids, a.inv, const_cast<uint16_t*>(a.rpos), a.N, a.M, a.L, a.ppb, a.B, s);
                     if (rc) return rc;
                     if (!a.recorded) *a.rpos_ready = 1;
                 }
