@@ -482,7 +482,7 @@ __global__ __launch_bounds__(128 * WR * WC, WAVES) void bounds_stream_kernel(Bou
 // largest in the histogram's bins up to the one that holds it, 1024 bins over the range of those that are finite.  A workgroup reads the
 // bounds of `per` neighbouring queries into LDS first.  (Bit by bit, with a ballot per bit, limit and 64 bounds: 3 times as long.)
 template <int V>
-__global__ __launch_bounds__(256) void pick_limits_kernel(const uint32_t* __restrict__ bounds, int S, int nq, int per, int j, int near_rank,
+__global__ __launch_bounds__(256) void pick_limits_kernel(const uint32_t* __restrict__ bounds, int S, int nq, int per, int j, int near_rank, float flat,
                                                           uint32_t* __restrict__ limits, uint32_t* __restrict__ last_round) {
     constexpr int kBins = 1024, kMine = kBins / 64;
     __shared__ uint32_t s_hist[4][kBins];
@@ -533,6 +533,8 @@ __global__ __launch_bounds__(256) void pick_limits_kernel(const uint32_t* __rest
             most = wave_max_i32(most);
             limit[w] = __ballot(upto >= rank) ? (uint32_t)most : kInf;          // (infinite where there are fewer)
         }
+        // Bounds too close together for what a short traversal finds: the first round would find no distance that rules a partition out.
+        if (f_lo + range < flat * __builtin_bit_cast(float, limit[0])) limit[0] = limit[1] = limit[2] = kInf;
         if (q0 + q < nq) {
             if (lane < kLimits) limits[(int64_t)lane * nq + q0 + q] = lane == 0 ? limit[0] : (lane == 1 ? limit[1] : (lane == 2 ? limit[2] : limit[3]));
             if (lane == 0) last_round[q0 + q] = 0;
@@ -769,7 +771,7 @@ int pick_items(const QueryArgs& a, void* ws_, int round, int rounds, hipStream_t
         const dim3 grid((unsigned)((a.nq + per - 1) / per));
 #define DCIH_LIMITS(V)                                                                                              \
     hipLaunchKernelGGL(pick_limits_kernel<V>, grid, dim3(256), (size_t)S * (per + 1) * 4, s, bounds, S, a.nq, per, \
-                       a.pick_rank, min(32 * a.pick_rank, max(4 * a.pick_rank, S / 2)), limits, last)
+                       a.pick_rank, min(32 * a.pick_rank, max(4 * a.pick_rank, S / 2)), a.pick_flat, limits, last)
         if (S <= 64) DCIH_LIMITS(1); else if (S <= 128) DCIH_LIMITS(2); else if (S <= 256) DCIH_LIMITS(4);
         else if (S <= 512) DCIH_LIMITS(8); else if (S <= 1024) DCIH_LIMITS(16); else DCIH_LIMITS(32);
 #undef DCIH_LIMITS

@@ -123,6 +123,7 @@ struct QueryArgs {
     int pick_rule;           // DCIH_OPT_ROUNDS value
     double pick_first;       // partitions per query the first round is expected to take
     double share;            // share of all items that are expected to be traversed (1 but for such calls)
+    float pick_flat;         // a query whose furthest bound is within this factor of round 1's limit takes every partition at once
     float* dense;            // null, or [nq][N]: the step-by-step kernel stores every candidate's score here instead of keeping a top-k
 };
 // About how many promotions a partition's traversal takes before it stops: k_stop of them by a window's

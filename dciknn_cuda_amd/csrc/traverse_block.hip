@@ -1158,12 +1158,13 @@ __global__ __launch_bounds__(NT, MINW) void traverse_block_picked_kernel(QueryAr
     traverse_block_item<NT, MINW, COMPACT>(a, y, b, qi);
 }
 // What more than the launch above covers (more partitions of a query at the same bound than one expects): strides over the rest.
-__global__ __launch_bounds__(256, 3) void traverse_block_rest_kernel(QueryArgs a, BlockLayout y, int64_t covered) {
+template <int NT, int MINW, bool COMPACT>
+__global__ __launch_bounds__(NT, MINW) void traverse_block_rest_kernel(QueryArgs a, BlockLayout y, int64_t covered) {
     int64_t first;
     const int64_t count = picked_run(a.picked_count, (int)(blockIdx.x % (unsigned)a.xcds), a.xcds, first);
     for (int64_t w = covered + blockIdx.x / (unsigned)a.xcds; w < count; w += gridDim.x / (unsigned)a.xcds) {
         const int32_t item = __builtin_amdgcn_readfirstlane(a.picked[first + w]);
-        traverse_block_item<256, 3, false>(a, y, item % a.B, item / a.B);
+        traverse_block_item<NT, MINW, COMPACT>(a, y, item % a.B, item / a.B);
         __syncthreads();          // the next item reuses the tables
     }
 }
@@ -1289,6 +1290,19 @@ static int launch_block(const QueryArgs& a, const BlockLayout& y, int64_t items,
     return 0;
 }
 
+template <int NT, int MINW, bool COMPACT>
+static int launch_rest(const QueryArgs& a, const BlockLayout& y, int64_t workgroups, int64_t covered, hipStream_t s) {
+    static DeviceOnce once;
+    const int rc = once.run([]() -> int {
+        DCIH_HIP(hipFuncSetAttribute((const void*)traverse_block_rest_kernel<NT, MINW, COMPACT>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        return 0;
+    });
+    if (rc) return rc;
+    hipLaunchKernelGGL((traverse_block_rest_kernel<NT, MINW, COMPACT>), dim3((unsigned)workgroups), dim3(NT), y.lds_bytes, s, a, y, covered);
+    DCIH_HIP(hipGetLastError());
+    return 0;
+}
+
 int query_block(const QueryArgs& a_query, hipStream_t s) {
     QueryArgs a_in = a_query;
     a_in.expect_promotions = (float)((double)a_in.k_stop * (double)a_in.T);
@@ -1345,18 +1359,15 @@ int query_block(const QueryArgs& a_query, hipStream_t s) {
         int rc = launch_block(a, y, each * X, s);
         if (rc) return rc;
         if (each * X < (int64_t)a.nq * a.B) {
-            static DeviceOnce once;
-            rc = once.run([]() -> int {
-                DCIH_HIP(hipFuncSetAttribute((const void*)traverse_block_rest_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-                return 0;
-            });
+            if (two_passes) {
+                rc = launch_rest<kWave, 6, true>(a, y, X * 32 * min((int64_t)24, (int64_t)(160 * 1024 / y.lds_bytes)), each, s);
+            } else {
+                QueryArgs rest = a;
+                rest.full_tables = 1;
+                const BlockLayout y4 = make_block_layout(rest);
+                rc = launch_rest<kBlockThreads, 3, false>(rest, y4, X * 32 * wide_fit(y4), each, s);
+            }
             if (rc) return rc;
-            QueryArgs rest = a;
-            rest.full_tables = 1;
-            rest.wide_items = nullptr;
-            const BlockLayout y4 = make_block_layout(rest);
-            hipLaunchKernelGGL(traverse_block_rest_kernel, dim3((unsigned)(X * 32 * wide_fit(y4))), dim3(256), y4.lds_bytes, s, rest, y4, each);
-            DCIH_HIP(hipGetLastError());
         }
     }
     for (int q0 = a_in.picked ? a_in.nq : 0; q0 < a_in.nq; q0 += (q0 < lead ? lead : per_launch)) {
