@@ -488,6 +488,7 @@ bool plan_rounds(QueryArgs& a) {
     a.pick_rank = rank;
     a.pick_first = first;
     a.share = share;
+    a.pick_near = can_dense && takes_dense_kernel(a) && near_bytes(a) <= ((size_t)1 << 30) ? 1 : 0;
     return true;
 }
 
