@@ -620,7 +620,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
                       int num_neighbours, int blind, int num_outer_iterations,
                       int max_num_candidates, int block_size, int thread_size,
                       int32_t* d_nn, float* d_dists, uint64_t* d_counters, void* stream,
-                      bool fixed, bool float_ids, const char* who) {
+                      bool fixed, bool float_ids, const char* who, bool whole = false) {
     const std::string me(who);
     if (!h) return fail(DCIH_EINVAL, me + ": null handle");
     if (dim != h->dim) return fail(DCIH_EINVAL, me + ": dim differs from the index's");
@@ -687,7 +687,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     a.rows8 = nullptr; a.rows8_rec = 0; a.rows8_bounds = nullptr; a.query8 = nullptr;
     a.picked = nullptr; a.picked_count = nullptr; a.picked_expect = a.picked_cover = 0; a.only = nullptr; a.only_round = 0;
     a.share = 1.0; a.pick_first = 0.0; a.pick_rounds = a.pick_rank = a.pick_near = 0;
-    a.near_bounds = nullptr; a.near_limit = nullptr; a.near_stride = 0; a.near_shift = a.near_tiles = 0; a.pick_rule = fixed ? 1 : h->rounds;
+    a.near_bounds = nullptr; a.near_limit = nullptr; a.near_stride = 0; a.near_shift = a.near_tiles = 0; a.pick_rule = fixed || whole ? 1 : h->rounds;
     a.phase_ticks = h->d_phase_ticks;
     a.stop_hint = nullptr;
     a.N = h->n;
@@ -798,6 +798,11 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     const size_t ws_bytes = qp_bytes + part_bytes + gs_bytes + redo_bytes + 256 + dense_bytes + wide_bytes;
     if (fixed && ws_bytes + q8_bytes > kScratchBytes) { a.rows8 = nullptr; q8_bytes = 0; }
     int rc = get_ws(ws_bytes + q8_bytes + (a.pick_rounds ? bounds_bytes(a) : 0));
+    if (rc && a.pick_rounds) {      // no room for the bounds: everything is traversed, which needs less (the same results)
+        (void)hipGetLastError();
+        return query_impl(h, dim, num_queries, d_query, num_neighbours, blind, num_outer_iterations, max_num_candidates,
+                          block_size, thread_size, d_nn, d_dists, d_counters, stream, fixed, float_ids, who, true);
+    }
     if (rc) return rc;
     char* base = ws_base;
     float* d_qproj = (float*)base;

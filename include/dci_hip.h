@@ -79,6 +79,10 @@ enum {
  * (only the new rows are projected), 2 = merge: the old slices are split into sorted
  * runs of the new ones, the new points sorted, the runs merged (error where the shape
  * does not allow it: partitions of more than 32256 points).  All give the same index.
+ * DCIH_OPT_ROUNDS: whether a query under automatic choice first bounds the distance of
+ * every partition's nearest point from below and then traverses, in rounds, only the
+ * partitions that can still hold a result: 0 = where it is estimated to be faster,
+ * 1 = never, 2 = wherever the shape allows it.  Results are the same to the bit.
  */
 enum { DCIH_OPT_TRAVERSAL = 0, DCIH_OPT_DENSE_MIN_PROMOTIONS = 1, DCIH_OPT_FORGET_HINTS = 2, DCIH_OPT_APPEND = 3,
        DCIH_OPT_ROUNDS = 4 };

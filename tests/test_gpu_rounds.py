@@ -147,6 +147,38 @@ def test_rounds_in_a_graph(gpu, k, T, outer):
     dci.free()
 
 
+def test_no_room_for_the_bounds(gpu):
+    """A recorded call cannot enlarge the workspace: what fits the one that whole traversals left is answered by them."""
+    from dciknn_cuda_amd import _capi
+    n, dim, nq, B, k = 30000, 48, 10000, 16, 3      # (the build's own workspace is smaller than the queries')
+    X, Q = _rows("clusters", n, nq, dim, 22)
+    dci = gpu.DCI(dim, 2, 7, B, 2, seed=9)
+    dci.add(X)
+    want = _ask(dci, dci._lib, NEVER, Q, k, 100)
+    ids = torch.empty((nq, k), dtype=torch.int32, device="cuda")
+    dists = torch.empty((nq, k), dtype=torch.float32, device="cuda")
+
+    def call(stream):
+        _capi.check(dci._lib.dcih_query(dci._dci_inst, dim, nq, Q.data_ptr(), k, 0, 100, 10 * k, B, 2,
+                                        ids.data_ptr(), dists.data_ptr(), None, stream))
+    s = torch.cuda.Stream()
+    call(s.cuda_stream)
+    s.synchronize()
+    _capi.check(dci._lib.dcih_set_option(dci._dci_inst, _capi.OPT_ROUNDS, ALWAYS))
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        call(torch.cuda.current_stream().cuda_stream)
+    for _ in range(3):
+        ids.fill_(-5)
+        dists.fill_(-5.0)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(ids, want[0]) and torch.equal(dists, want[1])
+    del g
+    dci.free()
+
+
 def test_what_asks_for_everything_gets_everything(gpu):
     """Counters and blind queries are of whole traversals, also where rounds are asked for."""
     from dciknn_cuda_amd import _capi
