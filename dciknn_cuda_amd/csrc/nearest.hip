@@ -401,9 +401,13 @@ bool nearest_supported(int64_t N, int dim, int k) {
 // Whether that is faster than all distances and a selection from them.  Few rows: those are a kernel of a few microseconds, until the
 // distances take as long as a second kernel's start (rows x dim, queries, all distances / this, us: 3000 x 100, 64: 15 / 17, 256: 22 / 17;
 // 1500 x 64 never gains, 4096: 59 / 64).  Many rows: one query gains nothing from a tile of 64 (60000 x 300, 4: 41 / 46, 16: 53 / 46,
-// 256: 637 / 75; 200000 x 64, 16: 42 / 53, 64: 102 / 60; 10000 x 32, 1: 15 / 13).
+// 256: 637 / 75; 200000 x 64, 16: 42 / 53, 64: 102 / 60; 10000 x 32, 1: 15 / 13), of short rows fewer still (100000 x 16, 32: 28 / 32, 64:
+// 38 / 34).  Long rows: few workgroups, one after another through the columns, wait longer than all distances take, until there are some
+// dozens of tiles (2048 x 960, 48: 44 / 55, 128: 68 / 56; 8192 x 300, 4: 24 / 26, 16: 28 / 26).
 bool nearest_pays(int64_t N, int dim, int nq) {
-    return N >= 8192 ? nq >= N / 4096 : N >= 2048 && (double)N * (double)nq * (double)dim >= 6e7;
+    const double pairs = (double)N * (double)nq;
+    if (N < 8192) return N >= 2048 && pairs >= 2.5e5 && pairs * (double)dim >= 6e7;
+    return (int64_t)nq * (dim < 64 ? 2048 : 4096) >= N && (dim <= 100 || pairs >= 1e5);
 }
 size_t nearest_least_bytes(int64_t N, int nq) { return (size_t)nq * (size_t)((N + 31) / 32) * 4; }
 
