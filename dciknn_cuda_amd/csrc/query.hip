@@ -483,6 +483,10 @@ bool plan_rounds(QueryArgs& a) {
     // of 241 elements, 42 partitions, 985 queries: 0.95 ms whole, 2.2 in rounds, 1.03 so), and rounds have to promise more.
     const bool short_stops = expected_promotions(a) < 0.02 * (double)a.ppb;
     if (!fits || (a.pick_rule == 0 && rounds > (short_stops ? 0.6 : 0.85) * whole)) return false;
+    // One to three results of traversals that leave out near rows bound little: everything else follows in the later rounds (32 queries, 64
+    // partitions of 8000 normal rows of 32, k = 3: 539 us whole, 710 in rounds; of 6000, k = 1: 378, 415; k = 10: 401, 229), and calls of
+    // one item for every workgroup gain less than that costs (14 queries, 64 partitions of 4000, k = 1: 155, 193; 32 queries: 295, 189).
+    if (a.pick_rule == 0 && a.k < 4 && (whole < 250.0 || expected_promotions(a) < 0.3 * (double)a.ppb)) return false;
     a.pick_flat = short_stops ? 1.3f : 0.0f;
     a.pick_rounds = few ? 2 : (whole > 1500.0 || a.pick_rule == 2 ? kMostRounds : 2);
     a.pick_rank = rank;

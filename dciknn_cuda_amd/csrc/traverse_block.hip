@@ -1182,6 +1182,7 @@ __global__ __launch_bounds__(NT, MINW) void traverse_block_list_kernel(QueryArgs
 }
 
 constexpr int kBlockThreads = 256;
+constexpr float kFewPromotions = 16.0f;      // items of fewer get no more wavefronts and no larger tables where a call has few items
 constexpr int kNarrowThreads = 128;     // workgroups of two wavefronts: more (query, partition) items per CU
 constexpr int kLeadQueries = 32;
 constexpr size_t kMostLds = 160 * 1024 - 512;
@@ -1263,7 +1264,8 @@ static int launch_block(const QueryArgs& a, const BlockLayout& y, int64_t items,
     // Items fewer than the device holds of them: each has sixteen wavefronts where that is one to a CU, eight up to four.  (1M x 128,
     // thread_size 2, one query: 118 us of four wavefronts, 88 of sixteen; 928 items 288 of four, 263 of eight; sixteen at two to a CU: 237, 182 of eight.)
     const int64_t cus = (int64_t)a.xcds * 32;
-    if (a.few_items && items <= 4 * cus) {
+    // (Items of a few promotions have too little for more than four to do: 896 items of 2000 points, thread_size 2, k = 1: 92 us of four, 112 of eight.)
+    if (a.few_items && items <= 4 * cus && a.expect_promotions >= kFewPromotions) {
         if (a.picked) DCIH_LAUNCH_KERNEL((traverse_block_picked_kernel<512, 4, false>), 512, items);
         else if (items <= cus) DCIH_LAUNCH_KERNEL((traverse_block_kernel<1024, 4, false>), 1024, items);
         else DCIH_LAUNCH_KERNEL((traverse_block_kernel<512, 4, false>), 512, items);
@@ -1317,7 +1319,7 @@ int query_block(const QueryArgs& a_query, hipStream_t s) {
         a_in.expect_steps = (float)(0.9 * expected_stop(a_in));
         a_in.expect_promotions = (float)expected_promotions(a_in);
         const int64_t items = a_in.picked ? a_in.picked_expect : (int64_t)a_in.nq * a_in.B;
-        for (int few = 2; few >= 1 && !a_in.few_items; few--) {
+        for (int few = a_in.expect_promotions >= kFewPromotions ? 2 : 1; few >= 1 && !a_in.few_items; few--) {
             QueryArgs wide = a_in;
             wide.full_tables = 1;
             wide.few_items = few;
