@@ -1182,7 +1182,9 @@ __global__ __launch_bounds__(NT, MINW) void traverse_block_list_kernel(QueryArgs
 }
 
 constexpr int kBlockThreads = 256;
-constexpr float kFewPromotions = 16.0f;      // items of fewer get no more wavefronts and no larger tables where a call has few items
+// Whether an item of a call of few items has work for more than four wavefronts: more than a few promotions, or a long partition (thread_size 2,
+// k = 1, four / eight wavefronts, us: 896 items of 2000 points 92 / 112, 900 of 8000 113 / 129; 256 of 16000 192 / 162, 900 of 16000 161 / 145).
+inline bool worth_more_wavefronts(const QueryArgs& a) { return a.expect_promotions >= 16.0f || a.ppb >= 10000; }
 constexpr int kNarrowThreads = 128;     // workgroups of two wavefronts: more (query, partition) items per CU
 constexpr int kLeadQueries = 32;
 constexpr size_t kMostLds = 160 * 1024 - 512;
@@ -1264,8 +1266,7 @@ static int launch_block(const QueryArgs& a, const BlockLayout& y, int64_t items,
     // Items fewer than the device holds of them: each has sixteen wavefronts where that is one to a CU, eight up to four.  (1M x 128,
     // thread_size 2, one query: 118 us of four wavefronts, 88 of sixteen; 928 items 288 of four, 263 of eight; sixteen at two to a CU: 237, 182 of eight.)
     const int64_t cus = (int64_t)a.xcds * 32;
-    // (Items of a few promotions have too little for more than four to do: 896 items of 2000 points, thread_size 2, k = 1: 92 us of four, 112 of eight.)
-    if (a.few_items && items <= 4 * cus && a.expect_promotions >= kFewPromotions) {
+    if (a.few_items && items <= 4 * cus && worth_more_wavefronts(a)) {
         if (a.picked) DCIH_LAUNCH_KERNEL((traverse_block_picked_kernel<512, 4, false>), 512, items);
         else if (items <= cus) DCIH_LAUNCH_KERNEL((traverse_block_kernel<1024, 4, false>), 1024, items);
         else DCIH_LAUNCH_KERNEL((traverse_block_kernel<512, 4, false>), 512, items);
@@ -1319,7 +1320,7 @@ int query_block(const QueryArgs& a_query, hipStream_t s) {
         a_in.expect_steps = (float)(0.9 * expected_stop(a_in));
         a_in.expect_promotions = (float)expected_promotions(a_in);
         const int64_t items = a_in.picked ? a_in.picked_expect : (int64_t)a_in.nq * a_in.B;
-        for (int few = a_in.expect_promotions >= kFewPromotions ? 2 : 1; few >= 1 && !a_in.few_items; few--) {
+        for (int few = worth_more_wavefronts(a_in) ? 2 : 1; few >= 1 && !a_in.few_items; few--) {
             QueryArgs wide = a_in;
             wide.full_tables = 1;
             wide.few_items = few;
