@@ -89,7 +89,7 @@ __global__ __launch_bounds__(kPackThreads) void pack_queries_kernel(PackArgs a) 
         for (int i = 0; i < 8; i++) centre[i] = s_centre[o * 8 + i];
         v8h h = round_octet(x, centre, scale, 0.5f * kHalfMax, sq, err);
 #pragma unroll
-        for (int i = 0; i < 8; i++) h[i] = (_Float16)((float)h[i] * -2.0f);      // (exact)
+        for (int i = 0; i < 8; i++) h[i] = (_Float16)((float)h[i] * -2.0f);      // (exact, and finite: half the largest at most)
         *reinterpret_cast<v8h*>(a.frags + (((int64_t)blockIdx.x * a.steps + (o >> 1)) * 64 + (o & 1) * 32 + qt) * 8) = h;
     }
     sq += lane_xor<4>(sq); sq += lane_xor<2>(sq); sq += lane_xor<1>(sq);

@@ -102,9 +102,9 @@ __device__ inline void place_octet(int dim, int j, float (&x)[8]) {
         for (int i = 0; i < 8; i++) x[i] = 0.0f;
 }
 // Rounds x - centre to 16 bits and sums the squares of the rounded values and of what was rounded off (the subtraction's
-// own rounding is allowed for where the sums are used).  What does not fit, or is not finite, makes the first sum so: it is cut to
-// `most` and to zero, the second sum infinite for the latter.  (16-bit floats below 2^-14, which the matrix cores may
-// take as zeros, are allowed for in rounding_floor.)
+// own rounding is allowed for where the sums are used).  No rounded value is larger than `most`: where the sum of an octet's squares
+// does not say so, its values are cut to that one by one, and to zero what is not finite, which makes the second sum infinite.
+// (16-bit floats below 2^-14, which the matrix cores may take as zeros, are allowed for in rounding_floor.)
 __device__ inline v8h round_octet(const float (&x)[8], const float (&centre)[8], float scale, float most, float& sq, float& err) {
     v8h out;
     float s2 = 0.0f, e2 = 0.0f;
@@ -119,7 +119,7 @@ __device__ inline v8h round_octet(const float (&x)[8], const float (&centre)[8],
         e2 = __builtin_fmaf(oa, oa, e2);
         e2 = __builtin_fmaf(ob, ob, e2);
     }
-    if (!(s2 < 8.0f * most * most && e2 < 1e30f)) {
+    if (!(s2 < most * most && e2 < 1e30f)) {
         s2 = e2 = 0.0f;
 #pragma unroll
         for (int i = 0; i < 8; i++) {

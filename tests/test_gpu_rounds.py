@@ -103,6 +103,24 @@ def test_rows_off_their_boundaries(gpu):
     _same(gpu, x, q, 2, 7, 20, 10, 10, 500)
 
 
+# A query's elements leave the range of 16-bit floats at 2^16 times what puts the sampled queries' largest at 64 .. 128, and twice
+# its elements, which the product takes, a factor of two before: single elements either side of both.  The rows' column holds values
+# of one sign in every second partition, so that no other row of a partition makes up for an infinite product.
+@pytest.mark.parametrize("T,outer", [(2, 1500), (10, 5000)], ids=["batch", "dense"])
+@pytest.mark.parametrize("dim,nq", [(24, 30), (33, 61), (24, 100), (264, 200), (33, 400), (24, 1100)])
+def test_one_element_far_from_the_others(gpu, dim, nq, T, outer):
+    n, B = 40000, 16
+    X, Q = _rows("normal", n, nq, dim, dim + nq)
+    part = torch.arange(n, device="cuda") // (n // B)
+    X[:, 0] = 1e-3 * (2.0 * (part % 2) - 1.0)
+    Q[:, 0] = 0.0
+    sampled = {nq * r // 16 for r in range(16)}
+    others = [q for q in range(nq) if q not in sampled]
+    for i, q in enumerate(others[:14]):
+        Q[q, 0] = (1.5 if i % 2 else -1.5) * 2.0 ** (7 + i // 2)
+    _same(gpu, X, Q, 2, 7, B, T, 10, outer, "dim %d nq %d" % (dim, nq))
+
+
 @pytest.mark.parametrize("k,T,outer", [(3, 2, 100), (10, 10, 5000)], ids=["batch", "dense"])
 def test_more_partitions_at_one_bound_than_expected(gpu, k, T, outer):
     """Queries that are not finite bound nothing: all their partitions come in round 1, far more items than its
