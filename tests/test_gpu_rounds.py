@@ -103,6 +103,23 @@ def test_rows_off_their_boundaries(gpu):
     _same(gpu, x, q, 2, 7, 20, 10, 10, 500)
 
 
+def test_rounds_run_the_kernel_of_whole_calls(gpu):
+    """The traversal kernel is chosen for all items: bounds that rule nothing out leave them all to it."""
+    from dciknn_cuda_amd import _capi
+    X, Q = _rows("normal", 100000, 300, 16, 2)
+    dci = gpu.DCI(16, 2, 10, 58, 2, seed=1)
+    dci.add(X)
+    _capi.check(dci._lib.dcih_profile(dci._dci_inst, 1))
+    ran = []
+    for rounds in (NEVER, 0, ALWAYS):
+        _ask(dci, dci._lib, rounds, Q, 30, 500)
+        t = (_capi.ctypes.c_float * _capi.NUM_TIMERS)()
+        _capi.check(dci._lib.dcih_last_timings(dci._dci_inst, t))
+        ran.append(bool(t[_capi.T_BATCH] > 0))
+    dci.free()
+    assert ran[0] == ran[1] == ran[2], ran
+
+
 # A query's elements leave the range of 16-bit floats at 2^16 times what puts the sampled queries' largest at 64 .. 128, and twice
 # its elements, which the product takes, a factor of two before: single elements either side of both.  The rows' column holds values
 # of one sign in every second partition, so that no other row of a partition makes up for an infinite product.
