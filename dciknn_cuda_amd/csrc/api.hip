@@ -154,6 +154,8 @@ struct dcih_index {
     int dense_by_cost = 1;              // until that option is set
     int append_mode = 0;                // DCIH_OPT_APPEND value
     int rounds = 0;                     // DCIH_OPT_ROUNDS value
+    int64_t route[4] = {0, 0, 0, 0};    // dcih_debug_route
+    uint32_t* d_round_items = nullptr;  // dcih_debug_round_items
     unsigned long long* d_phase_ticks = nullptr;   // optional profile of the batch kernel
     // grow-only workspace: query scratch, and the unsorted keys during a build
     void* ws = nullptr;
@@ -671,6 +673,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     };
 
     h->ev_valid[DCIH_T_BATCH] = h->ev_valid[DCIH_T_DENSE] = false;
+    for (int64_t& r : h->route) r = 0;
     QueryArgs a;
     a.skeys = h->d_skeys; a.sids = h->d_sids; a.inv = h->d_inv; a.data = h->d_data; a.query = d_query;
     a.rpos = h->d_rpos; a.rpos_ready = &h->rpos_ready; a.recorded = recorded ? 1 : 0;
@@ -685,10 +688,12 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     a.hand_over_at = 0;
     a.expect_steps = a.expect_promotions = 0.0f;
     a.rows8 = nullptr; a.rows8_rec = 0; a.rows8_bounds = nullptr; a.query8 = nullptr;
-    a.picked = nullptr; a.picked_count = nullptr; a.picked_expect = a.picked_cover = 0; a.only = nullptr; a.only_round = 0;
-    a.share = 1.0; a.pick_first = 0.0; a.pick_rounds = a.pick_rank = a.pick_near = 0;
+    a.picked = nullptr; a.picked_count = nullptr; a.picked_expect = a.picked_cover = 0; a.picked_exact = 0; a.only = nullptr; a.only_round = 0;
+    a.share = 1.0; a.pick_first = 0.0; a.pick_rounds = a.pick_rank = a.pick_near = a.pick_sample = 0; a.pick_most = 1.0f;
     a.near_bounds = nullptr; a.near_limit = nullptr; a.near_stride = 0; a.near_shift = a.near_tiles = 0; a.pick_rule = fixed || whole ? 1 : h->rounds;
     a.phase_ticks = h->d_phase_ticks;
+    a.round_items = h->d_round_items;
+    a.selected = &h->route[3];
     a.stop_hint = nullptr;
     a.N = h->n;
     a.ppb = (h->n + block_size - 1) / block_size;
@@ -804,6 +809,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
                           block_size, thread_size, d_nn, d_dists, d_counters, stream, fixed, float_ids, who, true);
     }
     if (rc) return rc;
+    h->route[0] = a.pick_rounds; h->route[1] = a.pick_near; h->route[2] = a.pick_sample;
     char* base = ws_base;
     float* d_qproj = (float*)base;
     a.qproj = d_qproj;
@@ -929,6 +935,18 @@ int dcih_set_option(dcih_index* h, int option, int value) {
         return DCIH_OK;
     }
     return fail(DCIH_EINVAL, "dcih_set_option: unknown option or value");
+}
+
+int dcih_debug_route(const dcih_index* h, int64_t* route) {
+    if (!h || !route) return fail(DCIH_EINVAL, "dcih_debug_route: null argument");
+    for (int i = 0; i < 4; i++) route[i] = h->route[i];
+    return DCIH_OK;
+}
+
+int dcih_debug_round_items(dcih_index* h, uint32_t* d_items) {
+    if (!h) return fail(DCIH_EINVAL, "dcih_debug_round_items: null handle");
+    h->d_round_items = d_items;
+    return DCIH_OK;
 }
 
 int dcih_phase_profile(dcih_index* h, uint64_t* d_ticks) {

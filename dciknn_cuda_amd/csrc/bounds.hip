@@ -20,6 +20,12 @@
 // further away has those partitions taken again), later one within the k-th distance found.  512 queries on 10M unit vectors of 96: 21.4 -> 15.3 ms,
 // 500 on 1M rows of 960 3.2 -> 2.6.
 //
+// Traversals that stop after a small part of a partition may find rows that lie further away than most partitions' bounds: then everything is
+// traversed all the same, in rounds that each wait for their slowest item, behind bounds that ruled nothing out.  Whether that is so depends
+// on the rows.  So such a call first traverses all partitions of a few of its queries, compares their results with bounds of a
+// few partitions, and where these rule out too little for rounds to pay takes everything at once, without the other bounds
+// (sample_decide_kernel; the device's own decision, nobody waits for it).
+//
 // The bound.  Rows and queries, less a common centre, are rounded to 16-bit floats x', q' (scaled by powers of two, so that
 // nothing overflows; what does, or is not finite, has an unbounded error).  |x - q| >= |x' - q'| - |x - x'| - |q - q'|,
 // the two errors being summed where the rounding is done, and |x' - q'|^2 = |x'|^2 + |q'|^2 - 2 x'.q' comes
@@ -102,7 +108,7 @@ __global__ __launch_bounds__(kPackThreads) void pack_queries_kernel(PackArgs a) 
 
 struct BoundArgs {
     const float* data;
-    int64_t n, ppb;
+    int64_t n, ppb, step;                 // step: rows from a partition to the next one taken (ppb, or more for a sample of them)
     int dim, steps, nq, tiles;
     int column_steps;                     // staged at a time (even)
     int next_part, next_tile;             // from a workgroup's row tile to its next one
@@ -110,6 +116,7 @@ struct BoundArgs {
     const Header* header; const float2* qinfo; const _Float16* frags;
     uint32_t* bounds;                     // [B * parts][nq] float bits
     uint32_t* tile_bounds;                // null, or the same of every near_rows(RT) rows
+    const uint32_t* skip;                 // null, or where it says so nothing is formed
 };
 
 // The rows a near tile holds: one wavefront's, 64 at least.
@@ -141,7 +148,7 @@ struct BoundTile {
 
     // Row tile rt of partition b.
     __device__ __forceinline__ void take(int b, int rt) {
-        const int64_t off = (int64_t)b * a.ppb, first = off + (int64_t)rt * R;
+        const int64_t off = (int64_t)b * a.step, first = off + (int64_t)rt * R;
         rows = (int)min((int64_t)R, min(a.n, off + a.ppb) - first);
         base = a.data + first * a.dim;
         out = a.bounds + ((int64_t)b * a.parts + rt * a.parts / a.row_tiles) * a.nq;
@@ -330,6 +337,7 @@ __global__ __launch_bounds__(64 * WC, WAVES) void bounds_resident_kernel(BoundAr
     float* s_red = s_n + Tile::R;
     float* s_centre = s_red + 2 * Tile::kWaves;
     v8h* s_rows = reinterpret_cast<v8h*>(s_centre + a.steps * kStep);
+    if (a.skip && *a.skip) return;
     Tile y(a);
     y.take((int)(blockIdx.x / (unsigned)a.row_tiles), (int)(blockIdx.x % (unsigned)a.row_tiles));
     if (y.rows <= 0) return;
@@ -383,6 +391,7 @@ __global__ __launch_bounds__(128 * WR * WC, WAVES) void bounds_stream_kernel(Bou
     float* s_red = s_n + 2 * Tile::R;                         // [2][2 * kWaves]
     float* s_centre = s_red + 4 * Tile::kWaves;
     v8h* s_rows = reinterpret_cast<v8h*>(s_centre + a.steps * kStep);
+    if (a.skip && *a.skip) return;
     Tile y(a);
     y.copy_centre(s_centre);
     int b = (int)(blockIdx.x / (unsigned)a.row_tiles), rt = (int)(blockIdx.x % (unsigned)a.row_tiles);
@@ -548,13 +557,14 @@ __global__ __launch_bounds__(256) void pick_limits_kernel(const uint32_t* __rest
 // which workgroups came to reserve their places, a die's 832 items of 17242 points were of five partitions, and took twice as long.)
 // One workgroup per kListQueries queries of a partition; the first launch counts, the second adds up the counts before its own.
 struct ListArgs {
-    const uint32_t* bounds; const uint32_t* limits;
+    const uint32_t* bounds; const uint32_t* limits; const uint32_t* skip;
     const float* worst; int64_t worst_stride;      // the k-th distance each query has so far
     uint32_t* last_round;                          // the round that last took a partition of the query
     int B, parts, nq, groups, round, rounds, near;
     int32_t* items; uint32_t* count; uint32_t* part_counts;
 };
 __device__ inline bool takes_item(const ListArgs& a, int b, int q) {
+    if (a.skip && *a.skip) return a.round == 0;
     uint32_t v = a.bounds[(int64_t)b * a.parts * a.nq + q];
     for (int p = 1; p < a.parts; p++) v = min(v, a.bounds[((int64_t)b * a.parts + p) * a.nq + q]);
     // a round takes what lies between two limits, the last one everything above the last limit
@@ -617,9 +627,56 @@ Shape shape_of(const QueryArgs& a) {
     return {4, 2, 1, 4, false, true};
 }
 
+// The sample of a call's queries: every (nq / S)-th, and all their partitions as a round's items, by partition, then query.
+__device__ inline int sample_query(int s, int S, int nq) { return (int)((int64_t)nq * s / S); }
+__global__ __launch_bounds__(256) void sample_items_kernel(const float* __restrict__ query, int nq, int dim, int B, int S, float* __restrict__ rows,
+                                                           int32_t* __restrict__ items, uint32_t* __restrict__ count, uint32_t* __restrict__ last_round) {
+    const int at = blockIdx.x * 256 + threadIdx.x, all = gridDim.x * 256;
+    for (int e = at; e < S * dim; e += all) rows[e] = query[(int64_t)sample_query(e / dim, S, nq) * dim + e % dim];
+    for (int e = at; e < S * B; e += all) items[e] = sample_query(e % S, S, nq) * B + e / S;
+    // (nearest query of the sample from below, and whether it is this one)
+    for (int q = at; q < nq; q += all) {
+        const int s = (int)(((int64_t)q * S + S - 1) / nq);
+        last_round[q] = s < S && sample_query(s, S, nq) == q ? kSampleRound : 0u;
+    }
+    if (at == 0) *count = (uint32_t)(S * B);
+}
+// Whether more than `most` of the sample's (query, partition) pairs have bounds within the query's k-th result.
+__global__ __launch_bounds__(256) void sample_decide_kernel(const uint32_t* __restrict__ bounds, int S, int nq, int B, int parts, const float* __restrict__ worst,
+                                                            int64_t worst_stride, float most, uint32_t* __restrict__ skip) {
+    __shared__ uint32_t s_need;
+    if (threadIdx.x == 0) s_need = 0;
+    __syncthreads();
+    uint32_t need = 0;
+    for (int e = threadIdx.x; e < B * S; e += 256) {
+        const int b = e / S, s = e % S;
+        uint32_t v = kInf;
+        for (int p = 0; p < parts; p++) v = min(v, bounds[((int64_t)b * parts + p) * S + s]);
+        need += __builtin_bit_cast(float, v) > worst[(int64_t)sample_query(s, S, nq) * worst_stride] ? 0u : 1u;
+    }
+    need = wave_sum_u32(need);
+    if ((threadIdx.x & 63) == 0) atomicAdd(&s_need, need);
+    __syncthreads();
+    if (threadIdx.x == 0) { skip[0] = (float)s_need > most * (float)(B * S) ? 1u : 0u; skip[1] = s_need; }
+}
+
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
-struct Room { size_t header, counts, qinfo, frags, bounds, limits, last, items, part_counts, near, total; int steps, tiles, parts; };
+struct Room { size_t header, counts, qinfo, frags, bounds, limits, last, items, part_counts, near, sample, sample_rows, total; int steps, tiles, parts; };
+// The sample as a call of its own, over every (B / kSampleParts)-th partition.
+constexpr int kSampleParts = 12;
+int sample_stride(const QueryArgs& a) { return a.B / min(a.B, kSampleParts); }
+QueryArgs sample_call(const QueryArgs& a, const float* rows) {
+    QueryArgs c = a;
+    c.query = rows;
+    c.nq = a.pick_sample;
+    c.B = (a.B + sample_stride(a) - 1) / sample_stride(a);
+    c.k = 1;
+    c.kcap = 0;                           // (nothing of it is kept, so nothing to clear)
+    c.part = nullptr;
+    c.pick_sample = c.pick_near = 0;
+    return c;
+}
 Room room_of(const QueryArgs& a) {
     Room r;
     r.steps = (a.dim + 2 * kStep - 1) / (2 * kStep) * 2;       // an even number of them
@@ -641,6 +698,11 @@ Room room_of(const QueryArgs& a) {
     r.items = o;  o += align256((size_t)a.nq * a.B * 4);
     r.part_counts = o; o += align256((size_t)a.B * ((a.nq + kListQueries - 1) / kListQueries) * 4);
     r.near = o;   o += a.pick_near ? align256(near_bytes(a)) : 0;
+    r.sample = r.sample_rows = o;
+    if (a.pick_sample) {
+        o += room_of(sample_call(a, nullptr)).total;
+        r.sample_rows = o; o += align256((size_t)a.pick_sample * a.dim * 4);
+    }
     r.total = o;
     return r;
 }
@@ -717,10 +779,10 @@ static int launch_stream(const BoundArgs& p, int xcds, hipStream_t s) {
     return 0;
 }
 
-static int products(const QueryArgs& a, const Room& r, char* ws, hipStream_t s) {
-    BoundArgs p{a.data, a.N, a.ppb, a.dim, r.steps, a.nq, r.tiles, 0, 0, 0, a.B, 0, r.parts,
+static int products(const QueryArgs& a, const Room& r, char* ws, int64_t step, const uint32_t* skip, hipStream_t s) {
+    BoundArgs p{a.data, a.N, a.ppb, step, a.dim, r.steps, a.nq, r.tiles, 0, 0, 0, a.B, 0, r.parts,
                 (const Header*)(ws + r.header), (const float2*)(ws + r.qinfo), (const _Float16*)(ws + r.frags),
-                (uint32_t*)(ws + r.bounds), a.pick_near ? (uint32_t*)(ws + r.near) : nullptr};
+                (uint32_t*)(ws + r.bounds), a.pick_near ? (uint32_t*)(ws + r.near) : nullptr, skip};
     const Shape y = shape_of(a);
     if (!y.stream) {
         constexpr int R = 128;
@@ -754,10 +816,38 @@ static int products(const QueryArgs& a, const Room& r, char* ws, hipStream_t s) 
     return columns <= 128 ? launch_stream<4, 2, 1, 4, 128, 2, true>(p, a.xcds, s) : launch_stream<4, 2, 1, 4, 256, 2, true>(p, a.xcds, s);
 }
 
-int partition_bounds(const QueryArgs& a, void* ws, hipStream_t s) {
+int pack_bounds(const QueryArgs& a, void* ws, hipStream_t s) { return pack(a, room_of(a), (char*)ws, s); }
+
+int partition_bounds(const QueryArgs& a, void* ws_, hipStream_t s) {
+    char* ws = (char*)ws_;
     const Room r = room_of(a);
-    const int rc = pack(a, r, (char*)ws, s);
-    return rc ? rc : products(a, r, (char*)ws, s);
+    return products(a, r, ws, a.ppb, a.pick_sample ? (const uint32_t*)(ws + r.counts) + kSkipWord : nullptr, s);
+}
+
+int sample_items(const QueryArgs& a, void* ws_, Picked& p, hipStream_t s) {
+    char* ws = (char*)ws_;
+    const Room r = room_of(a);
+    uint32_t* count = (uint32_t*)(ws + r.counts) + kSampleWord;
+    hipLaunchKernelGGL(sample_items_kernel, dim3(32), dim3(256), 0, s, a.query, a.nq, a.dim, a.B, a.pick_sample, (float*)(ws + r.sample_rows),
+                       (int32_t*)(ws + r.items), count, (uint32_t*)(ws + r.last));
+    DCIH_HIP(hipGetLastError());
+    p = Picked{(const int32_t*)(ws + r.items), count, (const uint32_t*)(ws + r.last), nullptr, nullptr, 0, 0, 0};
+    return 0;
+}
+
+int sample_decide(const QueryArgs& a, void* ws_, hipStream_t s) {
+    char* ws = (char*)ws_;
+    const Room r = room_of(a);
+    const QueryArgs c = sample_call(a, (const float*)(ws + r.sample_rows));
+    const Room rc_room = room_of(c);
+    char* ws_c = ws + r.sample;
+    int rc = pack(c, rc_room, ws_c, s);
+    if (!rc) rc = products(c, rc_room, ws_c, (int64_t)sample_stride(a) * a.ppb, nullptr, s);
+    if (rc) return rc;
+    hipLaunchKernelGGL(sample_decide_kernel, dim3(1), dim3(256), 0, s, (const uint32_t*)(ws_c + rc_room.bounds), c.nq, a.nq, c.B, rc_room.parts,
+                       (const float*)a.out_dists + (a.k - 1), (int64_t)a.k, a.pick_most, (uint32_t*)(ws + r.counts) + kSkipWord);
+    DCIH_HIP(hipGetLastError());
+    return 0;
 }
 
 int pick_items(const QueryArgs& a, void* ws_, int round, int rounds, hipStream_t s) {
@@ -778,7 +868,7 @@ int pick_items(const QueryArgs& a, void* ws_, int round, int rounds, hipStream_t
         DCIH_HIP(hipGetLastError());
     }
     const int groups = (a.nq + kListQueries - 1) / kListQueries;
-    ListArgs p{bounds, limits, a.out_dists + (a.k - 1), a.k, last, a.B, r.parts, a.nq, groups, round, rounds, a.pick_near,
+    ListArgs p{bounds, limits, a.pick_sample ? (const uint32_t*)(ws + r.counts) + kSkipWord : nullptr, a.out_dists + (a.k - 1), a.k, last, a.B, r.parts, a.nq, groups, round, rounds, a.pick_near,
                (int32_t*)(ws + r.items), (uint32_t*)(ws + r.counts) + round, (uint32_t*)(ws + r.part_counts)};
     const dim3 grid((unsigned)((int64_t)a.B * groups));
     hipLaunchKernelGGL(list_items_kernel<true>, grid, dim3(256), 0, s, p);

@@ -755,6 +755,7 @@ int query_exhaustive(const QueryArgs& a, void* ws, int chunk, hipStream_t s) {
         if (a.pick_rule != 1 && nearest_supported(a.N, a.dim, a.k) && (a.pick_rule == 2 || nearest_pays(a.N, a.dim, nqc))) {
             const int rc = query_nearest(a, q0, nqc, d_dist, (float*)((char*)ws + align256((size_t)chunk * (size_t)a.N * 4)), s);
             if (rc) return rc;
+            if (a.selected) *a.selected += nqc;
             continue;
         }
         // as many queries per wavefront as leave a wavefront to every SIMD (a row is read once for all of them)

@@ -107,6 +107,9 @@ struct QueryArgs {
     // a call in rounds (bounds.hip)
     const int32_t* picked;   // null = all nq * B items, else the round's, of which every die takes one run
     const uint32_t* picked_count;
+    uint32_t* round_items;   // null, or device words for the number of items of every round, then the sample's decision
+    int64_t* selected;       // (host) counts the queries that nearest.hip answers
+    int picked_exact;        // 1: picked_expect is their number
     int64_t picked_expect;   // about how many there are
     int64_t picked_cover;    // ... and how many there seldom are more of: what a launch of one workgroup per item covers
     const uint32_t* only;    // merge: null, or only the queries whose word here is only_round
@@ -118,6 +121,8 @@ struct QueryArgs {
     int64_t near_stride;
     int near_shift, near_tiles;
     int pick_near;           // 1: a call in rounds goes to the dense kernel and keeps those bounds
+    int pick_sample;         // 0, or: so many queries are traversed whole first, and decide
+    float pick_most;         // share of pairs that rounds may have to take: where the sample's bounds leave more, everything is taken at once
     int pick_rounds;         // 0: everything is traversed at once
     int pick_rank;           // the first round takes the partitions of so many nearest rows
     int pick_rule;           // DCIH_OPT_ROUNDS value
@@ -242,9 +247,11 @@ __device__ inline int64_t picked_run(const uint32_t* d_count, int x, int X, int6
     return min(each, max((int64_t)0, count - first));
 }
 // Calls in rounds (bounds.hip): lower bounds of every (query, partition)'s nearest distance, and the items each
-// round takes.  Scratch of bounds_bytes(); bounds_cost: about how long the bounds take, us.  partition_bounds also
-// clears a.part.
+// round takes.  Scratch of bounds_bytes(); bounds_cost: about how long the bounds take, us.  pack_bounds
+// comes first and also clears a.part.
 constexpr int kPickCountWords = 64, kMostRounds = 4;
+constexpr int kSampleWord = 8, kSkipWord = 9;      // of the count words: the sample's items, whether rounds are skipped, and the pairs that says so by
+constexpr uint32_t kSampleRound = 0x10000;         // of the sample's queries while their results are merged
 struct Picked {
     const int32_t* items; const uint32_t* count; const uint32_t* last_round;
     const uint32_t* near_bounds; const float* near_limit; int64_t near_stride; int near_shift, near_tiles;
@@ -253,7 +260,12 @@ bool bounds_supported(const QueryArgs& a);
 size_t bounds_bytes(const QueryArgs& a);
 size_t near_bytes(const QueryArgs& a);      // the part of it that pick_near adds
 double bounds_cost(const QueryArgs& a);
+int pack_bounds(const QueryArgs& a, void* ws, hipStream_t s);
 int partition_bounds(const QueryArgs& a, void* ws, hipStream_t s);
+// Where a.pick_sample is set, after pack_bounds: all items of that many queries, and, once they are traversed and merged, whether the
+// bounds are formed at all (else everything comes in round 1).
+int sample_items(const QueryArgs& a, void* ws, Picked& p, hipStream_t s);
+int sample_decide(const QueryArgs& a, void* ws, hipStream_t s);
 int pick_items(const QueryArgs& a, void* ws, int round, int rounds, hipStream_t s);
 Picked picked_items(const QueryArgs& a, void* ws, int round);
 // Whether a call is worth its rounds; sets a.pick_rounds, a.pick_first and a.share.

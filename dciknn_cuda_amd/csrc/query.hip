@@ -458,7 +458,7 @@ bool takes_dense_kernel(const QueryArgs& a) {
 }
 
 bool plan_rounds(QueryArgs& a) {
-    a.pick_rounds = a.pick_near = 0;
+    a.pick_rounds = a.pick_near = a.pick_sample = 0;
     a.share = 1.0;
     if (a.mode != 0 || a.pick_rule == 1 || !bounds_supported(a)) return false;
     // The r nearest rows of a query lie in about B (1 - e^(-r/B)) partitions (rows in no particular order).  Round 1
@@ -487,17 +487,29 @@ bool plan_rounds(QueryArgs& a) {
     // distances lie close together, and every partition is traversed after all.  Such queries then take all in one round (unit vectors
     // of 241 elements, 42 partitions, 985 queries: 0.95 ms whole, 2.2 in rounds, 1.03 so), and rounds have to promise more.
     const bool short_stops = expected_promotions(a) < 0.02 * (double)a.ppb;
+    // Traversals that stop after less than a twentieth of their partition (and those of the batch kernel) may find too little for bounds to rule
+    // anything out; a sample of the queries says so (bounds.hip).  That takes as long as an item does, and each round waits for its
+    // slowest item too, so calls of less than 25 times that are traversed whole.  (1215 shapes: without this rule and the sample 110 took more than
+    // 3 % longer than whole, up to five times as long; with them the sample costs what takes everything 2 to 7 %.)
+    const bool by_batch = !(can_dense && takes_dense_kernel(a));
+    const bool sampled = by_batch || expected_promotions(a) < 0.05 * (double)a.ppb;
+    if (sampled && a.pick_rule == 0 && whole < 25.0 * time(1.0 / ((double)a.nq * B))) return false;
     if (!fits || (a.pick_rule == 0 && rounds > (short_stops ? 0.6 : 0.85) * whole)) return false;
     // One to three results of traversals that leave out near rows bound little: everything else follows in the later rounds (32 queries, 64
     // partitions of 8000 normal rows of 32, k = 3: 539 us whole, 710 in rounds; of 6000, k = 1: 378, 415; k = 10: 401, 229), and calls of
     // one item for every workgroup gain less than that costs (14 queries, 64 partitions of 4000, k = 1: 155, 193; 32 queries: 295, 189).
     if (a.pick_rule == 0 && a.k < 4 && (whole < 250.0 || expected_promotions(a) < 0.3 * (double)a.ppb)) return false;
     a.pick_flat = short_stops ? 1.3f : 0.0f;
-    a.pick_rounds = few ? 2 : (whole > 1500.0 || a.pick_rule == 2 ? kMostRounds : 2);
+    a.pick_rounds = few ? 2 : (whole > 1500.0 || a.pick_rule == 2 ? (by_batch ? 3 : kMostRounds) : 2);
     a.pick_rank = rank;
     a.pick_first = first;
     a.share = share;
-    a.pick_near = can_dense && takes_dense_kernel(a) && near_bytes(a) <= ((size_t)1 << 30) ? 1 : 0;
+    a.pick_near = !sampled && near_bytes(a) <= ((size_t)1 << 30) ? 1 : 0;
+    a.pick_sample = sampled ? std::min(a.nq, std::max(2, std::min(16, 1024 / a.B))) : 0;
+    // Up to which share of the sample's pairs rounds pay: the fewer results, the further away the k-th of the first rounds lies than
+    // that of all.  (Five kinds of rows, 16 to 300 elements, 30000 to a million: shares from which rounds begin to take longer are 0.31 to
+    // 0.37 for 5 results, 0.39 to 0.51 for 10 and 0.75 for 30; all of them at a share of 0.7, 10 results: 0.69 to 0.94 of whole calls' rate.)
+    a.pick_most = a.pick_rule == 2 ? 2.0f : (float)(0.75 * (double)a.k / ((double)a.k + 7.5));
     return true;
 }
 
@@ -619,7 +631,26 @@ int query(const QueryArgs& a_in, void* bounds_ws, hipStream_t s, hipEvent_t* ev,
         const int rc = traverse(a);
         if (rc) return rc;
     } else {      // rounds (bounds.hip): the results of one bound what the next has to take
-        int rc = partition_bounds(a, bounds_ws, s);
+        int rc = pack_bounds(a, bounds_ws, s);
+        if (a.pick_sample && !rc) {
+            Picked p;
+            rc = sample_items(a, bounds_ws, p, s);
+            if (rc) return rc;
+            a.picked = p.items;
+            a.picked_count = p.count;
+            a.picked_expect = a.picked_cover = (int64_t)a.pick_sample * a.B;
+            a.picked_exact = 1;
+            rc = traverse(a);
+            a.only = p.last_round;
+            a.only_round = kSampleRound;
+            if (!rc) rc = merge_lists(a, s);
+            if (!rc) rc = sample_decide(a, bounds_ws, s);
+            if (a.round_items && !rc)
+                DCIH_HIP(hipMemcpyAsync(a.round_items + kMostRounds, p.count + (kSkipWord - kSampleWord), 2 * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
+            a.picked_exact = 0;
+            a.only = nullptr;
+        }
+        if (!rc) rc = partition_bounds(a, bounds_ws, s);
         const double all = (double)a.nq * (double)a.B * a.share, first = (double)a.nq * a.pick_first;
         for (int round = 0; round < a.pick_rounds && !rc; round++) {
             if (round > 0) rc = merge_lists(a, s);
@@ -627,6 +658,7 @@ int query(const QueryArgs& a_in, void* bounds_ws, hipStream_t s, hipEvent_t* ev,
             const Picked p = picked_items(a, bounds_ws, round);
             a.picked = p.items;
             a.picked_count = p.count;
+            if (a.round_items && !rc) DCIH_HIP(hipMemcpyAsync(a.round_items + round, p.count, sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
             a.near_bounds = p.near_bounds; a.near_limit = p.near_limit; a.near_stride = p.near_stride;
             a.near_shift = p.near_shift; a.near_tiles = p.near_tiles;
             a.picked_expect = (int64_t)fmax(round ? all - first : first, 1.0);

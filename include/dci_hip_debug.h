@@ -50,6 +50,21 @@ int64_t dcih_debug_launch_map(int xcds, int block_size, int num_queries, int64_t
  */
 int dcih_debug_positions(dcih_index* h, uint16_t* d_inv, uint16_t* d_rpos, void* stream);
 
+/*
+ * What the handle's last dcih_query took (no counterpart in the reference): route receives
+ * [0] its rounds (0: everything was traversed at once, or nothing was), [1] whether bounds of
+ * tiles of rows were kept for the dense kernel, [2] the queries that were traversed whole first
+ * to decide about rounds, [3] the queries whose results were selected by bounds of all rows.
+ */
+int dcih_debug_route(const dcih_index* h, int64_t* route);
+/*
+ * d_items is NULL (off) or a device array of 6 uint32 to which later queries in rounds write
+ * the number of (query, partition) pairs of each round, then, where some queries decided about
+ * the rounds, whether everything was taken at once and how many of the pairs they looked at
+ * could not be ruled out.
+ */
+int dcih_debug_round_items(dcih_index* h, uint32_t* d_items);
+
 #ifdef __cplusplus
 }
 #endif

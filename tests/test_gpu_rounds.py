@@ -19,12 +19,32 @@ def _ask(dci, lib, rounds, Q, k, outer, **kw):
     return ids.clone(), dists.clone()
 
 
-def _same(gpu, X, Q, M, L, B, T, k, outer, tag=""):
+def _route(dci):
+    """(rounds, bounds of tiles kept, queries of the sample, queries selected by bounds of all rows) of the last call."""
+    from dciknn_cuda_amd import _capi
+    route = (_capi.ctypes.c_int64 * 4)()
+    _capi.check(dci._lib.dcih_debug_route(dci._dci_inst, route))
+    return tuple(route)
+
+
+def _count_items(dci):
+    """A tensor that later calls write the items of every round to, then what the sample decided."""
+    from dciknn_cuda_amd import _capi
+    items = torch.zeros(6, dtype=torch.int32, device="cuda")
+    _capi.check(dci._lib.dcih_debug_round_items(dci._dci_inst, items.data_ptr()))
+    return items
+
+
+def _same(gpu, X, Q, M, L, B, T, k, outer, tag="", near=None):
     dci = gpu.DCI(X.shape[1], M, L, B, T, seed=3)
     dci.add(X)
     want = _ask(dci, dci._lib, NEVER, Q, k, outer)
+    assert _route(dci) == (0, 0, 0, 0), tag
     got = _ask(dci, dci._lib, ALWAYS, Q, k, outer)
+    route = _route(dci)
     dci.free()
+    assert route[0] >= 2 or route[3] == len(Q), (tag, route)      # the call did go in rounds (or its results were selected)
+    assert near is None or route[1] == near, (tag, route)
     assert torch.equal(got[0], want[0]), tag
     assert torch.equal(got[1].view(torch.int32), want[1].view(torch.int32)), tag
     return want
@@ -101,6 +121,51 @@ def test_rows_off_their_boundaries(gpu):
     q.copy_(Q)
     assert x.data_ptr() % 16 == 4 and q.data_ptr() % 16 == 4
     _same(gpu, x, q, 2, 7, 20, 10, 10, 500)
+
+
+# Traversals of a small part of their partitions: a sample of the queries decides whether bounds are formed at all.  Rows that bounds tell
+# apart and rows that they do not, more queries than the sample and as many, partitions by the dozen and a few.
+@pytest.mark.parametrize("kind,dim,outcome", [("normal", 8, 0), ("grid", 64, 1), ("normal", 64, None), ("broken", 16, None)])
+def test_a_sample_decides_about_rounds(gpu, kind, dim, outcome):
+    n, nq, B, T, k, outer = 30000, 4000, 58, 2, 5, 100
+    X, Q = _rows(kind, n, nq, dim, 8)
+    dci = gpu.DCI(dim, 2, 10, B, T, seed=3)
+    dci.add(X)
+    want = _ask(dci, dci._lib, NEVER, Q, k, outer)
+    items = _count_items(dci)
+    got = _ask(dci, dci._lib, 0, Q, k, outer)
+    assert _route(dci) == (3, 0, 16, 0)
+    items = items.tolist()
+    dci.free()
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1].view(torch.int32), want[1].view(torch.int32))
+    assert outcome is None or items[4] == outcome, items
+    if items[4]:
+        assert items[:3] == [nq * B, 0, 0], items
+    else:
+        assert 0 < items[0] < nq * B // 2 and items[5] < 16 * 15, items
+
+
+@pytest.mark.parametrize("nq", [1, 2, 15, 16, 17, 31, 100])
+@pytest.mark.parametrize("B", [2, 11, 12, 13, 25, 300])
+def test_samples_of_few_queries_and_partitions(gpu, nq, B):
+    X, Q = _rows("clusters", 40 * B + 7, nq, 19, nq + B)
+    _same(gpu, X, Q, 2, 6, B, 2, 2, 6, "nq %d B %d" % (nq, B))
+
+
+@pytest.mark.parametrize("kind,dim,k,T,outer", [("normal", 64, 5, 2, 100), ("clusters", 64, 3, 2, 30)])
+def test_more_items_in_a_later_round_than_its_launch_covers(gpu, kind, dim, k, T, outer):
+    """A launch of the batch kernel in a later round covers three tenths of all items, 65536 at least."""
+    n, nq, B = 30000, 4000, 58
+    X, Q = _rows(kind, n, nq, dim, 8)
+    dci = gpu.DCI(dim, 2, 10, B, T, seed=3)
+    dci.add(X)
+    want = _ask(dci, dci._lib, NEVER, Q, k, outer)
+    items = _count_items(dci)
+    got = _ask(dci, dci._lib, ALWAYS, Q, k, outer)
+    items = items.tolist()
+    dci.free()
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1].view(torch.int32), want[1].view(torch.int32))
+    assert kind != "normal" or max(items[1:3]) > 0.3 * nq * B, items
 
 
 def test_rounds_run_the_kernel_of_whole_calls(gpu):
