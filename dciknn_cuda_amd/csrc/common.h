@@ -323,6 +323,33 @@ __device__ __forceinline__ void bitonic_sort_u64_by(unsigned long long* s, int n
     bitonic_sort_u64(s, n, tid);
 }
 __device__ inline void bitonic_sort_u64_by256(unsigned long long* s, int n) { bitonic_sort_u64_by<256, 4>(s, n, (int)threadIdx.x); }
+// The k <= 512 smallest of `total` entries, ascending, to buf[0, k) of 1024 words, by 256 threads: `chunk(first, n)` puts n of them, 256 at most,
+// to buf[768, ...).  What is not below the k-th smallest of those seen at the last sort is dropped, so sorts are few unless the entries descend.
+constexpr int kKeepChunk = 256, kKeepRoom = 1024, kKeepAt = kKeepRoom - kKeepChunk;
+template <class Chunk>
+__device__ __forceinline__ void keep_smallest(unsigned long long* buf, uint32_t& s_count, int64_t total, int k, Chunk chunk) {
+    const int tid = threadIdx.x;
+    unsigned long long below = ~0ull;
+    __syncthreads();
+    if (tid == 0) s_count = 0;
+    for (int64_t first = 0; first < total; first += kKeepChunk) {
+        const int n = (int)min((int64_t)kKeepChunk, total - first);
+        chunk(first, n);
+        __syncthreads();
+        const unsigned long long e = tid < n ? buf[kKeepAt + tid] : ~0ull;
+        if (e < below) buf[atomicAdd(&s_count, 1u)] = e;
+        __syncthreads();
+        const int have = (int)s_count;
+        if (have > kKeepAt - kKeepChunk || first + kKeepChunk >= total) {      // no room for another chunk, or done
+            for (int j = have + tid; j < kKeepRoom; j += kKeepChunk) buf[j] = ~0ull;
+            bitonic_sort_u64_by256(buf, kKeepRoom);
+            __syncthreads();
+            below = buf[k - 1];
+            if (tid == 0) s_count = (uint32_t)min(have, k);
+            __syncthreads();
+        }
+    }
+}
 #endif
 
 }  // namespace dcih

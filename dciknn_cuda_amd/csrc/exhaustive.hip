@@ -13,6 +13,8 @@
 // columns copied out.  The traversal counters have closed forms too: every
 // index entry is visited once, every point is a candidate, and the outer steps
 // follow from the window counts on either side of the positioning search.
+#include <type_traits>
+
 #include "bucket_core.h"
 #include "common.h"
 #include "kernels.h"
@@ -44,22 +46,10 @@ typedef const __attribute__((address_space(4))) v4f_any cv4f;
 // wavefront where rows and queries are few.  (500 queries, 3000 rows of 100:
 // 86 us before, 22 now; 4000 queries, 9582 rows: 440 us with the queries read where they are used, 364 ahead.)
 template <int QN>
-__global__ __launch_bounds__(kExRows) void exact_dists_kernel(
-    const float* __restrict__ data, int64_t N, int dim, const float* __restrict__ query, int nq,
-    float* __restrict__ out) {
+__device__ __forceinline__ void exact_tile(float* tile, const float* __restrict__ data, int64_t N, int dim, int64_t row0, int lane,
+                                           const cfloat* (&qv)[QN], float (&acc)[QN]) {
 #pragma clang fp contract(off)     // no fused multiply-add: product and sum are rounded separately
-    __shared__ float tile[kExRows * kExPitch];
     constexpr int kTpr = kExCols / 4, kLoads = kTpr;      // lanes per row; 16-byte reads per lane and chunk
-    const int lane = threadIdx.x;
-    const int64_t row0 = (int64_t)blockIdx.x * kExRows;
-    const int q0 = blockIdx.y * QN;
-    float acc[QN];
-    const cfloat* qv[QN];             // wave-uniform: read through the scalar cache
-#pragma unroll
-    for (int j = 0; j < QN; j++) {
-        acc[j] = 0.0f;
-        qv[j] = (const cfloat*)(uintptr_t)(query + (int64_t)min(q0 + j, nq - 1) * dim);
-    }
     const int kq = (lane % kTpr) * 4, r_in = lane / kTpr;
     v4f pre[kLoads];
     auto prefetch = [&](int k0) {      // (past the last row: that row again; past the row's end: its last 16 bytes)
@@ -143,6 +133,23 @@ __global__ __launch_bounds__(kExRows) void exact_dists_kernel(
             }
         }
     }
+}
+template <int QN>
+__global__ __launch_bounds__(kExRows) void exact_dists_kernel(
+    const float* __restrict__ data, int64_t N, int dim, const float* __restrict__ query, int nq,
+    float* __restrict__ out) {
+    __shared__ float tile[kExRows * kExPitch];
+    const int lane = threadIdx.x;
+    const int64_t row0 = (int64_t)blockIdx.x * kExRows;
+    const int q0 = blockIdx.y * QN;
+    float acc[QN];
+    const cfloat* qv[QN];             // wave-uniform: read through the scalar cache
+#pragma unroll
+    for (int j = 0; j < QN; j++) {
+        acc[j] = 0.0f;
+        qv[j] = (const cfloat*)(uintptr_t)(query + (int64_t)min(q0 + j, nq - 1) * dim);
+    }
+    exact_tile<QN>(tile, data, N, dim, row0, lane, qv, acc);
     const int64_t row = row0 + lane;
     if (row >= N) return;
 #pragma unroll
@@ -159,17 +166,8 @@ __global__ __launch_bounds__(kExRows) void exact_dists_kernel(
 // more) is sorted.  (Sorting the whole row of 3000: 32 us for 500 queries, and 5 us to cut it.)
 constexpr int kSelThreads = 256, kSelItems = 16, kSelLen = kSelThreads * kSelItems, kSelCap = 2048;
 constexpr int kSelMaxK = kSelThreads;
-__global__ __launch_bounds__(kSelThreads) void select_rows_kernel(const float* __restrict__ dists, int64_t N, int len,
-                                                                  int kc, unsigned long long* __restrict__ part,
-                                                                  int32_t* __restrict__ out_ids, float* __restrict__ out_dists,
-                                                                  int float_ids) {
-    __shared__ unsigned long long buf[kSelCap];
-    __shared__ uint32_t s_count;
+__device__ __forceinline__ void select_piece(unsigned long long* buf, uint32_t& s_count, const float* row, int n, int kc) {
     const int tid = threadIdx.x;
-    const int64_t first = (int64_t)blockIdx.x * len;
-    const int n = (int)min((int64_t)len, N - first);
-    const float* row = dists + (int64_t)blockIdx.y * N + first;
-    unsigned long long* out = part + ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * kc;
     uint32_t v[kSelItems];       // (distances are not negative: their bits order as they do)
     uint32_t least = 0xffffffffu;
     int at = 0;
@@ -223,6 +221,18 @@ __global__ __launch_bounds__(kSelThreads) void select_rows_kernel(const float* _
         for (int j = count + tid; j < np; j += kSelThreads) buf[j] = ~0ull;
         if (np >= kSelThreads) bitonic_sort_u64_by256(buf, np); else bitonic_sort_u64(buf, np);
     }
+}
+__global__ __launch_bounds__(kSelThreads) void select_rows_kernel(const float* __restrict__ dists, int64_t N, int len,
+                                                                  int kc, unsigned long long* __restrict__ part,
+                                                                  int32_t* __restrict__ out_ids, float* __restrict__ out_dists,
+                                                                  int float_ids) {
+    __shared__ unsigned long long buf[kSelCap];
+    __shared__ uint32_t s_count;
+    const int tid = threadIdx.x;
+    const int64_t first = (int64_t)blockIdx.x * len;
+    const int n = (int)min((int64_t)len, N - first);
+    unsigned long long* out = part + ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * kc;
+    select_piece(buf, s_count, dists + (int64_t)blockIdx.y * N + first, n, kc);
     for (int j = tid; j < kc; j += kSelThreads) {
         const unsigned long long e = buf[j];
         if (out_ids) {               // (the only piece of the row, and kc = k: these are the results)
@@ -233,6 +243,80 @@ __global__ __launch_bounds__(kSelThreads) void select_rows_kernel(const float* _
         } else {
             out[j] = e == ~0ull ? e : e + (unsigned long long)first;      // (ids of the whole row; no carry into the distance)
         }
+    }
+}
+
+
+// The same for the queries of a list whose length is known on the device only (nearest.hip's, of bounds that say too little): left[0] of them, their
+// numbers, and a counter for every eight, zero.  A workgroup takes a piece of the rows and eight queries, forms their distances into `rows`, selects the
+// piece's best, and whoever finishes a query's last piece merges them.  (200 queries, 200000 rows of 64, one query not finite: 164 us in all, 4930 where the
+// query's workgroup went through all rows by itself; all of them: 1144, 4820; distances of all from the beginning: 300.)
+constexpr int kListed = 8, kListedLen = 2048;
+__host__ __device__ inline int listed_pieces(int64_t N) { return (int)((N + kListedLen - 1) / kListedLen); }
+__global__ __launch_bounds__(kSelThreads) void listed_rows_kernel(const float* __restrict__ data, int64_t N, int dim, const float* __restrict__ query, int nq,
+                                                                  int k, int float_ids, float* rows, unsigned long long* part,
+                                                                  uint32_t* left, int32_t* __restrict__ out_ids, float* __restrict__ out_dists) {
+    __shared__ __align__(16) float tile[kSelThreads / kWave][kExRows * kExPitch];
+    __shared__ unsigned long long buf[kSelCap];
+    __shared__ uint32_t s_count, s_last;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const uint32_t count = left[0];
+    const int pieces = listed_pieces(N);
+    const int64_t tasks = (int64_t)((count + kListed - 1) / kListed) * pieces;
+    for (int64_t t = blockIdx.x; t < tasks; t += gridDim.x) {
+        const int group = (int)(t / pieces), piece = (int)(t % pieces), here = min(kListed, (int)count - group * kListed);
+        const int64_t first = (int64_t)piece * kListedLen;
+        const int n = (int)min((int64_t)kListedLen, N - first);
+        auto distances = [&](auto qn) __attribute__((always_inline)) {
+            constexpr int QN = decltype(qn)::value;
+            int q[QN];
+            const cfloat* qv[QN];
+#pragma unroll
+            for (int j = 0; j < QN; j++) {
+                q[j] = __builtin_amdgcn_readfirstlane((int)left[1 + group * kListed + min(j, here - 1)]);
+                qv[j] = (const cfloat*)(uintptr_t)(query + (int64_t)q[j] * dim);
+            }
+            for (int i = 0; i < n; i += kSelThreads) {      // (the same number of times for every wavefront)
+                float acc[QN] = {};
+                const int64_t row0 = first + i + wave * kExRows, row = row0 + lane;
+                exact_tile<QN>(tile[wave], data, N, dim, row0, lane, qv, acc);
+#pragma unroll
+                for (int j = 0; j < QN; j++)
+                    if (j < here && row < first + n) rows[(int64_t)q[j] * N + row] = (float)sqrt((double)acc[j]);
+            }
+        };
+        if (here <= 2) distances(std::integral_constant<int, 2>()); else distances(std::integral_constant<int, kListed>());
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // (read again by this workgroup only)
+        __syncthreads();
+        for (int j = 0; j < here; j++) {
+            const int qj = (int)left[1 + group * kListed + j];
+            select_piece(buf, s_count, rows + (int64_t)qj * N + first, n, k);
+            unsigned long long* out = part + ((int64_t)(group * kListed + j) * pieces + piece) * k;
+            for (int e = tid; e < k; e += kSelThreads)
+                __hip_atomic_store(&out[e], buf[e] == ~0ull ? buf[e] : buf[e] + (unsigned long long)first, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();
+        }
+        // (The pieces of a query are of several dies.  Their entries are written and read past the dies' own caches and have arrived before they are
+        // counted; a fence would write back all of a die's cache, distances and all.)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (tid == 0) s_last = atomicAdd(&left[1 + nq + group], 1u) == (uint32_t)pieces - 1 ? 1u : 0u;
+        __syncthreads();
+        if (s_last) {
+            for (int j = 0; j < here; j++) {
+                const int64_t qj = left[1 + group * kListed + j];
+                const unsigned long long* from = part + (int64_t)(group * kListed + j) * pieces * k;
+                keep_smallest(buf, s_count, (int64_t)pieces * k, k, [&](int64_t at, int m) {
+                    if (tid < m) buf[kKeepAt + tid] = __hip_atomic_load(&from[at + tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                });
+                for (int e = tid; e < k; e += kSelThreads) {
+                    const int32_t id = (int32_t)(uint32_t)buf[e];
+                    out_ids[qj * k + e] = float_ids ? __builtin_bit_cast(int32_t, (float)id) : id;
+                    out_dists[qj * k + e] = __builtin_bit_cast(float, (uint32_t)(buf[e] >> 32));
+                }
+            }
+        }
+        __syncthreads();      // (the next task's tables)
     }
 }
 
@@ -698,11 +782,17 @@ static ExSelect exhaustive_select(int64_t N, int k) {
     return e;
 }
 
+// What is selected of every piece, or the smallest bounds of every 32 rows.
+static size_t select_bytes(int64_t N, int chunk, int k) {
+    const ExSelect e = exhaustive_select(N, k);
+    return align256(max((size_t)chunk * max((size_t)e.pieces, k <= 128 ? (size_t)listed_pieces(N) : 0) * e.kc * sizeof(unsigned long long),
+                        nearest_least_bytes(N, chunk)));
+}
+
 size_t exhaustive_ws_bytes(int64_t N, int chunk, int k) {
     const size_t cells = (size_t)chunk * (size_t)N;
     if (exhaustive_selects(k)) {
-        const ExSelect e = exhaustive_select(N, k);
-        return align256(cells * 4) + align256(max((size_t)chunk * e.pieces * e.kc * sizeof(unsigned long long), nearest_least_bytes(N, chunk)));
+        return align256(cells * 4) + select_bytes(N, chunk, k) + align256(nearest_left_bytes(chunk));
     }
     return 3 * align256(cells * 4) + align256(segsort_tmp_bytes(chunk, N, 1));
 }
@@ -753,8 +843,18 @@ int query_exhaustive(const QueryArgs& a, void* ws, int chunk, hipStream_t s) {
     for (int q0 = 0; q0 < a.nq; q0 += chunk) {
         const int nqc = min(chunk, a.nq - q0);
         if (a.pick_rule != 1 && nearest_supported(a.N, a.dim, a.k) && (a.pick_rule == 2 || nearest_pays(a.N, a.dim, nqc))) {
-            const int rc = query_nearest(a, q0, nqc, d_dist, (float*)((char*)ws + align256((size_t)chunk * (size_t)a.N * 4)), s);
+            char* rest = (char*)ws + align256((size_t)chunk * (size_t)a.N * 4);
+            uint32_t* left = (uint32_t*)(rest + select_bytes(a.N, chunk, a.k));
+            bool leaves = false;
+            const int rc = query_nearest(a, q0, nqc, d_dist, (float*)rest, left, s, leaves);
             if (rc) return rc;
+            if (leaves) {      // (as many workgroups as the device holds at a time, at most)
+                const int64_t tasks = (int64_t)((nqc + kListed - 1) / kListed) * listed_pieces(a.N);
+                hipLaunchKernelGGL(listed_rows_kernel, dim3((unsigned)min((int64_t)a.xcds * 32 * 3, tasks)), dim3(kSelThreads), 0, s, a.data, a.N, a.dim,
+                                   a.query + (int64_t)q0 * a.dim, nqc, a.k, a.float_ids, d_dist, (unsigned long long*)rest, left,
+                                   a.out_ids + (int64_t)q0 * a.k, a.out_dists + (int64_t)q0 * a.k);
+                DCIH_HIP(hipGetLastError());
+            }
             if (a.selected) *a.selected += nqc;
             continue;
         }

@@ -283,7 +283,10 @@ int query_exhaustive(const QueryArgs& a, void* ws, int chunk, hipStream_t s);
 bool nearest_supported(int64_t N, int dim, int k);
 bool nearest_pays(int64_t N, int dim, int nq);
 size_t nearest_least_bytes(int64_t N, int nq);
-int query_nearest(const QueryArgs& a, int q0, int nq, float* d_bounds, float* d_least, hipStream_t s);
+// Queries whose bounds rule out too little are left in large tables (`leaves`): d_left receives their number, then their numbers, then as many
+// words as queries that are zero.
+size_t nearest_left_bytes(int nq);
+int query_nearest(const QueryArgs& a, int q0, int nq, float* d_bounds, float* d_least, uint32_t* d_left, hipStream_t s, bool& leaves);
 // The pieces of it that the dense-row traversal (query_dense) shares: rows of N values
 // at rank_rows_input(ws), `rows` <= chunk of them; rank_rows sorts every row by (value,
 // column) and writes the first k columns (id = column, or -1 for +inf when asked).

@@ -32,7 +32,7 @@ constexpr int kNearestMaxK = 128, kNearestMaxDim = 4096;
 template <int RT, int OCT, bool OCTETS>
 __global__ __launch_bounds__(kPackThreads, 2) void bound_rows_kernel(const float* __restrict__ data, int64_t N, int dim,
                                                                   const float* __restrict__ query, int nq, float* __restrict__ out,
-                                                                  float* __restrict__ least) {
+                                                                  float* __restrict__ least, uint32_t* __restrict__ left) {
     constexpr int T = 64 * RT, kGroups = 2 * T / 32;            // groups of eight rows or queries per wavefront
     constexpr int kColumns = 64 * OCT, kSteps = kColumns / kStep;
     constexpr int kHalf = 4 * RT * kSteps * 64;
@@ -44,6 +44,8 @@ __global__ __launch_bounds__(kPackThreads, 2) void bound_rows_kernel(const float
     float* s_ulp = s_sq + 2 * T;                                // [2 T]
     float* s_centre = s_ulp + 2 * T;                            // [width]
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (left)      // what the kernels below take as cleared: the length of the list of queries, and their counters
+        for (int e = (int)blockIdx.x * kPackThreads + tid; e <= nq; e += (int)gridDim.x * kPackThreads) left[e ? nq + e : 0] = 0;
     // Tiles in order, all queries' of some rows first, an eighth of the order to each XCD (workgroups go round them): its L2 then reads
     // an eighth of the rows.
     const uint32_t tile = blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8, q_tiles = ((uint32_t)nq + T - 1) / T;
@@ -190,15 +192,73 @@ __device__ __forceinline__ float add_square(float sum, float x, float q) {
     return out;
 }
 
+constexpr int kCap = 1024, kGroupCap = 1024, kPatch = 2304;      // (floats of rows per wavefront at a time)
+// The distances of entries [from, to) of a list of row numbers, by a whole workgroup.  A wavefront takes 8 to 64 rows, few where there are few, and
+// 256 to 32 columns of them at a time through LDS (`mine`: kPatch floats of its own), the next ones' reads under way; then each lane adds up its own row's.
+__device__ __forceinline__ void list_distances(unsigned long long* buf, int from, int to, float* mine, const float* s_q, const float* __restrict__ data,
+                                               int dim, int wave, int lane) {
+    const int quarter = (to - from + 3) / 4, wide = quarter > 32 ? 3 : quarter > 16 ? 4 : quarter > 8 ? 5 : 6;
+    const int per = 512 >> wide, columns = 4 << wide, pitch = columns + 4;
+    const int kq = (lane & ((1 << wide) - 1)) * 4, r_in = lane >> wide, r_step = 64 >> wide;
+    for (int g0 = from + wave * per; g0 < to; g0 += 4 * per) {
+        const int count = min(per, to - g0), loads = (count + r_step - 1) / r_step;
+        const float* x[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) x[i] = data + (int64_t)(uint32_t)buf[g0 + min(i * r_step + r_in, count - 1)] * dim;
+        v4f pre[8];
+        auto fetch = [&](int k0) {      // (past the row's end: its last 16 bytes)
+#pragma unroll
+            for (int i = 0; i < 8; i++) if (i < loads) pre[i] = *reinterpret_cast<const v4f_any*>(x[i] + min(k0 + kq, dim - 4));
+        };
+        fetch(0);
+        float sum = 0.0f;
+        for (int k0 = 0; k0 < dim; k0 += columns) {
+            __builtin_amdgcn_wave_barrier();
+            const int col = min(k0 + kq, dim - 4) - k0;     // (a row's last quad may begin before its place, its head is then there already)
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                if (i < loads) {
+                    float* t = mine + (i * r_step + r_in) * pitch + col;
+                    if (k0 + kq + 4 <= dim) {
+                        *reinterpret_cast<v4f*>(t) = pre[i];
+                    } else {
+                        if (col >= 0) t[0] = pre[i].x;
+                        if (col >= -1) t[1] = pre[i].y;
+                        if (col >= -2) t[2] = pre[i].z;
+                        if (col >= -3) t[3] = pre[i].w;
+                    }
+                }
+            if (k0 + columns < dim) fetch(k0 + columns);
+            __builtin_amdgcn_wave_barrier();
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            const float* t = mine + min(lane, per - 1) * pitch;
+            const int kc = min(columns, dim - k0);
+            int kk = 0;
+#pragma unroll 4
+            for (; kk + 4 <= kc; kk += 4) {
+                const v4f v = *reinterpret_cast<const v4f*>(t + kk), y = *reinterpret_cast<const v4f*>(s_q + k0 + kk);
+                sum = add_square(sum, v.x, y.x);
+                sum = add_square(sum, v.y, y.y);
+                sum = add_square(sum, v.z, y.z);
+                sum = add_square(sum, v.w, y.w);
+            }
+            for (; kk < kc; kk++) sum = add_square(sum, t[kk], s_q[k0 + kk]);
+        }
+        if (lane < count)      // (the square root: as in exact_dists_kernel)
+            buf[g0 + lane] = ((unsigned long long)__builtin_bit_cast(uint32_t, (float)sqrt((double)sum)) << 32) | (uint32_t)buf[g0 + lane];
+    }
+}
 // One query per workgroup.  The rows whose bound is among the k smallest, and some further ones, are listed, their distances
 // formed, and the k-th of these says which other rows have to be listed too: hardly ever any.  Bounds are read only of groups of 32 rows
-// whose smallest one counts.  More than the lists take (rows that cannot be told apart, or whose squares no float holds): all rows, 256 at a time.  Bound by
-// the five reads that wait for each other (500 queries, 3000 rows: 9 us).
-constexpr int kCap = 1024, kGroupCap = 1024, kPatch = 2304;      // (floats of rows per wavefront at a time)
+// whose smallest one counts.  More than the lists take (rows that cannot be told apart, or whose squares no float holds): all rows, in tables of
+// fewer than kAloneRows here, else by query_listed (exhaustive.hip).  Bound by the five reads that wait for each other (500 queries, 3000 rows: 9 us).
+// (500 queries, one of them not finite, 3000 rows of 100: 118 us with a sort for every 256 rows, 94 now, 29 from all distances.)
+constexpr int kAloneRows = 8192;
 __global__ __launch_bounds__(kPackThreads) void nearest_rows_kernel(const float* __restrict__ bounds, const float* __restrict__ least,
                                                                     const float* __restrict__ data, int64_t N,
                                                                     int dim, const float* __restrict__ query, int k, int float_ids,
-                                                                    int32_t* __restrict__ out_ids, float* __restrict__ out_dists) {
+                                                                    int32_t* __restrict__ out_ids, float* __restrict__ out_dists,
+                                                                    uint32_t* __restrict__ left) {
     __shared__ unsigned long long buf[kCap];
     __shared__ __align__(16) float patch[4][kPatch];
     __shared__ uint32_t s_count, s_groups, s_limit;
@@ -265,60 +325,8 @@ __global__ __launch_bounds__(kPackThreads) void nearest_rows_kernel(const float*
         __syncthreads();
         return s_count <= (uint32_t)kCap;
     };
-    // The distances of entries [from, to) of the list.  A wavefront takes 8 to 64 rows, few where there are few, and 256 to 32 columns
-    // of them at a time through LDS, the next ones' reads under way; then each lane adds up its own row's.
-    float* mine = patch[wave];
     auto distances = [&](int from, int to) {
-        const int quarter = (to - from + 3) / 4, wide = quarter > 32 ? 3 : quarter > 16 ? 4 : quarter > 8 ? 5 : 6;
-        const int per = 512 >> wide, columns = 4 << wide, pitch = columns + 4;
-        const int kq = (lane & ((1 << wide) - 1)) * 4, r_in = lane >> wide, r_step = 64 >> wide;
-        for (int g0 = from + wave * per; g0 < to; g0 += 4 * per) {
-            const int count = min(per, to - g0), loads = (count + r_step - 1) / r_step;
-            const float* x[8];
-#pragma unroll
-            for (int i = 0; i < 8; i++) x[i] = data + (int64_t)(uint32_t)buf[g0 + min(i * r_step + r_in, count - 1)] * dim;
-            v4f pre[8];
-            auto fetch = [&](int k0) {      // (past the row's end: its last 16 bytes)
-#pragma unroll
-                for (int i = 0; i < 8; i++) if (i < loads) pre[i] = *reinterpret_cast<const v4f_any*>(x[i] + min(k0 + kq, dim - 4));
-            };
-            fetch(0);
-            float sum = 0.0f;
-            for (int k0 = 0; k0 < dim; k0 += columns) {
-                __builtin_amdgcn_wave_barrier();
-                const int col = min(k0 + kq, dim - 4) - k0;     // (a row's last quad may begin before its place, its head is then there already)
-#pragma unroll
-                for (int i = 0; i < 8; i++)
-                    if (i < loads) {
-                        float* t = mine + (i * r_step + r_in) * pitch + col;
-                        if (k0 + kq + 4 <= dim) {
-                            *reinterpret_cast<v4f*>(t) = pre[i];
-                        } else {
-                            if (col >= 0) t[0] = pre[i].x;
-                            if (col >= -1) t[1] = pre[i].y;
-                            if (col >= -2) t[2] = pre[i].z;
-                            if (col >= -3) t[3] = pre[i].w;
-                        }
-                    }
-                if (k0 + columns < dim) fetch(k0 + columns);
-                __builtin_amdgcn_wave_barrier();
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                const float* t = mine + min(lane, per - 1) * pitch;
-                const int kc = min(columns, dim - k0);
-                int kk = 0;
-#pragma unroll 4
-                for (; kk + 4 <= kc; kk += 4) {
-                    const v4f v = *reinterpret_cast<const v4f*>(t + kk), y = *reinterpret_cast<const v4f*>(s_q + k0 + kk);
-                    sum = add_square(sum, v.x, y.x);
-                    sum = add_square(sum, v.y, y.y);
-                    sum = add_square(sum, v.z, y.z);
-                    sum = add_square(sum, v.w, y.w);
-                }
-                for (; kk < kc; kk++) sum = add_square(sum, t[kk], s_q[k0 + kk]);
-            }
-            if (lane < count)      // (the square root: as in exact_dists_kernel)
-                buf[g0 + lane] = ((unsigned long long)__builtin_bit_cast(uint32_t, (float)sqrt((double)sum)) << 32) | (uint32_t)buf[g0 + lane];
-        }
+        list_distances(buf, from, to, patch[wave], s_q, data, dim, wave, lane);
         __syncthreads();
     };
     auto sort = [&](int count) {
@@ -355,17 +363,16 @@ __global__ __launch_bounds__(kPackThreads) void nearest_rows_kernel(const float*
             }
         }
     }
-    if (!fits) {      // buf[0, k) the best so far, 256 more behind them at a time
-        for (int j = tid; j < 512; j += kPackThreads) buf[j] = ~0ull;
-        __syncthreads();
-        for (int64_t j0 = 0; j0 < N; j0 += 256) {
-            const int n = (int)min((int64_t)256, N - j0);
-            for (int j = tid; j < 256; j += kPackThreads) buf[256 + j] = j < n ? (unsigned long long)(uint32_t)(j0 + j) : ~0ull;
-            __syncthreads();
-            distances(256, 256 + n);
-            bitonic_sort_u64_by256(buf, 512);
-            __syncthreads();
+    if (!fits) {
+        if (N >= kAloneRows) {
+            if (tid == 0) left[1 + atomicAdd(&left[0], 1u)] = blockIdx.x;
+            return;
         }
+        keep_smallest(buf, s_count, N, k, [&](int64_t first, int n) {
+            buf[kKeepAt + tid] = (unsigned long long)(uint32_t)(first + tid);
+            __syncthreads();
+            list_distances(buf, kKeepAt, kKeepAt + n, patch[wave], s_q, data, dim, wave, lane);
+        });
     }
     for (int j = tid; j < k; j += kPackThreads) {
         const unsigned long long e = buf[j];
@@ -376,7 +383,7 @@ __global__ __launch_bounds__(kPackThreads) void nearest_rows_kernel(const float*
 }
 
 template <int RT, int OCT, bool OCTETS>
-int launch_bounds(const float* data, int64_t N, int dim, const float* query, int nq, float* out, float* least, hipStream_t s) {
+int launch_bounds(const float* data, int64_t N, int dim, const float* query, int nq, float* out, float* least, uint32_t* left, hipStream_t s) {
     constexpr int T = 64 * RT, columns = 64 * OCT;
     const size_t lds = (size_t)2 * 2 * T * columns * 2 + 2 * 2 * T * 4 + (size_t)((dim + columns - 1) / columns * columns) * 4;
     static DeviceOnce once;
@@ -387,7 +394,7 @@ int launch_bounds(const float* data, int64_t N, int dim, const float* query, int
     if (rc) return rc;
     const int64_t tiles = ((N + T - 1) / T) * ((nq + T - 1) / T);
     hipLaunchKernelGGL((bound_rows_kernel<RT, OCT, OCTETS>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(kPackThreads), lds, s,
-                       data, N, dim, query, nq, out, least);
+                       data, N, dim, query, nq, out, least, left);
     DCIH_HIP(hipGetLastError());
     return 0;
 }
@@ -410,17 +417,20 @@ bool nearest_pays(int64_t N, int dim, int nq) {
     return (int64_t)nq * (dim < 64 ? 2048 : 4096) >= N && (dim <= 100 || pairs >= 1e5);
 }
 size_t nearest_least_bytes(int64_t N, int nq) { return (size_t)nq * (size_t)((N + 31) / 32) * 4; }
+size_t nearest_left_bytes(int nq) { return (2 * (size_t)nq + 1) * 4; }
 
-int query_nearest(const QueryArgs& a, int q0, int nq, float* d_bounds, float* d_least, hipStream_t s) {
+int query_nearest(const QueryArgs& a, int q0, int nq, float* d_bounds, float* d_least, uint32_t* d_left, hipStream_t s, bool& leaves) {
     const float* query = a.query + (int64_t)q0 * a.dim;
+    leaves = a.N >= kAloneRows;
+    uint32_t* left = leaves ? d_left : nullptr;
     const bool octets = a.dim % 8 == 0, large = ((a.N + 127) / 128) * ((nq + 127) / 128) >= 512;
     const auto bounds = large ? (octets ? launch_bounds<2, 1, true> : launch_bounds<2, 1, false>)
                       : a.dim > 64 ? (octets ? launch_bounds<1, 2, true> : launch_bounds<1, 2, false>)
                                    : octets ? launch_bounds<1, 1, true> : launch_bounds<1, 1, false>;
-    const int rc = bounds(a.data, a.N, a.dim, query, nq, d_bounds, d_least, s);
+    const int rc = bounds(a.data, a.N, a.dim, query, nq, d_bounds, d_least, left, s);
     if (rc) return rc;
     hipLaunchKernelGGL(nearest_rows_kernel, dim3((unsigned)nq), dim3(kPackThreads), (size_t)((a.dim + 3) & ~3) * 4, s, d_bounds, d_least, a.data, a.N,
-                       a.dim, query, a.k, a.float_ids, a.out_ids + (int64_t)q0 * a.k, a.out_dists + (int64_t)q0 * a.k);
+                       a.dim, query, a.k, a.float_ids, a.out_ids + (int64_t)q0 * a.k, a.out_dists + (int64_t)q0 * a.k, left);
     DCIH_HIP(hipGetLastError());
     return 0;
 }

@@ -313,6 +313,40 @@ def test_nearest_of_all_rows(gpu, kind, n, dim, nq, k):
     assert torch.equal(got[1].view(torch.int32), want[1].view(torch.int32))
 
 
+# Queries whose bounds rule out too little: all rows of small tables by the query's own workgroup, of larger ones in pieces of 2048 rows by
+# several.  Tables either side of where that changes and of a whole number of pieces, one such query, some, all of them, rows in ascending
+# and in descending order of distance.
+@pytest.mark.parametrize("n", [6401, 8191, 8192, 8193, 10239, 10240, 10241, 100003])
+@pytest.mark.parametrize("kind,k", [("one", 1), ("some", 33), ("dup", 10), ("all", 100), ("ascending", 7), ("descending", 100)])
+def test_nearest_where_bounds_say_little(gpu, n, kind, k):
+    dim, nq = 21, 37
+    X, Q = _rows("dup" if kind == "dup" else "normal", n, nq, dim, n + k)
+    if kind == "one":
+        Q[nq - 1, 3] = float("nan")
+    elif kind == "some":
+        Q[1::5, dim - 1] = float("inf")
+        Q[2::7, 0] = -float("nan")
+    elif kind == "dup":
+        X[: n // 2] = X[0]
+        Q[:] = X[0] + 1e-3
+    elif kind == "all":
+        X[:] = 1e6 * X[:1] + 1e-4 * X
+    else:
+        order = torch.arange(n, device="cuda", dtype=torch.float32) / n
+        X[:] = 0.0
+        X[:, 5] = 3000.0 + (order if kind == "ascending" else 1.0 - order)
+        Q[:] = 0.0
+        Q[:, 7] = 1e30 if kind == "descending" else 0.0
+    dci = gpu.DCI(dim, 2, 7, max(2, n // (8 * k)), 10, seed=3)
+    dci.add(X)
+    want = _ask(dci, dci._lib, NEVER, Q, k, 5000)
+    got = _ask(dci, dci._lib, ALWAYS, Q, k, 5000)
+    assert _route(dci)[3] == nq
+    dci.free()
+    assert torch.equal(got[0], want[0])
+    assert torch.equal(got[1].view(torch.int32), want[1].view(torch.int32))
+
+
 def test_nearest_of_many_rows(gpu):      # more than 512 workgroups of the product
     X, Q = _rows("clusters", 40000, 500, 72, 12)
     Q[7] = float("nan")
@@ -320,6 +354,7 @@ def test_nearest_of_many_rows(gpu):      # more than 512 workgroups of the produ
     dci.add(X)
     want = _ask(dci, dci._lib, NEVER, Q, 64, 100)
     got = _ask(dci, dci._lib, 0, Q, 64, 100)
+    assert _route(dci)[3] == 500
     dci.free()
     assert torch.equal(got[0], want[0])
     assert torch.equal(got[1].view(torch.int32), want[1].view(torch.int32))
