@@ -842,7 +842,7 @@ int query_exhaustive(const QueryArgs& a, void* ws, int chunk, hipStream_t s) {
     const ExSelect sel = exhaustive_select(a.N, a.k);
     for (int q0 = 0; q0 < a.nq; q0 += chunk) {
         const int nqc = min(chunk, a.nq - q0);
-        if (a.pick_rule != 1 && nearest_supported(a.N, a.dim, a.k) && (a.pick_rule == 2 || nearest_pays(a.N, a.dim, nqc))) {
+        if (a.pick_rule != 1 && nearest_supported(a.N, a.dim, a.k) && (a.pick_rule == 2 || nearest_pays(a.N, a.dim, a.k, nqc))) {
             char* rest = (char*)ws + align256((size_t)chunk * (size_t)a.N * 4);
             uint32_t* left = (uint32_t*)(rest + select_bytes(a.N, chunk, a.k));
             bool leaves = false;

@@ -281,7 +281,7 @@ int query_exhaustive(const QueryArgs& a, void* ws, int chunk, hipStream_t s);
 // The same for few results (nearest.hip): distances only of the rows whose lower bound says that they can be among them.
 // d_bounds: [nq][N] floats; d_least: nearest_least_bytes.
 bool nearest_supported(int64_t N, int dim, int k);
-bool nearest_pays(int64_t N, int dim, int nq);
+bool nearest_pays(int64_t N, int dim, int k, int nq);
 size_t nearest_least_bytes(int64_t N, int nq);
 // Queries whose bounds rule out too little are left in large tables (`leaves`): d_left receives their number, then their numbers, then as many
 // words as queries that are zero.

@@ -411,10 +411,17 @@ bool nearest_supported(int64_t N, int dim, int k) {
 // 256: 637 / 75; 200000 x 64, 16: 42 / 53, 64: 102 / 60; 10000 x 32, 1: 15 / 13), of short rows fewer still (100000 x 16, 32: 28 / 32, 64:
 // 38 / 34).  Long rows: few workgroups, one after another through the columns, wait longer than all distances take, until there are some
 // dozens of tiles (2048 x 960, 48: 44 / 55, 128: 68 / 56; 8192 x 300, 4: 24 / 26, 16: 28 / 26).
-bool nearest_pays(int64_t N, int dim, int nq) {
-    const double pairs = (double)N * (double)nq;
-    if (N < 8192) return N >= 2048 && pairs >= 2.5e5 && pairs * (double)dim >= 6e7;
-    return (int64_t)nq * (dim < 64 ? 2048 : 4096) >= N && (dim <= 100 || pairs >= 1e5);
+// More results than the sort of one wavefront takes need more work to pay for theirs (8500 x 900, 128 results, 12: 70 / 108; 45000 x 64, 64, 24: 27 / 30),
+// many queries rows that cost more than their own sorts (2500 x 16, 36, 4000: 55 / 83), and large tables a third launch's time.  (9213 shapes, 2100 to
+// 150000 rows of 16 to 900, 10 to 128 results: by a rule that does not look at k 692 took more than 2 % longer than all distances, the worst half as long
+// again; by this one 70, the worst 18 %.)
+bool nearest_pays(int64_t N, int dim, int k, int nq) {
+    const bool many = k >= 32;
+    const double pairs = (double)N * (double)nq, work = pairs * (double)dim;
+    if (N < kAloneRows)
+        return N >= 2048 && (double)N * dim >= (many ? 2e5 : 8e4) && pairs >= (many ? 3.75e5 : 2.5e5) && work >= (many ? 9e7 : 6e7);
+    return (double)nq * (dim < 64 ? 2048.0 : 4096.0) >= (many ? 2.0 : 1.0) * (double)N && work >= (many ? 8e7 : 2e7) &&
+           (dim <= 100 || pairs >= (many ? 2e5 : 1e5)) && (dim <= 600 || pairs >= (many ? 8e5 : 4e5));
 }
 size_t nearest_least_bytes(int64_t N, int nq) { return (size_t)nq * (size_t)((N + 31) / 32) * 4; }
 size_t nearest_left_bytes(int nq) { return (2 * (size_t)nq + 1) * 4; }
