@@ -1329,7 +1329,8 @@ int query_block(const QueryArgs& a_query, hipStream_t s) {
         // (a round may have any number: by an expected one alone all of 30000 items went through the variant for few, 1000 queries, 58 partitions
         // of 1724 normal rows of 300, k = 30, 4.5 ms whole, 7.3 in rounds)
         const int64_t items = a_in.picked && a_in.picked_exact ? a_in.picked_expect : (int64_t)a_in.nq * a_in.B;
-        for (int few = worth_more_wavefronts(a_in) ? 2 : 1; few >= 1 && !a_in.few_items; few--) {
+        // (larger tables pay up to four items a CU: 1100 items of 3800 points, L = 15, 64 promotions: 771 us with them, 550 without)
+        for (int few = worth_more_wavefronts(a_in) && items <= (int64_t)a_in.xcds * 32 * 4 ? 2 : 1; few >= 1 && !a_in.few_items; few--) {
             QueryArgs wide = a_in;
             wide.full_tables = 1;
             wide.few_items = few;
