@@ -826,6 +826,8 @@ int fill_positions_by_first(const int32_t* d_sids, const uint16_t* d_inv, uint16
         return 0;
     });
     if (rc) return rc;
+    // (neighbouring slices that are short as one: they and their ids lie side by side)
+    while (ppb <= 1024 && B > 1) { ppb *= 2; B = (B + 1) / 2; }
     hipLaunchKernelGGL(positions_by_first_kernel, dim3((unsigned)B, (unsigned)by), dim3(512), (size_t)ppb * 2, s, d_sids, d_inv, d_rpos, n, L, ppb);
     DCIH_HIP(hipGetLastError());
     return 0;
