@@ -422,20 +422,21 @@ __global__ __launch_bounds__(NT, NT / 256) void rank_row_kernel(const float* __r
     for (int r = 0; r < IPT; r++)
         if (tid * IPT + r < n) store(tid * IPT + r, key[r], rp[r] & 0xffffu);
 }
-// Longer rows, and rows fewer than CUs: `parts` workgroups to a row, each of which finds the part of the order that is its own,
+// Rows fewer than CUs, of 8192 to 32768 items: `parts` workgroups to a row, each of which finds the part of the order that is its own,
 // lists that part's items in LDS and ranks them there as above.  The parts are cut at bins of an even division of the row's range:
 // every workgroup counts all of the row, 4096 bins, and cuts where the bins pass p / parts of it.  Where a part does not fit
 // (distances that cluster) or a distance is not finite, its first and last item are found by their digits instead, eight bits of
 // (distance, number) at a time.  Bound by vector issue and LDS operations, of the passes over the row and of the ranking.
 // (Ranks of 64 rows of 20000: 61 us by the segmented sort, 30 in four parts each; read again by each of the four passes: 34.  16 rows of
-// 16000: 30 -> 16 us; of 50000: 74 -> 50.)
+// 16000: 30 -> 16 us.  Whole-number rows, whose distances are often equal, 64 of 20480: 44.  Few different distances, 49 of 40 rows of 20480: 72 -> 96.)
 constexpr int kRankMaxN = 1024 * 16;
-constexpr int kPartThreads = 1024, kPartBins = 4096, kPartMaxN = 65536;      // (numbers of 16 bits)
+constexpr int kPartThreads = 1024, kPartBins = 4096, kPartMaxN = 32768;
+constexpr int part_work(int ipt) { return ipt <= 6 ? 4096 : 2048; }      // (what LDS leaves; a power of two)
 constexpr size_t part_lds(int ipt) {
     const size_t items = (size_t)kPartThreads * ipt;
-    return 160 * 4 + (size_t)kPartThreads * 8 + (2 * items + 4 + rank_counter_words(kPartThreads, ipt)) * 4 + items * 2;
+    return 160 * 4 + (size_t)part_work(ipt) * 8 + (2 * items + 4 + rank_counter_words(kPartThreads, ipt)) * 4 + items * 2;
 }
-template <int IPT, int ROW>      // ROW: items of the whole row per thread, in registers; 0: read again by every pass
+template <int IPT, int ROW>      // ROW: items of the whole row per thread, in registers
 __global__ __launch_bounds__(kPartThreads, 4) void rank_part_kernel(const float* __restrict__ dists, int n, int k, int float_ids,
                                                                  int32_t* __restrict__ out_ids, float* __restrict__ out_vals) {
     constexpr int NT = kPartThreads, kItems = NT * IPT, kWaves = NT / kWave;
@@ -447,7 +448,7 @@ __global__ __launch_bounds__(kPartThreads, 4) void rank_part_kernel(const float*
     uint32_t* cut = misc + 64;                                           // [parts + 1] bins, parts at most 32,
     uint32_t* cut_at = misc + 112;                                       // and the items before them
     unsigned long long* work = reinterpret_cast<unsigned long long*>(misc + 160);
-    uint32_t* list = reinterpret_cast<uint32_t*>(work + NT);             // [kItems + 4]; the bins first
+    uint32_t* list = reinterpret_cast<uint32_t*>(work + part_work(IPT));      // [kItems + 4]; the bins first
     uint32_t* cnt = list + kItems + 4;                                   // [rank_counter_words]
     uint32_t* bits = cnt + rank_counter_words(NT, IPT);                                       // [kItems]: the part's distances, in order of their numbers
     uint16_t* number = reinterpret_cast<uint16_t*>(bits + kItems);       // [kItems]
@@ -457,7 +458,7 @@ __global__ __launch_bounds__(kPartThreads, 4) void rank_part_kernel(const float*
     out_ids += (int64_t)blockIdx.y * k;
     out_vals += (int64_t)blockIdx.y * k;
     const int share = (n + kWaves - 1) / kWaves, from = min(n, wave * share), to = min(n, from + share);      // this wavefront's items
-    uint32_t w[ROW ? ROW : 1];
+    uint32_t w[ROW];
 #pragma unroll
     for (int r = 0; r < ROW; r++) w[r] = __builtin_bit_cast(uint32_t, row[min(from + r * kWave + lane, n - 1)]);
     auto each = [&](auto use) __attribute__((always_inline)) {           // use(number, bits, whether there is one): all lanes, in order
@@ -466,10 +467,16 @@ __global__ __launch_bounds__(kPartThreads, 4) void rank_part_kernel(const float*
             if (from + r * kWave >= to) break;
             use(from + r * kWave + lane, w[r], from + r * kWave + lane < to);
         }
-        if constexpr (ROW == 0) {
-#pragma unroll 8
-            for (int j = from + lane; j < to + lane; j += kWave) use(j, __builtin_bit_cast(uint32_t, row[min(j, n - 1)]), j < to);
-        }
+    };
+    // One more of `what`; the first lane's by a single addition for all lanes that have it (rows of few distinct distances: one word's additions queue up).
+    auto count_in = [&](uint32_t what, bool in) __attribute__((always_inline)) {
+        const unsigned long long have = __ballot(in);
+        if (have == 0) return;
+        const int lead = (int)__builtin_ctzll(have);
+        const uint32_t lead_what = (uint32_t)__builtin_amdgcn_readlane((int)what, lead);
+        const unsigned long long same = __ballot(in && what == lead_what);
+        if (lane == lead) atomicAdd(&list[what], (uint32_t)__popcll(same));
+        if (in && what != lead_what) atomicAdd(&list[what], 1u);
     };
     // Exclusive sum over the workgroup's threads.
     auto scan = [&](uint32_t sum) {
@@ -502,7 +509,7 @@ __global__ __launch_bounds__(kPartThreads, 4) void rank_part_kernel(const float*
     auto bin_of = [&](uint32_t b) { return (uint32_t)((__builtin_bit_cast(float, b) - lo) * scale) >> 20; };
     auto cut_of = [&](int p) { return (uint32_t)((int64_t)n * p / parts); };
     if (even) {
-        each([&](int, uint32_t b, bool in) { if (in) atomicAdd(&list[bin_of(b)], 1u); });
+        each([&](int, uint32_t b, bool in) { count_in(bin_of(b), in); });
         __syncthreads();
         constexpr int kPer = kPartBins / NT;
         uint32_t v[kPer], sum = 0;
@@ -533,27 +540,34 @@ __global__ __launch_bounds__(kPartThreads, 4) void rank_part_kernel(const float*
     if (even) {
         first = cut_at[part];
     } else {
+        uint32_t place[2] = {first, cut_of(part + 1)};      // the items with so many others before them, both at once
+        unsigned long long found[2] = {0, 0};
+        const bool wanted[2] = {place[0] != 0, place[1] != (uint32_t)n};
 #pragma unroll 1
-        for (int end = 0; end < 2; end++) {      // the item with `place` others before it
-            uint32_t place = end ? cut_of(part + 1) : first;
-            if (place == 0 || place == (uint32_t)n) continue;
-            unsigned long long found = 0;
-#pragma unroll 1
-            for (int shift = 40; shift >= 0; shift -= 8) {
+        for (int shift = 40; shift >= 0; shift -= 8) {
+            __syncthreads();
+            if (tid < 512) list[tid] = 0;
+            __syncthreads();
+            each([&](int j, uint32_t b, bool in) {
+                const unsigned long long e = item_of(b, j);
+#pragma unroll
+                for (int end = 0; end < 2; end++)
+                    if (wanted[end]) count_in(256u * end + ((uint32_t)(e >> shift) & 255u), in && (e >> shift >> 8) == found[end]);
+            });
+            __syncthreads();
+#pragma unroll
+            for (int end = 0; end < 2; end++) {
+                if (!wanted[end]) continue;
+                const uint32_t v = tid < 256 ? list[256 * end + tid] : 0, run = scan(v);
+                if (run <= place[end] && place[end] < run + v) { extremes[6] = (uint32_t)tid; extremes[7] = place[end] - run; }      // (one thread)
                 __syncthreads();
-                if (tid < 256) list[tid] = 0;
+                found[end] = found[end] << 8 | extremes[6];
+                place[end] = extremes[7];
                 __syncthreads();
-                each([&](int j, uint32_t b, bool in) {
-                    const unsigned long long e = item_of(b, j);
-                    if (in && (e >> shift >> 8) == found) atomicAdd(&list[(uint32_t)(e >> shift) & 255u], 1u);
-                });
-                __syncthreads();
-                uint32_t digit = 0;
-                for (; digit < 255u && list[digit] <= place; digit++) place -= list[digit];      // (the same for all threads)
-                found = found << 8 | digit;
             }
-            (end ? item1 : item0) = found;
         }
+        if (wanted[0]) item0 = found[0];
+        if (wanted[1]) item1 = found[1];
     }
     if (first >= (uint32_t)k) return;
     // The part's items, in order of their numbers.
@@ -597,6 +611,7 @@ __global__ __launch_bounds__(kPartThreads, 4) void rank_part_kernel(const float*
     int fix_rank = -1;
     uint32_t fix_item = 0;
     bool ranked = false;
+    int sorted = 0;
     const float part_lo = __builtin_bit_cast(float, extremes[2]), part_scale = 4294966016.0f / (__builtin_bit_cast(float, extremes[3]) - part_lo);
     if (extremes[3] < kInfBits && part_scale < 4e38f) {
 #pragma unroll
@@ -606,8 +621,8 @@ __global__ __launch_bounds__(kPartThreads, 4) void rank_part_kernel(const float*
             rp[r] = (uint32_t)j;
         }
         auto before = [&](int x, int z) __attribute__((always_inline)) { return bits[x] != bits[z] ? bits[x] < bits[z] : x < z; };
-        ranked = lds_bucket_ranks<NT, IPT, rank_bits(kItems), true>(key, rp, count, part_scale, list, cnt, misc, work, NT, tid, fix_rank, fix_item,
-                                                                    before);
+        ranked = lds_bucket_ranks<NT, IPT, rank_bits(kItems), true, true>(key, rp, count, part_scale, list, cnt, misc, work, part_work(IPT), tid, fix_rank,
+                                                                          fix_item, before, [&](int x) { return bits[x]; }, &sorted);
     }
     auto store = [&](uint32_t place, uint32_t b, uint32_t item) {
         if (place >= (uint32_t)k) return;
@@ -624,6 +639,7 @@ __global__ __launch_bounds__(kPartThreads, 4) void rank_part_kernel(const float*
             if (r < own) order[rp[r] >> 16] = (uint16_t)(r * NT + tid);
         __syncthreads();
         if (fix_rank >= 0) order[fix_rank] = (uint16_t)fix_item;
+        for (int i = tid; i < sorted; i += NT) order[sorted_place(work, i)] = (uint16_t)(work[i] & ((1u << kSortedNumberBits) - 1u));
         __syncthreads();
         for (int j = tid; j < count; j += NT) store(first + (uint32_t)j, bits[order[j]], number[order[j]]);
         return;
@@ -676,7 +692,8 @@ static int launch_parts(const float* d_dist, int parts, int rows, int n, int k, 
 }
 // How many workgroups to a row: as many as leave one to a CU, if they hold it; 1: the kernels for whole rows.  (With rows on the device
 // twice, 64 of 16000, 4 / 6 parts: 33 / 52 us.  Short rows lose by the passes over the whole, 64 of 4000: 16 us whole, 18 in parts; 9582:
-// 28, 26.  More than 16 gain nothing.)
+// 28, 26.  More than 16 gain nothing.  Rows that do not stay in registers, past 32768, would be read again by every pass: 16 of 40000, whole 79 us, in parts 65;
+// 32, 87 and 95; 16 whose distances are few different numbers, 78 and 164.)
 constexpr int part_items(int64_t n, int parts) { return (int)(n / parts) * 21 / 20 + 64; }      // (bins are a few items)
 static int rank_parts(int64_t n, int rows) {
     const int parts = (int)min((int64_t)16, (int64_t)256 / rows);
@@ -685,8 +702,7 @@ static int rank_parts(int64_t n, int rows) {
 static int rank_rows_in_parts(const float* d_dist, int parts, int rows, int n, int k, int float_ids, int32_t* out_ids, float* out_vals, hipStream_t s) {
     const int most = part_items(n, parts);
     const auto launch = n <= 20480 ? (most <= 4096 ? launch_parts<4, 20> : most <= 6144 ? launch_parts<6, 20> : launch_parts<10, 20>)
-                      : n <= 32768 ? (most <= 4096 ? launch_parts<4, 32> : most <= 6144 ? launch_parts<6, 32> : launch_parts<10, 32>)
-                                   : (most <= 4096 ? launch_parts<4, 0> : most <= 6144 ? launch_parts<6, 0> : launch_parts<10, 0>);
+                                   : (most <= 4096 ? launch_parts<4, 32> : most <= 6144 ? launch_parts<6, 32> : launch_parts<10, 32>);
     return launch(d_dist, parts, rows, n, k, float_ids, out_ids, out_vals, s);
 }
 

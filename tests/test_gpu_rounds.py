@@ -66,6 +66,8 @@ def _rows(kind, n, nq, dim, seed):
         x = x[torch.randint(0, max(1, n // 8), (n + nq,), generator=g, device="cuda")]
     elif kind == "grid":
         x = torch.randint(0, 3, (n + nq, dim), generator=g, device="cuda").float()
+    elif kind == "whole":           # whole numbers: many equal distances
+        x = (40.0 * x).round()
     elif kind == "offset":          # squared lengths a million times the distances'
         x = x + 3000.0
     elif kind == "scales":          # rows from 1e-6 to 1e6: most of them outside what 16-bit floats of one scale hold
@@ -362,7 +364,7 @@ def test_nearest_of_many_rows(gpu):      # more than 512 workgroups of the produ
 
 # Rows ranked by several workgroups (few rows) and by one (many): sizes at the edges of both, of the rows that are kept in registers
 # and of the numbers of 16 bits; distances spread evenly, equal, in clusters too dense for a part, and not finite.
-@pytest.mark.parametrize("kind", ["normal", "grid", "zero", "huge", "broken"])
+@pytest.mark.parametrize("kind", ["normal", "grid", "whole", "zero", "huge", "broken"])
 @pytest.mark.parametrize("n", [8191, 8192, 10001, 16384, 16385, 20480, 20481, 32768, 32769, 65536, 65537])
 def test_ranking_in_parts(gpu, kind, n):
     X, Q = _rows(kind, n, 300, 9, n)
