@@ -43,6 +43,7 @@ namespace {
 constexpr int kWholeDim = 256;            // rows up to here can be kept in LDS whole
 constexpr int kMostParts = 2048;           // bounds kept per query
 constexpr int kLimits = kMostRounds;       // per query: of the rounds but the last, and round 1's limit of what is near
+constexpr int kMostDies = 32;             // tickets cleared
 constexpr int kListQueries = 1024;        // queries of a partition listed by one workgroup
 
 struct Header { float row_scale, query_scale; };      // the centre follows, kCentre floats in
@@ -561,7 +562,7 @@ struct ListArgs {
     const float* worst; int64_t worst_stride;      // the k-th distance each query has so far
     uint32_t* last_round;                          // the round that last took a partition of the query
     int B, parts, nq, groups, round, rounds, near;
-    int32_t* items; uint32_t* count; uint32_t* part_counts;
+    int32_t* items; uint32_t* count; uint32_t* part_counts; uint32_t* ticket;
 };
 __device__ inline bool takes_item(const ListArgs& a, int b, int q) {
     if (a.skip && *a.skip) return a.round == 0;
@@ -602,6 +603,7 @@ __global__ __launch_bounds__(256) void list_items_kernel(ListArgs a) {
         return;
     }
     uint32_t at = s_before[0] + s_before[1] + s_before[2] + s_before[3];
+    if (blockIdx.x == 0 && tid < kMostDies) a.ticket[tid] = 0;
     if (blockIdx.x + 1 == gridDim.x && tid == 0) *a.count = at + s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
     for (int w = 0; w < wave; w++) at += s_wave[w];
 #pragma unroll
@@ -630,7 +632,7 @@ Shape shape_of(const QueryArgs& a) {
 // The sample of a call's queries: every (nq / S)-th, and all their partitions as a round's items, by partition, then query.
 __device__ inline int sample_query(int s, int S, int nq) { return (int)((int64_t)nq * s / S); }
 __global__ __launch_bounds__(256) void sample_items_kernel(const float* __restrict__ query, int nq, int dim, int B, int S, float* __restrict__ rows,
-                                                           int32_t* __restrict__ items, uint32_t* __restrict__ count, uint32_t* __restrict__ last_round) {
+                                                           int32_t* __restrict__ items, uint32_t* __restrict__ count, uint32_t* __restrict__ ticket, uint32_t* __restrict__ last_round) {
     const int at = blockIdx.x * 256 + threadIdx.x, all = gridDim.x * 256;
     for (int e = at; e < S * dim; e += all) rows[e] = query[(int64_t)sample_query(e / dim, S, nq) * dim + e % dim];
     for (int e = at; e < S * B; e += all) items[e] = sample_query(e % S, S, nq) * B + e / S;
@@ -640,6 +642,7 @@ __global__ __launch_bounds__(256) void sample_items_kernel(const float* __restri
         last_round[q] = s < S && sample_query(s, S, nq) == q ? kSampleRound : 0u;
     }
     if (at == 0) *count = (uint32_t)(S * B);
+    if (at < kMostDies) ticket[at] = 0;
 }
 // Whether more than `most` of the sample's (query, partition) pairs have bounds within the query's k-th result.
 __global__ __launch_bounds__(256) void sample_decide_kernel(const uint32_t* __restrict__ bounds, int S, int nq, int B, int parts, const float* __restrict__ worst,
@@ -829,9 +832,9 @@ int sample_items(const QueryArgs& a, void* ws_, Picked& p, hipStream_t s) {
     const Room r = room_of(a);
     uint32_t* count = (uint32_t*)(ws + r.counts) + kSampleWord;
     hipLaunchKernelGGL(sample_items_kernel, dim3(32), dim3(256), 0, s, a.query, a.nq, a.dim, a.B, a.pick_sample, (float*)(ws + r.sample_rows),
-                       (int32_t*)(ws + r.items), count, (uint32_t*)(ws + r.last));
+                       (int32_t*)(ws + r.items), count, (uint32_t*)(ws + r.counts) + kTicketWord, (uint32_t*)(ws + r.last));
     DCIH_HIP(hipGetLastError());
-    p = Picked{(const int32_t*)(ws + r.items), count, (const uint32_t*)(ws + r.last), nullptr, nullptr, 0, 0, 0};
+    p = Picked{(const int32_t*)(ws + r.items), count, (const uint32_t*)(ws + r.last), (uint32_t*)(ws + r.counts) + kTicketWord, nullptr, nullptr, 0, 0, 0};
     return 0;
 }
 
@@ -869,7 +872,8 @@ int pick_items(const QueryArgs& a, void* ws_, int round, int rounds, hipStream_t
     }
     const int groups = (a.nq + kListQueries - 1) / kListQueries;
     ListArgs p{bounds, limits, a.pick_sample ? (const uint32_t*)(ws + r.counts) + kSkipWord : nullptr, a.out_dists + (a.k - 1), a.k, last, a.B, r.parts, a.nq, groups, round, rounds, a.pick_near,
-               (int32_t*)(ws + r.items), (uint32_t*)(ws + r.counts) + round, (uint32_t*)(ws + r.part_counts)};
+               (int32_t*)(ws + r.items), (uint32_t*)(ws + r.counts) + round, (uint32_t*)(ws + r.part_counts),
+               (uint32_t*)(ws + r.counts) + kTicketWord};
     const dim3 grid((unsigned)((int64_t)a.B * groups));
     hipLaunchKernelGGL(list_items_kernel<true>, grid, dim3(256), 0, s, p);
     hipLaunchKernelGGL(list_items_kernel<false>, grid, dim3(256), 0, s, p);
@@ -880,7 +884,8 @@ int pick_items(const QueryArgs& a, void* ws_, int round, int rounds, hipStream_t
 Picked picked_items(const QueryArgs& a, void* ws_, int round) {
     char* ws = (char*)ws_;
     const Room r = room_of(a);
-    Picked p{(const int32_t*)(ws + r.items), (const uint32_t*)(ws + r.counts) + round, (const uint32_t*)(ws + r.last), nullptr, nullptr, 0, 0, 0};
+    Picked p{(const int32_t*)(ws + r.items), (const uint32_t*)(ws + r.counts) + round, (const uint32_t*)(ws + r.last),
+             (uint32_t*)(ws + r.counts) + kTicketWord, nullptr, nullptr, 0, 0, 0};
     if (a.pick_near) {
         p.near_bounds = (const uint32_t*)(ws + r.near);
         // (later rounds: the k-th distance found so far)

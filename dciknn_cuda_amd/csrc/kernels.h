@@ -109,9 +109,9 @@ struct QueryArgs {
     const uint32_t* picked_count;
     uint32_t* round_items;   // null, or device words for the number of items of every round, then the sample's decision
     int64_t* selected;       // (host) counts the queries that nearest.hip answers
-    int picked_exact;        // 1: picked_expect is their number
-    int64_t picked_expect;   // about how many there are
-    int64_t picked_cover;    // ... and how many there seldom are more of: what a launch of one workgroup per item covers
+    uint32_t* picked_ticket; // a zeroed word per die: the dense kernel's workgroups take their items by it
+    int64_t picked_exact;    // their number, where it is known: 0 otherwise
+    int64_t picked_cover;    // how many there seldom are more of: what a launch of the batch kernel covers by a workgroup each
     const uint32_t* only;    // merge: null, or only the queries whose word here is only_round
     uint32_t only_round;
     // dense kernel, in rounds: lower bounds per tile of 2^near_shift rows ([B * near_tiles][nq]) and the distance of each query from
@@ -250,10 +250,10 @@ __device__ inline int64_t picked_run(const uint32_t* d_count, int x, int X, int6
 // round takes.  Scratch of bounds_bytes(); bounds_cost: about how long the bounds take, us.  pack_bounds
 // comes first and also clears a.part.
 constexpr int kPickCountWords = 64, kMostRounds = 4;
-constexpr int kSampleWord = 8, kSkipWord = 9;      // of the count words: the sample's items, whether rounds are skipped, and the pairs that says so by
+constexpr int kSampleWord = 8, kSkipWord = 9, kTicketWord = 16;      // of the count words: the sample's items, whether rounds are skipped, the pairs that says so by, a ticket per die
 constexpr uint32_t kSampleRound = 0x10000;         // of the sample's queries while their results are merged
 struct Picked {
-    const int32_t* items; const uint32_t* count; const uint32_t* last_round;
+    const int32_t* items; const uint32_t* count; const uint32_t* last_round; uint32_t* ticket;
     const uint32_t* near_bounds; const float* near_limit; int64_t near_stride; int near_shift, near_tiles;
 };
 bool bounds_supported(const QueryArgs& a);

@@ -638,8 +638,8 @@ int query(const QueryArgs& a_in, void* bounds_ws, hipStream_t s, hipEvent_t* ev,
             if (rc) return rc;
             a.picked = p.items;
             a.picked_count = p.count;
-            a.picked_expect = a.picked_cover = (int64_t)a.pick_sample * a.B;
-            a.picked_exact = 1;
+            a.picked_ticket = p.ticket;
+            a.picked_exact = a.picked_cover = (int64_t)a.pick_sample * a.B;
             rc = traverse(a);
             a.only = p.last_round;
             a.only_round = kSampleRound;
@@ -651,23 +651,20 @@ int query(const QueryArgs& a_in, void* bounds_ws, hipStream_t s, hipEvent_t* ev,
             a.only = nullptr;
         }
         if (!rc) rc = partition_bounds(a, bounds_ws, s);
-        const double all = (double)a.nq * (double)a.B * a.share, first = (double)a.nq * a.pick_first;
         for (int round = 0; round < a.pick_rounds && !rc; round++) {
             if (round > 0) rc = merge_lists(a, s);
             if (!rc) rc = pick_items(a, bounds_ws, round, a.pick_rounds, s);
             const Picked p = picked_items(a, bounds_ws, round);
             a.picked = p.items;
             a.picked_count = p.count;
+            a.picked_ticket = p.ticket;
             if (a.round_items && !rc) DCIH_HIP(hipMemcpyAsync(a.round_items + round, p.count, sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
             a.near_bounds = p.near_bounds; a.near_limit = p.near_limit; a.near_stride = p.near_stride;
             a.near_shift = p.near_shift; a.near_tiles = p.near_tiles;
-            a.picked_expect = (int64_t)fmax(round ? all - first : first, 1.0);
-            // (at least what costs 25 us where it has no item: what is not covered takes twice as long)
-            a.picked_cover = std::max((int64_t)(round ? 0.6 * first : 1.25 * first) + 64, (int64_t)131072);
             // The batch kernel's first launch covers all that may come in the first round, where queries whose bounds lie close together take
             // every partition: strides over the rest take up to twice as long, a workgroup without an item 0.2 ns.  (4000 queries, 58 partitions
             // of 17242 normal rows of 128: 15.2 ms whole, 18.9 in rounds that covered 131072 items.)
-            if (use_block) a.picked_cover = round ? std::max((int64_t)(0.3 * (double)a.nq * (double)a.B), (int64_t)65536) : (int64_t)a.nq * a.B;
+            a.picked_cover = round ? std::max((int64_t)(0.3 * (double)a.nq * (double)a.B), (int64_t)65536) : (int64_t)a.nq * a.B;
             if (!rc) rc = traverse(a);
             a.only = round > 0 ? p.last_round : nullptr;
             a.only_round = (uint32_t)round;

@@ -1328,7 +1328,7 @@ int query_block(const QueryArgs& a_query, hipStream_t s) {
         a_in.expect_promotions = (float)expected_promotions(a_in);
         // (a round may have any number: by an expected one alone all of 30000 items went through the variant for few, 1000 queries, 58 partitions
         // of 1724 normal rows of 300, k = 30, 4.5 ms whole, 7.3 in rounds)
-        const int64_t items = a_in.picked && a_in.picked_exact ? a_in.picked_expect : (int64_t)a_in.nq * a_in.B;
+        const int64_t items = a_in.picked && a_in.picked_exact ? a_in.picked_exact : (int64_t)a_in.nq * a_in.B;
         // (larger tables pay up to four items a CU: 1100 items of 3800 points, L = 15, 64 promotions: 771 us with them, 550 without)
         for (int few = worth_more_wavefronts(a_in) && items <= (int64_t)a_in.xcds * 32 * 4 ? 2 : 1; few >= 1 && !a_in.few_items; few--) {
             QueryArgs wide = a_in;
@@ -1371,7 +1371,7 @@ int query_block(const QueryArgs& a_query, hipStream_t s) {
                                                0xffffffffLL / 256 / X);
         int rc = launch_block(a, y, each * X, s);
         if (rc) return rc;
-        if (each * X < (int64_t)a.nq * a.B && !(a.picked_exact && each * X >= a.picked_expect)) {
+        if (each * X < (int64_t)a.nq * a.B && !(a.picked_exact && each * X >= a.picked_exact)) {
             if (two_passes) {
                 rc = launch_rest<kWave, 6, true>(a, y, X * 32 * min((int64_t)24, (int64_t)(160 * 1024 / y.lds_bytes)), each, s);
             } else {
