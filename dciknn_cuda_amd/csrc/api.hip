@@ -155,6 +155,7 @@ struct dcih_index {
     int append_mode = 0;                // DCIH_OPT_APPEND value
     int rounds = 0;                     // DCIH_OPT_ROUNDS value
     int64_t route[4] = {0, 0, 0, 0};    // dcih_debug_route
+    volatile uint32_t* blind = nullptr; // (pinned) set by queries in rounds whose bounds said nothing: the next ones use the rows' codes
     uint32_t* d_round_items = nullptr;  // dcih_debug_round_items
     unsigned long long* d_phase_ticks = nullptr;   // optional profile of the batch kernel
     // grow-only workspace: query scratch, and the unsorted keys during a build
@@ -201,6 +202,7 @@ int draw_directions(dcih_index* h) {
 // The rows change: their codes are formed anew, in the same room if it holds them.
 void forget_rows8(dcih_index* h) {
     h->rows8_ready = h->rows8_no_room = false;
+    if (h->blind) *h->blind = 0;
     h->rows8_demand = 0.0;
 }
 
@@ -693,6 +695,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     a.near_bounds = nullptr; a.near_limit = nullptr; a.near_stride = 0; a.near_shift = a.near_tiles = 0; a.pick_rule = fixed || whole ? 1 : h->rounds;
     a.phase_ticks = h->d_phase_ticks;
     a.round_items = h->d_round_items;
+    a.blind_word = nullptr;
     a.selected = &h->route[3];
     a.stop_hint = nullptr;
     a.N = h->n;
@@ -759,12 +762,22 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     }
 
     (void)plan_rounds(a);
+    if (a.pick_near) {
+        if (!h->blind && !recorded) {
+            void* p = nullptr;
+            if (hipHostMalloc(&p, sizeof(uint32_t), hipHostMallocDefault) == hipSuccess) { h->blind = (volatile uint32_t*)p; *h->blind = 0; }
+            else (void)hipGetLastError();
+        }
+        void* p = nullptr;
+        if (h->blind && hipHostGetDevicePointer(&p, (void*)h->blind, 0) == hipSuccess) a.blind_word = (uint32_t*)p;
+    }
+    const bool bounds_failed = h->blind && *h->blind;      // (of earlier calls: it steers work, never results)
     size_t q8_bytes = 0;
-    if (!blind && !a.pick_near && dense_traversal_supported(a, nullptr)) {      // (near rows only: few enough to be read whole)
+    if (!blind && (!a.pick_near || bounds_failed) && dense_traversal_supported(a, nullptr)) {      // (near rows only: few enough to be read whole)
         const bool all_dense = takes_dense_kernel(a);
         bool use = false;
         const double per_item = std::min((double)a.ppb, expected_promotions(a));
-        const int rc8 = use_rows8(h, all_dense ? (double)num_queries * block_size * per_item * a.share : 0.0, all_dense && !fixed, s, use);
+        const int rc8 = use_rows8(h, all_dense ? (double)num_queries * block_size * per_item * (bounds_failed ? 1.0 : a.share) : 0.0, all_dense && !fixed, s, use);
         if (rc8) return rc8;
         if (use) {
             a.rows8 = h->d_rows8; a.rows8_rec = rows8_record_bytes(dim); a.rows8_bounds = (uint32_t*)(h->d_rows8 + rows8_records(h, h->n));
@@ -1032,6 +1045,7 @@ int dcih_free(dcih_index* h) {
     for (auto& e : h->ev) if (e) (void)hipEventDestroy(e);
     if (h->busy) (void)hipEventDestroy(h->busy);
     if (h->rows8_event) (void)hipEventDestroy(h->rows8_event);
+    if (h->blind) (void)hipHostFree((void*)h->blind);
     delete h;
     return DCIH_OK;
 }

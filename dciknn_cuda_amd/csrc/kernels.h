@@ -108,6 +108,7 @@ struct QueryArgs {
     const int32_t* picked;   // null = all nq * B items, else the round's, of which every die takes one run
     const uint32_t* picked_count;
     uint32_t* round_items;   // null, or device words for the number of items of every round, then the sample's decision
+    uint32_t* blind_word;    // null, or (the host's memory) set where bounds say nothing of queries' nearest rows
     int64_t* selected;       // (host) counts the queries that nearest.hip answers
     uint32_t* picked_ticket; // a zeroed word per die: the dense kernel's workgroups take their items by it
     int64_t picked_exact;    // their number, where it is known: 0 otherwise

@@ -147,6 +147,33 @@ def test_a_sample_decides_about_rounds(gpu, kind, dim, outcome):
         assert 0 < items[0] < nq * B // 2 and items[5] < 16 * 15, items
 
 
+@pytest.mark.parametrize("dim", [40, 200])
+def test_bounds_that_say_nothing(gpu, dim):
+    """Clusters much further apart than they are wide, and a column that drowns the others: all partitions come in round 1, several times as
+    many as the dense kernel's workgroups, by whole rows at first and by the rows' codes in later calls; other rows after that."""
+    n, nq, B, T, k, outer = 60000, 500, 60, 10, 10, 5000
+    dci = gpu.DCI(dim, 2, 7, B, T, seed=3)
+    for kind in ("far", "column", "normal"):
+        X, Q = _rows("normal", n, nq, dim, dim)
+        if kind == "far":
+            at = 5000.0 * torch.randn(20, dim, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+            X += at[torch.arange(n, device="cuda") % 20]
+            Q += at[torch.arange(nq, device="cuda") % 20]
+        elif kind == "column":
+            X[:, 3] *= 1e5
+            Q[:, 3] *= 1e5
+        dci.clear()
+        dci.add(X)
+        want = _ask(dci, dci._lib, NEVER, Q, k, outer)
+        items = _count_items(dci)
+        for call in range(3):
+            got = _ask(dci, dci._lib, 0, Q, k, outer)
+            assert _route(dci)[0] >= 2 and _route(dci)[1] == 1, (kind, call)      # in rounds, with the tiles' bounds
+            assert torch.equal(got[0], want[0]) and torch.equal(got[1].view(torch.int32), want[1].view(torch.int32)), (kind, call)
+            assert kind == "normal" or int(items[0]) > 0.9 * nq * B, (kind, items.tolist())
+    dci.free()
+
+
 @pytest.mark.parametrize("nq", [1, 2, 15, 16, 17, 31, 100])
 @pytest.mark.parametrize("B", [2, 11, 12, 13, 25, 300])
 def test_samples_of_few_queries_and_partitions(gpu, nq, B):
