@@ -6,12 +6,14 @@
 // bounds, for every (query, partition), the distance of the partition's nearest row from below --
 // a matrix product on the matrix cores whose epilogue keeps a minimum -- and then traverses
 //   first the partitions whose bound is within what the query's k nearest rows are bounded by,
-//   then, as far as their bound does not exceed the k-th distance found so far, those within the bounds of the 2 k and of the 4 k nearest,
+//   then, as far as their bound does not exceed the k-th distance found so far, those within the bounds of the 2 k nearest and, the
+//     dense kernel's, of the 4 k nearest,
 //   last all others whose bound does not exceed it.
 // What is left out lies further than that, so the results are those of traversing everything; where
 // traversals miss near rows (low recall), or a bound is poor, the later rounds are larger, up to everything.
 // (123457 normal rows of 67 elements, 37 partitions, 7 results, half of the pairs needed: 27 pairs a query in three rounds, 22 in
-// four.  Calls of about a millisecond take the first and the last round only: a round's launches would cost more than the pairs it saves.)
+// four.  The batch kernel's calls take three: a fourth traversed 0.03 ms' worth of 8.9 on a million rows and
+// cost as much again in launches.  Calls of about a millisecond take the first and the last round only: a round's launches would cost more than the pairs it saves.)
 // The k nearest rows are told apart by bounds of parts of a partition: among S of them, k nearest rows that fall into
 // the same part are k^2 / 2 S, which is what the first limit is too large by.
 //
@@ -51,12 +53,13 @@ constexpr int kCentre = 16;
 
 // The first workgroups round 32 queries each, into the order the matrix instructions take them
 // ([32 queries][16 elements]: 64 lanes of 8), times -2; all of them clear what the later launches
-// take as cleared: the bounds (infinite), the partitions' lists (empty) and the lists' lengths.
+// take as cleared: the bounds (infinite), the bounds of near tiles where they are formed by atomics (infinite), and the
+// partitions' lists of results (empty).
 struct PackArgs {
     const float* query; const float* data;
     int64_t n;
     int nq, dim, steps, tiles;            // steps: of 16 elements; tiles: of 32 queries
-    Header* header; uint32_t* counts;
+    Header* header;
     float2* qinfo;                        // [tiles * 32]: |q'|^2 and an upper bound of |q - q'|
     _Float16* frags;
     uint32_t* bounds; int64_t num_bounds;
@@ -624,7 +627,17 @@ __global__ __launch_bounds__(256) void list_items_kernel(ListArgs a) {
 }
 
 // How the product is cut: row tiles and query tiles per wavefront, wavefronts along rows and queries; rows streamed or a tile of them
-// resident, and read once or once for every pass over the queries.
+// resident, and read once or once for every pass over the queries.  Up to 128 queries the rows' bytes bound it (512 columns: 160 us
+// for 819 MB, 5.1 TB/s), so all queries are taken in one pass with as few accumulators as hold them, and with them as many reading
+// wavefronts; above, the matrix cores, and a wavefront of 4x2 tiles reads 6 fragments for 8 products, one of 2x2 4 for 4.  us on 400000
+// rows in 10 partitions, columns/queries, the cut taken first:
+//   1x1 against 1x2 tiles:            64/32 28, 29    128/32 48, 50    512/32 160, 170    and at 48 queries 1x2 30, 44; 49, 65; 168, 274
+//   1x2 against 2x2 (2x2 wavefronts): 64/64 30, 45    128/64 49, 53    512/64 167, 158    and at 128 queries 2x2 46, 40; 56, 65; 181, 289
+//   2x2 against 4x2:                  64/128 46, 47   128/128 56, 59   200/128 82, 90     and at 192 queries 4x2 49, 62; 60, 80; 98, 131
+//   2x2 against 2x4, past 256 columns (rows are not kept whole there): 512/128 181, 268; at 192 queries 2x4 288, 276; 512 320, 567
+//   streamed against resident rows:   64/192 49, 53   64/1024 113, 95  200/1024 236, 202  and at 4096 queries resident 260, 349; 404, 505; 622, 798
+// (resident rows are up to 16 % the faster ones from 512 queries on where there are as many rows; streamed ones keep fewer rows' workgroups busy).
+// Rows of up to 128 columns are rounded once, whole; longer ones a stretch at a time.
 struct Shape { int rt, ct, wr, wc; bool stream, one; };
 Shape shape_of(const QueryArgs& a) {
     if (a.nq <= 32) return {1, 1, 4, 1, true, a.dim <= 128};
@@ -737,6 +750,9 @@ size_t near_bytes(const QueryArgs& a) {
     return (size_t)near_tiles_of(a) * a.B * a.nq * 4;
 }
 
+// us.  The constants are half of what the product reaches (400000 rows of 128, 4096 queries: 1.04 PFLOP/s; 512 columns, 32 queries: 5.1 TB/s;
+// 10M rows of 96, 512 queries, with the bounds of near tiles: 0.51 PFLOP/s and 1.9 TB/s): listing and limits come to the rest, and rounds
+// are not to be chosen where they gain little.  12 us: packing the queries and the launches.
 double bounds_cost(const QueryArgs& a) {
     const Shape y = shape_of(a);
     const int R = kTile * y.rt * y.wr;
@@ -748,7 +764,7 @@ double bounds_cost(const QueryArgs& a) {
 }
 
 static int pack(const QueryArgs& a, const Room& r, char* ws, hipStream_t s) {
-    PackArgs p{a.query, a.data, a.N, a.nq, a.dim, r.steps, r.tiles, (Header*)(ws + r.header), (uint32_t*)(ws + r.counts),
+    PackArgs p{a.query, a.data, a.N, a.nq, a.dim, r.steps, r.tiles, (Header*)(ws + r.header),
                (float2*)(ws + r.qinfo), (_Float16*)(ws + r.frags), (uint32_t*)(ws + r.bounds), (int64_t)a.B * r.parts * a.nq, (uint32_t*)(ws + r.near),
                a.pick_near && shape_of(a).rt * kTile < near_rows(shape_of(a).rt) ? (int64_t)near_bytes(a) / 4 : 0,
                a.part, (int64_t)a.nq * a.B * a.kcap};

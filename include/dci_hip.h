@@ -82,7 +82,15 @@ enum {
  * DCIH_OPT_ROUNDS: whether a query under automatic choice first bounds the distance of
  * every partition's nearest point from below and then traverses, in rounds, only the
  * partitions that can still hold a result: 0 = where it is estimated to be faster,
- * 1 = never, 2 = wherever the shape allows it.  Results are the same to the bit.
+ * 1 = never, 2 = wherever the shape allows it.  Where it is estimated to depend on the rows,
+ * 0 first traverses all partitions of up to 16 queries of the call and lets the device decide
+ * from them.  The option also governs queries whose traversals would promote every point
+ * (see dcih_query), for up to 128 results: 0 and 2 let them rule points out by bounds formed on
+ * the matrix cores, where that is estimated to be faster or wherever the shape allows it, 1 forms
+ * all distances.  Results are the same to the bit in every case.  Room for the bounds (up to 1 GiB
+ * for those of 64 or 128 rows each, and 4 bytes per query and part of a partition) is
+ * part of the handle's workspace and stays with it until dcih_free; where there is none the
+ * call is traversed whole.
  */
 enum { DCIH_OPT_TRAVERSAL = 0, DCIH_OPT_DENSE_MIN_PROMOTIONS = 1, DCIH_OPT_FORGET_HINTS = 2, DCIH_OPT_APPEND = 3,
        DCIH_OPT_ROUNDS = 4 };

@@ -297,6 +297,7 @@ def test_no_room_for_the_bounds(gpu):
     g = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g, stream=s):
         call(torch.cuda.current_stream().cuda_stream)
+    assert _route(dci) == (0, 0, 0, 0)
     for _ in range(3):
         ids.fill_(-5)
         dists.fill_(-5.0)
@@ -305,6 +306,9 @@ def test_no_room_for_the_bounds(gpu):
         torch.cuda.synchronize()
         assert torch.equal(ids, want[0]) and torch.equal(dists, want[1])
     del g
+    got = _ask(dci, dci._lib, ALWAYS, Q, k, 100)      # (not recorded, the same call takes the room and goes in rounds)
+    assert _route(dci)[0] >= 2
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
     dci.free()
 
 
