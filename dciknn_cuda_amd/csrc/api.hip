@@ -690,7 +690,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     a.hand_over_at = 0;
     a.expect_steps = a.expect_promotions = 0.0f;
     a.rows8 = nullptr; a.rows8_rec = 0; a.rows8_bounds = nullptr; a.query8 = nullptr;
-    a.picked = nullptr; a.picked_count = nullptr; a.picked_exact = a.picked_cover = 0; a.picked_ticket = nullptr; a.only = nullptr; a.only_round = 0;
+    a.picked = nullptr; a.picked_count = nullptr; a.picked_exact = a.picked_cover = a.picked_expect = 0; a.picked_ticket = nullptr; a.only = nullptr; a.only_round = 0;
     a.share = 1.0; a.pick_first = 0.0; a.pick_rounds = a.pick_rank = a.pick_near = a.pick_sample = 0; a.pick_most = 1.0f;
     a.near_bounds = nullptr; a.near_limit = nullptr; a.near_stride = 0; a.near_shift = a.near_tiles = 0; a.pick_rule = fixed || whole ? 1 : h->rounds;
     a.phase_ticks = h->d_phase_ticks;

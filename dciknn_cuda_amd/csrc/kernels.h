@@ -112,6 +112,7 @@ struct QueryArgs {
     int64_t* selected;       // (host) counts the queries that nearest.hip answers
     uint32_t* picked_ticket; // a zeroed word per die: the dense kernel's workgroups take their items by it
     int64_t picked_exact;    // their number, where it is known: 0 otherwise
+    int64_t picked_expect;   // about how many there are, 0: few
     int64_t picked_cover;    // how many there seldom are more of: what a launch of the batch kernel covers by a workgroup each
     const uint32_t* only;    // merge: null, or only the queries whose word here is only_round
     uint32_t only_round;

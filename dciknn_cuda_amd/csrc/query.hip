@@ -640,6 +640,7 @@ int query(const QueryArgs& a_in, void* bounds_ws, hipStream_t s, hipEvent_t* ev,
             a.picked_count = p.count;
             a.picked_ticket = p.ticket;
             a.picked_exact = a.picked_cover = (int64_t)a.pick_sample * a.B;
+            a.picked_expect = 0;
             rc = traverse(a);
             a.only = p.last_round;
             a.only_round = kSampleRound;
@@ -665,6 +666,7 @@ int query(const QueryArgs& a_in, void* bounds_ws, hipStream_t s, hipEvent_t* ev,
             // every partition: strides over the rest take up to twice as long, a workgroup without an item 0.2 ns.  (4000 queries, 58 partitions
             // of 17242 normal rows of 128: 15.2 ms whole, 18.9 in rounds that covered 131072 items.)
             a.picked_cover = round ? std::max((int64_t)(0.3 * (double)a.nq * (double)a.B), (int64_t)65536) : (int64_t)a.nq * a.B;
+            a.picked_expect = round ? 0 : (int64_t)((double)a.nq * a.pick_first);
             if (!rc) rc = traverse(a);
             a.only = round > 0 ? p.last_round : nullptr;
             a.only_round = (uint32_t)round;

@@ -306,9 +306,11 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
 
     // (a die's items number below 2^28; the step is read where it is used: one more scalar carried through the loop
     //  costs 1 % where a call is a few rounds of items)
-    // The items of a round, whose number the launch does not know, are handed out in order as workgroups come to ask for one.
+    // The items of a round, whose number the launch does not know, are handed out in order as workgroups come to ask for one: the
+    // last ones that start do, those before them take one item each.
     auto next_slot = [&](int slot) -> int {
         if constexpr (!PICKED) return slot + fresh_args()->step;
+        if (slot < fresh_args()->step) return 0x7fffffff;
         if (tid == 0) misc[dSlot] = atomicAdd(&fresh_args()->a.picked_ticket[xcd], 1u);
         __syncthreads();
         const int taken = __builtin_amdgcn_readfirstlane((int)misc[dSlot]);
@@ -1405,9 +1407,17 @@ int query_dense_items(const QueryArgs& a_in, hipStream_t s) {
         args.step = 1;
         per_xcd = (most + args.first - 1) / args.first;
     }
-    // (a round's items: as many workgroups as the device holds, each asks for the next one.  500 queries, 100 partitions of 2000 rows of 960, all
-    // of them in the first round: 10.3 ms by strides, 7.7 so; rows that bounds tell apart, 1.28 and 1.17.)
-    if (a.picked) per_xcd = min((int64_t)32 * per_cu, most);
+    // A round's items: as many workgroups as the device holds, each asks for the next one.  500 queries, 100 partitions of 2000 rows of 960, all
+    // of them in the first round: 10.3 ms by strides, 7.7 so; rows that bounds tell apart, 1.28 and 1.17.  To ask takes the time in which no wavefront
+    // of the workgroup works, so of as many items as in order the expected number have a workgroup each before these (10000 queries,
+    // 400 partitions of 25000 unit vectors of 96, a million items: 410 ms all asking, 387 so; 512 queries, 49000 items:
+    // 15.3 and 15.0; a million mixture rows in 100 partitions, 1000 queries, 10000 items: 2.40, 2.38).
+    if (a.picked) {
+        const int64_t resident = min((int64_t)32 * per_cu, most);
+        const int64_t fit = 0xffffffffLL / ((int64_t)a.xcds * y.nt), expect = min(min(fit, most), a.picked_expect / a.xcds);
+        per_xcd = y.ipt <= 15 && expect >= resident * 8 ? expect : resident;
+        args.step = (int)(per_xcd - resident);
+    }
     const unsigned grid = (unsigned)(per_xcd * a.xcds);
 #define DCIH_DENSE(NT, IPT, WAVES) rc = a.picked ? launch_dense<NT, IPT, WAVES, true>(args, grid, s) : launch_dense<NT, IPT, WAVES, false>(args, grid, s)
     int rc;

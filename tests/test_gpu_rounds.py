@@ -2,6 +2,7 @@
 that can hold a result (DCIH_OPT_ROUNDS), against the same queries traversed as a whole: ids and distances
 must be equal to the bit, whatever the rows are, because a partition is left out only where none of its rows can
 be as near as the k-th result.  Every traversal kernel that can run a round is covered."""
+import math
 import numpy as np
 import pytest
 import torch
@@ -145,6 +146,31 @@ def test_a_sample_decides_about_rounds(gpu, kind, dim, outcome):
         assert items[:3] == [nq * B, 0, 0], items
     else:
         assert 0 < items[0] < nq * B // 2 and items[5] < 16 * 15, items
+
+
+# Where many items are expected the dense kernel's launch holds a workgroup for each, and the last ones to start go on by tickets: as
+# many items as expected, several times as many, and a few; partitions of 300 rows (64 threads a workgroup) and of 2500.
+@pytest.mark.parametrize("kind,least,most", [("normal", 0.5, 2.0), ("far", 2.0, 20.0), ("apart", 0.0, 0.8)])
+@pytest.mark.parametrize("B", [100, 12])
+def test_a_workgroup_for_every_expected_item(gpu, kind, least, most, B):
+    n, nq, dim, k = 30000, 10000 if B == 100 else 3000, 24, 5
+    X, Q = _rows("normal", n, nq, dim, B)
+    if kind != "normal":            # clusters in every partition, or each in one of them
+        at = 5000.0 * torch.randn(100, dim, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+        rows = torch.arange(n, device="cuda")
+        X += at[rows % 100 if kind == "far" else rows * 100 // n]
+        Q += at[torch.arange(nq, device="cuda") % 100]
+    dci = gpu.DCI(dim, 2, 7, B, 10, seed=3)
+    dci.add(X)
+    want = _ask(dci, dci._lib, NEVER, Q, k, 5000)
+    items = _count_items(dci)
+    got = _ask(dci, dci._lib, ALWAYS, Q, k, 5000)
+    assert _route(dci)[0] == 4
+    dci.free()
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1].view(torch.int32), want[1].view(torch.int32))
+    expected = nq * (B * (1.0 - math.exp(-k / B)) + 0.5)
+    assert expected >= 8 * 8 * 32 * (4 if B == 12 else 16)      # (dies, items a workgroup, CUs of a die, workgroups a CU)
+    assert least * expected <= int(items[0]) <= most * expected, (items.tolist(), expected)
 
 
 @pytest.mark.parametrize("dim", [40, 200])
