@@ -509,7 +509,13 @@ __global__ __launch_bounds__(kPartThreads, 4) void rank_part_kernel(const float*
     auto bin_of = [&](uint32_t b) { return (uint32_t)((__builtin_bit_cast(float, b) - lo) * scale) >> 20; };
     auto cut_of = [&](int p) { return (uint32_t)((int64_t)n * p / parts); };
     if (even) {
-        each([&](int, uint32_t b, bool in) { count_in(bin_of(b), in); });
+        // (where the wavefront's first items lie in one bin by the half dozen; else the test for each costs more than it saves: 64 normal rows of
+        // 20000 44.1 us with it, 42.7 without, 20 of 32768 45, 40.7; half of a row at one distance takes 111, 244 where each item is added by itself)
+        const uint32_t some = bin_of(w[0]);
+        if (__popcll(__ballot(some == (uint32_t)__builtin_amdgcn_readfirstlane((int)some))) >= 6)
+            each([&](int, uint32_t b, bool in) { count_in(bin_of(b), in); });
+        else
+            each([&](int, uint32_t b, bool in) { if (in) atomicAdd(&list[bin_of(b)], 1u); });
         __syncthreads();
         constexpr int kPer = kPartBins / NT;
         uint32_t v[kPer], sum = 0;
