@@ -612,7 +612,7 @@ __global__ __launch_bounds__(256) void list_items_kernel(ListArgs a) {
         return;
     }
     uint32_t at = s_before[0] + s_before[1] + s_before[2] + s_before[3];
-    if (blockIdx.x == 0 && tid < kMostDies) a.ticket[tid] = 0;
+    if (blockIdx.x == 0 && tid < kMostDies) a.ticket[tid * kTicketStride] = 0;
     if (blockIdx.x + 1 == gridDim.x && tid == 0) *a.count = at + s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
     for (int w = 0; w < wave; w++) at += s_wave[w];
 #pragma unroll
@@ -661,7 +661,7 @@ __global__ __launch_bounds__(256) void sample_items_kernel(const float* __restri
         last_round[q] = s < S && sample_query(s, S, nq) == q ? kSampleRound : 0u;
     }
     if (at == 0) *count = (uint32_t)(S * B);
-    if (at < kMostDies) ticket[at] = 0;
+    if (at < kMostDies) ticket[at * kTicketStride] = 0;
 }
 // Whether more than `most` of the sample's (query, partition) pairs have bounds within the query's k-th result.
 __global__ __launch_bounds__(256) void sample_decide_kernel(const uint32_t* __restrict__ bounds, int S, int nq, int B, int parts, const float* __restrict__ worst,

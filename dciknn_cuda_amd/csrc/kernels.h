@@ -251,8 +251,8 @@ __device__ inline int64_t picked_run(const uint32_t* d_count, int x, int X, int6
 // Calls in rounds (bounds.hip): lower bounds of every (query, partition)'s nearest distance, and the items each
 // round takes.  Scratch of bounds_bytes(); bounds_cost: about how long the bounds take, us.  pack_bounds
 // comes first and also clears a.part.
-constexpr int kPickCountWords = 64, kMostRounds = 4;
-constexpr int kSampleWord = 8, kSkipWord = 9, kTicketWord = 16;      // of the count words: the sample's items, whether rounds are skipped, the pairs that says so by, a ticket per die
+constexpr int kPickCountWords = 64 + 32 * 32, kMostRounds = 4;
+constexpr int kSampleWord = 8, kSkipWord = 9, kTicketWord = 64, kTicketStride = 32;      // of the count words: the sample's items, whether rounds are skipped, the pairs that says so by, a ticket per die
 constexpr uint32_t kSampleRound = 0x10000;         // of the sample's queries while their results are merged
 struct Picked {
     const int32_t* items; const uint32_t* count; const uint32_t* last_round; uint32_t* ticket;
