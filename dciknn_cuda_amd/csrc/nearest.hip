@@ -415,11 +415,14 @@ bool nearest_supported(int64_t N, int dim, int k) {
 // many queries rows that cost more than their own sorts (2500 x 16, 36, 4000: 55 / 83), and large tables a third launch's time.  (9213 shapes, 2100 to
 // 150000 rows of 16 to 900, 10 to 128 results: by a rule that does not look at k 692 took more than 2 % longer than all distances, the worst half as long
 // again; by this one 70, the worst 18 %.)
+// A thousand million products pay for two dozen queries' tiles whatever the rest is (150000 x 300, 64, 36: all distances 389, 99; 87722 x 772, 96, 36: 378,
+// 166; of the same shapes none that takes longer is added, of fewer queries some: 70000 x 900, 128, 16: 146 / 199).
 bool nearest_pays(int64_t N, int dim, int k, int nq) {
     const bool many = k >= 32;
     const double pairs = (double)N * (double)nq, work = pairs * (double)dim;
     if (N < kAloneRows)
         return N >= 2048 && (double)N * dim >= (many ? 2e5 : 8e4) && pairs >= (many ? 3.75e5 : 2.5e5) && work >= (many ? 9e7 : 6e7);
+    if (nq >= 24 && work >= 1e9) return true;
     return (double)nq * (dim < 64 ? 2048.0 : 4096.0) >= (many ? 2.0 : 1.0) * (double)N && work >= (many ? 8e7 : 2e7) &&
            (dim <= 100 || pairs >= (many ? 2e5 : 1e5)) && (dim <= 600 || pairs >= (many ? 8e5 : 4e5));
 }
