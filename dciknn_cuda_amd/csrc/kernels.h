@@ -21,10 +21,16 @@ size_t segsort_tmp_bytes(int num_indices, int64_t n, int block_size);
 // sorted slice (the inverse of d_sids) as a 16-bit value (only meaningful when a partition
 // holds at most 65536 points).  d_lids: null, or [num_indices][n] receiving the ids relative
 // to their partition's first point as 16-bit values (no kernel reads them any more; the
-// index does not keep them).
+// index does not keep them).  values: the keys are distances, many of which may be equal or infinite, and not projections: always sorted by digits.
 int segsort(const float* d_keys, int64_t key_stride, int num_indices, int64_t n, int block_size,
             float* d_skeys, int32_t* d_sids, uint16_t* d_inv, uint16_t* d_lids, void* d_tmp,
-            hipStream_t s, bool float_ids = false);
+            hipStream_t s, bool float_ids = false, bool values = false);
+
+// The same for slices of ppb <= 25600 points by one distribution into buckets (bucketsort.hip); a slice that it does not suit is left alone
+// but for an id of -1 in its first place.
+bool bucketsort_supported(int64_t ppb);
+int bucketsort(const float* d_keys, int64_t key_stride, int num_indices, int64_t n, int64_t ppb, int B, float* d_skeys, int32_t* d_sids,
+               uint16_t* d_inv, hipStream_t s);
 
 // Appending: the index over n1 points from the sorted arrays of the index over their first
 // n0 points (same block_size) and the unsorted keys of the others (index i's key of point id

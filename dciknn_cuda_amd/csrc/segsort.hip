@@ -5,7 +5,8 @@
 // insertion_sort (src/dci_cuda_kernel.cu:113-146,190-247), where each of
 // block_size*thread_size threads quicksorts whole slices serially.
 //
-// Here a (key, position-in-slice) pair is one 64-bit word whose unsigned order
+// Slices of 65 to 25600 projections are distributed into buckets (bucketsort.hip); the kernels here sort what that leaves, distances and
+// other lengths.  A (key, position-in-slice) pair is one 64-bit word whose unsigned order
 // is the wanted order.  A slice of up to 32256 points is sorted by one
 // workgroup entirely in LDS: one coalesced read of the keys, one coalesced
 // write of the sorted keys and ids.  Longer slices are sorted tile by tile and
@@ -36,7 +37,9 @@ struct SegGeom {
     int64_t tail_from;
     int b_first;
     int float_ids;    // 1: ids are stored as float32 values in the same place
+    int left_only;    // 1: only the slices that the bucket kernel has left
 };
+constexpr int32_t kLeft = -1;          // in the place of a slice's first id
 __device__ inline int32_t stored_id(int float_ids, uint32_t id) {
     return float_ids ? __builtin_bit_cast(int32_t, (float)(int)id) : (int32_t)id;
 }
@@ -114,9 +117,9 @@ __global__ void segsort_tile_kernel(const float* __restrict__ keys, SegGeom g,
 // scan make every pass stable, so equal keys keep ascending ids.  Nibbles that
 // are constant over the slice (typically the exponent's) are skipped.  The
 // per-pass cost that does not depend on the slice (scan, barriers) grows with
-// the thread count, so the workgroup is the smallest of 64 / 128 / 256 / 512
+// the thread count, so the workgroup is the smaller of 256 / 512
 // threads that covers the slice with at most ~45 (512 threads: 63) items per
-// thread; a single wavefront needs no barrier at all.  Global traffic: keys
+// thread.  Global traffic: keys
 // read once (all reads of a thread in flight together), sorted keys / ids /
 // inverse written once, all coalesced.
 constexpr int kRadixMax = 63 * 512;
@@ -126,11 +129,9 @@ constexpr int kRadixTile = 30 * 1024; // longest tile of a slice that needs merg
 constexpr int radix_lds_bytes(int threads, int ipt) { return (ipt * threads + 8 * threads + 64) * 4; }
 
 template <int kRadixThreads, int IPT>
-__global__ __launch_bounds__(kRadixThreads, (kRadixThreads == 256 && IPT > 45) ? 2 : 1) void segsort_radix_kernel(
-    const float* __restrict__ keys, SegGeom g, float* __restrict__ skeys,
-    int32_t* __restrict__ sids, uint16_t* __restrict__ inv, uint16_t* __restrict__ lids,
-    unsigned long long* __restrict__ packed) {
-    extern __shared__ uint32_t rs[];
+__device__ __forceinline__ void radix_slice(uint32_t* rs, int64_t flat, const float* __restrict__ keys, const SegGeom& g, float* __restrict__ skeys,
+                                            int32_t* __restrict__ sids, uint16_t* __restrict__ inv, uint16_t* __restrict__ lids,
+                                            unsigned long long* __restrict__ packed) {
     uint32_t* stage = rs;                                         // IPT*1024 words
     uint16_t* stage16 = reinterpret_cast<uint16_t*>(rs);
     uint32_t* cnt32 = rs + IPT * kRadixThreads;                      // digit counters, [16][threads] 16-bit
@@ -144,9 +145,9 @@ __global__ __launch_bounds__(kRadixThreads, (kRadixThreads == 256 && IPT > 45) ?
     const bool tail = g.tail_from >= 0;
     const int tiles = packed && !tail ? g.tiles : 1;
     const int parts = tail ? g.B - g.b_first : g.B;
-    const int tile = (int)(blockIdx.x % tiles);
-    const int b = (int)((blockIdx.x / tiles) % parts) + (tail ? g.b_first : 0);
-    const int64_t i = blockIdx.x / ((int64_t)tiles * parts);
+    const int tile = (int)(flat % tiles);
+    const int b = (int)((flat / tiles) % parts) + (tail ? g.b_first : 0);
+    const int64_t i = flat / ((int64_t)tiles * parts);
     const int64_t off = (int64_t)b * g.ppb;
     const int64_t t0 = tail ? max((int64_t)0, g.tail_from - off) : (packed ? (int64_t)tile * g.tile_size : 0);
     const int64_t nseg = min(g.n - off, g.ppb) - t0;
@@ -231,6 +232,52 @@ __global__ __launch_bounds__(kRadixThreads, (kRadixThreads == 256 && IPT > 45) ?
         if (lids) lids[base + j] = (uint16_t)id;
         if (inv) inv[base + j] = pos_of[j];
     }
+}
+
+template <int kRadixThreads, int IPT>
+__global__ __launch_bounds__(kRadixThreads, (kRadixThreads == 256 && IPT > 45) ? 2 : 1) void segsort_radix_kernel(
+    const float* __restrict__ keys, SegGeom g, float* __restrict__ skeys,
+    int32_t* __restrict__ sids, uint16_t* __restrict__ inv, uint16_t* __restrict__ lids,
+    unsigned long long* __restrict__ packed) {
+    extern __shared__ uint32_t rs[];
+    if (g.left_only) {                                        // (the bucket kernel has done the others)
+        const int64_t off = (int64_t)(blockIdx.x % g.B) * g.ppb;
+        if (off >= g.n || sids[(blockIdx.x / g.B) * g.n + off] != kLeft) return;
+    }
+    radix_slice<kRadixThreads, IPT>(rs, blockIdx.x, keys, g, skeys, sids, inv, lids, packed);
+}
+// Only the slices that the bucket kernel has left, usually none, where there are many: a workgroup looks at 64 of them at a time.  (A
+// workgroup for each costs 40 us of 130 for 62500 slices of 320 points.)
+template <int kRadixThreads, int IPT>
+__global__ __launch_bounds__(kRadixThreads) void segsort_left_kernel(const float* __restrict__ keys, SegGeom g, int64_t slices, float* __restrict__ skeys,
+                                                                     int32_t* __restrict__ sids, uint16_t* __restrict__ inv) {
+    extern __shared__ uint32_t rs[];
+    for (int64_t first = blockIdx.x; first < slices; first += (int64_t)gridDim.x * kWave) {
+        const int64_t mine = first + (int64_t)(threadIdx.x & (kWave - 1)) * gridDim.x;
+        const int64_t at = (int64_t)(mine % g.B) * g.ppb;
+        unsigned long long left = __ballot(mine < slices && at < g.n && sids[(mine / g.B) * g.n + at] == kLeft);
+        while (left) {
+            const int next = __ffsll((long long)left) - 1;
+            left &= left - 1ull;
+            __syncthreads();                                  // (all have seen the marks, and the last slice's room is free)
+            radix_slice<kRadixThreads, IPT>(rs, first + (int64_t)next * gridDim.x, keys, g, skeys, sids, inv, nullptr, nullptr);
+        }
+    }
+}
+template <int NT, int IPT>
+static int launch_left(const float* d_keys, const SegGeom& g, int num_indices, float* d_skeys, int32_t* d_sids, uint16_t* d_inv, hipStream_t s) {
+    const size_t lds = (size_t)radix_lds_bytes(NT, IPT);
+    static DeviceOnce once;
+    const int rc = once.run([lds]() -> int {
+        DCIH_HIP(hipFuncSetAttribute((const void*)segsort_left_kernel<NT, IPT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        return 0;
+    });
+    if (rc) return rc;
+    const int64_t slices = (int64_t)num_indices * g.B;
+    hipLaunchKernelGGL((segsort_left_kernel<NT, IPT>), dim3((unsigned)min(slices, (int64_t)(NT == 64 ? 2048 : 512))), dim3(NT), lds, s,
+                       d_keys, g, slices, d_skeys, d_sids, d_inv);
+    DCIH_HIP(hipGetLastError());
+    return 0;
 }
 
 template <int NT, int IPT>
@@ -352,6 +399,7 @@ __global__ __launch_bounds__(NT, WPS) void segsort_radix1w_kernel(
     if (n <= 0) return;
     const int64_t base = i * g.n + off;
     const float* kin = keys + i * g.kstride + off;
+    if (g.left_only && sids[base] != kLeft) return;           // (the bucket kernel has done it)
 
     if (tid < 2) misc[32 + tid] = tid ? 0xffffffffu : 0u;        // OR / AND of all keys
     uint32_t w[IPT];
@@ -693,7 +741,7 @@ static int next_pow2(int v) {
 
 int segsort(const float* d_keys, int64_t key_stride, int num_indices, int64_t n, int block_size,
             float* d_skeys, int32_t* d_sids, uint16_t* d_inv, uint16_t* d_lids, void* d_tmp,
-            hipStream_t s, bool float_ids) {
+            hipStream_t s, bool float_ids, bool values) {
     if (n <= 0) return 0;
     if (key_stride < n) return fail(-1, "segsort: key rows overlap");
     SegGeom g;
@@ -706,6 +754,7 @@ int segsort(const float* d_keys, int64_t key_stride, int num_indices, int64_t n,
     g.tail_from = -1;
     g.b_first = 0;
     g.float_ids = float_ids ? 1 : 0;
+    g.left_only = 0;
     const int np2 = next_pow2((int)min((int64_t)kTileCap, g.ppb));
     // at most kTileCap / 1024 elements per thread (the inverse-permutation pass relies on it)
     const int threads = max(64, min(1024, np2 / 2));
@@ -713,6 +762,15 @@ int segsort(const float* d_keys, int64_t key_stride, int num_indices, int64_t n,
     const int64_t blocks = (int64_t)num_indices * g.B * g.tiles;
     if (blocks > 0x7fffffffLL) return fail(-1, "segsort: too many slices for one launch");
 
+    if (!values && !d_lids && bucketsort_supported(g.ppb)) {
+        const int rc = bucketsort(d_keys, key_stride, num_indices, n, g.ppb, g.B, d_skeys, d_sids, d_inv, s);
+        if (rc) return rc;
+        // (few long slices: a launch of a workgroup for each looks at the marks as fast)
+#define DCIH_LEFT(NT, IPT) if (g.ppb <= (int64_t)(NT) * (IPT)) return launch_left<NT, IPT>(d_keys, g, num_indices, d_skeys, d_sids, d_inv, s)
+        DCIH_LEFT(64, 9); DCIH_LEFT(64, 21); DCIH_LEFT(256, 21); DCIH_LEFT(256, 35);
+#undef DCIH_LEFT
+        g.left_only = 1;
+    }
     static DeviceOnce once;
     {
         const int rc = once.run([]() -> int {
@@ -732,9 +790,7 @@ int segsort(const float* d_keys, int64_t key_stride, int num_indices, int64_t n,
         // slices of 15 k to 19968 points: the one-word kernel, two workgroups per CU
         if (g.ppb > 15000 && g.ppb <= 512 * 39)
             return launch_radix1w<512, 39, 4>(d_keys, g, num_indices, d_skeys, d_sids, d_inv, d_lids, s);
-        DCIH_RADIX(64, 9); DCIH_RADIX(64, 17); DCIH_RADIX(64, 25); DCIH_RADIX(64, 33);
-        DCIH_RADIX(128, 21); DCIH_RADIX(128, 27); DCIH_RADIX(128, 33);
-        DCIH_RADIX(256, 21); DCIH_RADIX(256, 27); DCIH_RADIX(256, 33); DCIH_RADIX(256, 39); DCIH_RADIX(256, 45);
+        DCIH_RADIX(256, 33); DCIH_RADIX(256, 39); DCIH_RADIX(256, 45);
         DCIH_RADIX(256, 51); DCIH_RADIX(256, 57);      // two workgroups share a CU: one's passes cover the other's loads and stores
         DCIH_RADIX(512, 33); DCIH_RADIX(512, 39); DCIH_RADIX(512, 45);
         DCIH_RADIX(512, 51); DCIH_RADIX(512, 57); DCIH_RADIX(512, 63);
@@ -884,7 +940,7 @@ int segsort_append(const float* d_old_skeys, const int32_t* d_old_sids, int64_t 
         g.kstride = key_stride; g.n = n1; g.B = block_size; g.ppb = ag.p1;
         g.tiles = 1; g.tile_size = 0;
         g.tail_from = n0;
-        g.float_ids = 0;
+        g.float_ids = 0; g.left_only = 0;
         g.b_first = (int)(n0 / ag.p1);
         int64_t longest = 0;                               // longest run of new points in one partition
         for (int b = g.b_first; b < block_size; b++)
