@@ -129,6 +129,10 @@ struct dcih_index {
     uint16_t* d_rpos = nullptr;         // [I][n] the same, in the order of each composite's first simple index (room kept by the
                                         // build, filled by the first query that runs the batch traversal kernel)
     int rpos_ready = 0;
+    uint16_t* d_point_rows = nullptr;   // null, or room for every point's positions side by side (where windows are wide; filled by a call
+                                        // in rounds, once such calls have asked for more than that costs)
+    int point_rows_ready = 0;
+    double point_rows_demand = 0.0;     // points looked at by such calls so far, in indexes' worth
     // 8-bit codes of the rows and the partitions' bounds behind them (rows8.hip): room taken and codes formed
     // once the dense kernel's calls have asked for more candidate rows than forming them costs
     unsigned char* d_rows8 = nullptr;
@@ -218,6 +222,8 @@ int release_sorted(dcih_index* h) {
     h->d_inv = nullptr;
     h->d_rpos = nullptr;
     h->rpos_ready = 0;
+    h->d_point_rows = nullptr;
+    h->point_rows_ready = 0;
     forget_rows8(h);
     h->d_stop_hint = nullptr;
     return 0;
@@ -295,11 +301,13 @@ int ensure_arena(dcih_index* h, int which, size_t bytes) {
 
 // Where the arrays of an index of n points lie inside an arena.
 struct ArenaLayout {
-    size_t keys, ids, inv, rpos, hint, total;   // byte offsets, and the size of it all
+    bool point_rows_pay;
+    size_t keys, ids, inv, rpos, point_rows, hint, total;   // byte offsets, and the size of it all
     bool small_parts;                           // partitions of at most 65536 points: 16-bit tables exist
 };
-ArenaLayout arena_layout(int I, int64_t n, int block_size) {
+ArenaLayout arena_layout(int M, int L, int64_t n, int block_size, int thread_size) {
     ArenaLayout y;
+    const int I = M * L;
     const size_t cells = (size_t)I * (size_t)n;
     y.small_parts = (n + block_size - 1) / block_size <= 65536;
     const size_t b_keys = align_up(cells * sizeof(float));
@@ -311,10 +319,14 @@ ArenaLayout arena_layout(int I, int64_t n, int block_size) {
     y.ids = b_keys;
     y.inv = y.ids + b_ids;
     y.rpos = y.inv + b_inv;
-    y.hint = y.rpos + b_inv;
+    y.point_rows = y.rpos + b_inv;
+    y.point_rows_pay = y.small_parts && point_rows_pay((n + block_size - 1) / block_size, M, L, thread_size);
+    y.hint = y.point_rows + (y.point_rows_pay ? align_up(point_rows_bytes(n, M, L)) : 0);
     y.total = y.hint + b_hint;
     return y;
 }
+
+constexpr double kPointRowsDemand = 16.0;
 
 size_t rows8_records(const dcih_index* h, int64_t n) { return align_up((size_t)n * rows8_record_bytes(h->dim)); }
 size_t rows8_room(const dcih_index* h, int64_t n, int block_size) {
@@ -445,10 +457,10 @@ int dcih_set_directions(dcih_index* h, const float* h_dirs) {
 // With merge_from > 0 the live index (over the first merge_from points, in the other arena) is
 // merged with the sorted new points instead of everything being sorted again.
 static int sort_into(dcih_index* h, int which, const float* d_keys, int64_t key_stride,
-                     int64_t num_points, const float* d_data, int block_size, void* d_tmp,
+                     int64_t num_points, const float* d_data, int block_size, int thread_size, void* d_tmp,
                      hipStream_t s, int64_t merge_from = 0) {
     const int I = num_indices(h);
-    const ArenaLayout y = arena_layout(I, num_points, block_size);
+    const ArenaLayout y = arena_layout(h->M, h->L, num_points, block_size, thread_size);
     char* base = (char*)h->arena[which];
     float* skeys = (float*)(base + y.keys);
     int32_t* sids = (int32_t*)(base + y.ids);
@@ -470,6 +482,9 @@ static int sort_into(dcih_index* h, int which, const float* d_keys, int64_t key_
     h->d_skeys = skeys; h->d_sids = sids; h->d_inv = inv; h->d_stop_hint = hint;
     h->d_rpos = y.small_parts ? (uint16_t*)(base + y.rpos) : nullptr;
     h->rpos_ready = 0;
+    h->d_point_rows = y.point_rows_pay ? (uint16_t*)(base + y.point_rows) : nullptr;
+    h->point_rows_ready = 0;
+    h->point_rows_demand = 0.0;
     forget_rows8(h);
     h->cur = which;
     h->d_data = d_data;
@@ -499,7 +514,7 @@ int dcih_add(dcih_index* h, int dim, int64_t num_points, const float* d_data,
     if (rc) return rc;
     release_rows(h);                // (rows of appends before a clear: this index borrows its rows)
     if (h->rows8_bytes < rows8_room(h, num_points, block_size)) release_rows8(h);
-    rc = ensure_arena(h, h->cur, arena_layout(I, num_points, block_size).total);
+    rc = ensure_arena(h, h->cur, arena_layout(h->M, h->L, num_points, block_size, thread_size).total);
     if (rc == DCIH_OK) rc = ensure_ws(h, b_keys + align_up(tmp_bytes), s);
     if (rc == DCIH_OK) {
         float* d_keys = (float*)h->ws;
@@ -507,7 +522,7 @@ int dcih_add(dcih_index* h, int dim, int64_t num_points, const float* d_data,
         rc = project(h->d_dirs, I, d_data, num_points, dim, d_keys, num_points, s);
         mark(h, DCIH_T_PROJECT, 1, s);
         if (rc == DCIH_OK)
-            rc = sort_into(h, h->cur, d_keys, num_points, num_points, d_data, block_size,
+            rc = sort_into(h, h->cur, d_keys, num_points, num_points, d_data, block_size, thread_size,
                            tmp_bytes ? (void*)((char*)h->ws + b_keys) : nullptr, s);
         else
             (void)hipStreamSynchronize(s);
@@ -573,8 +588,8 @@ int dcih_append(dcih_index* h, int dim, int64_t num_points, const float* d_data,
     }
     const size_t tmp_bytes = merge ? segsort_append_tmp_bytes(I, total) : segsort_tmp_bytes(I, total, block_size);
     rc = ensure_arena(h, h->n > 0 ? spare : h->cur,
-                          std::max(arena_layout(I, total, block_size).total,
-                                   arena_layout(I, cap, block_size).total));
+                          std::max(arena_layout(h->M, h->L, total, block_size, thread_size).total,
+                                   arena_layout(h->M, h->L, cap, block_size, thread_size).total));
     if (rc == DCIH_OK && tmp_bytes) rc = ensure_ws(h, align_up(tmp_bytes), s);
     hipError_t e = hipSuccess;
     if (rc == DCIH_OK && h->n > 0 && rows != h->d_data)        // rows (and projections) indexed so far
@@ -596,7 +611,7 @@ int dcih_append(dcih_index* h, int dim, int64_t num_points, const float* d_data,
     }
     if (rc == DCIH_OK)
         // the partition boundaries move with the total, so every slice is formed again
-        rc = sort_into(h, h->n > 0 ? spare : h->cur, ukeys, cap, total, rows, block_size,
+        rc = sort_into(h, h->n > 0 ? spare : h->cur, ukeys, cap, total, rows, block_size, thread_size,
                        tmp_bytes ? h->ws : nullptr, s, merge ? h->n : 0);
     else
         (void)hipStreamSynchronize(s);
@@ -679,6 +694,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     QueryArgs a;
     a.skeys = h->d_skeys; a.sids = h->d_sids; a.inv = h->d_inv; a.data = h->d_data; a.query = d_query;
     a.rpos = h->d_rpos; a.rpos_ready = &h->rpos_ready; a.recorded = recorded ? 1 : 0;
+    a.point_rows = nullptr;
     a.hints_cold = 0;
     a.mode = h->traversal; a.item_list = nullptr; a.item_count = nullptr; a.dense = nullptr;
     a.xcds = h->xcds; a.q_first = 0; a.q_count = num_queries;
@@ -822,6 +838,18 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
                           block_size, thread_size, d_nn, d_dists, d_counters, stream, fixed, float_ids, who, true);
     }
     if (rc) return rc;
+    // A point's positions side by side for the dense kernel's near rows.  To form them takes as long as the look-ups of all points by eight queries.
+    if (a.pick_rounds && a.pick_near && h->d_point_rows && point_rows_pay(a.ppb, a.M, a.L, a.T)) {
+        h->point_rows_demand += (double)num_queries * a.share;
+        if (!h->point_rows_ready && h->point_rows_demand >= kPointRowsDemand) {
+            rc = fill_point_rows(h->d_inv, h->d_point_rows, h->n, h->M, h->L, s);
+            if (rc) return rc;
+            a.point_rows = h->d_point_rows;
+            if (!recorded) h->point_rows_ready = 1;
+        } else if (h->point_rows_ready) {
+            a.point_rows = h->d_point_rows;
+        }
+    }
     h->route[0] = a.pick_rounds; h->route[1] = a.pick_near; h->route[2] = a.pick_sample;
     char* base = ws_base;
     float* d_qproj = (float*)base;

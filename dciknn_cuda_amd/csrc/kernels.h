@@ -49,6 +49,11 @@ int segsort_append(const float* d_old_skeys, const int32_t* d_old_sids, int64_t 
 int fill_positions_by_first(const int32_t* d_sids, const uint16_t* d_inv, uint16_t* d_rpos, int64_t n, int M, int L, int64_t ppb, int B,
                             hipStream_t s);
 
+// point_rows from inv (see QueryArgs), and whether the dense kernel's calls in rounds are better off with them.
+size_t point_rows_bytes(int64_t n, int M, int L);
+int fill_point_rows(const uint16_t* d_inv, uint16_t* d_rows, int64_t n, int M, int L, hipStream_t s);
+bool point_rows_pay(int64_t ppb, int M, int L, int T);
+
 struct QueryArgs {
     const float* skeys;      // [I][N] sorted projections
     const int32_t* sids;     // [I][N] point ids in the same order
@@ -57,6 +62,7 @@ struct QueryArgs {
                              // slice is the position, in this simple index, of the point that stands at place s of the
                              // first one's slice (null if ppb > 65536; filled on the first use, see fill_positions_by_first)
     int* rpos_ready;         // host flag of the index: rpos has been filled
+    const uint16_t* point_rows;   // null, or [N][M][L up to a multiple of 8] inv's positions, a point's side by side (the last one of a composite repeated)
     int recorded;            // 1: the call is recorded into a graph, its kernels do not run now
     const float* data;       // [N][dim]
     const float* query;      // [nq][dim]

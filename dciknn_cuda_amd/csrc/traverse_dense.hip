@@ -61,6 +61,9 @@ struct DenseLayout {
     int sort_cap, quota;
     int front8, quota8;   // the same buffer where rows are compared by their codes: words kept, entries per wavefront between two merges
     int tiles;        // 1: rows of at most 128 elements, 16-byte aligned, distances wanted: whole batches of 64 rows
+    int by_windows;   // 1: candidates are found by the windows' first lanes and the rows of near tiles, no time is kept per point
+    int off_tab, tab_cap;   // then the step tables of all composites, uint16 per window, and
+    int off_hist;     // the histogram of steps
     size_t lds_bytes;
 };
 
@@ -87,6 +90,9 @@ constexpr int kBins = 256;               // of the histogram of scores, which li
 // ceil((p+1)/T) + floor((n+T-3-p)/T) + 1 <= n/T + 3.  (A layout holds that many, so every item fits it.)
 int64_t dense_max_windows(const QueryArgs& a) { return (int64_t)a.L * (a.ppb / a.T + 3); }
 
+// (point_rows are there where the rule of point_rows_pay says so)
+bool by_windows(const QueryArgs& a) { return a.picked && a.near_bounds && a.point_rows && dense_max_windows(a) <= 9 * 512 && a.M * (dense_max_windows(a) + 1) < 32768; }
+
 DenseLayout dense_layout_for(const QueryArgs& a, int nt, int ipt) {
     DenseLayout y;
     const int I = a.M * a.L;
@@ -98,7 +104,16 @@ DenseLayout dense_layout_for(const QueryArgs& a, int nt, int ipt) {
     y.off_idx = o;      o += 4 * I * 4;
     y.off_seg = o;      o += (6 * a.L + 2) * 4;
     y.off_q = o;        o += ((a.dim + 3) & ~3) * 4;
-    y.off_time = o;     o += (int)(((a.ppb + 1) & ~(int64_t)1) * 2);
+    y.by_windows = by_windows(a) ? 1 : 0;
+    y.off_time = y.off_tab = y.off_hist = o;
+    y.tab_cap = (int)((dense_max_windows(a) + 1) & ~(int64_t)1);
+    if (y.by_windows) {
+        o += 2 * a.M * y.tab_cap;
+        o = (o + 3) & ~3;
+        y.off_hist = o; o += 2 * y.tab_cap + 8;
+    } else {
+        o += (int)(((a.ppb + 1) & ~(int64_t)1) * 2);
+    }
     o = (o + 15) & ~15;
     // k best plus room for candidates that beat the current k-th: the wavefronts fill
     // a quota each between two merges
@@ -231,10 +246,13 @@ struct DenseTables {
     }
 };
 
-// WAVES: wavefronts per SIMD the registers are shared out for.  PICKED: the items are those of a call's round.  (Both in one
+// WAVES: wavefronts per SIMD the registers are shared out for.  kPicked: the items are those of a call's round.  (Both in one
 // kernel cost whole calls 3 %: 5000 items of 1350 rows, 418 and 429 us.)
-template <int NT, int IPT, int WAVES, bool PICKED>
+// kWindows: of these, where few points are the first lane of a window and only the rows of near tiles can be results.
+enum DenseKind { kWhole, kPicked, kWindows };
+template <int NT, int IPT, int WAVES, int KIND>
 __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
+    constexpr bool PICKED = KIND != kWhole, WINDOWS = KIND == kWindows;
     // The arguments are read where they are used, through a pointer that every phase makes opaque again:
     // read once, ahead of the loop over the items, they would be carried through it in spilled registers.
     typedef const DenseArgs __attribute__((address_space(4)))* ArgsPtr;
@@ -345,7 +363,7 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
         if (args->a.phase_ticks) tick = wall_clock64();
         if (tid < dMiscWords) misc[tid] = 0;
         for (int j = tid; j < args->a.dim; j += NT) tb.q[j] = args->a.query[(int64_t)qi * args->a.dim + j];
-        for (int pt = tid; pt < n; pt += NT) tb.time[pt] = (uint16_t)((kNever << 1) & 0xffffu);
+        if constexpr (!WINDOWS) for (int pt = tid; pt < n; pt += NT) tb.time[pt] = (uint16_t)((kNever << 1) & 0xffffu);
         uint32_t probes = 0;
         {
             const int per_wave = (I + kWaves - 1) / kWaves;
@@ -408,8 +426,9 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
                     // window j at place nl - 1 - j, right window j at nl + j; a position pos
                     // belongs to the window at place (pos + nl * T - p - 1) / T and is its first
                     // lane where that division leaves no remainder.
+                    // (by windows both in one word)
                     tb.tabbase[i] = at;
-                    tb.shift[i] = nl * T - p - 1;
+                    tb.shift[i] = (nl * T - p - 1) | (WINDOWS ? (at + m * args->y.tab_cap) << 16 : 0);
                     const int w_left = at + nl - 1, w_right = at + nl;
                     if (corner) {
                         tb.seg[2 * h] = at; tb.segstream[2 * h] = 2 * h + 1; tb.segw[2 * h] = w_right;
@@ -430,6 +449,12 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
             }
             __syncthreads();
             const int W = __builtin_amdgcn_readfirstlane((int)misc[dWin]);
+            // (where the composite's steps go: a table of its own, or the room of the ranking's lists)
+            auto step_table = [&](const DenseTables& tb) __attribute__((always_inline)) {
+                if constexpr (!WINDOWS) return tb.rank16;
+                ArgsPtr args = fresh_args();
+                return reinterpret_cast<uint16_t*>(smem + args->y.off_tab) + m * args->y.tab_cap;
+            };
 
             // The step of every window is its place in the order of priorities, stored doubled with bit 0
             // set: a lookup subtracts one where the point is not the window's first lane, which
@@ -480,9 +505,10 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
                         for (int i = 0; i < E; i++) v[i] = s64[lane * E + i];
                         wave_sort_u64(v, lane);
                         __builtin_amdgcn_wave_barrier();                // the table takes the words' room
+                        uint16_t* steps = step_table(tb);
 #pragma unroll
                         for (int i = 0; i < E; i++)
-                            if (v[i] != ~0ull) tb.rank16[(uint32_t)v[i] & 0xffffu] = step_of(v[i], lane * E + i);
+                            if (v[i] != ~0ull) steps[(uint32_t)v[i] & 0xffffu] = step_of(v[i], lane * E + i);
                     }
                 };
                 if (np == kWave) by_one_wave(std::integral_constant<int, 1>{});
@@ -497,9 +523,10 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
 #pragma unroll
                         for (int e = 0; e < 2; e++) mine[e] = e * NT < np ? s64[e * NT + tid] : 0ull;
                         __syncthreads();                    // the table takes the sorted words' room
+                        uint16_t* steps = step_table(tb);
 #pragma unroll
                         for (int e = 0; e < 2; e++)
-                            if (e * NT + tid < W) tb.rank16[(uint32_t)mine[e] & 0xffffu] = step_of(mine[e], e * NT + tid);
+                            if (e * NT + tid < W) steps[(uint32_t)mine[e] & 0xffffu] = step_of(mine[e], e * NT + tid);
                     }
                 }
             }
@@ -605,13 +632,14 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
                     kWaves * kWlist * 2 / 8, tid, fix_rank, fix_place, before);
                 if (ranked) {
                     __syncthreads();                    // the table takes the lists' room
+                    uint16_t* steps = step_table(tb);
                     int own = W - tid * IPT;            // (opaque: no lane masks kept for it across the ranking)
                     asm volatile("" : "+v"(own));
 #pragma unroll
                     for (int r = 0; r < IPT; r++)
-                        if (r < own) tb.rank16[rp[r] & 0xffffu] = (uint16_t)(((rp[r] >> 16) << 1) | 1);
+                        if (r < own) steps[rp[r] & 0xffffu] = (uint16_t)(((rp[r] >> 16) << 1) | 1);
                     __syncthreads();
-                    if (fix_rank >= 0) tb.rank16[fix_place] = (uint16_t)((fix_rank << 1) | 1);
+                    if (fix_rank >= 0) steps[fix_place] = (uint16_t)((fix_rank << 1) | 1);
                 }
             }
             if (ranked) break;
@@ -636,12 +664,13 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
                 const uint32_t varying = misc[dOr] ^ misc[dAnd];
                 lds_radix_passes<NT, IPT>(k, rp, tb.stage, tb.stage + IPT * NT + 4, scan_tmp, varying);
                 __syncthreads();
+                uint16_t* steps = step_table(tb);
                 uint32_t no_step = 0;
 #pragma unroll
                 for (int r = 0; r < IPT; r++) {
                     const int sp = tid * IPT + r;
                     const bool never = k[r] >= kInfBits;
-                    if (sp < W) tb.rank16[rp[r] & 0xffffu] = never ? (uint16_t)kNever : (uint16_t)((sp << 1) | 1);      // (the first W sorted items are the windows)
+                    if (sp < W) steps[rp[r] & 0xffffu] = never ? (uint16_t)kNever : (uint16_t)((sp << 1) | 1);      // (the first W sorted items are the windows)
                     no_step += sp < W && never ? 1u : 0u;
                 }
                 if (no_step) atomicAdd(&misc[dNoStep], no_step);
@@ -664,6 +693,7 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
             // phase is bound by vector-ALU issue, so the lookups are kept branch-free and short:
             // for a power-of-two T two points at a time in packed 16-bit arithmetic, otherwise
             // with 24-bit multiplies (32-bit ones run at a quarter of the rate).
+            if constexpr (!WINDOWS) {
             const uint16_t* invm = args->a.inv + (int64_t)m * args->a.L * args->a.N + off;
             auto store_time = [&](int pt, uint32_t b) __attribute__((always_inline)) {
                 const uint32_t old = tb.time[pt];      // ties: the earlier composite stays
@@ -813,22 +843,147 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
             }
             __syncthreads();
             PHASE_END(3);
+            }
         }
+        // ---- by windows: a point's windows in a composite end at the latest of their steps, and what the stop counts are the windows whose
+        // first lane is a point none of whose other windows there comes later.  So the first lanes of all windows are looked up instead of
+        // all points, and later the points of near tiles (25000 points, windows of 128, 24 simple indices: 4700 first lanes, 600000 positions).
+        // A point's positions lie side by side (point_rows), eight at a time: 16 bytes for each look-up of a composite.  Bound by the
+        // reads, each from a line of its own, and their latency: several points a lane are under way together.  Without a time per point an
+        // item takes 28 instead of 75 KB of LDS: four workgroups of four wavefronts to a CU instead of two of eight.  (512 queries on 10M unit
+        // vectors of 96, 51700 items: 12.8 -> 6.6 ms in all, with the candidates of near tiles listed together, below.)
+        const int lp = (args->a.L + 7) & ~7;
+        // the latest (doubled, with bit 0 set, or kNever) of the steps of the windows that hold points pts under composites ms
+        auto latest = [&](auto utag, const int (&pts)[decltype(utag)::value], const int (&ms)[decltype(utag)::value],
+                          uint32_t (&late)[decltype(utag)::value]) __attribute__((always_inline)) {
+            constexpr int U = decltype(utag)::value;
+            ArgsPtr args = fresh_args();
+            const int L = args->a.L, M = args->a.M;
+            const uint16_t* rows = args->a.point_rows + off * M * lp;
+            const uint32_t tab_at = (uint32_t)(uintptr_t)(lds_u16*)reinterpret_cast<uint16_t*>(smem + args->y.off_tab);
+            const uint32_t q_sh = T <= 256 ? 8u : 0u, q_magic = (uint32_t)(((1ull << (32 - q_sh)) + (uint32_t)T - 1) / (uint32_t)T);
+#pragma unroll
+            for (int u = 0; u < U; u++) late[u] = 0;
+            for (int h0 = 0; h0 < L; h0 += 8) {
+                u32x4 v[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) v[u] = *reinterpret_cast<const u32x4*>(rows + (uint32_t)((pts[u] * M + ms[u]) * lp + h0));
+                auto four = [&](int half) __attribute__((always_inline)) {
+                    uint32_t at[4][U];                       // the windows' places in the tables, then their steps
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+#pragma unroll
+                        for (int u = 0; u < U; u++) {
+                            const int i = ms[u] * L + min(h0 + 4 * half + e, L - 1);      // (past the last: that one again, here and in the table)
+                            const uint32_t place = (uint32_t)tb.shift[i];
+                            const uint32_t wd = half ? (e < 2 ? v[u].z : v[u].w) : (e < 2 ? v[u].x : v[u].y);
+                            const uint32_t xs = ((e & 1 ? wd >> 16 : wd & 0xffffu) + (place & 0xffffu)) << q_sh;
+                            uint32_t w;
+                            asm("v_mul_hi_u32_u24 %0, %1, %2" : "=v"(w) : "s"(q_magic), "v"(xs));
+                            at[e][u] = tab_at + 2 * (w + (place >> 16));
+                        }
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+#pragma unroll
+                        for (int u = 0; u < U; u++) late[u] = max(late[u], (uint32_t)*(const lds_u16*)at[e][u]);
+                };
+                four(0);
+                if (h0 + 4 < L) four(1);
+            }
+        };
         // ---- stop step from the histogram of the steps of lane-0 candidates -----------
         const int HW = ((int)maxw + 2) / 2;                 // 32-bit words of the histogram (two steps each)
-        for (int w = tid; w < HW; w += NT) tb.stage[w] = 0;
-        if (tid == 0) { misc[dArmed] = 0xffffffffu; misc[dMaxc] = 0xffffffffu; }
+        uint32_t* hist = WINDOWS ? reinterpret_cast<uint32_t*>(smem + args->y.off_hist) : tb.stage;
+        for (int w = tid; w < HW; w += NT) hist[w] = 0;
+        if (tid == 0) { misc[dArmed] = 0xffffffffu; misc[dMaxc] = 0xffffffffu; misc[dMore] = 0; }
         __syncthreads();
-        for (int pt = tid; pt < n; pt += NT) {
-            const uint32_t v = tb.time[pt];
-            if ((v & 1u) && (v >> 1) != (kNever & 0x7fffu)) atomicAdd(&tb.stage[v >> 2], 1u << (((v >> 1) & 1u) * 16));
+        if constexpr (WINDOWS) {
+            // (step, composite, point) of the first lanes that are promoted there, then of those those that no composite promotes sooner
+            constexpr int kListed = NT * IPT / 2, U = 4;
+            constexpr unsigned long long kSooner = 1ull << 63;
+            unsigned long long* list = reinterpret_cast<unsigned long long*>(tb.stage);
+            const uint16_t* tab = reinterpret_cast<const uint16_t*>(smem + args->y.off_tab);
+            const int M = args->a.M, L = args->a.L;
+            auto sooner = [&](uint32_t late, int m, uint32_t step, int own) { return (late >> 1) < step || ((late >> 1) == step && m < own); };
+            const int parts = n / (T * kWave) + 1, wave_s = __builtin_amdgcn_readfirstlane(wave);      // (of 64 windows, of a simple index)
+            for (int c0 = wave_s * U; c0 < I * parts; c0 += kWaves * U) {
+                int pts[U], ms[U];
+                uint32_t mine[U], late[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int c = min(c0 + u, I * parts - 1), i = c / parts;
+                    const uint32_t place = (uint32_t)tb.shift[i];
+                    const int shift = (int)(place & 0xffffu);
+                    const int j = (shift + T - 1) / T + (c - i * parts) * kWave + lane, at = j * T - shift;
+                    mine[u] = c0 + u < I * parts && at < n ? (uint32_t)tab[(place >> 16) + (uint32_t)j] : kNever;
+                    ms[u] = i / L;
+                    pts[u] = args->a.sids[(int64_t)i * args->a.N + off + min(at, n - 1)];
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) pts[u] -= (int)off;
+                latest(std::integral_constant<int, U>{}, pts, ms, late);
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const bool in = mine[u] != kNever && late[u] <= mine[u];
+                    const unsigned long long all = __ballot(in);
+                    if (all == 0) continue;
+                    uint32_t first = 0;
+                    if (lane == 0) first = atomicAdd(&misc[dMore], (uint32_t)__popcll(all));
+                    first = (uint32_t)__builtin_amdgcn_readfirstlane((int)first);
+                    const uint32_t slot = first + (uint32_t)__popcll(all & ((1ull << lane) - 1ull));
+                    if (in && slot < (uint32_t)kListed)
+                        list[slot] = ((unsigned long long)(mine[u] >> 1) << 32) | ((uint32_t)ms[u] << 16) | (uint32_t)pts[u];
+                    if (first + (uint32_t)__popcll(all) > (uint32_t)kListed) {      // (no room left: looked at here)
+                        bool real = in && slot >= (uint32_t)kListed;
+                        for (int m = 0; m < M; m++) {
+                            const int one_pt[1] = {pts[u]}, one_m[1] = {m};
+                            uint32_t l1[1];
+                            latest(std::integral_constant<int, 1>{}, one_pt, one_m, l1);
+                            if (m != ms[u] && sooner(l1[0], m, mine[u] >> 1, ms[u])) real = false;
+                        }
+                        if (real) atomicAdd(&hist[mine[u] >> 2], 1u << ((mine[u] >> 1 & 1u) * 16));
+                    }
+                }
+            }
+            __syncthreads();
+            const int listed = min((int)misc[dMore], kListed), pairs = listed * (M - 1);      // (with every other composite)
+            for (int e0 = 0; e0 < pairs; e0 += NT * U) {
+                int pts[U], ms[U], es[U];
+                uint32_t late[U], step[U], own[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int e = min(e0 + u * NT + tid, pairs - 1), other = e / listed;
+                    es[u] = e - other * listed;
+                    const unsigned long long v = list[es[u]];
+                    pts[u] = (int)((uint32_t)v & 0xffffu);
+                    own[u] = (uint32_t)v >> 16;
+                    step[u] = (uint32_t)(v >> 32) & 0x7fffu;
+                    ms[u] = (int)own[u] + 1 + other;
+                    if (ms[u] >= M) ms[u] -= M;
+                }
+                latest(std::integral_constant<int, U>{}, pts, ms, late);
+#pragma unroll
+                for (int u = 0; u < U; u++)
+                    if (sooner(late[u], ms[u], step[u], (int)own[u])) reinterpret_cast<uint32_t*>(list)[2 * es[u] + 1] = (uint32_t)(kSooner >> 32);
+            }
+            if (pairs > 0) __syncthreads();
+            for (int e = tid; e < listed; e += NT) {
+                const uint32_t step = (uint32_t)(list[e] >> 32);
+                if (!(step >> 31)) atomicAdd(&hist[step >> 1], 1u << ((step & 1u) * 16));
+            }
+        } else {
+            for (int pt = tid; pt < n; pt += NT) {
+                const uint32_t v = tb.time[pt];
+                if ((v & 1u) && (v >> 1) != (kNever & 0x7fffu)) atomicAdd(&hist[v >> 2], 1u << (((v >> 1) & 1u) * 16));
+            }
         }
         __syncthreads();
         {
             const int per = (HW + NT - 1) / NT;           // words per thread, contiguous
             const int w0 = tid * per, w1 = min(HW, w0 + per);
             uint32_t sum = 0;
-            for (int w = w0; w < w1; w++) { const uint32_t v = tb.stage[w]; sum += (v & 0xffffu) + (v >> 16); }
+            for (int w = w0; w < w1; w++) { const uint32_t v = hist[w]; sum += (v & 0xffffu) + (v >> 16); }
             uint32_t incl = sum;
 #pragma unroll
             for (int o = 1; o < kWave; o <<= 1) {
@@ -842,7 +997,7 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
             const uint32_t need_k = (uint32_t)args->a.k_stop;
             const uint32_t need_c = (uint32_t)min((int64_t)0x7fffffff, max((int64_t)1, args->a.max_cand));
             for (int w = w0; w < w1; w++) {
-                const uint32_t v = tb.stage[w];
+                const uint32_t v = hist[w];
                 const uint32_t c_lo = run + (v & 0xffffu), c_hi = c_lo + (v >> 16);
                 if (run < need_k && c_lo >= need_k) atomicMin(&misc[dArmed], (uint32_t)(2 * w));
                 else if (c_lo < need_k && c_hi >= need_k) atomicMin(&misc[dArmed], (uint32_t)(2 * w + 1));
@@ -885,14 +1040,19 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
         uint32_t* near_bits = scan_tmp + 48;
         const bool near = PICKED && args->a.near_bounds != nullptr;
         const int near_shift = args->a.near_shift;
+        uint16_t* near_list = reinterpret_cast<uint16_t*>(tb.stage);      // the near tiles
         if (near) {
             if (tid < 16) near_bits[tid] = 0;
+            if (tid == 0) { misc[dMore] = 0; misc[dWin] = 0; }
             __syncthreads();
             const float most = args->a.near_limit[(int64_t)qi * args->a.near_stride];
             const uint32_t* bounds = args->a.near_bounds + (int64_t)b * args->a.near_tiles * args->a.nq + qi;
             const int tiles = (n + (1 << near_shift) - 1) >> near_shift;
             for (int t = tid; t < tiles; t += NT)
-                if (!(__builtin_bit_cast(float, bounds[(int64_t)t * args->a.nq]) > most)) atomicOr(&near_bits[t >> 5], 1u << (t & 31));
+                if (!(__builtin_bit_cast(float, bounds[(int64_t)t * args->a.nq]) > most)) {
+                    atomicOr(&near_bits[t >> 5], 1u << (t & 31));
+                    near_list[atomicAdd(&misc[dMore], 1u)] = (uint16_t)t;
+                }
             __syncthreads();
         }
         // lists at least `want` candidates, while points are left
@@ -913,7 +1073,19 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
                     list_pos = 0;
                 }
                 const int pt = at + lane;
-                const uint32_t v = pt < end ? (uint32_t)tb.time[pt] : 0xffffu;
+                uint32_t v = 0xffffu;
+                if constexpr (WINDOWS) {
+                    const int pts[1] = {min(pt, end - 1)};
+                    for (int m = 0; m < fresh_args()->a.M; m++) {
+                        const int ms[1] = {m};
+                        uint32_t late[1];
+                        latest(std::integral_constant<int, 1>{}, pts, ms, late);
+                        v = min(v, late[0]);
+                    }
+                    if (pt >= end) v = 0xffffu;
+                } else if (pt < end) {
+                    v = tb.time[pt];
+                }
                 const bool is_cand = (v >> 1) <= t_lim;
                 const unsigned long long m = __ballot(is_cand);
                 if (is_cand) wl[list_len + __popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)pt;
@@ -1091,14 +1263,151 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
         // Bound by the latency of the records' reads (eight 16-byte reads per lane under way).  12801 candidates
         // of 96 elements, k = 100, two workgroups per CU: 75 us per item, 140 by whole rows; 1285 of 960
         // elements, k = 10: 55, and 198 by whole rows.
-        uint32_t* hist = tb.stage;
+        unsigned long long* res = tb.sortbuf;                      // where the result lies
+        // ---- few candidates in near tiles, as nearly always: all wavefronts list them together, form their distances, eight rows and more to a
+        // wavefront under way, and sort them.  (3.5 tiles of 128 rows and 230 candidates an item, k = 100: 51 us when every wavefront kept to its
+        // share of the points, most of them waiting for one.)
+        bool few = false;
+        if (near) {
+            const int tiles = (int)misc[dMore];
+            // room: the tiles, the results, the candidates
+            const int tile_bytes = (2 * tiles + 7) & ~7;
+            int room = NT;
+            while (room < 1024 && tile_bytes + 2 * room * 10 <= args->y.whole_bytes) room <<= 1;
+            res = reinterpret_cast<unsigned long long*>(reinterpret_cast<unsigned char*>(tb.stage) + tile_bytes);
+            uint16_t* cand = reinterpret_cast<uint16_t*>(res + room);
+            if (tile_bytes + room * 10 <= args->y.whole_bytes) {
+                constexpr int U = WINDOWS ? 2 : 1;
+                const int rows = tiles << near_shift;
+                for (int r0 = 0; r0 < rows; r0 += NT * U) {
+                    int pts[U];
+                    uint32_t v[U];
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        const int r = r0 + u * NT + tid;
+                        const int pt = r < rows ? ((int)near_list[r >> near_shift] << near_shift) + (r & ((1 << near_shift) - 1)) : n;
+                        v[u] = pt < n ? 0u : 0xffffu;
+                        pts[u] = min(pt, n - 1);
+                    }
+                    if constexpr (WINDOWS) {
+                        uint32_t first[U];
+#pragma unroll
+                        for (int u = 0; u < U; u++) first[u] = 0xffffu;
+                        for (int m = 0; m < fresh_args()->a.M; m++) {
+                            int ms[U];
+                            uint32_t late[U];
+#pragma unroll
+                            for (int u = 0; u < U; u++) ms[u] = m;
+                            latest(std::integral_constant<int, U>{}, pts, ms, late);
+#pragma unroll
+                            for (int u = 0; u < U; u++) first[u] = min(first[u], late[u]);
+                        }
+#pragma unroll
+                        for (int u = 0; u < U; u++) v[u] = max(v[u], first[u]);
+                    } else {
+#pragma unroll
+                        for (int u = 0; u < U; u++) v[u] = max(v[u], (uint32_t)tb.time[pts[u]]);
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        const bool in = (v[u] >> 1) <= t_lim;
+                        const unsigned long long all = __ballot(in);
+                        if (all == 0) continue;
+                        uint32_t slot = 0;
+                        if (lane == 0) slot = atomicAdd(&misc[dWin], (uint32_t)__popcll(all));
+                        slot = (uint32_t)__builtin_amdgcn_readfirstlane((int)slot) + (uint32_t)__popcll(all & ((1ull << lane) - 1ull));
+                        if (in && slot < (uint32_t)room) cand[slot] = (uint16_t)pts[u];
+                    }
+                }
+                __syncthreads();
+                const int count = __builtin_amdgcn_readfirstlane((int)misc[dWin]);
+                if (count <= room) {
+                    few = true;
+                    fresh_thread_ids();
+                    // GL lanes to a row of at most 4 GL elements, eight rows to a lane group; the sums and their order are those of wave_row_dists
+                    auto some_rows = [&](auto gtag) __attribute__((always_inline)) {
+                        constexpr int GL = decltype(gtag)::value, kRows8 = 8 * (kWave / GL);
+                        const int grp = lane / GL, sl = lane & (GL - 1), j = sl * 4;
+                        const bool has = j < args->a.dim;
+                        float q0 = 0.f, q1 = 0.f, q2 = 0.f, q3 = 0.f;
+                        if (has) { q0 = tb.q[j]; q1 = tb.q[j + 1]; q2 = tb.q[j + 2]; q3 = tb.q[j + 3]; }
+                        const float* base = args->a.data + off * args->a.dim + (has ? j : 0);
+                        for (int c0 = wave * kRows8; c0 < count; c0 += kWaves * kRows8) {
+                            float acc[8];
+                            v4f x[8];
+#pragma unroll
+                            for (int r = 0; r < 8; r++) x[r] = *reinterpret_cast<const v4f*>(base + (int)cand[min(c0 + grp * 8 + r, count - 1)] * args->a.dim);
+#pragma unroll
+                            for (int r = 0; r < 8; r++) {
+                                float s2 = 0.f;
+                                float dd = x[r].x - q0; s2 = __builtin_fmaf(dd, dd, s2);
+                                dd = x[r].y - q1; s2 = __builtin_fmaf(dd, dd, s2);
+                                dd = x[r].z - q2; s2 = __builtin_fmaf(dd, dd, s2);
+                                dd = x[r].w - q3; s2 = __builtin_fmaf(dd, dd, s2);
+                                acc[r] = has ? s2 : 0.f;
+                            }
+                            float v4[4], v2[2];
+#pragma unroll
+                            for (int i = 0; i < 4; i++) {
+                                const bool up = (sl & (GL / 2)) != 0;
+                                v4[i] = (up ? acc[i + 4] : acc[i]) + lane_xor<GL / 2>(up ? acc[i] : acc[i + 4]);
+                            }
+#pragma unroll
+                            for (int i = 0; i < 2; i++) {
+                                const bool up = (sl & (GL / 4)) != 0;
+                                v2[i] = (up ? v4[i + 2] : v4[i]) + lane_xor<GL / 4>(up ? v4[i] : v4[i + 2]);
+                            }
+                            const bool up = (sl & (GL / 8)) != 0;
+                            float v = (up ? v2[1] : v2[0]) + lane_xor<GL / 8>(up ? v2[0] : v2[1]);
+                            if constexpr (GL > 16) v += lane_xor<2>(v);
+                            v += lane_xor<1>(v);
+                            const int c = c0 + grp * 8 + sl / (GL / 8);
+                            if ((sl & (GL / 8 - 1)) == 0 && c < count) res[c] = pack(__builtin_bit_cast(uint32_t, sqrtf(v)), (int)cand[c]);
+                        }
+                    };
+                    if (!args->y.tiles) {
+                        for (int c0 = wave_u * 8; c0 < count; c0 += kWaves * 8) {
+                            int pts[8];
+#pragma unroll
+                            for (int r = 0; r < 8; r++) pts[r] = (int)cand[min(c0 + r, count - 1)];
+                            const float d = eight_rows(pts);
+                            const int c = c0 + (lane >> 3);
+                            if ((lane & 7) == 0 && c < count) res[c] = pack(__builtin_bit_cast(uint32_t, d), (int)cand[c]);
+                        }
+                    } else if (args->a.dim <= 64) {
+                        some_rows(std::integral_constant<int, 16>{});
+                    } else {
+                        some_rows(std::integral_constant<int, 32>{});
+                    }
+                    int np = count <= kWave ? kWave : NT;
+                    while (np < count) np <<= 1;
+                    for (int j = count + tid; j < np; j += NT) res[j] = ~0ull;
+                    if (NT > kWave && np == kWave) {
+                        __syncthreads();
+                        if (wave == 0) {
+                            unsigned long long v[1] = {res[lane]};
+                            wave_sort_u64(v, lane);
+                            res[lane] = v[0];
+                        }
+                        __syncthreads();
+                    } else {
+                        bitonic_sort_u64_by<NT, NT == 64 ? 4 : 2>(res, np, tid);
+                    }
+                    topn = min(count, args->a.kcap);
+                    if (wave == 0) ncand = (uint32_t)count;
+                    if (tid == 0 && misc[dUse8] == kCodesDoubted) misc[dUse8] = kCodesOn;      // (the codes were not asked)
+                    if (tid == 0 && misc[dUse8] == kCodesTried) misc[dUse8] = kCodesTried + kCodesFailed;
+                }
+            }
+            __syncthreads();
+        }
+        uint32_t* bins = tb.stage;
         unsigned long long cut = ~0ull;                         // entries above it are out
         unsigned long long pend = ~0ull;                        // lane's entry of a batch that did not fit the share
         bool have_pend = false, first = true, last = false;
         float h_lo = 0.f, h_scale = 0.f;                        // (no histogram while the scale is 0)
         int batches = 0;
-        unsigned long long* res = tb.sortbuf;                      // where the result lies
-        for (;;) {
+        while (!few) {
             const bool codes = path >= kCodes8;
             const int front = codes ? args->y.front8 : args->a.kcap, quota = codes ? args->y.quota8 : args->y.quota;
             const int CB = path == kRows ? 8 : (path == kCodes64 ? 32 : kWave);
@@ -1110,10 +1419,10 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
             //  be counted among the nearest, where the conversion would put it)
             auto count = [&](bool keep, unsigned long long e) {
                 const float at_bin = (score(e) - h_lo) * h_scale;
-                if (keep && at_bin < (float)kBins) atomicAdd(&hist[max(0, (int)at_bin)], 1u);
+                if (keep && at_bin < (float)kBins) atomicAdd(&bins[max(0, (int)at_bin)], 1u);
             };
             auto tighten = [&]() {
-                const u32x4 c = reinterpret_cast<const u32x4*>(hist)[lane];
+                const u32x4 c = reinterpret_cast<const u32x4*>(bins)[lane];
                 const uint32_t c1 = c.x + c.y, c2 = c1 + c.z, upto = wave_scan_u32(c2 + c.w), before = upto - (c2 + c.w);
                 const uint32_t want = (uint32_t)args->a.kcap;
                 const unsigned long long m = __ballot(upto >= want);
@@ -1181,7 +1490,7 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
                         valid = (lane & 7) == 0 && (lane >> 3) < nb;
                     } else {      // blind: scored by the promoting step (:498-505), no row is read
                         const int pt = (int)cur[min(lane, nb - 1)];
-                        e = pack((uint32_t)tb.time[pt] >> 1, pt);
+                        e = pack(WINDOWS ? 0u : (uint32_t)tb.time[pt] >> 1, pt);
                     }
                     list_pos += nb;
                     batches++;
@@ -1204,7 +1513,7 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
                     const uint32_t least = wave_min_u32(bits);
                     const int most = wave_max_i32(bits == 0x7fffffffu ? 0 : (int)bits);
                     if (lane == 0) { scan_tmp[24 + wave] = least; scan_tmp[40 + wave] = (uint32_t)most; }
-                    for (int j = tid; j < kBins; j += NT) hist[j] = 0;
+                    for (int j = tid; j < kBins; j += NT) bins[j] = 0;
                     __syncthreads();
                     uint32_t lo = 0x7fffffffu, hi = 0;
                     for (int w2 = 0; w2 < kWaves; w2++) { lo = min(lo, scan_tmp[24 + w2]); hi = max(hi, scan_tmp[40 + w2]); }
@@ -1353,20 +1662,26 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
 
 #undef PHASE_END
 
-template <int NT, int IPT, int WAVES, bool PICKED>
+template <int NT, int IPT, int WAVES, int KIND>
 int launch_dense(const DenseArgs& args, unsigned grid, hipStream_t s) {
     static DeviceOnce once;
     const int rc = once.run([]() -> int {
-        DCIH_HIP(hipFuncSetAttribute((const void*)traverse_dense_kernel<NT, IPT, WAVES, PICKED>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        DCIH_HIP(hipFuncSetAttribute((const void*)traverse_dense_kernel<NT, IPT, WAVES, KIND>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         return 0;
     });
     if (rc) return rc;
-    hipLaunchKernelGGL((traverse_dense_kernel<NT, IPT, WAVES, PICKED>), dim3(grid), dim3(NT), args.y.lds_bytes, s, args);
+    hipLaunchKernelGGL((traverse_dense_kernel<NT, IPT, WAVES, KIND>), dim3(grid), dim3(NT), args.y.lds_bytes, s, args);
     DCIH_HIP(hipGetLastError());
     return 0;
 }
 
 }  // namespace
+
+// By windows: n / T + 3 first lanes of every simple index cost two reads from random lines and L look-ups each, by points
+// every one of the n costs one look-up that a coalesced read feeds; a read of a line of its own takes as long as a dozen look-ups.
+bool point_rows_pay(int64_t ppb, int M, int L, int T) {
+    return ppb <= 32766 && (double)(ppb / T + 3) * (double)(L + 24) < 0.7 * (double)ppb && (int64_t)L * (ppb / T + 3) <= 9 * 512 && M <= 64 && L <= 64;
+}
 
 bool dense_traversal_supported(const QueryArgs& a, size_t* lds_bytes) {
     if (!a.inv || a.ppb > 32766 || a.T < 1) return false;
@@ -1421,7 +1736,9 @@ int query_dense_items(const QueryArgs& a_in, hipStream_t s) {
         args.step = (int)(per_xcd - resident);
     }
     const unsigned grid = (unsigned)(per_xcd * a.xcds);
-#define DCIH_DENSE(NT, IPT, WAVES) rc = a.picked ? launch_dense<NT, IPT, WAVES, true>(args, grid, s) : launch_dense<NT, IPT, WAVES, false>(args, grid, s)
+#define DCIH_DENSE(NT, IPT, WAVES) \
+    rc = y.by_windows && IPT <= 9 ? launch_dense<NT, IPT, WAVES, IPT <= 9 ? kWindows : kPicked>(args, grid, s) \
+         : (a.picked ? launch_dense<NT, IPT, WAVES, kPicked>(args, grid, s) : launch_dense<NT, IPT, WAVES, kWhole>(args, grid, s))
     int rc;
     if (y.nt == 64) {
         if (y.ipt == 5) DCIH_DENSE(64, 5, 4); else DCIH_DENSE(64, 9, 4);

@@ -106,6 +106,27 @@ def test_rows_of_every_kind(gpu, kind, shape, dim):
     assert ids.shape == (150, k)
 
 
+# Wide windows: the first lanes of the windows and the rows of near tiles are looked up instead of all points, with positions side by side in
+# eights (one, a whole eight, one more, two eights less one), windows of and not of a power of two, above 256; formed once enough was asked for.
+@pytest.mark.parametrize("kind", ["normal", "sorted", "dup", "whole", "broken", "zero"])
+@pytest.mark.parametrize("shape", [(9001, 24, 1, 1, 3, 64, 5, 400), (20000, 96, 3, 8, 4, 128, 100, 100), (9000, 33, 2, 9, 5, 100, 10, 60),
+                                   (30000, 16, 2, 15, 4, 64, 9, 50), (24000, 200, 2, 4, 2, 300, 20, 40), (2400, 64, 4, 5, 6, 48, 3, 30)],
+                         ids=["one", "eight", "nine", "fifteen", "four", "short"])
+def test_wide_windows(gpu, kind, shape):
+    n, dim, M, L, B, T, k, outer = shape
+    X, Q = _rows(kind, n, 70, dim, n + dim)
+    dci = gpu.DCI(dim, M, L, B, T, seed=5)
+    dci.add(X)
+    want = _ask(dci, dci._lib, NEVER, Q, k, outer)
+    for again in range(3):
+        got = _ask(dci, dci._lib, ALWAYS, Q, k, outer)
+        assert _route(dci)[0] >= 2, again
+        assert torch.equal(got[0], want[0]), again
+        assert torch.equal(got[1].view(torch.int32), want[1].view(torch.int32)), again
+    assert _route(dci)[1] == 1
+    dci.free()
+
+
 @pytest.mark.parametrize("n,B", [(130, 2), (257, 128), (1000, 999), (4096, 32), (4097, 32), (31 * 129, 31)])
 def test_partitions_at_the_edges_of_tiles(gpu, n, B):
     """Partitions of 1, 2, 3, 65, 128, 129 rows, some of them empty, more results asked for than a partition holds."""
