@@ -320,7 +320,7 @@ ArenaLayout arena_layout(int M, int L, int64_t n, int block_size, int thread_siz
     y.inv = y.ids + b_ids;
     y.rpos = y.inv + b_inv;
     y.point_rows = y.rpos + b_inv;
-    y.point_rows_pay = y.small_parts && point_rows_pay((n + block_size - 1) / block_size, M, L, thread_size);
+    y.point_rows_pay = y.small_parts && point_rows_fit((n + block_size - 1) / block_size, M, L, thread_size);
     y.hint = y.point_rows + (y.point_rows_pay ? align_up(point_rows_bytes(n, M, L)) : 0);
     y.total = y.hint + b_hint;
     return y;
@@ -839,7 +839,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     }
     if (rc) return rc;
     // A point's positions side by side for the dense kernel's near rows.  To form them takes as long as the look-ups of all points by eight queries.
-    if (a.pick_rounds && a.pick_near && h->d_point_rows && point_rows_pay(a.ppb, a.M, a.L, a.T)) {
+    if (a.pick_rounds && a.pick_near && h->d_point_rows && point_rows_fit(a.ppb, a.M, a.L, a.T) && point_rows_pay(a)) {
         h->point_rows_demand += (double)num_queries * a.share;
         if (!h->point_rows_ready && h->point_rows_demand >= kPointRowsDemand) {
             rc = fill_point_rows(h->d_inv, h->d_point_rows, h->n, h->M, h->L, s);

@@ -52,7 +52,7 @@ int fill_positions_by_first(const int32_t* d_sids, const uint16_t* d_inv, uint16
 // point_rows from inv (see QueryArgs), and whether the dense kernel's calls in rounds are better off with them.
 size_t point_rows_bytes(int64_t n, int M, int L);
 int fill_point_rows(const uint16_t* d_inv, uint16_t* d_rows, int64_t n, int M, int L, hipStream_t s);
-bool point_rows_pay(int64_t ppb, int M, int L, int T);
+bool point_rows_fit(int64_t ppb, int M, int L, int T);
 
 struct QueryArgs {
     const float* skeys;      // [I][N] sorted projections
@@ -244,6 +244,7 @@ int query_block(const QueryArgs& a, hipStream_t s);
 // through the lists the batch kernel filled (a.dense_items) or, with a.mode == 3,
 // through all items.
 bool dense_traversal_supported(const QueryArgs& a, size_t* lds_bytes);
+bool point_rows_pay(const QueryArgs& a);
 int query_dense_items(const QueryArgs& a, hipStream_t s);
 
 // 8-bit codes of rows and queries (rows8.hip); bounds: 3 * B words.

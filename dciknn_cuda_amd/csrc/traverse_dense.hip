@@ -90,7 +90,7 @@ constexpr int kBins = 256;               // of the histogram of scores, which li
 // ceil((p+1)/T) + floor((n+T-3-p)/T) + 1 <= n/T + 3.  (A layout holds that many, so every item fits it.)
 int64_t dense_max_windows(const QueryArgs& a) { return (int64_t)a.L * (a.ppb / a.T + 3); }
 
-// (point_rows are there where the rule of point_rows_pay says so)
+// (point_rows are there where the rules of point_rows_fit and point_rows_pay say so)
 bool by_windows(const QueryArgs& a) { return a.picked && a.near_bounds && a.point_rows && dense_max_windows(a) <= 9 * 512 && a.M * (dense_max_windows(a) + 1) < 32768; }
 
 DenseLayout dense_layout_for(const QueryArgs& a, int nt, int ipt) {
@@ -1679,7 +1679,13 @@ int launch_dense(const DenseArgs& args, unsigned grid, hipStream_t s) {
 
 // By windows: n / T + 3 first lanes of every simple index cost two reads from random lines and L look-ups each, by points
 // every one of the n costs one look-up that a coalesced read feeds; a read of a line of its own takes as long as a dozen look-ups.
-bool point_rows_pay(int64_t ppb, int M, int L, int T) {
+// That line is where the room for them is kept.  What decides beyond it is the LDS: a time for every point leaves two workgroups to a CU from about
+// 16000 points on (1M rows, 12 indices, windows of 96 in partitions of 25000: 6.17 ms by points, 3.29 by windows; 8 indices, windows of 64, 16667: 2.47,
+// 1.81; of 10000, windows of 64 to 128, four kinds of rows: 0.96 to 1.06; below, 0.80 to 1.07), and calls that wait for single items lose a tenth.
+bool point_rows_pay(const QueryArgs& a) {
+    return a.pick_rule == 2 || (a.ppb >= 8000 && (double)a.nq * (double)a.B * a.share >= 4096.0);
+}
+bool point_rows_fit(int64_t ppb, int M, int L, int T) {
     return ppb <= 32766 && (double)(ppb / T + 3) * (double)(L + 24) < 0.7 * (double)ppb && (int64_t)L * (ppb / T + 3) <= 9 * 512 && M <= 64 && L <= 64;
 }
 
