@@ -159,7 +159,9 @@ struct dcih_index {
     int append_mode = 0;                // DCIH_OPT_APPEND value
     int rounds = 0;                     // DCIH_OPT_ROUNDS value
     int64_t route[4] = {0, 0, 0, 0};    // dcih_debug_route
-    volatile uint32_t* blind = nullptr; // (pinned) set by queries in rounds whose bounds said nothing: the next ones use the rows' codes
+    int confirm_rests = 0;              // calls in rounds that went without confirm.hip, since the last one with it
+    int index_calls = 0;                // queries since the index was formed
+    volatile uint32_t* blind = nullptr; // (pinned: three words) set by queries in rounds whose bounds said nothing: the next ones use the rows' codes; then the items that confirm.hip answered and left, of those it counts
     uint32_t* d_round_items = nullptr;  // dcih_debug_round_items
     unsigned long long* d_phase_ticks = nullptr;   // optional profile of the batch kernel
     // grow-only workspace: query scratch, and the unsorted keys during a build
@@ -482,6 +484,7 @@ static int sort_into(dcih_index* h, int which, const float* d_keys, int64_t key_
     h->d_skeys = skeys; h->d_sids = sids; h->d_inv = inv; h->d_stop_hint = hint;
     h->d_rpos = y.small_parts ? (uint16_t*)(base + y.rpos) : nullptr;
     h->rpos_ready = 0;
+    h->index_calls = 0;
     h->d_point_rows = y.point_rows_pay ? (uint16_t*)(base + y.point_rows) : nullptr;
     h->point_rows_ready = 0;
     h->point_rows_demand = 0.0;
@@ -706,12 +709,14 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     a.hand_over_at = 0;
     a.expect_steps = a.expect_promotions = 0.0f;
     a.rows8 = nullptr; a.rows8_rec = 0; a.rows8_bounds = nullptr; a.query8 = nullptr;
-    a.picked = nullptr; a.picked_count = nullptr; a.picked_exact = a.picked_cover = a.picked_expect = 0; a.picked_ticket = nullptr; a.only = nullptr; a.only_round = 0;
-    a.share = 1.0; a.pick_first = 0.0; a.pick_rounds = a.pick_rank = a.pick_near = a.pick_sample = 0; a.pick_most = 1.0f;
+    a.picked = nullptr; a.picked_count = nullptr; a.picked_exact = a.picked_cover = a.picked_expect = 0; a.picked_ticket = nullptr; a.left = nullptr; a.left_count = nullptr; a.left_cap = 0; a.only = nullptr; a.only_round = 0;
+    a.share = 1.0; a.pick_first = 0.0; a.pick_rounds = a.pick_rank = a.pick_near = a.pick_confirm = a.pick_sample = 0; a.pick_most = 1.0f;
     a.near_bounds = nullptr; a.near_limit = nullptr; a.near_stride = 0; a.near_shift = a.near_tiles = 0; a.pick_rule = fixed || whole ? 1 : h->rounds;
     a.phase_ticks = h->d_phase_ticks;
     a.round_items = h->d_round_items;
-    a.blind_word = nullptr;
+    a.blind_word = a.confirm_word = nullptr;
+    a.confirm_had = a.confirm_lost = 0;
+    a.confirm_again = a.index_calls = 0;
     a.selected = &h->route[3];
     a.stop_hint = nullptr;
     a.N = h->n;
@@ -777,15 +782,20 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
         return rc;
     }
 
+    // (where earlier calls' items had to be left, every 64th call tries again)
+    if (h->blind) { a.confirm_had = h->blind[1]; a.confirm_lost = h->blind[2]; }
+    a.confirm_again = h->confirm_rests >= 63;
+    a.index_calls = h->index_calls++;
     (void)plan_rounds(a);
-    if (a.pick_near) {
+    h->confirm_rests = a.pick_rounds && !a.pick_confirm ? h->confirm_rests + 1 : 0;
+    if (a.pick_near || a.pick_confirm) {
         if (!h->blind && !recorded) {
             void* p = nullptr;
-            if (hipHostMalloc(&p, sizeof(uint32_t), hipHostMallocDefault) == hipSuccess) { h->blind = (volatile uint32_t*)p; *h->blind = 0; }
+            if (hipHostMalloc(&p, 3 * sizeof(uint32_t), hipHostMallocDefault) == hipSuccess) { h->blind = (volatile uint32_t*)p; h->blind[0] = h->blind[1] = h->blind[2] = 0; }
             else (void)hipGetLastError();
         }
         void* p = nullptr;
-        if (h->blind && hipHostGetDevicePointer(&p, (void*)h->blind, 0) == hipSuccess) a.blind_word = (uint32_t*)p;
+        if (h->blind && hipHostGetDevicePointer(&p, (void*)h->blind, 0) == hipSuccess) { a.blind_word = a.pick_near ? (uint32_t*)p : nullptr; a.confirm_word = (uint32_t*)p + 1; }
     }
     const bool bounds_failed = h->blind && *h->blind;      // (of earlier calls: it steers work, never results)
     size_t q8_bytes = 0;
@@ -987,6 +997,12 @@ int dcih_debug_route(const dcih_index* h, int64_t* route) {
 int dcih_debug_round_items(dcih_index* h, uint32_t* d_items) {
     if (!h) return fail(DCIH_EINVAL, "dcih_debug_round_items: null handle");
     h->d_round_items = d_items;
+    return DCIH_OK;
+}
+
+int dcih_debug_confirmed(const dcih_index* h, uint32_t* counts) {
+    if (!h || !counts) return fail(DCIH_EINVAL, "dcih_debug_confirmed: null argument");
+    for (int i = 0; i < 2; i++) counts[i] = h->blind ? h->blind[1 + i] : 0u;
     return DCIH_OK;
 }
 

@@ -44,7 +44,7 @@ namespace {
 
 constexpr int kWholeDim = 256;            // rows up to here can be kept in LDS whole
 constexpr int kMostParts = 2048;           // bounds kept per query
-constexpr int kLimits = kMostRounds;       // per query: of the rounds but the last, and round 1's limit of what is near
+constexpr int kLimits = kMostRounds;       // per query: of the rounds but the last, and how far a near row of round 1 may be
 constexpr int kMostDies = 32;             // tickets cleared
 constexpr int kListQueries = 1024;        // queries of a partition listed by one workgroup
 
@@ -495,7 +495,7 @@ __global__ __launch_bounds__(128 * WR * WC, WAVES) void bounds_stream_kernel(Bou
 // largest in the histogram's bins up to the one that holds it, 1024 bins over the range of those that are finite.  A workgroup reads the
 // bounds of `per` neighbouring queries into LDS first.  (Bit by bit, with a ballot per bit, limit and 64 bounds: 3 times as long.)
 template <int V>
-__global__ __launch_bounds__(256) void pick_limits_kernel(const uint32_t* __restrict__ bounds, int S, int nq, int per, int j, int near_rank, float flat,
+__global__ __launch_bounds__(256) void pick_limits_kernel(const uint32_t* __restrict__ bounds, int S, int nq, int per, int j, int near_rank, int tight_rank, float flat,
                                                           uint32_t* __restrict__ limits, uint32_t* __restrict__ last_round, uint32_t* __restrict__ blind) {
     constexpr int kBins = 1024, kMine = kBins / 64;
     __shared__ uint32_t s_hist[4][kBins];
@@ -532,10 +532,10 @@ __global__ __launch_bounds__(256) void pick_limits_kernel(const uint32_t* __rest
 #pragma unroll
         for (int i = 0; i < kMine; i++) { mine[i] = hist[lane * kMine + i]; sum += mine[i]; }
         const uint32_t upto = wave_scan_u32(sum);
-        uint32_t limit[kLimits];
+        uint32_t limit[kLimits + 1];          // (the last one: of confirm.hip's first round)
 #pragma unroll
-        for (int w = 0; w < kLimits; w++) {
-            const uint32_t rank = (uint32_t)(w == kMostRounds - 1 ? near_rank : j << w);
+        for (int w = 0; w < kLimits + 1; w++) {
+            const uint32_t rank = (uint32_t)(w == kLimits ? tight_rank : (w == kLimits - 1 ? near_rank : j << w));
             uint32_t run = upto - sum;
             int at = kBins - 1;
 #pragma unroll
@@ -550,11 +550,11 @@ __global__ __launch_bounds__(256) void pick_limits_kernel(const uint32_t* __rest
         // Bounds that say nothing of the nearest: candidates of any distance are wanted, or round 2 would take them all again.  (1000 queries, 100
         // partitions of 10000 rows of 128 in clusters a thousand times further apart than they are wide: 32 ms whole, 67 with whole rows read twice,
         // 33 once and, from the second call on, by the rows' codes, which near rows do without otherwise.)
-        if (limit[0] == 0) limit[kMostRounds - 1] = kInf; else all_blind = false;
+        if (limit[0] == 0) limit[kLimits - 1] = limit[kLimits] = kInf; else all_blind = false;
         // Bounds too close together for what a short traversal finds: the first round would find no distance that rules a partition out.
         if (f_lo + range < flat * __builtin_bit_cast(float, limit[0])) limit[0] = limit[1] = limit[2] = kInf;
         if (q0 + q < nq) {
-            if (lane < kLimits) limits[(int64_t)lane * nq + q0 + q] = lane == 0 ? limit[0] : (lane == 1 ? limit[1] : (lane == 2 ? limit[2] : limit[3]));
+            if (lane <= kLimits) limits[(int64_t)lane * nq + q0 + q] = lane == 0 ? limit[0] : (lane == 1 ? limit[1] : (lane == 2 ? limit[2] : (lane == 3 ? limit[3] : limit[4])));
             if (lane == 0) last_round[q0 + q] = 0;
         }
         __builtin_amdgcn_wave_barrier();
@@ -571,6 +571,8 @@ struct ListArgs {
     const float* worst; int64_t worst_stride;      // the k-th distance each query has so far
     uint32_t* last_round;                          // the round that last took a partition of the query
     int B, parts, nq, groups, round, rounds, near;
+    uint32_t* rests; uint32_t* confirm_word; int confirm_dies;      // (0: confirm.hip has no part in the call)
+    const float* near_then; float* near_now;       // how far rows counted in the round before, and in this one
     int32_t* items; uint32_t* count; uint32_t* part_counts; uint32_t* ticket;
 };
 __device__ inline bool takes_item(const ListArgs& a, int b, int q) {
@@ -584,8 +586,11 @@ __device__ inline bool takes_item(const ListArgs& a, int b, int q) {
     const float worst = a.worst[(int64_t)q * a.worst_stride];
     if (__builtin_bit_cast(float, v) > worst) return false;
     if (v > a.limits[(int64_t)(a.round - 1) * a.nq + q]) return true;
-    // round 1 took no candidates further away than its limit: where its k-th is, its partitions are taken again
-    return a.near && a.round == 1 && !(worst <= __builtin_bit_cast(float, a.limits[(int64_t)(kLimits - 1) * a.nq + q]));
+    // the round before took no candidates further away than its limit: where the k-th so far is, its partitions and those before are taken again
+    // (by the traversals alone only round 1's limit can be that)
+    const float wide = __builtin_bit_cast(float, a.limits[(int64_t)(kLimits - 1) * a.nq + q]);
+    if (a.confirm_dies == 0) return a.near && a.round == 1 && !(worst <= wide);
+    return !(worst <= (a.round == 1 && a.rests[1] ? wide : a.near_then[q]));
 }
 template <bool COUNT>
 __global__ __launch_bounds__(256) void list_items_kernel(ListArgs a) {
@@ -612,7 +617,31 @@ __global__ __launch_bounds__(256) void list_items_kernel(ListArgs a) {
         return;
     }
     uint32_t at = s_before[0] + s_before[1] + s_before[2] + s_before[3];
-    if (blockIdx.x == 0 && tid < kMostDies) a.ticket[tid * kTicketStride] = 0;
+    // What confirm.hip has made of the items it counts, in earlier rounds: for it, and for later calls.
+    if (a.confirm_dies > 0 && blockIdx.x == 0 && wave == 3) {
+        const uint32_t* left = a.ticket + (kLeftWord - kTicketWord) + (lane & (kMostDies - 1)) * kTicketStride;
+        const uint32_t had = wave_sum_u32(a.round > 0 && lane < a.confirm_dies ? left[1] + left[kConfirmPass + 1] : 0u);
+        const uint32_t lost = wave_sum_u32(a.round > 0 && lane < a.confirm_dies ? left[2] : 0u);
+        if (lane == 0) {
+            a.rests[0] = lost > 16 + had ? 1u : 0u;
+            if (a.round == 0) a.rests[1] = 0;
+            if (a.confirm_word && a.round > 0) {
+                reinterpret_cast<volatile uint32_t*>(a.confirm_word)[0] = had;
+                reinterpret_cast<volatile uint32_t*>(a.confirm_word)[1] = lost;
+            }
+        }
+    }
+    if (blockIdx.x == 0 && tid < kMostDies) {
+        uint32_t* left = a.ticket + (kLeftWord - kTicketWord) + tid * kTicketStride;
+        a.ticket[tid * kTicketStride] = left[0] = left[kConfirmPass] = 0;
+        if (a.round == 0) left[1] = left[2] = left[kConfirmPass + 1] = left[kConfirmPass + 2] = left[kConfirmPilot + 1] = left[kConfirmPilot + 2] = 0;
+    }
+    // (of queries that have no k results yet, rows as near as round 1's partitions may hold: all rows come in the last round)
+    if (a.confirm_dies > 0 && a.round > 0 && b == 0)
+        for (int q = q0 + tid; q < q1; q += 256) {
+            const float worst = a.worst[(int64_t)q * a.worst_stride], wide = __builtin_bit_cast(float, a.limits[(int64_t)(kLimits - 1) * a.nq + q]);
+            a.near_now[q] = a.round + 1 < a.rounds && !(worst < __builtin_inff()) ? wide : worst;
+        }
     if (blockIdx.x + 1 == gridDim.x && tid == 0) *a.count = at + s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
     for (int w = 0; w < wave; w++) at += s_wave[w];
 #pragma unroll
@@ -684,7 +713,7 @@ __global__ __launch_bounds__(256) void sample_decide_kernel(const uint32_t* __re
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
-struct Room { size_t header, counts, qinfo, frags, bounds, limits, last, items, part_counts, near, sample, sample_rows, total; int steps, tiles, parts; };
+struct Room { size_t header, counts, qinfo, frags, bounds, limits, last, items, part_counts, near, left, sample, sample_rows, total; int steps, tiles, parts; };
 // The sample as a call of its own, over every (B / kSampleParts)-th partition.
 constexpr int kSampleParts = 12;
 int sample_stride(const QueryArgs& a) { return a.B / min(a.B, kSampleParts); }
@@ -696,9 +725,11 @@ QueryArgs sample_call(const QueryArgs& a, const float* rows) {
     c.k = 1;
     c.kcap = 0;                           // (nothing of it is kept, so nothing to clear)
     c.part = nullptr;
-    c.pick_sample = c.pick_near = 0;
+    c.pick_sample = c.pick_near = c.pick_confirm = 0;
     return c;
 }
+// Items a die's run of a round's list holds at most.
+int64_t left_cap(const QueryArgs& a) { return ((int64_t)a.nq * a.B + a.xcds - 1) / a.xcds; }
 Room room_of(const QueryArgs& a) {
     Room r;
     r.steps = (a.dim + 2 * kStep - 1) / (2 * kStep) * 2;       // an even number of them
@@ -715,11 +746,12 @@ Room room_of(const QueryArgs& a) {
     r.qinfo = o;  o += align256((size_t)r.tiles * kTile * sizeof(float2));
     r.frags = o;  o += align256((size_t)r.tiles * r.steps * 64 * 16);
     r.bounds = o; o += align256((size_t)a.B * r.parts * a.nq * 4);
-    r.limits = o; o += align256((size_t)kLimits * a.nq * 4);
+    r.limits = o; o += align256((size_t)(kLimits + 3) * a.nq * 4);
     r.last = o;   o += align256((size_t)a.nq * 4);
     r.items = o;  o += align256((size_t)a.nq * a.B * 4);
     r.part_counts = o; o += align256((size_t)a.B * ((a.nq + kListQueries - 1) / kListQueries) * 4);
-    r.near = o;   o += a.pick_near ? align256(near_bytes(a)) : 0;
+    r.near = o;   o += a.pick_near || a.pick_confirm ? align256(near_bytes(a)) : 0;
+    r.left = o;   o += a.pick_confirm ? align256((size_t)2 * left_cap(a) * a.xcds * 4) : 0;
     r.sample = r.sample_rows = o;
     if (a.pick_sample) {
         o += room_of(sample_call(a, nullptr)).total;
@@ -766,7 +798,7 @@ double bounds_cost(const QueryArgs& a) {
 static int pack(const QueryArgs& a, const Room& r, char* ws, hipStream_t s) {
     PackArgs p{a.query, a.data, a.N, a.nq, a.dim, r.steps, r.tiles, (Header*)(ws + r.header),
                (float2*)(ws + r.qinfo), (_Float16*)(ws + r.frags), (uint32_t*)(ws + r.bounds), (int64_t)a.B * r.parts * a.nq, (uint32_t*)(ws + r.near),
-               a.pick_near && shape_of(a).rt * kTile < near_rows(shape_of(a).rt) ? (int64_t)near_bytes(a) / 4 : 0,
+               (a.pick_near || a.pick_confirm) && shape_of(a).rt * kTile < near_rows(shape_of(a).rt) ? (int64_t)near_bytes(a) / 4 : 0,
                a.part, (int64_t)a.nq * a.B * a.kcap};
     const int64_t clear = (p.num_part + p.num_bounds + p.num_near + kPackThreads * 16 - 1) / (kPackThreads * 16);
     const unsigned blocks = (unsigned)max((int64_t)r.tiles, min((int64_t)2048, clear));
@@ -807,7 +839,7 @@ static int launch_stream(const BoundArgs& p, int xcds, hipStream_t s) {
 static int products(const QueryArgs& a, const Room& r, char* ws, int64_t step, const uint32_t* skip, hipStream_t s) {
     BoundArgs p{a.data, a.N, a.ppb, step, a.dim, r.steps, a.nq, r.tiles, 0, 0, 0, a.B, 0, r.parts,
                 (const Header*)(ws + r.header), (const float2*)(ws + r.qinfo), (const _Float16*)(ws + r.frags),
-                (uint32_t*)(ws + r.bounds), a.pick_near ? (uint32_t*)(ws + r.near) : nullptr, skip};
+                (uint32_t*)(ws + r.bounds), a.pick_near || a.pick_confirm ? (uint32_t*)(ws + r.near) : nullptr, skip};
     const Shape y = shape_of(a);
     if (!y.stream) {
         constexpr int R = 128;
@@ -856,7 +888,7 @@ int sample_items(const QueryArgs& a, void* ws_, Picked& p, hipStream_t s) {
     hipLaunchKernelGGL(sample_items_kernel, dim3(32), dim3(256), 0, s, a.query, a.nq, a.dim, a.B, a.pick_sample, (float*)(ws + r.sample_rows),
                        (int32_t*)(ws + r.items), count, (uint32_t*)(ws + r.counts) + kTicketWord, (uint32_t*)(ws + r.last));
     DCIH_HIP(hipGetLastError());
-    p = Picked{(const int32_t*)(ws + r.items), count, (const uint32_t*)(ws + r.last), (uint32_t*)(ws + r.counts) + kTicketWord, nullptr, nullptr, 0, 0, 0};
+    p = Picked{(const int32_t*)(ws + r.items), count, (const uint32_t*)(ws + r.last), (uint32_t*)(ws + r.counts) + kTicketWord, nullptr, nullptr, nullptr, 0, 0, 0};
     return 0;
 }
 
@@ -875,6 +907,10 @@ int sample_decide(const QueryArgs& a, void* ws_, hipStream_t s) {
     return 0;
 }
 
+// How far rows count in a round of confirm.hip's: in round 1 as picked, later one of two rows in turn.
+static float* near_limits(char* ws, const Room& r, int nq, int round) {
+    return (float*)(ws + r.limits) + (int64_t)(round <= 0 ? kLimits : kLimits + 1 + (round & 1)) * nq;
+}
 int pick_items(const QueryArgs& a, void* ws_, int round, int rounds, hipStream_t s) {
     char* ws = (char*)ws_;
     const Room r = room_of(a);
@@ -884,9 +920,11 @@ int pick_items(const QueryArgs& a, void* ws_, int round, int rounds, hipStream_t
     if (round == 0) {
         const int S = a.B * r.parts, per = a.nq >= 8192 && S <= 512 ? 16 : 4;
         const dim3 grid((unsigned)((a.nq + per - 1) / per));
+        const int near_rank = min(32 * a.pick_rank, max(4 * a.pick_rank, S / 2));
+        const int tight_rank = 4 * a.pick_rank;
 #define DCIH_LIMITS(V)                                                                                              \
     hipLaunchKernelGGL(pick_limits_kernel<V>, grid, dim3(256), (size_t)S * (per + 1) * 4, s, bounds, S, a.nq, per, \
-                       a.pick_rank, min(32 * a.pick_rank, max(4 * a.pick_rank, S / 2)), a.pick_flat, limits, last, \
+                       a.pick_rank, near_rank, a.pick_confirm ? tight_rank : near_rank, a.pick_flat, limits, last, \
                        a.blind_word)
         if (S <= 64) DCIH_LIMITS(1); else if (S <= 128) DCIH_LIMITS(2); else if (S <= 256) DCIH_LIMITS(4);
         else if (S <= 512) DCIH_LIMITS(8); else if (S <= 1024) DCIH_LIMITS(16); else DCIH_LIMITS(32);
@@ -895,6 +933,7 @@ int pick_items(const QueryArgs& a, void* ws_, int round, int rounds, hipStream_t
     }
     const int groups = (a.nq + kListQueries - 1) / kListQueries;
     ListArgs p{bounds, limits, a.pick_sample ? (const uint32_t*)(ws + r.counts) + kSkipWord : nullptr, a.out_dists + (a.k - 1), a.k, last, a.B, r.parts, a.nq, groups, round, rounds, a.pick_near,
+                 (uint32_t*)(ws + r.counts) + kRestsWord, a.pick_confirm ? a.confirm_word : nullptr, a.pick_confirm ? a.xcds : 0, near_limits(ws, r, a.nq, round - 1), near_limits(ws, r, a.nq, round),
                (int32_t*)(ws + r.items), (uint32_t*)(ws + r.counts) + round, (uint32_t*)(ws + r.part_counts),
                (uint32_t*)(ws + r.counts) + kTicketWord};
     const dim3 grid((unsigned)((int64_t)a.B * groups));
@@ -904,16 +943,29 @@ int pick_items(const QueryArgs& a, void* ws_, int round, int rounds, hipStream_t
     return 0;
 }
 
+int confirm_round(QueryArgs& a, void* ws_, hipStream_t s) {
+    char* ws = (char*)ws_;
+    const Room r = room_of(a);
+    uint32_t* counts = (uint32_t*)(ws + r.counts);
+    a.left = nullptr;
+    const int rc = confirm_items(a, a.pick_sample ? counts + kSkipWord : nullptr, counts + kRestsWord, (int32_t*)(ws + r.left), counts + kLeftWord, left_cap(a), s);
+    a.left = (const int32_t*)(ws + r.left);
+    a.left_count = counts + kLeftWord;
+    a.left_cap = left_cap(a);
+    return rc;
+}
+
 Picked picked_items(const QueryArgs& a, void* ws_, int round) {
     char* ws = (char*)ws_;
     const Room r = room_of(a);
     Picked p{(const int32_t*)(ws + r.items), (const uint32_t*)(ws + r.counts) + round, (const uint32_t*)(ws + r.last),
-             (uint32_t*)(ws + r.counts) + kTicketWord, nullptr, nullptr, 0, 0, 0};
-    if (a.pick_near) {
+             (uint32_t*)(ws + r.counts) + kTicketWord, nullptr, nullptr, nullptr, 0, 0, 0};
+    if (a.pick_near || a.pick_confirm) {
         p.near_bounds = (const uint32_t*)(ws + r.near);
-        // (later rounds: the k-th distance found so far)
-        p.near_limit = round ? a.out_dists + (a.k - 1) : (const float*)(ws + r.limits) + (int64_t)(kLimits - 1) * a.nq;
-        p.near_stride = round ? a.k : 1;
+        // (later rounds': the k-th distance found so far, as list_items_kernel has noted it for confirm.hip)
+        p.confirm_limit = near_limits(ws, r, a.nq, round);
+        p.near_limit = round == 0 ? (const float*)(ws + r.limits) + (int64_t)(kLimits - 1) * a.nq : (a.pick_confirm ? p.confirm_limit : a.out_dists + (a.k - 1));
+        p.near_stride = round && !a.pick_confirm ? a.k : 1;
         p.near_shift = near_rows(shape_of(a).rt) == 64 ? 6 : 7;
         p.near_tiles = (int)near_tiles_of(a);
     }

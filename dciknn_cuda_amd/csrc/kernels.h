@@ -119,8 +119,12 @@ struct QueryArgs {
     // a call in rounds (bounds.hip)
     const int32_t* picked;   // null = all nq * B items, else the round's, of which every die takes one run
     const uint32_t* picked_count;
+    const int32_t* left;     // null, or per die of these those that confirm.hip has left, and how many (kAllLeft: all of them, not listed)
+    const uint32_t* left_count;
+    int64_t left_cap;
     uint32_t* round_items;   // null, or device words for the number of items of every round, then the sample's decision
     uint32_t* blind_word;    // null, or (the host's memory) set where bounds say nothing of queries' nearest rows
+    uint32_t* confirm_word;  // null, or (the host's memory) two words: items that confirm.hip answered and left, of those it counts
     int64_t* selected;       // (host) counts the queries that nearest.hip answers
     uint32_t* picked_ticket; // a zeroed word per die: the dense kernel's workgroups take their items by it
     int64_t picked_exact;    // their number, where it is known: 0 otherwise
@@ -135,10 +139,14 @@ struct QueryArgs {
     int64_t near_stride;
     int near_shift, near_tiles;
     int pick_near;           // 1: a call in rounds goes to the dense kernel and keeps those bounds
+    int pick_confirm;        // 1: rounds' items go through confirm.hip first, which needs those bounds too
     int pick_sample;         // 0, or: so many queries are traversed whole first, and decide
     float pick_most;         // share of pairs that rounds may have to take: where the sample's bounds leave more, everything is taken at once
     int pick_rounds;         // 0: everything is traversed at once
     int pick_rank;           // the first round takes the partitions of so many nearest rows
+    uint32_t confirm_had, confirm_lost;   // of the items that confirm.hip counted in the last call that it was part of, those that it answered and left
+    int confirm_again;       // 1: whatever they say, it is tried
+    int index_calls;         // queries of this index before
     int pick_rule;           // DCIH_OPT_ROUNDS value
     double pick_first;       // partitions per query the first round is expected to take
     double share;            // share of all items that are expected to be traversed (1 but for such calls)
@@ -256,20 +264,36 @@ int code_rows(const float* d_data, int64_t n, int dim, int64_t ppb, int B, unsig
 int code_queries(const float* d_query, int nq, int dim, unsigned char* d_recs, hipStream_t s);
 
 // The run of a list of `count` items that die x of X takes: its first item and their number.
-__device__ inline int64_t picked_run(const uint32_t* d_count, int x, int X, int64_t& first) {
-    const int64_t count = *d_count, each = (count + X - 1) / X;
+__device__ inline int64_t run_of_die(int64_t count, int x, int X, int64_t& first) {
+    const int64_t each = (count + X - 1) / X;
     first = each * x;
     return min(each, max((int64_t)0, count - first));
 }
 // Calls in rounds (bounds.hip): lower bounds of every (query, partition)'s nearest distance, and the items each
 // round takes.  Scratch of bounds_bytes(); bounds_cost: about how long the bounds take, us.  pack_bounds
 // comes first and also clears a.part.
-constexpr int kPickCountWords = 64 + 32 * 32, kMostRounds = 4;
-constexpr int kSampleWord = 8, kSkipWord = 9, kTicketWord = 64, kTicketStride = 32;      // of the count words: the sample's items, whether rounds are skipped, the pairs that says so by, a ticket per die
+constexpr int kPickCountWords = 64 + 2 * 32 * 32, kMostRounds = 4;
+// of the count words: the sample's items, whether rounds are skipped, the pairs that says so by, whether confirm.hip rests, and did so in round 1; per die a ticket, and the items that confirm.hip left, then of some those that it answered and left
+constexpr int kSampleWord = 8, kSkipWord = 9, kRestsWord = 12, kRestedWord = 13, kTicketWord = 64, kTicketStride = 32, kLeftWord = kTicketWord + 32 * 32, kConfirmPass = 8, kConfirmPilot = 16;      // (where the counts of confirm.hip's first pass, and of its pilot, lie in a die's words)
+constexpr int kPilotItems = 64;      // tried ahead, per die, where nothing is known yet
+// A round's items of die x: its run of the round's list, or what confirm.hip has left of that.
+constexpr uint32_t kAllLeft = 0xffffffffu;
+template <class A>
+__device__ inline int64_t picked_run(const A& a, int x, const int32_t*& items) {
+    const uint32_t left = a.left ? a.left_count[x * kTicketStride] : kAllLeft;
+    if (left != kAllLeft) {
+        items = a.left + x * a.left_cap;
+        return (int64_t)left;
+    }
+    int64_t first;
+    const int64_t count = run_of_die(*a.picked_count, x, a.xcds, first);
+    items = a.picked + first;
+    return count;
+}
 constexpr uint32_t kSampleRound = 0x10000;         // of the sample's queries while their results are merged
 struct Picked {
     const int32_t* items; const uint32_t* count; const uint32_t* last_round; uint32_t* ticket;
-    const uint32_t* near_bounds; const float* near_limit; int64_t near_stride; int near_shift, near_tiles;
+    const uint32_t* near_bounds; const float* near_limit; const float* confirm_limit; int64_t near_stride; int near_shift, near_tiles;
 };
 bool bounds_supported(const QueryArgs& a);
 size_t bounds_bytes(const QueryArgs& a);
@@ -282,6 +306,11 @@ int partition_bounds(const QueryArgs& a, void* ws, hipStream_t s);
 int sample_items(const QueryArgs& a, void* ws, Picked& p, hipStream_t s);
 int sample_decide(const QueryArgs& a, void* ws, hipStream_t s);
 int pick_items(const QueryArgs& a, void* ws, int round, int rounds, hipStream_t s);
+// Answers those of a round's items that need no traversal (confirm.hip); a.left.. become the others.
+bool confirm_supported(const QueryArgs& a);
+bool confirm_scans(const QueryArgs& a);      // whether that needs rpos
+int confirm_items(const QueryArgs& a, const uint32_t* skip, uint32_t* rests, int32_t* left, uint32_t* left_count, int64_t left_cap, hipStream_t s);
+int confirm_round(QueryArgs& a, void* ws, hipStream_t s);
 Picked picked_items(const QueryArgs& a, void* ws, int round);
 // Whether a call is worth its rounds; sets a.pick_rounds, a.pick_first and a.share.
 bool plan_rounds(QueryArgs& a);

@@ -457,8 +457,22 @@ bool takes_dense_kernel(const QueryArgs& a) {
     return c.dense < c.batch;
 }
 
+// Whether a round's items go through confirm.hip first.  That takes about 0.02 us of an item where items fill the device, a traversal 0.03 to 0.25; it loses where
+// partitions are short (137 rows of 41, windows of 10: 427 us without, 466 with; 127 of 675: 1.50 ms, 2.48; 947 of 168: 4.99, 1.07) and where it has to leave
+// too many (331 rows, a sixth of the items left: 2.64, 3.15; 2818 rows, a twelfth: 9.19, 5.86).  Calls that are over soon have to be answered as a whole, or
+// they wait for a traversal as well (455 items, 25 left: 278 us, 444; 5800, a fifth left: 1.44, 1.55 ms), and the positions by the first simple index, which
+// it reads, are not formed for the first small call of an index (one that is formed anew for a few lookups).
+static bool confirm_pays(const QueryArgs& a, double items, bool by_dense) {
+    if (a.pick_rule == 2) return true;
+    const double item = by_dense ? traversal_costs(a, 0.0).dense_item : 1.0;
+    if (item < 0.024) return false;
+    if (items <= 4096.0 && confirm_scans(a) && !*a.rpos_ready && a.index_calls == 0) return false;
+    const double may = items <= 16384.0 ? 1.0 / 256.0 : fmin(1.0, (item - 0.022) / 0.02);
+    return a.confirm_again || (double)a.confirm_lost <= (items <= 16384.0 ? 0.0 : 16.0) + may * (double)a.confirm_had;
+}
+
 bool plan_rounds(QueryArgs& a) {
-    a.pick_rounds = a.pick_near = a.pick_sample = 0;
+    a.pick_rounds = a.pick_near = a.pick_confirm = a.pick_sample = 0;
     a.share = 1.0;
     if (a.mode != 0 || a.pick_rule == 1 || !bounds_supported(a)) return false;
     // The r nearest rows of a query lie in about B (1 - e^(-r/B)) partitions (rows in no particular order).  Round 1
@@ -505,6 +519,7 @@ bool plan_rounds(QueryArgs& a) {
     a.pick_first = first;
     a.share = share;
     a.pick_near = !sampled && near_bytes(a) <= ((size_t)1 << 30) ? 1 : 0;
+    a.pick_confirm = confirm_supported(a) && near_bytes(a) <= ((size_t)1 << 30) && confirm_pays(a, (double)a.nq * first, can_dense && takes_dense_kernel(a)) ? 1 : 0;
     a.pick_sample = sampled ? std::min(a.nq, std::max(2, std::min(16, 1024 / a.B))) : 0;
     // Up to which share of the sample's pairs rounds pay: the fewer results, the further away the k-th of the first rounds lies than
     // that of all.  (Five kinds of rows, 16 to 300 elements, 30000 to a million: shares from which rounds begin to take longer are 0.31 to
@@ -666,8 +681,21 @@ int query(const QueryArgs& a_in, void* bounds_ws, hipStream_t s, hipEvent_t* ev,
             // every partition: strides over the rest take up to twice as long, a workgroup without an item 0.2 ns.  (4000 queries, 58 partitions
             // of 17242 normal rows of 128: 15.2 ms whole, 18.9 in rounds that covered 131072 items.)
             a.picked_cover = round ? std::max((int64_t)(0.3 * (double)a.nq * (double)a.B), (int64_t)65536) : (int64_t)a.nq * a.B;
+            if (a.pick_confirm && round) a.picked_cover = std::min(a.picked_cover, (int64_t)16384);
             a.picked_expect = round ? 0 : (int64_t)((double)a.nq * a.pick_first);
+            if (a.pick_confirm && !rc) {
+                if (confirm_scans(a) && a.rpos_ready && !*a.rpos_ready) {
+                    rc = fill_positions_by_first(a.sids, a.inv, const_cast<uint16_t*>(a.rpos), a.N, a.M, a.L, a.ppb, a.B, s);
+                    if (!rc && !a.recorded) *a.rpos_ready = 1;
+                }
+                a.near_limit = p.confirm_limit;
+                if (!rc) rc = confirm_round(a, bounds_ws, s);
+                a.near_limit = p.near_limit;
+                a.picked_expect = 0;
+                if (!a.pick_near) a.near_bounds = nullptr;
+            }
             if (!rc) rc = traverse(a);
+            a.left = nullptr;
             a.only = round > 0 ? p.last_round : nullptr;
             a.only_round = (uint32_t)round;
         }

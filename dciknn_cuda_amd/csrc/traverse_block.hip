@@ -1148,14 +1148,15 @@ __global__ __launch_bounds__(NT, MINW) void traverse_block_kernel(QueryArgs a, B
 template <int NT, int MINW, bool COMPACT>
 __global__ __launch_bounds__(NT, MINW) void traverse_block_picked_kernel(QueryArgs a, BlockLayout y) {
     const uint32_t X = (uint32_t)a.xcds, die = blockIdx.x % X, w = blockIdx.x / X;
-    const uint32_t count = *a.picked_count, each = (count + X - 1) / X, at = die * each + w;
+    const uint32_t count = *a.picked_count;
     int b, qi;
     // all of them: as whole calls take them (8250 and 7650 us where a die has a run of the list)
-    if (count == (uint32_t)a.nq * (uint32_t)a.B && count <= gridDim.x) {
+    if (count == (uint32_t)a.nq * (uint32_t)a.B && count <= gridDim.x && !(a.left && a.left_count[0] != kAllLeft)) {
         if (!block_item((int64_t)blockIdx.x, a.xcds, a.B, a.nq, b, qi)) return;
     } else {
-        if (w >= each || at >= count) return;
-        const int32_t item = a.picked[at];
+        const int32_t* items;
+        if ((int64_t)w >= picked_run(a, (int)die, items)) return;
+        const int32_t item = items[w];
         b = item % a.B; qi = item / a.B;
     }
     b = __builtin_amdgcn_readfirstlane(b); qi = __builtin_amdgcn_readfirstlane(qi);
@@ -1167,10 +1168,10 @@ __global__ __launch_bounds__(NT, MINW) void traverse_block_picked_kernel(QueryAr
 // What more than the launch above covers (more partitions of a query at the same bound than one expects): strides over the rest.
 template <int NT, int MINW, bool COMPACT>
 __global__ __launch_bounds__(NT, MINW) void traverse_block_rest_kernel(QueryArgs a, BlockLayout y, int64_t covered) {
-    int64_t first;
-    const int64_t count = picked_run(a.picked_count, (int)(blockIdx.x % (unsigned)a.xcds), a.xcds, first);
+    const int32_t* items;
+    const int64_t count = picked_run(a, (int)(blockIdx.x % (unsigned)a.xcds), items);
     for (int64_t w = covered + blockIdx.x / (unsigned)a.xcds; w < count; w += gridDim.x / (unsigned)a.xcds) {
-        const int32_t item = __builtin_amdgcn_readfirstlane(a.picked[first + w]);
+        const int32_t item = __builtin_amdgcn_readfirstlane(items[w]);
         traverse_block_item<NT, MINW, COMPACT>(a, y, item % a.B, item / a.B);
         __syncthreads();          // the next item reuses the tables
     }

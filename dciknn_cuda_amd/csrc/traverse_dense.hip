@@ -301,9 +301,7 @@ __global__ __launch_bounds__(NT, WAVES) void traverse_dense_kernel(DenseArgs) {
     int64_t my_count;
     const int32_t* my_items = nullptr;
     if constexpr (PICKED) {
-        int64_t first;
-        my_count = picked_run(args->a.picked_count, xcd, X, first);
-        my_items = args->a.picked + first;
+        my_count = picked_run(args->a, xcd, my_items);
     } else if (args->a.dense_items != nullptr && args->a.mode != 3) {
         my_count = (int64_t)args->a.dense_count[xcd];
         my_items = args->a.dense_items + (int64_t)xcd * args->a.dense_cap;

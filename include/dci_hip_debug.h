@@ -64,6 +64,11 @@ int dcih_debug_route(const dcih_index* h, int64_t* route);
  * could not be ruled out.
  */
 int dcih_debug_round_items(dcih_index* h, uint32_t* d_items);
+/*
+ * counts receives, of the last finished query in rounds that looked at near rows alone before it traversed anything, how many of the (query,
+ * partition) pairs that it counts were answered so and how many were left to a traversal (zeros: no such query yet).
+ */
+int dcih_debug_confirmed(const dcih_index* h, uint32_t* counts);
 
 #ifdef __cplusplus
 }
