@@ -130,7 +130,11 @@ __host__ __device__ constexpr int near_rows(int rt) { return kTile * (rt < 2 ? 2
 // rows of a partition, each wavefront RT x CT accumulators of 32 x 32.  A row's squared length is where its
 // accumulators start (or is added at their end), so what is left to do with a sum is to keep the smallest, in the lane that holds the
 // query's column.
-template <int RT, int CT, int WR, int WC, int COLUMNS, bool OCTETS>
+// QD: steps of the queries that are under way.  A step is multiplied in 256 cycles, less than a read from the L2 takes, and where rows are streamed one
+// wavefront of a SIMD multiplies: with two steps ahead 512 queries on 10M rows of 96 take 1956 us, with six 1872; 500 on 1M rows of 960, two and four,
+// 1483, 1430.  (Two stretches of rows under way instead of one change nothing: the multiplying side is the slower one.  Without the
+// multiplications 1169 and 807 us, with every tile reading the same rows 1814 and 1255.)
+template <int RT, int CT, int WR, int WC, int COLUMNS, bool OCTETS, int QD = 2>
 struct BoundTile {
     static constexpr int kWaves = WR * WC, R = kTile * RT * WR, kGroups = R / 8 / kWaves, kOctets = COLUMNS / 64;
     static_assert(kGroups >= 1 && kOctets >= 1, "eight rows per wavefront at least");
@@ -229,10 +233,10 @@ struct BoundTile {
         return v;
     }
     // The queries' steps in the order a wavefront multiplies them: all of tiles first .. first + CT - 1, then of those kPass
-    // further on, and from the beginning again.  q8 holds the next two; a step's registers take the step after the next one once it has
+    // further on, and from the beginning again.  q8 holds the next QD; a step's registers take the step QD further on once it has
     // been multiplied, no sooner, or the compiler copies them, which waits for what is under way.
     struct Queries {
-        v8h q8[2][CT];
+        v8h q8[QD][CT];
         uint32_t at, group, left;         // bytes from a.frags on: the step read next and its tiles' first one; steps left of those
         uint32_t first, end, stride;      // the first tiles; past the last; from tiles to the next tiles
         uint32_t mine[CT];                // the lane's place in a step
@@ -259,12 +263,13 @@ struct BoundTile {
         y.left = (uint32_t)a.steps;
 #pragma unroll
         for (int c = 0; c < CT; c++) y.mine[c] = c * bytes + lane * 16;
-        read_queries(y, y.q8[0]);
-        next_step(y);
-        read_queries(y, y.q8[1]);
-        next_step(y);
+#pragma unroll
+        for (int u = 0; u < QD; u++) {
+            read_queries(y, y.q8[u]);
+            next_step(y);
+        }
     }
-    // The next ns (an even number of) steps.
+    // The next ns (a multiple of QD) steps.
     __device__ __forceinline__ void multiply_steps(v16f (&acc)[RT][CT], const v8h* rows_at, int pitch, Queries& y, int ns) const {
         v8h x8[2][RT];
 #pragma unroll
@@ -283,9 +288,10 @@ struct BoundTile {
             __builtin_amdgcn_sched_barrier(0);
             y.at = then.at; y.group = then.group; y.left = then.left;
         };
-        for (int s = 0; s < ns; s += 2) {
-            one(rows_at + (s + 1) * 64, x8[0], x8[1], y.q8[0]);
-            one(rows_at + min(s + 2, ns - 1) * 64, x8[1], x8[0], y.q8[1]);
+        static_assert(QD % 2 == 0, "the rows' steps take two turns");
+        for (int s = 0; s < ns; s += QD) {
+#pragma unroll
+            for (int u = 0; u < QD; u++) one(rows_at + min(s + u + 1, ns - 1) * 64, x8[u & 1], x8[(u + 1) & 1], y.q8[u]);
         }
     }
     // The smallest sum of each of 32 CT queries over the wavefront's rows -> their bounds; q: the lane's query of the first 64.
@@ -385,9 +391,9 @@ __global__ __launch_bounds__(64 * WC, WAVES) void bounds_resident_kernel(BoundAr
 // (One set of wavefronts for both cannot: their reads of the queries would wait for the reads of rows issued before them,
 // 592 us for 512 queries on 2M rows of 96.)  ONE: a row is no longer than COLUMNS, and all queries are taken past it while it lies there;
 // else its columns come once for every pass over 32 CT WC queries.
-template <int RT, int CT, int WR, int WC, int COLUMNS, int WAVES, bool ONE, bool OCTETS>
+template <int RT, int CT, int WR, int WC, int COLUMNS, int WAVES, bool ONE, bool OCTETS, int QD>
 __global__ __launch_bounds__(128 * WR * WC, WAVES) void bounds_stream_kernel(BoundArgs a) {
-    typedef BoundTile<RT, CT, WR, WC, COLUMNS, OCTETS> Tile;
+    typedef BoundTile<RT, CT, WR, WC, COLUMNS, OCTETS, QD> Tile;
     constexpr int kPass = CT * WC;
     extern __shared__ __align__(16) unsigned char smem[];
     const int pitch = a.column_steps, half = Tile::R * pitch * 2;      // 16-byte words
@@ -809,13 +815,13 @@ static int pack(const QueryArgs& a, const Room& r, char* ws, hipStream_t s) {
     return 0;
 }
 
-template <int RT, int CT, int WR, int WC, int COLUMNS, int WAVES, bool ONE>
+template <int RT, int CT, int WR, int WC, int COLUMNS, int WAVES, bool ONE, int QD = 2>
 static int launch_stream(const BoundArgs& p, int xcds, hipStream_t s) {
     constexpr int R = kTile * RT * WR, NT = 128 * WR * WC, kColumnSteps = COLUMNS / kStep;
     BoundArgs a = p;
     // stretches of columns of about the same length
     const int stretches = ONE ? 1 : (p.steps + kColumnSteps - 1) / kColumnSteps;
-    a.column_steps = (p.steps + 2 * stretches - 1) / (2 * stretches) * 2;
+    a.column_steps = (p.steps + QD * stretches - 1) / (QD * stretches) * QD;
     const size_t lds = (size_t)2 * R * 4 + 4 * WR * WC * 4 + (size_t)p.steps * kStep * 4 + (size_t)2 * R * a.column_steps * kStep * 2;
     a.row_tiles = (int)((p.ppb + R - 1) / R);
     // as many workgroups as the device holds at a time
@@ -825,13 +831,13 @@ static int launch_stream(const BoundArgs& p, int xcds, hipStream_t s) {
     a.next_tile = (int)(grid % a.row_tiles);
     static DeviceOnce once;
     const int rc = once.run([]() -> int {
-        DCIH_HIP(hipFuncSetAttribute((const void*)bounds_stream_kernel<RT, CT, WR, WC, COLUMNS, WAVES, ONE, true>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-        DCIH_HIP(hipFuncSetAttribute((const void*)bounds_stream_kernel<RT, CT, WR, WC, COLUMNS, WAVES, ONE, false>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        DCIH_HIP(hipFuncSetAttribute((const void*)bounds_stream_kernel<RT, CT, WR, WC, COLUMNS, WAVES, ONE, true, QD>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        DCIH_HIP(hipFuncSetAttribute((const void*)bounds_stream_kernel<RT, CT, WR, WC, COLUMNS, WAVES, ONE, false, QD>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         return 0;
     });
     if (rc) return rc;
-    if (p.dim % 8 == 0) hipLaunchKernelGGL((bounds_stream_kernel<RT, CT, WR, WC, COLUMNS, WAVES, ONE, true>), dim3((unsigned)grid), dim3(NT), lds, s, a);
-    else hipLaunchKernelGGL((bounds_stream_kernel<RT, CT, WR, WC, COLUMNS, WAVES, ONE, false>), dim3((unsigned)grid), dim3(NT), lds, s, a);
+    if (p.dim % 8 == 0) hipLaunchKernelGGL((bounds_stream_kernel<RT, CT, WR, WC, COLUMNS, WAVES, ONE, true, QD>), dim3((unsigned)grid), dim3(NT), lds, s, a);
+    else hipLaunchKernelGGL((bounds_stream_kernel<RT, CT, WR, WC, COLUMNS, WAVES, ONE, false, QD>), dim3((unsigned)grid), dim3(NT), lds, s, a);
     DCIH_HIP(hipGetLastError());
     return 0;
 }
@@ -869,8 +875,14 @@ static int products(const QueryArgs& a, const Room& r, char* ws, int64_t step, c
         return columns <= 128 ? launch_stream<1, 2, 4, 1, 128, 4, true>(p, a.xcds, s) : launch_stream<1, 2, 4, 1, 64, 4, false>(p, a.xcds, s);
     }
     if (y.wr == 2) return columns <= 128 ? launch_stream<2, 2, 2, 2, 128, 3, true>(p, a.xcds, s) : launch_stream<2, 2, 2, 2, 64, 4, false>(p, a.xcds, s);
-    if (y.ct == 4) return launch_stream<2, 4, 1, 4, 256, 2, false>(p, a.xcds, s);
-    return columns <= 128 ? launch_stream<4, 2, 1, 4, 128, 2, true>(p, a.xcds, s) : launch_stream<4, 2, 1, 4, 256, 2, true>(p, a.xcds, s);
+    // (these have one multiplying wavefront per SIMD: as many steps of the queries ahead as divide the rows' steps)
+    const bool fours = r.steps % 4 == 0;
+    if (y.ct == 4) return fours ? launch_stream<2, 4, 1, 4, 256, 2, false, 4>(p, a.xcds, s) : launch_stream<2, 4, 1, 4, 256, 2, false>(p, a.xcds, s);
+    if (columns <= 128) {
+        if (fours) return launch_stream<4, 2, 1, 4, 128, 2, true, 4>(p, a.xcds, s);
+        return r.steps % 6 == 0 ? launch_stream<4, 2, 1, 4, 128, 2, true, 6>(p, a.xcds, s) : launch_stream<4, 2, 1, 4, 128, 2, true>(p, a.xcds, s);
+    }
+    return fours ? launch_stream<4, 2, 1, 4, 256, 2, true, 4>(p, a.xcds, s) : launch_stream<4, 2, 1, 4, 256, 2, true>(p, a.xcds, s);
 }
 
 int pack_bounds(const QueryArgs& a, void* ws, hipStream_t s) { return pack(a, room_of(a), (char*)ws, s); }
