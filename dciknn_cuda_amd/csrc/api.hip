@@ -161,6 +161,7 @@ struct dcih_index {
     int64_t route[4] = {0, 0, 0, 0};    // dcih_debug_route
     int confirm_rests = 0;              // calls in rounds that went without confirm.hip, since the last one with it
     int index_calls = 0;                // queries since the index was formed
+    size_t near_room = (size_t)1 << 30; // what the bounds of a call's tiles may take
     volatile uint32_t* blind = nullptr; // (pinned: three words) set by queries in rounds whose bounds said nothing: the next ones use the rows' codes; then the items that confirm.hip answered and left, of those it counts
     uint32_t* d_round_items = nullptr;  // dcih_debug_round_items
     unsigned long long* d_phase_ticks = nullptr;   // optional profile of the batch kernel
@@ -642,7 +643,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
                       int num_neighbours, int blind, int num_outer_iterations,
                       int max_num_candidates, int block_size, int thread_size,
                       int32_t* d_nn, float* d_dists, uint64_t* d_counters, void* stream,
-                      bool fixed, bool float_ids, const char* who, bool whole = false) {
+                      bool fixed, bool float_ids, const char* who, bool whole = false, bool later_part = false) {
     const std::string me(who);
     if (!h) return fail(DCIH_EINVAL, me + ": null handle");
     if (dim != h->dim) return fail(DCIH_EINVAL, me + ": dim differs from the index's");
@@ -713,6 +714,8 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     a.share = 1.0; a.pick_first = 0.0; a.pick_rounds = a.pick_rank = a.pick_near = a.pick_confirm = a.pick_sample = 0; a.pick_most = 1.0f;
     a.near_bounds = nullptr; a.near_limit = nullptr; a.near_stride = 0; a.near_shift = a.near_tiles = 0; a.pick_rule = fixed || whole ? 1 : h->rounds;
     a.phase_ticks = h->d_phase_ticks;
+    a.near_room = h->near_room;
+    a.pick_parts = 1;
     a.round_items = h->d_round_items;
     a.blind_word = a.confirm_word = nullptr;
     a.confirm_had = a.confirm_lost = 0;
@@ -787,6 +790,16 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     a.confirm_again = h->confirm_rests >= 255;
     a.index_calls = h->index_calls++;
     (void)plan_rounds(a);
+    if (a.pick_parts > 1) {
+        const int part = (num_queries + a.pick_parts - 1) / a.pick_parts;
+        for (int q = 0; q < num_queries; q += part) {
+            const int rc = query_impl(h, dim, std::min(part, num_queries - q), d_query + (size_t)q * dim, num_neighbours, blind, num_outer_iterations, max_num_candidates,
+                                      block_size, thread_size, d_nn + (size_t)q * num_neighbours, d_dists + (size_t)q * num_neighbours, d_counters, stream, fixed, float_ids, who,
+                                      whole, later_part || q > 0);
+            if (rc) return rc;
+        }
+        return DCIH_OK;
+    }
     h->confirm_rests = a.pick_rounds && !a.pick_confirm ? h->confirm_rests + 1 : 0;
     if (a.pick_near || a.pick_confirm) {
         if (!h->blind && !recorded) {
@@ -885,7 +898,8 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     }
     // events in the order query() records them: traversal start, batch kernel end, dense
     // kernel end, traversal end, merge end
-    hipEvent_t qev[5] = {h->ev[2 * DCIH_T_TRAVERSE], h->ev[2 * DCIH_T_BATCH + 1], h->ev[2 * DCIH_T_DENSE + 1],
+    // (of a call in parts the traversal starts with the first one's)
+    hipEvent_t qev[5] = {later_part ? nullptr : h->ev[2 * DCIH_T_TRAVERSE], h->ev[2 * DCIH_T_BATCH + 1], h->ev[2 * DCIH_T_DENSE + 1],
                          h->ev[2 * DCIH_T_TRAVERSE + 1], h->ev[2 * DCIH_T_MERGE + 1]};
     bool ran[2] = {false, false};
     rc = query(a, base + ws_bytes + q8_bytes, s, h->profiling ? qev : nullptr, ran);
@@ -1003,6 +1017,12 @@ int dcih_debug_round_items(dcih_index* h, uint32_t* d_items) {
 int dcih_debug_confirmed(const dcih_index* h, uint32_t* counts) {
     if (!h || !counts) return fail(DCIH_EINVAL, "dcih_debug_confirmed: null argument");
     for (int i = 0; i < 2; i++) counts[i] = h->blind ? h->blind[1 + i] : 0u;
+    return DCIH_OK;
+}
+
+int dcih_debug_near_room(dcih_index* h, int64_t bytes) {
+    if (!h || bytes < 1) return fail(DCIH_EINVAL, "dcih_debug_near_room: null handle or no room");
+    h->near_room = (size_t)bytes;
     return DCIH_OK;
 }
 

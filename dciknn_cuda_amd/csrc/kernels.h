@@ -140,6 +140,8 @@ struct QueryArgs {
     int near_shift, near_tiles;
     int pick_near;           // 1: a call in rounds goes to the dense kernel and keeps those bounds
     int pick_confirm;        // 1: rounds' items go through confirm.hip first, which needs those bounds too
+    size_t near_room;        // what the tiles' bounds of a call may take
+    int pick_parts;          // above 1: what plan_rounds would do with the call if it came in so many parts
     int pick_sample;         // 0, or: so many queries are traversed whole first, and decide
     float pick_most;         // share of pairs that rounds may have to take: where the sample's bounds leave more, everything is taken at once
     int pick_rounds;         // 0: everything is traversed at once

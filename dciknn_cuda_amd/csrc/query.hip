@@ -473,6 +473,7 @@ static bool confirm_pays(const QueryArgs& a, double items, bool by_dense) {
 
 bool plan_rounds(QueryArgs& a) {
     a.pick_rounds = a.pick_near = a.pick_confirm = a.pick_sample = 0;
+    a.pick_parts = 1;
     a.share = 1.0;
     if (a.mode != 0 || a.pick_rule == 1 || !bounds_supported(a)) return false;
     // The r nearest rows of a query lie in about B (1 - e^(-r/B)) partitions (rows in no particular order).  Round 1
@@ -518,8 +519,18 @@ bool plan_rounds(QueryArgs& a) {
     a.pick_rank = rank;
     a.pick_first = first;
     a.share = share;
-    a.pick_near = !sampled && near_bytes(a) <= ((size_t)1 << 30) ? 1 : 0;
-    a.pick_confirm = confirm_supported(a) && near_bytes(a) <= ((size_t)1 << 30) && confirm_pays(a, (double)a.nq * first, can_dense && takes_dense_kernel(a)) ? 1 : 0;
+    a.pick_near = !sampled;
+    a.pick_confirm = confirm_supported(a) && confirm_pays(a, (double)a.nq * first, can_dense && takes_dense_kernel(a)) ? 1 : 0;
+    // Where the tiles' bounds take more than their room, the dense kernel's calls come as parts of the queries that keep within it, one after the other.  All that
+    // each does again is to read the rows once.  (10000 queries on 10M unit vectors of 96: 397 ms without these bounds, 144 in parts; on 20M normal rows of 64 221, 153;
+    // 60000 on 1M rows of 128 at the defaults 132, 22.4, with room for all 21.6; 20000 on 3M unit vectors 407, 172; where bounds rule out little, 30000 on 2M
+    // normal rows of 64, 3124, 3187.)  A part of the batch kernel's calls takes its own sample and waits for its own slowest items: 60000 queries, windows
+    // of 2, 46.0 ms without the tiles' bounds, 48.9 in two parts.
+    const size_t near = near_bytes(a);
+    if (near > a.near_room) {
+        if (a.pick_near) a.pick_parts = (int)std::min<size_t>((size_t)a.nq, (near + a.near_room - 1) / a.near_room);
+        a.pick_near = a.pick_confirm = 0;
+    }
     a.pick_sample = sampled ? std::min(a.nq, std::max(2, std::min(16, 1024 / a.B))) : 0;
     // Up to which share of the sample's pairs rounds pay: the fewer results, the further away the k-th of the first rounds lies than
     // that of all.  (Five kinds of rows, 16 to 300 elements, 30000 to a million: shares from which rounds begin to take longer are 0.31 to
@@ -641,7 +652,7 @@ int query(const QueryArgs& a_in, void* bounds_ws, hipStream_t s, hipEvent_t* ev,
         DCIH_HIP(hipGetLastError());
         return 0;
     };
-    if (ev) (void)hipEventRecord(ev[0], s);
+    if (ev && ev[0]) (void)hipEventRecord(ev[0], s);
     if (!a.pick_rounds) {
         const int rc = traverse(a);
         if (rc) return rc;

@@ -69,6 +69,10 @@ int dcih_debug_round_items(dcih_index* h, uint32_t* d_items);
  * partition) pairs that it counts were answered so and how many were left to a traversal (zeros: no such query yet).
  */
 int dcih_debug_confirmed(const dcih_index* h, uint32_t* counts);
+/*
+ * How much a query in rounds may take for its bounds of parts of partitions before it is answered in several parts of its queries (1 GiB).
+ */
+int dcih_debug_near_room(dcih_index* h, int64_t bytes);
 
 #ifdef __cplusplus
 }

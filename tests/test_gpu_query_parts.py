@@ -1,0 +1,32 @@
+"""Calls in rounds whose bounds of tiles take more than their room come in parts of their queries: the same ids and distances, to the bit, whether
+the last part is as large as the others, a single query, or every query is a part of its own, and where no room is enough for one.  (The
+batch kernel's calls stay whole.)"""
+import pytest
+import torch
+
+from test_gpu_rounds import ALWAYS, NEVER, _ask, _count_items, _rows
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("parts", [2, 3, 7, 50, 99, 10 ** 6])
+@pytest.mark.parametrize("shape", [(20000, 64, 2, 7, 50, 10, 10, 5000, 99), (24001, 40, 2, 6, 48, 4, 4, 2000, 99), (36000, 48, 2, 15, 60, 128, 30, 10, 99)],
+                         ids=["dense", "batch", "wide"])
+def test_same_as_whole(gpu, shape, parts):
+    from dciknn_cuda_amd import _capi
+    n, dim, M, L, B, T, k, outer, nq = shape
+    X, Q = _rows("clusters", n, nq, dim, 5)
+    dci = gpu.DCI(dim, M, L, B, T, seed=3)
+    dci.add(X)
+    want = _ask(dci, dci._lib, NEVER, Q, k, outer)
+    # (tiles of 64 or 128 rows, partitions padded to whole ones of up to 512 rows: between n / 128 and that of them)
+    tiles = B * (((n + B - 1) // B + 511) // 512 * 512 // 64)
+    _capi.check(dci._lib.dcih_debug_near_room(dci._dci_inst, max(1, tiles * nq * 4 // (2 * parts))))
+    items = _count_items(dci)
+    for again in range(2):
+        got = _ask(dci, dci._lib, ALWAYS, Q, k, outer)
+        assert torch.equal(got[0], want[0]), again
+        assert torch.equal(got[1].view(torch.int32), want[1].view(torch.int32)), again
+    if parts == 50 and T != 4:      # the last part is four queries at most; all of them take ten partitions and more each
+        assert 0 < int(items[:4].sum()) <= 4 * B, items
+    dci.free()
