@@ -53,6 +53,7 @@ SIGNATURES = {
     "dcih_debug_route": (_c.c_int, [_c.c_void_p, _c.POINTER(_c.c_int64)]),
     "dcih_debug_round_items": (_c.c_int, [_c.c_void_p, _c.c_void_p]),
     "dcih_debug_near_room": (_c.c_int, [_c.c_void_p, _c.c_int64]),
+    "dcih_debug_plan": (_c.c_int, [_c.c_void_p, _c.POINTER(_c.c_int64)]),
     "dcih_debug_confirmed": (_c.c_int, [_c.c_void_p, _c.c_void_p]),
     "dcih_debug_positions": (_c.c_int, [_c.c_void_p, _c.c_void_p, _c.c_void_p, _c.c_void_p]),
     "dcih_profile": (_c.c_int, [_c.c_void_p, _c.c_int]),

@@ -159,6 +159,7 @@ struct dcih_index {
     int append_mode = 0;                // DCIH_OPT_APPEND value
     int rounds = 0;                     // DCIH_OPT_ROUNDS value
     int64_t route[4] = {0, 0, 0, 0};    // dcih_debug_route
+    int64_t plan[3] = {0, 0, 0};        // the first of dcih_debug_plan's values
     int confirm_rests = 0;              // calls in rounds that went without confirm.hip, since the last one with it
     int index_calls = 0;                // queries since the index was formed
     size_t near_room = (size_t)1 << 30; // what the bounds of a call's tiles may take
@@ -695,6 +696,8 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
 
     h->ev_valid[DCIH_T_BATCH] = h->ev_valid[DCIH_T_DENSE] = false;
     for (int64_t& r : h->route) r = 0;
+    if (!later_part) h->plan[0] = h->plan[2] = 0;
+    if (!later_part) h->plan[1] = 1;
     QueryArgs a;
     a.skeys = h->d_skeys; a.sids = h->d_sids; a.inv = h->d_inv; a.data = h->d_data; a.query = d_query;
     a.rpos = h->d_rpos; a.rpos_ready = &h->rpos_ready; a.recorded = recorded ? 1 : 0;
@@ -721,6 +724,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     a.confirm_had = a.confirm_lost = 0;
     a.confirm_again = a.index_calls = 0;
     a.selected = &h->route[3];
+    a.window_launches = &h->plan[2];
     a.stop_hint = nullptr;
     a.N = h->n;
     a.ppb = (h->n + block_size - 1) / block_size;
@@ -798,6 +802,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
                                       whole, later_part || q > 0);
             if (rc) return rc;
         }
+        h->plan[1] = a.pick_parts;
         return DCIH_OK;
     }
     h->confirm_rests = a.pick_rounds && !a.pick_confirm ? h->confirm_rests + 1 : 0;
@@ -873,6 +878,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
             a.point_rows = h->d_point_rows;
         }
     }
+    h->plan[0] = a.pick_rounds ? a.pick_confirm : 0;
     h->route[0] = a.pick_rounds; h->route[1] = a.pick_near; h->route[2] = a.pick_sample;
     char* base = ws_base;
     float* d_qproj = (float*)base;
@@ -1017,6 +1023,12 @@ int dcih_debug_round_items(dcih_index* h, uint32_t* d_items) {
 int dcih_debug_confirmed(const dcih_index* h, uint32_t* counts) {
     if (!h || !counts) return fail(DCIH_EINVAL, "dcih_debug_confirmed: null argument");
     for (int i = 0; i < 2; i++) counts[i] = h->blind ? h->blind[1 + i] : 0u;
+    return DCIH_OK;
+}
+
+int dcih_debug_plan(const dcih_index* h, int64_t* plan) {
+    if (!h || !plan) return fail(DCIH_EINVAL, "dcih_debug_plan: null argument");
+    for (int i = 0; i < 3; i++) plan[i] = h->plan[i];
     return DCIH_OK;
 }
 

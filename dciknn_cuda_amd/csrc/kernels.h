@@ -126,6 +126,7 @@ struct QueryArgs {
     uint32_t* blind_word;    // null, or (the host's memory) set where bounds say nothing of queries' nearest rows
     uint32_t* confirm_word;  // null, or (the host's memory) two words: items that confirm.hip answered and left, of those it counts
     int64_t* selected;       // (host) counts the queries that nearest.hip answers
+    int64_t* window_launches;   // (host) counts the launches of the dense kernel that look up first lanes of windows
     uint32_t* picked_ticket; // a zeroed word per die: the dense kernel's workgroups take their items by it
     int64_t picked_exact;    // their number, where it is known: 0 otherwise
     int64_t picked_expect;   // about how many there are, 0: few

@@ -1740,6 +1740,7 @@ int query_dense_items(const QueryArgs& a_in, hipStream_t s) {
         args.step = (int)(per_xcd - resident);
     }
     const unsigned grid = (unsigned)(per_xcd * a.xcds);
+    if (y.by_windows) ++*a.window_launches;
 #define DCIH_DENSE(NT, IPT, WAVES) \
     rc = y.by_windows && IPT <= 9 ? launch_dense<NT, IPT, WAVES, IPT <= 9 ? kWindows : kPicked>(args, grid, s) \
          : (a.picked ? launch_dense<NT, IPT, WAVES, kPicked>(args, grid, s) : launch_dense<NT, IPT, WAVES, kWhole>(args, grid, s))

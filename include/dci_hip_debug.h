@@ -70,6 +70,11 @@ int dcih_debug_round_items(dcih_index* h, uint32_t* d_items);
  */
 int dcih_debug_confirmed(const dcih_index* h, uint32_t* counts);
 /*
+ * How the handle's last dcih_query was planned: plan receives [0] whether near rows were looked at alone before anything was traversed, [1] the parts
+ * of its queries in which it was answered, [2] launches of the dense kernel that looked up the windows' first lanes instead of all points.
+ */
+int dcih_debug_plan(const dcih_index* h, int64_t* plan);
+/*
  * How much a query in rounds may take for its bounds of parts of partitions before it is answered in several parts of its queries (1 GiB).
  */
 int dcih_debug_near_room(dcih_index* h, int64_t bytes);
