@@ -163,8 +163,8 @@ __device__ __forceinline__ bool confirm_item(const ConfirmArgs& a, unsigned char
     const float* base = a.data + off * a.dim;
     const int rows = ntiles << a.near_shift, in_tile = (1 << a.near_shift) - 1;
     {
-        // (what a distance is rounded by is far below the factor; squares that underflow say nothing)
-        const float most2 = fmaxf(most * most * 1.0001f, 1e-30f);
+        // (what a distance is rounded by is far below the factor; squares that underflow say nothing; a limit that is not a number is none)
+        const float most2 = most == most ? fmaxf(most * most * 1.0001f, 1e-30f) : __builtin_inff();
         const bool head = vec4 && a.dim >= 64;
         const int sl = lane & 7;
         float q0 = 0.f, q1 = 0.f, q2 = 0.f, q3 = 0.f;

@@ -50,3 +50,28 @@ def test_same_as_whole(gpu, shape, kind):
     assert answered + left > 0
     if kind == "clusters" and shape != "results":      # rows whose nearest are promoted first
         assert answered > left, (answered, left)
+
+
+@pytest.mark.parametrize("dim", [40, 64, 128, 132])
+@pytest.mark.parametrize("per,nq", [(600, 3), (900, 3), (600, 20)])
+def test_a_distance_that_is_not_a_number_limits_nothing(gpu, dim, per, nq):
+    """A query whose k-th result so far has the distance NaN takes rows at any distance in the rounds that follow.  Two clusters 200 times as far
+    apart as they are wide, so that round 1's limit, a bound, lies below the distances of all but a few finite rows; rows that are not finite,
+    which are promoted with windows that begin with a finite projection, stand at the k-th place until then."""
+    B, k = 24, 8
+    X, Q = _rows("normal", B * per, nq, dim, per + dim)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(3)
+    for rows in (X, Q):
+        rows += 200.0 * torch.randint(0, 2, (len(rows), 1), generator=g, device="cuda") - 100.0
+    X[7:31, 3] = float("nan")
+    dci = gpu.DCI(dim, 1, 2, B, 64, seed=4)
+    dci.add(X)
+    want = _ask(dci, dci._lib, NEVER, Q, k, 5000)
+    assert torch.isfinite(want[1]).all()
+    for again in range(2):
+        got = _ask(dci, dci._lib, ALWAYS, Q, k, 5000)
+        assert _confirmed(dci)[0] > 0
+        assert torch.equal(got[0], want[0]), again
+        assert torch.equal(got[1].view(torch.int32), want[1].view(torch.int32)), again
+    dci.free()
