@@ -805,7 +805,8 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
         h->plan[1] = a.pick_parts;
         return DCIH_OK;
     }
-    h->confirm_rests = a.pick_rounds && !a.pick_confirm ? h->confirm_rests + 1 : 0;
+    if (a.pick_confirm) h->confirm_rests = 0;
+    else if (a.pick_rounds) h->confirm_rests++;
     if (a.pick_near || a.pick_confirm) {
         if (!h->blind && !recorded) {
             void* p = nullptr;

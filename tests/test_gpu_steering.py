@@ -1,0 +1,45 @@
+"""What a handle remembers of its calls to choose the way of the next ones.  (It never shows in results; other tests compare the ways.)"""
+import pytest
+import torch
+
+from test_gpu_rounds import _route, _rows
+
+pytestmark = pytest.mark.gpu
+
+
+def _plan(dci):
+    """(near rows looked at alone first, parts, launches by windows' first lanes) of the last call."""
+    from dciknn_cuda_amd import _capi
+    plan = (_capi.ctypes.c_int64 * 3)()
+    _capi.check(dci._lib.dcih_debug_plan(dci._dci_inst, plan))
+    return tuple(plan)
+
+
+# Rows of which half of the partitions are needed and too many of each are near: items have to be left to the traversals
+N, DIM, M, L, B, T, K, OUTER, QUERIES = 123457, 67, 3, 5, 37, 3, 7, 1000, 1000
+
+
+@pytest.fixture()
+def of_no_use(gpu):
+    """A handle on whose calls near rows alone have just been of no use, its rows and queries."""
+    X, Q = _rows("normal", N, QUERIES, DIM, 5)
+    dci = gpu.DCI(DIM, M, L, B, T, seed=3)
+    dci.add(X)
+    dci.query(Q, K, OUTER, return_int=True)
+    assert _route(dci)[0] >= 2 and _plan(dci)[0] == 1
+    torch.cuda.synchronize()
+    dci.query(Q, K, OUTER, return_int=True)
+    assert _route(dci)[0] >= 2 and _plan(dci)[0] == 0
+    yield dci, X, Q
+    dci.free()
+
+
+def test_near_rows_are_tried_again_whatever_comes_between(of_no_use):
+    dci, _, Q = of_no_use
+    for call in range(300):
+        dci.query(Q, K, OUTER, return_int=True)
+        if _plan(dci)[0]:
+            break
+        dci.query(Q[:1], K, OUTER, return_int=True)      # traversed whole
+        assert _route(dci)[0] == 0
+    assert 200 < call < 256
