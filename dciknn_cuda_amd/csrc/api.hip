@@ -113,6 +113,22 @@ void* scratch_of(int device) {
 }
 }  // namespace
 
+// What confirm.hip has made of queries of one shape, for the plans of the next ones of that shape (other numbers of results, stops and windows leave
+// other items).  Forgotten when the index is formed anew, or for a fifth shape.
+constexpr int kNearRecords = 4;
+struct NearRecord {
+    int k = 0, outer = 0, T = 0, maxc = 0;   // the shape (zeros: none)
+    uint32_t tag = 0;                   // what its words have to bear: calls still under way may write those of an earlier record
+    int rests = 0;                      // calls in rounds that went without confirm.hip, since the last one with it
+    uint64_t last = 0;                  // the last call
+};
+// Words that the device writes and the host reads when it plans a call: they steer work, never results.
+struct HostWords {
+    uint32_t blind;                     // set by queries in rounds whose bounds said nothing: the next ones use the rows' codes
+    uint32_t pad;
+    uint64_t near[kNearRecords];        // tag << 48 | items left << 24 | items answered, of those that confirm.hip counts
+};
+
 struct dcih_index {
     int dim = 0, M = 0, L = 0, device = 0;
     int xcds = 8;                       // accelerator dies of the device
@@ -160,10 +176,13 @@ struct dcih_index {
     int rounds = 0;                     // DCIH_OPT_ROUNDS value
     int64_t route[4] = {0, 0, 0, 0};    // dcih_debug_route
     int64_t plan[3] = {0, 0, 0};        // the first of dcih_debug_plan's values
-    int confirm_rests = 0;              // calls in rounds that went without confirm.hip, since the last one with it
+    NearRecord near_records[kNearRecords];
+    int near_last = -1;                 // the one of the last call that confirm.hip was part of
+    uint32_t near_tag = 0;              // of the last record that was begun
+    uint64_t near_calls = 0;            // calls that had a record
     int index_calls = 0;                // queries since the index was formed
     size_t near_room = (size_t)1 << 30; // what the bounds of a call's tiles may take
-    volatile uint32_t* blind = nullptr; // (pinned: three words) set by queries in rounds whose bounds said nothing: the next ones use the rows' codes; then the items that confirm.hip answered and left, of those it counts
+    volatile HostWords* words = nullptr;   // (pinned, from the first query in rounds that writes them)
     uint32_t* d_round_items = nullptr;  // dcih_debug_round_items
     unsigned long long* d_phase_ticks = nullptr;   // optional profile of the batch kernel
     // grow-only workspace: query scratch, and the unsorted keys during a build
@@ -210,8 +229,39 @@ int draw_directions(dcih_index* h) {
 // The rows change: their codes are formed anew, in the same room if it holds them.
 void forget_rows8(dcih_index* h) {
     h->rows8_ready = h->rows8_no_room = false;
-    if (h->blind) *h->blind = 0;
+    if (h->words) h->words->blind = 0;
     h->rows8_demand = 0.0;
+}
+
+int find_near_record(const dcih_index* h, int k, int outer, int T, int maxc) {
+    for (int i = 0; i < kNearRecords; i++) {
+        const NearRecord& r = h->near_records[i];
+        if (r.k == k && r.outer == outer && r.T == T && r.maxc == maxc) return i;
+    }
+    return -1;
+}
+int begin_near_record(dcih_index* h, int k, int outer, int T, int maxc) {
+    int at = 0;
+    for (int i = 1; i < kNearRecords; i++)
+        if (h->near_records[i].last < h->near_records[at].last) at = i;
+    h->near_tag = h->near_tag % 0xffffu + 1u;
+    NearRecord r;
+    r.k = k; r.outer = outer; r.T = T; r.maxc = maxc; r.tag = h->near_tag;
+    h->near_records[at] = r;
+    return at;
+}
+// The items that were answered and left, as far as calls have written them.
+void read_near_record(const dcih_index* h, int at, uint32_t& had, uint32_t& lost) {
+    had = lost = 0;
+    if (at < 0 || !h->words) return;
+    const uint64_t w = h->words->near[at];
+    if ((uint32_t)(w >> 48) != h->near_records[at].tag) return;
+    had = (uint32_t)w & 0xffffffu;
+    lost = (uint32_t)(w >> 24) & 0xffffffu;
+}
+void forget_near_records(dcih_index* h) {
+    for (NearRecord& r : h->near_records) r = NearRecord();
+    h->near_last = -1;
 }
 
 void release_rows8(dcih_index* h) {
@@ -487,6 +537,7 @@ static int sort_into(dcih_index* h, int which, const float* d_keys, int64_t key_
     h->d_rpos = y.small_parts ? (uint16_t*)(base + y.rpos) : nullptr;
     h->rpos_ready = 0;
     h->index_calls = 0;
+    forget_near_records(h);
     h->d_point_rows = y.point_rows_pay ? (uint16_t*)(base + y.point_rows) : nullptr;
     h->point_rows_ready = 0;
     h->point_rows_demand = 0.0;
@@ -720,7 +771,9 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     a.near_room = h->near_room;
     a.pick_parts = 1;
     a.round_items = h->d_round_items;
-    a.blind_word = a.confirm_word = nullptr;
+    a.blind_word = nullptr;
+    a.confirm_word = nullptr;
+    a.confirm_tag = 0;
     a.confirm_had = a.confirm_lost = 0;
     a.confirm_again = a.index_calls = 0;
     a.selected = &h->route[3];
@@ -790,8 +843,9 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     }
 
     // (where earlier calls' items had to be left, every 256th call tries again: such a try took 0.7 ms longer than 1.5)
-    if (h->blind) { a.confirm_had = h->blind[1]; a.confirm_lost = h->blind[2]; }
-    a.confirm_again = h->confirm_rests >= 255;
+    int record = find_near_record(h, num_neighbours, num_outer_iterations, thread_size, max_num_candidates);
+    read_near_record(h, record, a.confirm_had, a.confirm_lost);
+    a.confirm_again = record >= 0 && h->near_records[record].rests >= 255;
     a.index_calls = h->index_calls++;
     (void)plan_rounds(a);
     if (a.pick_parts > 1) {
@@ -805,18 +859,28 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
         h->plan[1] = a.pick_parts;
         return DCIH_OK;
     }
-    if (a.pick_confirm) h->confirm_rests = 0;
-    else if (a.pick_rounds) h->confirm_rests++;
+    if (a.pick_confirm) {
+        if (record < 0) record = begin_near_record(h, num_neighbours, num_outer_iterations, thread_size, max_num_candidates);
+        h->near_records[record].rests = 0;
+        h->near_last = record;
+    } else if (record >= 0 && a.pick_rounds) {
+        h->near_records[record].rests++;
+    }
+    if (record >= 0) h->near_records[record].last = ++h->near_calls;
     if (a.pick_near || a.pick_confirm) {
-        if (!h->blind && !recorded) {
+        if (!h->words && !recorded) {
             void* p = nullptr;
-            if (hipHostMalloc(&p, 3 * sizeof(uint32_t), hipHostMallocDefault) == hipSuccess) { h->blind = (volatile uint32_t*)p; h->blind[0] = h->blind[1] = h->blind[2] = 0; }
+            if (hipHostMalloc(&p, sizeof(HostWords), hipHostMallocDefault) == hipSuccess) { std::memset(p, 0, sizeof(HostWords)); h->words = (volatile HostWords*)p; }
             else (void)hipGetLastError();
         }
         void* p = nullptr;
-        if (h->blind && hipHostGetDevicePointer(&p, (void*)h->blind, 0) == hipSuccess) { a.blind_word = a.pick_near ? (uint32_t*)p : nullptr; a.confirm_word = (uint32_t*)p + 1; }
+        if (h->words && hipHostGetDevicePointer(&p, (void*)h->words, 0) == hipSuccess) {
+            HostWords* d_words = (HostWords*)p;
+            if (a.pick_near) a.blind_word = &d_words->blind;
+            if (a.pick_confirm) { a.confirm_word = (unsigned long long*)&d_words->near[record]; a.confirm_tag = h->near_records[record].tag; }
+        }
     }
-    const bool bounds_failed = h->blind && *h->blind;      // (of earlier calls: it steers work, never results)
+    const bool bounds_failed = h->words && h->words->blind;      // (of earlier calls)
     size_t q8_bytes = 0;
     if (!blind && (!a.pick_near || bounds_failed) && dense_traversal_supported(a, nullptr)) {      // (near rows only: few enough to be read whole)
         const bool all_dense = takes_dense_kernel(a);
@@ -1023,7 +1087,7 @@ int dcih_debug_round_items(dcih_index* h, uint32_t* d_items) {
 
 int dcih_debug_confirmed(const dcih_index* h, uint32_t* counts) {
     if (!h || !counts) return fail(DCIH_EINVAL, "dcih_debug_confirmed: null argument");
-    for (int i = 0; i < 2; i++) counts[i] = h->blind ? h->blind[1 + i] : 0u;
+    read_near_record(h, h->near_last, counts[0], counts[1]);
     return DCIH_OK;
 }
 
@@ -1122,7 +1186,7 @@ int dcih_free(dcih_index* h) {
     for (auto& e : h->ev) if (e) (void)hipEventDestroy(e);
     if (h->busy) (void)hipEventDestroy(h->busy);
     if (h->rows8_event) (void)hipEventDestroy(h->rows8_event);
-    if (h->blind) (void)hipHostFree((void*)h->blind);
+    if (h->words) (void)hipHostFree((void*)h->words);
     delete h;
     return DCIH_OK;
 }

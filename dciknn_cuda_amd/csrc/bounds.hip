@@ -578,7 +578,7 @@ struct ListArgs {
     const float* worst; int64_t worst_stride;      // the k-th distance each query has so far
     uint32_t* last_round;                          // the round that last took a partition of the query
     int B, parts, nq, groups, round, rounds, near;
-    uint32_t* rests; uint32_t* confirm_word; int confirm_dies;      // (0: confirm.hip has no part in the call)
+    uint32_t* rests; unsigned long long* confirm_word; uint32_t confirm_tag; int confirm_dies;      // (0: confirm.hip has no part in the call)
     const float* near_then; float* near_now;       // how far rows counted in the round before, and in this one
     int32_t* items; uint32_t* count; uint32_t* part_counts; uint32_t* ticket;
 };
@@ -633,8 +633,10 @@ __global__ __launch_bounds__(256) void list_items_kernel(ListArgs a) {
             a.rests[0] = lost > 16 + had ? 1u : 0u;
             if (a.round == 0) a.rests[1] = 0;
             if (a.confirm_word && a.round > 0) {
-                reinterpret_cast<volatile uint32_t*>(a.confirm_word)[0] = had;
-                reinterpret_cast<volatile uint32_t*>(a.confirm_word)[1] = lost;
+                // (one store, so that the host reads what belongs together; their ratio is what matters)
+                uint32_t h = had, l = lost;
+                while ((h | l) >> 24) { h >>= 1; l >>= 1; }
+                *reinterpret_cast<volatile unsigned long long*>(a.confirm_word) = (unsigned long long)a.confirm_tag << 48 | (unsigned long long)l << 24 | h;
             }
         }
     }
@@ -946,7 +948,7 @@ int pick_items(const QueryArgs& a, void* ws_, int round, int rounds, hipStream_t
     }
     const int groups = (a.nq + kListQueries - 1) / kListQueries;
     ListArgs p{bounds, limits, a.pick_sample ? (const uint32_t*)(ws + r.counts) + kSkipWord : nullptr, a.out_dists + (a.k - 1), a.k, last, a.B, r.parts, a.nq, groups, round, rounds, a.pick_near,
-                 (uint32_t*)(ws + r.counts) + kRestsWord, a.pick_confirm ? a.confirm_word : nullptr, a.pick_confirm ? a.xcds : 0, near_limits(ws, r, a.nq, round - 1), near_limits(ws, r, a.nq, round),
+                 (uint32_t*)(ws + r.counts) + kRestsWord, a.pick_confirm ? a.confirm_word : nullptr, a.confirm_tag, a.pick_confirm ? a.xcds : 0, near_limits(ws, r, a.nq, round - 1), near_limits(ws, r, a.nq, round),
                (int32_t*)(ws + r.items), (uint32_t*)(ws + r.counts) + round, (uint32_t*)(ws + r.part_counts),
                (uint32_t*)(ws + r.counts) + kTicketWord};
     const dim3 grid((unsigned)((int64_t)a.B * groups));

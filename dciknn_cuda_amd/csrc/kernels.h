@@ -124,7 +124,8 @@ struct QueryArgs {
     int64_t left_cap;
     uint32_t* round_items;   // null, or device words for the number of items of every round, then the sample's decision
     uint32_t* blind_word;    // null, or (the host's memory) set where bounds say nothing of queries' nearest rows
-    uint32_t* confirm_word;  // null, or (the host's memory) two words: items that confirm.hip answered and left, of those it counts
+    unsigned long long* confirm_word;   // null, or (the host's memory) confirm_tag << 48 | items that confirm.hip left << 24 | answered, of those it counts
+    uint32_t confirm_tag;
     int64_t* selected;       // (host) counts the queries that nearest.hip answers
     int64_t* window_launches;   // (host) counts the launches of the dense kernel that look up first lanes of windows
     uint32_t* picked_ticket; // a zeroed word per die: the dense kernel's workgroups take their items by it
@@ -147,7 +148,7 @@ struct QueryArgs {
     float pick_most;         // share of pairs that rounds may have to take: where the sample's bounds leave more, everything is taken at once
     int pick_rounds;         // 0: everything is traversed at once
     int pick_rank;           // the first round takes the partitions of so many nearest rows
-    uint32_t confirm_had, confirm_lost;   // of the items that confirm.hip counted in the last call that it was part of, those that it answered and left
+    uint32_t confirm_had, confirm_lost;   // of the items that confirm.hip counted in the last call of this shape that it was part of, those that it answered and left
     int confirm_again;       // 1: whatever they say, it is tried
     int index_calls;         // queries of this index before
     int pick_rule;           // DCIH_OPT_ROUNDS value

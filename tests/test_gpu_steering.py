@@ -43,3 +43,30 @@ def test_near_rows_are_tried_again_whatever_comes_between(of_no_use):
         dci.query(Q[:1], K, OUTER, return_int=True)      # traversed whole
         assert _route(dci)[0] == 0
     assert 200 < call < 256
+
+
+@pytest.mark.parametrize("other", ["results", "steps", "rows", "appended rows"])
+def test_what_near_rows_were_no_use_for_says_nothing_of_other_calls(of_no_use, other):
+    dci, X, Q = of_no_use
+    if other in ("rows", "appended rows"):
+        dci.clear()
+        if other == "rows":
+            dci.add(X)
+        else:
+            dci.append(X)
+    k, outer = K + (other == "results"), OUTER - 100 * (other == "steps")
+    dci.query(Q, k, outer, return_int=True)
+    assert _route(dci)[0] >= 2 and _plan(dci)[0] == 1
+    torch.cuda.synchronize()
+    dci.query(Q, K, OUTER, return_int=True)      # (of its own record, which the other call has left as it was, or begun)
+    assert _route(dci)[0] >= 2 and _plan(dci)[0] == 0
+
+
+def test_many_shapes_of_queries_in_turn(of_no_use):
+    """More of them than records are kept: each is tried again when its record was given to another."""
+    dci, _, Q = of_no_use
+    for turn in range(2):
+        for k in range(K + 1, K + 6):
+            dci.query(Q, k, OUTER, return_int=True)
+            assert _plan(dci)[0] == 1, (turn, k)
+            torch.cuda.synchronize()
