@@ -775,7 +775,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     a.confirm_word = nullptr;
     a.confirm_tag = 0;
     a.confirm_had = a.confirm_lost = 0;
-    a.confirm_again = a.index_calls = 0;
+    a.index_calls = 0;
     a.selected = &h->route[3];
     a.window_launches = &h->plan[2];
     a.stop_hint = nullptr;
@@ -842,10 +842,10 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
         return rc;
     }
 
-    // (where earlier calls' items had to be left, every 256th call tries again: such a try took 0.7 ms longer than 1.5)
+    // (where earlier calls' items had to be left, every 256th call tries again, as if nothing were on record: a few items go ahead)
     int record = find_near_record(h, num_neighbours, num_outer_iterations, thread_size, max_num_candidates);
     read_near_record(h, record, a.confirm_had, a.confirm_lost);
-    a.confirm_again = record >= 0 && h->near_records[record].rests >= 255;
+    if (record >= 0 && h->near_records[record].rests >= 255) a.confirm_had = a.confirm_lost = 0;
     a.index_calls = h->index_calls++;
     (void)plan_rounds(a);
     if (a.pick_parts > 1) {

@@ -149,7 +149,6 @@ struct QueryArgs {
     int pick_rounds;         // 0: everything is traversed at once
     int pick_rank;           // the first round takes the partitions of so many nearest rows
     uint32_t confirm_had, confirm_lost;   // of the items that confirm.hip counted in the last call of this shape that it was part of, those that it answered and left
-    int confirm_again;       // 1: whatever they say, it is tried
     int index_calls;         // queries of this index before
     int pick_rule;           // DCIH_OPT_ROUNDS value
     double pick_first;       // partitions per query the first round is expected to take

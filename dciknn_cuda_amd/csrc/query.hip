@@ -468,7 +468,7 @@ static bool confirm_pays(const QueryArgs& a, double items, bool by_dense) {
     if (item < 0.024) return false;
     if (items <= 4096.0 && confirm_scans(a) && !*a.rpos_ready && a.index_calls == 0) return false;
     const double may = items <= 16384.0 ? 1.0 / 256.0 : fmin(1.0, (item - 0.022) / 0.02);
-    return a.confirm_again || (double)a.confirm_lost <= (items <= 16384.0 ? 0.0 : 16.0) + may * (double)a.confirm_had;
+    return (double)a.confirm_lost <= (items <= 16384.0 ? 0.0 : 16.0) + may * (double)a.confirm_had;
 }
 
 bool plan_rounds(QueryArgs& a) {

@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+from test_gpu_confirm import _confirmed
 from test_gpu_rounds import _route, _rows
 
 pytestmark = pytest.mark.gpu
@@ -43,6 +44,10 @@ def test_near_rows_are_tried_again_whatever_comes_between(of_no_use):
         dci.query(Q[:1], K, OUTER, return_int=True)      # traversed whole
         assert _route(dci)[0] == 0
     assert 200 < call < 256
+    # (a few items ahead of the others, up to 64 a die, and no more of them: the others go to the traversals at once)
+    torch.cuda.synchronize()
+    answered, left = _confirmed(dci)
+    assert answered == 0 and 17 < left <= 17 + 64 * 8
 
 
 @pytest.mark.parametrize("other", ["results", "steps", "rows", "appended rows"])
