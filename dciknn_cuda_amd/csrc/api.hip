@@ -765,7 +765,7 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     a.expect_steps = a.expect_promotions = 0.0f;
     a.rows8 = nullptr; a.rows8_rec = 0; a.rows8_bounds = nullptr; a.query8 = nullptr;
     a.picked = nullptr; a.picked_count = nullptr; a.picked_exact = a.picked_cover = a.picked_expect = 0; a.picked_ticket = nullptr; a.left = nullptr; a.left_count = nullptr; a.left_cap = 0; a.only = nullptr; a.only_round = 0;
-    a.share = 1.0; a.pick_first = 0.0; a.pick_rounds = a.pick_rank = a.pick_near = a.pick_confirm = a.pick_sample = 0; a.pick_most = 1.0f;
+    a.share = 1.0; a.pick_first = 0.0; a.pick_rounds = a.pick_rank = a.pick_near = a.pick_confirm = a.may_confirm = a.pick_sample = 0; a.pick_most = 1.0f;
     a.near_bounds = nullptr; a.near_limit = nullptr; a.near_stride = 0; a.near_shift = a.near_tiles = 0; a.pick_rule = fixed || whole ? 1 : h->rounds;
     a.phase_ticks = h->d_phase_ticks;
     a.near_room = h->near_room;
@@ -924,7 +924,19 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     const size_t wide_bytes = align_up((size_t)a.wide_cap * sizeof(int32_t));
     const size_t ws_bytes = qp_bytes + part_bytes + gs_bytes + redo_bytes + 256 + dense_bytes + wide_bytes;
     if (fixed && ws_bytes + q8_bytes > kScratchBytes) { a.rows8 = nullptr; q8_bytes = 0; }
-    int rc = get_ws(ws_bytes + q8_bytes + (a.pick_rounds ? bounds_bytes(a) : 0));
+    // (room for confirm.hip also where this call goes without it: the next one like it may not, and may be recorded, when nothing can grow)
+    const size_t need = ws_bytes + q8_bytes + (a.pick_rounds ? bounds_bytes(a) : 0);
+    size_t most = need;
+    if (a.pick_rounds && a.may_confirm && !a.pick_confirm) {
+        QueryArgs with = a;
+        with.pick_confirm = 1;
+        most = ws_bytes + q8_bytes + bounds_bytes(with);
+    }
+    int rc = get_ws(most);
+    if (rc && most > need) {
+        (void)hipGetLastError();
+        rc = get_ws(need);
+    }
     if (rc && a.pick_rounds) {      // no room for the bounds: everything is traversed, which needs less (the same results)
         (void)hipGetLastError();
         return query_impl(h, dim, num_queries, d_query, num_neighbours, blind, num_outer_iterations, max_num_candidates,

@@ -142,6 +142,7 @@ struct QueryArgs {
     int near_shift, near_tiles;
     int pick_near;           // 1: a call in rounds goes to the dense kernel and keeps those bounds
     int pick_confirm;        // 1: rounds' items go through confirm.hip first, which needs those bounds too
+    int may_confirm;         // 1: a later call like this one may
     size_t near_room;        // what the tiles' bounds of a call may take
     int pick_parts;          // above 1: what plan_rounds would do with the call if it came in so many parts
     int pick_sample;         // 0, or: so many queries are traversed whole first, and decide

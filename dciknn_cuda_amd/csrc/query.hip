@@ -462,10 +462,13 @@ bool takes_dense_kernel(const QueryArgs& a) {
 // too many (331 rows, a sixth of the items left: 2.64, 3.15; 2818 rows, a twelfth: 9.19, 5.86).  Calls that are over soon have to be answered as a whole, or
 // they wait for a traversal as well (455 items, 25 left: 278 us, 444; 5800, a fifth left: 1.44, 1.55 ms), and the positions by the first simple index, which
 // it reads, are not formed for the first small call of an index (one that is formed anew for a few lookups).
-static bool confirm_pays(const QueryArgs& a, double items, bool by_dense) {
+// may_pay: whether it can be so for such a call at all, whatever the index's calls so far.
+static bool confirm_pays(const QueryArgs& a, double items, bool by_dense, int& may_pay) {
+    may_pay = 1;
     if (a.pick_rule == 2) return true;
     const double item = by_dense ? traversal_costs(a, 0.0).dense_item : 1.0;
-    if (item < 0.024) return false;
+    may_pay = item >= 0.024;
+    if (!may_pay) return false;
     if (items <= 4096.0 && confirm_scans(a) && !*a.rpos_ready && a.index_calls == 0) return false;
     const double may = items <= 16384.0 ? 1.0 / 256.0 : fmin(1.0, (item - 0.022) / 0.02);
     return (double)a.confirm_lost <= (items <= 16384.0 ? 0.0 : 16.0) + may * (double)a.confirm_had;
@@ -520,7 +523,8 @@ bool plan_rounds(QueryArgs& a) {
     a.pick_first = first;
     a.share = share;
     a.pick_near = !sampled;
-    a.pick_confirm = confirm_supported(a) && confirm_pays(a, (double)a.nq * first, can_dense && takes_dense_kernel(a)) ? 1 : 0;
+    a.may_confirm = 0;
+    a.pick_confirm = confirm_supported(a) && confirm_pays(a, (double)a.nq * first, can_dense && takes_dense_kernel(a), a.may_confirm) ? 1 : 0;
     // Where the tiles' bounds take more than their room, the dense kernel's calls come as parts of the queries that keep within it, one after the other.  All that
     // each does again is to read the rows once.  (10000 queries on 10M unit vectors of 96: 397 ms without these bounds, 144 in parts; on 20M normal rows of 64 221, 153;
     // 60000 on 1M rows of 128 at the defaults 132, 22.4, with room for all 21.6; 20000 on 3M unit vectors 407, 172; where bounds rule out little, 30000 on 2M
@@ -529,7 +533,7 @@ bool plan_rounds(QueryArgs& a) {
     const size_t near = near_bytes(a);
     if (near > a.near_room) {
         if (a.pick_near) a.pick_parts = (int)std::min<size_t>((size_t)a.nq, (near + a.near_room - 1) / a.near_room);
-        a.pick_near = a.pick_confirm = 0;
+        a.pick_near = a.pick_confirm = a.may_confirm = 0;
     }
     a.pick_sample = sampled ? std::min(a.nq, std::max(2, std::min(16, 1024 / a.B))) : 0;
     // Up to which share of the sample's pairs rounds pay: the fewer results, the further away the k-th of the first rounds lies than

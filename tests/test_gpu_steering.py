@@ -75,3 +75,39 @@ def test_many_shapes_of_queries_in_turn(of_no_use):
             dci.query(Q, k, OUTER, return_int=True)
             assert _plan(dci)[0] == 1, (turn, k)
             torch.cuda.synchronize()
+
+
+def test_a_call_fits_the_room_of_the_one_before_it(gpu):
+    """An index's first small call goes without near rows, the next one not: it finds its room all the same, also where nothing can grow, under
+    capture (and where no build has left a workspace that holds it by chance)."""
+    from dciknn_cuda_amd import _capi
+    n, dim, nq, B, T, k = 200_000, 64, 32, 100, 10, 10
+    X, Q = _rows("clusters", n, nq, dim, 6)
+    dci = gpu.DCI(dim, 2, 7, B, T, seed=3)
+    dci.append(X)
+    ids = torch.empty((nq, k), dtype=torch.int32, device="cuda")
+    dists = torch.empty((nq, k), dtype=torch.float32, device="cuda")
+
+    def call(stream):
+        _capi.check(dci._lib.dcih_query(dci._dci_inst, dim, nq, Q.data_ptr(), k, 0, 5000, 10 * k, B, T,
+                                        ids.data_ptr(), dists.data_ptr(), None, stream))
+    s = torch.cuda.Stream()
+    call(s.cuda_stream)
+    s.synchronize()
+    assert _route(dci)[0] >= 2 and _plan(dci)[0] == 0
+    want = ids.clone(), dists.clone()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        call(torch.cuda.current_stream().cuda_stream)
+    assert _route(dci)[0] >= 2 and _plan(dci)[0] == 1
+    for _ in range(3):
+        ids.fill_(-5)
+        dists.fill_(-5.0)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(ids, want[0]) and torch.equal(dists, want[1])
+        call(0)                                # eager work between the replays
+        torch.cuda.synchronize()
+    del g
+    dci.free()
