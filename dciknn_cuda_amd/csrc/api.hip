@@ -145,9 +145,12 @@ struct dcih_index {
     uint16_t* d_rpos = nullptr;         // [I][n] the same, in the order of each composite's first simple index (room kept by the
                                         // build, filled by the first query that runs the batch traversal kernel)
     int rpos_ready = 0;
-    uint16_t* d_point_rows = nullptr;   // null, or room for every point's positions side by side (where windows are wide; filled by a call
-                                        // in rounds, once such calls have asked for more than that costs)
+    // every point's positions side by side (where windows are wide): room taken and filled by a call in rounds, once such calls
+    // have asked for more than that costs
+    uint16_t* d_point_rows = nullptr;
+    size_t point_rows_room = 0;
     int point_rows_ready = 0;
+    bool point_rows_no_room = false;    // there was no memory for them: not asked for again until the next build
     double point_rows_demand = 0.0;     // points looked at by such calls so far, in indexes' worth
     // 8-bit codes of the rows and the partitions' bounds behind them (rows8.hip): room taken and codes formed
     // once the dense kernel's calls have asked for more candidate rows than forming them costs
@@ -233,6 +236,45 @@ void forget_rows8(dcih_index* h) {
     h->rows8_demand = 0.0;
 }
 
+void forget_point_rows(dcih_index* h) {
+    h->point_rows_ready = 0;
+    h->point_rows_no_room = false;
+    h->point_rows_demand = 0.0;
+}
+// For an index of n points: the room goes where it does not hold the points' positions, or none would be looked up.
+void fit_point_rows(dcih_index* h, int64_t n, int block_size, int thread_size) {
+    if (!h->d_point_rows) return;
+    if (point_rows_fit((n + block_size - 1) / block_size, h->M, h->L, thread_size) && point_rows_bytes(n, h->M, h->L) <= h->point_rows_room) return;
+    (void)hipFree(h->d_point_rows);
+    h->d_point_rows = nullptr;
+    h->point_rows_room = 0;
+    h->point_rows_ready = 0;
+}
+// Whether the positions are there for a call on stream `s`; fills the table when calls have asked for enough.
+constexpr double kPointRowsDemand = 16.0;
+int use_point_rows(dcih_index* h, double points, bool recorded, hipStream_t s, bool& use) {
+    use = h->point_rows_ready != 0;
+    h->point_rows_demand += points;
+    if (use || h->point_rows_demand < kPointRowsDemand || h->point_rows_no_room) return 0;
+    const size_t need = point_rows_bytes(h->n, h->M, h->L);
+    if (need > h->point_rows_room) {
+        if (recorded) return 0;
+        if (h->d_point_rows) { DCIH_HIP(hipFree(h->d_point_rows)); h->d_point_rows = nullptr; h->point_rows_room = 0; }
+        if (hipMalloc((void**)&h->d_point_rows, need) != hipSuccess) {      // points' times do as well
+            (void)hipGetLastError();
+            h->d_point_rows = nullptr;
+            h->point_rows_no_room = true;
+            return 0;
+        }
+        h->point_rows_room = need;
+    }
+    const int rc = fill_point_rows(h->d_inv, h->d_point_rows, h->n, h->M, h->L, s);
+    if (rc) return rc;
+    if (!recorded) h->point_rows_ready = 1;
+    use = true;
+    return 0;
+}
+
 int find_near_record(const dcih_index* h, int k, int outer, int T, int maxc) {
     for (int i = 0; i < kNearRecords; i++) {
         const NearRecord& r = h->near_records[i];
@@ -276,8 +318,7 @@ int release_sorted(dcih_index* h) {
     h->d_inv = nullptr;
     h->d_rpos = nullptr;
     h->rpos_ready = 0;
-    h->d_point_rows = nullptr;
-    h->point_rows_ready = 0;
+    forget_point_rows(h);
     forget_rows8(h);
     h->d_stop_hint = nullptr;
     return 0;
@@ -355,13 +396,11 @@ int ensure_arena(dcih_index* h, int which, size_t bytes) {
 
 // Where the arrays of an index of n points lie inside an arena.
 struct ArenaLayout {
-    bool point_rows_pay;
-    size_t keys, ids, inv, rpos, point_rows, hint, total;   // byte offsets, and the size of it all
+    size_t keys, ids, inv, rpos, hint, total;   // byte offsets, and the size of it all
     bool small_parts;                           // partitions of at most 65536 points: 16-bit tables exist
 };
-ArenaLayout arena_layout(int M, int L, int64_t n, int block_size, int thread_size) {
+ArenaLayout arena_layout(int I, int64_t n, int block_size) {
     ArenaLayout y;
-    const int I = M * L;
     const size_t cells = (size_t)I * (size_t)n;
     y.small_parts = (n + block_size - 1) / block_size <= 65536;
     const size_t b_keys = align_up(cells * sizeof(float));
@@ -373,14 +412,10 @@ ArenaLayout arena_layout(int M, int L, int64_t n, int block_size, int thread_siz
     y.ids = b_keys;
     y.inv = y.ids + b_ids;
     y.rpos = y.inv + b_inv;
-    y.point_rows = y.rpos + b_inv;
-    y.point_rows_pay = y.small_parts && point_rows_fit((n + block_size - 1) / block_size, M, L, thread_size);
-    y.hint = y.point_rows + (y.point_rows_pay ? align_up(point_rows_bytes(n, M, L)) : 0);
+    y.hint = y.rpos + b_inv;
     y.total = y.hint + b_hint;
     return y;
 }
-
-constexpr double kPointRowsDemand = 16.0;
 
 size_t rows8_records(const dcih_index* h, int64_t n) { return align_up((size_t)n * rows8_record_bytes(h->dim)); }
 size_t rows8_room(const dcih_index* h, int64_t n, int block_size) {
@@ -511,10 +546,10 @@ int dcih_set_directions(dcih_index* h, const float* h_dirs) {
 // With merge_from > 0 the live index (over the first merge_from points, in the other arena) is
 // merged with the sorted new points instead of everything being sorted again.
 static int sort_into(dcih_index* h, int which, const float* d_keys, int64_t key_stride,
-                     int64_t num_points, const float* d_data, int block_size, int thread_size, void* d_tmp,
+                     int64_t num_points, const float* d_data, int block_size, void* d_tmp,
                      hipStream_t s, int64_t merge_from = 0) {
     const int I = num_indices(h);
-    const ArenaLayout y = arena_layout(h->M, h->L, num_points, block_size, thread_size);
+    const ArenaLayout y = arena_layout(I, num_points, block_size);
     char* base = (char*)h->arena[which];
     float* skeys = (float*)(base + y.keys);
     int32_t* sids = (int32_t*)(base + y.ids);
@@ -538,9 +573,7 @@ static int sort_into(dcih_index* h, int which, const float* d_keys, int64_t key_
     h->rpos_ready = 0;
     h->index_calls = 0;
     forget_near_records(h);
-    h->d_point_rows = y.point_rows_pay ? (uint16_t*)(base + y.point_rows) : nullptr;
-    h->point_rows_ready = 0;
-    h->point_rows_demand = 0.0;
+    forget_point_rows(h);
     forget_rows8(h);
     h->cur = which;
     h->d_data = d_data;
@@ -570,7 +603,8 @@ int dcih_add(dcih_index* h, int dim, int64_t num_points, const float* d_data,
     if (rc) return rc;
     release_rows(h);                // (rows of appends before a clear: this index borrows its rows)
     if (h->rows8_bytes < rows8_room(h, num_points, block_size)) release_rows8(h);
-    rc = ensure_arena(h, h->cur, arena_layout(h->M, h->L, num_points, block_size, thread_size).total);
+    fit_point_rows(h, num_points, block_size, thread_size);
+    rc = ensure_arena(h, h->cur, arena_layout(I, num_points, block_size).total);
     if (rc == DCIH_OK) rc = ensure_ws(h, b_keys + align_up(tmp_bytes), s);
     if (rc == DCIH_OK) {
         float* d_keys = (float*)h->ws;
@@ -578,7 +612,7 @@ int dcih_add(dcih_index* h, int dim, int64_t num_points, const float* d_data,
         rc = project(h->d_dirs, I, d_data, num_points, dim, d_keys, num_points, s);
         mark(h, DCIH_T_PROJECT, 1, s);
         if (rc == DCIH_OK)
-            rc = sort_into(h, h->cur, d_keys, num_points, num_points, d_data, block_size, thread_size,
+            rc = sort_into(h, h->cur, d_keys, num_points, num_points, d_data, block_size,
                            tmp_bytes ? (void*)((char*)h->ws + b_keys) : nullptr, s);
         else
             (void)hipStreamSynchronize(s);
@@ -644,8 +678,7 @@ int dcih_append(dcih_index* h, int dim, int64_t num_points, const float* d_data,
     }
     const size_t tmp_bytes = merge ? segsort_append_tmp_bytes(I, total) : segsort_tmp_bytes(I, total, block_size);
     rc = ensure_arena(h, h->n > 0 ? spare : h->cur,
-                          std::max(arena_layout(h->M, h->L, total, block_size, thread_size).total,
-                                   arena_layout(h->M, h->L, cap, block_size, thread_size).total));
+                          std::max(arena_layout(I, total, block_size).total, arena_layout(I, cap, block_size).total));
     if (rc == DCIH_OK && tmp_bytes) rc = ensure_ws(h, align_up(tmp_bytes), s);
     hipError_t e = hipSuccess;
     if (rc == DCIH_OK && h->n > 0 && rows != h->d_data)        // rows (and projections) indexed so far
@@ -667,7 +700,7 @@ int dcih_append(dcih_index* h, int dim, int64_t num_points, const float* d_data,
     }
     if (rc == DCIH_OK)
         // the partition boundaries move with the total, so every slice is formed again
-        rc = sort_into(h, h->n > 0 ? spare : h->cur, ukeys, cap, total, rows, block_size, thread_size,
+        rc = sort_into(h, h->n > 0 ? spare : h->cur, ukeys, cap, total, rows, block_size,
                        tmp_bytes ? h->ws : nullptr, s, merge ? h->n : 0);
     else
         (void)hipStreamSynchronize(s);
@@ -685,6 +718,7 @@ int dcih_append(dcih_index* h, int dim, int64_t num_points, const float* d_data,
         h->own_rows = cap;
     }
     h->ukeys_rows = total;
+    fit_point_rows(h, total, block_size, thread_size);
     return DCIH_OK;
 }
 
@@ -944,16 +978,11 @@ static int query_impl(dcih_index* h, int dim, int num_queries, const float* d_qu
     }
     if (rc) return rc;
     // A point's positions side by side for the dense kernel's near rows.  To form them takes as long as the look-ups of all points by eight queries.
-    if (a.pick_rounds && a.pick_near && h->d_point_rows && point_rows_fit(a.ppb, a.M, a.L, a.T) && point_rows_pay(a)) {
-        h->point_rows_demand += (double)num_queries * a.share;
-        if (!h->point_rows_ready && h->point_rows_demand >= kPointRowsDemand) {
-            rc = fill_point_rows(h->d_inv, h->d_point_rows, h->n, h->M, h->L, s);
-            if (rc) return rc;
-            a.point_rows = h->d_point_rows;
-            if (!recorded) h->point_rows_ready = 1;
-        } else if (h->point_rows_ready) {
-            a.point_rows = h->d_point_rows;
-        }
+    if (a.pick_rounds && a.pick_near && point_rows_fit(a.ppb, a.M, a.L, a.T) && point_rows_pay(a)) {
+        bool use = false;
+        rc = use_point_rows(h, (double)num_queries * a.share, recorded, s, use);
+        if (rc) return rc;
+        if (use) a.point_rows = h->d_point_rows;
     }
     h->plan[0] = a.pick_rounds ? a.pick_confirm : 0;
     h->route[0] = a.pick_rounds; h->route[1] = a.pick_near; h->route[2] = a.pick_sample;
@@ -1192,6 +1221,7 @@ int dcih_free(dcih_index* h) {
     (void)release_index(h);
     release_rows(h);
     release_rows8(h);
+    if (h->d_point_rows) (void)hipFree(h->d_point_rows);
     (void)release_arena(h);
     if (h->ws) (void)hipFree(h->ws);
     if (h->d_dirs) (void)hipFree(h->d_dirs);

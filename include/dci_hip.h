@@ -185,7 +185,11 @@ int dcih_append(dcih_index* h, int dim, int64_t num_points, const float* d_data,
  * kernel's calls have asked for twice as many candidates as there are rows of 96 to 1024
  * elements, the call that gets there forms 8-bit codes of the rows, about a quarter of
  * their size (without memory for them whole rows are compared).
- * Later calls compare rows by their codes first; results do not depend on it.  Under
+ * Later calls compare rows by their codes first; results do not depend on it.  Where windows
+ * are wide (from about 48 points, partitions of 8000 points and more) calls in rounds that have asked
+ * for 16 times as many points as the index holds form a table of every point's positions,
+ * 2 * num_comp_indices * (num_simp_indices up to a multiple of 8) bytes a point, which stays for the indexes
+ * that follow as long as it holds theirs (without memory for it nothing is formed).  Under
  * stream capture nothing is allocated and no codes are formed; what calls before the
  * capture have allocated and formed is used.
  *

@@ -111,3 +111,104 @@ def test_a_call_fits_the_room_of_the_one_before_it(gpu):
         torch.cuda.synchronize()
     del g
     dci.free()
+
+
+def _held(make):
+    """Device bytes that the handle made by `make` holds, and it."""
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    dci = make()
+    torch.cuda.synchronize()
+    return before - torch.cuda.mem_get_info()[0], dci
+
+
+def test_no_room_is_held_for_positions_that_nothing_looks_up(gpu):
+    """Wide windows, partitions too short for first lanes to be looked up: index and the build's workspace are all that is held."""
+    n, M, L = 1_000_000, 2, 15
+    X = torch.randn(n, 32, generator=torch.Generator(device="cuda").manual_seed(1), device="cuda")
+
+    def make():
+        dci = gpu.DCI(32, M, L, 900, 128, seed=3)
+        dci.add(X)
+        return dci
+    gpu.DCI(32, M, L, 900, 128, seed=3).free()      # (what the library itself takes at its first use)
+    held, dci = _held(make)
+    dci.free()
+    # keys, ids and two tables of positions, 12 bytes an entry, and the unsorted keys of the build: 4 more
+    assert held < 16 * n * M * L + (16 << 20), held
+
+
+@pytest.mark.parametrize("then", ["add", "add more", "append", "other stream"])
+def test_positions_side_by_side_are_those_of_the_index(gpu, then):
+    """The table of positions by points is formed anew for every index, whether its room holds it or not."""
+    from dciknn_cuda_amd import _capi
+    from test_gpu_rounds import ALWAYS, NEVER, _ask
+    M, L, B, T, k, outer, dim = 2, 9, 4, 100, 8, 60, 24
+    X, Q = _rows("normal", 30000, 80, dim, 7)
+    dci = gpu.DCI(dim, M, L, B, T, seed=5)
+
+    def check():
+        want = _ask(dci, dci._lib, NEVER, Q, k, outer)
+        for again in range(3):      # (formed once enough was asked for)
+            got = _ask(dci, dci._lib, ALWAYS, Q, k, outer)
+            assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), again
+        assert _plan(dci)[2] > 0
+    (dci.append if then == "append" else dci.add)(X[:24000])
+    check()
+    if then == "append":
+        dci.append(X[24000:])
+    else:
+        dci.clear()
+        X = X.flip(0).contiguous()
+        dci.add(X[:24000] if then == "add" else X)
+    if then == "other stream":
+        torch.cuda.synchronize()
+        with torch.cuda.stream(torch.cuda.Stream()):
+            check()
+    else:
+        check()
+    dci.free()
+
+
+def test_positions_side_by_side_in_a_graph(gpu):
+    """Recorded before they were formed, recorded when there is room for them but another index's, and recorded when they stand."""
+    from dciknn_cuda_amd import _capi
+    from test_gpu_rounds import ALWAYS, NEVER, _ask
+    M, L, B, T, k, outer, dim, nq = 2, 9, 4, 100, 8, 60, 24, 80
+    X, Q = _rows("normal", 24000, nq, dim, 7)
+    ids = torch.empty((nq, k), dtype=torch.int32, device="cuda")
+    dists = torch.empty((nq, k), dtype=torch.float32, device="cuda")
+    dci = gpu.DCI(dim, M, L, B, T, seed=5)
+
+    def call(stream, queries=Q):
+        _capi.check(dci._lib.dcih_query(dci._dci_inst, dim, len(queries), queries.data_ptr(), k, 0, outer, 10 * k, B, T,
+                                        ids.data_ptr(), dists.data_ptr(), None, stream))
+    s = torch.cuda.Stream()
+    for turn in ("none", "room", "formed"):
+        if turn != "formed":
+            dci.clear()
+            X = X.flip(0).contiguous()
+            dci.add(X)
+        want = _ask(dci, dci._lib, NEVER, Q, k, outer)
+        if turn == "none":      # (too few queries for the table, with room for all of them)
+            _capi.check(dci._lib.dcih_set_option(dci._dci_inst, _capi.OPT_ROUNDS, ALWAYS))
+            call(0, Q[:12])
+        _capi.check(dci._lib.dcih_set_option(dci._dci_inst, _capi.OPT_ROUNDS, ALWAYS))
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            call(torch.cuda.current_stream().cuda_stream)
+        assert _route(dci)[0] >= 2 and (_plan(dci)[2] > 0) == (turn != "none"), turn
+        for _ in range(3):
+            ids.fill_(-5)
+            dists.fill_(-5.0)
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(ids, want[0]) and torch.equal(dists, want[1]), turn
+            if turn != "room":
+                call(0)                            # eager work between the replays
+                torch.cuda.synchronize()
+                assert torch.equal(ids, want[0]) and torch.equal(dists, want[1]), turn
+        del g
+    dci.free()
