@@ -93,7 +93,7 @@ int64_t dense_max_windows(const QueryArgs& a) { return (int64_t)a.L * (a.ppb / a
 // (point_rows are there where the rules of point_rows_fit and point_rows_pay say so)
 bool by_windows(const QueryArgs& a) { return a.picked && a.near_bounds && a.point_rows && dense_max_windows(a) <= 9 * 512 && a.M * (dense_max_windows(a) + 1) < 32768; }
 
-DenseLayout dense_layout_for(const QueryArgs& a, int nt, int ipt) {
+DenseLayout dense_layout_for(const QueryArgs& a, int nt, int ipt, bool windows_only) {
     DenseLayout y;
     const int I = a.M * a.L;
     y.nt = nt;
@@ -104,7 +104,7 @@ DenseLayout dense_layout_for(const QueryArgs& a, int nt, int ipt) {
     y.off_idx = o;      o += 4 * I * 4;
     y.off_seg = o;      o += (6 * a.L + 2) * 4;
     y.off_q = o;        o += ((a.dim + 3) & ~3) * 4;
-    y.by_windows = by_windows(a) ? 1 : 0;
+    y.by_windows = windows_only ? 1 : 0;
     y.off_time = y.off_tab = y.off_hist = o;
     y.tab_cap = (int)((dense_max_windows(a) + 1) & ~(int64_t)1);
     if (y.by_windows) {
@@ -152,24 +152,33 @@ DenseLayout dense_layout_for(const QueryArgs& a, int nt, int ipt) {
 // fit a CU's LDS, else eight (7021 windows per composite, items taken up by strides: 22.2 ms; four wavefronts per
 // workgroup and eight per CU 25.8).  With more, 128 registers spill in the ranking (17: 46 ms), so there eight wavefronts per CU, of
 // two workgroups as far as a thread can hold the windows.
-DenseLayout make_dense_layout(const QueryArgs& a) {
+DenseLayout dense_layout(const QueryArgs& a, bool windows_only) {
     const int64_t windows = dense_max_windows(a);
     if (a.ppb <= kNarrowPoints)
         for (int i : {5, 9})
-            if (windows <= (int64_t)64 * i) return dense_layout_for(a, 64, i);
+            if (windows <= (int64_t)64 * i) return dense_layout_for(a, 64, i, windows_only);
     for (int i : {5, 9})
         if (windows <= (int64_t)256 * i) {
-            const DenseLayout y = dense_layout_for(a, 256, i);
+            const DenseLayout y = dense_layout_for(a, 256, i, windows_only);
             if (4 * y.lds_bytes <= kLdsBytes) return y;
             break;
         }
     for (int i : {5, 9, 13, 15})
-        if (windows <= (int64_t)512 * i) return dense_layout_for(a, 512, i);
-    if (windows <= (int64_t)256 * 33) return dense_layout_for(a, 256, 33);
-    if (windows <= (int64_t)512 * 21) return dense_layout_for(a, 512, 21);
+        if (windows <= (int64_t)512 * i) return dense_layout_for(a, 512, i, windows_only);
+    if (windows <= (int64_t)256 * 33) return dense_layout_for(a, 256, 33, windows_only);
+    if (windows <= (int64_t)512 * 21) return dense_layout_for(a, 512, 21, windows_only);
     DenseLayout none;
     none.ipt = 0;
     return none;
+}
+constexpr size_t kMostDenseLds = 160 * 1024 - 512;
+// By windows only where that fits: the step tables of many composites can take more room than the points' times.
+DenseLayout make_dense_layout(const QueryArgs& a) {
+    if (by_windows(a)) {
+        const DenseLayout y = dense_layout(a, true);
+        if (y.ipt > 0 && y.lds_bytes <= kMostDenseLds) return y;
+    }
+    return dense_layout(a, false);
 }
 
 // Sums of N rows' lane values over a group of N lanes at once: on entry lane s of the group
@@ -1695,7 +1704,7 @@ bool dense_traversal_supported(const QueryArgs& a, size_t* lds_bytes) {
     const DenseLayout y = make_dense_layout(a);
     if (y.ipt == 0) return false;
     if (lds_bytes) *lds_bytes = y.lds_bytes;
-    return y.lds_bytes <= 160 * 1024 - 512;
+    return y.lds_bytes <= kMostDenseLds;
 }
 
 int query_dense_items(const QueryArgs& a_in, hipStream_t s) {

@@ -212,3 +212,19 @@ def test_positions_side_by_side_in_a_graph(gpu):
                 assert torch.equal(ids, want[0]) and torch.equal(dists, want[1]), turn
         del g
     dci.free()
+
+
+@pytest.mark.parametrize("dim", [64, 4096])
+def test_steps_of_many_composites_do_not_fit_a_workgroup(gpu, dim):
+    """64 composites of 64 simple indices: the steps of all their windows fit a workgroup's memory beside a short query, not beside a long one,
+    whose calls look up all points as before."""
+    from test_gpu_rounds import ALWAYS, NEVER, _ask
+    X, Q = _rows("normal", 4000, 40, dim, 11)
+    dci = gpu.DCI(dim, 64, 64, 4, 250, seed=5)
+    dci.add(X)
+    want = _ask(dci, dci._lib, NEVER, Q, 5, 20)
+    for again in range(2):
+        got = _ask(dci, dci._lib, ALWAYS, Q, 5, 20)
+        assert _route(dci)[0] >= 2 and (_plan(dci)[2] > 0) == (dim == 64)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), again
+    dci.free()
