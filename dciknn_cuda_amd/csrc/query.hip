@@ -499,7 +499,7 @@ bool plan_rounds(QueryArgs& a) {
         fits = fits && (dense || (can_block && block_takes_lists(a)));      // (the step-by-step kernel takes no round's items)
         return dense ? c.dense : c.batch;
     };
-    const double whole = time(1.0), rounds = time(first / B) + (few ? 15.0 : time(share - first / B)) + bounds_cost(a) + 30.0;
+    const double whole = time(1.0), traversals = time(first / B) + (few ? 15.0 : time(share - first / B)), rounds = traversals + bounds_cost(a) + 30.0;
     (void)time(share);
     // Traversals that stop after less than one promotion of fifty points find rows further away than the bounds of most partitions where
     // distances lie close together, and every partition is traversed after all.  Such queries then take all in one round (unit vectors
@@ -530,9 +530,25 @@ bool plan_rounds(QueryArgs& a) {
     // 60000 on 1M rows of 128 at the defaults 132, 22.4, with room for all 21.6; 20000 on 3M unit vectors 407, 172; where bounds rule out little, 30000 on 2M
     // normal rows of 64, 3124, 3187.)  A part of the batch kernel's calls takes its own sample and waits for its own slowest items: 60000 queries, windows
     // of 2, 46.0 ms without the tiles' bounds, 48.9 in two parts.
+    // Left to choose, only parts that would go in rounds with these bounds themselves, and whose reading of the rows again and launches take less
+    // than a third of what the traversals are estimated to: that much, and mostly more, these bounds saved above.
     const size_t near = near_bytes(a);
     if (near > a.near_room) {
-        if (a.pick_near) a.pick_parts = (int)std::min<size_t>((size_t)a.nq, (near + a.near_room - 1) / a.near_room);
+        if (a.pick_near) {
+            QueryArgs part = a;
+            int parts = (int)std::min<size_t>((size_t)a.nq, (near + a.near_room - 1) / a.near_room);
+            for (;; parts += 1 + parts / 8) {      // (few queries' tiles can be smaller ones, and their bounds more)
+                parts = std::min(parts, a.nq);
+                part.nq = (a.nq + parts - 1) / parts;
+                if (part.nq == 1 || near_bytes(part) <= a.near_room) break;
+            }
+            bool pays = a.pick_rule == 2;
+            if (!pays && near_bytes(part) <= a.near_room) {
+                const double again = (double)(parts - 1) * (bounds_cost(part) + 60.0) + bounds_cost(part) - bounds_cost(a);
+                pays = again < 0.3 * traversals && plan_rounds(part) && part.pick_near;
+            }
+            if (pays) a.pick_parts = parts;
+        }
         a.pick_near = a.pick_confirm = a.may_confirm = 0;
     }
     a.pick_sample = sampled ? std::min(a.nq, std::max(2, std::min(16, 1024 / a.B))) : 0;

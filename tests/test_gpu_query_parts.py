@@ -30,3 +30,28 @@ def test_same_as_whole(gpu, shape, parts):
     if parts == 50 and T != 4:      # the last part is four queries at most; all of them take ten partitions and more each
         assert 0 < int(items[:4].sum()) <= 4 * B, items
     dci.free()
+
+
+@pytest.mark.parametrize("float_ids", [False, True])
+@pytest.mark.parametrize("parts", [2, 5, 250])
+def test_chosen_by_itself(gpu, parts, float_ids):
+    """Left to choose, a call comes in parts as long as these are calls in rounds with bounds of tiles themselves; else it goes in rounds as a whole,
+    without those bounds."""
+    from dciknn_cuda_amd import _capi
+    from test_gpu_rounds import _route
+    from test_gpu_steering import _plan
+    n, dim, B, nq, k = 200_000, 64, 100, 2000, 10
+    X, Q = _rows("clusters", n, nq, dim, 5)
+    dci = gpu.DCI(dim, 2, 7, B, 10, seed=3)
+    dci.add(X)
+    want = _ask(dci, dci._lib, NEVER, Q, k, 5000)
+    _capi.check(dci._lib.dcih_set_option(dci._dci_inst, _capi.OPT_ROUNDS, 0))
+    dci.query(Q, k, 5000)
+    assert _route(dci)[0] >= 2 and _route(dci)[1] == 1 and _plan(dci)[1] == 1
+    # (partitions of 2000 rows, tiles of 128, whole ones of up to 512 rows)
+    _capi.check(dci._lib.dcih_debug_near_room(dci._dci_inst, B * 16 * nq * 4 // parts))
+    for again in range(2):
+        ids, dists = dci.query(Q, k, 5000, return_int=not float_ids)
+        assert _route(dci)[0] >= 2 and _route(dci)[1] == (parts < 250) and (_plan(dci)[1] > 1) == (parts < 250)
+        assert torch.equal(ids.int(), want[0]) and torch.equal(dists, want[1]), again
+    dci.free()
