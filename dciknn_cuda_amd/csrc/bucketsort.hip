@@ -17,7 +17,8 @@
 // Bound by LDS and vector issue, a third to two thirds as fast as memory alone would allow: a key costs six randomly addressed LDS operations
 // (the radix kernels 44 to 58) and about 80 instructions, its slice is read once and written once.  20M Gaussian keys, us, by digits and so: slices of 277 points
 // 526, 70; 1111 285, 70; 4000 229, 72; 8000 240, 81; 10000 220, 83; 13000 218, 98; 17142 246, 103; 25000 304, 127.  Slices that are left cost
-// the attempt on top: 20 different keys in 17142 221, 270; many equal ones in pairs and dozens 243, 460.
+// the attempt on top: rows that are there 32 times each, one after the other (all slices left), slices of 100 points 256, 498; 277 531, 427; 1111 281, 324;
+// 2000 203, 334; 4000 220, 363; 8000 231, 372; 17142 249, 367; 25000 292, 468.  20 different keys in 17142 237, 265.
 #include <type_traits>
 
 #include "common.h"

@@ -53,12 +53,10 @@ __device__ inline unsigned long long pack_key(float key, uint32_t pos) {
 // slice and the result goes straight to skeys/sids; otherwise the packed words
 // go to `packed` for the merge passes.
 template <bool FINAL>
-__global__ void segsort_tile_kernel(const float* __restrict__ keys, SegGeom g,
-                                    float* __restrict__ skeys, int32_t* __restrict__ sids,
-                                    uint16_t* __restrict__ inv, uint16_t* __restrict__ lids,
-                                    unsigned long long* __restrict__ packed, int np2) {
-    extern __shared__ unsigned long long s[];
-    const int64_t flat = blockIdx.x;
+__device__ __forceinline__ void tile_slice(unsigned long long* s, int64_t flat, const float* __restrict__ keys, const SegGeom& g,
+                                           float* __restrict__ skeys, int32_t* __restrict__ sids,
+                                           uint16_t* __restrict__ inv, uint16_t* __restrict__ lids,
+                                           unsigned long long* __restrict__ packed, int np2) {
     const int tile = (int)(flat % g.tiles);
     const int b = (int)((flat / g.tiles) % g.B);
     const int64_t i = flat / ((int64_t)g.tiles * g.B);
@@ -104,6 +102,14 @@ __global__ void segsort_tile_kernel(const float* __restrict__ keys, SegGeom g,
         __syncthreads();
         for (int j = threadIdx.x; j < m; j += blockDim.x) inv[base + j] = (uint16_t)pos_of[j];
     }
+}
+template <bool FINAL>
+__global__ void segsort_tile_kernel(const float* __restrict__ keys, SegGeom g,
+                                    float* __restrict__ skeys, int32_t* __restrict__ sids,
+                                    uint16_t* __restrict__ inv, uint16_t* __restrict__ lids,
+                                    unsigned long long* __restrict__ packed, int np2) {
+    extern __shared__ unsigned long long s[];
+    tile_slice<FINAL>(s, blockIdx.x, keys, g, skeys, sids, inv, lids, packed, np2);
 }
 
 // ---------------------------------------------------------------------------
@@ -247,11 +253,14 @@ __global__ __launch_bounds__(kRadixThreads, (kRadixThreads == 256 && IPT > 45) ?
     radix_slice<kRadixThreads, IPT>(rs, blockIdx.x, keys, g, skeys, sids, inv, lids, packed);
 }
 // Only the slices that the bucket kernel has left, usually none, where there are many: a workgroup looks at 64 of them at a time.  (A
-// workgroup for each costs 40 us of 130 for 62500 slices of 320 points.)
+// workgroup for each costs 40 us of 130 for 62500 slices of 320 points.)  All may be left as well, of tables that hold many copies of a row, so the shapes fit the
+// slice as closely as those that sorted every slice, and as many workgroups start as the device holds (20M keys in copies, with four shapes and half as
+// many workgroups: slices of 100 points 1967 us, now 498; 277 781, 427; 2000 780, 334; 4000 476, 363).
+constexpr int kLeftByWave = 128;       // up to this the bitonic sort is faster, one wavefront's (100 points: 345 us of those 498; by digits 1800 of 1967)
 template <int kRadixThreads, int IPT>
 __global__ __launch_bounds__(kRadixThreads) void segsort_left_kernel(const float* __restrict__ keys, SegGeom g, int64_t slices, float* __restrict__ skeys,
                                                                      int32_t* __restrict__ sids, uint16_t* __restrict__ inv) {
-    extern __shared__ uint32_t rs[];
+    extern __shared__ __align__(16) uint32_t rs[];
     for (int64_t first = blockIdx.x; first < slices; first += (int64_t)gridDim.x * kWave) {
         const int64_t mine = first + (int64_t)(threadIdx.x & (kWave - 1)) * gridDim.x;
         const int64_t at = (int64_t)(mine % g.B) * g.ppb;
@@ -260,7 +269,10 @@ __global__ __launch_bounds__(kRadixThreads) void segsort_left_kernel(const float
             const int next = __ffsll((long long)left) - 1;
             left &= left - 1ull;
             __syncthreads();                                  // (all have seen the marks, and the last slice's room is free)
-            radix_slice<kRadixThreads, IPT>(rs, first + (int64_t)next * gridDim.x, keys, g, skeys, sids, inv, nullptr, nullptr);
+            if constexpr (kRadixThreads * IPT <= kLeftByWave)
+                tile_slice<true>(reinterpret_cast<unsigned long long*>(rs), first + (int64_t)next * gridDim.x, keys, g, skeys, sids, inv, nullptr, nullptr, kLeftByWave);
+            else
+                radix_slice<kRadixThreads, IPT>(rs, first + (int64_t)next * gridDim.x, keys, g, skeys, sids, inv, nullptr, nullptr);
         }
     }
 }
@@ -274,7 +286,7 @@ static int launch_left(const float* d_keys, const SegGeom& g, int num_indices, f
     });
     if (rc) return rc;
     const int64_t slices = (int64_t)num_indices * g.B;
-    hipLaunchKernelGGL((segsort_left_kernel<NT, IPT>), dim3((unsigned)min(slices, (int64_t)(NT == 64 ? 2048 : 512))), dim3(NT), lds, s,
+    hipLaunchKernelGGL((segsort_left_kernel<NT, IPT>), dim3((unsigned)min(slices, (int64_t)(NT * IPT <= kLeftByWave ? 8192 : (4096 * 64) / NT))), dim3(NT), lds, s,
                        d_keys, g, slices, d_skeys, d_sids, d_inv);
     DCIH_HIP(hipGetLastError());
     return 0;
@@ -767,7 +779,8 @@ int segsort(const float* d_keys, int64_t key_stride, int num_indices, int64_t n,
         if (rc) return rc;
         // (few long slices: a launch of a workgroup for each looks at the marks as fast)
 #define DCIH_LEFT(NT, IPT) if (g.ppb <= (int64_t)(NT) * (IPT)) return launch_left<NT, IPT>(d_keys, g, num_indices, d_skeys, d_sids, d_inv, s)
-        DCIH_LEFT(64, 9); DCIH_LEFT(64, 21); DCIH_LEFT(256, 21); DCIH_LEFT(256, 35);
+        DCIH_LEFT(64, 2); DCIH_LEFT(64, 5); DCIH_LEFT(64, 9); DCIH_LEFT(64, 13); DCIH_LEFT(64, 17); DCIH_LEFT(64, 21); DCIH_LEFT(64, 25);
+        DCIH_LEFT(64, 33); DCIH_LEFT(128, 21); DCIH_LEFT(128, 27); DCIH_LEFT(128, 33); DCIH_LEFT(256, 21); DCIH_LEFT(256, 27); DCIH_LEFT(256, 35);
 #undef DCIH_LEFT
         g.left_only = 1;
     }

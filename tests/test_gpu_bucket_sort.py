@@ -81,3 +81,61 @@ def test_positions_are_the_inverse(gpu, n, block_size):
                 assert (np.diff(keys[i, a:a + per]) >= 0).all()
         dci.clear()
     dci.free()
+
+
+def _copies(rng, rows, n, of):
+    """Each key `of` times, one after the other: more than a bucket may hold."""
+    return np.ascontiguousarray(np.repeat(rng.standard_normal((rows, -(-n // of))), of, axis=1)[:, :n], dtype=np.float32)
+
+
+# the ends of every shape that sorts what is left
+@pytest.mark.parametrize("per", [65, 100, 128, 129, 1345, 1600, 1601, 2112, 2113, 2688, 2689, 3456, 3457, 4224, 4225, 5376, 5377, 6912, 6913, 8960])
+def test_copies_of_rows(gpu, per):
+    """Slices of which none, some and all are left."""
+    rng = np.random.default_rng(per)
+    keys = _copies(rng, 3, 4 * per - 1, 32)
+    keys[1] = rng.standard_normal(keys.shape[1])
+    keys[2, per:2 * per] = rng.standard_normal(per)
+    got_k, got_i = engine_segsort(keys, 4)
+    want_k, want_i = _sorted(keys, 4)
+    np.testing.assert_array_equal(got_i, want_i)
+    np.testing.assert_array_equal(got_k.view(np.uint32), want_k.view(np.uint32))
+
+
+@pytest.mark.parametrize("per,block_size", [(80, 12000), (300, 5000), (2200, 1500)])
+def test_copies_of_rows_in_many_slices(gpu, per, block_size):
+    """More of them than workgroups start."""
+    rng = np.random.default_rng(per)
+    n = per * block_size
+    keys = _copies(rng, 2, n, 32)
+    keys[1, n // 2:] = rng.standard_normal(n - n // 2)
+    got_k, got_i = engine_segsort(keys, block_size)
+    want = keys.reshape(2, block_size, per)
+    order = np.argsort(want, axis=2, kind="stable")
+    np.testing.assert_array_equal(got_i.reshape(2, block_size, per), order + per * np.arange(block_size)[None, :, None])
+    np.testing.assert_array_equal(got_k.reshape(2, block_size, per), np.take_along_axis(want, order, axis=2))
+
+
+def test_copies_of_rows_cost_no_multiple(gpu):
+    """All slices left: the attempt and the sort by digits, about three times as long here as where none is left (twelve times when few workgroups
+    shared them, each with room for slices six times as long)."""
+    from dciknn_cuda_amd import _capi
+    rows, n, block_size = 20, 500_000, 5000
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    plain = torch.randn(rows, n, generator=gen, device="cuda")
+    copies = plain[:, :n // 32 + 1].repeat_interleave(32, 1)[:, :n].contiguous()
+    out = torch.empty_like(plain), torch.empty(plain.shape, dtype=torch.int32, device="cuda")
+
+    def best(keys):
+        times = []
+        for _ in range(8):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            _capi.check(_capi.lib().dcih_segsort(keys.data_ptr(), rows, n, block_size, out[0].data_ptr(), out[1].data_ptr(),
+                                                 torch.cuda.current_stream().cuda_stream))
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+    a, b = best(plain), best(copies)
+    assert b < 7 * a, (a, b)
