@@ -228,3 +228,24 @@ def test_steps_of_many_composites_do_not_fit_a_workgroup(gpu, dim):
         assert _route(dci)[0] >= 2 and (_plan(dci)[2] > 0) == (dim == 64)
         assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), again
     dci.free()
+
+
+@pytest.mark.parametrize("kind", ["normal", "sorted", "dup", "broken", "zero"])
+@pytest.mark.parametrize("shape", [(20000, 96, 3, 8, 4, 128, 100, 100), (30000, 16, 2, 15, 4, 64, 9, 50), (24000, 64, 4, 5, 4, 48, 3, 150), (18000, 33, 3, 9, 3, 100, 10, 60),
+                                   (24000, 40, 16, 2, 4, 48, 5, 150), (24001, 24, 8, 1, 4, 64, 9, 150)],
+                         ids=["eight", "fifteen", "four composites", "three", "many composites", "one index each"])
+def test_all_items_by_first_lanes(gpu, kind, shape):
+    """Rounds whose items all go to the kernel that looks up first lanes of windows: several composites, and more promotions by first lanes (one a window and composite)
+    than a workgroup lists, half as many as it ranks windows of a composite (the last two)."""
+    from test_gpu_rounds import ALWAYS, NEVER, _ask
+    n, dim, M, L, B, T, k, outer = shape
+    X, Q = _rows(kind, n, 70, dim, n + dim)
+    dci = gpu.DCI(dim, M, L, B, T, seed=5)
+    dci.add(X)
+    want = _ask(dci, dci._lib, NEVER, Q, k, outer)
+    for again in range(3):
+        got = _ask(dci, dci._lib, ALWAYS, Q, k, outer)
+        assert torch.equal(got[0], want[0]), again
+        assert torch.equal(got[1].view(torch.int32), want[1].view(torch.int32)), again
+    assert _route(dci)[0] >= 2 and _plan(dci)[0] == 0 and _plan(dci)[2] > 0
+    dci.free()
