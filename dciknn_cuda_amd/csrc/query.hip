@@ -709,7 +709,7 @@ int query(const QueryArgs& a_in, void* bounds_ws, hipStream_t s, hipEvent_t* ev,
             a.near_bounds = p.near_bounds; a.near_limit = p.near_limit; a.near_stride = p.near_stride;
             a.near_shift = p.near_shift; a.near_tiles = p.near_tiles;
             // The batch kernel's first launch covers all that may come in the first round, where queries whose bounds lie close together take
-            // every partition: strides over the rest take up to twice as long, a workgroup without an item 0.2 ns.  (4000 queries, 58 partitions
+            // every partition: strides over the rest take up to twice as long, a workgroup without an item 0.5 ns.  (4000 queries, 58 partitions
             // of 17242 normal rows of 128: 15.2 ms whole, 18.9 in rounds that covered 131072 items.)
             a.picked_cover = round ? std::max((int64_t)(0.3 * (double)a.nq * (double)a.B), (int64_t)65536) : (int64_t)a.nq * a.B;
             if (a.pick_confirm && round) a.picked_cover = std::min(a.picked_cover, (int64_t)16384);

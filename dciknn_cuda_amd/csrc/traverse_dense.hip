@@ -1686,9 +1686,10 @@ int launch_dense(const DenseArgs& args, unsigned grid, hipStream_t s) {
 
 // By windows: n / T + 3 first lanes of every simple index cost two reads from random lines and L look-ups each, by points
 // every one of the n costs one look-up that a coalesced read feeds; a read of a line of its own takes as long as a dozen look-ups.
-// That line is where the room for them is kept.  What decides beyond it is the LDS: a time for every point leaves two workgroups to a CU from about
-// 16000 points on (1M rows, 12 indices, windows of 96 in partitions of 25000: 6.17 ms by points, 3.29 by windows; 8 indices, windows of 64, 16667: 2.47,
-// 1.81; of 10000, windows of 64 to 128, four kinds of rows: 0.96 to 1.06; below, 0.80 to 1.07), and calls that wait for single items lose a tenth.
+// What decides beyond that is the LDS: a time for every point takes room that leaves fewer workgroups to a CU, two from about 16000 points on.  1000 queries on 1M
+// rows, us by points and by windows: unit vectors, 8 indices, windows of 128, partitions of 8000 points 1437, 1297; 10000 1602, 1462; 12500 1826, 1638; 16129
+// 2393, 1818.  Normal rows, 12 indices, windows of 96: 1360, 1223; 1664, 1422; 2105, 1622; 3778, 2400.  A noisy manifold, 12 indices, windows of 64: 1550, 1577; 1602,
+// 1573; 2539, 2437; 3948, 3944.  Shorter partitions give between 0.80 and 1.07 of their times by points, and calls that wait for single items lose a tenth.
 bool point_rows_pay(const QueryArgs& a) {
     return a.pick_rule == 2 || (a.ppb >= 8000 && (double)a.nq * (double)a.B * a.share >= 4096.0);
 }

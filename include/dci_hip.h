@@ -90,7 +90,8 @@ enum {
  * all distances.  Results are the same to the bit in every case.  Room for the bounds (up to 1 GiB
  * for those of 64 or 128 rows each, and 4 bytes per query and part of a partition) is
  * part of the handle's workspace and stays with it until dcih_free; where there is none the
- * call is traversed whole.
+ * call is traversed whole.  A call whose bounds would take more than that 1 GiB is answered in parts
+ * of its queries, one after the other on the same stream, where that is estimated to be faster.
  */
 enum { DCIH_OPT_TRAVERSAL = 0, DCIH_OPT_DENSE_MIN_PROMOTIONS = 1, DCIH_OPT_FORGET_HINTS = 2, DCIH_OPT_APPEND = 3,
        DCIH_OPT_ROUNDS = 4 };
@@ -269,7 +270,9 @@ int dcih_set_option(dcih_index* h, int option, int value);
  * the reference).  After dcih_profile(h, 1) every dcih_add / dcih_query
  * brackets its kernels with events; dcih_last_timings waits for them and
  * writes DCIH_NUM_TIMERS durations in milliseconds (-1 for a kernel that has
- * not run since profiling was switched on).
+ * not run since profiling was switched on).  Of a query that was answered in parts
+ * (see DCIH_OPT_ROUNDS) DCIH_T_TRAVERSE and DCIH_T_DENSE reach from the first part's start to the
+ * last one's end, with what lies between the parts; DCIH_T_QPROJECT and DCIH_T_MERGE are the last part's.
  */
 int dcih_profile(dcih_index* h, int enable);
 int dcih_last_timings(dcih_index* h, float* h_ms);

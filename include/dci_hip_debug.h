@@ -55,13 +55,14 @@ int dcih_debug_positions(dcih_index* h, uint16_t* d_inv, uint16_t* d_rpos, void*
  * [0] its rounds (0: everything was traversed at once, or nothing was), [1] whether bounds of
  * tiles of rows were kept for the dense kernel, [2] the queries that were traversed whole first
  * to decide about rounds, [3] the queries whose results were selected by bounds of all rows.
+ * Of a query that was answered in parts these are the last part's.
  */
 int dcih_debug_route(const dcih_index* h, int64_t* route);
 /*
  * d_items is NULL (off) or a device array of 6 uint32 to which later queries in rounds write
  * the number of (query, partition) pairs of each round, then, where some queries decided about
  * the rounds, whether everything was taken at once and how many of the pairs they looked at
- * could not be ruled out.
+ * could not be ruled out.  Every part of a query that is answered in parts writes its own over them.
  */
 int dcih_debug_round_items(dcih_index* h, uint32_t* d_items);
 /*
