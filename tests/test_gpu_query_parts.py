@@ -55,3 +55,44 @@ def test_chosen_by_itself(gpu, parts, float_ids):
         assert _route(dci)[0] >= 2 and _route(dci)[1] == (parts < 250) and (_plan(dci)[1] > 1) == (parts < 250)
         assert torch.equal(ids.int(), want[0]) and torch.equal(dists, want[1]), again
     dci.free()
+
+
+def test_in_a_graph(gpu):
+    """Parts are recorded like any other call: after one that has taken the room, and replayed on other queries in the same buffer."""
+    from dciknn_cuda_amd import _capi
+    from test_gpu_rounds import _route
+    from test_gpu_steering import _plan
+    n, dim, B, T, nq, k, outer, parts = 30_000, 24, 12, 10, 400, 5, 500, 3
+    X, Q = _rows("clusters", n, 2 * nq, dim, 9)
+    dci = gpu.DCI(dim, 2, 7, B, T, seed=3)
+    dci.add(X)
+    want = [_ask(dci, dci._lib, NEVER, q, k, outer) for q in (Q[:nq], Q[nq:])]
+    _capi.check(dci._lib.dcih_set_option(dci._dci_inst, _capi.OPT_ROUNDS, ALWAYS))
+    _capi.check(dci._lib.dcih_debug_near_room(dci._dci_inst, B * 40 * nq * 4 // parts))      # (tiles of 64 rows)
+    q = Q[:nq].clone()
+    ids = torch.empty((nq, k), dtype=torch.int32, device="cuda")
+    dists = torch.empty((nq, k), dtype=torch.float32, device="cuda")
+
+    def call(stream):
+        _capi.check(dci._lib.dcih_query(dci._dci_inst, dim, nq, q.data_ptr(), k, 0, outer, 10 * k, B, T, ids.data_ptr(), dists.data_ptr(), None, stream))
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    call(s.cuda_stream)
+    s.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        call(torch.cuda.current_stream().cuda_stream)
+    assert _route(dci)[0] >= 2 and _route(dci)[1] == 1 and _plan(dci)[1] >= 2
+    for turn in (0, 1, 0, 1):
+        q.copy_(Q[turn * nq:(turn + 1) * nq])
+        ids.fill_(-5)
+        dists.fill_(-5.0)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(ids, want[turn][0]) and torch.equal(dists, want[turn][1]), turn
+        call(0)                                # eager work between the replays
+        torch.cuda.synchronize()
+        assert torch.equal(ids, want[turn][0]) and torch.equal(dists, want[turn][1]), turn
+    del g
+    dci.free()
