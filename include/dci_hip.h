@@ -193,6 +193,8 @@ int dcih_append(dcih_index* h, int dim, int64_t num_points, const float* d_data,
  * that follow as long as it holds theirs (without memory for it nothing is formed).  Under
  * stream capture nothing is allocated and no codes are formed; what calls before the
  * capture have allocated and formed is used.
+ * A recorded call reads the index's tables as they stood: after dcih_add, dcih_append or
+ * dcih_clear it has to be recorded again before it is replayed.
  *
  * blind != 0 (query_config.blind, :498-505, :754-773, :859-864): the same
  * traversal under the same stop rule, but no distance is computed.  d_nn is
